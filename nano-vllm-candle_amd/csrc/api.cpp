@@ -454,9 +454,72 @@ static void free_kv(nvllm_model* m) {
     m->d_block_tables = nullptr; m->d_ids = nullptr; m->d_pos = m->d_slot = m->d_tile_row0 = m->d_tile_nrows = m->d_tile_slot = m->d_last_rows = m->d_tile_order = m->d_tile_last = m->d_group_order = nullptr;
     m->resid = m->slabs = m->qbuf = m->logits = m->d_maxval = m->red = nullptr; m->xh = m->xl = m->xh2 = m->xl2 = m->ctxh = m->ctxl = nullptr; m->ssqA = m->ssqB = nullptr; m->d_next = nullptr; m->part_val = nullptr; m->part_idx = nullptr; m->argmax_scratch = nullptr; m->attn_po = m->attn_pml = nullptr;
     m->tap_h = m->tap_res = nullptr; m->cosv = m->sinv = nullptr; m->tickets = nullptr; m->qkv_out = nullptr; m->d_keys = nullptr; m->d_temps = nullptr;
-    if (m->h_stage) (void)hipHostFree(m->h_stage);
-    m->h_stage = nullptr;
+    stage_release(m);
     m->num_blocks = 0;
+}
+
+int stage_alloc(nvllm_model* m, size_t ints) {
+    Staging& g = m->stage;
+    g.ints = (ints + 63) / 64 * 64;
+    HIPCHK(m->ctx, hipHostMalloc((void**)&g.host, g.ints * Staging::kSlots * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
+    HIPCHK(m->ctx, hipHostGetDevicePointer((void**)&g.dev, g.host, 0));
+    for (hipEvent_t& e : g.ev) HIPCHK(m->ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    return NVLLM_OK;
+}
+void stage_release(nvllm_model* m) {
+    Staging& g = m->stage;
+    if (g.host) (void)hipHostFree(g.host);
+    for (hipEvent_t e : g.ev) if (e) (void)hipEventDestroy(e);
+    g = Staging();
+    m->table_news.clear();
+}
+int stage_begin(nvllm_model* m) {
+    Staging& g = m->stage;
+    g.slot = (g.slot + 1) % Staging::kSlots;
+    if (g.busy[g.slot]) {
+        if (g.recorded[g.slot]) {
+            HIPCHK(m->ctx, hipEventSynchronize(g.ev[g.slot]));
+            g.busy[g.slot] = false;
+        } else {
+            HIPCHK(m->ctx, hipStreamSynchronize(m->ctx->stream));
+            for (bool& b : g.busy) b = false;
+        }
+    }
+    g.used = 0;
+    g.n_runs = g.longest = 0;
+    return NVLLM_OK;
+}
+static int* stage_room(nvllm_model* m, int* dst, size_t n, int pairs) {
+    Staging& g = m->stage;
+    const size_t ints = n << pairs;
+    if (g.n_runs == kStageRuns || g.used + ints > g.ints) return nullptr;
+    g.args.run[g.n_runs++] = StageRun{dst, (int)g.used, (int)n, pairs};
+    g.longest = std::max(g.longest, (int)ints);
+    int* p = g.host + (size_t)g.slot * g.ints + g.used;
+    g.used = std::min(g.ints, (g.used + ints + 3) / 4 * 4);
+    return p;
+}
+static void stage_idle(nvllm_model* m) { for (bool& b : m->stage.busy) b = false; }  // the stream has been waited for
+int* stage_put(nvllm_model* m, int* dst, size_t n) { return stage_room(m, dst, n, 0); }
+int stage_flush(nvllm_model* m, bool more) {
+    Staging& g = m->stage;
+    if (!m->table_news.empty()) {
+        int* p = stage_room(m, m->d_block_tables, m->table_news.size(), 1);
+        if (p) for (int at : m->table_news) { *p++ = at; *p++ = m->h_block_tables[at]; }
+        // steps that took blocks and failed can leave more than the block holds: the whole table instead
+        else HIPCHK(m->ctx, hipMemcpyAsync(m->d_block_tables, m->h_block_tables.data(), m->h_block_tables.size() * 4, hipMemcpyHostToDevice, m->ctx->stream));
+        m->table_news.clear();
+    }
+    if (!g.n_runs) return NVLLM_OK;
+    g.args.src = g.dev + (size_t)g.slot * g.ints;
+    HIPCHK(m->ctx, launch_stage(g.args, g.n_runs, g.longest, m->ctx->stream));
+    g.busy[g.slot] = true;
+    g.recorded[g.slot] = false;
+    if (more) {
+        HIPCHK(m->ctx, hipEventRecord(g.ev[g.slot], m->ctx->stream));
+        g.recorded[g.slot] = true;
+    }
+    return NVLLM_OK;
 }
 
 extern "C" int nvllm_model_destroy(nvllm_model* m) {
@@ -815,9 +878,10 @@ extern "C" int nvllm_kv_alloc(nvllm_model* m, int num_blocks, int block_size, in
     if (!rc) rc = dmalloc(ctx, &m->argmax_scratch, (size_t)max_seqs + 1);
     if (!rc) HIPCHK(ctx, hipMemsetAsync(m->argmax_scratch, 0, ((size_t)max_seqs + 1) * 8, ctx->stream));
     if (rc) return rc;
-    m->h_stage_bytes = (R * 24 + (size_t)max_seqs * 4) * sizeof(int) + 256;
-    HIPCHK(ctx, hipHostMalloc(&m->h_stage, m->h_stage_bytes, hipHostMallocDefault));
     rc = m->dec ? m->dec->kv_alloc(m) : qwen3_kv_alloc(m);
+    // three ints a row and up to 21 a tile of a row (empty tiles of the groups of four included), the head's rows, every block a
+    // step can take, each run padded to four
+    if (!rc) rc = stage_alloc(m, R * 24 + (size_t)max_seqs + 2 * (size_t)num_blocks + (m->dec ? m->dec->plan_ints(m) : 0) + 4 * kStageRuns);
     if (rc) { m->num_blocks = 0; return rc; }
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     return NVLLM_OK;
@@ -1353,7 +1417,11 @@ static int ensure_blocks(nvllm_model* m, SeqState& s, int len) {
     while ((int)s.blocks.size() < need) {
         const int b = m->free_blocks.back();
         m->free_blocks.pop_back();
-        m->h_block_tables[(size_t)s.slot * m->max_blocks + s.blocks.size()] = b;
+        const size_t at = (size_t)s.slot * m->max_blocks + s.blocks.size();
+        if (m->h_block_tables[at] != b) {
+            m->h_block_tables[at] = b;
+            m->table_news.push_back((int)at);
+        }
         s.blocks.push_back(b);
     }
     return NVLLM_OK;
@@ -1471,39 +1539,29 @@ struct RowPlan {
     std::vector<int> pos, slot, tile_row0, tile_nrows, tile_slot, last_rows;
 };
 
-// upload one chunk's metadata through the pinned staging buffer (one H2D copy per array kind)
-static int upload_chunk(nvllm_model* m, const RowPlan& p, int r0, int R, int t0, int T, const std::vector<int>& last_local) {
-    nvllm_ctx* ctx = m->ctx;
-    hipStream_t s = ctx->stream;
-    HIPCHK(ctx, hipStreamSynchronize(s));  // staging buffer reuse
-    int* st = (int*)m->h_stage;
-    int* h_ids = st; int* h_pos = st + R; int* h_slot = st + 2 * R;
-    int* h_t0 = st + 3 * R; int* h_tn = h_t0 + T; int* h_ts = h_tn + T; int* h_last = h_ts + T;
-    memcpy(h_ids, p.ids.data() + r0, (size_t)R * 4);
-    memcpy(h_pos, p.pos.data() + r0, (size_t)R * 4);
-    memcpy(h_slot, p.slot.data() + r0, (size_t)R * 4);
-    for (int i = 0; i < T; ++i) { h_t0[i] = p.tile_row0[t0 + i] - r0; h_tn[i] = p.tile_nrows[t0 + i]; h_ts[i] = p.tile_slot[t0 + i]; }
-    for (size_t i = 0; i < last_local.size(); ++i) h_last[i] = last_local[i];
+// one chunk's metadata into the pinned block (stage_begin before, stage_flush after)
+static int upload_chunk(nvllm_model* m, const RowPlan& p, int r0, int R, int t0, int T, const std::vector<int>& last_local, bool device_ids = false) {
+    auto put = [&](const void* src, void* dst, size_t n) {
+        int* h = stage_put(m, (int*)dst, n);
+        if (h && src) memcpy(h, src, n * 4);
+        return h;
+    };
+    const bool ids = device_ids || put(p.ids.data() + r0, m->d_ids, R);
+    const bool rows = put(p.pos.data() + r0, m->d_pos, R) && put(p.slot.data() + r0, m->d_slot, R);
+    int *h_t0 = put(nullptr, m->d_tile_row0, T), *h_tn = put(p.tile_nrows.data() + t0, m->d_tile_nrows, T), *h_ts = put(p.tile_slot.data() + t0, m->d_tile_slot, T);
+    const bool last = last_local.empty() || put(last_local.data(), m->d_last_rows, last_local.size());
     // attention load balance: q-tiles ordered by context length, longest first (stable for ties); an empty padding tile
     // (prefill groups of four) has no last row: it sorts as -1, behind every real tile
-    int* h_ord = h_last + m->max_seqs;
-    int* h_tl = h_ord + T;  // position of each tile's last row (-1: padding tile)
+    int* h_ord = put(nullptr, m->d_tile_order, T);
+    int* h_tl = put(nullptr, m->d_tile_last, T);  // position of each tile's last row (-1: padding tile)
+    const int G = T % kPrefillTileGroup == 0 ? T / kPrefillTileGroup : 0;
+    int* h_go = G ? put(nullptr, m->d_group_order, G) : h_tl;
+    if (!ids || !rows || !h_t0 || !h_tn || !h_ts || !last || !h_ord || !h_tl || !h_go) return fail(m->ctx, NVLLM_ESTATE, "internal: metadata block of %zu ints too small", m->stage.ints);
+    for (int i = 0; i < T; ++i) h_t0[i] = p.tile_row0[t0 + i] - r0;
     for (int i = 0; i < T; ++i) h_tl[i] = p.tile_nrows[t0 + i] > 0 ? p.pos[p.tile_row0[t0 + i] + p.tile_nrows[t0 + i] - 1] : -1;
     for (int i = 0; i < T; ++i) h_ord[i] = i;
     std::stable_sort(h_ord, h_ord + T, [&](int x, int y) { return h_tl[x] > h_tl[y]; });
-    HIPCHK(ctx, hipMemcpyAsync(m->d_ids, h_ids, (size_t)R * 4, hipMemcpyHostToDevice, s));
-    HIPCHK(ctx, hipMemcpyAsync(m->d_pos, h_pos, (size_t)R * 4, hipMemcpyHostToDevice, s));
-    HIPCHK(ctx, hipMemcpyAsync(m->d_slot, h_slot, (size_t)R * 4, hipMemcpyHostToDevice, s));
-    HIPCHK(ctx, hipMemcpyAsync(m->d_tile_row0, h_t0, (size_t)T * 4, hipMemcpyHostToDevice, s));
-    HIPCHK(ctx, hipMemcpyAsync(m->d_tile_nrows, h_tn, (size_t)T * 4, hipMemcpyHostToDevice, s));
-    HIPCHK(ctx, hipMemcpyAsync(m->d_tile_slot, h_ts, (size_t)T * 4, hipMemcpyHostToDevice, s));
-    if (!last_local.empty())
-        HIPCHK(ctx, hipMemcpyAsync(m->d_last_rows, h_last, last_local.size() * 4, hipMemcpyHostToDevice, s));
-    HIPCHK(ctx, hipMemcpyAsync(m->d_tile_order, h_ord, (size_t)T * 4, hipMemcpyHostToDevice, s));
-    HIPCHK(ctx, hipMemcpyAsync(m->d_tile_last, h_tl, (size_t)T * 4, hipMemcpyHostToDevice, s));
-    if (T % kPrefillTileGroup == 0) {  // prefill attention: groups of four q-tiles, longest context first
-        int* h_go = h_tl + T;
-        const int G = T / kPrefillTileGroup;
+    if (G) {  // prefill attention: groups of four q-tiles, longest context first
         std::vector<int> glast(G);
         for (int g = 0; g < G; ++g) {
             int mx = -1;
@@ -1516,7 +1574,6 @@ static int upload_chunk(nvllm_model* m, const RowPlan& p, int r0, int R, int t0,
         // a CU, so the longest context gets the shortest of the next block as its neighbour and the CU to itself sooner
         const int per = std::max(1, 256 / std::max(1, m->kv_l));
         for (int b0 = per; b0 < G; b0 += 2 * per) std::reverse(h_go + b0, h_go + std::min(G, b0 + per));
-        HIPCHK(ctx, hipMemcpyAsync(m->d_group_order, h_go, (size_t)G * 4, hipMemcpyHostToDevice, s));
     }
     return NVLLM_OK;
 }
@@ -1620,7 +1677,6 @@ static int step_impl(nvllm_model* m, int n_seqs, const int64_t* seq_ids, const u
     }
     // carried state moves on with the rows: if this step fails, the sequences start again
     if (recurrent) for (int i = 0; i < n_seqs; ++i) m->seqs[seq_ids[i]].cached = 0;
-    HIPCHK(ctx, hipMemcpyAsync(m->d_block_tables, m->h_block_tables.data(), m->h_block_tables.size() * 4, hipMemcpyHostToDevice, ctx->stream));
     m->want_logits = last_logits != nullptr || temperatures != nullptr || score != nullptr;  // sampling reads the last-row logits on the device
     m->cur_n = n_seqs;
     m->cur_max_len = *std::max_element(lens, lens + n_seqs);
@@ -1649,6 +1705,8 @@ static int step_impl(nvllm_model* m, int n_seqs, const int64_t* seq_ids, const u
     for (int i = 0; i < n_seqs; ++i) kv_read_tokens += lens[i];
     int r0 = 0, logits_row = 0;
     size_t hr = 0;  // next head row
+    // more wanted rows than the head's buffers hold: every chunk's logits leave before the next chunk's come
+    const bool score_at_once = score && (int)head_rows.size() > m->max_seqs;
     std::vector<int> row_seq(total_rows);
     { int r = 0; for (int i = 0; i < n_seqs; ++i) for (int t = start[i]; t < lens[i]; ++t) row_seq[r++] = i; }
     while (r0 < total_rows) {
@@ -1669,7 +1727,8 @@ static int step_impl(nvllm_model* m, int n_seqs, const int64_t* seq_ids, const u
         }
         std::vector<int> last_local;
         for (; hr < head_rows.size() && head_rows[hr] < r0 + R; ++hr) last_local.push_back(head_rows[hr] - r0);
-        int rc = upload_chunk(m, p, r0, R, 0, (int)p.tile_row0.size(), last_local);
+        int rc = stage_begin(m);
+        if (!rc) rc = upload_chunk(m, p, r0, R, 0, (int)p.tile_row0.size(), last_local);
         if (rc) return rc;
         if (m->dec) {
             std::vector<int> local(p.tile_row0);
@@ -1677,9 +1736,11 @@ static int step_impl(nvllm_model* m, int n_seqs, const int64_t* seq_ids, const u
             rc = m->dec->plan_chunk(m, p.pos.data() + r0, p.slot.data() + r0, row_seq.data() + r0, R, local.data(), (int)local.size(), qt);
             if (rc) return rc;
         }
-        rc = forward_chunk(m, R, (int)p.tile_row0.size(), qt, (int)last_local.size(), score ? 0 : logits_row);
+        rc = stage_flush(m, r0 + R < total_rows);
         if (rc) return rc;
-        if (score && !last_local.empty()) {
+        rc = forward_chunk(m, R, (int)p.tile_row0.size(), qt, (int)last_local.size(), score_at_once ? 0 : logits_row);
+        if (rc) return rc;
+        if (score_at_once && !last_local.empty()) {
             rc = download_logits(m, (int)last_local.size(), score->logits + (size_t)logits_row * m->cfg.vocab_size);
             if (rc) return rc;
         }
@@ -1701,7 +1762,12 @@ static int step_impl(nvllm_model* m, int n_seqs, const int64_t* seq_ids, const u
         HIPCHK(ctx, hipStreamSynchronize(ctx->stream));  // keys / temperatures are read from pageable host memory above
     }
     if (score) {
+        if (!score_at_once && !head_rows.empty()) {
+            const int rc = download_logits(m, (int)head_rows.size(), score->logits);
+            if (rc) return rc;
+        }
         HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+        stage_idle(m);
         const int rc_os = oneshot_check(ctx);
         if (rc_os) return rc_os;
         for (int i = 0; i < n_seqs; ++i) {
@@ -1715,6 +1781,7 @@ static int step_impl(nvllm_model* m, int n_seqs, const int64_t* seq_ids, const u
     }
     int rc = finish_logits(m, n_seqs, next_ids, last_logits);
     if (rc) return rc;
+    stage_idle(m);
     m->last_ids.assign(seq_ids, seq_ids + n_seqs);
     m->last_lens.assign(lens, lens + n_seqs);
     m->decode_resident = all_single && total_rows <= m->max_rows;
@@ -1738,21 +1805,21 @@ static int decode_core(nvllm_model* m) {
     if (n > m->max_rows) return fail(ctx, NVLLM_ESTATE, "%d decode rows > %d rows of step buffers", n, m->max_rows);
     HIPCHK(ctx, hipSetDevice(ctx->device));
     hipStream_t s = ctx->stream;
-    bool table_dirty = false;
     for (int i = 0; i < n; ++i) {
         auto it = m->seqs.find(m->last_ids[i]);
         if (it == m->seqs.end()) return fail(ctx, NVLLM_ESTATE, "sequence %lld of the previous step is gone", (long long)m->last_ids[i]);
         SeqState& st = it->second;
         const int len = m->last_lens[i] + 1;
         if (len > m->rope_len) return fail(ctx, NVLLM_EINVAL, "sequence %d would exceed max positions %d", i, m->rope_len);
-        const size_t before = st.blocks.size();
         int rc = ensure_blocks(m, st, len);
         if (rc) return rc;
-        table_dirty |= st.blocks.size() != before;
     }
-    if (table_dirty)
-        HIPCHK(ctx, hipMemcpyAsync(m->d_block_tables, m->h_block_tables.data(), m->h_block_tables.size() * 4, hipMemcpyHostToDevice, s));
     if (m->decode_resident) {
+        if (!m->table_news.empty()) {
+            int rc = stage_begin(m);
+            if (!rc) rc = stage_flush(m, true);
+            if (rc) return rc;
+        }
         // ids <- last greedy ids, pos += 1: the batch metadata is already on the device
         HIPCHK(ctx, launch_advance_decode(m->d_ids, m->d_next, m->d_pos, n, s));
     } else {
@@ -1761,11 +1828,13 @@ static int decode_core(nvllm_model* m) {
         std::vector<int> last_local(n);
         for (int i = 0; i < n; ++i) {
             const SeqState& st = m->seqs[m->last_ids[i]];
-            p.ids.push_back(0); p.pos.push_back(m->last_lens[i]); p.slot.push_back(st.slot);
+            p.pos.push_back(m->last_lens[i]); p.slot.push_back(st.slot);
             p.tile_row0.push_back(i); p.tile_nrows.push_back(1); p.tile_slot.push_back(st.slot);
             last_local[i] = i;
         }
-        int rc0 = upload_chunk(m, p, 0, n, 0, n, last_local);
+        int rc0 = stage_begin(m);
+        if (!rc0) rc0 = upload_chunk(m, p, 0, n, 0, n, last_local, true);
+        if (!rc0) rc0 = stage_flush(m, true);
         if (rc0) return rc0;
         HIPCHK(ctx, hipMemcpyAsync(m->d_ids, m->d_next, (size_t)n * 4, hipMemcpyDeviceToDevice, s));
         m->decode_resident = true;

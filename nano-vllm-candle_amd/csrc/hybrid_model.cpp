@@ -77,8 +77,8 @@ struct HybridModel : DecoderImpl {
     float *y = nullptr, *ctx_f[2] = {nullptr, nullptr}, *act_f = nullptr;  // 32-bit mode
     bf16_bits *ctx2h = nullptr, *ctx2l = nullptr;                          // the second mixer's context
     ExpertsScratch experts;
-    int *d_seg = nullptr, *h_seg = nullptr, n_seg = 0;       // first row, rows, slot, first piece of every segment of the chunk
-    int *d_piece = nullptr, n_piece = 0, piece_cap = 0;      // first row, rows of every 16-token piece (staged behind h_seg)
+    int *d_seg = nullptr, n_seg = 0;                         // first row, rows, slot, first piece of every segment of the chunk
+    int *d_piece = nullptr, n_piece = 0, piece_cap = 0;      // first row, rows of every 16-token piece
     float *pc_pair = nullptr, *pc_q = nullptr, *pc_w = nullptr, *pc_k = nullptr, *pc_decay = nullptr;
     int opt_scan = 0;                                        // recurrences: token by token in prompt chunks too
     int opt_plain = 0;                                       // attention: the plain kernel instead of the matrix-core ones
@@ -93,6 +93,7 @@ struct HybridModel : DecoderImpl {
     int64_t kv_read_bytes(int len) const override;
     int tile_rows(int qt) const override { return qt == 1 ? 1 : kBiasTileRows; }
     bool recurrent() const override { return has_state; }
+    size_t plan_ints(const nvllm_model* m) const override { return (size_t)4 * m->max_seqs + 2 * piece_cap; }
     int plan_chunk(nvllm_model* m, const int* pos, const int* slot, const int* seq, int R, const int* tile_row0, int n_tiles, int qt) override;
     int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last, int logits_row0) override;
     int option(const char* name, int value) override {
@@ -345,9 +346,8 @@ void HybridModel::free_kv() {
         *p = nullptr;
     }
     if (d_seg) (void)hipFree(d_seg);
-    if (h_seg) (void)hipHostFree(h_seg);
     if (d_piece) (void)hipFree(d_piece);
-    d_seg = h_seg = d_piece = nullptr;
+    d_seg = d_piece = nullptr;
     n_seg = n_piece = 0;
 }
 
@@ -709,7 +709,6 @@ int HybridModel::kv_alloc(nvllm_model* m) {
     for (auto& b : pieces) if (!rc && b.n) rc = dmalloc(ctx, b.p, (size_t)piece_cap * b.n);
     if (!rc) rc = dmalloc(ctx, &d_seg, (size_t)4 * m->max_seqs);
     if (!rc) rc = dmalloc(ctx, &d_piece, (size_t)2 * piece_cap);
-    if (!rc) HIPCHK(ctx, hipHostMalloc((void**)&h_seg, ((size_t)4 * m->max_seqs + 2 * piece_cap) * sizeof(int), hipHostMallocDefault));
     m->rope_len = (int)std::min<int64_t>((int64_t)m->max_blocks * kBlockTokens, 1 << 20);  // positions a block table covers
     for (RopeTable& r : ropes) if (!rc) rc = r.upload(ctx, m->rope_len);
     return rc;
@@ -719,22 +718,27 @@ int HybridModel::kv_alloc(nvllm_model* m) {
 // forward over one chunk of rows
 // ---------------------------------------------------------------------------------------------------
 int HybridModel::plan_chunk(nvllm_model* m, const int*, const int* slot, const int* seq, int R, const int*, int, int qt) {
-    nvllm_ctx* ctx = m->ctx;
     n_seg = n_piece = 0;
     if (qt == 1) return NVLLM_OK;
     const int cap = m->max_seqs;
-    int *h_piece0 = h_seg + 3 * cap, *h_row0 = h_seg + 4 * cap, *h_n = h_row0 + piece_cap;
     for (int r = 0; r < R; ++n_seg) {
         int e = r;
         while (e < R && seq[e] == seq[r]) ++e;
-        h_seg[n_seg] = r; h_seg[cap + n_seg] = e - r; h_seg[2 * cap + n_seg] = slot[r];
+        n_piece += (e - r + kPiece - 1) / kPiece;
+        r = e;
+    }
+    int *h_row = stage_put(m, d_seg, n_seg), *h_rows = stage_put(m, d_seg + cap, n_seg), *h_slot = stage_put(m, d_seg + 2 * cap, n_seg), *h_piece0 = stage_put(m, d_seg + 3 * cap, n_seg);
+    int *h_row0 = stage_put(m, d_piece, n_piece), *h_n = stage_put(m, d_piece + piece_cap, n_piece);
+    if (!h_row || !h_rows || !h_slot || !h_piece0 || !h_row0 || !h_n) return fail(m->ctx, NVLLM_ESTATE, "internal: the chunk's metadata does not fit its block");
+    n_seg = n_piece = 0;
+    for (int r = 0; r < R; ++n_seg) {
+        int e = r;
+        while (e < R && seq[e] == seq[r]) ++e;
+        h_row[n_seg] = r; h_rows[n_seg] = e - r; h_slot[n_seg] = slot[r];
         h_piece0[n_seg] = n_piece;
         for (; r < e; r += kPiece, ++n_piece) { h_row0[n_piece] = r; h_n[n_piece] = std::min(kPiece, e - r); }
         r = e;
     }
-    // the staging buffer is free: the tile upload before this call waited for the stream
-    HIPCHK(ctx, hipMemcpyAsync(d_seg, h_seg, (size_t)4 * cap * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(ctx, hipMemcpyAsync(d_piece, h_row0, (size_t)2 * piece_cap * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
     return NVLLM_OK;
 }
 

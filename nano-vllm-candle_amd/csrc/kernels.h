@@ -374,6 +374,18 @@ hipError_t launch_prefetch_ranges(const PrefetchRange* d_ranges, int n_ranges, u
 // debug: XCC_ID of every workgroup of a (gx,gy,gz) grid, out[linear workgroup id]
 hipError_t launch_xcc_map(int gx, int gy, int gz, int threads, int* out, hipStream_t s);
 // token feedback for nvllm_decode_next: ids[i] = next[i]; pos[i] += 1
+// A step's metadata: runs of ints in one pinned host block, each to an array of its own on the device
+struct StageRun {
+    int* dst = nullptr;
+    int src = 0, n = 0;  // first int in the block (a multiple of 4), ints; pairs: n (index, value) pairs
+    int pairs = 0;
+};
+constexpr int kStageRuns = 24;
+struct StageArgs {
+    const int* src = nullptr;  // device address of the pinned block
+    StageRun run[kStageRuns];
+};
+hipError_t launch_stage(const StageArgs& a, int n_runs, int longest, hipStream_t s);
 hipError_t launch_advance_decode(uint32_t* ids, const uint32_t* next, int* pos, int n, hipStream_t s);
 
 }  // namespace nvllm

@@ -57,7 +57,7 @@ struct LatentModel : DecoderImpl {
     // expanded prompt attention: scratch keys / values, the chunk's cache tiles (device) and segments
     f16_bits *kx = nullptr, *vx = nullptr;
     int exp_cap = 0, exp_n = 0;        // entries allocated; entries of this chunk (0: the absorbed form)
-    int *d_exp = nullptr, *d_tile_exp = nullptr, *h_exp = nullptr;
+    int *d_exp = nullptr, *d_tile_exp = nullptr;
     struct Segment { int pos0, n; };
     std::vector<Segment> segments;
     float *y1 = nullptr, *y2 = nullptr, *ctx_f = nullptr, *act_f = nullptr, *cq_f = nullptr;  // 32-bit mode
@@ -76,6 +76,7 @@ struct LatentModel : DecoderImpl {
     int64_t kv_read_bytes(int len) const override;
     int tile_rows(int qt) const override { return qt == 1 ? 1 : kLatentTileRows; }
     bool recurrent() const override { return has_state; }
+    size_t plan_ints(const nvllm_model* m) const override { return (size_t)3 * exp_cap + m->max_rows + scan.plan_ints(); }
     int plan_chunk(nvllm_model* m, const int* pos, const int* slot, const int* seq, int R, const int* tile_row0, int n_tiles, int qt) override;
     int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last, int logits_row0) override;
 };
@@ -213,8 +214,6 @@ void LatentModel::free_kv() {
     L.x2h = L.x2l = nullptr;
     L.kx = L.vx = nullptr;
     L.d_exp = L.d_tile_exp = nullptr;
-    if (L.h_exp) (void)hipHostFree(L.h_exp);
-    L.h_exp = nullptr;
     L.exp_cap = L.exp_n = 0;
     L.y1 = L.y2 = L.ctx_f = L.act_f = L.cq_f = nullptr;
     L.cqh = L.cql = nullptr;
@@ -508,7 +507,6 @@ int LatentModel::kv_alloc(nvllm_model* m) {
         if (!rc) rc = dmalloc(ctx, &L.vx, (size_t)L.exp_cap * 32 * vx_row);
         if (!rc) rc = dmalloc(ctx, &L.d_exp, (size_t)3 * L.exp_cap);
         if (!rc) rc = dmalloc(ctx, &L.d_tile_exp, R);
-        if (!rc) HIPCHK(ctx, hipHostMalloc((void**)&L.h_exp, ((size_t)3 * L.exp_cap + R) * sizeof(int), hipHostMallocDefault));
     }
     if (rc) return rc;
     // rotation tables, one per rotation: angle p * f_i
@@ -537,22 +535,28 @@ int LatentModel::plan_chunk(nvllm_model* m, const int* pos, const int* slot, con
     bool all = false;
     for (const LatentLayer& w : L.layers)
         if (!w.scan.on()) { all |= w.c.window <= 0; widest = std::max(widest, w.c.window); }
+    auto first_tile = [&](int r) { return all ? 0 : std::max(0, pos[r] - widest + 1) >> 5; };
     int n = 0;
-    int *h_slot = L.h_exp, *h_tile = L.h_exp + L.exp_cap, *h_pos0 = L.h_exp + 2 * L.exp_cap, *h_te = L.h_exp + 3 * L.exp_cap;
+    for (int r = 0; r < R;) {
+        int e = r;
+        while (e < R && seq[e] == seq[r]) ++e;
+        n += (pos[e - 1] >> 5) + 1 - first_tile(r);
+        if (n > L.exp_cap) return NVLLM_OK;  // much context for few rows: absorbed
+        r = e;
+    }
+    int *h_slot = stage_put(m, L.d_exp, n), *h_tile = stage_put(m, L.d_exp + L.exp_cap, n), *h_pos0 = stage_put(m, L.d_exp + 2 * L.exp_cap, n), *h_te = stage_put(m, L.d_tile_exp, n_tiles);
+    if (!h_slot || !h_tile || !h_pos0 || !h_te) return fail(ctx, NVLLM_ESTATE, "internal: the chunk's metadata does not fit its block");
+    n = 0;
     int k = 0;  // q-tile
     for (int r = 0; r < R;) {
         int e = r;
         while (e < R && seq[e] == seq[r]) ++e;
-        const int lo = all ? 0 : std::max(0, pos[r] - widest + 1) >> 5, hi = (pos[e - 1] >> 5) + 1;
-        if (n + hi - lo > L.exp_cap) return NVLLM_OK;  // much context for few rows: absorbed
+        const int lo = first_tile(r), hi = (pos[e - 1] >> 5) + 1;
         for (; k < n_tiles && tile_row0[k] < e; ++k) h_te[k] = n - lo;
         for (int t = lo; t < hi; ++t, ++n) { h_slot[n] = slot[r]; h_tile[n] = t; h_pos0[n] = pos[r]; }
         L.segments.push_back({pos[r], e - r});
         r = e;
     }
-    // the staging buffer is free: the tile upload before this call waited for the stream
-    HIPCHK(ctx, hipMemcpyAsync(L.d_exp, L.h_exp, (size_t)3 * L.exp_cap * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
-    HIPCHK(ctx, hipMemcpyAsync(L.d_tile_exp, h_te, (size_t)n_tiles * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
     L.exp_n = n;
     return NVLLM_OK;
 }

@@ -92,6 +92,22 @@ struct SeqState {
     int released = 0;  // leading blocks given back because no window reaches them (blocks[i] = -1)
 };
 
+// Pinned blocks for the metadata of chunks (stage_kernel): the host fills the next one while the device may still read the others.
+struct Staging {
+    static constexpr int kSlots = 4;
+    int *host = nullptr, *dev = nullptr;  // kSlots blocks of `ints`
+    size_t ints = 0, used = 0;
+    int slot = 0, n_runs = 0, longest = 0;
+    bool busy[kSlots] = {}, recorded[kSlots] = {};
+    hipEvent_t ev[kSlots] = {};
+    StageArgs args;
+};
+int stage_alloc(nvllm_model* m, size_t ints);
+void stage_release(nvllm_model* m);
+int stage_begin(nvllm_model* m);                    // a block the device no longer reads
+int* stage_put(nvllm_model* m, int* dst, size_t n); // room for n ints bound for dst; nullptr: the block is full
+int stage_flush(nvllm_model* m, bool more);         // launches; more: the stream is not waited for before the next block is filled
+
 struct DecoderImpl;  // decoder.h
 
 struct nvllm_model {
@@ -159,8 +175,8 @@ struct nvllm_model {
     int cur_n = 0;              // sequences of the step in flight
     int cur_max_len = 0;        // longest of them (tokens, the new ones included)
     size_t slab_floats = 0;
-    void* h_stage = nullptr;  // pinned
-    size_t h_stage_bytes = 0;
+    Staging stage;
+    std::vector<int> table_news;  // entries of h_block_tables the device does not have yet
     float *tap_h = nullptr, *tap_res = nullptr;
     bool taps = false;
     int tap_rows = 0;

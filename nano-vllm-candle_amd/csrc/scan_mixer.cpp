@@ -117,13 +117,11 @@ int ScanScratch::alloc(nvllm_model* m, bool f32) {
             if (!rc) rc = alloc_vec(ctx, reinterpret_cast<float**>(p), n_x / 2 + 16 * (n_x / std::max(1, m->max_rows)) / 2);  // read in whole 16-row blocks
     const size_t ints = (size_t)3 * seg_cap + 5 * piece_cap;
     if (!rc) rc = dmalloc(ctx, &d_plan, ints);
-    if (!rc) HIPCHK(ctx, hipHostMalloc((void**)&h_plan, ints * sizeof(int), hipHostMallocDefault));
     return rc;
 }
 void ScanScratch::release() {
     for (void* p : {(void*)x, (void*)dt, (void*)dbc, (void*)carry, (void*)carry_dt, (void*)xh, (void*)xl, (void*)d_plan})
         if (p) (void)hipFree(p);
-    if (h_plan) (void)hipHostFree(h_plan);
     *this = ScanScratch();
 }
 
@@ -133,8 +131,19 @@ int ScanScratch::plan(nvllm_model* m, const int* slot, const int* seq, int R) {
     if (!d_plan) return NVLLM_OK;
     // as many pieces as fill the chip beside the channels, of equal length
     const int want = std::max(1, kScanWaves / waves), longest = std::max(kShortestPiece, up((R + want - 1) / want, 16));
-    int *row0 = h_plan, *cnt = row0 + seg_cap, *sl = cnt + seg_cap;
-    int *p_row0 = sl + seg_cap, *p_n = p_row0 + piece_cap, *p_slot = p_n + piece_cap, *p_at = p_slot + piece_cap, *p_of = p_at + piece_cap;
+    int segs = 0, pieces = 0;
+    for (int r = 0; r < R; ++segs) {
+        int e = r;
+        while (e < R && seq[e] == seq[r]) ++e;
+        pieces += (e - r + longest - 1) / longest;
+        r = e;
+    }
+    int* h[8];
+    for (int i = 0; i < 8; ++i) {
+        h[i] = i < 3 ? stage_put(m, d_plan + i * seg_cap, segs) : stage_put(m, d_plan + 3 * seg_cap + (i - 3) * piece_cap, pieces);
+        if (!h[i]) return fail(ctx, NVLLM_ESTATE, "internal: the chunk's metadata does not fit its block");
+    }
+    int *row0 = h[0], *cnt = h[1], *sl = h[2], *p_row0 = h[3], *p_n = h[4], *p_slot = h[5], *p_at = h[6], *p_of = h[7];
     for (int r = 0; r < R; ++n_seg) {
         int e = r;
         while (e < R && seq[e] == seq[r]) ++e;
@@ -147,8 +156,6 @@ int ScanScratch::plan(nvllm_model* m, const int* slot, const int* seq, int R) {
         }
         r = e;
     }
-    // the staging buffer is free: the tile upload before this call waited for the stream
-    HIPCHK(ctx, hipMemcpyAsync(d_plan, h_plan, ((size_t)3 * seg_cap + 5 * piece_cap) * sizeof(int), hipMemcpyHostToDevice, ctx->stream));
     return NVLLM_OK;
 }
 

@@ -24,11 +24,12 @@ struct ScanMixer {
 struct ScanScratch {
     float *x = nullptr, *dt = nullptr, *dbc = nullptr, *carry = nullptr, *carry_dt = nullptr;
     bf16_bits *xh = nullptr, *xl = nullptr;
-    int *d_plan = nullptr, *h_plan = nullptr, piece_cap = 0, seg_cap = 0;
+    int *d_plan = nullptr, piece_cap = 0, seg_cap = 0;
     int n_seg = 0, n_piece = 0, several = 0;
     void reserve(const ScanMixer& w, size_t rows);
     int alloc(nvllm_model* m, bool f32);
     void release();
+    size_t plan_ints() const { return d_plan ? (size_t)3 * seg_cap + 5 * piece_cap : 0; }
     int plan(nvllm_model* m, const int* slot, const int* seq, int R);  // segments and pieces of a prompt chunk
 private:
     size_t n_x = 0, n_dt = 0, n_dbc = 0, n_carry = 0, n_carry_dt = 0;
