@@ -541,6 +541,33 @@ hipError_t launch_latent_rows(const LatentRowsArgs& a, int rows, hipStream_t s) 
 // ---------------------------------------------------------------------------------------------------
 // per-head products: wave = NT n-tiles x MT m-tiles of one head, fragments straight from memory
 // ---------------------------------------------------------------------------------------------------
+// features f0 .. f0 + 3 of one head's product in a row
+__device__ __forceinline__ void head_gemm_put(const HeadGemmArgs& a, int head, int f0, int row, f32x4 v) {
+    if (f0 >= a.n_valid || row >= a.M) return;
+    const bool whole = f0 + 4 <= a.n_valid;
+    if (a.decay_bias) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int f = min(f0 + r, a.n_valid - 1);
+            if (!a.decay_rate) {
+                v[r] = softplusf(v[r] + a.decay_bias[f]);
+            } else if (head == 0) {
+                v[r] = expf(-a.decay_rate[f] * softplusf(v[r] + a.decay_bias[f]));
+            } else {
+                v[r] = 1.0f / (1.0f + expf(-v[r]));
+            }
+        }
+    }
+    if (a.y) {
+        float* o = a.y + (size_t)row * a.y_row + (size_t)head * a.y_head + f0;
+        if (whole && ((a.y_row | a.y_head) & 3) == 0) *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
+        else
+            for (int r = 0; r < 4; ++r)
+                if (f0 + r < a.n_valid) o[r] = v[r];
+    }
+    if (a.yh) put_planes4(a.yh, a.yl, row, head * a.n_valid + f0, a.n_valid - f0, a.ld, a.packed, v);
+}
+
 template <int MT, int NT, bool EXACT>
 __global__ void __launch_bounds__(256) head_gemm_kernel(HeadGemmArgs a) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -599,38 +626,71 @@ __global__ void __launch_bounds__(256) head_gemm_kernel(HeadGemmArgs a) {
         }
     }
 #pragma unroll
-    for (int n = 0; n < NT; ++n) {
-        const int f0 = (nt0 + n) * 16 + grp * 4;
-        if (f0 >= a.n_valid || nt0 + n >= ntiles) continue;
-        const bool whole = f0 + 4 <= a.n_valid;
+    for (int n = 0; n < NT; ++n)
+        if (nt0 + n < ntiles)
 #pragma unroll
-        for (int b = 0; b < MT; ++b) {
-            const int row = m0 + b * 16 + l15;
-            if (row >= a.M) continue;
-            f32x4 v = acc[n][b];
-            if (a.decay_bias) {
+            for (int b = 0; b < MT; ++b) head_gemm_put(a, head, (nt0 + n) * 16 + grp * 4, m0 + b * 16 + l15, acc[n][b]);
+}
+
+// A 32-bit product of up to 64 rows: 16 features x MT row tiles x the whole K per workgroup, K dealt out to its NW waves, partial sums
+// met in LDS.  Bound by latency: a wave asks for U k-tiles of weights and rows at once, so a K of 1024 is one or two round trips to
+// memory, where one wave walking all of K with one k-tile in flight made 32.  Measured, 16 rows: the thirteen products of a decode step of
+// three 1024-wide layers (K 1024 to 4608, N 1024 to 8192, the head of 32768 x 1024) 40 us each before, 10 now.
+template <int MT, int NW>
+__global__ void __launch_bounds__(NW * 64) exact_rows_kernel(HeadGemmArgs a) {
+    constexpr int U = MT == 1 ? 4 : MT == 2 ? 3 : 2;
+    __shared__ f32x4 part[NW][MT][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int l15 = lane & 15, grp = lane >> 4;
+    const int KT = a.K >> 5, head = blockIdx.y, m0 = blockIdx.z * (MT * 16);
+    const uint4* wp = a.w + (size_t)head * a.w_head + (size_t)blockIdx.x * KT * 64 + lane;
+    const float* xp[MT];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int f = min(f0 + r, a.n_valid - 1);
-                    if (!a.decay_rate) {
-                        v[r] = softplusf(v[r] + a.decay_bias[f]);
-                    } else if (head == 0) {
-                        v[r] = expf(-a.decay_rate[f] * softplusf(v[r] + a.decay_bias[f]));
-                    } else {
-                        v[r] = 1.0f / (1.0f + expf(-v[r]));
-                    }
-                }
+    for (int b = 0; b < MT; ++b) xp[b] = a.x + (size_t)min(m0 + b * 16 + l15, a.M - 1) * a.x_row + (size_t)head * a.x_head + grp * 8;
+    f32x4 acc[MT];
+#pragma unroll
+    for (int b = 0; b < MT; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = wave; k0 < KT; k0 += U * NW) {
+        uint4 wf[U];
+        float xv[U][MT][8];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int kt = min(k0 + u * NW, KT - 1);
+            wf[u] = wp[(size_t)kt * 64];
+#pragma unroll
+            for (int b = 0; b < MT; ++b) {
+                *reinterpret_cast<float4*>(&xv[u][b][0]) = *reinterpret_cast<const float4*>(xp[b] + kt * 32);
+                *reinterpret_cast<float4*>(&xv[u][b][4]) = *reinterpret_cast<const float4*>(xp[b] + kt * 32 + 4);
             }
-            if (a.y) {
-                float* o = a.y + (size_t)row * a.y_row + (size_t)head * a.y_head + f0;
-                if (whole && ((a.y_row | a.y_head) & 3) == 0) *reinterpret_cast<float4*>(o) = make_float4(v[0], v[1], v[2], v[3]);
-                else
-                    for (int r = 0; r < 4; ++r)
-                        if (f0 + r < a.n_valid) o[r] = v[r];
+        }
+        __builtin_amdgcn_sched_barrier(0);  // all of them on their way before the first product waits
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (k0 + u * NW >= KT) break;  // the same for every lane of the wave
+            const uint32_t wd[4] = {wf[u].x, wf[u].y, wf[u].z, wf[u].w};
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float wv = (j & 1) ? __builtin_bit_cast(float, wd[j >> 1] & 0xffff0000u) : __builtin_bit_cast(float, wd[j >> 1] << 16);
+#pragma unroll
+                for (int b = 0; b < MT; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv, xv[u][b][j], acc[b], 0, 0, 0);
             }
-            if (a.yh) put_planes4(a.yh, a.yl, row, head * a.n_valid + f0, a.n_valid - f0, a.ld, a.packed, v);
         }
     }
+#pragma unroll
+    for (int b = 0; b < MT; ++b) part[wave][b][lane] = acc[b];
+    __syncthreads();
+    if (wave >= MT) return;
+    f32x4 v = part[0][wave][lane];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) v += part[w][wave][lane];
+    head_gemm_put(a, head, blockIdx.x * 16 + grp * 4, m0 + wave * 16 + l15, v);
+}
+template <int MT>
+static hipError_t exact_rows_launch(const HeadGemmArgs& a, hipStream_t s) {
+    const dim3 grid(a.N / 16, a.heads, (a.M + MT * 16 - 1) / (MT * 16));
+    if (a.K >= 2048) exact_rows_kernel<MT, 16><<<grid, 1024, 0, s>>>(a);
+    else exact_rows_kernel<MT, 8><<<grid, 512, 0, s>>>(a);
+    return hipGetLastError();
 }
 
 template <int MT, int NT>
@@ -643,6 +703,8 @@ static hipError_t head_gemm_launch(const HeadGemmArgs& a, hipStream_t s) {
 hipError_t launch_head_gemm(const HeadGemmArgs& a, hipStream_t s) {
     if (a.N % 16 || a.K % 32 || a.x_row % 4 || a.x_head % 4 || a.n_valid > a.N || (!a.y && !a.yh)) return hipErrorInvalidValue;
     if (a.M <= 0) return hipSuccess;
+    // few rows in 32 bits: K over a workgroup's waves, unless it is too short for them
+    if (a.exact && a.M <= 64 && a.K >= 256) return a.M <= 16 ? exact_rows_launch<1>(a, s) : a.M <= 32 ? exact_rows_launch<2>(a, s) : exact_rows_launch<4>(a, s);
     if (a.M <= 16) return head_gemm_launch<1, 1>(a, s);
     if (a.M <= 64) return head_gemm_launch<2, 1>(a, s);
     return head_gemm_launch<4, 2>(a, s);
