@@ -463,7 +463,6 @@ int stage_alloc(nvllm_model* m, size_t ints) {
     g.ints = (ints + 63) / 64 * 64;
     HIPCHK(m->ctx, hipHostMalloc((void**)&g.host, g.ints * Staging::kSlots * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
     HIPCHK(m->ctx, hipHostGetDevicePointer((void**)&g.dev, g.host, 0));
-    for (hipEvent_t& e : g.ev) HIPCHK(m->ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
     return NVLLM_OK;
 }
 void stage_release(nvllm_model* m) {
@@ -516,6 +515,7 @@ int stage_flush(nvllm_model* m, bool more) {
     g.busy[g.slot] = true;
     g.recorded[g.slot] = false;
     if (more) {
+        if (!g.ev[g.slot]) HIPCHK(m->ctx, hipEventCreateWithFlags(&g.ev[g.slot], hipEventDisableTiming));
         HIPCHK(m->ctx, hipEventRecord(g.ev[g.slot], m->ctx->stream));
         g.recorded[g.slot] = true;
     }
@@ -879,9 +879,10 @@ extern "C" int nvllm_kv_alloc(nvllm_model* m, int num_blocks, int block_size, in
     if (!rc) HIPCHK(ctx, hipMemsetAsync(m->argmax_scratch, 0, ((size_t)max_seqs + 1) * 8, ctx->stream));
     if (rc) return rc;
     rc = m->dec ? m->dec->kv_alloc(m) : qwen3_kv_alloc(m);
-    // three ints a row and up to 21 a tile of a row (empty tiles of the groups of four included), the head's rows, every block a
-    // step can take, each run padded to four
-    if (!rc) rc = stage_alloc(m, R * 24 + (size_t)max_seqs + 2 * (size_t)num_blocks + (m->dec ? m->dec->plan_ints(m) : 0) + 4 * kStageRuns);
+    // a chunk's metadata at most: three ints a row, five and a quarter a tile (every tile has a row, but for up to three that fill a
+    // sequence's last group of four), the head's rows, a pair for every block a step can take; each run padded to four
+    const size_t tiles = std::min(4 * R, R + 3 * (size_t)max_seqs);
+    if (!rc) rc = stage_alloc(m, 3 * R + 5 * tiles + tiles / 4 + (size_t)max_seqs + 2 * (size_t)num_blocks + (m->dec ? m->dec->plan_ints(m) : 0) + 4 * kStageRuns);
     if (rc) { m->num_blocks = 0; return rc; }
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     return NVLLM_OK;
@@ -1570,10 +1571,6 @@ static int upload_chunk(nvllm_model* m, const RowPlan& p, int r0, int R, int t0,
             h_go[g] = g;
         }
         std::stable_sort(h_go, h_go + G, [&](int x, int y) { return glast[x] > glast[y]; });
-        // every other block of 256 workgroups (256 / kv heads groups) backwards: workgroups i and i + 256 tend to share
-        // a CU, so the longest context gets the shortest of the next block as its neighbour and the CU to itself sooner
-        const int per = std::max(1, 256 / std::max(1, m->kv_l));
-        for (int b0 = per; b0 < G; b0 += 2 * per) std::reverse(h_go + b0, h_go + std::min(G, b0 + per));
     }
     return NVLLM_OK;
 }
