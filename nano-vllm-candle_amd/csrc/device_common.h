@@ -39,6 +39,20 @@ __device__ __forceinline__ float max3_raw(float a, float b, float c) {
     return r;
 }
 
+// eight values as f16 hi + lo (hi + lo = x to 22 bits), both to nearest even: pairs by v_cvt_pk_f16_f32, the remainder by one mixed
+// fused multiply-add per value
+__device__ __forceinline__ void split_f16x8(const float (&x)[8], f16x8& hi, f16x8& lo) {
+    typedef __attribute__((ext_vector_type(2))) float f32x2;
+    typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) {
+        const f16x2 h = __builtin_convertvector((f32x2){x[j], x[j + 1]}, f16x2);
+        const f16x2 l = __builtin_convertvector((f32x2){__builtin_fmaf((float)h[0], -1.0f, x[j]), __builtin_fmaf((float)h[1], -1.0f, x[j + 1])}, f16x2);
+        hi[j] = h[0]; hi[j + 1] = h[1];
+        lo[j] = l[0]; lo[j + 1] = l[1];
+    }
+}
+
 // SiluAndMul (src/layers/activation.rs:13-18) in the GEMM epilogues: x * sigmoid(x) * up with v_rcp_f32 (1 ulp) instead
 // of an IEEE division (a dozen instructions per element: 1.5 us of a 256 x 192 tile's epilogue).  exp overflow gives
 // rcp(inf) = 0, i.e. -0 for very negative gates; no NaN.  The fine-seam op keeps the division.
@@ -340,6 +354,14 @@ typedef __attribute__((address_space(3))) void* lptr_t;
         __builtin_amdgcn_sched_barrier(0);                             \
     } while (0)
 __device__ __forceinline__ uint32_t lds_address(const void* p) { return (uint32_t)(uintptr_t)(lptr_t)p; }
+
+// 1 KiB of LDS-DMA that hipcc's wait insertion does not see: `src` per lane, the wave's 1 KiB of LDS at byte address `lds` (uniform).  With
+// the builtin, every ordinary LDS read after it waits for vmcnt(0), which drains the copies meant to stay in flight; with this form
+// ordinary reads stay ordinary, and the kernel's own vmcnt waits are the only ones.  For kernels whose LDS-DMA is all of this form (M0 is
+// set here and is nobody else's).
+__device__ __forceinline__ void lds_dma16(const void* src, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+}
 
 // Barrier that PUBLISHES LDS-DMA data (global_load_lds): every wave first waits for its own DMA to land, then joins the
 // barrier; only then may any wave ds_read fragments another wave staged.  __syncthreads() alone is not enough: hipcc

@@ -2144,28 +2144,34 @@ __global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(A
 // ---------------------------------------------------------------------------------------------------
 // Prefill attention with LDS-staged K/V (same math as attn_paged_kernel, qwen3.rs:236-277).
 // One workgroup = FOUR consecutive q-tiles of ONE sequence (host pads every sequence's tile list to a multiple of four
-// with empty tiles) x one kv head; wave w owns q-tile w for the WHOLE context (no cross-wave combine).  Every 32-token
-// K/V tile is fetched ONCE per workgroup -- 16 KiB by LDS-DMA, 1 KiB per wave-instruction, already in MFMA fragment
-// order so the image is lane-linear -- and read from LDS by the waves that still need it (causal: wave w stops after the
-// tile that holds its last token); the next tile is in flight while the current one is consumed.  The decode kernel,
-// which prefill used before, had every wave fetch its own K/V tiles from global memory: no reuse across q-tiles.
+// with empty tiles) x one kv head x 4 NH waves: wave w owns q-tile w % 4 and every NH-th 32-token K/V tile of the context; with NH = 2
+// the two halves of a q-tile meet in LDS at the end.  A set of NH tiles is fetched ONCE per workgroup -- 16 KiB each by LDS-DMA, 1 KiB
+// per wave-instruction, already in MFMA fragment order so the image is lane-linear -- and read from LDS by the waves that still need it
+// (causal: a wave stops after the tile that holds its last token); two sets are in flight while one is consumed.
+// What bounds it: the chain of one wave through its tiles (QK^T, softmax, PV depend on each other), two waves per SIMD; by counters the
+// matrix cores are busy 45 % of the time, the VALU another 45 %.  NH = 2 halves the chain of the longest context, which sets the end of
+// a launch that does not fill the chip twice over.  Measured per launch (16 / 8 heads of 128) with a maximum across lanes, a rescale and
+// a drained ring in every tile, NH = 1: one prompt of 2391 tokens 109 us, now 65; 18.7 k tokens in prompts of 64 to 512, chunks of 4096
+// rows, 34.5 -> 30.7; 32 / 8 heads, 4050 tokens in prompts of 700 to 2000, 152 -> 118.  Both prompts with the other NH: 80, 42 (before
+// the other changes).
 // ---------------------------------------------------------------------------------------------------
-template <int HD, int QT>
-__global__ void __launch_bounds__(256, 2) attn_prefill_kernel(AttnArgs a) {
+template <int HD, int QT, int NH>
+__global__ void __launch_bounds__(NH * 256, 2) attn_prefill_kernel(AttnArgs a) {
     constexpr int DC = HD / 32, DT = HD / 16, NWV = 4;
     constexpr int TILE_FRAGS = 2 * DC + DT;  // 1 KiB fragments of one 32-token K/V tile: K lo half, K hi half, V
+    constexpr int SET = NH * TILE_FRAGS, COPIES = SET / (4 * NH);  // fragments of NH neighbouring tiles, copies of a wave for them
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-    uint4* lds = reinterpret_cast<uint4*>(smem_raw);  // [3 stages][TILE_FRAGS][64]
+    uint4* lds = reinterpret_cast<uint4*>(smem_raw);  // [3 stages][NH tiles][TILE_FRAGS][64]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l15 = lane & 15, grp = lane >> 4;
     // 1-D grid, kv heads fastest, groups in the host's longest-first order: the dispatcher hands out workgroups in index
     // order, so what is left over when all CU slots are taken (528 workgroups for 512 slots on a 4096-row chunk) must
-    // be the short contexts -- in launch order the late starters were long ones and set the kernel's end (stamps:
-    // start + 16 us, end 36.7 us against 30 us for the longest workgroup of the first wave)
+    // be the short contexts -- in launch order the late starters were long ones and set the kernel's end
     const int kv_heads = a.kv.kv_l;
     const int gi = (int)blockIdx.x / kv_heads, kh = (int)blockIdx.x - gi * kv_heads;
     const int grp4 = a.group_order ? __builtin_amdgcn_readfirstlane(a.group_order[gi]) : gi;
-    const int tile = grp4 * NWV + wave;
+    const int qw = wave & 3, part = wave >> 2;
+    const int tile = grp4 * NWV + qw;
     NVLLM_STAMP(a, 0);
     // wave-uniform values are made scalar explicitly (readfirstlane): the block-table lookup in stage() is then an s_load
     // on the scalar counter; as a vector load it made every iteration wait vmcnt(0) -- for the lookup's own round trip
@@ -2191,7 +2197,7 @@ __global__ void __launch_bounds__(256, 2) attn_prefill_kernel(AttnArgs a) {
         const int4 tl = *reinterpret_cast<const int4*>(a.tile_last + (size_t)grp4 * NWV);
         const int l0 = __builtin_amdgcn_readfirstlane(tl.x), l1 = __builtin_amdgcn_readfirstlane(tl.y),
                   l2 = __builtin_amdgcn_readfirstlane(tl.z), l3 = __builtin_amdgcn_readfirstlane(tl.w);
-        const int mine = wave == 0 ? l0 : wave == 1 ? l1 : wave == 2 ? l2 : l3;
+        const int mine = qw == 0 ? l0 : qw == 1 ? l1 : qw == 2 ? l2 : l3;
         my_last = mine >= 0 ? mine >> 5 : -1;
         const int mx = max(max(l0, l1), max(l2, l3));
         wg_last = mx >= 0 ? mx >> 5 : -1;
@@ -2208,35 +2214,37 @@ __global__ void __launch_bounds__(256, 2) attn_prefill_kernel(AttnArgs a) {
     const int* bt = a.block_tables + (size_t)slot * a.max_blocks;
     const _Float16* kbase = reinterpret_cast<const _Float16*>(a.kv.k);
     const _Float16* vbase = reinterpret_cast<const _Float16*>(a.kv.v);
-    // Block id of tile kt_ by an explicit scalar load (hipcc turns the plain bt[] read into a vector load once the kernel
-    // has issued LDS-DMA writes -- no "noclobber" proof -- and then waits vmcnt(0) for it every iteration, draining the
-    // K/V tiles in flight).  Issued one iteration before its use; blk_ready() is the wait, tied to the value.
-    auto blk_load = [&](int kt_) {
+    const uint32_t lds0 = lds_address(smem_raw);
+    const int last_set = wg_last / NH;
+    // Block id of a set of NH tiles (never across two blocks) by an explicit scalar load (hipcc turns the plain bt[] read into a vector
+    // load once the kernel has issued LDS-DMA writes -- no "noclobber" proof -- and then waits vmcnt(0) for it every iteration,
+    // draining the K/V tiles in flight).  Issued one iteration before its use; blk_ready() is the wait, tied to the value.
+    auto blk_load = [&](int it_) {
         int v;
-        const int* p = bt + (min(kt_, wg_last) >> 3);  // 8 tiles per 256-token block
+        const int* p = bt + (min(it_, last_set) * NH >> 3);  // 8 tiles per 256-token block
         asm volatile("s_load_dword %0, %1, 0x0" : "=s"(v) : "s"(p));
         return v;
     };
     auto blk_ready = [&](int& v) { asm volatile("s_waitcnt lgkmcnt(0)" : "+s"(v)::"memory"); };
-    // stage tile kt into buffer buf: fragment f of the tile goes to wave f % 4 (TILE_FRAGS / 4 DMA loads each)
-    auto stage = [&](int kt, int buf, int blk) {
-        const int T0 = kt << 5, tb = T0 & 255;
+    // stage a set into buffer buf: fragment f goes to wave f % (4 NH).  A pair's second tile may lie past the context: it is in the
+    // same block, nobody reads it
+    auto stage = [&](int it, int buf, int blk) {
+        const int tb = (it * NH << 5) & 255;
         const _Float16* kb = kbase + (size_t)(blk * kv_l + kh) * kBlockTokens * HD + (size_t)(tb >> 4) * (DC * 512) + lane * 8;
         const _Float16* vb = vbase + (size_t)(blk * kv_l + kh) * kBlockTokens * HD + (size_t)(tb >> 5) * (DT * 512) + lane * 8;
 #pragma unroll
-        for (int i = 0; i < TILE_FRAGS / NWV; ++i) {
-            const int f = wave + i * NWV;
-            const _Float16* src = f < 2 * DC ? kb + f * 512 : vb + (f - 2 * DC) * 512;
-            __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)(lds + (size_t)(buf * TILE_FRAGS + f) * 64), 16, 0, 0);
+        for (int i = 0; i < COPIES; ++i) {
+            const int f = wave + i * 4 * NH, second = f >= TILE_FRAGS, ft = second ? f - TILE_FRAGS : f;
+            const _Float16* src = ft < 2 * DC ? kb + (second * 2 * DC + ft) * 512 : vb + (second * DT + ft - 2 * DC) * 512;
+            lds_dma16(src, lds0 + (uint32_t)(buf * SET + f) * 1024);
         }
     };
-    // ring of three stages: tile kt+2 is issued right after the barrier that opens tile kt, so a tile has two
-    // iterations to land (with one tile ahead the loop ran at the latency of a 16 KiB fetch per iteration)
+    // ring of three stages: set it+2 is issued right after the barrier that opens set it, so a set has two iterations to land
     int blk_a = blk_load(0), blk_b = blk_load(1);
     blk_ready(blk_a);
     blk_ready(blk_b);
     stage(0, 0, blk_a);
-    if (wg_last >= 1) stage(1, 1, blk_b);
+    if (last_set >= 1) stage(1, 1, blk_b);
     int blk_pf = blk_load(2);
     f16x8 qh[QT][DC], ql[QT][DC];
 #pragma unroll
@@ -2260,11 +2268,12 @@ __global__ void __launch_bounds__(256, 2) attn_prefill_kernel(AttnArgs a) {
     float m[QT], lsum[QT];
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
-        m[t] = -1e30f;
+        m[t] = 0.f;
         lsum[t] = 0.f;
 #pragma unroll
         for (int d = 0; d < DT; ++d) o[t][d] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
+    bool fresh = true;  // this wave has seen no tile yet
     NVLLM_STAMP(a, 1);
 #ifdef NVLLM_STAMPS
     if (a.stamps && lane == 0) {  // iteration counts ride in two stamp slots
@@ -2273,102 +2282,142 @@ __global__ void __launch_bounds__(256, 2) attn_prefill_kernel(AttnArgs a) {
     }
 #endif
     int buf = 0;
-    for (int kt = 0; kt <= wg_last; ++kt, buf = buf == 2 ? 0 : buf + 1) {
-        // every wave waits for its own copies of tile kt (all but the TILE_FRAGS / NWV newest: those are tile kt+1),
-        // then the barrier publishes them and says the stage read in iteration kt-1 is free.  Raw barrier: a
-        // __syncthreads() here drains vmcnt(0) and with it the tile that is meant to stay in flight.
-        if (kt + 1 <= wg_last) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(TILE_FRAGS / NWV) : "memory");
+    for (int it = 0; it <= last_set; ++it, buf = buf == 2 ? 0 : buf + 1) {
+        // every wave waits for its own copies of set it (all but the COPIES newest: those are set it+1),
+        // then the barrier publishes them and says the stage read in iteration it-1 is free.  Raw barrier: a
+        // __syncthreads() here drains vmcnt(0) and with it the set that is meant to stay in flight.
+        if (it + 1 <= last_set) asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(COPIES) : "memory");
         else asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
         blk_ready(blk_pf);
-        if (kt + 2 <= wg_last) stage(kt + 2, buf == 0 ? 2 : buf - 1, blk_pf);
-        blk_pf = blk_load(kt + 3);
+        if (it + 2 <= last_set) stage(it + 2, buf == 0 ? 2 : buf - 1, blk_pf);
+        blk_pf = blk_load(it + 3);
+        const int kt = NH * it + part;
         if (kt > my_last) continue;                 // causal: this wave's rows end before this tile (it still stages)
+        const uint4* tile_lds = lds + (size_t)(buf * NH + part) * TILE_FRAGS * 64 + lane;
         const int T0 = kt << 5;
         const int tokA = T0 + grp * 4, tokB = T0 + 16 + grp * 4;
-        // fragment-outer loops: a K (V) fragment is read from LDS, used for both sub-tiles and dropped, instead of the
-        // whole 16 KiB tile sitting in 64 registers (the difference between one and two waves per SIMD)
+        // All K fragments of the tile are asked for before its first MFMA, all V fragments before the softmax, which hides them: left to
+        // the compiler, two fragments at a time were asked for and waited for, eight LDS round trips a tile.
+        uint4 fr[2 * DC];
+#pragma unroll
+        for (int c = 0; c < DC; ++c) { fr[2 * c] = tile_lds[c * 64]; fr[2 * c + 1] = tile_lds[(DC + c) * 64]; }
+        __builtin_amdgcn_sched_barrier(0);
         f32x4 sa[QT], sb[QT];
 #pragma unroll
-        for (int t = 0; t < QT; ++t) { sa[t] = f32x4{0.f, 0.f, 0.f, 0.f}; sb[t] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+        for (int t = 0; t < QT; ++t) { sa[t] = f32x4{-m[t], -m[t], -m[t], -m[t]}; sb[t] = sa[t]; }  // scores come out less the reference
 #pragma unroll
         for (int c = 0; c < DC; ++c) {
-            const f16x8 fa = __builtin_bit_cast(f16x8, lds[(size_t)(buf * TILE_FRAGS + c) * 64 + lane]);
-            const f16x8 fb = __builtin_bit_cast(f16x8, lds[(size_t)(buf * TILE_FRAGS + DC + c) * 64 + lane]);
+            const f16x8 fa = __builtin_bit_cast(f16x8, fr[2 * c]), fb = __builtin_bit_cast(f16x8, fr[2 * c + 1]);
 #pragma unroll
             for (int t = 0; t < QT; ++t) {
                 sa[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa, qh[t][c], sa[t], 0, 0, 0);
-                sa[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa, ql[t][c], sa[t], 0, 0, 0);
                 sb[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb, qh[t][c], sb[t], 0, 0, 0);
+            }
+#pragma unroll
+            for (int t = 0; t < QT; ++t) {
+                sa[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa, ql[t][c], sa[t], 0, 0, 0);
                 sb[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb, ql[t][c], sb[t], 0, 0, 0);
             }
         }
-        // Online softmax, written for the VALU: this block, not the MFMAs, set the kernel's time (30 of 45 us per launch
-        // as first written).  Raw v_exp_f32 (arguments are <= 0, a flushed denormal is 0 either way; exp2f() costs a
-        // compare, a select and an ldexp on top), v_max3 without the NaN canonicalisation fmaxf() pays per operand,
-        // the causal mask only on tiles that reach past the wave's first row, and no rescale of O when no row's
-        // maximum moved.
+        uint4 fv[DT];
+#pragma unroll
+        for (int d = 0; d < DT; ++d) fv[d] = tile_lds[(2 * DC + d) * 64];
+        __builtin_amdgcn_sched_barrier(0);
+        // Online softmax, written for the VALU: this block, not the MFMAs, sets the wave's time.  m is a reference near the row's maximum,
+        // not the maximum: it moves only when a score exceeds it by more than kSlack (p stays below 2^kSlack, well inside f16, and
+        // p / sum p does not depend on the reference), so the usual tile needs no maximum across lanes, no rescale of O and, the
+        // reference being the accumulators' start, no subtraction.  Every row that has a visible token has one in its wave's first tile,
+        // where the reference is set.  Raw v_exp_f32 (a flushed denormal is 0 either way), v_max3 without the NaN canonicalisation
+        // fmaxf() pays per operand, the causal mask only on tiles that reach past the wave's first row.
+        constexpr float kSlack = 8.f;
         f16x8 P[QT], Pl[QT];  // P as f16 hi + lo (see attn_paged_kernel): the prompt's own K/V-dependent rows keep 22 bits too
-        float alpha[QT];
-        auto softmax = [&](auto masked_c) {
-            constexpr bool MASKED = decltype(masked_c)::value;
+        if (T0 + 31 > first_pos) {
+#pragma unroll
+            for (int t = 0; t < QT; ++t)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    sa[t][r] = tokA + r <= my_pos[t] ? sa[t][r] : -1e30f;
+                    sb[t][r] = tokB + r <= my_pos[t] ? sb[t][r] : -1e30f;
+                }
+        }
+        float mt[QT];
+        bool moves = fresh;
+#pragma unroll
+        for (int t = 0; t < QT; ++t) {
+            mt[t] = max3_raw(sa[t][0], sa[t][1], sa[t][2]);
+            mt[t] = max3_raw(mt[t], sa[t][3], sb[t][0]);
+            mt[t] = max3_raw(mt[t], sb[t][1], sb[t][2]);
+            mt[t] = max3_raw(mt[t], sb[t][3], mt[t]);
+            moves = moves || mt[t] > kSlack;
+        }
+        if (__builtin_amdgcn_ballot_w64(moves) != 0) {
 #pragma unroll
             for (int t = 0; t < QT; ++t) {
-                float va[4], vb[4];
+                float up = max3_raw(mt[t], __shfl_xor(mt[t], 16), mt[t]);
+                up = max3_raw(up, __shfl_xor(up, 32), up);      // the row's maximum, the same in its four lanes
+                if (!fresh) up = fmaxf(up, 0.f);
+                else if (up <= -1e29f) up = 0.f;                // no visible token (and none to come)
+                const float alpha = __builtin_amdgcn_exp2f(-up);  // fresh: what it scales is 0
+                m[t] += up;
+                lsum[t] = fresh ? 0.f : lsum[t] * alpha;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    va[r] = (!MASKED || tokA + r <= my_pos[t]) ? sa[t][r] : -1e30f;
-                    vb[r] = (!MASKED || tokB + r <= my_pos[t]) ? sb[t][r] : -1e30f;
-                }
-                float mt = max3_raw(va[0], va[1], va[2]);
-                mt = max3_raw(mt, va[3], vb[0]);
-                mt = max3_raw(mt, vb[1], vb[2]);
-                mt = max3_raw(mt, vb[3], m[t]);                       // the running maximum is the same in the row's four lanes
-                mt = max3_raw(mt, __shfl_xor(mt, 16), mt);
-                const float mn = max3_raw(mt, __shfl_xor(mt, 32), mt);
-                alpha[t] = __builtin_amdgcn_exp2f(m[t] - mn);
-                m[t] = mn;
-                float ps = 0.f;
+                for (int r = 0; r < 4; ++r) { sa[t][r] -= up; sb[t][r] -= up; }
+                if (!fresh)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    float pa = __builtin_amdgcn_exp2f(va[r] - mn), pb = __builtin_amdgcn_exp2f(vb[r] - mn);
-                    if (MASKED) {  // exp2(-1e30 - mn) is 0 already unless mn itself is the -1e30 of a row with no valid token yet
-                        pa = (tokA + r <= my_pos[t]) ? pa : 0.f;
-                        pb = (tokB + r <= my_pos[t]) ? pb : 0.f;
-                    }
-                    ps += pa + pb;
-                    P[t][r] = (_Float16)pa;
-                    P[t][4 + r] = (_Float16)pb;
-                    Pl[t][r] = (_Float16)(pa - (float)P[t][r]);
-                    Pl[t][4 + r] = (_Float16)(pb - (float)P[t][4 + r]);
-                }
-                lsum[t] = lsum[t] * alpha[t] + ps;
+                    for (int d = 0; d < DT; ++d) { o[t][d][0] *= alpha; o[t][d][1] *= alpha; o[t][d][2] *= alpha; o[t][d][3] *= alpha; }
             }
-        };
-        if (T0 + 31 <= first_pos) softmax(std::false_type{});
-        else softmax(std::true_type{});
-        bool moved = false;
+            fresh = false;
+        }
 #pragma unroll
-        for (int t = 0; t < QT; ++t) moved = moved || alpha[t] != 1.0f;
-        if (__builtin_amdgcn_ballot_w64(moved) != 0) {
+        for (int t = 0; t < QT; ++t) {
+            float p[8];
 #pragma unroll
-            for (int d = 0; d < DT; ++d)
-#pragma unroll
-                for (int t = 0; t < QT; ++t) {
-                    o[t][d][0] *= alpha[t]; o[t][d][1] *= alpha[t]; o[t][d][2] *= alpha[t]; o[t][d][3] *= alpha[t];
-                }
+            for (int r = 0; r < 4; ++r) { p[r] = __builtin_amdgcn_exp2f(sa[t][r]); p[4 + r] = __builtin_amdgcn_exp2f(sb[t][r]); }
+            lsum[t] += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+            split_f16x8(p, P[t], Pl[t]);
         }
 #pragma unroll
         for (int d = 0; d < DT; ++d) {
-            const f16x8 fv = __builtin_bit_cast(f16x8, lds[(size_t)(buf * TILE_FRAGS + 2 * DC + d) * 64 + lane]);
 #pragma unroll
-            for (int t = 0; t < QT; ++t) {
-                o[t][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fv, P[t], o[t][d], 0, 0, 0);
-                o[t][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fv, Pl[t], o[t][d], 0, 0, 0);
-            }
+            for (int t = 0; t < QT; ++t) o[t][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, fv[d]), P[t], o[t][d], 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < QT; ++t) o[t][d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, fv[d]), Pl[t], o[t][d], 0, 0, 0);
         }
     }
     NVLLM_STAMP(a, 2);
-    // every wave owns its rows for the whole context: normalise and store (D[dim 4*grp+reg][q row l15] -> out[row][head dims])
+    if constexpr (NH == 2) {
+        // the odd tiles' half of every q-tile to LDS (the ring is free once all waves are here: no copy is in flight), the even ones' takes it
+        asm volatile("s_barrier" ::: "memory");
+        f32x4* obuf = reinterpret_cast<f32x4*>(smem_raw);                               // [4 q-tiles][QT][DT][64]
+        float2* mlbuf = reinterpret_cast<float2*>(obuf + (size_t)NWV * QT * DT * 64);   // [4][QT][64]
+        if (part) {
+#pragma unroll
+            for (int t = 0; t < QT; ++t) {
+                mlbuf[(qw * QT + t) * 64 + lane] = make_float2(m[t], lsum[t]);
+#pragma unroll
+                for (int d = 0; d < DT; ++d) obuf[((qw * QT + t) * DT + d) * 64 + lane] = o[t][d];
+            }
+        }
+        __syncthreads();
+        if (part) return;
+#pragma unroll
+        for (int t = 0; t < QT; ++t) {
+            const float2 other = mlbuf[(qw * QT + t) * 64 + lane];
+            float l1 = other.y;  // of the row: a half without a visible token has no reference
+            l1 += __shfl_xor(l1, 16);
+            l1 += __shfl_xor(l1, 32);
+            const float mo = l1 == 0.f ? m[t] : other.x, mn = fmaxf(m[t], mo);
+            const float f0 = __builtin_amdgcn_exp2f(m[t] - mn), f1 = __builtin_amdgcn_exp2f(mo - mn);
+            lsum[t] = lsum[t] * f0 + other.y * f1;
+#pragma unroll
+            for (int d = 0; d < DT; ++d) {
+                const f32x4 v = obuf[((qw * QT + t) * DT + d) * 64 + lane];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[t][d][r] = o[t][d][r] * f0 + v[r] * f1;
+            }
+        }
+    }
+    // normalise and store (D[dim 4*grp+reg][q row l15] -> out[row][head dims])
 #pragma unroll
     for (int t = 0; t < QT; ++t) {
         float l = lsum[t];
@@ -2454,20 +2503,25 @@ static hipError_t attn_launch_t(const AttnArgs& a, int n_tiles, int grid_z, hipS
     return attn_launch_v<HD, QT, NWV, FUSED, 0>(a, n_tiles, grid_z, s);
 }
 
+template <int HD, int NH>
+static hipError_t attn_prefill_launch(const AttnArgs& a, int groups, hipStream_t s) {
+    constexpr size_t ring = (size_t)3 * NH * (2 * (HD / 32) + HD / 16) * 1024, merge = NH == 2 ? (size_t)4 * 2 * 64 * (HD / 16 * 16 + 8) : 0;
+    constexpr size_t lds = ring > merge ? ring : merge;
+    static std::atomic<uint64_t> lds_set{0};
+    ensure_dyn_lds(reinterpret_cast<const void*>(attn_prefill_kernel<HD, 2, NH>), lds, lds_set);
+    attn_prefill_kernel<HD, 2, NH><<<groups * a.kv.kv_l, NH * 256, lds, s>>>(a);
+    return hipGetLastError();
+}
 // prefill: n_tiles (a multiple of 4: every sequence's tile list padded with empty tiles) q-tiles of 2 sub-tiles each
 hipError_t launch_attn_prefill(const AttnArgs& a, int n_tiles, hipStream_t s) {
     if (n_tiles <= 0) return hipSuccess;
     if (a.kv.vlo) return hipErrorNotSupported;  // 24-bit V: the caller runs prompt chunks through attn_paged_kernel<.., 2, ..>
     if (n_tiles % 4 || a.gqa < 1 || a.gqa > 16 || (a.kv.hd != 128 && a.kv.hd != 64)) return hipErrorInvalidValue;
-    dim3 grid((n_tiles / 4) * a.kv.kv_l);
-    if (a.kv.hd == 128) {
-        const size_t lds = (size_t)3 * (2 * 4 + 8) * 1024;
-        attn_prefill_kernel<128, 2><<<grid, 256, lds, s>>>(a);
-    } else {
-        const size_t lds = (size_t)3 * (2 * 2 + 4) * 1024;
-        attn_prefill_kernel<64, 2><<<grid, 256, lds, s>>>(a);
-    }
-    return hipGetLastError();
+    // fewer workgroups than two for every CU: the tiles of a context on two sets of waves (measurements at the kernel)
+    const int groups = n_tiles / 4;
+    const bool two = groups * a.kv.kv_l < 512;
+    if (a.kv.hd == 128) return two ? attn_prefill_launch<128, 2>(a, groups, s) : attn_prefill_launch<128, 1>(a, groups, s);
+    return two ? attn_prefill_launch<64, 2>(a, groups, s) : attn_prefill_launch<64, 1>(a, groups, s);
 }
 
 // rows: number of q rows (needed by the combine pass); n_parts_max: ceil(max context tiles / part_tiles)

@@ -264,3 +264,27 @@ def test_prefill_tile_gemm_equals_the_chunked_kernel(Ly, M, N, K, mode, packed):
     _lib.check(_lib.lib().nvllm_debug_gemm_tile_check(ctx.h, M, N, K, mode, packed, 2, C.byref(d), C.byref(r), C.byref(u0), C.byref(u1)), ctx.h)
     assert r.value > 0
     assert d.value <= 1e-5 * r.value, (d.value, r.value)
+
+
+# Prompt attention: one or two sets of waves per q-tile (the launch has two workgroups for every CU from 512 on), contexts that end in
+# either half of a pair of tiles, fewer tokens than a tile; values whose row maximum climbs by more than the softmax's slack (2^8) late, row
+# by row, or starts far below zero.  K and V are f16 values, q and P 22 bits: what is left is the f32 accumulation of up to 128 products
+# per score, 128 x 2^-24 of scores of order max(1, |climb|), which moves a probability by as much relatively.
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("B,T", [(1, 1), (1, 31), (1, 33), (1, 97), (3, 64), (2, 129), (1, 513), (40, 65), (70, 40)])
+@pytest.mark.parametrize("climb", [0.0, 40.0, -300.0])
+def test_prompt_attention_tiles_and_reference(Ly, oracle, rng, hd, B, T, climb):
+    nh, kv = 16, 8
+    q = rng.standard_normal((B, nh, T, hd)).astype(np.float32)
+    k = rng.standard_normal((B, kv, T, hd)).astype(np.float16).astype(np.float32)
+    v = rng.standard_normal((B, kv, T, hd)).astype(np.float16).astype(np.float32)
+    if climb:  # one direction of q and k adds up to `climb` to the scores, more for later keys
+        q[..., 0], k[..., 0] = hd ** 0.5, np.float16(climb) * (np.arange(T, dtype=np.float32) / T if climb > 0 else 1)
+        k = k.astype(np.float16).astype(np.float32)
+    y = Ly.Attention(nh, hd, hd ** -0.5)(q, k, v)
+    s = np.einsum("bhtd,bhsd->bhts", q.astype(np.float64), np.repeat(k, nh // kv, 1)) * hd ** -0.5
+    s = np.where(np.tril(np.ones((T, T), bool)), s, -np.inf)
+    p = np.exp(s - s.max(-1, keepdims=True))
+    ref = np.einsum("bhts,bhsd->bhtd", p / p.sum(-1, keepdims=True), np.repeat(v, nh // kv, 1))
+    y = y.reshape(B, T, nh, hd).transpose(0, 2, 1, 3)
+    assert np.abs(y - ref).max() < 128 * 2.0 ** -24 * max(1.0, abs(climb)) * np.abs(v).max()
