@@ -1012,6 +1012,10 @@ static bool fused_plan(const nvllm_model* m, int R, FusedPlan& p) {
     const int H = m->H, hd = m->hd, NQ = (m->nh_l + 2 * m->kv_l) * hd, KO = m->nh_l * hd, I2 = 2 * m->I_l;
     const bool tp = m->ctx->tp_size > 1;
     if (R > kFusedMaxRows || m->taps || m->opt_no_fused) return false;
+    // more than kRowMaxRows: only where every projection is the register-direct kernel's (below, slabs and staged forms fall behind the
+    // prompt path's tile products)
+    if (R > kRowMaxRows && !(gemm_rowdir_ok(NQ, H, 2, R) && gemm_rowdir_ok(H, KO, tp ? 2 : 0, R) && gemm_rowdir_ok(I2, H, 1, R) && gemm_rowdir_ok(H, m->I_l, tp ? 2 : 0, R)))
+        return false;
     auto fits = [&](int N, int K, int epi) {
         return m->opt_stream_combine && gemm_stream_ok(R, N, K, epi) && gemm_stream_slab_floats(R, N, K, epi) <= m->slab_floats;
     };
@@ -1237,7 +1241,7 @@ int gemm_slabs(nvllm_model* m, const bf16_bits* xh, const bf16_bits* xl, int ldx
         return NVLLM_OK;
     }
     if (x_packed) return fail(ctx, NVLLM_ESTATE, "packed activation planes reached a non-streaming GEMM");
-    if (R <= kFusedMaxRows && gemm_rowpar_ok(w.N, w.K, 2, R) &&
+    if (R <= kRowMaxRows && gemm_rowpar_ok(w.N, w.K, 2, R) &&
         (size_t)gemm_rowpar_splits(w.N, w.K, 2, R) * R * w.N <= m->slab_floats && !m->opt_no_rowpar) {
         RowParArgs ra;
         ra.xh = xh; ra.xl = xl; ra.ldx = ldx; ra.out = out; ra.M = R;
@@ -1275,7 +1279,7 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
     // operands in fragment order, so the kernel that produces its input planes writes them that way
     const int KO = m->nh_l * hd;
     const int tmin = m->opt_tile_min_wgs;
-    const bool tile_on = !packed && tmin > 0 && R > kFusedMaxRows;
+    const bool tile_on = !packed && tmin > 0 && R > kRowMaxRows;
     // K splits (f32 slabs summed by the consumer): up to 4 on prompt chunks; a few hundred decode rows are MFMA-bound
     // too (hi + lo planes: 4 flops per weight byte and row) and need up to 8 to fill the chip
     const int max_ks = R <= 512 ? 8 : 4;
@@ -1354,12 +1358,12 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
         // MLP (qwen3.rs:323-327)
         if (t_gu) {
             PROF(m, PROF_GEMM, launch_gemm_tile(m->xh, m->xl, w.gu, R, 2, nullptr, m->xh2, m->xl2, t_down ? 1 : 0, tmin, 1, nullptr, s));
-        } else if (!packed && R <= kFusedMaxRows && gemm_rowpar_ok(2 * m->I_l, H, 1, R)) {
+        } else if (!packed && R <= kRowMaxRows && gemm_rowpar_ok(2 * m->I_l, H, 1, R)) {
             // small gate/up: whole-K row-parallel kernel with the SiLU*mul epilogue
             RowParArgs rg;
             rg.xh = m->xh; rg.xl = m->xl; rg.ldx = H; rg.oh = m->xh2; rg.ol = m->xl2; rg.M = R;
             PROF(m, PROF_GEMM, launch_gemm_rowpar(rg, w.gu, 1, s));
-        } else if (packed || (R <= kFusedMaxRows && gemm_rowpar_ok(2 * m->I_l, H, 2, R) &&
+        } else if (packed || (R <= kRowMaxRows && gemm_rowpar_ok(2 * m->I_l, H, 2, R) &&
                               (size_t)gemm_rowpar_splits(2 * m->I_l, H, 2, R) * R * 2 * m->I_l <= m->slab_floats && !m->opt_no_rowpar)) {
             // big gate/up at few rows: stream it with K slices (f32 slabs of the INTERLEAVED gate/up rows),
             // then SiLU*mul on the summed slabs

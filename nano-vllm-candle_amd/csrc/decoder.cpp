@@ -10,13 +10,13 @@ ProductPlan plan_product(const nvllm_model* m, int R, const PackedW& w) {
     const size_t one = (size_t)R * w.N;
     p.max_split = (int)std::max<size_t>(1, std::min<size_t>(8, m->slab_floats / one));
     const int tmin = m->opt_tile_min_wgs;
-    if (tmin > 0 && R > kFusedMaxRows) {
+    if (tmin > 0 && R > kRowMaxRows) {
         const int ks = gemm_tile_splits(R, w.N, w.K, tmin, std::min(p.max_split, R <= 512 ? 8 : 4));
         if (ks > 0) { p.kind = P_TILE; p.packed = 1; p.max_split = std::min(p.max_split, R <= 512 ? 8 : 4); return p; }
     }
     const int ss = gemm_stream_splits(R, w.N, w.K);
     if (ss > 0 && (size_t)ss * one <= m->slab_floats) { p.kind = P_STREAM; p.packed = 1; return p; }
-    if (R <= kFusedMaxRows && gemm_rowpar_ok(w.N, w.K, 2, R) && (size_t)gemm_rowpar_splits(w.N, w.K, 2, R) * one <= m->slab_floats) {
+    if (R <= kRowMaxRows && gemm_rowpar_ok(w.N, w.K, 2, R) && (size_t)gemm_rowpar_splits(w.N, w.K, 2, R) * one <= m->slab_floats) {
         p.kind = P_ROW;
         p.packed = R >= 16 && gemm_rowdir_ok(w.N, w.K, 2, R);
     }
@@ -46,8 +46,8 @@ int run_product(nvllm_model* m, const ProductPlan& p, const bf16_bits* xh, const
 GluPlan plan_glu(const nvllm_model* m, int R, const PackedW& w, bool want_packed_out) {
     GluPlan g;
     const int tmin = m->opt_tile_min_wgs;
-    if (tmin > 0 && R > kFusedMaxRows && gemm_tile_ok(R, w.N, w.K, 2, tmin)) { g.kind = P_TILE; g.packed = 1; g.out_packed_ok = 1; return g; }
-    if (R <= kFusedMaxRows && gemm_rowpar_ok(w.N, w.K, 1, R)) {
+    if (tmin > 0 && R > kRowMaxRows && gemm_tile_ok(R, w.N, w.K, 2, tmin)) { g.kind = P_TILE; g.packed = 1; g.out_packed_ok = 1; return g; }
+    if (R <= kRowMaxRows && gemm_rowpar_ok(w.N, w.K, 1, R)) {
         g.kind = P_ROW;
         const bool dir = gemm_rowdir_ok(w.N, w.K, 1, R);
         g.packed = R >= 16 && dir;

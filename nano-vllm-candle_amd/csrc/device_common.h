@@ -166,6 +166,21 @@ __device__ __forceinline__ float rownorm_rinv_lds(const RowNorm& rn, const float
     const float t = lds_part[r] + lds_part[NR + r] + lds_part[2 * NR + r] + lds_part[3 * NR + r];
     return 1.0f / sqrtf(t * rn.inv_h + rn.eps);
 }
+// the same for the row blocks at m0, m0 + m_step, ... below M (as many as blockDim.x / (4 NR)): [block][4][NR] in LDS
+template <int NR>
+__device__ __forceinline__ void rownorm_partials_blocks(const RowNorm& rn, int m0, int m_step, int M, float* lds_part) {
+    if (!rn.ssq) return;
+    const int idx = (int)threadIdx.x, r = idx % NR, part = (idx / NR) & 3, m = m0 + idx / (4 * NR) * m_step;
+    int row = min(m + r, M - 1);
+    if (rn.row_idx) row = rn.row_idx[row];
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = rn.ssq[(size_t)min(part + 4 * i, rn.groups - 1) * rn.stride + row];
+    float t = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) t += (part + 4 * i) < rn.groups ? v[i] : 0.f;
+    if (m < M) lds_part[idx] = t;
+}
 // one row, one wave: lane g loads group g (groups <= 64)
 __device__ __forceinline__ float rownorm_rinv_wave(const RowNorm& rn, int row, int lane) {
     if (!rn.ssq) return 1.0f;

@@ -99,7 +99,7 @@ void ExpertsScratch::release() {
 // prompt chunks with enough rows per expert: groups of whole blocks of the prompt product
 static int tile_align(const nvllm_model* m, const ExpertsBlock& e, int R) {
     const int rows = R * e.top / e.experts;  // of an expert, on average
-    if (m->opt_tile_min_wgs <= 0 || R <= kFusedMaxRows || rows < (m->opt_tile_min_wgs == 1 ? 1 : 48)) return 0;
+    if (m->opt_tile_min_wgs <= 0 || R <= kRowMaxRows || rows < (m->opt_tile_min_wgs == 1 ? 1 : 48)) return 0;
     for (int align : {rows >= 320 ? 256 : 128, 256})
         if (gemm_tile_group_ok(e.up_rows(), e.Kw, align) && gemm_tile_group_ok(e.ldr, e.ff_p, align)) return align;
     return 0;

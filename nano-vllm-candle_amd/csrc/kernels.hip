@@ -1021,12 +1021,18 @@ __global__ void __launch_bounds__(NWN * NWK * 64) gemm_rowpar_kernel(RowParArgs 
 // go HBM/L2 -> VGPR in one round trip, the K slices meet in LDS once, wave t finishes n-tile t.
 // Measured on MI355X (tools/probe_l2.py, weights L2-warm): every LDS phase of the staged kernel above costs
 // 1.5-2 us of dependent latency; this form has none.  Epilogues as gemm_rowpar_kernel.
+// With more (row block, n-group) pairs than CUs a workgroup keeps its weight fragments and walks row blocks blockIdx.z,
+// + gridDim.z, ...; the next block's rows are on their way while the K slices of the current one meet.  A second round of workgroups
+// would fetch its weights again behind the first one's tail: Qwen3-0.6B layers, 117 rows, two row blocks per workgroup instead of two
+// rounds %M117%; 200 rows %M200%.
 // ---------------------------------------------------------------------------------------------------
-template <int NT, int NWK, int TK, int EPI>
-__global__ void __launch_bounds__(NWK * 64) gemm_rowdir_kernel(RowParArgs a, const uint4* __restrict__ wp, int N, int KT) {
+constexpr int kRowDirBlocks = 4;  // most row blocks of a workgroup
+template <int NT, int NWK, int TK, int EPI, bool LOOP>
+__device__ __forceinline__ void rowdir_body(const RowParArgs& a, const uint4* __restrict__ wp, int N, int KT) {
+    constexpr int UNROLL = LOOP ? 4 : NWK;  // LDS reads at once where the K slices meet: beside the kept weights all of them would spill
     static_assert(NT <= NWK, "wave t finishes n-tile t");
     constexpr int NR = 16;
-    // sred: [NT][16] ssq partials (epilogue 0) or [4][16] rinv partials (epilogue 1)
+    // sred: [NT][16] ssq partials (epilogue 0) or [4][16] rinv partials of every row block (epilogue 1)
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
     f32x4* red = reinterpret_cast<f32x4*>(smem_raw);                                // [NWK][NT][64]
     float* sred = reinterpret_cast<float*>(smem_raw + (size_t)NWK * NT * 1024);     // [NS][16]
@@ -1034,8 +1040,8 @@ __global__ void __launch_bounds__(NWK * 64) gemm_rowdir_kernel(RowParArgs a, con
     const int l15 = lane & 15, grp = lane >> 4;
     const int ntiles = N >> 4;
     const int tile0 = (int)blockIdx.x * NT;
-    const int m0 = blockIdx.z * NR;
-    const int M = a.M;
+    int m0 = blockIdx.z * NR;
+    const int M = a.M, m_step = LOOP ? gridDim.z * NR : 1 << 30;
     const int k0 = wave * TK;
     NVLLM_STAMP(a, 0);
 
@@ -1046,35 +1052,38 @@ __global__ void __launch_bounds__(NWK * 64) gemm_rowdir_kernel(RowParArgs a, con
 #pragma unroll
         for (int j = 0; j < TK; ++j) w[t][j] = wp[((size_t)nt * KT + k0 + j) * 64 + lane];
     }
-    const int xrow = min(m0 + l15, M - 1);
     uint4 xh[TK], xl[TK];
-    {
+    auto load_x = [&](int m) {
         // row-major: 16 rows x 64 B per wave-load; packed: one contiguous 1 KiB fragment (rows >= M of the last
         // block hold stale finite-or-not values whose products are never stored)
-        const size_t xo = a.x_packed ? (((size_t)(m0 >> 4) * KT + k0) << 9) + (size_t)lane * 8
-                                     : (size_t)xrow * a.ldx + (size_t)k0 * 32 + grp * 8;
+        const size_t xo = a.x_packed ? (((size_t)(m >> 4) * KT + k0) << 9) + (size_t)lane * 8
+                                     : (size_t)min(m + l15, M - 1) * a.ldx + (size_t)k0 * 32 + grp * 8;
         const int xs = a.x_packed ? 512 : 32;
 #pragma unroll
         for (int j = 0; j < TK; ++j) {
             xh[j] = *reinterpret_cast<const uint4*>(a.xh + xo + j * xs);
             xl[j] = *reinterpret_cast<const uint4*>(a.xl + xo + j * xs);
         }
-    }
+    };
+    load_x(m0);
     // epilogue operands of the finishing waves (independent of the product): behind the streaming loads
     const int ntile = min(tile0 + wave, ntiles - 1);
     const bool fin = wave < NT && (tile0 + wave) < ntiles;
-    const int row = m0 + l15;
     float4 r4 = make_float4(0.f, 0.f, 0.f, 0.f), nw4 = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto load_resid = [&](int m) { return *reinterpret_cast<const float4*>(a.resid_in + (size_t)min(m + l15, M - 1) * N + (size_t)ntile * 16 + grp * 4); };
     if constexpr (EPI == 0) {
         if (fin) {
             nw4 = *reinterpret_cast<const float4*>(a.next_w + (size_t)ntile * 16 + grp * 4);
-            if (row < M) r4 = *reinterpret_cast<const float4*>(a.resid_in + (size_t)row * N + (size_t)ntile * 16 + grp * 4);
+            r4 = load_resid(m0);
         }
     }
-    if constexpr (EPI == 1) rownorm_partials<NR>(a.rn, m0, M, sred);
+    if constexpr (EPI == 1 && LOOP) rownorm_partials_blocks<NR>(a.rn, m0, m_step, M, sred);
+    if constexpr (EPI == 1 && !LOOP) rownorm_partials<NR>(a.rn, m0, M, sred);
     __builtin_amdgcn_sched_barrier(0);  // every load above is issued before the first use below (one round trip)
     NVLLM_STAMP(a, 1);
 
+    for (;;) {
+    const int row = m0 + l15, m_next = LOOP ? m0 + m_step : M;
     f32x4 acc[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1095,11 +1104,18 @@ __global__ void __launch_bounds__(NWK * 64) gemm_rowdir_kernel(RowParArgs a, con
     NVLLM_STAMP(a, 2);
 #pragma unroll
     for (int t = 0; t < NT; ++t) red[(size_t)(wave * NT + t) * 64 + lane] = acc[t];
+    float4 r4_next = r4;
+    if (m_next < M) {  // the same for the whole workgroup
+        load_x(m_next);
+        if constexpr (EPI == 0)
+            if (fin) r4_next = load_resid(m_next);
+        __builtin_amdgcn_sched_barrier(0);
+    }
     __syncthreads();
     NVLLM_STAMP(a, 3);
     f32x4 sum = {0.f, 0.f, 0.f, 0.f};
     if (wave < NT) {
-#pragma unroll
+#pragma unroll UNROLL
         for (int k = 0; k < NWK; ++k) {
             const f32x4 v = red[(size_t)(k * NT + wave) * 64 + lane];
             sum[0] += v[0]; sum[1] += v[1]; sum[2] += v[2]; sum[3] += v[3];
@@ -1172,13 +1188,27 @@ __global__ void __launch_bounds__(NWK * 64) gemm_rowdir_kernel(RowParArgs a, con
             *reinterpret_cast<float4*>(a.out + (size_t)row * N + (size_t)ntile * 16 + grp * 4) = make_float4(sum[0], sum[1], sum[2], sum[3]);
     }
     NVLLM_STAMP(a, 4);
+    if (m_next >= M) break;
+    __syncthreads();  // red and sred are read
+    m0 = m_next;
+    if constexpr (EPI == 1) sred += 4 * NR;
+    r4 = r4_next;
+    }
+}
+template <int NT, int NWK, int TK, int EPI>
+__global__ void __launch_bounds__(NWK * 64) gemm_rowdir_kernel(RowParArgs a, const uint4* __restrict__ wp, int N, int KT) {
+    rowdir_body<NT, NWK, TK, EPI, false>(a, wp, N, KT);
+}
+template <int NT, int NWK, int TK, int EPI>
+__global__ void __launch_bounds__(NWK * 64) gemm_rowdir_loop_kernel(RowParArgs a, const uint4* __restrict__ wp, int N, int KT) {
+    rowdir_body<NT, NWK, TK, EPI, true>(a, wp, N, KT);
 }
 
 // shape of the register-direct kernel for (N, K, epi, M): nt == 0 -> not applicable
 struct RowDirShape { int nt, nwk, tk; };
 static RowDirShape rowdir_shape(int N, int K, int epi, int M) {
     RowDirShape none{0, 0, 0};
-    if (N % 16 || K % 32 || M > 128) return none;
+    if (N % 16 || K % 32 || M > 256) return none;
     const int KT = K / 32, ntiles = N / 16;
     if (KT % 16 || KT / 16 < 2 || KT / 16 > 8 || (KT / 16) % 2) return none;  // K in {1024, 2048, 3072, 4096}
     const int tk = KT / 16;
@@ -1267,11 +1297,24 @@ int gemm_rowpar_splits(int N, int K, int epi, int M) {
 
 template <int NT, int NWK, int TK, int EPI>
 static hipError_t rowdir_launch_t(const RowParArgs& a, const PackedW& w, hipStream_t s) {
-    const size_t lds = (size_t)NWK * NT * 1024 + (size_t)(NT > 4 ? NT : 4) * 16 * 4;
+    constexpr size_t red = (size_t)NWK * NT * 1024;
+    const int groups = (w.N / 16 + NT - 1) / NT, blocks = (a.M + 15) / 16;
+    // one round of the 256 CUs where a few row blocks per workgroup make it one, and where the 128 registers of a 1024-thread workgroup
+    // hold the weights beside the next block's rows
+    if constexpr (NT * TK + 2 * TK <= (EPI == 1 || EPI == 2 ? 24 : 18)) {
+        if (groups * blocks > 256) {
+            const size_t lds = red + (size_t)std::max(NT, 4 * kRowDirBlocks) * 16 * 4;
+            static std::atomic<uint64_t> lds_set{0};
+            ensure_dyn_lds(reinterpret_cast<const void*>(gemm_rowdir_loop_kernel<NT, NWK, TK, EPI>), lds, lds_set);
+            const int each = std::min(kRowDirBlocks, (groups * blocks + 255) / 256);
+            gemm_rowdir_loop_kernel<NT, NWK, TK, EPI><<<dim3(groups, 1, (blocks + each - 1) / each), NWK * 64, lds, s>>>(a, w.data, w.N, w.K / 32);
+            return hipGetLastError();
+        }
+    }
+    const size_t lds = red + (size_t)(NT > 4 ? NT : 4) * 16 * 4;
     static std::atomic<uint64_t> lds_set{0};
     ensure_dyn_lds(reinterpret_cast<const void*>(gemm_rowdir_kernel<NT, NWK, TK, EPI>), lds, lds_set);
-    dim3 grid((w.N / 16 + NT - 1) / NT, 1, (a.M + 15) / 16);
-    gemm_rowdir_kernel<NT, NWK, TK, EPI><<<grid, NWK * 64, lds, s>>>(a, w.data, w.N, w.K / 32);
+    gemm_rowdir_kernel<NT, NWK, TK, EPI><<<dim3(groups, 1, blocks), NWK * 64, lds, s>>>(a, w.data, w.N, w.K / 32);
     return hipGetLastError();
 }
 template <int EPI>

@@ -76,7 +76,8 @@ static int dmalloc(nvllm_ctx* c, T** p, size_t count) {
     return NVLLM_OK;
 }
 
-constexpr int kFusedMaxRows = 128;  // the fused decode path (deferred norms, row-parallel epilogues) handles up to this many rows
+constexpr int kFusedMaxRows = 256;  // the fused decode path (deferred norms, row-parallel epilogues) handles up to this many rows ...
+constexpr int kRowMaxRows = 128;    // ... and so many where a projection of the layer has no register-direct form; row-parallel products elsewhere
 constexpr int kMaxPending = 4;   // decode steps that may be enqueued before one is collected
 constexpr int kAttnMaxParts = 64;  // split-KV partitions per sequence (partition grows with context beyond 8K)
 
