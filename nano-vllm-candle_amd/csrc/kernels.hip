@@ -1023,8 +1023,8 @@ __global__ void __launch_bounds__(NWN * NWK * 64) gemm_rowpar_kernel(RowParArgs 
 // 1.5-2 us of dependent latency; this form has none.  Epilogues as gemm_rowpar_kernel.
 // With more (row block, n-group) pairs than CUs a workgroup keeps its weight fragments and walks row blocks blockIdx.z,
 // + gridDim.z, ...; the next block's rows are on their way while the K slices of the current one meet.  A second round of workgroups
-// would fetch its weights again behind the first one's tail: Qwen3-0.6B layers, 117 rows, two row blocks per workgroup instead of two
-// rounds %M117%; 200 rows %M200%.
+// would fetch its weights again behind the first one's tail.  Qwen3-0.6B, the four products of a layer: 117 rows 38.6 -> 35.9 us (gate/up
+// 13.1 -> 11.5), 200 rows 83 (chunked kernel) -> 50 us.
 // ---------------------------------------------------------------------------------------------------
 constexpr int kRowDirBlocks = 4;  // most row blocks of a workgroup
 template <int NT, int NWK, int TK, int EPI, bool LOOP>
