@@ -6,6 +6,7 @@ import json
 import os
 import struct
 from dataclasses import dataclass
+from itertools import accumulate
 
 import numpy as np
 
@@ -110,11 +111,16 @@ class CausalLM:
     # ---- the hot path ----
     @staticmethod
     def _step_args(seq_ids, token_lists):
+        """arguments of a step: one array of all tokens, with an address per sequence (an object per sequence and argument is slower
+        than the copy: 187 against 58 us for 64 sequences of 300 tokens, 664 against 151 for 200)"""
         n = len(seq_ids)
-        arrs = [np.ascontiguousarray(t, dtype=np.uint32) for t in token_lists]
         u32p = C.POINTER(C.c_uint32)
-        return (u32p, (C.c_int64 * n)(*[int(s) for s in seq_ids]), (u32p * n)(*[a.ctypes.data_as(u32p) for a in arrs]),
-                (C.c_int32 * n)(*[len(a) for a in arrs]), arrs)
+        arrs = [t if type(t) is np.ndarray and t.dtype == np.uint32 and t.ndim == 1 else np.ascontiguousarray(t, dtype=np.uint32) for t in token_lists]
+        lens = [len(a) for a in arrs]
+        flat = np.concatenate([a if a.ndim == 1 else a.reshape(-1)[:len(a)] for a in arrs] or [np.empty(0, np.uint32)])
+        starts = [flat.ctypes.data] + lens[:-1]
+        ptrs = (C.c_void_p * n)(*accumulate(starts, lambda at, k: at + 4 * k)) if n else (C.c_void_p * 0)()
+        return u32p, (C.c_int64 * n)(*map(int, seq_ids)), C.cast(ptrs, C.POINTER(u32p)), (C.c_int32 * n)(*lens), (flat, ptrs)
 
     def step_score(self, seq_ids, token_lists, is_prefill, wanted):
         """Process the tokens not cached yet (all of them when is_prefill) without sampling; wanted[i]: ascending positions

@@ -176,6 +176,11 @@ struct nvllm_model {
     int cur_n = 0;              // sequences of the step in flight
     int cur_max_len = 0;        // longest of them (tokens, the new ones included)
     size_t slab_floats = 0;
+    static constexpr size_t kOutSlot = 1 << 20;
+    static constexpr int kOutSlots = 16;
+    char* pin_out = nullptr;                  // pinned: up to kOutSlots slots for logits on their way to the caller, then a step's ids
+    int out_slots = 0;
+    hipEvent_t out_ev[kOutSlots] = {};
     Staging stage;
     std::vector<int> table_news;  // entries of h_block_tables the device does not have yet
     float *tap_h = nullptr, *tap_res = nullptr;
