@@ -163,7 +163,10 @@ struct nvllm_model {
     int opt_latent_wgs = 0;      // decode: workgroups the split of the visible context aims at (0: by latent size)
     int64_t latent_expanded = 0; // layer runs served by the expanded form so far
     int opt_latent_plain = 0;    // latent attention: the plain kernel instead of the matrix-core one (A/B, tests)
-    int opt_tile_min_wgs = 192;  // prefill tile GEMM: smallest grid it is used for (256-row tiles need rows to fill 256 CUs)
+    // prompt tile product: smallest grid it is used for.  Its blocks beat the chunked kernel's long before they fill the 256 CUs: prompt of
+    // one sequence on Qwen3-0.6B, smallest grid 192 / 128 / 64: 300 rows 3.97 / 3.93 / 3.43 ms, 512 rows 4.42 / 4.32 / 3.76, 1300 rows
+    // 6.89 / 5.79 / 5.78, 2391 rows 8.65 / 7.65 / 7.65 (800 rows 4.73 / 4.35 / 4.44); four 8B layers, 257 rows 1.74 / 1.65 / 1.65
+    int opt_tile_min_wgs = 64;
     unsigned* tickets = nullptr;             // arrival counters of the streaming GEMM's in-launch combine (zero between launches)
     float* qkv_out = nullptr;                // complete QKV sums of the streaming GEMM (its combine reads the slabs in m->slabs)
     uint32_t* d_next = nullptr;
