@@ -457,18 +457,18 @@ static void free_kv(nvllm_model* m) {
     m->resid = m->slabs = m->qbuf = m->logits = m->d_maxval = m->red = nullptr; m->xh = m->xl = m->xh2 = m->xl2 = m->ctxh = m->ctxl = nullptr; m->ssqA = m->ssqB = nullptr; m->d_next = nullptr; m->part_val = nullptr; m->part_idx = nullptr; m->argmax_scratch = nullptr; m->attn_po = m->attn_pml = nullptr;
     m->tap_h = m->tap_res = nullptr; m->cosv = m->sinv = nullptr; m->tickets = nullptr; m->qkv_out = nullptr; m->d_keys = nullptr; m->d_temps = nullptr;
     stage_release(m);
-    if (m->pin_out) (void)hipHostFree(m->pin_out);
-    for (hipEvent_t& e : m->out_ev) { if (e) (void)hipEventDestroy(e); e = nullptr; }
-    m->pin_out = nullptr;
-    m->out_slots = 0;
     m->num_blocks = 0;
 }
 
 int stage_alloc(nvllm_model* m, size_t ints) {
     Staging& g = m->stage;
     g.ints = (ints + 63) / 64 * 64;
-    HIPCHK(m->ctx, hipHostMalloc((void**)&g.host, g.ints * Staging::kSlots * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent));
+    // one allocation with what leaves a step (a pinned allocation costs more by its number than by its size)
+    const size_t in = g.ints * Staging::kSlots * sizeof(int), most = (size_t)m->max_seqs * m->cfg.vocab_size * 4, C = nvllm_model::kOutSlot;
+    m->out_slots = (int)std::min<size_t>(nvllm_model::kOutSlots, (most + C - 1) / C);
+    HIPCHK(m->ctx, hipHostMalloc((void**)&g.host, in + m->out_slots * C + (size_t)m->max_seqs * 4, hipHostMallocMapped | hipHostMallocCoherent));
     HIPCHK(m->ctx, hipHostGetDevicePointer((void**)&g.dev, g.host, 0));
+    m->pin_out = (char*)g.host + in;
     return NVLLM_OK;
 }
 void stage_release(nvllm_model* m) {
@@ -477,6 +477,9 @@ void stage_release(nvllm_model* m) {
     for (hipEvent_t e : g.ev) if (e) (void)hipEventDestroy(e);
     g = Staging();
     m->table_news.clear();
+    for (hipEvent_t& e : m->out_ev) { if (e) (void)hipEventDestroy(e); e = nullptr; }
+    m->pin_out = nullptr;
+    m->out_slots = 0;
 }
 int stage_begin(nvllm_model* m) {
     Staging& g = m->stage;
@@ -889,12 +892,6 @@ extern "C" int nvllm_kv_alloc(nvllm_model* m, int num_blocks, int block_size, in
     // sequence's last group of four), the head's rows, a pair for every block a step can take; each run padded to four
     const size_t tiles = std::min(4 * R, R + 3 * (size_t)max_seqs);
     if (!rc) rc = stage_alloc(m, 3 * R + 5 * tiles + tiles / 4 + (size_t)max_seqs + 2 * (size_t)num_blocks + (m->dec ? m->dec->plan_ints(m) : 0) + 4 * kStageRuns);
-    if (!rc) {
-        const size_t most = (size_t)max_seqs * m->cfg.vocab_size * 4;
-        m->out_slots = (int)std::min<size_t>(nvllm_model::kOutSlots, (most + nvllm_model::kOutSlot - 1) / nvllm_model::kOutSlot);
-        HIPCHK(ctx, hipHostMalloc((void**)&m->pin_out, (size_t)m->out_slots * nvllm_model::kOutSlot + (size_t)max_seqs * 4, hipHostMallocDefault));
-        for (int i = 0; i < m->out_slots; ++i) HIPCHK(ctx, hipEventCreateWithFlags(&m->out_ev[i], hipEventDisableTiming));
-    }
     if (rc) { m->num_blocks = 0; return rc; }
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     return NVLLM_OK;
@@ -1494,8 +1491,10 @@ static int download_slots(nvllm_model* m, int first, int step, int per, const ch
     hipStream_t s = m->ctx->stream;
     auto slot = [&](int c) { return first * per + c / step % per; };  // this thread's chunks: first, first + step, ...
     auto issue = [&](int c) {
-        const hipError_t e = hipMemcpyAsync(m->pin_out + (size_t)slot(c) * C, src + (size_t)c * C, std::min(C, bytes - (size_t)c * C), hipMemcpyDeviceToHost, s);
-        return e != hipSuccess ? e : hipEventRecord(m->out_ev[slot(c)], s);
+        hipEvent_t& ev = m->out_ev[slot(c)];
+        hipError_t e = ev ? hipSuccess : hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+        if (e == hipSuccess) e = hipMemcpyAsync(m->pin_out + (size_t)slot(c) * C, src + (size_t)c * C, std::min(C, bytes - (size_t)c * C), hipMemcpyDeviceToHost, s);
+        return e != hipSuccess ? e : hipEventRecord(ev, s);
     };
     hipError_t e = hipSetDevice(m->ctx->device);
     for (int c = first, k = 0; c < chunks && k < per && e == hipSuccess; c += step, ++k) e = issue(c);
