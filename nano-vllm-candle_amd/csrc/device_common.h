@@ -369,6 +369,19 @@ typedef __attribute__((address_space(3))) void* lptr_t;
         __builtin_amdgcn_sched_barrier(0);                             \
     } while (0)
 __device__ __forceinline__ uint32_t lds_address(const void* p) { return (uint32_t)(uintptr_t)(lptr_t)p; }
+// N (2 or 4) 16-byte LDS reads `STRIDE` bytes apart from `addr` + `off` (compile time once inlined) on, waited for in the same block
+template <int STRIDE>
+__device__ __forceinline__ void lds_read_fragments(bf16x8 (&x)[2], uint32_t addr, int off) {
+    asm volatile("ds_read_b128 %0, %2 offset:%3\n\tds_read_b128 %1, %2 offset:%4\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(x[0]), "=&v"(x[1]) : "v"(addr), "i"(off), "i"(off + STRIDE) : "memory");
+}
+template <int STRIDE>
+__device__ __forceinline__ void lds_read_fragments(bf16x8 (&x)[4], uint32_t addr, int off) {
+    asm volatile("ds_read_b128 %0, %4 offset:%5\n\tds_read_b128 %1, %4 offset:%6\n\tds_read_b128 %2, %4 offset:%7\n\tds_read_b128 %3, %4 offset:%8\n\t"
+                 "s_waitcnt lgkmcnt(0)"
+                 : "=&v"(x[0]), "=&v"(x[1]), "=&v"(x[2]), "=&v"(x[3])
+                 : "v"(addr), "i"(off), "i"(off + STRIDE), "i"(off + 2 * STRIDE), "i"(off + 3 * STRIDE) : "memory");
+}
 
 // 1 KiB of LDS-DMA that hipcc's wait insertion does not see: `src` per lane, the wave's 1 KiB of LDS at byte address `lds` (uniform).  With
 // the builtin, every ordinary LDS read after it waits for vmcnt(0), which drains the copies meant to stay in flight; with this form

@@ -3,7 +3,7 @@
 // (replaces candle_nn::Linear::forward, src/layers/linear.rs:35-36,72-77,184-198; src/models/qwen3.rs:205,278,324,326).
 //
 // One workgroup of 8 waves per (n-group, K slice): a wave owns NT n-tiles over its slice and keeps two SC-k-tile weight
-// sets in flight (HBM -> VGPR, 1 KiB wave-loads, refilled right after use); all 64 rows of x ride through LDS in
+// sets in flight (HBM -> VGPR, 1 KiB wave-loads, refilled right after use); all rows of x, padded to 32 or 64, ride through LDS in
 // KC-k-tile chunks (LDS-DMA, double buffered).  After the first chunk the barrier waits only for the wave's own x stage
 // (counted vmcnt), so the weight stream is never drained.  K is cut into `ks` slices over blockIdx.y so that about one
 // workgroup lands on every CU.
@@ -25,6 +25,11 @@
 
 namespace nvllm {
 
+// Bound by the weight bytes, whose rate is what is kept in flight (8 to 12 KiB per wave, 64 to 96 KiB per CU).  The x fragments are read by
+// asm that waits for itself: an ordinary LDS read behind the LDS-DMA made the compiler wait for vmcnt(0) at every chunk, stopping the weight
+// stream for a round trip.  MT: row blocks of 16; up to 32 rows two of them, half the LDS reads, matrix instructions and sums of four.
+// Both together, four 8B layers (24 rows): down_proj (100 MB) 29.3 -> 22.9 us, gate/up (200 MB) 46.7 -> 40.0, o_proj 12.5 -> 9.8, q/k/v
+// (50 MB) 15.2 -> 14.0; a step of 24 rows of 256 to 2048 tokens 0.876 -> 0.800 ms, of 64 rows of 64 to 512 0.908 -> 0.882.
 // NTL: weight loads non-temporal.  Every weight byte is read once, by one workgroup, so it need not displace the x planes
 // and slabs other workgroups re-read; measured (interleaved A/B, batch 64): Qwen3-32B 19.1 -> 18.1 ms/step, Qwen3-8B
 // 6.37 -> 6.43 -- it pays on the big matrices, so the host sets it from the matrix size.
@@ -33,9 +38,8 @@ namespace nvllm {
 // workgroups: with 8 waves those shapes land on 200 of the 256 CUs.
 // ABL (diagnostic build only, tools/ablate_stream.py): 1 = no MFMAs and no LDS fragment reads, 2 = no x staging, 3 = no weight
 // loads, 4 = no slab stores -- what is left of the kernel's time says which part bounds it.  0 in every product launch.
-template <int NT, int SC, int KC, int EPI, bool NTL, int NW = 8, int ABL = 0>
+template <int NT, int SC, int KC, int EPI, bool NTL, int NW = 8, int MT = 4, int ABL = 0>
 __global__ void __launch_bounds__(NW * 64) gemm_stream_kernel(StreamArgs a, const uint4* __restrict__ wp, int N, int KT, int kts) {
-    constexpr int MT = 4;
     constexpr int FRAGS = 2 * MT * KC;          // 1 KiB fragments per x chunk: [2 planes][MT][KC]
     constexpr int PER_WAVE = (FRAGS + NW - 1) / NW;  // LDS-DMA loads per wave and chunk (fragment f = wave + i * NW while f < FRAGS)
     static_assert(KC == 8 || KC == 4, "x chunks of 8 or 4 k-tiles");
@@ -94,14 +98,15 @@ __global__ void __launch_bounds__(NW * 64) gemm_stream_kernel(StreamArgs a, cons
                 for (int j = 0; j < SC; ++j) asm volatile("" ::"v"(w[t][j].x), "v"(w[t][j].y), "v"(w[t][j].z), "v"(w[t][j].w));
             return;
         }
+        // The fragments come by asm, each block with its own wait: in front of an ordinary LDS read behind an LDS-DMA the compiler puts a
+        // wait for vmcnt(0), which drained the weight stream at every chunk
+        const uint32_t xa = lds_address(lds) + (uint32_t)(buf * FRAGS * 1024 + lane * 16);
 #pragma unroll
         for (int j = 0; j < SC; ++j)
 #pragma unroll
             for (int plane = 0; plane < 2; ++plane) {
                 bf16x8 bx[MT];
-#pragma unroll
-                for (int b = 0; b < MT; ++b)
-                    bx[b] = __builtin_bit_cast(bf16x8, lds[(size_t)(buf * FRAGS + (plane * MT + b) * KC + k0 + j) * 64 + lane]);
+                lds_read_fragments<KC * 1024>(bx, xa, (plane * MT * KC + k0 + j) * 1024);
 #pragma unroll
                 for (int t = 0; t < NT; ++t) {
                     const bf16x8 wv = __builtin_bit_cast(bf16x8, w[t][j]);
@@ -344,9 +349,9 @@ size_t gemm_stream_slab_floats(int M, int N, int K, int epi) {
 static int g_stream_ablate = 0;
 void stream_gemm_set_ablate(int v) { g_stream_ablate = v; }
 #endif
-template <int NT, int SC, int KC, int EPI, int NW>
-static hipError_t stream_launch_t(const StreamShape& sh, const StreamArgs& a, const PackedW& w, hipStream_t s) {
-    const size_t lds = (size_t)2 * (2 * 4 * KC) * 1024;
+template <int NT, int SC, int KC, int EPI, int NW, int MT>
+static hipError_t stream_launch_m(const StreamShape& sh, const StreamArgs& a, const PackedW& w, hipStream_t s) {
+    const size_t lds = (size_t)2 * (2 * MT * KC) * 1024;
     const int waves = (w.N / 16 + NT - 1) / NT;
     dim3 grid((waves + NW - 1) / NW, sh.ks);
 #ifdef NVLLM_STAMPS
@@ -355,8 +360,8 @@ static hipError_t stream_launch_t(const StreamShape& sh, const StreamArgs& a, co
             static std::atomic<uint64_t> lds_set_ab{0};
 #define NVLLM_AB(V_)                                                                                                             \
     if (g_stream_ablate == V_) {                                                                                                 \
-        ensure_dyn_lds(reinterpret_cast<const void*>(gemm_stream_kernel<NT, SC, KC, EPI, true, NW, V_>), lds, lds_set_ab);       \
-        gemm_stream_kernel<NT, SC, KC, EPI, true, NW, V_><<<grid, NW * 64, lds, s>>>(a, w.data, w.N, w.K / 32, w.K / 32 / sh.ks); \
+        ensure_dyn_lds(reinterpret_cast<const void*>(gemm_stream_kernel<NT, SC, KC, EPI, true, NW, MT, V_>), lds, lds_set_ab);       \
+        gemm_stream_kernel<NT, SC, KC, EPI, true, NW, MT, V_><<<grid, NW * 64, lds, s>>>(a, w.data, w.N, w.K / 32, w.K / 32 / sh.ks); \
         return hipGetLastError();                                                                                                \
     }
             NVLLM_AB(1) NVLLM_AB(2) NVLLM_AB(3) NVLLM_AB(4)
@@ -367,14 +372,18 @@ static hipError_t stream_launch_t(const StreamShape& sh, const StreamArgs& a, co
     constexpr size_t nt_min_bytes = (size_t)80 << 20;  // measured: 32B shards gain from 80 MB up, 8B matrices below lose
     if (w.bytes() >= nt_min_bytes) {  // big matrix: non-temporal weight stream
         static std::atomic<uint64_t> lds_set_nt{0};
-        ensure_dyn_lds(reinterpret_cast<const void*>(gemm_stream_kernel<NT, SC, KC, EPI, true, NW>), lds, lds_set_nt);
-        gemm_stream_kernel<NT, SC, KC, EPI, true, NW><<<grid, NW * 64, lds, s>>>(a, w.data, w.N, w.K / 32, w.K / 32 / sh.ks);
+        ensure_dyn_lds(reinterpret_cast<const void*>(gemm_stream_kernel<NT, SC, KC, EPI, true, NW, MT>), lds, lds_set_nt);
+        gemm_stream_kernel<NT, SC, KC, EPI, true, NW, MT><<<grid, NW * 64, lds, s>>>(a, w.data, w.N, w.K / 32, w.K / 32 / sh.ks);
         return hipGetLastError();
     }
     static std::atomic<uint64_t> lds_set{0};
-    ensure_dyn_lds(reinterpret_cast<const void*>(gemm_stream_kernel<NT, SC, KC, EPI, false, NW>), lds, lds_set);
-    gemm_stream_kernel<NT, SC, KC, EPI, false, NW><<<grid, NW * 64, lds, s>>>(a, w.data, w.N, w.K / 32, w.K / 32 / sh.ks);
+    ensure_dyn_lds(reinterpret_cast<const void*>(gemm_stream_kernel<NT, SC, KC, EPI, false, NW, MT>), lds, lds_set);
+    gemm_stream_kernel<NT, SC, KC, EPI, false, NW, MT><<<grid, NW * 64, lds, s>>>(a, w.data, w.N, w.K / 32, w.K / 32 / sh.ks);
     return hipGetLastError();
+}
+template <int NT, int SC, int KC, int EPI, int NW>
+static hipError_t stream_launch_t(const StreamShape& sh, const StreamArgs& a, const PackedW& w, hipStream_t s) {
+    return a.M <= 32 ? stream_launch_m<NT, SC, KC, EPI, NW, 2>(sh, a, w, s) : stream_launch_m<NT, SC, KC, EPI, NW, 4>(sh, a, w, s);
 }
 template <int EPI>
 static hipError_t stream_dispatch(const StreamShape& sh, const StreamArgs& a, const PackedW& w, hipStream_t s) {
