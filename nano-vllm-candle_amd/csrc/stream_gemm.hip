@@ -19,6 +19,7 @@
 // all slabs in slice order -- deterministic -- and runs the epilogue.  That removes the separate sum / SiLU / norm launch
 // (about 4 us of boundary + start-up each) at the price of one workgroup per n-group reading ks slabs.
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 
 #include "device_common.h"
@@ -305,7 +306,12 @@ __global__ void __launch_bounds__(NW * 64) gemm_stream_kernel(StreamArgs a, cons
     }
 }
 
-// (n-tiles per wave, K slices, x chunk depth): about one 8-wave workgroup per CU, at most one round of the chip
+// (n-tiles per wave, K slices, x chunk depth, waves).  The shape of least cost per output column, in bytes of weights: what is read of them,
+// over the square root of the share of 224 workgroups there are (fewer leave bandwidth unused, one for every CU is the most), plus half of
+// what the slices write and their consumer reads back.  The rule and its two constants fit the best shape, or one within 4 us of a step of
+// 680 to 880, for all four matrices of an 8B layer at 17, 32 and 64 rows (all shapes of 60 to 400 workgroups timed inside the decode step).
+// Taking the most workgroups instead cost, over four layers at 24 and 64 rows, 22 and 40 us in q/k/v (16 slices where 8 or 4 do) and 20 and
+// 22 in gate/up (8 waves x 3 tiles x 4 slices against 13 x 1 x 2).
 struct StreamShape { int nt, ks, kc, nw; };
 static StreamShape stream_shape(int M, int N, int K, int epi, bool any_size) {
     StreamShape none{0, 0, 0, 8};
@@ -314,25 +320,28 @@ static StreamShape stream_shape(int M, int N, int K, int epi, bool any_size) {
     if (epi == 2 && (N / 16) % 2) return none;
     const int KT = K / 32, ntiles = N / 16;
     StreamShape best = none;
-    int best_wgs = 0;
-    for (int nw : {8, 10, 13}) {  // 8 first: a wider workgroup must bring strictly more workgroups to be taken
-        if (nw != 8 && (epi != 0 || M <= 16)) continue;  // only the slab form is instantiated for 10 / 13 waves
-        for (int kc : {8, 4})
-            for (int nt = 4; nt >= 1; --nt) {
-                if (epi == 2 && nt % 2) continue;
-                if (epi != 2 && nt == 4) continue;  // 4 tiles per wave only where SwiGLU needs pairs and 2 leave too many workgroups
-                if (nw == 13 && nt > 2) continue;   // 13 waves: 4 on one SIMD, <= 128 registers
+    float best_cost = INFINITY;
+    for (int nw : {8, 10, 13}) {
+        if (nw != 8 && epi != 0) continue;  // only the slab form is instantiated for 10 / 13 waves
+        for (int nt = 1; nt <= 4; ++nt) {
+            if (epi == 2 && nt % 2) continue;
+            if (epi != 2 && nt == 4) continue;  // 4 tiles per wave only where SwiGLU needs pairs and 2 leave too many workgroups
+            if (nw == 13 && nt > 2) continue;   // 13 waves: 4 on one SIMD, <= 128 registers
+            // of equal ones the first: few tiles per wave; the deeper x chunks (down_proj 862 against 868 us), with 13 waves the shallower
+            // ones (gate/up 843 against 848)
+            for (int kc : {nw == 13 ? 4 : 8, nw == 13 ? 8 : 4})
                 for (int ks = 1; ks <= 16; ++ks) {
                     if (KT % ks || (KT / ks) % kc || KT / ks < 2 * kc) continue;
                     const int ngroups = ((ntiles + nt - 1) / nt + nw - 1) / nw;
                     if (epi == 3 && ngroups > 64) continue;  // deferred-norm consumers sum <= 64 ssq groups
                     const int wgs = ngroups * ks;
-                    // most workgroups within one round of the chip; ties: deep x chunks, then fewer slices (fewer slabs)
-                    if (wgs <= 256 && (wgs > best_wgs || (wgs == best_wgs && nw == best.nw && kc == best.kc && ks < best.ks))) { best_wgs = wgs; best = StreamShape{nt, ks, kc, nw}; }
+                    if (wgs > 256 || wgs < (any_size ? 48 : 128)) continue;  // at most one round of the chip
+                    const float cost = 2.f * K / sqrtf(std::min(1.f, wgs / 224.f)) + 4.f * M * ks;
+                    if (cost < best_cost) { best_cost = cost; best = StreamShape{nt, ks, kc, nw}; }
                 }
-            }
+        }
     }
-    return best_wgs >= (any_size ? 48 : 128) ? best : none;
+    return best;
 }
 int gemm_stream_splits(int M, int N, int K) { return stream_shape(M, N, K, 0, false).ks; }
 bool gemm_stream_ok(int M, int N, int K, int epi) { return stream_shape(M, N, K, epi, true).nt != 0; }
