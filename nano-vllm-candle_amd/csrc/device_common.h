@@ -108,6 +108,15 @@ __device__ __forceinline__ uint4 ld_stream16(const void* p) {
     return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
+// a buffer of `bytes` bytes (uniform): loads at an offset past them return zeros without an access
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00027000);
+}
+// non-temporal, 16 bytes at lane offset + uniform offset
+__device__ __forceinline__ uint4 buffer_stream16(__amdgpu_buffer_rsrc_t r, int offset, int uniform_offset) {
+    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, offset, uniform_offset, 2));
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
@@ -226,14 +235,16 @@ __device__ __forceinline__ size_t vlo_packed_offset(int t_in_block, int d, int h
     const int g = (tt & 15) >> 2, j = ((tt >> 4) << 2) | (tt & 3);
     return ((size_t)(tile * (hd >> 5) + (d >> 5)) * 64 + (g << 4) + (d & 15)) * 16 + (size_t)(((d >> 4) & 1) << 3) + j;
 }
+// the byte that takes an f16 value h of x to 24 bits: the upper half of the remainder's f16, to nearest even
+__device__ __forceinline__ uint8_t residual24(float x, _Float16 h) {
+    const float xc = fminf(fmaxf(x, -65504.f), 65504.f);
+    const uint32_t b = __builtin_bit_cast(uint16_t, (_Float16)(xc - (float)h));
+    return (uint8_t)((b + 0x7Fu + ((b >> 8) & 1u)) >> 8);
+}
 __device__ __forceinline__ void store_v24(_Float16* v, uint8_t* vlo, int t_in_block, int d, int hd, float x) {
     const _Float16 h = f16_sat(x);
     v[v_packed_offset(t_in_block, d, hd)] = h;
-    if (vlo) {
-        const float xc = fminf(fmaxf(x, -65504.f), 65504.f);
-        const uint32_t b = __builtin_bit_cast(uint16_t, (_Float16)(xc - (float)h));
-        vlo[vlo_packed_offset(t_in_block, d, hd)] = (uint8_t)((b + 0x7Fu + ((b >> 8) & 1u)) >> 8);
-    }
+    if (vlo) vlo[vlo_packed_offset(t_in_block, d, hd)] = residual24(x, h);
 }
 
 // 24-bit K (KvLayout::klo): the same residual byte per K element, two QK^T fragments (head-dim chunks c, c+1 of one 16-token
@@ -246,11 +257,7 @@ __device__ __forceinline__ size_t klo_packed_offset(int t_in_block, int d, int h
 __device__ __forceinline__ void store_k24(_Float16* k, uint8_t* klo, int t_in_block, int d, int hd, float x) {
     const _Float16 h = f16_sat(x);
     k[k_packed_offset(t_in_block, d, hd)] = h;
-    if (klo) {
-        const float xc = fminf(fmaxf(x, -65504.f), 65504.f);
-        const uint32_t b = __builtin_bit_cast(uint16_t, (_Float16)(xc - (float)h));
-        klo[klo_packed_offset(t_in_block, d, hd)] = (uint8_t)((b + 0x7Fu + ((b >> 8) & 1u)) >> 8);
-    }
+    if (klo) klo[klo_packed_offset(t_in_block, d, hd)] = residual24(x, h);
 }
 
 // eight consecutive elements summed over the slabs of a split-K product (only the first `left` exist, the others are 0);

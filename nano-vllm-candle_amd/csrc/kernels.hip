@@ -1661,12 +1661,6 @@ hipError_t launch_kv_write_plain(const float* k, const float* v, int rows, const
 // ---------------------------------------------------------------------------------------------------
 // Decode (QT == 1) must keep two waves per SIMD (<= 256 registers): at 229 + 40 the compiler once dropped it to one
 // wave per SIMD on its own and the whole decode step lost 12 %
-// Where the prefetch of a tile PAST the end of a context goes: 16 KiB every workgroup shares (L1/L2-resident).  The decode
-// loop keeps its loads unconditional (a branch around them makes hipcc wait vmcnt(0) per load), and a wave leaves the
-// loop with two such prefetches in flight; pointed at the context's last tile they were 32 KiB of real L2 traffic per
-// wave (64 MB per launch at batch 64 beside 87 MB of K/V) that every wave then waited for at the combine barrier.
-__device__ uint4 g_attn_dummy_tile[1024];
-
 // VLO: 24-bit V (KvLayout::vlo): every V fragment comes with 8 residual bytes per lane (a 512-byte wave-load); shifted into
 // the high byte they ARE the residuals' f16 bit patterns, which a second P.V MFMA adds (the kernel is HBM-bound: V bytes x1.5)
 // gfx950, hipcc of ROCm 7.2: a v_mfma_f32_16x16x32_bf8_bf8 that takes as SrcC the result of a v_mfma_f32_16x16x32_f16 issued
@@ -1688,7 +1682,7 @@ __global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(A
     float* ml = reinterpret_cast<float*>(smem_raw);                          // [NWV][QT][2][16]
     f32x4* obuf = reinterpret_cast<f32x4*>(smem_raw + NWV * QT * 2 * 16 * 4);  // [NWV][QT][DT][64]
 
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l15 = lane & 15, grp = lane >> 4;
     // the tile: the grid's y in a fused step (<= 256 rows), part of x in the others, whose tiles can be more than y takes (65535)
     int tile = FUSED ? blockIdx.y : __builtin_amdgcn_readfirstlane((int)blockIdx.x / a.kv.kv_l);
@@ -1698,9 +1692,12 @@ __global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(A
     // slabs of all heads are 512 KiB in a row), which the memory turns out faster than as many places far apart.  Tiles go longest context
     // first, every other run of 256 workgroups backwards: workgroups i and i + 256 share a CU when two fit, so a long context gets a short
     // neighbour.  With the rows as the fast dimension: 200 rows of 64 to 1024 tokens 105 -> 98.5 us per launch, 24 of 256 to 2048 46 -> 41,
-    // prompts with a 24-bit cache 102 -> 88; 64 rows of 64 to 512, resident all at once, the same 23.6.
-    if (a.tile_order) {
-        const int per = max(1, 256 / a.kv.kv_l), g = __builtin_amdgcn_readfirstlane(tile / per), r = tile - g * per;
+    // prompts with a 24-bit cache 102 -> 88; 64 rows of 64 to 512, resident all at once, the same 23.6.  Up to 128 workgroups, with the
+    // parts of a row beside them, there is nothing to pair and the order's load is one more round trip: 16 rows of 100 to 800 tokens 1.258
+    // ms a step with it, 1.242 without; 24 rows on 8 heads of 256 to 2048 tokens, in two parts, 0.784 with it and 0.792 without.
+    if (a.tile_order && gridDim.x * gridDim.y > 128) {
+        const int per = max(1, 256 / a.kv.kv_l);
+        const int g = __builtin_amdgcn_readfirstlane(tile / per), r = tile - g * per;
         const int n_tiles = FUSED ? gridDim.y : __builtin_amdgcn_readfirstlane((int)gridDim.x / a.kv.kv_l), end = min(n_tiles, (g + 1) * per);
         tile = a.tile_order[g & 1 ? end - 1 - r : tile];
     }
@@ -1717,9 +1714,10 @@ __global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(A
         const int tok = t * tpq + l15 / gqa;
         const bool valid = (l15 < tpq * gqa) && (tok < nrows);
         my_row[t] = valid ? row0 + tok : -1;
-        my_pos[t] = valid ? a.pos[row0 + tok] : -1;
+        if constexpr (!FUSED) my_pos[t] = valid ? a.pos[row0 + tok] : -1;
     }
     const int pmax = a.pos[row0 + nrows - 1];
+    if constexpr (FUSED) my_pos[0] = pmax;  // uniform; what the lanes of no row (q = 0) sum up is never stored
     const int n_kv_tiles = (pmax >> 5) + 1;
     // split-KV (flash-decoding): workgroup blockIdx.z owns 32-token tiles [t_begin, t_end) and leaves an
     // un-normalised partial (m, l, O); every workgroup then has the same short dependent-load chain
@@ -1729,70 +1727,43 @@ __global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(A
     if (t_begin >= n_kv_tiles) return;  // uniform for the whole workgroup
 
     const int* bt = a.block_tables + (size_t)slot * a.max_blocks;
-    const _Float16* kbase = reinterpret_cast<const _Float16*>(a.kv.k);
-    const _Float16* vbase = reinterpret_cast<const _Float16*>(a.kv.v);
-    const uint8_t* vlobase = a.kv.vlo;
-    // one 32-token KV tile (tokens tb..tb+31 of block blk): 2*DC K fragments + DT V fragments, 16 KiB in 1 KiB wave-loads
-    auto load_tile_at = [&](int blk, int tb, uint4 (&ka)[DC], uint4 (&kb2)[DC], uint4 (&vf)[DT], uint4 (&vl)[RL]) {
-        auto ld = [&](const _Float16* p) -> uint4 { return ld_stream16(p); };
-        // packed K: the two 16-token tiles of this 32-token step are 2*DC contiguous 1 KiB fragments
-        const _Float16* kb = kbase + (size_t)(blk * kv_l + kh) * kBlockTokens * HD + (size_t)(tb >> 4) * (DC * 512) + lane * 8;
-#pragma unroll
-        for (int c = 0; c < DC; ++c) {
-            ka[c] = ld(kb + c * 512);
-            kb2[c] = ld(kb + (DC + c) * 512);
-        }
-        const _Float16* vb = vbase + (size_t)(blk * kv_l + kh) * kBlockTokens * HD + (size_t)(tb >> 5) * (DT * 512);
-#pragma unroll
-        for (int d = 0; d < DT; ++d) vf[d] = ld(vb + d * 512 + lane * 8);
-        if constexpr (VLO) {
-            const uint8_t* vlb = vlobase + (size_t)(blk * kv_l + kh) * kBlockTokens * HD + (size_t)(tb >> 5) * (DL * 1024) + lane * 16;
-#pragma unroll
-            for (int d = 0; d < DL; ++d) vl[d] = ld_stream16(vlb + d * 1024);
-        }
-        if constexpr (KLO) {
-            const uint8_t* klb = a.kv.klo + (size_t)(blk * kv_l + kh) * kBlockTokens * HD + (size_t)(tb >> 4) * ((DC / 2) * 1024) + lane * 16;
-#pragma unroll
-            for (int i = 0; i < DC; ++i) vl[DL + i] = ld_stream16(klb + i * 1024);
-        }
-    };
+    // one 32-token KV tile: 2*DC K fragments (the two 16-token tiles are contiguous) + DT V fragments, 16 KiB in 1 KiB wave-loads.  A tile
+    // past the end (kt >= t_end: a wave leaves its loop with up to two such prefetches) is the same instructions over buffers of no bytes:
+    // they return zeros and cost no access.  A branch around the loads instead makes hipcc wait for vmcnt(0) per load.
     auto load_tile = [&](int kt, uint4 (&ka)[DC], uint4 (&kb2)[DC], uint4 (&vf)[DT], uint4 (&vl)[RL]) {
-        const int T0 = kt << 5;
-        load_tile_at(bt[T0 >> 8], T0 & 255, ka, kb2, vf, vl);
-    };
-    // tile kt if it exists (kt < t_end), else the shared dummy tile (same instruction stream, no K/V traffic)
-    // avoid: a tile that must not be touched yet (see the fused prologue): its 32-token neighbour in the block is read instead
-    auto load_tile_or_dummy = [&](int kt, int t_end_, uint4 (&ka)[DC], uint4 (&kb2)[DC], uint4 (&vf)[DT], uint4 (&vl)[RL], int avoid = -1) {
-        const bool real = kt < t_end_;
-        const int T0 = min(kt, t_end_ - 1) << 5;
-        const int blk = bt[T0 >> 8], tb = (T0 & 255) ^ (kt == avoid ? 32 : 0);
-        const _Float16* dummy = reinterpret_cast<const _Float16*>(g_attn_dummy_tile) + lane * 8;
-        const _Float16* kb = real ? kbase + (size_t)(blk * kv_l + kh) * kBlockTokens * HD + (size_t)(tb >> 4) * (DC * 512) + lane * 8 : dummy;
-        const _Float16* vb = real ? vbase + (size_t)(blk * kv_l + kh) * kBlockTokens * HD + (size_t)(tb >> 5) * (DT * 512) + lane * 8 : dummy;
+        const int T0 = min(kt, t_end - 1) << 5;
+        const int slab = bt[T0 >> 8] * kv_l + kh, tb = T0 & 255, bytes = kt < t_end ? kBlockTokens * HD * 2 : 0;
+        const auto rk = buffer_of(reinterpret_cast<const char*>(a.kv.k) + (size_t)slab * (kBlockTokens * HD * 2), bytes);
+        const auto rv = buffer_of(reinterpret_cast<const char*>(a.kv.v) + (size_t)slab * (kBlockTokens * HD * 2), bytes);
+        const int ko = (tb >> 4) * (DC * 1024), vo = (tb >> 5) * (DT * 1024);
 #pragma unroll
         for (int c = 0; c < DC; ++c) {
-            ka[c] = ld_stream16(kb + c * 512);
-            kb2[c] = ld_stream16(kb + (DC + c) * 512);
+            ka[c] = buffer_stream16(rk, lane * 16 + c * 1024, ko);
+            kb2[c] = buffer_stream16(rk, lane * 16 + c * 1024, ko + DC * 1024);
         }
 #pragma unroll
-        for (int d = 0; d < DT; ++d) vf[d] = ld_stream16(vb + d * 512);
+        for (int d = 0; d < DT; ++d) vf[d] = buffer_stream16(rv, lane * 16 + (d % 4) * 1024, vo + d / 4 * 4096);
         if constexpr (VLO) {
-            const uint8_t* vlb = real ? vlobase + (size_t)(blk * kv_l + kh) * kBlockTokens * HD + (size_t)(tb >> 5) * (DL * 1024) + lane * 16
-                                      : reinterpret_cast<const uint8_t*>(g_attn_dummy_tile) + lane * 16;
+            const auto rl = buffer_of(a.kv.vlo + (size_t)slab * (kBlockTokens * HD), bytes / 2);
 #pragma unroll
-            for (int d = 0; d < DL; ++d) vl[d] = ld_stream16(vlb + d * 1024);
+            for (int d = 0; d < DL; ++d) vl[d] = buffer_stream16(rl, lane * 16 + d * 1024, (tb >> 5) * (DL * 1024));
         }
         if constexpr (KLO) {
-            const uint8_t* klb = real ? a.kv.klo + (size_t)(blk * kv_l + kh) * kBlockTokens * HD + (size_t)(tb >> 4) * ((DC / 2) * 1024) + lane * 16
-                                      : reinterpret_cast<const uint8_t*>(g_attn_dummy_tile) + lane * 16;
+            const auto rl = buffer_of(a.kv.klo + (size_t)slab * (kBlockTokens * HD), bytes / 2);
 #pragma unroll
-            for (int i = 0; i < DC; ++i) vl[DL + i] = ld_stream16(klb + i * 1024);
+            for (int i = 0; i < DC; ++i) vl[DL + i] = buffer_stream16(rl, lane * 16 + i * 1024, (tb >> 4) * ((DC / 2) * 1024));
         }
     };
     // decode register sets (QT == 1): two 32-token tiles (32 KiB) of this wave are in flight at any time
     uint4 kaA[DC], kbA[DC], vfA[DT], kaB[DC], kbB[DC], vfB[DT];
     uint4 vlA[RL], vlB[RL];
     f16x8 qh[QT][DC], ql[QT][DC];
+    // fused decode: the new token's K and V, and the residual bytes of both, from the wave whose tile it falls into to that wave's lanes
+    // (over obuf, which nobody writes before every wave is through its tiles)
+    _Float16* new_k = reinterpret_cast<_Float16*>(obuf);
+    _Float16* new_v = new_k + HD;
+    uint8_t *new_kl = reinterpret_cast<uint8_t*>(new_v + HD), *new_vl = new_kl + HD;
+    int new_tile = -1;  // ... the tile, in that wave
     if constexpr (FUSED) {
         // Decode, fused prologue (replaces a separate launch): this workgroup is the only consumer of q heads
         // kh*gqa.. of its row and the only producer of that row's K/V for kv head kh.  The QKV GEMM's split-K
@@ -1803,14 +1774,20 @@ __global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(A
         const int row = row0;
         const int pos = a.pos[row];
         const float* qkv_row = a.qkv + (size_t)row * a.ldqkv;
-        const bool owner = (pos >> 5) >= t_begin && (pos >> 5) < t_end;  // split-KV: one workgroup writes K/V
+        // the wave whose tile holds the new token makes its K and V, patches them into the tile it has loaded and stores them for later steps:
+        // no wave waits for another one, for a store or with its first tile (split-KV: one workgroup has such a wave).  With wave 0 as the
+        // maker, its stores waited for and a barrier behind them, and with prefetches past the end that read a shared dummy tile: a 0.6B step
+        // of one row of 137 tokens 0.974 ms, now 0.908; 32 rows of 131 to 638 1.435 -> 1.388; 64 of 64 to 512 1.479 -> 1.429; 130 of 64 to
+        // 1024 3.456 -> 3.302; with a 24-bit cache 64 rows 1.995 -> 1.907.
+        const int last = pos >> 5;
+        const bool maker = last >= t_begin && last < t_end && ((last - t_begin) % NWV) == wave;
         // ---- every load of the prologue first, unconditionally (clamped lanes), so they overlap: a branch
         // ---- around a load costs a full vmcnt(0) round trip each on this compiler
         const int ln = min(lane, half - 1);
         const float* pk = qkv_row + (size_t)(a.nh_l + kh) * HD;
         const float* pv = qkv_row + (size_t)(a.nh_l + kv_l + kh) * HD;
         float kx1 = 0.f, kx2 = 0.f, vx1 = 0.f, vx2 = 0.f, knw1 = 0.f, knw2 = 0.f, kc = 0.f, ks = 0.f;
-        if (wave == 0) {  // block-level branch: one wave produces the row's K/V for this kv head
+        if (maker) {
             kx1 = pk[ln]; kx2 = pk[ln + half]; vx1 = pv[ln]; vx2 = pv[ln + half];
             knw1 = a.kn[ln]; knw2 = a.kn[ln + half];
             kc = a.cos[(size_t)pos * half + ln]; ks = a.sin[(size_t)pos * half + ln];
@@ -1835,23 +1812,15 @@ __global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(A
         }
         // deferred input norm of this row: lane g loads group g (groups <= 64), summed below
         const float ssq_g = (a.rn.ssq && lane < a.rn.groups) ? a.rn.ssq[(size_t)lane * a.rn.stride + row] : 0.f;
-        // This wave's first KV tile goes in flight BEHIND the prologue's own loads (vmcnt retires in order, so the
-        // prologue never waits for it) and lands while it computes; a second set would push the kernel to one wave
-        // per SIMD.  The tile that holds the new token's slot must NOT be touched before wave 0 has written it: a fill
-        // of those lines still in flight when the stores pass would leave this CU's L1 with the old bytes, and the
-        // re-read after the barrier would hit them (seen as rare wrong K/V under memory load: several contexts decoding
-        // on one GPU).  Such a wave (contexts of <= 4 tiles only) prefetches the neighbouring 32-token tile of the same
-        // block instead -- valid memory, never used -- and reads its real tile after the barrier.
-        // Wave 0 (the K/V producer) prefetches nothing here: its vmcnt(0) behind the K/V stores would also wait for the
-        // tile (vmcnt retires in order) -- 16 KiB queued behind every other wave's first tile -- and the whole workgroup
-        // waits for wave 0 at the barrier (in-kernel stamps: 7 us to the barrier, 3 us in it).  It loads its first tile
-        // after the barrier instead.
-        if (wave != 0) load_tile_or_dummy(t_begin + wave, t_end, kaA, kbA, vfA, vlA, pos >> 5);
+        // This wave's first KV tile goes in flight BEHIND the prologue's own loads (vmcnt retires in order, so the prologue never waits for
+        // it) and lands while it computes; a second set would push the kernel to one wave per SIMD.  The new token's place in its tile still
+        // holds old bytes, or the new ones if the stores below pass first: the tile is patched before it is used.
+        load_tile(t_begin + wave, kaA, kbA, vfA, vlA);
         const float ri = a.rn.ssq ? 1.0f / sqrtf(wave_sum(ssq_g) * a.rn.inv_h + a.rn.eps) : 1.0f;
         for (int sl0 = 1; sl0 < a.n_slabs; sl0 += 2) {  // split-K slabs of the generic path's QKV GEMM, two per trip
             const size_t so0 = (size_t)sl0 * a.slab_stride, so1 = (size_t)min(sl0 + 1, a.n_slabs - 1) * a.slab_stride;
             const float m1 = sl0 + 1 < a.n_slabs ? 1.f : 0.f;
-            if (wave == 0) {
+            if (maker) {
                 const float a0 = pk[so0 + ln], a1 = pk[so0 + ln + half], a2 = pv[so0 + ln], a3 = pv[so0 + ln + half];
                 const float b0 = pk[so1 + ln], b1 = pk[so1 + ln + half], b2 = pv[so1 + ln], b3 = pv[so1 + ln + half];
                 kx1 += a0; kx2 += a1; vx1 += a2; vx2 += a3;
@@ -1870,29 +1839,6 @@ __global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(A
                 x[c][0] += m1 * q1[c][0].x; x[c][1] += m1 * q1[c][0].y; x[c][2] += m1 * q1[c][0].z; x[c][3] += m1 * q1[c][0].w;
                 x[c][4] += m1 * q1[c][1].x; x[c][5] += m1 * q1[c][1].y; x[c][6] += m1 * q1[c][1].z; x[c][7] += m1 * q1[c][1].w;
             }
-        }
-        // ---- K / V of the new token (wave 0 of the owning workgroup)
-        if (wave == 0) {
-            const bool act = lane < half;
-            kx1 = act ? kx1 * ri : 0.f; kx2 = act ? kx2 * ri : 0.f;
-            const float kss = wave_sum(kx1 * kx1 + kx2 * kx2);
-            const float krinv = 1.0f / sqrtf(kss / (float)HD + a.eps);
-            if (owner && act) {
-                const int blk = bt[pos >> 8];
-                const float n1 = (kx1 * krinv) * knw1, n2 = (kx2 * krinv) * knw2;
-                const size_t vo = (size_t)(blk * kv_l + kh) * kBlockTokens * HD;
-                _Float16* k = reinterpret_cast<_Float16*>(a.kv.k) + vo;
-                uint8_t* klo = KLO ? a.kv.klo + vo : nullptr;
-                store_k24(k, klo, pos & 255, lane, HD, n1 * kc - n2 * ks);
-                store_k24(k, klo, pos & 255, lane + half, HD, n2 * kc + n1 * ks);
-                _Float16* v = reinterpret_cast<_Float16*>(a.kv.v) + vo;
-                uint8_t* vlo = VLO ? a.kv.vlo + vo : nullptr;
-                store_v24(v, vlo, pos & 255, lane, HD, vx1 * ri);
-                store_v24(v, vlo, pos & 255, lane + half, HD, vx2 * ri);
-            }
-            // make the new token visible to the other waves of THIS workgroup (same CU: write-through L1 -> L2)
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
         // ---- q: deferred input norm, RMSNorm over head_dim, RoPE (chunk c pairs with c + DC/2 in the same lane)
         float ss = 0.f;
@@ -1920,9 +1866,37 @@ __global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(A
                 ql[0][c + DC / 2][j] = (_Float16)(y2 - (float)h2);
             }
         }
+        // ---- K / V of the new token
+        if (maker) {
+            new_tile = last;
+            const bool act = lane < half;
+            kx1 = act ? kx1 * ri : 0.f; kx2 = act ? kx2 * ri : 0.f;
+            const float kss = wave_sum(kx1 * kx1 + kx2 * kx2);
+            const float krinv = 1.0f / sqrtf(kss / (float)HD + a.eps);
+            if (act) {
+                const int blk = bt[pos >> 8];
+                const float n1 = (kx1 * krinv) * knw1, n2 = (kx2 * krinv) * knw2;
+                const float y[4] = {n1 * kc - n2 * ks, n2 * kc + n1 * ks, vx1 * ri, vx2 * ri};
+                const size_t vo = (size_t)(blk * kv_l + kh) * kBlockTokens * HD;
+                _Float16* k = reinterpret_cast<_Float16*>(a.kv.k) + vo;
+                uint8_t* klo = KLO ? a.kv.klo + vo : nullptr;
+                _Float16* v = reinterpret_cast<_Float16*>(a.kv.v) + vo;
+                uint8_t* vlo = VLO ? a.kv.vlo + vo : nullptr;
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    const int dim = lane + e * half;
+                    store_k24(k, klo, pos & 255, dim, HD, y[e]);
+                    store_v24(v, vlo, pos & 255, dim, HD, y[2 + e]);
+                    new_k[dim] = f16_sat(y[e]);
+                    new_v[dim] = f16_sat(y[2 + e]);
+                    if constexpr (KLO) new_kl[dim] = residual24(y[e], f16_sat(y[e]));
+                    if constexpr (VLO != 0) new_vl[dim] = residual24(y[2 + e], f16_sat(y[2 + e]));
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        }
         NVLLM_STAMP(a, 1);
-        __syncthreads();  // the new token's K/V (written by wave 0 above) is visible from here on
-        NVLLM_STAMP(a, 2);
+        NVLLM_STAMP(a, 2);  // no barrier in between any more: the loop's segment starts here
     } else {
 #pragma unroll
         for (int t = 0; t < QT; ++t)
@@ -2058,43 +2032,71 @@ __global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(A
             // decode: two named register sets, both in flight; a set is refilled (two tiles ahead) right after it is
             // consumed.  Prefetches are unconditional (tile index clamped): no branch around loads.
             int kt = t_begin + wave;
-            if constexpr (FUSED) {
-                const int last = pmax >> 5;  // the tile wave 0 has just written the new token into
-                if (kt < t_end && kt == last) {
-                    // no line of this tile can be in this CU's L1 (nobody touched it before the barrier); the agent-scope
-                    // acquire (buffer_inv sc1) makes that independent of who else shares the CU.  Rare path: short contexts.
-                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-                    load_tile(kt, kaA, kbA, vfA, vlA);
-                } else if (wave == 0) {
-                    load_tile_or_dummy(kt, t_end, kaA, kbA, vfA, vlA);  // wave 0 skipped the early prefetch
+            if constexpr (!FUSED) load_tile(kt, kaA, kbA, vfA, vlA);  // (the fused prologue has sent for it)
+            if constexpr (!ONE_SET) load_tile(kt + NWV, kaB, kbB, vfB, vlB);
+            // the new token into its place of a tile: K's lanes l15 == token % 16 of the token half, V's lane group and halfword
+            auto patch = [&](uint4 (&ka)[DC], uint4 (&kb2)[DC], uint4 (&vf)[DT], uint4 (&vl)[RL]) {
+                const int tt = pmax & 31, e = (tt >> 4) * 4 + (tt & 3);
+                const bool kl = l15 == (tt & 15);
+                const bool ka_lane = kl && tt < 16, kb_lane = kl && tt >= 16, v_lane = grp == ((tt & 15) >> 2);
+#pragma unroll
+                for (int c = 0; c < DC; ++c) {
+                    const uint4 n = *reinterpret_cast<const uint4*>(new_k + c * 32 + grp * 8);
+                    ka[c].x = ka_lane ? n.x : ka[c].x; ka[c].y = ka_lane ? n.y : ka[c].y; ka[c].z = ka_lane ? n.z : ka[c].z; ka[c].w = ka_lane ? n.w : ka[c].w;
+                    kb2[c].x = kb_lane ? n.x : kb2[c].x; kb2[c].y = kb_lane ? n.y : kb2[c].y; kb2[c].z = kb_lane ? n.z : kb2[c].z; kb2[c].w = kb_lane ? n.w : kb2[c].w;
                 }
-                if constexpr (!ONE_SET) load_tile_or_dummy(kt + NWV, t_end, kaB, kbB, vfB, vlB);
-            } else {
-                load_tile(min(kt, t_end - 1), kaA, kbA, vfA, vlA);
-                if constexpr (!ONE_SET) load_tile(min(kt + NWV, t_end - 1), kaB, kbB, vfB, vlB);
-            }
-            // refills past the end: the shared dummy tile (fused kernel: the one the model runs); the plain-q variant
-            // (fine-seam op, tuning bench) keeps the clamped re-read -- the extra address selects would spill it
-            auto refill = [&](int kt_next, uint4 (&ka)[DC], uint4 (&kb2)[DC], uint4 (&vf)[DT], uint4 (&vl)[RL]) {
-                if constexpr (FUSED) load_tile_or_dummy(kt_next, t_end, ka, kb2, vf, vl);
-                else load_tile(min(kt_next, t_end - 1), ka, kb2, vf, vl);
+                uint32_t mask[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) mask[i] = v_lane && (e >> 1) == i ? ((e & 1) ? 0xffff0000u : 0x0000ffffu) : 0u;
+                const uint16_t* nv = reinterpret_cast<const uint16_t*>(new_v);
+#pragma unroll
+                for (int d = 0; d < DT; ++d) {
+                    const uint32_t n = nv[d * 16 + l15] * 0x10001u;
+                    vf[d].x = (vf[d].x & ~mask[0]) | (n & mask[0]); vf[d].y = (vf[d].y & ~mask[1]) | (n & mask[1]);
+                    vf[d].z = (vf[d].z & ~mask[2]) | (n & mask[2]); vf[d].w = (vf[d].w & ~mask[3]) | (n & mask[3]);
+                }
+                if constexpr (VLO != 0) {
+                    uint32_t m8[2];
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) m8[i] = v_lane && (e >> 2) == i ? 0xffu << ((e & 3) * 8) : 0u;
+#pragma unroll
+                    for (int d = 0; d < DT; ++d) {
+                        const uint32_t n = new_vl[d * 16 + l15] * 0x1010101u;
+                        uint32_t &w0 = (d & 1) ? vl[d >> 1].z : vl[d >> 1].x, &w1 = (d & 1) ? vl[d >> 1].w : vl[d >> 1].y;
+                        w0 = (w0 & ~m8[0]) | (n & m8[0]);
+                        w1 = (w1 & ~m8[1]) | (n & m8[1]);
+                    }
+                }
+                if constexpr (KLO) {
+#pragma unroll
+                    for (int c = 0; c < DC; ++c) {
+                        const uint2 n = *reinterpret_cast<const uint2*>(new_kl + c * 32 + grp * 8);
+                        uint4 &pa = vl[DL + (c >> 1)], &pb = vl[DL + DC / 2 + (c >> 1)];
+                        uint32_t &a0 = (c & 1) ? pa.z : pa.x, &a1 = (c & 1) ? pa.w : pa.y, &b0 = (c & 1) ? pb.z : pb.x, &b1 = (c & 1) ? pb.w : pb.y;
+                        a0 = ka_lane ? n.x : a0; a1 = ka_lane ? n.y : a1;
+                        b0 = kb_lane ? n.x : b0; b1 = kb_lane ? n.y : b1;
+                    }
+                }
             };
             if constexpr (ONE_SET) {
                 // 24-bit cache: one 24 KiB set per wave and two waves per SIMD (a second set needs > 256 registers: half the
                 // workgroups resident, two rounds) -- the other seven waves of the CU cover this wave's round trip
                 while (kt < t_end) {
+                    if (FUSED && kt == new_tile) patch(kaA, kbA, vfA, vlA);
                     compute_tile(kt, kaA, kbA, vfA, vlA);
-                    refill(kt + NWV, kaA, kbA, vfA, vlA);
+                    load_tile(kt + NWV, kaA, kbA, vfA, vlA);
                     kt += NWV;
                 }
             } else {
                 while (kt < t_end) {
+                    if (FUSED && kt == new_tile) patch(kaA, kbA, vfA, vlA);
                     compute_tile(kt, kaA, kbA, vfA, vlA);
-                    refill(kt + 2 * NWV, kaA, kbA, vfA, vlA);
+                    load_tile(kt + 2 * NWV, kaA, kbA, vfA, vlA);
                     kt += NWV;
                     if (kt >= t_end) break;
+                    if (FUSED && kt == new_tile) patch(kaB, kbB, vfB, vlB);
                     compute_tile(kt, kaB, kbB, vfB, vlB);
-                    refill(kt + 2 * NWV, kaB, kbB, vfB, vlB);
+                    load_tile(kt + 2 * NWV, kaB, kbB, vfB, vlB);
                     kt += NWV;
                 }
             }

@@ -1,7 +1,7 @@
 """In-kernel timeline of one decode step of the bench workload (Qwen3-0.6B, 64 sequences, prompts U[64,512] seed 0) from
 the stamped diagnostic build:  make -C nano-vllm-candle_amd/csrc stamps && NVLLM_LIB=libnvllm_amd_stamps.so python
 tools/stamp_timeline.py.   Stamps are s_memrealtime (100 MHz): 0 entry, 1 loads issued (GEMM) / prologue done (attention),
-2 MFMAs done (GEMM) / barrier passed (attention), 3 LDS reduce barrier passed (GEMM) / KV loop done (attention), 4 end.
+2 MFMAs done (GEMM) / the same place (attention), 3 LDS reduce barrier passed (GEMM) / KV loop done (attention), 4 end.
 Read the SHARES, not the length: the stamps cost time themselves."""
 import ctypes as C
 import os
