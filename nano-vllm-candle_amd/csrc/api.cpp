@@ -1191,8 +1191,8 @@ static int forward_chunk_fused(nvllm_model* m, const FusedPlan& fp, int R, int n
         }
         PROF(m, PROF_EMPTY, hipSuccess);  // calibration: an event pair around nothing, at the attention launch's place
         STAMPS(aa, m);
-        if (qt == 2 && !aa.kv.vlo) PROF(m, PROF_ATTN, launch_attn_prefill(aa, n_tiles, s));
-        else PROF(m, PROF_ATTN, launch_attn_paged(aa, n_tiles, qt, R, parts_max, s));
+        if (qt == 2) PROF(m, PROF_ATTN, launch_attn_prefill(aa, n_tiles, s));
+        else PROF(m, PROF_ATTN, launch_attn_paged(aa, n_tiles, R, parts_max, s));
         // o_proj (+ residual + post-attention norm prep; qwen3.rs:278, :393)
         int rc = row_linear(fp.o, w.o, m->ctxh, m->ctxl, KO, w.ln2, m->ssqA, packed);
         if (rc) return rc;
@@ -1349,8 +1349,8 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
             parts_max = m->attn_parts_max;
         }
         STAMPS(aa, m);
-        if (qt == 2 && !aa.kv.vlo) PROF(m, PROF_ATTN, launch_attn_prefill(aa, n_tiles, s));
-        else PROF(m, PROF_ATTN, launch_attn_paged(aa, n_tiles, qt, R, parts_max, s));
+        if (qt == 2) PROF(m, PROF_ATTN, launch_attn_prefill(aa, n_tiles, s));
+        else PROF(m, PROF_ATTN, launch_attn_paged(aa, n_tiles, R, parts_max, s));
         // output projection (qwen3.rs:278) + TP all-reduce
         int o_slabs = 1;
         if (t_o) PROF(m, PROF_GEMM, launch_gemm_tile(m->xh, m->xl, w.o, R, 0, m->slabs, nullptr, nullptr, 0, tmin, max_ks, &o_slabs, s));
@@ -1744,7 +1744,7 @@ static int step_impl(nvllm_model* m, int n_seqs, const int64_t* seq_ids, const u
     for (int i = 0; i < n_seqs; ++i) if (lens[i] - start[i] != 1) all_single = false;
     const int qt = all_single ? 1 : 2;
     const int tpt = m->dec ? m->dec->tile_rows(qt) : attn_tokens_per_tile(m->gqa, qt);
-    const bool tile_groups = qt == 2 && !m->dec && m->vlocache.empty();
+    const bool tile_groups = qt == 2 && !m->dec;
     const int32_t* want_next = score ? score->want_pos : nullptr;
     std::vector<int> head_rows;  // rows the head runs on, in output order: every sequence's last one, or the wanted ones
     for (int i = 0; i < n_seqs; ++i) {
@@ -2476,11 +2476,11 @@ extern "C" int nvllm_debug_attn_bench(nvllm_ctx* ctx, int B, int nh, int kv, int
         parts_max = ((max_len + 31) / 32 + a.part_tiles - 1) / a.part_tiles;
         if (parts_max > kAttnMaxParts) return fail(ctx, NVLLM_EINVAL, "too many parts");
     }
-    for (int i = 0; i < 3; ++i) HIPCHK(ctx, launch_attn_paged(a, B, 1, B, parts_max, s));
+    for (int i = 0; i < 3; ++i) HIPCHK(ctx, launch_attn_paged(a, B, B, parts_max, s));
     HIPCHK(ctx, hipEventRecord(ctx->ev0, s));
     for (int i = 0; i < iters; ++i) {
         a.kv.k = rk[i % nrot]; a.kv.v = rv[i % nrot];
-        HIPCHK(ctx, launch_attn_paged(a, B, 1, B, parts_max, s));
+        HIPCHK(ctx, launch_attn_paged(a, B, B, parts_max, s));
     }
     HIPCHK(ctx, hipEventRecord(ctx->ev1, s));
     HIPCHK(ctx, hipEventSynchronize(ctx->ev1));

@@ -283,8 +283,9 @@ struct AttnArgs {
     unsigned long long* stamps = nullptr;  // diagnostic build only: [workgroup][16 waves][8] s_memrealtime stamps
 #endif
 };
-// qt = q sub-tiles (of 16 MFMA rows) per workgroup: 1 (decode) or 2 (prefill)
-hipError_t launch_attn_paged(const AttnArgs& a, int n_tiles, int qt, int rows, int n_parts_max, hipStream_t s);
+// decode: one row per workgroup and kv head
+hipError_t launch_attn_paged(const AttnArgs& a, int n_tiles, int rows, int n_parts_max, hipStream_t s);
+// qt = q sub-tiles (of 16 MFMA rows) per q-tile: 1 (decode) or 2 (prefill)
 inline int attn_tokens_per_tile(int gqa, int qt) { return (16 / gqa) * qt; }
 // prefill form with LDS-staged K/V shared by four q-tiles (qt = 2) of one sequence: n_tiles is a multiple of 4, tiles
 // 4b..4b+3 belong to one sequence (tile_slot[4b]), a sequence's last group is padded with empty tiles (tile_nrows = 0)

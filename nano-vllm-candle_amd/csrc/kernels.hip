@@ -1647,19 +1647,19 @@ hipError_t launch_kv_write_plain(const float* k, const float* v, int rows, const
 }
 
 // ---------------------------------------------------------------------------------------------------
-// Paged causal GQA attention (prefill q-tiles and decode rows through the same kernel).
+// Paged causal GQA attention of decode rows.
 // Replaces qwen3.rs:236-277: GQA interleaved expand (q head h -> kv head h/(nh/kv)), scores*scale,
 // additive -1e9 mask for j>i (masked terms are exactly 0 after the f32 softmax, so they are skipped),
 // f32 softmax, p.v.  A KV cache is mathematically equivalent to the reference's full recompute (causal).
 //
-// One workgroup = one q-tile (QT sub-tiles of 16 MFMA rows = (16/gqa) tokens x gqa q-heads) x one kv head.
+// One workgroup = one row (its gqa q-heads in the 16 MFMA rows; QT = 1) x one kv head.
 // Its 4 waves take alternate 32-token KV tiles; K and V fragments go straight from HBM to VGPRs:
 //   S^T[token][qrow]  = K[token][:] . q[qrow][:]      A = K frag (16 rows x 64 B per wave-load), B = q (f16 hi+lo)
 //   O^T[dim][qrow]   += V^T[dim][token] . P[token][qrow]   A = V packed frag (1 KiB wave-load), B = P straight
 //                                                          from the S accumulators (no lane movement)
 // Both products keep the q row on lane&15, so the online-softmax state (m, l) is per-lane.
 // ---------------------------------------------------------------------------------------------------
-// Decode (QT == 1) must keep two waves per SIMD (<= 256 registers): at 229 + 40 the compiler once dropped it to one
+// It must keep two waves per SIMD (<= 256 registers): at 229 + 40 the compiler once dropped it to one
 // wave per SIMD on its own and the whole decode step lost 12 %
 // VLO: 24-bit V (KvLayout::vlo): every V fragment comes with 8 residual bytes per lane (a 512-byte wave-load); shifted into
 // the high byte they ARE the residuals' f16 bit patterns, which a second P.V MFMA adds (the kernel is HBM-bound: V bytes x1.5)
@@ -1670,13 +1670,37 @@ hipError_t launch_kv_write_plain(const float* k, const float* v, int rows, const
 // data dependency pins this statement between producer and consumer; 20 wait states cover a 16-pass producer.
 __device__ __forceinline__ void mfma_result_settled(f32x4& acc) { asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(acc)); }
 
+// ... of all accumulators of a wave: each statement waits, for the compiler may put a producer between two of them
+template <int QT, int DT>
+__device__ __forceinline__ void mfma_results_settled(f32x4 (&o)[QT][DT]) {
+#pragma unroll
+    for (int t = 0; t < QT; ++t)
+#pragma unroll
+        for (int d = 0; d < DT; d += 4)
+            asm volatile("s_nop 7\n\ts_nop 7\n\ts_nop 3" : "+v"(o[t][d]), "+v"(o[t][d + 1]), "+v"(o[t][d + 2]), "+v"(o[t][d + 3]));
+}
+// eight f16 as bf8 (the B operand of a residual product; two mantissa bits leave that 2^-12-sized term 12 % accurate)
+__device__ __forceinline__ long bf8x8(const f16x8& x) {
+    int w0 = 0, w1 = 0;
+    w0 = __builtin_amdgcn_cvt_pk_bf8_f32((float)x[0], (float)x[1], w0, false);
+    w0 = __builtin_amdgcn_cvt_pk_bf8_f32((float)x[2], (float)x[3], w0, true);
+    w1 = __builtin_amdgcn_cvt_pk_bf8_f32((float)x[4], (float)x[5], w1, false);
+    w1 = __builtin_amdgcn_cvt_pk_bf8_f32((float)x[6], (float)x[7], w1, true);
+    return (long)(((unsigned long long)(unsigned)w1 << 32) | (unsigned)w0);
+}
+// one of the two 8-byte residual fragments in a lane's 16 bytes
+__device__ __forceinline__ long bf8_half(const uint4& w, int second) {
+    return (long)(second ? ((unsigned long long)w.w << 32) | w.z : ((unsigned long long)w.y << 32) | w.x);
+}
+
 // VLO: 0 = 16-bit cache, 1 = 24-bit V, 2 = 24-bit K and V (KvLayout::klo too: four more 1 KiB wave-loads per tile, one bf8 MFMA
 // per QK^T fragment against q in bf8)
 template <int HD, int QT, int NWV, bool FUSED, int VLO = 0>
-__global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(AttnArgs a) {
+__global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
+    static_assert(QT == 1, "one row of each head: decode (prompts: attn_prefill_kernel)");
     constexpr int DC = HD / 32, DT = HD / 16, DL = VLO ? DT / 2 : 1;  // DL: 1 KiB residual fragments per tile (two PV fragments each)
     constexpr bool KLO = VLO == 2;
-    constexpr bool ONE_SET = VLO != 0 && QT == 1;  // decode with a 24-bit cache: one tile set in flight per wave (see the loop)
+    constexpr bool ONE_SET = VLO != 0;  // decode with a 24-bit cache: one tile set in flight per wave (see the loop)
     constexpr int RL = DL + (KLO ? DC : 0);  // residual registers per tile: V's DL, then K's [token half][DC / 2]
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
     float* ml = reinterpret_cast<float*>(smem_raw);                          // [NWV][QT][2][16]
@@ -1691,8 +1715,8 @@ __global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(A
     // kv heads are the fast part of the grid: the heads of a row start together, and what they read at one time lies side by side (a block's
     // slabs of all heads are 512 KiB in a row), which the memory turns out faster than as many places far apart.  Tiles go longest context
     // first, every other run of 256 workgroups backwards: workgroups i and i + 256 share a CU when two fit, so a long context gets a short
-    // neighbour.  With the rows as the fast dimension: 200 rows of 64 to 1024 tokens 105 -> 98.5 us per launch, 24 of 256 to 2048 46 -> 41,
-    // prompts with a 24-bit cache 102 -> 88; 64 rows of 64 to 512, resident all at once, the same 23.6.  Up to 128 workgroups, with the
+    // neighbour.  With the rows as the fast dimension: 200 rows of 64 to 1024 tokens 105 -> 98.5 us per launch, 24 of 256 to 2048 46 -> 41;
+    // 64 rows of 64 to 512, resident all at once, the same 23.6.  Up to 128 workgroups, with the
     // parts of a row beside them, there is nothing to pair and the order's load is one more round trip: 16 rows of 100 to 800 tokens 1.258
     // ms a step with it, 1.242 without; 24 rows on 8 heads of 256 to 2048 tokens, in two parts, 0.784 with it and 0.792 without.
     if (a.tile_order && gridDim.x * gridDim.y > 128) {
@@ -1754,7 +1778,7 @@ __global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(A
             for (int i = 0; i < DC; ++i) vl[DL + i] = buffer_stream16(rl, lane * 16 + i * 1024, (tb >> 4) * ((DC / 2) * 1024));
         }
     };
-    // decode register sets (QT == 1): two 32-token tiles (32 KiB) of this wave are in flight at any time
+    // register sets: two 32-token tiles (32 KiB) of this wave are in flight at any time
     uint4 kaA[DC], kbA[DC], vfA[DT], kaB[DC], kbB[DC], vfB[DT];
     uint4 vlA[RL], vlB[RL];
     f16x8 qh[QT][DC], ql[QT][DC];
@@ -1769,7 +1793,6 @@ __global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(A
         // kh*gqa.. of its row and the only producer of that row's K/V for kv head kh.  The QKV GEMM's split-K
         // slabs are summed here; q/k get RMSNorm over head_dim then RoPE (qwen3.rs:224-234) exactly as
         // qk_norm_rope_kvwrite_kernel does for prefill.
-        static_assert(QT == 1, "fused prologue is for single-row (decode) tiles");
         constexpr int half = HD / 2;
         const int row = row0;
         const int pos = a.pos[row];
@@ -1924,14 +1947,7 @@ __global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(A
 #pragma unroll
         for (int t = 0; t < QT; ++t)
 #pragma unroll
-            for (int c = 0; c < DC; ++c) {
-                int w0 = 0, w1 = 0;
-                w0 = __builtin_amdgcn_cvt_pk_bf8_f32((float)qh[t][c][0], (float)qh[t][c][1], w0, false);
-                w0 = __builtin_amdgcn_cvt_pk_bf8_f32((float)qh[t][c][2], (float)qh[t][c][3], w0, true);
-                w1 = __builtin_amdgcn_cvt_pk_bf8_f32((float)qh[t][c][4], (float)qh[t][c][5], w1, false);
-                w1 = __builtin_amdgcn_cvt_pk_bf8_f32((float)qh[t][c][6], (float)qh[t][c][7], w1, true);
-                q8[t][c] = (long)(((unsigned long long)(unsigned)w1 << 32) | (unsigned)w0);
-            }
+            for (int c = 0; c < DC; ++c) q8[t][c] = bf8x8(qh[t][c]);
     }
     f32x4 o[QT][DT];
     float m[QT], lsum[QT];
@@ -1998,14 +2014,7 @@ __global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(A
             }
             lsum[t] = lsum[t] * alpha + ps;
             [[maybe_unused]] long P8 = 0;
-            if constexpr (VLO) {
-                int w0 = 0, w1 = 0;
-                w0 = __builtin_amdgcn_cvt_pk_bf8_f32((float)P[0], (float)P[1], w0, false);
-                w0 = __builtin_amdgcn_cvt_pk_bf8_f32((float)P[2], (float)P[3], w0, true);
-                w1 = __builtin_amdgcn_cvt_pk_bf8_f32((float)P[4], (float)P[5], w1, false);
-                w1 = __builtin_amdgcn_cvt_pk_bf8_f32((float)P[6], (float)P[7], w1, true);
-                P8 = (long)(((unsigned long long)(unsigned)w1 << 32) | (unsigned)w0);
-            }
+            if constexpr (VLO) P8 = bf8x8(P);
 #pragma unroll
             for (int d = 0; d < DT; ++d) {
                 f32x4 acc = o[t][d];
@@ -2026,9 +2035,8 @@ __global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(A
         }
     };
     {
-        // Each wave takes every NWV-th 32-token tile.  Decode runs 16 waves per workgroup (one per
-        // 32 tokens up to 512 of context): a sequence's whole K/V is in flight in one HBM round trip.
-        if constexpr (QT == 1) {
+        // Each wave takes every NWV-th 32-token tile.
+        {
             // decode: two named register sets, both in flight; a set is refilled (two tiles ahead) right after it is
             // consumed.  Prefetches are unconditional (tile index clamped): no branch around loads.
             int kt = t_begin + wave;
@@ -2099,13 +2107,6 @@ __global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(A
                     load_tile(kt + 2 * NWV, kaB, kbB, vfB, vlB);
                     kt += NWV;
                 }
-            }
-        } else {
-            uint4 ka[DC], kb2[DC], vf[DT];
-            uint4 vl[RL];
-            for (int kt = t_begin + wave; kt < t_end; kt += NWV) {
-                load_tile(kt, ka, kb2, vf, vl);
-                compute_tile(kt, ka, kb2, vf, vl);
             }
         }
     }
@@ -2200,12 +2201,16 @@ __global__ void __launch_bounds__(NWV * 64, QT == 1 ? 2 : 1) attn_paged_kernel(A
 // a launch that does not fill the chip twice over.  Measured per launch (16 / 8 heads of 128) with a maximum across lanes, a rescale and
 // a drained ring in every tile, NH = 1: one prompt of 2391 tokens 109 us, now 65; 18.7 k tokens in prompts of 64 to 512, chunks of 4096
 // rows, 34.5 -> 30.7; 32 / 8 heads, 4050 tokens in prompts of 700 to 2000, 152 -> 118.  Both prompts with the other NH: 80, 42 (before
-// the other changes).
+// the other changes).  VLO: a 24-bit cache (see attn_paged_kernel), whose residual fragments ride in the same ring: 5.4 k tokens in prompts
+// of 48 to 400, 88 us with K and V straight to registers for every q-tile of its own, now 39 and, with NH = 2, 30.
 // ---------------------------------------------------------------------------------------------------
-template <int HD, int QT, int NH>
+template <int HD, int QT, int NH, int VLO>
 __global__ void __launch_bounds__(NH * 256, 2) attn_prefill_kernel(AttnArgs a) {
     constexpr int DC = HD / 32, DT = HD / 16, NWV = 4;
-    constexpr int TILE_FRAGS = 2 * DC + DT;  // 1 KiB fragments of one 32-token K/V tile: K lo half, K hi half, V
+    constexpr bool KLO = VLO == 2;
+    constexpr int DL = VLO ? DT / 2 : 0;               // 1 KiB residual fragments of V (two PV fragments each) ...
+    constexpr int V0 = 2 * DC, VL0 = V0 + DT, KL0 = VL0 + DL;  // ... and of K: [token half][DC / 2]
+    constexpr int TILE_FRAGS = KL0 + (KLO ? DC : 0);  // 1 KiB fragments of one 32-token K/V tile: K lo half, K hi half, V, residuals
     constexpr int SET = NH * TILE_FRAGS, COPIES = SET / (4 * NH);  // fragments of NH neighbouring tiles, copies of a wave for them
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
     uint4* lds = reinterpret_cast<uint4*>(smem_raw);  // [3 stages][NH tiles][TILE_FRAGS][64]
@@ -2282,7 +2287,12 @@ __global__ void __launch_bounds__(NH * 256, 2) attn_prefill_kernel(AttnArgs a) {
 #pragma unroll
         for (int i = 0; i < COPIES; ++i) {
             const int f = wave + i * 4 * NH, second = f >= TILE_FRAGS, ft = second ? f - TILE_FRAGS : f;
-            const _Float16* src = ft < 2 * DC ? kb + (second * 2 * DC + ft) * 512 : vb + (second * DT + ft - 2 * DC) * 512;
+            const void* src = ft < V0 ? kb + (second * 2 * DC + ft) * 512 : vb + (second * DT + ft - V0) * 512;
+            if constexpr (VLO != 0) {
+                const size_t slab = (size_t)(blk * kv_l + kh) * kBlockTokens * HD + (size_t)(tb >> 5) * (HD * 32) + lane * 16;
+                if (ft >= KL0) src = a.kv.klo + slab + (second * DC + ft - KL0) * 1024;
+                else if (ft >= VL0) src = a.kv.vlo + slab + (second * DL + ft - VL0) * 1024;
+            }
             lds_dma16(src, lds0 + (uint32_t)(buf * SET + f) * 1024);
         }
     };
@@ -2311,6 +2321,13 @@ __global__ void __launch_bounds__(NH * 256, 2) attn_prefill_kernel(AttnArgs a) {
                 ql[t][c][j] = (_Float16)(x[j] - (float)h);
             }
         }
+    [[maybe_unused]] long q8[QT][DC];  // 24-bit K: q as bf8, against the residual bytes
+    if constexpr (KLO) {
+#pragma unroll
+        for (int t = 0; t < QT; ++t)
+#pragma unroll
+            for (int c = 0; c < DC; ++c) q8[t][c] = bf8x8(qh[t][c]);
+    }
     f32x4 o[QT][DT];
     float m[QT], lsum[QT];
 #pragma unroll
@@ -2348,10 +2365,29 @@ __global__ void __launch_bounds__(NH * 256, 2) attn_prefill_kernel(AttnArgs a) {
         uint4 fr[2 * DC];
 #pragma unroll
         for (int c = 0; c < DC; ++c) { fr[2 * c] = tile_lds[c * 64]; fr[2 * c + 1] = tile_lds[(DC + c) * 64]; }
+        [[maybe_unused]] uint4 frl[KLO ? DC : 1];
+        if constexpr (KLO)
+#pragma unroll
+            for (int c = 0; c < DC; ++c) frl[c] = tile_lds[(KL0 + c) * 64];
         __builtin_amdgcn_sched_barrier(0);
         f32x4 sa[QT], sb[QT];
 #pragma unroll
         for (int t = 0; t < QT; ++t) { sa[t] = f32x4{-m[t], -m[t], -m[t], -m[t]}; sb[t] = sa[t]; }  // scores come out less the reference
+        // Residual bytes are bf8 numbers, operands as they are, and come first: the f16 products wait once for all of them (see
+        // mfma_result_settled)
+        if constexpr (KLO) {
+#pragma unroll
+            for (int c = 0; c < DC; ++c) {
+                const long la = bf8_half(frl[c >> 1], c & 1), lb = bf8_half(frl[DC / 2 + (c >> 1)], c & 1);
+#pragma unroll
+                for (int t = 0; t < QT; ++t) {
+                    sa[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf8_bf8(la, q8[t][c], sa[t], 0, 0, 0);
+                    sb[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf8_bf8(lb, q8[t][c], sb[t], 0, 0, 0);
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < QT; ++t) { mfma_result_settled(sa[t]); mfma_result_settled(sb[t]); }
+        }
 #pragma unroll
         for (int c = 0; c < DC; ++c) {
             const f16x8 fa = __builtin_bit_cast(f16x8, fr[2 * c]), fb = __builtin_bit_cast(f16x8, fr[2 * c + 1]);
@@ -2368,7 +2404,11 @@ __global__ void __launch_bounds__(NH * 256, 2) attn_prefill_kernel(AttnArgs a) {
         }
         uint4 fv[DT];
 #pragma unroll
-        for (int d = 0; d < DT; ++d) fv[d] = tile_lds[(2 * DC + d) * 64];
+        for (int d = 0; d < DT; ++d) fv[d] = tile_lds[(V0 + d) * 64];
+        [[maybe_unused]] uint4 fvl[VLO ? DL : 1];
+        if constexpr (VLO != 0)
+#pragma unroll
+            for (int d = 0; d < DL; ++d) fvl[d] = tile_lds[(VL0 + d) * 64];
         __builtin_amdgcn_sched_barrier(0);
         // Online softmax, written for the VALU: this block, not the MFMAs, sets the wave's time.  m is a reference near the row's maximum,
         // not the maximum: it moves only when a score exceeds it by more than kSlack (p stays below 2^kSlack, well inside f16, and
@@ -2422,6 +2462,16 @@ __global__ void __launch_bounds__(NH * 256, 2) attn_prefill_kernel(AttnArgs a) {
             for (int r = 0; r < 4; ++r) { p[r] = __builtin_amdgcn_exp2f(sa[t][r]); p[4 + r] = __builtin_amdgcn_exp2f(sb[t][r]); }
             lsum[t] += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
             split_f16x8(p, P[t], Pl[t]);
+        }
+        if constexpr (VLO != 0) {
+            long P8[QT];
+#pragma unroll
+            for (int t = 0; t < QT; ++t) P8[t] = bf8x8(P[t]);
+#pragma unroll
+            for (int d = 0; d < DT; ++d)
+#pragma unroll
+                for (int t = 0; t < QT; ++t) o[t][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf8_bf8(bf8_half(fvl[d >> 1], d & 1), P8[t], o[t][d], 0, 0, 0);
+            mfma_results_settled(o);
         }
 #pragma unroll
         for (int d = 0; d < DT; ++d) {
@@ -2550,19 +2600,28 @@ static hipError_t attn_launch_t(const AttnArgs& a, int n_tiles, int grid_z, hipS
     return attn_launch_v<HD, QT, NWV, FUSED, 0>(a, n_tiles, grid_z, s);
 }
 
-template <int HD, int NH>
-static hipError_t attn_prefill_launch(const AttnArgs& a, int groups, hipStream_t s) {
-    constexpr size_t ring = (size_t)3 * NH * (2 * (HD / 32) + HD / 16) * 1024, merge = NH == 2 ? (size_t)4 * 2 * 64 * (HD / 16 * 16 + 8) : 0;
+template <int HD, int NH, int VLO>
+static hipError_t attn_prefill_launch_v(const AttnArgs& a, int groups, hipStream_t s) {
+    constexpr int frags = 2 * (HD / 32) + HD / 16 + (VLO ? HD / 32 : 0) + (VLO == 2 ? HD / 32 : 0);
+    constexpr size_t ring = (size_t)3 * NH * frags * 1024, merge = NH == 2 ? (size_t)4 * 2 * 64 * (HD / 16 * 16 + 8) : 0;
     constexpr size_t lds = ring > merge ? ring : merge;
     static std::atomic<uint64_t> lds_set{0};
-    ensure_dyn_lds(reinterpret_cast<const void*>(attn_prefill_kernel<HD, 2, NH>), lds, lds_set);
-    attn_prefill_kernel<HD, 2, NH><<<groups * a.kv.kv_l, NH * 256, lds, s>>>(a);
+    ensure_dyn_lds(reinterpret_cast<const void*>(attn_prefill_kernel<HD, 2, NH, VLO>), lds, lds_set);
+    attn_prefill_kernel<HD, 2, NH, VLO><<<groups * a.kv.kv_l, NH * 256, lds, s>>>(a);
     return hipGetLastError();
+}
+template <int HD, int NH>
+static hipError_t attn_prefill_launch(const AttnArgs& a, int groups, hipStream_t s) {
+    if constexpr (HD == 128) {  // a 24-bit cache is served for head_dim 128 only; the pool refuses it otherwise
+        if (a.kv.klo) return attn_prefill_launch_v<HD, NH, 2>(a, groups, s);
+        if (a.kv.vlo) return attn_prefill_launch_v<HD, NH, 1>(a, groups, s);
+    } else if (a.kv.vlo) return hipErrorNotSupported;
+    return attn_prefill_launch_v<HD, NH, 0>(a, groups, s);
 }
 // prefill: n_tiles (a multiple of 4: every sequence's tile list padded with empty tiles) q-tiles of 2 sub-tiles each
 hipError_t launch_attn_prefill(const AttnArgs& a, int n_tiles, hipStream_t s) {
     if (n_tiles <= 0) return hipSuccess;
-    if (a.kv.vlo) return hipErrorNotSupported;  // 24-bit V: the caller runs prompt chunks through attn_paged_kernel<.., 2, ..>
+    if (a.kv.klo && !a.kv.vlo) return hipErrorInvalidValue;  // 24-bit K comes with 24-bit V only
     if (n_tiles % 4 || a.gqa < 1 || a.gqa > 16 || (a.kv.hd != 128 && a.kv.hd != 64)) return hipErrorInvalidValue;
     // fewer workgroups than two for every CU: the tiles of a context on two sets of waves (measurements at the kernel)
     const int groups = n_tiles / 4;
@@ -2572,21 +2631,19 @@ hipError_t launch_attn_prefill(const AttnArgs& a, int n_tiles, hipStream_t s) {
 }
 
 // rows: number of q rows (needed by the combine pass); n_parts_max: ceil(max context tiles / part_tiles)
-hipError_t launch_attn_paged(const AttnArgs& a, int n_tiles, int qt, int rows, int n_parts_max, hipStream_t s) {
+hipError_t launch_attn_paged(const AttnArgs& a, int n_tiles, int rows, int n_parts_max, hipStream_t s) {
     if (n_tiles <= 0) return hipSuccess;
     if (a.gqa < 1 || a.gqa > 16) return hipErrorInvalidValue;
     const bool split = a.part_tiles > 0 && n_parts_max > 1;
-    if (split && (qt != 1 || !a.part_o || !a.part_ml || n_parts_max > a.max_parts)) return hipErrorInvalidValue;
+    if (split && (!a.part_o || !a.part_ml || n_parts_max > a.max_parts)) return hipErrorInvalidValue;
     AttnArgs b = a;
     if (!split) b.part_tiles = 0;
     const int gz = split ? n_parts_max : 1;
     hipError_t e = hipErrorInvalidValue;
     const bool fused = a.qkv != nullptr;  // decode rows straight from the QKV GEMM's slabs
-    if (fused && (qt != 1 || n_tiles != rows)) return hipErrorInvalidValue;  // fused decode: tile i is row i
-    if (a.kv.hd == 128 && qt == 1) e = fused ? attn_launch_t<128, 1, 4, true>(b, n_tiles, gz, s) : attn_launch_t<128, 1, 4, false>(b, n_tiles, gz, s);
-    else if (a.kv.hd == 128 && qt == 2) e = attn_launch_t<128, 2, 4, false>(b, n_tiles, gz, s);
-    else if (a.kv.hd == 64 && qt == 1) e = fused ? attn_launch_t<64, 1, 4, true>(b, n_tiles, gz, s) : attn_launch_t<64, 1, 4, false>(b, n_tiles, gz, s);
-    else if (a.kv.hd == 64 && qt == 2) e = attn_launch_t<64, 2, 4, false>(b, n_tiles, gz, s);
+    if (fused && n_tiles != rows) return hipErrorInvalidValue;  // fused decode: tile i is row i
+    if (a.kv.hd == 128) e = fused ? attn_launch_t<128, 1, 4, true>(b, n_tiles, gz, s) : attn_launch_t<128, 1, 4, false>(b, n_tiles, gz, s);
+    else if (a.kv.hd == 64) e = fused ? attn_launch_t<64, 1, 4, true>(b, n_tiles, gz, s) : attn_launch_t<64, 1, 4, false>(b, n_tiles, gz, s);
     if (e != hipSuccess || !split) return e;
     const int items = rows * a.nh_l;
     if (a.kv.hd == 128) attn_combine_kernel<128><<<(items + 3) / 4, 256, 0, s>>>(b, rows);

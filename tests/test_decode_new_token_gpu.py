@@ -23,7 +23,10 @@ def test_steps_equal_the_prompt(hd, bits, rows):
     rng = np.random.default_rng(hd + bits)
     tokens = [rng.integers(0, cfg.vocab_size, k + 3) for k in LENGTHS]
     m.step(list(range(n)), [t[:-3] for t in tokens], True)
-    # the prompt's kernels sum the same products in another order and from keys whose f16 may round the other way: 2^-11 of the largest logit
+    # the prompt's kernels sum the same products in another order and from keys whose f16 may round the other way: 2^-11 of the largest logit.
+    # With 24 bits the residual products keep an eighth of what 2^-12 leaves, in the prompt's kernel as in the decode one: 2^-14
+    bound = 2.0 ** (-11 if bits == 16 else -14)
+    worst = 0.0
     want = {}
     for i in range(n):
         for k in (1, 2, 3):
@@ -35,5 +38,7 @@ def test_steps_equal_the_prompt(hd, bits, rows):
         for k in (1, 2, 3):
             _, got = m.step(g, [tokens[i][:len(tokens[i]) - 3 + k] for i in g], False, want_logits=True)
             for r, i in enumerate(g):
-                assert np.abs(got[r] - want[i, k]).max() < 2.0 ** -11 * np.abs(want[i, k]).max(), (LENGTHS[i], k)
+                worst = max(worst, np.abs(got[r] - want[i, k]).max() / np.abs(want[i, k]).max())
+                assert worst < bound, (LENGTHS[i], k)
+    print(f"[parity] {hd} {bits} {rows}: worst {worst:.3e}, bound {bound:.3e}")
     m.close()
