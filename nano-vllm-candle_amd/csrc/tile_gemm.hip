@@ -28,6 +28,8 @@
 // RoPE), half-split RoPE (rotary_embedding.rs:82-107: features d and d+64 sit in the same lane, accumulators j and j+4),
 // then q (scaled) to the f32 q buffer, K and V as f16 into the paged cache in their fragment orders.  No f32 QKV
 // round trip through HBM and no separate row kernel.
+// MODE 9: the same into a 24-bit cache, the residual bytes beside the f16 values: 4096 rows of a 0.6B layer, the f32 product 60 us and the row
+// kernel 31, now 75 in one.
 #include <algorithm>
 #include <cmath>
 
@@ -70,6 +72,7 @@ int tile_gemm_stamps_count() { return g_tile_stamp_launch; }
 template <int NTW, int WN, int MODE>
 __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
     constexpr bool GROUPS = MODE == 5 || MODE == 6 || MODE == 7, GATHER = MODE == 5 || MODE == 7;
+    constexpr bool QKV = MODE == 3 || MODE == 9, LO = MODE == 9;  // LO: a 24-bit cache
     constexpr int WM = 8 / WN;             // waves along the rows, 4 row tiles (64 rows) each
     constexpr int XT = WM * 4;             // row tiles per workgroup
     constexpr int FRW = WN * NTW;          // 1 KiB fragments per stage: W ...
@@ -111,7 +114,7 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
     // land under the K loop; in the epilogue they were 8 us of latency chain per workgroup (stamps)
     [[maybe_unused]] int e_pos[4], e_blk[4], e_slot0 = 0;
     [[maybe_unused]] bool e_one_seq = true;  // this lane's four tokens belong to one sequence
-    if constexpr (MODE == 3) {
+    if constexpr (QKV) {
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
             const int rowc = min(mb * (WM * 64) + wm * 64 + b * 16 + l15, a.M - 1);
@@ -144,7 +147,7 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
         if (f < FRW) {
             // MODE 3: the block's two heads are nb and NB + nb, not neighbours: a V head (whose epilogue is scattered
             // 2-byte cache stores) then always shares its workgroup with a q head, and the V tail spreads over twice the CUs
-            const int ntile = MODE == 3 ? (f < NTW ? nb : a.NB + nb) * NTW + f % NTW : nb * FRW + f;
+            const int ntile = QKV ? (f < NTW ? nb : a.NB + nb) * NTW + f % NTW : nb * FRW + f;
             src[i] = wbase + ((size_t)ntile * a.KT + kt0) * 64;
         } else {
             const int g = f - FRW, plane = g / XT, mt = min(mb * XT + (g % XT), mtiles - 1);
@@ -273,8 +276,8 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
                 }
             }
         }
-    } else if constexpr (MODE == 3) {
-        static_assert(MODE != 3 || (NTW == 8 && WN == 2), "one wave tile = one 128-wide head");
+    } else if constexpr (QKV) {
+        static_assert(!QKV || (NTW == 8 && WN == 2), "one wave tile = one 128-wide head");
         const QkvArgs& q = a.q;
         const int hh = wn == 0 ? nb : a.NB + nb;  // this wave's head: [q heads | k heads | v heads]
         const int nh = q.nh_l, kvl = q.kv.kv_l;
@@ -294,6 +297,7 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
             if (nvalid > 0 && __builtin_amdgcn_ballot_w64(!okl) == 0) {
                 constexpr int LDV = 72;  // halves per feature row: 64 tokens + 3 shift, padded to a multiple of 4
                 _Float16* vt = reinterpret_cast<_Float16*>(smem_raw) + (size_t)wm * (128 * LDV);
+                [[maybe_unused]] uint8_t* vtl = reinterpret_cast<uint8_t*>(smem_raw) + (size_t)WM * (128 * LDV) * 2 + (size_t)wm * (128 * LDV);  // residual bytes
                 const int sh = P0 & 3;
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
@@ -301,7 +305,12 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
 #pragma unroll
                     for (int j = 0; j < 8; ++j)
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) vt[(j * 16 + grp * 4 + r) * LDV + b * 16 + l15 + sh] = f16_sat(acc[j][b][r] * ri);
+                        for (int r = 0; r < 4; ++r) {
+                            const float y = acc[j][b][r] * ri;
+                            const int at = (j * 16 + grp * 4 + r) * LDV + b * 16 + l15 + sh;
+                            vt[at] = f16_sat(y);
+                            if constexpr (LO) vtl[at] = residual24(y, f16_sat(y));
+                        }
                 }
                 const int blkA = __builtin_amdgcn_readfirstlane(e_blk[0]);                       // block of position P0
                 const int blkB = __builtin_amdgcn_readlane(e_blk[(nvalid - 1) >> 4], (nvalid - 1) & 15);  // ... of the last valid token
@@ -312,6 +321,7 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
                     const int p = P0 + tfirst;       // multiple of 4
                     const int blk = (p >> 8) == (P0 >> 8) ? blkA : blkB;
                     _Float16* vdst = reinterpret_cast<_Float16*>(q.kv.v) + (size_t)(blk * kvl + kvh) * kBlockTokens * 128;
+                    [[maybe_unused]] uint8_t* vldst = LO ? q.kv.vlo + (size_t)(blk * kvl + kvh) * kBlockTokens * 128 : nullptr;
                     const int tib = p & 255, tile32 = tib >> 5, tt = tib & 31;
                     const bool full = tfirst >= 0 && tfirst + 3 < nvalid;
 #pragma unroll
@@ -319,6 +329,15 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
                         const int d = lane * 2 + e;
                         const uint2 w = *reinterpret_cast<const uint2*>(vt + d * LDV + 4 * cq);
                         const size_t off = ((size_t)(tile32 * 8 + (d >> 4)) * 64 + ((tt & 15) >> 2) * 16 + (d & 15)) * 8 + (tt >> 4) * 4;
+                        if constexpr (LO) {
+                            const uint32_t wl = *reinterpret_cast<const uint32_t*>(vtl + d * LDV + 4 * cq);
+                            uint8_t* to = vldst + vlo_packed_offset(tib, d, 128);  // the word's four bytes are neighbours there too
+                            if (full) *reinterpret_cast<uint32_t*>(to) = wl;
+                            else
+#pragma unroll
+                                for (int i = 0; i < 4; ++i)
+                                    if (tfirst + i >= 0 && tfirst + i < nvalid) to[i] = (uint8_t)(wl >> (8 * i));
+                        }
                         if (full) {
                             *reinterpret_cast<uint2*>(vdst + off) = w;
                         } else {
@@ -385,6 +404,18 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
                             const f16x4 v = {f16_sat(acc[j][b][0]), f16_sat(acc[j][b][1]), f16_sat(acc[j][b][2]), f16_sat(acc[j][b][3])};
                             *reinterpret_cast<f16x4*>(k + k_packed_offset(pos & 255, j * 16 + grp * 4, 128)) = v;
                         }
+                        if constexpr (LO) {
+                            if (q.kv.klo) {  // four neighbouring bytes as well
+                                uint8_t* kl = q.kv.klo + (size_t)(e_blk[b] * kvl + (hh - nh)) * kBlockTokens * 128;
+#pragma unroll
+                                for (int j = 0; j < 8; ++j) {
+                                    uint32_t w4 = 0;
+#pragma unroll
+                                    for (int r = 0; r < 4; ++r) w4 |= (uint32_t)residual24(acc[j][b][r], f16_sat(acc[j][b][r])) << (8 * r);
+                                    *reinterpret_cast<uint32_t*>(kl + klo_packed_offset(pos & 255, j * 16 + grp * 4, 128)) = w4;
+                                }
+                            }
+                        }
                     }
                 }
             };
@@ -408,7 +439,9 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
 #pragma unroll
                     for (int j = 0; j < 8; ++j)
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) v[v_packed_offset(pos & 255, j * 16 + grp * 4 + r, 128)] = f16_sat(acc[j][b][r] * ri);
+                        for (int r = 0; r < 4; ++r)
+                            store_v24(v, LO ? q.kv.vlo + (size_t)(e_blk[b] * kvl + (hh - nh - kvl)) * kBlockTokens * 128 : nullptr, pos & 255, j * 16 + grp * 4 + r, 128,
+                                      acc[j][b][r] * ri);
                 }
             }
         }
@@ -559,10 +592,11 @@ hipError_t launch_gemm_tile_qkv(const bf16_bits* xh, const bf16_bits* xl, const 
                                 hipStream_t s) {
     if (!gemm_tile_qkv_ok(M, w.N, w.K, qa.kv.hd, min_wgs) || w.N != (qa.nh_l + 2 * qa.kv.kv_l) * 128) return hipErrorNotSupported;
     if (qa.rn.ssq && qa.rn.groups != 1) return hipErrorNotSupported;
+    if (qa.kv.klo && !qa.kv.vlo) return hipErrorInvalidValue;  // 24-bit K comes with 24-bit V only
     TileArgs a;
     a.xh = reinterpret_cast<const uint4*>(xh); a.xl = reinterpret_cast<const uint4*>(xl); a.wp = w.data;
     a.M = M; a.N = w.N; a.KT = w.K / 32; a.q = qa;
-    return tile_launch_t<8, 2, 3>(a, 1, s);
+    return qa.kv.vlo ? tile_launch_t<8, 2, 9>(a, 1, s) : tile_launch_t<8, 2, 3>(a, 1, s);
 }
 
 // rows of a block, features of a block: 256 x 256, 256 x 192 or 128 x 256 (few rows per group)
