@@ -531,11 +531,14 @@ hipError_t launch_gemm(const GemmPlan& p, const bf16_bits* xh, const bf16_bits* 
 }
 
 // ---------------------------------------------------------------------------------------------------
-// LM head for decode (<= 64 rows): logits = x.W^T (Qwen3ForCausalLM::compute_logits, qwen3.rs:542-550) with
+// LM head for decode: logits = x.W^T (Qwen3ForCausalLM::compute_logits, qwen3.rs:542-550) with
 // the greedy arg-max (llm_engine.rs:135-142, LAST max wins) in the epilogue.  The vocabulary matrix is the
 // largest stream of a step (311 MB for Qwen3-0.6B), read exactly once: one workgroup per CU, 8 waves, each wave
 // owns NT n-tiles for the WHOLE K and keeps two 2-k-tile weight sets (2*NT KiB each) in flight while all 64 rows
 // of x ride through LDS in 8-k-tile chunks (double buffered, every wave stages one k-tile of a chunk).
+// More rows: slices of 64, the workgroups of one group of columns beside each other on an XCD, so that the matrix comes from memory once
+// and from that XCD's L2 for the other slices; bound by the matrix cores from about 100 rows on.  0.6B steps: 65 rows 1.715 -> 1.63 ms,
+// 100 rows 1.919 -> 1.83, 129 rows 2.452 -> 2.24, 200 rows (head 377 -> 160 us) 3.082 -> 2.85, each against the chunked kernel.
 // ---------------------------------------------------------------------------------------------------
 template <int MT, int NT, int NCH>
 __global__ void __launch_bounds__(512) lmhead_kernel(const uint16_t* __restrict__ xh, const uint16_t* __restrict__ xl, int ldx,
@@ -549,14 +552,22 @@ __global__ void __launch_bounds__(512) lmhead_kernel(const uint16_t* __restrict_
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int l15 = lane & 15, grp = lane >> 4;
     const int ntiles = N >> 4;
-    const int nt0 = ((int)blockIdx.x * NW + wave) * NT;
+    const int n_groups = (ntiles + NW * NT - 1) / (NW * NT), slices = (M + MT * 16 - 1) / (MT * 16);
+    int group = blockIdx.x, row0 = 0;
+    if (slices > 1) {  // more than 64 rows
+        const int slot = (int)blockIdx.x >> 3;
+        row0 = (slot % slices) * MT * 16;
+        group = (slot / slices) * 8 + ((int)blockIdx.x & 7);
+        if (group >= n_groups) return;  // whole workgroup, before any barrier
+    }
+    const int nt0 = (group * NW + wave) * NT;
     // deferred-norm partials first, while no other registers are live: 16 independent loads, parked in LDS
-    rownorm_partials<MT * 16>(rn, 0, M, lds_rn);
+    rownorm_partials<MT * 16>(rn, row0, M, lds_rn);
     __builtin_amdgcn_sched_barrier(0);
     unsigned xoff[MT];  // element offset of this lane's 16-byte piece in row block b (k-tile 0), < 2^32 elements
 #pragma unroll
     for (int b = 0; b < MT; ++b) {
-        int r = min(b * 16 + l15, M - 1);
+        int r = min(row0 + b * 16 + l15, M - 1);
         if (rn.row_idx) r = rn.row_idx[r];
         xoff[b] = (unsigned)r * (unsigned)ldx + (unsigned)(wave * 32 + grp * 8);
     }
@@ -591,9 +602,13 @@ __global__ void __launch_bounds__(512) lmhead_kernel(const uint16_t* __restrict_
 #pragma unroll
             for (int plane = 0; plane < 2; ++plane) {  // hi plane, then lo plane: MT x-fragments live at a time
                 bf16x8 bx[MT];
+                if constexpr (MT == 4) {  // by asm that waits for itself, see gemm_stream_kernel (64 rows 1.326 -> 1.314 ms a step; fewer rows lose)
+                    lds_read_fragments<KC * 1024>(bx, lds_address(lds) + (uint32_t)(buf * FRAGS * 1024 + lane * 16), (plane * MT * KC + k0 + j) * 1024);
+                } else {
 #pragma unroll
-                for (int b = 0; b < MT; ++b)
-                    bx[b] = __builtin_bit_cast(bf16x8, lds[(size_t)(buf * FRAGS + (plane * MT + b) * KC + k0 + j) * 64 + lane]);
+                    for (int b = 0; b < MT; ++b)
+                        bx[b] = __builtin_bit_cast(bf16x8, lds[(size_t)(buf * FRAGS + (plane * MT + b) * KC + k0 + j) * 64 + lane]);
+                }
 #pragma unroll
                 for (int a = 0; a < NT; ++a) {
                     const bf16x8 wv = __builtin_bit_cast(bf16x8, w[a][j]);
@@ -660,10 +675,10 @@ __global__ void __launch_bounds__(512) lmhead_kernel(const uint16_t* __restrict_
 #pragma unroll
                 for (int r = 0; r < 4; ++r) acc[a][b][r] = soft_cap(acc[a][b][r], rn.softcap);
     }
-    const int wg = (int)blockIdx.x * NW + wave;
+    const int wg = group * NW + wave;
 #pragma unroll
     for (int b = 0; b < MT; ++b) {
-        const int row = b * 16 + l15;
+        const int row = row0 + b * 16 + l15;
         float bv = -INFINITY;
         int bi = -1;
 #pragma unroll
@@ -684,7 +699,7 @@ __global__ void __launch_bounds__(512) lmhead_kernel(const uint16_t* __restrict_
             if (oi >= 0 && (bi < 0 || ov > bv || (ov == bv && oi > bi))) { bv = ov; bi = oi; }
         }
         if (grp == 0 && row < M) {  // part_*[row][wave]: one workgroup per row finishes (argmax_rows_kernel)
-            const size_t n_parts = (size_t)gridDim.x * NW;
+            const size_t n_parts = (size_t)n_groups * NW;
             part_val[(size_t)row * n_parts + wg] = bv;
             part_idx[(size_t)row * n_parts + wg] = bi;
         }
@@ -744,13 +759,14 @@ static hipError_t lmhead_launch_t(const bf16_bits* xh, const bf16_bits* xl, int 
     static std::atomic<uint64_t> lds_set{0};
     ensure_dyn_lds(reinterpret_cast<const void*>(lmhead_kernel<MT, NT, NCH>), lds, lds_set);
     const int waves = (w.N / 16 + NT - 1) / NT;
-    lmhead_kernel<MT, NT, NCH><<<(waves + 7) / 8, 512, lds, s>>>(xh, xl, ldx, w.data, out, M, w.N, w.K / 32, part_val, part_idx, rn);
+    const int groups = (waves + 7) / 8, slices = (M + MT * 16 - 1) / (MT * 16);
+    lmhead_kernel<MT, NT, NCH><<<slices > 1 ? (groups + 7) / 8 * 8 * slices : groups, 512, lds, s>>>(xh, xl, ldx, w.data, out, M, w.N, w.K / 32, part_val, part_idx, rn);
     return hipGetLastError();
 }
 
 GemmPlan plan_lmhead(int M, int N, int K) {
     GemmPlan p = plan_gemm(M, N, K, 1);
-    if (M > 64 || K % 256 || N % 16) return p;
+    if (K % 256 || N % 16) return p;
     // one workgroup (8 waves) per CU: n-tiles per wave so that the grid fits the 256 CUs in one round
     const int ntiles = N / 16;
     int nt = (ntiles + 2047) / 2048;
@@ -766,7 +782,7 @@ hipError_t launch_gemm_argmax(const GemmPlan& p, const bf16_bits* xh, const bf16
     x.part_val = part_val; x.part_idx = part_idx;
     if (rn) x.rn = *rn;
     if (p.lm_nt > 0) {
-        if (M < 1 || M > 64 || w.K % 256) return hipErrorInvalidValue;
+        if (M < 1 || w.K % 256) return hipErrorInvalidValue;
         const int mt = M <= 16 ? 1 : M <= 32 ? 2 : 4;
 #define NVLLM_LM(MT_, NT_)                                                                                                   \
     if (mt == MT_ && p.lm_nt == NT_)                                                                                       \

@@ -12,8 +12,7 @@ pytestmark = pytest.mark.gpu
 def test_every_row_of_a_decode_batch_is_its_own_answer(kv, heads, rows):
     import nano_vllm_candle_amd as pkg
 
-    cfg = pkg.Qwen3Config.tiny()
-    cfg.num_attention_heads, cfg.num_key_value_heads, cfg.num_hidden_layers = heads, kv, 2
+    cfg = pkg.Qwen3Config.tiny(hidden_size=256, num_attention_heads=heads, num_key_value_heads=kv)  # (256: the head in slices of 64 rows)
     m = pkg.Qwen3ForCausalLM.from_synthetic(cfg, 3)
     m.kv_alloc(rows + 3, rows + 1, 512)
     rng = np.random.default_rng(rows + kv)
