@@ -1147,7 +1147,22 @@ static int forward_chunk_fused(nvllm_model* m, const FusedPlan& fp, int R, int n
         const LayerW& w = m->layers[l];
         QkvArgs qa;
         qa.n_slabs = 1;
-        if (fp.qkv == G_ROW) {
+        qa.slab_stride = (int64_t)R * NQ; qa.qn = w.qn; qa.kn = w.kn; qa.eps = eps;
+        qa.cos = m->cosv; qa.sin = m->sinv; qa.pos = m->d_pos; qa.slot = m->d_slot; qa.block_tables = m->d_block_tables;
+        qa.max_blocks = m->max_blocks; qa.nh_l = m->nh_l;
+        qa.q_scale = powf((float)hd, -0.5f) * 1.4426950408889634f;
+        qa.q_out = m->qbuf; qa.rn = rn;
+        qa.kv.k = m->kcache[l]; qa.kv.v = m->vcache[l]; qa.kv.kv_l = m->kv_l; qa.kv.hd = hd;
+        qa.kv.vlo = m->vlocache.empty() ? nullptr : m->vlocache[l];
+        qa.kv.klo = m->klocache.empty() ? nullptr : m->klocache[l];
+        const bool fuse_qk = qt == 1 && n_tiles == R && !m->opt_no_attn_prologue;
+        const bool qkv_whole = !fuse_qk && fp.qkv == G_ROW && m->opt_tile_fuse_qk && gemm_rowdir_qkv_ok(NQ, H, hd, R);
+        if (qkv_whole) {
+            RowParArgs rq;
+            rq.xh = m->xh; rq.xl = m->xl; rq.ldx = H; rq.M = R; rq.x_packed = packed; rq.rn = rn; rq.q = qa;
+            STAMPS(rq, m);
+            PROF(m, PROF_GEMM, launch_gemm_rowdir_qkv(rq, w.qkv, s));
+        } else if (fp.qkv == G_ROW) {
             RowParArgs rq;
             rq.xh = m->xh; rq.xl = m->xl; rq.ldx = H; rq.out = m->slabs; rq.M = R; rq.x_packed = packed;
             STAMPS(rq, m);
@@ -1163,16 +1178,7 @@ static int forward_chunk_fused(nvllm_model* m, const FusedPlan& fp, int R, int n
             PROF(m, PROF_GEMM, launch_gemm(pq, m->xh, m->xl, H, w.qkv, m->slabs, R, s));
             qa.qkv = m->slabs; qa.n_slabs = pq.n_split;
         }
-        qa.slab_stride = (int64_t)R * NQ; qa.qn = w.qn; qa.kn = w.kn; qa.eps = eps;
-        qa.cos = m->cosv; qa.sin = m->sinv; qa.pos = m->d_pos; qa.slot = m->d_slot; qa.block_tables = m->d_block_tables;
-        qa.max_blocks = m->max_blocks; qa.nh_l = m->nh_l;
-        qa.q_scale = powf((float)hd, -0.5f) * 1.4426950408889634f;
-        qa.q_out = m->qbuf; qa.rn = rn;
-        qa.kv.k = m->kcache[l]; qa.kv.v = m->vcache[l]; qa.kv.kv_l = m->kv_l; qa.kv.hd = hd;
-        qa.kv.vlo = m->vlocache.empty() ? nullptr : m->vlocache[l];
-        qa.kv.klo = m->klocache.empty() ? nullptr : m->klocache[l];
-        const bool fuse_qk = qt == 1 && n_tiles == R && !m->opt_no_attn_prologue;
-        if (!fuse_qk) PROF(m, PROF_QK, launch_qk_norm_rope_kvwrite(qa, R, s));
+        if (!fuse_qk && !qkv_whole) PROF(m, PROF_QK, launch_qk_norm_rope_kvwrite(qa, R, s));
         AttnArgs aa;
         aa.q = m->qbuf; aa.kv = qa.kv; aa.block_tables = m->d_block_tables; aa.max_blocks = m->max_blocks;
         aa.tile_row0 = m->d_tile_row0; aa.tile_nrows = m->d_tile_nrows; aa.tile_slot = m->d_tile_slot; aa.pos = m->d_pos;

@@ -314,10 +314,14 @@ struct RowParArgs {
     RowNorm rn;
     GluSpec glu;                     // epilogue 1
     int x_packed = 0, o_packed = 0;  // xh/xl resp. oh/ol in xpack_off order (register-direct kernel only)
+    QkvArgs q;                       // launch_gemm_rowdir_qkv
 #ifdef NVLLM_STAMPS
     unsigned long long* stamps = nullptr;  // diagnostic build only: [workgroup][16 waves][8] s_memrealtime stamps
 #endif
 };
+// short prompts: the QKV product with q/k norm, rotation and the cache's writes in its epilogue (heads of 128, K = 1024), rn deferred
+bool gemm_rowdir_qkv_ok(int N, int K, int hd, int M);
+hipError_t launch_gemm_rowdir_qkv(const RowParArgs& a, const PackedW& w, hipStream_t s);
 bool gemm_rowpar_supported(int N, int K);
 // true when launch_gemm_rowpar would run the register-direct kernel (the one that accepts packed planes)
 bool gemm_rowdir_ok(int N, int K, int epi, int M);

@@ -538,7 +538,7 @@ hipError_t launch_gemm(const GemmPlan& p, const bf16_bits* xh, const bf16_bits* 
 // of x ride through LDS in 8-k-tile chunks (double buffered, every wave stages one k-tile of a chunk).
 // More rows: slices of 64, the workgroups of one group of columns beside each other on an XCD, so that the matrix comes from memory once
 // and from that XCD's L2 for the other slices; bound by the matrix cores from about 100 rows on.  0.6B steps: 65 rows 1.715 -> 1.63 ms,
-// 100 rows 1.919 -> 1.83, 129 rows 2.452 -> 2.24, 200 rows (head 377 -> 160 us) 3.082 -> 2.85, each against the chunked kernel.
+// 100 rows 1.919 -> 1.83, 129 rows 2.452 -> 2.24, 200 rows (head 377 -> 176 us) 3.082 -> 2.85, each against the chunked kernel.
 // ---------------------------------------------------------------------------------------------------
 template <int MT, int NT, int NCH>
 __global__ void __launch_bounds__(512) lmhead_kernel(const uint16_t* __restrict__ xh, const uint16_t* __restrict__ xl, int ldx,
@@ -1052,6 +1052,7 @@ __device__ __forceinline__ void rowdir_body(const RowParArgs& a, const uint4* __
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
     f32x4* red = reinterpret_cast<f32x4*>(smem_raw);                                // [NWK][NT][64]
     float* sred = reinterpret_cast<float*>(smem_raw + (size_t)NWK * NT * 1024);     // [NS][16]
+    [[maybe_unused]] float* head_ss = sred + 4 * NR;   // epilogue 5: [NT][16]
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int l15 = lane & 15, grp = lane >> 4;
     const int ntiles = N >> 4;
@@ -1093,8 +1094,18 @@ __device__ __forceinline__ void rowdir_body(const RowParArgs& a, const uint4* __
             r4 = load_resid(m0);
         }
     }
+    // epilogue 5: this row's position and cache block
+    [[maybe_unused]] int pos = 0, blk = 0;
+    if constexpr (EPI == 5) {
+        static_assert(EPI != 5 || (NT == 8 && !LOOP), "a workgroup's features are one head of 128");
+        if (wave < NT) {
+            const int r = min(m0 + l15, M - 1);
+            pos = a.q.pos[r];
+            blk = a.q.block_tables[(size_t)a.q.slot[r] * a.q.max_blocks + (pos >> 8)];
+        }
+    }
     if constexpr (EPI == 1 && LOOP) rownorm_partials_blocks<NR>(a.rn, m0, m_step, M, sred);
-    if constexpr (EPI == 1 && !LOOP) rownorm_partials<NR>(a.rn, m0, M, sred);
+    if constexpr ((EPI == 1 || EPI == 5) && !LOOP) rownorm_partials<NR>(a.rn, m0, M, sred);
     __builtin_amdgcn_sched_barrier(0);  // every load above is issued before the first use below (one round trip)
     NVLLM_STAMP(a, 1);
 
@@ -1126,6 +1137,18 @@ __device__ __forceinline__ void rowdir_body(const RowParArgs& a, const uint4* __
         if constexpr (EPI == 0)
             if (fin) r4_next = load_resid(m_next);
         __builtin_amdgcn_sched_barrier(0);
+    }
+    // epilogue 5: what the rotation and the norm of this wave's 16 features and of those it is paired with need
+    [[maybe_unused]] f32x4 cs, sn, w_own, w_other;
+    if constexpr (EPI == 5) {
+        if (wave < NT && (int)blockIdx.x < a.q.nh_l + a.q.kv.kv_l) {
+            const float* w8 = (int)blockIdx.x < a.q.nh_l ? a.q.qn : a.q.kn;
+            const size_t at = (size_t)pos * 64 + (wave & 3) * 16 + grp * 4;
+            cs = *reinterpret_cast<const f32x4*>(a.q.cos + at);
+            sn = *reinterpret_cast<const f32x4*>(a.q.sin + at);
+            w_own = *reinterpret_cast<const f32x4*>(w8 + wave * 16 + grp * 4);
+            w_other = *reinterpret_cast<const f32x4*>(w8 + (wave ^ 4) * 16 + grp * 4);
+        }
     }
     __syncthreads();
     NVLLM_STAMP(a, 3);
@@ -1188,6 +1211,48 @@ __device__ __forceinline__ void rowdir_body(const RowParArgs& a, const uint4* __
             const size_t o = a.o_packed ? xpack_off(row, pair * 16 + grp * 4, I >> 5) : (size_t)row * I + (size_t)pair * 16 + grp * 4;
             *reinterpret_cast<uint2*>(a.oh + o) = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
             *reinterpret_cast<uint2*>(a.ol + o) = make_uint2(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16));
+        }
+    } else if constexpr (EPI == 5) {
+        // qwen3.rs:208-234 on the head: norm over its 128 features (q, k), half-split rotation (features d and d + 64: tiles t and t + 4),
+        // then q to the f32 buffer and k, v into the cache.  The f32 sums' way through memory and the row kernel's launch (4.5 us and the gap
+        // before it) for a longer epilogue: rule and figures at gemm_rowdir_qkv_ok
+        const QkvArgs& q = a.q;
+        const int head = blockIdx.x;
+        const float ri = rownorm_rinv_lds<NR>(a.rn, sred, l15);
+        __syncthreads();  // every finishing wave is done reading red
+        if (wave < NT) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) sum[r] *= ri;
+            red[(size_t)wave * 64 + lane] = sum;
+            float ss = (sum[0] * sum[0] + sum[1] * sum[1]) + (sum[2] * sum[2] + sum[3] * sum[3]);
+            ss += __shfl_xor(ss, 16);
+            ss += __shfl_xor(ss, 32);
+            if (grp == 0) head_ss[wave * NR + l15] = ss;
+        }
+        __syncthreads();
+        if (wave < NT && row < M) {
+            const int kv_l = q.kv.kv_l, f0 = wave * 16 + grp * 4;
+            if (head < q.nh_l + kv_l) {
+                float ss = 0.f;
+#pragma unroll
+                for (int k = 0; k < NT; ++k) ss += head_ss[k * NR + l15];
+                const float rinv = 1.0f / sqrtf(ss / 128.0f + q.eps), turn = wave < 4 ? -1.0f : 1.0f;
+                const f32x4 other = red[(size_t)(wave ^ 4) * 64 + lane];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) sum[r] = (sum[r] * rinv) * w_own[r] * cs[r] + turn * ((other[r] * rinv) * w_other[r] * sn[r]);
+            }
+            if (head < q.nh_l) {
+                *reinterpret_cast<float4*>(q.q_out + (size_t)row * (q.nh_l * 128) + (size_t)head * 128 + f0) =
+                    make_float4(sum[0] * q.q_scale, sum[1] * q.q_scale, sum[2] * q.q_scale, sum[3] * q.q_scale);
+            } else {
+                const bool is_k = head < q.nh_l + kv_l;
+                const size_t slab = (size_t)(blk * kv_l + head - q.nh_l - (is_k ? 0 : kv_l)) * kBlockTokens * 128;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    if (is_k) store_k24(reinterpret_cast<_Float16*>(q.kv.k) + slab, q.kv.klo ? q.kv.klo + slab : nullptr, pos & 255, f0 + r, 128, sum[r]);
+                    else store_v24(reinterpret_cast<_Float16*>(q.kv.v) + slab, q.kv.vlo ? q.kv.vlo + slab : nullptr, pos & 255, f0 + r, 128, sum[r]);
+                }
+            }
         }
     } else if constexpr (EPI >= 3) {
         if (fin && row < M) {
@@ -1317,7 +1382,7 @@ static hipError_t rowdir_launch_t(const RowParArgs& a, const PackedW& w, hipStre
     const int groups = (w.N / 16 + NT - 1) / NT, blocks = (a.M + 15) / 16;
     // one round of the 256 CUs where a few row blocks per workgroup make it one, and where the 128 registers of a 1024-thread workgroup
     // hold the weights beside the next block's rows
-    if constexpr (NT * TK + 2 * TK <= (EPI == 1 || EPI == 2 ? 24 : 18)) {
+    if constexpr (EPI != 5 && NT * TK + 2 * TK <= (EPI == 1 || EPI == 2 ? 24 : 18)) {
         if (groups * blocks > 256) {
             const size_t lds = red + (size_t)std::max(NT, 4 * kRowDirBlocks) * 16 * 4;
             static std::atomic<uint64_t> lds_set{0};
@@ -1327,7 +1392,7 @@ static hipError_t rowdir_launch_t(const RowParArgs& a, const PackedW& w, hipStre
             return hipGetLastError();
         }
     }
-    const size_t lds = red + (size_t)(NT > 4 ? NT : 4) * 16 * 4;
+    const size_t lds = red + (size_t)(EPI == 5 ? NT + 4 : NT > 4 ? NT : 4) * 16 * 4;
     static std::atomic<uint64_t> lds_set{0};
     ensure_dyn_lds(reinterpret_cast<const void*>(gemm_rowdir_kernel<NT, NWK, TK, EPI>), lds, lds_set);
     gemm_rowdir_kernel<NT, NWK, TK, EPI><<<dim3(groups, 1, blocks), NWK * 64, lds, s>>>(a, w.data, w.N, w.K / 32);
@@ -1341,6 +1406,20 @@ static hipError_t rowdir_dispatch(const RowDirShape& d, const RowParArgs& a, con
     if constexpr (EPI >= 2) { NVLLM_RD(4, 2) NVLLM_RD(4, 4) NVLLM_RD(2, 6) NVLLM_RD(2, 8) NVLLM_RD(1, 2) NVLLM_RD(1, 4) NVLLM_RD(1, 6) NVLLM_RD(1, 8) }
 #undef NVLLM_RD
     return hipErrorNotSupported;
+}
+
+// One round of workgroups (a head x 16 rows) that fills more than half the chip: 0.6B prompts of 90, 117 and 128 tokens 1.576 -> 1.521, 1.625 ->
+// 1.547 and 1.656 -> 1.563 ms; fewer rows gain nothing (64: 1.321 -> 1.312; 16, where the plain product spreads a head over 8 workgroups, 1.135
+// -> 1.199), a second round neither (129: 1.840 -> 1.863, 200: 2.112 -> 2.105).
+bool gemm_rowdir_qkv_ok(int N, int K, int hd, int M) {
+    const int wgs = N / 128 * ((M + 15) / 16);
+    return hd == 128 && K == 1024 && N % 128 == 0 && wgs > 128 && wgs <= 256 && rowdir_shape(N, K, 2, M).nt != 0;
+}
+hipError_t launch_gemm_rowdir_qkv(const RowParArgs& a, const PackedW& w, hipStream_t s) {
+    if (!gemm_rowdir_qkv_ok(w.N, w.K, a.q.kv.hd, a.M) || w.N != (a.q.nh_l + 2 * a.q.kv.kv_l) * 128) return hipErrorNotSupported;
+    if (a.q.kv.klo && !a.q.kv.vlo) return hipErrorInvalidValue;  // 24-bit K comes with 24-bit V only
+    if (a.M <= 0) return hipSuccess;
+    return rowdir_launch_t<8, 16, 2, 5>(a, w, s);
 }
 
 template <int MT, int NWN, int NWK, int TPW, int PH, int EPI>
