@@ -493,19 +493,21 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
 }
 
 // ---- host side -------------------------------------------------------------------------------------
-// Shape of the launch for an [M][N] output: block geometry (NTW, WN) and K splits.  Candidates: 256 x 256 and 256 x 192
-// (WN 2) and 128 x 256 (WN 4, NTW 4) for outputs too narrow or too short to fill the chip with 256-row blocks; mode 0
-// may split K (f32 slabs, summed by the consumer like the chunked kernel's).  Cost in microseconds = chip rounds x one
-// block's MFMA time (hi + lo planes, half the dense peak as the sustained rate, the narrow block charged 25 % more for
-// its LDS reads per MFMA) + the slabs' write and re-read when K is split.  ntw == 0: not covered, or fewer than
-// min_wgs workgroups.
+// Shape of the launch for an [M][N] output: block geometry (NTW, WN) and K splits.  Candidates: 256 x 256 and 256 x 192 (WN 2), and 128 x 256
+// and 128 x 128 (WN 4, NTW 4 and 2) for outputs too narrow or too short to fill the chip with bigger blocks; mode 0 may split K (f32 slabs,
+// summed by the consumer like the chunked kernel's).  Cost in microseconds = chip rounds x one block's MFMA time (hi + lo planes, half the
+// dense peak as the sustained rate, the narrow blocks charged for their LDS reads per MFMA: 25 %, and 100 % for 128 x 128) + the slabs'
+// write and re-read when K is split.  Without 128 x 128 blocks and with them, ms: 0.6B prompts of 257 tokens 3.41 -> 3.01, 512 3.73 -> 3.39,
+// 1024 5.09 -> 4.98, from 1300 on the same; four prompts of 64 to 200 tokens of a 1024-wide decoder 0.929 -> 0.858.  Charged 60 % instead
+// they take over where they lose: 2391 tokens 7.62 -> 7.94, 18.7 k tokens 41.9 -> 44.8.
+// ntw == 0: not covered, or fewer than min_wgs workgroups.
 struct TileShape { int ntw = 0, wn = 0, ks = 1; };
 static TileShape tile_shape(int M, int N, int K, int mode, int min_wgs, int max_split) {
     TileShape best;
     if (M < 1 || K % 64 != 0 || K < 128 || N % 32 != 0) return best;
     const int KT = K / 32;
     double best_cost = 0;
-    const int cand[3][2] = {{8, 2}, {6, 2}, {4, 4}};
+    const int cand[4][2] = {{8, 2}, {6, 2}, {4, 4}, {2, 4}};
     for (const auto& c : cand) {
         const int ntw = c[0], wn = c[1], cols = wn * ntw * 16, rows = (8 / wn) * 64;
         if (N % cols != 0 || (mode == 2 && ntw % 2)) continue;
@@ -514,7 +516,7 @@ static TileShape tile_shape(int M, int N, int K, int mode, int min_wgs, int max_
             if (KT % (2 * ks) != 0 || (ks > 1 && KT / ks < 8)) continue;
             const int64_t wgs = blocks * ks;
             if (wgs < min_wgs) continue;
-            const double block_us = 4.0 * rows * cols * (double)(K / ks) / (2.5e15 * 0.5 / 256) * 1e6 * (wn == 4 ? 1.25 : 1.0);
+            const double block_us = 4.0 * rows * cols * (double)(K / ks) / (2.5e15 * 0.5 / 256) * 1e6 * (ntw == 2 ? 2.0 : wn == 4 ? 1.25 : 1.0);
             const double slab_us = ks > 1 ? 2.0 * ks * (double)M * N * 4 / 4e12 * 1e6 : 0.0;
             const double cost = (double)((wgs + 255) / 256) * block_us + slab_us;
             if (!best.ntw || cost < best_cost) { best.ntw = ntw; best.wn = wn; best.ks = ks; best_cost = cost; }
@@ -565,18 +567,22 @@ hipError_t launch_gemm_tile(const bf16_bits* xh, const bf16_bits* xl, const Pack
     a.M = M; a.N = w.N; a.KT = w.K / 32;
     if (n_slabs) *n_slabs = t.ks;
     if (mode == 0) {
+        if (t.ntw == 2) return tile_launch_t<2, 4, 0>(a, t.ks, s);
         if (t.wn == 4) return tile_launch_t<4, 4, 0>(a, t.ks, s);
         return t.ntw == 8 ? tile_launch_t<8, 2, 0>(a, t.ks, s) : tile_launch_t<6, 2, 0>(a, t.ks, s);
     }
     if (mode == 2) {
+        if (t.ntw == 2) return tile_launch_t<2, 4, 2>(a, 1, s);
         if (t.wn == 4) return tile_launch_t<4, 4, 2>(a, 1, s);
         return t.ntw == 8 ? tile_launch_t<8, 2, 2>(a, 1, s) : tile_launch_t<6, 2, 2>(a, 1, s);
     }
     if (mode == 4) {
+        if (t.ntw == 2) return tile_launch_t<2, 4, 4>(a, 1, s);
         if (t.wn == 4) return tile_launch_t<4, 4, 4>(a, 1, s);
         return t.ntw == 8 ? tile_launch_t<8, 2, 4>(a, 1, s) : tile_launch_t<6, 2, 4>(a, 1, s);
     }
     if (mode == 4 + ACT_GELU) {
+        if (t.ntw == 2) return tile_launch_t<2, 4, 8>(a, 1, s);
         if (t.wn == 4) return tile_launch_t<4, 4, 8>(a, 1, s);
         return t.ntw == 8 ? tile_launch_t<8, 2, 8>(a, 1, s) : tile_launch_t<6, 2, 8>(a, 1, s);
     }
