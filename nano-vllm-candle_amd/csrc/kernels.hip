@@ -1821,8 +1821,27 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
         tile = a.tile_order[g & 1 ? end - 1 - r : tile];
     }
     // fused decode: every q-tile is one row and tile i is row i (no tile_row0/tile_nrows round trip)
-    const int row0 = FUSED ? tile : a.tile_row0[tile], nrows = FUSED ? 1 : a.tile_nrows[tile], slot = a.tile_slot[tile];
+    const int row0 = FUSED ? tile : a.tile_row0[tile], nrows = FUSED ? 1 : a.tile_nrows[tile];
     const int gqa = a.gqa, tpq = 16 / gqa;
+    // fused decode: what needs the row alone is asked for before the slot, the position and the block table are waited for (a 0.6B step of
+    // one row 0.907 -> 0.890 ms, of 16 rows 1.227 -> 1.208, of 64 with a 24-bit cache 1.890 -> 1.846; 64 and more rows the same)
+    [[maybe_unused]] float x[DC][8], qw[DC][8], ssq_g = 0.f;
+    [[maybe_unused]] const float* qkv_row = FUSED ? a.qkv + (size_t)row0 * a.ldqkv : nullptr;
+    [[maybe_unused]] const int qrow_ok = l15 < gqa;
+    [[maybe_unused]] const float* pq = qkv_row + (size_t)(qrow_ok ? kh * gqa + l15 : 0) * HD + grp * 8;
+    if constexpr (FUSED) {
+#pragma unroll
+        for (int c = 0; c < DC; ++c) {
+            *reinterpret_cast<float4*>(&x[c][0]) = *reinterpret_cast<const float4*>(pq + c * 32);
+            *reinterpret_cast<float4*>(&x[c][4]) = *reinterpret_cast<const float4*>(pq + c * 32 + 4);
+            *reinterpret_cast<float4*>(&qw[c][0]) = *reinterpret_cast<const float4*>(a.qn + c * 32 + grp * 8);
+            *reinterpret_cast<float4*>(&qw[c][4]) = *reinterpret_cast<const float4*>(a.qn + c * 32 + grp * 8 + 4);
+        }
+        // deferred input norm of this row: lane g loads group g (groups <= 64), summed below
+        if (a.rn.ssq && lane < a.rn.groups) ssq_g = a.rn.ssq[(size_t)lane * a.rn.stride + row0];
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    const int slot = a.tile_slot[tile];
     const int kv_l = a.kv.kv_l;
     const int ldq = a.nh_l * HD;
 
@@ -1891,7 +1910,6 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
         constexpr int half = HD / 2;
         const int row = row0;
         const int pos = a.pos[row];
-        const float* qkv_row = a.qkv + (size_t)row * a.ldqkv;
         // the wave whose tile holds the new token makes its K and V, patches them into the tile it has loaded and stores them for later steps:
         // no wave waits for another one, for a store or with its first tile (split-KV: one workgroup has such a wave).  With wave 0 as the
         // maker, its stores waited for and a barrier behind them, and with prefetches past the end that read a shared dummy tile: a 0.6B step
@@ -1910,16 +1928,7 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
             knw1 = a.kn[ln]; knw2 = a.kn[ln + half];
             kc = a.cos[(size_t)pos * half + ln]; ks = a.sin[(size_t)pos * half + ln];
         }
-        float x[DC][8], qw[DC][8], cs[DC / 2][8], sn[DC / 2][8];
-        const int qrow_ok = my_row[0] >= 0;
-        const float* pq = qkv_row + (size_t)(qrow_ok ? my_head : 0) * HD + grp * 8;
-#pragma unroll
-        for (int c = 0; c < DC; ++c) {
-            *reinterpret_cast<float4*>(&x[c][0]) = *reinterpret_cast<const float4*>(pq + c * 32);
-            *reinterpret_cast<float4*>(&x[c][4]) = *reinterpret_cast<const float4*>(pq + c * 32 + 4);
-            *reinterpret_cast<float4*>(&qw[c][0]) = *reinterpret_cast<const float4*>(a.qn + c * 32 + grp * 8);
-            *reinterpret_cast<float4*>(&qw[c][4]) = *reinterpret_cast<const float4*>(a.qn + c * 32 + grp * 8 + 4);
-        }
+        float cs[DC / 2][8], sn[DC / 2][8];
 #pragma unroll
         for (int c = 0; c < DC / 2; ++c) {
             const size_t o = (size_t)pos * half + c * 32 + grp * 8;
@@ -1928,8 +1937,6 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
             *reinterpret_cast<float4*>(&sn[c][0]) = *reinterpret_cast<const float4*>(a.sin + o);
             *reinterpret_cast<float4*>(&sn[c][4]) = *reinterpret_cast<const float4*>(a.sin + o + 4);
         }
-        // deferred input norm of this row: lane g loads group g (groups <= 64), summed below
-        const float ssq_g = (a.rn.ssq && lane < a.rn.groups) ? a.rn.ssq[(size_t)lane * a.rn.stride + row] : 0.f;
         // This wave's first KV tile goes in flight BEHIND the prologue's own loads (vmcnt retires in order, so the prologue never waits for
         // it) and lands while it computes; a second set would push the kernel to one wave per SIMD.  The new token's place in its tile still
         // holds old bytes, or the new ones if the stores below pass first: the tile is patched before it is used.
