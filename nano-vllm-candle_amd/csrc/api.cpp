@@ -1055,9 +1055,7 @@ static bool fused_plan(const nvllm_model* m, int R, FusedPlan& p) {
     else p.gu = G_GENERIC;  // generic kernel with the SwiGLU epilogue (no K split)
     const bool no_xpack = m->opt_no_xpack != 0;
     auto takes_packed = [&](int kind, int N, int K, int epi) { return kind == G_STREAM || (kind == G_ROW && gemm_rowdir_ok(N, K, epi, R)); };
-    // fewer than 16 rows: a fragment-order plane is 15/16 padding (a 1-row step would load 1 KiB per k-tile where a
-    // row-major plane serves 64 bytes to all 16 lanes): batch 1 measured 960 -> 1017 tokens/s with row-major planes
-    p.packed = !no_xpack && R >= 16 && m->I_l % 32 == 0 && takes_packed(p.qkv, NQ, H, 2) && takes_packed(p.o, H, KO, tp ? 2 : 0) &&
+    p.packed = !no_xpack && R >= kPackedMinRows && m->I_l % 32 == 0 && takes_packed(p.qkv, NQ, H, 2) && takes_packed(p.o, H, KO, tp ? 2 : 0) &&
                takes_packed(p.gu, I2, H, 1) && takes_packed(p.down, H, m->I_l, tp ? 2 : 0);
     return true;
 }

@@ -18,7 +18,7 @@ ProductPlan plan_product(const nvllm_model* m, int R, const PackedW& w) {
     if (ss > 0 && (size_t)ss * one <= m->slab_floats) { p.kind = P_STREAM; p.packed = 1; return p; }
     if (R <= kRowMaxRows && gemm_rowpar_ok(w.N, w.K, 2, R) && (size_t)gemm_rowpar_splits(w.N, w.K, 2, R) * one <= m->slab_floats) {
         p.kind = P_ROW;
-        p.packed = R >= 16 && gemm_rowdir_ok(w.N, w.K, 2, R);
+        p.packed = R >= kPackedMinRows && gemm_rowdir_ok(w.N, w.K, 2, R);
     }
     return p;
 }
@@ -50,7 +50,7 @@ GluPlan plan_glu(const nvllm_model* m, int R, const PackedW& w, bool want_packed
     if (R <= kRowMaxRows && gemm_rowpar_ok(w.N, w.K, 1, R)) {
         g.kind = P_ROW;
         const bool dir = gemm_rowdir_ok(w.N, w.K, 1, R);
-        g.packed = R >= 16 && dir;
+        g.packed = R >= kPackedMinRows && dir;
         g.out_packed_ok = dir;
         return g;
     }
