@@ -1304,10 +1304,15 @@ static RowDirShape rowdir_shape(int N, int K, int epi, int M) {
         // one row block (<= 16 rows, e.g. batch 1): the grid is the n-groups alone, so fewer tiles per workgroup put the
         // matrix on more CUs (0.6B gate/up: 64 -> 192 workgroups)
         if (M <= 16 && ntiles / 2 <= 512) nt = 2;
+        else if (M <= 32 && nt == 6 && 2 * ((ntiles + 5) / 6) < 256) nt = 4;  // two row blocks: below
     } else {
         nt = 4;
         if (nt * tk > 16) nt = 2;
         if (nt * tk > 16) return none;
+        // two row blocks whose workgroups do not fill the chip: fewer tiles each (0.6B QKV 128 -> 256 workgroups, gate/up 128 -> 192).  Steps
+        // of 17, 24, 32 rows, 100 to 300 tokens: 1.090 -> 1.041, 1.117 -> 1.064, 1.147 -> 1.091 ms; QKV alone 1.067, 1.087, 1.118, gate/up alone
+        // 1.070, 1.092, 1.127, gate/up with two tiles 1.088, 1.109, 1.138; two decoders of other designs 3 to 5 %
+        if (M > 16 && M <= 32 && nt == 4 && 2 * ((ntiles + 3) / 4) < 256) nt = 2;
         if (M <= 16 && ntiles <= 512) nt = 1;  // as above (0.6B QKV: 64 -> 256 workgroups)
     }
     // weights are streamed once per row block: big matrices belong to the 64-row kernel
@@ -1403,7 +1408,7 @@ static hipError_t rowdir_dispatch(const RowDirShape& d, const RowParArgs& a, con
 #define NVLLM_RD(NT_, TK_) if (d.nt == NT_ && d.tk == TK_) return rowdir_launch_t<NT_, 16, TK_, EPI>(a, w, s);
     if constexpr (EPI == 0) { NVLLM_RD(1, 2) NVLLM_RD(1, 4) NVLLM_RD(1, 6) NVLLM_RD(1, 8) NVLLM_RD(2, 2) NVLLM_RD(2, 4) NVLLM_RD(2, 6) NVLLM_RD(4, 2) NVLLM_RD(4, 4) }
     if constexpr (EPI == 1) { NVLLM_RD(6, 2) NVLLM_RD(4, 2) NVLLM_RD(4, 4) NVLLM_RD(2, 2) NVLLM_RD(2, 4) NVLLM_RD(2, 6) NVLLM_RD(2, 8) }
-    if constexpr (EPI >= 2) { NVLLM_RD(4, 2) NVLLM_RD(4, 4) NVLLM_RD(2, 6) NVLLM_RD(2, 8) NVLLM_RD(1, 2) NVLLM_RD(1, 4) NVLLM_RD(1, 6) NVLLM_RD(1, 8) }
+    if constexpr (EPI >= 2) { NVLLM_RD(4, 2) NVLLM_RD(4, 4) NVLLM_RD(2, 2) NVLLM_RD(2, 4) NVLLM_RD(2, 6) NVLLM_RD(2, 8) NVLLM_RD(1, 2) NVLLM_RD(1, 4) NVLLM_RD(1, 6) NVLLM_RD(1, 8) }
 #undef NVLLM_RD
     return hipErrorNotSupported;
 }
