@@ -524,8 +524,8 @@ __global__ void __launch_bounds__(256, 2) bias_prefill_kernel(BiasAttnArgs a, in
                     if (hidden(tokB + r)) sb[u][r] = -1e30f;
                 }
             }
-            float mt = fmaxf(max3_raw(sa[u][0], sa[u][1], sa[u][2]), max3_raw(sa[u][3], sb[u][0], sb[u][1]));
-            mt = max3_raw(mt, sb[u][2], sb[u][3]);
+            float mt = fmaxf(max3(sa[u][0], sa[u][1], sa[u][2]), max3(sa[u][3], sb[u][0], sb[u][1]));
+            mt = max3(mt, sb[u][2], sb[u][3]);
             mt = fmaxf(mt, __shfl_xor(mt, 16));
             mt = fmaxf(mt, __shfl_xor(mt, 32));
             const float mn = fmaxf(m[u], mt), alpha = __builtin_amdgcn_exp2f(m[u] - mn);

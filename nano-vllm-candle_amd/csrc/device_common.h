@@ -31,13 +31,10 @@ __device__ __forceinline__ _Float16 f16_sat(float x) { return (_Float16)fminf(fm
 // carries 13..14 significant bits, and the reader rebuilds r's f16 by a byte shift (no arithmetic).
 __device__ __forceinline__ void store_v24(_Float16* v, uint8_t* vlo, int t_in_block, int d, int hd, float x);
 
-// max of three without the canonicalising v_max_f32 x, x that fmaxf() adds per operand (operands here are MFMA results
-// and finite constants: no signalling NaN to quiet)
-__device__ __forceinline__ float max3_raw(float a, float b, float c) {
-    float r;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
+// max of three in one v_maximum3_f32, NaN if one of them is: fmaxf() would add a canonicalising v_max_f32 x, x per operand.  Not inline
+// assembly: the operands are matrix results, and the compiler puts the wait states between a matrix instruction and its reader (8 for a
+// 16x16x32 product) only where it knows the reader.
+__device__ __forceinline__ float max3(float a, float b, float c) { return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c); }
 
 // eight values as f16 hi + lo (hi + lo = x to 22 bits), both to nearest even: pairs by v_cvt_pk_f16_f32, the remainder by one mixed
 // fused multiply-add per value

@@ -2521,7 +2521,7 @@ __global__ void __launch_bounds__(NH * 256, 2) attn_prefill_kernel(AttnArgs a) {
         // not the maximum: it moves only when a score exceeds it by more than kSlack (p stays below 2^kSlack, well inside f16, and
         // p / sum p does not depend on the reference), so the usual tile needs no maximum across lanes, no rescale of O and, the
         // reference being the accumulators' start, no subtraction.  Every row that has a visible token has one in its wave's first tile,
-        // where the reference is set.  Raw v_exp_f32 (a flushed denormal is 0 either way), v_max3 without the NaN canonicalisation
+        // where the reference is set.  Raw v_exp_f32 (a flushed denormal is 0 either way), v_maximum3 without the canonicalisation
         // fmaxf() pays per operand, the causal mask only on tiles that reach past the wave's first row.
         constexpr float kSlack = 8.f;
         f16x8 P[QT], Pl[QT];  // P as f16 hi + lo (see attn_paged_kernel): the prompt's own K/V-dependent rows keep 22 bits too
@@ -2538,17 +2538,17 @@ __global__ void __launch_bounds__(NH * 256, 2) attn_prefill_kernel(AttnArgs a) {
         bool moves = fresh;
 #pragma unroll
         for (int t = 0; t < QT; ++t) {
-            mt[t] = max3_raw(sa[t][0], sa[t][1], sa[t][2]);
-            mt[t] = max3_raw(mt[t], sa[t][3], sb[t][0]);
-            mt[t] = max3_raw(mt[t], sb[t][1], sb[t][2]);
-            mt[t] = max3_raw(mt[t], sb[t][3], mt[t]);
+            mt[t] = max3(sa[t][0], sa[t][1], sa[t][2]);
+            mt[t] = max3(mt[t], sa[t][3], sb[t][0]);
+            mt[t] = max3(mt[t], sb[t][1], sb[t][2]);
+            mt[t] = max3(mt[t], sb[t][3], mt[t]);
             moves = moves || mt[t] > kSlack;
         }
         if (__builtin_amdgcn_ballot_w64(moves) != 0) {
 #pragma unroll
             for (int t = 0; t < QT; ++t) {
-                float up = max3_raw(mt[t], __shfl_xor(mt[t], 16), mt[t]);
-                up = max3_raw(up, __shfl_xor(up, 32), up);      // the row's maximum, the same in its four lanes
+                float up = max3(mt[t], __shfl_xor(mt[t], 16), mt[t]);
+                up = max3(up, __shfl_xor(up, 32), up);      // the row's maximum, the same in its four lanes
                 if (!fresh) up = fmaxf(up, 0.f);
                 else if (up <= -1e29f) up = 0.f;                // no visible token (and none to come)
                 const float alpha = __builtin_amdgcn_exp2f(-up);  // fresh: what it scales is 0
