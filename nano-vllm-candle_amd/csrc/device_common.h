@@ -389,10 +389,11 @@ __device__ __forceinline__ void lds_read_fragments(bf16x8 (&x)[4], uint32_t addr
 
 // 1 KiB of LDS-DMA that hipcc's wait insertion does not see: `src` per lane, the wave's 1 KiB of LDS at byte address `lds` (uniform).  With
 // the builtin, every ordinary LDS read after it waits for vmcnt(0), which drains the copies meant to stay in flight; with this form
-// ordinary reads stay ordinary, and the kernel's own vmcnt waits are the only ones.  For kernels whose LDS-DMA is all of this form (M0 is
-// set here and is nobody else's).
+// ordinary reads stay ordinary, and the kernel's own vmcnt waits are the only ones.  For kernels whose LDS-DMA is all of this form.  The
+// compiler writes M0 as the operand's register (a write inside the statement would be unknown to it); the wait state behind that write is
+// the statement's own.
 __device__ __forceinline__ void lds_dma16(const void* src, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"{m0}"(lds), "v"(src) : "memory");
 }
 
 // Barrier that PUBLISHES LDS-DMA data (global_load_lds): every wave first waits for its own DMA to land, then joins the

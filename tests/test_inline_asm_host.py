@@ -1,5 +1,6 @@
 """CPU: what the kernels' inline assembly may hold.  The compiler inserts the wait states between a matrix instruction and a reader of its
-result, but not in front of an asm statement, which it does not look into."""
+result, but not in front of an asm statement, which it does not look into; and it knows of the registers a statement writes from its
+operands alone."""
 import glob
 import os
 import re
@@ -37,3 +38,9 @@ def test_the_statements_are_found():
 def test_no_vector_arithmetic(where):
     # a vector instruction in asm may read a matrix result before its wait states are over
     assert not re.search(r"\bv_\w+", templates(where[2])), where
+
+
+@pytest.mark.parametrize("where", asm_statements(), ids=lambda w: f"{w[0]}:{w[1]}")
+def test_no_register_is_written_behind_the_compilers_back(where):
+    # M0 above all: the LDS-DMA builtin and indexed registers read it, set up wherever the compiler likes
+    assert not re.search(r"\bs_\w+\s+m0\b", templates(where[2])), where
