@@ -1324,7 +1324,7 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
         qa.kv.k = m->kcache[l]; qa.kv.v = m->vcache[l]; qa.kv.kv_l = m->kv_l; qa.kv.hd = hd;
         qa.kv.vlo = m->vlocache.empty() ? nullptr : m->vlocache[l];
         qa.kv.klo = m->klocache.empty() ? nullptr : m->klocache[l];
-        const bool fuse_qk = qt == 1 && n_tiles == R;  // decode: every q-tile is one row
+        const bool fuse_qk = qt == 1 && n_tiles == R && R <= kAttnFusedMaxRows;  // decode: every q-tile is one row
         int rcg = NVLLM_OK;
         if (t_qkv_fused && !fuse_qk) {
             // prompt chunk: q/k-norm + RoPE + KV write + q output in the QKV GEMM's epilogue (one wave tile = one head)

@@ -283,6 +283,7 @@ struct AttnArgs {
     unsigned long long* stamps = nullptr;  // diagnostic build only: [workgroup][16 waves][8] s_memrealtime stamps
 #endif
 };
+constexpr int kAttnFusedMaxRows = 65535;  // with AttnArgs::qkv the rows are the grid's y, which ends there
 // decode: one row per workgroup and kv head
 hipError_t launch_attn_paged(const AttnArgs& a, int n_tiles, int rows, int n_parts_max, hipStream_t s);
 // qt = q sub-tiles (of 16 MFMA rows) per q-tile: 1 (decode) or 2 (prefill)

@@ -1808,7 +1808,7 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l15 = lane & 15, grp = lane >> 4;
-    // the tile: the grid's y in a fused step (<= 256 rows), part of x in the others, whose tiles can be more than y takes (65535)
+    // the tile: the grid's y in the fused form (its callers have at most kAttnFusedMaxRows rows), part of x in the other
     int tile = FUSED ? blockIdx.y : __builtin_amdgcn_readfirstlane((int)blockIdx.x / a.kv.kv_l);
     const int kh = FUSED ? blockIdx.x : blockIdx.x - tile * a.kv.kv_l;
     NVLLM_STAMP(a, 0);
@@ -2748,7 +2748,7 @@ hipError_t launch_attn_paged(const AttnArgs& a, int n_tiles, int rows, int n_par
     const int gz = split ? n_parts_max : 1;
     hipError_t e = hipErrorInvalidValue;
     const bool fused = a.qkv != nullptr;  // decode rows straight from the QKV GEMM's slabs
-    if (fused && n_tiles != rows) return hipErrorInvalidValue;  // fused decode: tile i is row i
+    if (fused && (n_tiles != rows || rows > kAttnFusedMaxRows)) return hipErrorInvalidValue;  // fused decode: tile i is row i
     if (a.kv.hd == 128) e = fused ? attn_launch_t<128, 1, 4, true>(b, n_tiles, gz, s) : attn_launch_t<128, 1, 4, false>(b, n_tiles, gz, s);
     else if (a.kv.hd == 64) e = fused ? attn_launch_t<64, 1, 4, true>(b, n_tiles, gz, s) : attn_launch_t<64, 1, 4, false>(b, n_tiles, gz, s);
     if (e != hipSuccess || !split) return e;

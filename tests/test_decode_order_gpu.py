@@ -30,3 +30,23 @@ def test_every_row_of_a_decode_batch_is_its_own_answer(kv, heads, rows):
         m.seq_free(rows)
         assert np.abs(one[0] - got[i]).max() < 5e-4 * np.abs(got[i]).max()
     m.close()
+
+
+def test_more_rows_than_a_grid_axis_takes():
+    """a decode step of more than 65535 sequences, against the same sequences in steps of 4097"""
+    import nano_vllm_candle_amd as pkg
+
+    rows, part = 65600, 4097
+    cfg = pkg.Qwen3Config.tiny(vocab_size=256, num_hidden_layers=1, num_attention_heads=2, num_key_value_heads=1, max_position_embeddings=256)
+    m = pkg.Qwen3ForCausalLM.from_synthetic(cfg, 3)
+    m.kv_alloc(rows, rows, 512)
+    toks = np.random.default_rng(0).integers(0, cfg.vocab_size, (rows, 2)).astype(np.uint32)
+    m.step(list(range(rows)), [t[:1] for t in toks], True)
+    _, got = m.step(list(range(rows)), list(toks), False, want_logits=True)
+    for a in range(0, rows, part):
+        ids = list(range(a, min(rows, a + part)))
+        m.step(ids, [t[:1] for t in toks[ids]], True)
+        _, want = m.step(ids, list(toks[ids]), False, want_logits=True)
+        # other kernels for the products, and q through memory: their rounding, two 16-bit planes a product (2^-15), one layer
+        assert np.abs(got[ids] - want).max() < 5e-4 * np.abs(want).max(), a
+    m.close()
