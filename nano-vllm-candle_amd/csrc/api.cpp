@@ -516,14 +516,15 @@ int stage_flush(nvllm_model* m, bool more) {
         if (p) for (int at : m->table_news) { *p++ = at; *p++ = m->h_block_tables[at]; }
         // steps that took blocks and failed can leave more than the block holds: the whole table instead
         else HIPCHK(m->ctx, hipMemcpyAsync(m->d_block_tables, m->h_block_tables.data(), m->h_block_tables.size() * 4, hipMemcpyHostToDevice, m->ctx->stream));
-        m->table_news.clear();
     }
-    if (!g.n_runs) return NVLLM_OK;
-    g.args.src = g.dev + (size_t)g.slot * g.ints;
-    HIPCHK(m->ctx, launch_stage(g.args, g.n_runs, g.longest, m->ctx->stream));
-    g.busy[g.slot] = true;
-    g.recorded[g.slot] = false;
-    if (more) {
+    if (g.n_runs) {
+        g.args.src = g.dev + (size_t)g.slot * g.ints;
+        HIPCHK(m->ctx, m->opt_stage_fail > 0 ? (--m->opt_stage_fail, hipErrorLaunchFailure) : launch_stage(g.args, g.n_runs, g.longest, m->ctx->stream));
+        g.busy[g.slot] = true;
+        g.recorded[g.slot] = false;
+    }
+    m->table_news.clear();  // not before they are on their way: an entry is noted once
+    if (g.n_runs && more) {
         if (!g.ev[g.slot]) HIPCHK(m->ctx, hipEventCreateWithFlags(&g.ev[g.slot], hipEventDisableTiming));
         HIPCHK(m->ctx, hipEventRecord(g.ev[g.slot], m->ctx->stream));
         g.recorded[g.slot] = true;
@@ -1993,6 +1994,7 @@ extern "C" int nvllm_debug_set_option(nvllm_model* m, const char* name, int valu
         m->opt_kv_v_bits = value; return NVLLM_OK;
     }
     if (!strcmp(name, "oneshot_skip_push")) { m->opt_oneshot_skip_push = std::max(0, value); return NVLLM_OK; }  // test hook
+    if (!strcmp(name, "stage_fail")) { m->opt_stage_fail = std::max(0, value); return NVLLM_OK; }  // test hook
     if (!strcmp(name, "no_fused")) { m->opt_no_fused = value; return NVLLM_OK; }    // decode through the generic path
     if (!strcmp(name, "no_xpack")) { m->opt_no_xpack = value; return NVLLM_OK; }    // row-major activation planes
     if (!strcmp(name, "no_rowpar")) { m->opt_no_rowpar = value; return NVLLM_OK; }  // generic path: no whole-K row-parallel GEMMs

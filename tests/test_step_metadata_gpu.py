@@ -50,3 +50,21 @@ def test_many_chunks_and_tables_after_failed_steps(design, max_seqs, rows):
             lists = [np.append(p, 7) for p in prompts]
             a, b = (x.step(ids, lists, False, want_logits=True) for x in (m, fresh))
             assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("design", ["qwen3", "gopunex"])
+def test_tables_after_a_failed_launch(design):
+    """a step whose metadata launch fails has taken its blocks: the next one must still tell the device of them"""
+    from nano_vllm_candle_amd._lib import NvllmError
+
+    m, fresh = _model(design, 3, 8, 64), _model(design, 3, 8, 64)
+    rng = np.random.default_rng(0)
+    prompts = [rng.integers(0, 300, n) for n in (20, 300, 7)]
+    ids = [0, 1, 2]
+    m.set_option("stage_fail", 1)
+    with pytest.raises(NvllmError):
+        m.step(ids, prompts, True)
+    want = fresh.step(ids, prompts, True, want_logits=True)
+    got = m.step(ids, prompts, False, want_logits=True)  # nothing is cached: the same rows, in the blocks of the failed step
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    m.close(), fresh.close()
