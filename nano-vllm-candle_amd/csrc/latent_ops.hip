@@ -693,6 +693,22 @@ static hipError_t exact_rows_launch(const HeadGemmArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
+// one element of a 32-bit product, term by term
+__device__ __forceinline__ float exact_dot(const HeadGemmArgs& a, int head, int tile, int feature, int row) {
+    const int KT = a.K >> 5;
+    const uint4* wp = a.w + (size_t)head * a.w_head + (size_t)tile * KT * 64 + feature;
+    const float* xp = a.x + (size_t)row * a.x_row + (size_t)head * a.x_head;
+    float sum = 0.f;
+    for (int k = 0; k < KT * 4; ++k) {  // eight at a time
+        const uint4 w = wp[k * 16];
+        const uint32_t wd[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            sum += __builtin_bit_cast(float, (j & 1) ? wd[j >> 1] & 0xffff0000u : wd[j >> 1] << 16) * xp[k * 8 + j];
+    }
+    return sum;
+}
+
 // Eight f32 as three bf16 fragments that sum up to them exactly: each is what the one before left, cut to eight significant bits.  An
 // infinity is its first part alone, NaN stays NaN.
 __device__ __forceinline__ void split_exact(const float (&x)[8], uint4 (&f)[3]) {
@@ -768,6 +784,23 @@ __global__ void __launch_bounds__(256, 2) exact_tile_kernel(HeadGemmArgs a) {
     for (int kt = 0; kt < KT; kt += 2) {
         step(kt, x0, w0, w1);
         if (kt + 1 < KT) step(kt + 1, x1, w1, w0);
+    }
+    // A second or third part that is zero times an infinite weight is NaN where the product is infinite: those elements again, undivided
+    uint32_t nans = 0;
+#pragma unroll
+    for (int i = 0; i < NT * MT * 4; ++i) {
+        const float v = acc[i / (4 * MT)][(i >> 2) % MT][i & 3];
+        nans |= v != v ? 1u << i : 0u;
+    }
+    while (nans) {
+        const int at = __ffs(nans) - 1, n = at / (4 * MT), b = (at >> 2) % MT;
+        nans &= nans - 1;
+        const float v = exact_dot(a, head, min(nt0 + n, ntiles - 1), grp * 4 + (at & 3), min(m0 + b * 16 + l15, a.M - 1));
+#pragma unroll
+        for (int i = 0; i < NT * MT * 4; ++i) {
+            f32x4& to = acc[i / (4 * MT)][(i >> 2) % MT];
+            to[i & 3] = i == at ? v : to[i & 3];
+        }
     }
 #pragma unroll
     for (int n = 0; n < NT; ++n)

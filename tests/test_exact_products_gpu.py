@@ -26,3 +26,29 @@ def test_prompt_of_rows(name, rows):
     # what the layer tests allow this decoder's 32-bit mode: a few hundred f32 sums through a handful of layers
     assert row_err(got, ref) < TOL["float32"]
     m.close()
+
+
+@pytest.mark.parametrize("rows", [64, 65, 130])
+def test_infinite_weights(rows):
+    """a product with an infinite weight is infinite on both sides of the row count where the kernel changes, and nothing else is touched"""
+    import nano_vllm_candle_amd as pkg
+
+    cfg = CONFIGS["mixed"]
+    w = sharp_weights(cfg)
+    c = pkg.GopunexConfig.from_dict(cfg, {k: np.shape(v) for k, v in w.items()})
+    toks = np.random.default_rng(1).integers(0, cfg["vocab"], rows).tolist()
+
+    def logits(weights):
+        m = pkg.GopunexForCausalLM.from_state_dict(c, weights, dtype="float32")
+        m.kv_alloc(140, 130, max_batched_tokens=256)
+        out = m.step_score([0], [toks], True, [list(range(rows))])
+        m.close()
+        return out
+
+    want = logits(w)
+    head = np.array(w["head"], np.float32)
+    head[5, 7], head[300, 70] = np.inf, -np.inf
+    got = logits({**w, "head": head})
+    assert np.isinf(got[:, [5, 300]]).all()
+    keep = [i for i in range(cfg["vocab"]) if i not in (5, 300)]
+    assert np.array_equal(got[:, keep], want[:, keep])
