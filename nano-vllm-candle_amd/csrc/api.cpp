@@ -851,8 +851,8 @@ extern "C" int nvllm_kv_alloc(nvllm_model* m, int num_blocks, int block_size, in
     // every row-sized buffer holds max_rows rows; a decode step has one row per sequence, so max_seqs rows must fit
     m->max_rows = std::max({max_batched_tokens, max_seqs, 16});
     if (m->opt_oneshot_allreduce && ctx->tp_size > 1 && !ctx->null_comm) {
-        // collective: every rank of the group reaches this with the same option (slot = the largest fused decode message)
-        (void)oneshot_setup(ctx, (size_t)kFusedMaxRows * m->H);
+        // collective: every rank of the group reaches this with the same option
+        (void)oneshot_setup(ctx, (size_t)kOneshotMaxRows * m->H);
     } else if (ctx->oneshot) {
         oneshot_free(ctx);  // option switched off: back to the communicator's all-reduce (same decision on every rank)
     }

@@ -82,6 +82,9 @@ static int dmalloc(nvllm_ctx* c, T** p, size_t count) {
 constexpr int kPackedMinRows = 4;
 constexpr int kFusedMaxRows = 256;  // the fused decode path (deferred norms, row-parallel epilogues) handles up to this many rows ...
 constexpr int kRowMaxRows = 128;    // ... and so many where a projection of the layer has no register-direct form; row-parallel products elsewhere
+// one-shot all-reduce: messages of up to this many rows; its slots are sized for them (uncached memory on every peer).  Longer ones go
+// through the communicator, in decode steps of more rows too: what the one-shot form does for those was never measured
+constexpr int kOneshotMaxRows = 128;
 constexpr int kMaxPending = 4;   // decode steps that may be enqueued before one is collected
 constexpr int kAttnMaxParts = 64;  // split-KV partitions per sequence (partition grows with context beyond 8K)
 

@@ -206,3 +206,34 @@ def test_oneshot_allreduce_gives_up_with_an_error_code_on_every_rank(oracle):
             assert row_rel_err(lg, rlg) < LOGITS_TOL and ids.tolist() == rid.tolist(), (rank, step)
         for s, t in zip(ref, rid):
             s.append(int(t))
+
+
+@pytest.mark.parametrize("rows", [128, 129, 256])
+def test_oneshot_allreduce_ends_at_128_rows(rows):
+    # longer messages go through the communicator whatever decode steps are fused: the one-shot slots are sized for 128 rows
+    import nano_vllm_candle_amd as pkg
+
+    cfg = pkg.Qwen3Config.tiny(hidden_size=1024, num_attention_heads=8, num_key_value_heads=4, head_dim=128, intermediate_size=2048, num_hidden_layers=1)
+    tp, toks = 2, np.random.default_rng(rows).integers(0, cfg.vocab_size, rows).tolist()
+    calls, errors = [None] * tp, []
+
+    def worker(rank):
+        try:
+            ctx = pkg.Context(0, tp_rank=rank, tp_size=tp, loopback_group=f"ends{rows}")
+            m = pkg.Qwen3ForCausalLM.from_synthetic(cfg, seed=4, ctx=ctx)
+            m.set_option("oneshot_allreduce", 1)
+            m.kv_alloc(4, 2, 512)
+            m.step([0], [toks], True)
+            calls[rank] = m.counter("oneshot_calls")
+            m.close()
+            ctx.close()
+        except Exception as e:  # noqa: BLE001
+            errors.append((rank, repr(e)))
+
+    threads = [threading.Thread(target=worker, args=(r,)) for r in range(tp)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join(timeout=60)
+    assert not errors, errors
+    assert calls == [2 if rows <= 128 else 0] * tp
