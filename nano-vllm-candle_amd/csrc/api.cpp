@@ -1182,7 +1182,7 @@ static int forward_chunk_fused(nvllm_model* m, const FusedPlan& fp, int R, int n
         aa.q = m->qbuf; aa.kv = qa.kv; aa.block_tables = m->d_block_tables; aa.max_blocks = m->max_blocks;
         aa.tile_row0 = m->d_tile_row0; aa.tile_nrows = m->d_tile_nrows; aa.tile_slot = m->d_tile_slot; aa.pos = m->d_pos;
         aa.tile_last = m->d_tile_last;
-        if (qt == 2) aa.group_order = m->d_group_order;
+        if (qt == 2) { aa.group_order = m->d_group_order; aa.longest = m->cur_max_len; }
         aa.nh_l = m->nh_l; aa.gqa = m->gqa; aa.out_hi = m->ctxh; aa.out_lo = m->ctxl; aa.out_packed = packed;
         if (qt == 1) aa.tile_order = m->d_tile_order;
         if (fuse_qk) {
@@ -1340,7 +1340,7 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
         aa.q = m->qbuf; aa.kv = qa.kv; aa.block_tables = m->d_block_tables; aa.max_blocks = m->max_blocks;
         aa.tile_row0 = m->d_tile_row0; aa.tile_nrows = m->d_tile_nrows; aa.tile_slot = m->d_tile_slot; aa.pos = m->d_pos;
         aa.tile_last = m->d_tile_last;
-        if (qt == 2) aa.group_order = m->d_group_order;
+        if (qt == 2) { aa.group_order = m->d_group_order; aa.longest = m->cur_max_len; }
         aa.nh_l = m->nh_l; aa.gqa = m->gqa; aa.out_hi = m->xh; aa.out_lo = m->xl; aa.out_packed = packed || t_o;
         if (qt == 1) aa.tile_order = m->d_tile_order;
         if (fuse_qk) {
@@ -2260,7 +2260,7 @@ extern "C" int nvllm_op_attention(nvllm_ctx* ctx, const float* q, const float* k
     HIPCHK(ctx, launch_kv_write_plain(kr, vr, rows, dpos, dslot, dbt, bps, kvl, s));
     AttnArgs a;
     a.q = qr; a.kv = kvl; a.block_tables = dbt; a.max_blocks = bps; a.tile_row0 = dt0; a.tile_nrows = dtn; a.tile_slot = dts;
-    a.pos = dpos; a.nh_l = nh; a.gqa = gqa; a.out_f32 = out;
+    a.pos = dpos; a.nh_l = nh; a.gqa = gqa; a.out_f32 = out; a.longest = T;
     HIPCHK(ctx, launch_attn_prefill(a, nt, s));
     HIPCHK(ctx, hipStreamSynchronize(s));
     return NVLLM_OK;

@@ -255,6 +255,7 @@ struct AttnArgs {
     const int* tile_last = nullptr;    // optional (prefill kernel): position of the tile's last row, -1 for an empty tile;
                                        // saves the kernel a chain of dependent metadata loads per workgroup
     const int* pos = nullptr;          // [rows]
+    int longest = 0;                   // prefill: tokens of the longest context among the rows, or an upper bound
     // load balance (decode): tile_order[rank] = tile index, longest context first; walked forwards in even and backwards in odd runs of
     // 256 workgroups, so that co-resident workgroups (ids i and i+256 share a CU when two fit) pair a long sequence with a short one.
     // nullptr = launch order.

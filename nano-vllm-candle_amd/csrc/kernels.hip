@@ -2308,7 +2308,7 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
 // a launch that does not fill the chip twice over.  Measured per launch (16 / 8 heads of 128) with a maximum across lanes, a rescale and
 // a drained ring in every tile, NH = 1: one prompt of 2391 tokens 109 us, now 65; 18.7 k tokens in prompts of 64 to 512, chunks of 4096
 // rows, 34.5 -> 30.7; 32 / 8 heads, 4050 tokens in prompts of 700 to 2000, 152 -> 118.  Both prompts with the other NH: 80, 42 (before
-// the other changes).  VLO: a 24-bit cache (see attn_paged_kernel), whose residual fragments ride in the same ring: 5.4 k tokens in prompts
+// the other changes); when to take which: attn_prefill_two.  VLO: a 24-bit cache (see attn_paged_kernel), whose residual fragments ride in the same ring: 5.4 k tokens in prompts
 // of 48 to 400, 88 us with K and V straight to registers for every q-tile of its own, now 39 and, with NH = 2, 30.
 // ---------------------------------------------------------------------------------------------------
 template <int HD, int QT, int NH, int VLO>
@@ -2725,14 +2725,24 @@ static hipError_t attn_prefill_launch(const AttnArgs& a, int groups, hipStream_t
     } else if (a.kv.vlo) return hipErrorNotSupported;
     return attn_prefill_launch_v<HD, NH, 0>(a, groups, s);
 }
+// Two sets of waves halve the chain of the longest context and pay a merge, and 512 threads with twice the LDS leave a CU one workgroup
+// where it took two: they need fewer than 512 workgroups (measurements at the kernel), and contexts long enough for it, longer ones where
+// the launch is more than one round of the 256 CUs.  A 24-bit cache, with half as much work again in a tile, gains earlier.  0.6B, prompts x
+// tokens, ms with one set and with two.  16 bits, one round: 1 x 100 1.368 / 1.417, 1 x 250 2.100 / 2.113, 1 x 380 3.177 / 3.156, 1 x 500
+// 3.341 / 3.283, 1 x 1000 4.649 / 4.493; more: 48 x 20 4.06 / 4.28, 60 x 60 7.64 / 7.94, 8 x 380 7.32 / 7.49, 5 x 700 7.80 / 7.89, 3 x 1000
+// 7.71 / 7.68, 2 x 1300 7.59 / 7.34, 1 x 2391 7.99 / 7.53.  24 bits, one round: 1 x 100 1.492 / 1.508, 1 x 150 1.890 / 1.877, 1 x 250 2.351 /
+// 2.256; more: 24 x 100 6.51 / 6.79, 8 x 380 7.80 / 7.83, 5 x 500 7.06 / 6.87, 1 x 2391 10.10 / 8.65.
+static bool attn_prefill_two(int wgs, int longest, bool lo) {
+    const int from = lo ? 160 : 384;
+    return wgs < 512 && longest >= (wgs > 256 ? from * 8 / 3 : from);
+}
 // prefill: n_tiles (a multiple of 4: every sequence's tile list padded with empty tiles) q-tiles of 2 sub-tiles each
 hipError_t launch_attn_prefill(const AttnArgs& a, int n_tiles, hipStream_t s) {
     if (n_tiles <= 0) return hipSuccess;
     if (a.kv.klo && !a.kv.vlo) return hipErrorInvalidValue;  // 24-bit K comes with 24-bit V only
     if (n_tiles % 4 || a.gqa < 1 || a.gqa > 16 || (a.kv.hd != 128 && a.kv.hd != 64)) return hipErrorInvalidValue;
-    // fewer workgroups than two for every CU: the tiles of a context on two sets of waves (measurements at the kernel)
     const int groups = n_tiles / 4;
-    const bool two = groups * a.kv.kv_l < 512;
+    const bool two = attn_prefill_two(groups * a.kv.kv_l, a.longest, a.kv.vlo);
     if (a.kv.hd == 128) return two ? attn_prefill_launch<128, 2>(a, groups, s) : attn_prefill_launch<128, 1>(a, groups, s);
     return two ? attn_prefill_launch<64, 2>(a, groups, s) : attn_prefill_launch<64, 1>(a, groups, s);
 }

@@ -274,6 +274,18 @@ def test_prefill_tile_gemm_equals_the_chunked_kernel(Ly, M, N, K, mode, packed):
 @pytest.mark.parametrize("B,T", [(1, 1), (1, 31), (1, 33), (1, 97), (3, 64), (2, 129), (1, 513), (40, 65), (70, 40)])
 @pytest.mark.parametrize("climb", [0.0, 40.0, -300.0])
 def test_prompt_attention_tiles_and_reference(Ly, oracle, rng, hd, B, T, climb):
+    check_prompt_attention(Ly, rng, hd, B, T, climb)
+
+
+# ... on both sides of where a q-tile's waves become two sets: by the length of the contexts within one round of the CUs and, with more
+# workgroups, by a longer one
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("B,T", [(1, 383), (1, 384), (1, 417), (4, 400), (6, 400), (3, 1023), (3, 1024), (2, 1089)])
+def test_prompt_attention_of_long_contexts(Ly, rng, hd, B, T):
+    check_prompt_attention(Ly, rng, hd, B, T, 40.0)
+
+
+def check_prompt_attention(Ly, rng, hd, B, T, climb):
     nh, kv = 16, 8
     q = rng.standard_normal((B, nh, T, hd)).astype(np.float32)
     k = rng.standard_normal((B, kv, T, hd)).astype(np.float16).astype(np.float32)
