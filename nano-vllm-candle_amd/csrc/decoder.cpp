@@ -86,7 +86,7 @@ int run_glu(nvllm_model* m, const GluPlan& g, const bf16_bits* xh, const bf16_bi
 
 int run_act(nvllm_model* m, const ProductPlan& p, nvllm::Act act, const bf16_bits* xh, const bf16_bits* xl, const PackedW& w, int R, bf16_bits* oh, bf16_bits* ol, int out_packed) {
     hipStream_t s = m->ctx->stream;
-    if (p.kind == P_TILE && gemm_tile_ok(R, w.N, w.K, 4 + act, m->opt_tile_min_wgs)) {
+    if (p.kind == P_TILE && gemm_tile_act_ok(R, w.N, w.K, act, m->opt_tile_min_wgs, p.max_split)) {
         PROF(m, PROF_GEMM, launch_gemm_tile(xh, xl, w, R, 4 + act, nullptr, oh, ol, out_packed, m->opt_tile_min_wgs, 1, nullptr, s));
         ++m->tile_launches;
     } else if (p.kind == P_ROW && gemm_rowdir_ok(w.N, w.K, 3 + act, R)) {

@@ -195,6 +195,7 @@ hipError_t launch_qk_norm_rope_kvwrite(const QkvArgs& a, int rows, hipStream_t s
 // xpack_off order); mode 4 + act: the activation of every feature as hi/lo planes [M][N].  min_wgs: smallest grid the kernel is used for (a 256-row tile needs many rows to fill 256 CUs).
 // hipErrorNotSupported = shape not covered.
 bool gemm_tile_ok(int M, int N, int K, int mode, int min_wgs);
+bool gemm_tile_act_ok(int M, int N, int K, int act, int min_wgs, int max_split);  // ... with the activation in the epilogue, and faster so
 // mode 0 with n_slabs != nullptr may split K (narrow outputs, 128-row blocks): out = [*n_slabs][M][N], up to max_split slabs
 int gemm_tile_splits(int M, int N, int K, int min_wgs, int max_split);  // 0 = shape not covered
 hipError_t launch_gemm_tile(const bf16_bits* xh, const bf16_bits* xl, const PackedW& w, int M, int mode, float* out,

@@ -501,12 +501,11 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
 // 1024 5.09 -> 4.98, from 1300 on the same; four prompts of 64 to 200 tokens of a 1024-wide decoder 0.929 -> 0.858.  Charged 60 % instead
 // they take over where they lose: 2391 tokens 7.62 -> 7.94, 18.7 k tokens 41.9 -> 44.8.
 // ntw == 0: not covered, or fewer than min_wgs workgroups.
-struct TileShape { int ntw = 0, wn = 0, ks = 1; };
+struct TileShape { int ntw = 0, wn = 0, ks = 1; double cost = 0; };
 static TileShape tile_shape(int M, int N, int K, int mode, int min_wgs, int max_split) {
     TileShape best;
     if (M < 1 || K % 64 != 0 || K < 128 || N % 32 != 0) return best;
     const int KT = K / 32;
-    double best_cost = 0;
     const int cand[4][2] = {{8, 2}, {6, 2}, {4, 4}, {2, 4}};
     for (const auto& c : cand) {
         const int ntw = c[0], wn = c[1], cols = wn * ntw * 16, rows = (8 / wn) * 64;
@@ -519,13 +518,24 @@ static TileShape tile_shape(int M, int N, int K, int mode, int min_wgs, int max_
             const double block_us = 4.0 * rows * cols * (double)(K / ks) / (2.5e15 * 0.5 / 256) * 1e6 * (ntw == 2 ? 2.0 : wn == 4 ? 1.25 : 1.0);
             const double slab_us = ks > 1 ? 2.0 * ks * (double)M * N * 4 / 4e12 * 1e6 : 0.0;
             const double cost = (double)((wgs + 255) / 256) * block_us + slab_us;
-            if (!best.ntw || cost < best_cost) { best.ntw = ntw; best.wn = wn; best.ks = ks; best_cost = cost; }
+            if (!best.ntw || cost < best.cost) best = TileShape{ntw, wn, ks, cost};
         }
     }
     return best;
 }
 
 bool gemm_tile_ok(int M, int N, int K, int mode, int min_wgs) { return tile_shape(M, N, K, mode, min_wgs, 1).ntw != 0; }
+// An activation in the epilogue wants the whole K in one workgroup.  Where splitting K would fill the chip instead, the product of f32 slabs
+// and a launch that sums them and applies the activation, about 5 us, can be the faster pair; by the cost above.  129 rows, N 4608, K 1024:
+// 72 workgroups, 27 us; N 9216, K 2048: 50.  Decode steps of decoders with these, always the epilogue and by this rule: 129 rows 0.891 ->
+// 0.870 and 0.761 -> 0.713 ms, 200 rows 1.095 -> 1.091 and 0.876 -> 0.839, 256 rows 1.275 -> 1.268 and 0.937 -> 0.905, 400 rows the same.
+// min_wgs 1 (whenever the shape fits) takes the epilogue.
+bool gemm_tile_act_ok(int M, int N, int K, int act, int min_wgs, int max_split) {
+    const TileShape one = tile_shape(M, N, K, 4 + act, min_wgs, 1);
+    if (!one.ntw || min_wgs == 1) return one.ntw != 0;
+    const TileShape split = tile_shape(M, N, K, 0, min_wgs, max_split);
+    return split.ks == 1 || one.cost <= split.cost + 5.0;
+}
 int gemm_tile_splits(int M, int N, int K, int min_wgs, int max_split) { return tile_shape(M, N, K, 0, min_wgs, max_split).ntw ? tile_shape(M, N, K, 0, min_wgs, max_split).ks : 0; }
 
 template <int NTW, int WN, int MODE>
