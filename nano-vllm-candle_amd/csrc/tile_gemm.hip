@@ -279,6 +279,8 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
     } else if constexpr (QKV) {
         static_assert(!QKV || (NTW == 8 && WN == 2), "one wave tile = one 128-wide head");
         const QkvArgs& q = a.q;
+        // the rows of the deferred norm below: compared as unsigned, the prologue's signed indices are not taken for the same values and kept
+        // (spilled, in MODE 9) through the K loop
         const int hh = wn == 0 ? nb : a.NB + nb;  // this wave's head: [q heads | k heads | v heads]
         const int nh = q.nh_l, kvl = q.kv.kv_l;
         // V heads: in the cache's PV fragment order TOKENS are the fast index (8 per 16-byte slot), while a lane here
@@ -301,7 +303,7 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
                 const int sh = P0 & 3;
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
-                    const float ri = rownorm_rinv(q.rn, min(row0 + b * 16 + l15, a.M - 1));
+                    const float ri = rownorm_rinv(q.rn, (int)min((unsigned)(row0 + b * 16 + l15), (unsigned)(a.M - 1)));
 #pragma unroll
                     for (int j = 0; j < 8; ++j)
 #pragma unroll
@@ -366,7 +368,7 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
                 constexpr int b = decltype(bc)::value;
                 const int row = row0 + b * 16 + l15;
                 const int pos = e_pos[b];
-                const float ri = rownorm_rinv(q.rn, min(row, a.M - 1));  // deferred input norm (1 when the planes were normalised)
+                const float ri = rownorm_rinv(q.rn, (int)min((unsigned)row, (unsigned)(a.M - 1)));  // deferred input norm (1 when the planes were normalised)
                 // whole-vector arithmetic on the f32x4 accumulators: hipcc pairs it into v_pk_mul / v_pk_fma (two lanes' worth
                 // of flops per instruction) -- this epilogue is VALU-bound (every wave of the chip is in it at once)
                 f32x4 ss4 = {0.f, 0.f, 0.f, 0.f};
