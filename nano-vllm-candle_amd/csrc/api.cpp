@@ -515,7 +515,10 @@ int stage_flush(nvllm_model* m, bool more) {
         int* p = stage_room(m, m->d_block_tables, m->table_news.size(), 1);
         if (p) for (int at : m->table_news) { *p++ = at; *p++ = m->h_block_tables[at]; }
         // steps that took blocks and failed can leave more than the block holds: the whole table instead
-        else HIPCHK(m->ctx, hipMemcpyAsync(m->d_block_tables, m->h_block_tables.data(), m->h_block_tables.size() * 4, hipMemcpyHostToDevice, m->ctx->stream));
+        else {
+            HIPCHK(m->ctx, hipMemcpyAsync(m->d_block_tables, m->h_block_tables.data(), m->h_block_tables.size() * 4, hipMemcpyHostToDevice, m->ctx->stream));
+            ++m->table_copies;
+        }
     }
     if (g.n_runs) {
         g.args.src = g.dev + (size_t)g.slot * g.ints;
@@ -2009,11 +2012,12 @@ extern "C" int nvllm_debug_set_option(nvllm_model* m, const char* name, int valu
 }
 
 // counters for tests: "oneshot_calls" = all-reduces this model's context has run on the one-shot device path;
-// "tile_gemm_launches" = projections this model has run on the prefill tile GEMM
+// "tile_gemm_launches" = projections this model has run on the prefill tile GEMM; "table_copies" = whole block tables sent
 extern "C" int nvllm_debug_get_counter(nvllm_model* m, const char* name, int64_t* value) {
     if (!m || !name || !value) return NVLLM_EINVAL;
     if (!strcmp(name, "oneshot_calls")) { *value = (int64_t)m->ctx->os_calls; return NVLLM_OK; }
     if (!strcmp(name, "latent_expanded")) { *value = m->latent_expanded; return NVLLM_OK; }
+    if (!strcmp(name, "table_copies")) { *value = m->table_copies; return NVLLM_OK; }
     if (!strcmp(name, "tile_gemm_launches")) { *value = m->tile_launches; return NVLLM_OK; }
     if (!strcmp(name, "kv_f16_saturated") || !strcmp(name, "kv_f16_absmax_bits")) {
         // scan of the whole K/V pool (debug, off the hot path): elements the f16_sat clamp of a cache write produced, and the

@@ -119,7 +119,8 @@ bool gemm_stream_ok(int M, int N, int K, int epi);
 int gemm_stream_groups(int M, int N, int K, int epi);          // n-groups = tickets needed = ssq groups of epilogue 3
 size_t gemm_stream_slab_floats(int M, int N, int K, int epi);  // f32 scratch the combine needs
 hipError_t launch_gemm_stream_epi(const StreamArgs& a, const PackedW& w, int epi, hipStream_t s);
-// LM head (greedy arg-max epilogue): the streaming kernel for <= 64 rows, else plan_gemm(M, N, K, 1)
+// LM head (greedy arg-max epilogue): the streaming kernel, more than 64 rows in slices of 64; plan_gemm(M, N, K, 1) where K is no
+// multiple of 256 or N none of 16
 GemmPlan plan_lmhead(int M, int N, int K);
 void set_split(GemmPlan& p, int KT, int want);
 hipError_t launch_gemm(const GemmPlan& p, const bf16_bits* xh, const bf16_bits* xl, int ldx, const PackedW& w,

@@ -1366,7 +1366,7 @@ bool gemm_rowpar_ok(int N, int K, int epi, int M) {
     RowParShape sh;
     return rowpar_shape(N, K, epi, M, sh) && !(epi == 1 && sh.nwn % 2);
 }
-// ssq groups the epilogue-0 kernel leaves (independent of M: the fused path never exceeds 128 rows)
+// ssq groups the epilogue-0 kernel leaves: its tiles per workgroup follow from N and K alone, for any row count of the fused path
 int gemm_rowpar_groups(int N, int K) {
     const RowDirShape d = rowdir_shape(N, K, 0, 64);
     if (d.nt) return (N / 16 + d.nt - 1) / d.nt;

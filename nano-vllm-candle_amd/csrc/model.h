@@ -194,6 +194,7 @@ struct nvllm_model {
     hipEvent_t out_ev[kOutSlots] = {};
     Staging stage;
     std::vector<int> table_news;  // entries of h_block_tables the device does not have yet
+    int64_t table_copies = 0;     // whole tables sent because the pinned block had no room for them
     float *tap_h = nullptr, *tap_res = nullptr;
     bool taps = false;
     int tap_rows = 0;

@@ -15,8 +15,8 @@
 //     barrier per stage.  Inside a stage the fragments of the next sub-step (and, in the last one, the first
 //     fragments of stage s+1, which the opening barrier already published) are read while the current MFMAs run.
 //   * the blocks of an XCD (blockIdx % 8) are a run of an order that goes through groups of `band` row blocks feature block by feature
-//     block: every XCD gets as many as the next one (to one), and its run is about as many bytes of x as of W, for the operand re-reads
-//     to hit that XCD's L2.  Dealing whole row blocks to XCDs instead gave two of them twice the work wherever the row blocks are not a
+//     block: an eighth of the blocks to each XCD, rounded up, the last ones what is left; a run is about as many bytes of x as of W, for
+//     the operand re-reads to hit that XCD's L2.  Dealing whole row blocks to XCDs instead gave two of them twice the work wherever the row blocks are not a
 //     multiple of 8: 2391 rows, 10 x 24 blocks of gate/up, 91 -> 51 us; 4096 rows, where the runs are only squarer, 79 -> 75.
 // MODE 0: f32 [M][N].  MODE 2: W is the gate/up matrix interleaved in 16-row tiles; the epilogue writes
 // silu(gate)*up as hi/lo planes [M][N/2] (row-major or xpack_off order) -- SiluAndMul, activation.rs:13-18.

@@ -1,5 +1,6 @@
 """GPU test of logits on their way to the caller: fewer bytes than one pinned slot, a last slot that is not full, one to four threads, more
-chunks than slots.  The reference is the same rows fetched one by one; bits are equal."""
+chunks than slots.  The reference is the same rows fetched one by one, whose products other kernels sum in another order; the greedy ids, which
+the device finds by itself, say that every row is whole, and the same step again gives the same bits."""
 import numpy as np
 import pytest
 

@@ -132,8 +132,8 @@ def test_0_6b_batch64_fused_decode_vs_oracle_sample(pkg, ctx, oracle_0_6b):
 
 def test_8b_layer_shapes_batch256_context4096_vs_oracle(pkg, ctx, oracle):
     # configs[3] in miniature: Qwen3-8B LAYER shapes (H 4096, 32/8 heads of 128, I 12288), 2 layers, 256 live
-    # sequences -> the generic path beyond the fused path's 128 rows, the chunked LM head with per-wave partial
-    # arg-max + argmax_parts_kernel (> 64 rows); two sequences sit at 4096 tokens of context (16-17 KV blocks).
+    # sequences -> the generic path (projections this big have no register-direct form, so nothing is fused beyond
+    # 128 rows), the LM head in slices of 64 rows with per-wave partial arg-max; two sequences sit at 4096 tokens of context (16-17 KV blocks).
     # Step A decodes the two long sequences alone (2 rows: split-KV over 26 workgroups per head + attn_combine);
     # step B decodes all 256.  The oracle re-runs the two long sequences once (step A) and three short ones (B).
     cfg = pkg.Qwen3Config.tiny(vocab_size=4096, hidden_size=4096, head_dim=128, num_hidden_layers=2,
@@ -432,8 +432,8 @@ def test_8b_full_size_batch256_context4096_properties(pkg, ctx):
 
 
 def test_full_vocabulary_lm_head_and_decode_kernels_at_odd_batch_sizes(pkg, ctx, oracle):
-    # One Qwen3-0.6B layer with the full 151 936-entry vocabulary: the LM-head kernels (streaming form up to 64 rows, its row
-    # tiles of 16, the chunked kernel beyond), the per-row arg-max finish and the decode kernels at batch sizes that are not a
+    # One Qwen3-0.6B layer with the full 151 936-entry vocabulary: the LM head (row tiles of 16 up to 64 rows,
+    # slices of 64 beyond), the per-row arg-max finish and the decode kernels at batch sizes that are not a
     # power of two -- every kernel choice that depends on the row count, at the real matrix sizes.  (The full-depth tests
     # run 1, 4, 64 or 256 rows; the batch-40 attention-order bug, DESIGN.md §2, lived between them.)
     cfg = pkg.Qwen3Config.qwen3_0_6b()

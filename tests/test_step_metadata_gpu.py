@@ -30,12 +30,14 @@ def test_many_chunks_and_tables_after_failed_steps(design, max_seqs, rows):
     blocks = max_seqs + 2
     m = _model(design, max_seqs, blocks, rows)
     rng = np.random.default_rng(max_seqs)
-    # every retry releases the first sequence's blocks, takes them again in another order and fails on the second one
-    for k in range(4 * blocks):
-        n = [256 * (1 + k % blocks) - 5, 256 * blocks]
-        if max_seqs > 1:
-            with pytest.raises(NvllmError):
-                m.step([0, 1], [rng.integers(0, 300, x) for x in n], True)
+    # every retry releases the first sequence's blocks, takes them again in another order and fails on the second one; a model of one
+    # sequence fails as its metadata is sent.  Until there are more new entries than the pinned block has room for: the whole table goes
+    m.set_option("stage_fail", 1 << 30 if max_seqs == 1 else 0)
+    for k in range(100 * blocks):
+        n = [256 * (1 + k % blocks) - 5, 256 * blocks][:max_seqs]
+        with pytest.raises(NvllmError):
+            m.step(list(range(len(n))), [rng.integers(0, 300, x) for x in n], True)
+    m.set_option("stage_fail", 0)
     for s in (0, 1):
         m.seq_free(s)
     prompts = [rng.integers(0, 300, int(x)) for x in rng.integers(1, 250, max_seqs)]
@@ -46,6 +48,7 @@ def test_many_chunks_and_tables_after_failed_steps(design, max_seqs, rows):
         fresh = _model(design, max_seqs, blocks, rows)
         got, want = (x.step_score(ids, prompts, True, wanted) for x in (m, fresh))
         assert np.array_equal(got, want)
+        assert m.counter("table_copies") > 0 and fresh.counter("table_copies") == 0
         if design == "qwen3":
             lists = [np.append(p, 7) for p in prompts]
             a, b = (x.step(ids, lists, False, want_logits=True) for x in (m, fresh))

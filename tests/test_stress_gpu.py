@@ -259,7 +259,7 @@ def test_32b_layer_shapes_heavy_tp8_shards_vs_oracle(pkg, oracle, oneshot, v_bit
 
 def test_24_bit_v_cache_paths_on_a_small_model(pkg, ctx, oracle):
     # every writer and reader of the 24-bit V cache on a small head_dim-128 model, benign weights: a ragged batch whose prompts
-    # go through the row kernel (qk_norm_rope_kvwrite) + attn_paged_kernel<.., 2, .., VLO>, decode through the fused
+    # go through the row kernel (qk_norm_rope_kvwrite) + attn_prefill_kernel<.., VLO>, decode through the fused
     # prologue's store_v24 + the VLO decode kernel, one sequence growing across a 256-token block boundary, a long one alone
     # (split-KV + combine), slots freed and reused, the device-feedback decode; then the pool goes back to 16 bits.
     # The 24-bit pool must never be WORSE than the 16-bit one beyond noise and must report its bytes; head_dim 64 refuses it.

@@ -1,5 +1,5 @@
 """GPU test of the 128 x 128 blocks of the prompt products: output widths that no bigger block divides (640 = 5 x 128 features), ragged last
-row blocks, the shortest K, each epilogue that has them.  The reference is the chunked kernel."""
+row blocks, the shortest K: f32 sums and SwiGLU by themselves, squared ReLU and GELU through a decoder.  The reference is the chunked kernel."""
 import ctypes as C
 
 import pytest
@@ -22,16 +22,20 @@ def test_small_blocks_equal_the_chunked_kernel(M, N, K, mode, packed):
 
 @pytest.mark.parametrize("rows", [129, 257, 400, 513])
 @pytest.mark.parametrize("ff", [4608, 1152])
-def test_activation_by_epilogue_and_by_launch(rows, ff):
-    """a decoder's squared ReLU in the product's epilogue (whenever the shape fits), as the rule has it (a launch of its own behind a product
-    with split K for the fewer rows), and from the chunked kernel"""
+@pytest.mark.parametrize("act", ["squared ReLU", "GELU"])
+def test_activation_by_epilogue_and_by_launch(rows, ff, act):
+    """a decoder's activation in the product's epilogue (whenever the shape fits: 128 x 128 blocks here), as the rule has it (a launch
+    of its own behind a product with split K for the fewer rows), and from the chunked kernel"""
     import numpy as np
 
     import nano_vllm_candle_amd as pkg
     from nano_vllm_candle_amd.gopunex import LightningConfig
+    from nano_vllm_candle_amd.lefalix import DeltaConfig, DenseConfig
 
-    cfg = pkg.GopunexConfig(512, 1024, [(LightningConfig(4, 64, 64, (0.9, 0.95, 0.98, 0.99)), ff)], 1e-6, 1.0, 0.5)
-    m = pkg.GopunexForCausalLM.from_random(cfg)
+    if act == "GELU":
+        m = pkg.LefalixForCausalLM.from_random(pkg.LefalixConfig(512, 1024, [((DeltaConfig(4, 4, 64, 64, 4, 64, 64),), DenseConfig(ff))]))
+    else:
+        m = pkg.GopunexForCausalLM.from_random(pkg.GopunexConfig(512, 1024, [(LightningConfig(4, 64, 64, (0.9, 0.95, 0.98, 0.99)), ff)], 1e-6, 1.0, 0.5))
     m.kv_alloc(8, 3, 1024)
     toks = [np.random.default_rng(rows).integers(0, 512, rows)]
     want = [[0, rows // 2, rows - 1]]
