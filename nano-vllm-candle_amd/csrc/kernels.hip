@@ -1752,7 +1752,7 @@ hipError_t launch_kv_write_plain(const float* k, const float* v, int rows, const
 // additive -1e9 mask for j>i (masked terms are exactly 0 after the f32 softmax, so they are skipped),
 // f32 softmax, p.v.  A KV cache is mathematically equivalent to the reference's full recompute (causal).
 //
-// One workgroup = one row (its gqa q-heads in the 16 MFMA rows; QT = 1) x one kv head.
+// One workgroup = one row (its gqa q-heads in the 16 MFMA rows) x one kv head.
 // Its 4 waves take alternate 32-token KV tiles; K and V fragments go straight from HBM to VGPRs:
 //   S^T[token][qrow]  = K[token][:] . q[qrow][:]      A = K frag (16 rows x 64 B per wave-load), B = q (f16 hi+lo)
 //   O^T[dim][qrow]   += V^T[dim][token] . P[token][qrow]   A = V packed frag (1 KiB wave-load), B = P straight
@@ -1795,16 +1795,15 @@ __device__ __forceinline__ long bf8_half(const uint4& w, int second) {
 
 // VLO: 0 = 16-bit cache, 1 = 24-bit V, 2 = 24-bit K and V (KvLayout::klo too: four more 1 KiB wave-loads per tile, one bf8 MFMA
 // per QK^T fragment against q in bf8)
-template <int HD, int QT, int NWV, bool FUSED, int VLO = 0>
+template <int HD, int NWV, bool FUSED, int VLO = 0>
 __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
-    static_assert(QT == 1, "one row of each head: decode (prompts: attn_prefill_kernel)");
     constexpr int DC = HD / 32, DT = HD / 16, DL = VLO ? DT / 2 : 1;  // DL: 1 KiB residual fragments per tile (two PV fragments each)
     constexpr bool KLO = VLO == 2;
     constexpr bool ONE_SET = VLO != 0;  // decode with a 24-bit cache: one tile set in flight per wave (see the loop)
     constexpr int RL = DL + (KLO ? DC : 0);  // residual registers per tile: V's DL, then K's [token half][DC / 2]
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-    float* ml = reinterpret_cast<float*>(smem_raw);                          // [NWV][QT][2][16]
-    f32x4* obuf = reinterpret_cast<f32x4*>(smem_raw + NWV * QT * 2 * 16 * 4);  // [NWV][QT][DT][64]
+    float* ml = reinterpret_cast<float*>(smem_raw);                          // [NWV][2][16]
+    f32x4* obuf = reinterpret_cast<f32x4*>(smem_raw + NWV * 2 * 16 * 4);  // [NWV][DT][64]
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l15 = lane & 15, grp = lane >> 4;
@@ -1850,17 +1849,14 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
     const int kv_l = a.kv.kv_l;
     const int ldq = a.nh_l * HD;
 
-    int my_row[QT], my_pos[QT];
+    int my_row, my_pos;
     const int my_head = kh * gqa + (l15 % gqa);
-#pragma unroll
-    for (int t = 0; t < QT; ++t) {
-        const int tok = t * tpq + l15 / gqa;
-        const bool valid = (l15 < tpq * gqa) && (tok < nrows);
-        my_row[t] = valid ? row0 + tok : -1;
-        if constexpr (!FUSED) my_pos[t] = valid ? a.pos[row0 + tok] : -1;
-    }
+    const int tok = l15 / gqa;
+    const bool valid = (l15 < tpq * gqa) && (tok < nrows);
+    my_row = valid ? row0 + tok : -1;
+    if constexpr (!FUSED) my_pos = valid ? a.pos[row0 + tok] : -1;
     const int pmax = a.pos[row0 + nrows - 1];
-    if constexpr (FUSED) my_pos[0] = pmax;  // uniform; what the lanes of no row (q = 0) sum up is never stored
+    if constexpr (FUSED) my_pos = pmax;  // uniform; what the lanes of no row (q = 0) sum up is never stored
     const int n_kv_tiles = (pmax >> 5) + 1;
     // split-KV (flash-decoding): workgroup blockIdx.z owns 32-token tiles [t_begin, t_end) and leaves an
     // un-normalised partial (m, l, O); every workgroup then has the same short dependent-load chain
@@ -1900,7 +1896,7 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
     // register sets: two 32-token tiles (32 KiB) of this wave are in flight at any time
     uint4 kaA[DC], kbA[DC], vfA[DT], kaB[DC], kbB[DC], vfB[DT];
     uint4 vlA[RL], vlB[RL];
-    f16x8 qh[QT][DC], ql[QT][DC];
+    f16x8 qh[DC], ql[DC];
     // fused decode: the new token's K and V, and the residual bytes of both, from the wave whose tile it falls into to that wave's lanes
     // (over obuf, which nobody writes before every wave is through its tiles)
     _Float16* new_k = reinterpret_cast<_Float16*>(obuf);
@@ -1990,10 +1986,10 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
                 const float y1 = (n1 * cs[c][j] - n2 * sn[c][j]) * a.q_scale;
                 const float y2 = (n2 * cs[c][j] + n1 * sn[c][j]) * a.q_scale;
                 const _Float16 h1 = (_Float16)y1, h2 = (_Float16)y2;
-                qh[0][c][j] = h1;
-                ql[0][c][j] = (_Float16)(y1 - (float)h1);
-                qh[0][c + DC / 2][j] = h2;
-                ql[0][c + DC / 2][j] = (_Float16)(y2 - (float)h2);
+                qh[c][j] = h1;
+                ql[c][j] = (_Float16)(y1 - (float)h1);
+                qh[c + DC / 2][j] = h2;
+                ql[c + DC / 2][j] = (_Float16)(y2 - (float)h2);
             }
         }
         // ---- K / V of the new token
@@ -2029,116 +2025,104 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
         NVLLM_STAMP(a, 2);  // no barrier in between any more: the loop's segment starts here
     } else {
 #pragma unroll
-        for (int t = 0; t < QT; ++t)
-#pragma unroll
-            for (int c = 0; c < DC; ++c) {
-                float x[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-                if (my_row[t] >= 0) {
-                    const float4* p = reinterpret_cast<const float4*>(a.q + (size_t)my_row[t] * ldq + (size_t)my_head * HD +
-                                                                      c * 32 + grp * 8);
-                    const float4 u = p[0], w = p[1];
-                    x[0] = u.x; x[1] = u.y; x[2] = u.z; x[3] = u.w; x[4] = w.x; x[5] = w.y; x[6] = w.z; x[7] = w.w;
-                }
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const _Float16 h = (_Float16)x[j];
-                    qh[t][c][j] = h;
-                    ql[t][c][j] = (_Float16)(x[j] - (float)h);
-                }
+        for (int c = 0; c < DC; ++c) {
+            float x[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+            if (my_row >= 0) {
+                const float4* p = reinterpret_cast<const float4*>(a.q + (size_t)my_row * ldq + (size_t)my_head * HD +
+                                                                  c * 32 + grp * 8);
+                const float4 u = p[0], w = p[1];
+                x[0] = u.x; x[1] = u.y; x[2] = u.z; x[3] = u.w; x[4] = w.x; x[5] = w.y; x[6] = w.z; x[7] = w.w;
             }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const _Float16 h = (_Float16)x[j];
+                qh[c][j] = h;
+                ql[c][j] = (_Float16)(x[j] - (float)h);
+            }
+        }
     }
 
     // 24-bit K: q once more as bf8 (the B operand of the residual MFMA; two mantissa bits leave that 2^-12-sized term 12 % accurate)
-    [[maybe_unused]] long q8[QT][DC];
+    [[maybe_unused]] long q8[DC];
     if constexpr (KLO) {
 #pragma unroll
-        for (int t = 0; t < QT; ++t)
-#pragma unroll
-            for (int c = 0; c < DC; ++c) q8[t][c] = bf8x8(qh[t][c]);
+        for (int c = 0; c < DC; ++c) q8[c] = bf8x8(qh[c]);
     }
-    f32x4 o[QT][DT];
-    float m[QT], lsum[QT];
+    f32x4 o[DT];
+    float m = -1e30f, lsum = 0.f;
 #pragma unroll
-    for (int t = 0; t < QT; ++t) {
-        m[t] = -1e30f;
-        lsum[t] = 0.f;
-#pragma unroll
-        for (int d = 0; d < DT; ++d) o[t][d] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int d = 0; d < DT; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     auto compute_tile = [&](int kt, const uint4 (&ka)[DC], const uint4 (&kb2)[DC], const uint4 (&vf)[DT], const uint4 (&vl)[RL]) {
         const int T0 = kt << 5;
         const int tokA = T0 + grp * 4, tokB = T0 + 16 + grp * 4;
+        f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int t = 0; t < QT; ++t) {
-            f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int c = 0; c < DC; ++c) {
-                const f16x8 fa = __builtin_bit_cast(f16x8, ka[c]);
-                const f16x8 fb = __builtin_bit_cast(f16x8, kb2[c]);
-                sa = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa, qh[t][c], sa, 0, 0, 0);
-                sa = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa, ql[t][c], sa, 0, 0, 0);
-                sb = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb, qh[t][c], sb, 0, 0, 0);
-                sb = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb, ql[t][c], sb, 0, 0, 0);
-                if constexpr (KLO) {  // the K residual bytes are bf8 numbers: A operands as they are
-                    const uint4 pa = vl[DL + (c >> 1)], pb = vl[DL + DC / 2 + (c >> 1)];
-                    const unsigned long long la = (c & 1) ? ((unsigned long long)pa.w << 32) | pa.z : ((unsigned long long)pa.y << 32) | pa.x;
-                    const unsigned long long lb = (c & 1) ? ((unsigned long long)pb.w << 32) | pb.z : ((unsigned long long)pb.y << 32) | pb.x;
-                    mfma_result_settled(sa);
-                    mfma_result_settled(sb);
-                    sa = __builtin_amdgcn_mfma_f32_16x16x32_bf8_bf8((long)la, q8[t][c], sa, 0, 0, 0);
-                    sb = __builtin_amdgcn_mfma_f32_16x16x32_bf8_bf8((long)lb, q8[t][c], sb, 0, 0, 0);
-                    mfma_result_settled(sa);  // ... and the next chunk's f16 MFMAs read these as SrcC
-                    mfma_result_settled(sb);
-                }
+        for (int c = 0; c < DC; ++c) {
+            const f16x8 fa = __builtin_bit_cast(f16x8, ka[c]);
+            const f16x8 fb = __builtin_bit_cast(f16x8, kb2[c]);
+            sa = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa, qh[c], sa, 0, 0, 0);
+            sa = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa, ql[c], sa, 0, 0, 0);
+            sb = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb, qh[c], sb, 0, 0, 0);
+            sb = __builtin_amdgcn_mfma_f32_16x16x32_f16(fb, ql[c], sb, 0, 0, 0);
+            if constexpr (KLO) {  // the K residual bytes are bf8 numbers: A operands as they are
+                const uint4 pa = vl[DL + (c >> 1)], pb = vl[DL + DC / 2 + (c >> 1)];
+                const unsigned long long la = (c & 1) ? ((unsigned long long)pa.w << 32) | pa.z : ((unsigned long long)pa.y << 32) | pa.x;
+                const unsigned long long lb = (c & 1) ? ((unsigned long long)pb.w << 32) | pb.z : ((unsigned long long)pb.y << 32) | pb.x;
+                mfma_result_settled(sa);
+                mfma_result_settled(sb);
+                sa = __builtin_amdgcn_mfma_f32_16x16x32_bf8_bf8((long)la, q8[c], sa, 0, 0, 0);
+                sb = __builtin_amdgcn_mfma_f32_16x16x32_bf8_bf8((long)lb, q8[c], sb, 0, 0, 0);
+                mfma_result_settled(sa);  // ... and the next chunk's f16 MFMAs read these as SrcC
+                mfma_result_settled(sb);
             }
-            float mt = -1e30f;
+        }
+        float mt = -1e30f;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                if (tokA + r <= my_pos[t]) mt = fmaxf(mt, sa[r]);
-                if (tokB + r <= my_pos[t]) mt = fmaxf(mt, sb[r]);
-            }
-            mt = fmaxf(mt, __shfl_xor(mt, 16));
-            mt = fmaxf(mt, __shfl_xor(mt, 32));
-            const float mn = fmaxf(m[t], mt);
-            const float alpha = exp2f(m[t] - mn);
-            m[t] = mn;
-            // P as f16 hi + f16 lo (22 bits): a second P.V MFMA per fragment, free in an HBM-bound kernel.  A single f16 P
-            // carries 2^-12 of rounding noise per probability, whose realisation depends on how the context is walked
-            // (waves, split-KV parts): at 4097 tokens of context that alone moved the logits by 4e-4 over 8 layers
-            // (tools/dbg_alone_vs_batch.py).
-            f16x8 P, Pl;
-            float ps = 0.f;
+        for (int r = 0; r < 4; ++r) {
+            if (tokA + r <= my_pos) mt = fmaxf(mt, sa[r]);
+            if (tokB + r <= my_pos) mt = fmaxf(mt, sb[r]);
+        }
+        mt = fmaxf(mt, __shfl_xor(mt, 16));
+        mt = fmaxf(mt, __shfl_xor(mt, 32));
+        const float mn = fmaxf(m, mt);
+        const float alpha = exp2f(m - mn);
+        m = mn;
+        // P as f16 hi + f16 lo (22 bits): a second P.V MFMA per fragment, free in an HBM-bound kernel.  A single f16 P
+        // carries 2^-12 of rounding noise per probability, whose realisation depends on how the context is walked
+        // (waves, split-KV parts): at 4097 tokens of context that alone moved the logits by 4e-4 over 8 layers
+        // (tools/dbg_alone_vs_batch.py).
+        f16x8 P, Pl;
+        float ps = 0.f;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float pa = (tokA + r <= my_pos[t]) ? exp2f(sa[r] - mn) : 0.f;
-                const float pb = (tokB + r <= my_pos[t]) ? exp2f(sb[r] - mn) : 0.f;
-                ps += pa + pb;
-                P[r] = (_Float16)pa;
-                P[4 + r] = (_Float16)pb;
-                Pl[r] = (_Float16)(pa - (float)P[r]);
-                Pl[4 + r] = (_Float16)(pb - (float)P[4 + r]);
-            }
-            lsum[t] = lsum[t] * alpha + ps;
-            [[maybe_unused]] long P8 = 0;
-            if constexpr (VLO) P8 = bf8x8(P);
+        for (int r = 0; r < 4; ++r) {
+            const float pa = (tokA + r <= my_pos) ? exp2f(sa[r] - mn) : 0.f;
+            const float pb = (tokB + r <= my_pos) ? exp2f(sb[r] - mn) : 0.f;
+            ps += pa + pb;
+            P[r] = (_Float16)pa;
+            P[4 + r] = (_Float16)pb;
+            Pl[r] = (_Float16)(pa - (float)P[r]);
+            Pl[4 + r] = (_Float16)(pb - (float)P[4 + r]);
+        }
+        lsum = lsum * alpha + ps;
+        [[maybe_unused]] long P8 = 0;
+        if constexpr (VLO) P8 = bf8x8(P);
 #pragma unroll
-            for (int d = 0; d < DT; ++d) {
-                f32x4 acc = o[t][d];
-                acc[0] *= alpha; acc[1] *= alpha; acc[2] *= alpha; acc[3] *= alpha;
-                const f16x8 fv = __builtin_bit_cast(f16x8, vf[d]);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(fv, P, acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(fv, Pl, acc, 0, 0, 0);
-                // the residual bytes ARE bf8 (e5m2) numbers: one fp8-family MFMA against P in bf8 adds the 2^-12-sized term
-                // (P's two mantissa bits leave it 12 % accurate: 2^-15 of V) without unpacking anything
-                if constexpr (VLO) {
-                    const uint4 pr = vl[d >> 1];
-                    const unsigned long long lo8 = (d & 1) ? ((unsigned long long)pr.w << 32) | pr.z : ((unsigned long long)pr.y << 32) | pr.x;
-                    mfma_result_settled(acc);
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf8_bf8((long)lo8, P8, acc, 0, 0, 0);
-                }
-                o[t][d] = acc;
+        for (int d = 0; d < DT; ++d) {
+            f32x4 acc = o[d];
+            acc[0] *= alpha; acc[1] *= alpha; acc[2] *= alpha; acc[3] *= alpha;
+            const f16x8 fv = __builtin_bit_cast(f16x8, vf[d]);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(fv, P, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(fv, Pl, acc, 0, 0, 0);
+            // the residual bytes ARE bf8 (e5m2) numbers: one fp8-family MFMA against P in bf8 adds the 2^-12-sized term
+            // (P's two mantissa bits leave it 12 % accurate: 2^-15 of V) without unpacking anything
+            if constexpr (VLO) {
+                const uint4 pr = vl[d >> 1];
+                const unsigned long long lo8 = (d & 1) ? ((unsigned long long)pr.w << 32) | pr.z : ((unsigned long long)pr.y << 32) | pr.x;
+                mfma_result_settled(acc);
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf8_bf8((long)lo8, P8, acc, 0, 0, 0);
             }
+            o[d] = acc;
         }
     };
     {
@@ -2220,77 +2204,60 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
 
     // combine the NWV waves' partial (m, l, O)
     NVLLM_STAMP(a, 3);
-#pragma unroll
-    for (int t = 0; t < QT; ++t) {
-        float l = lsum[t];
-        l += __shfl_xor(l, 16);
-        l += __shfl_xor(l, 32);
-        lsum[t] = l;
-        if (grp == 0) {
-            ml[((wave * QT + t) * 2 + 0) * 16 + l15] = m[t];
-            ml[((wave * QT + t) * 2 + 1) * 16 + l15] = l;
-        }
+    lsum += __shfl_xor(lsum, 16);
+    lsum += __shfl_xor(lsum, 32);
+    if (grp == 0) {
+        ml[(wave * 2 + 0) * 16 + l15] = m;
+        ml[(wave * 2 + 1) * 16 + l15] = lsum;
     }
     __syncthreads();
-    float ltot[QT];
+    float ms = -1e30f;
 #pragma unroll
-    for (int t = 0; t < QT; ++t) {
-        float ms = -1e30f;
+    for (int w = 0; w < NWV; ++w) ms = fmaxf(ms, ml[(w * 2 + 0) * 16 + l15]);
+    float ltot = 0.f;
 #pragma unroll
-        for (int w = 0; w < NWV; ++w) ms = fmaxf(ms, ml[((w * QT + t) * 2 + 0) * 16 + l15]);
-        float lt = 0.f;
+    for (int w = 0; w < NWV; ++w)
+        ltot += ml[(w * 2 + 1) * 16 + l15] * exp2f(ml[(w * 2 + 0) * 16 + l15] - ms);
+    const float f = exp2f(m - ms);
 #pragma unroll
-        for (int w = 0; w < NWV; ++w)
-            lt += ml[((w * QT + t) * 2 + 1) * 16 + l15] * exp2f(ml[((w * QT + t) * 2 + 0) * 16 + l15] - ms);
-        ltot[t] = lt;
-        const float f = exp2f(m[t] - ms);
-#pragma unroll
-        for (int d = 0; d < DT; ++d) {
-            o[t][d][0] *= f; o[t][d][1] *= f; o[t][d][2] *= f; o[t][d][3] *= f;
-        }
+    for (int d = 0; d < DT; ++d) {
+        o[d][0] *= f; o[d][1] *= f; o[d][2] *= f; o[d][3] *= f;
     }
     // every wave publishes its rescaled O; then wave w sums dim-tiles w, w+NWV, ... over all waves
 #pragma unroll
-    for (int t = 0; t < QT; ++t)
-#pragma unroll
-        for (int d = 0; d < DT; ++d) obuf[((wave * QT + t) * DT + d) * 64 + lane] = o[t][d];
+    for (int d = 0; d < DT; ++d) obuf[(wave * DT + d) * 64 + lane] = o[d];
     __syncthreads();
     const int n_parts = a.part_tiles ? (n_kv_tiles + a.part_tiles - 1) / a.part_tiles : 1;
-#pragma unroll
-    for (int t = 0; t < QT; ++t) {
-        if (my_row[t] < 0) continue;
-        const size_t base = (size_t)my_row[t] * ldq + (size_t)my_head * HD + grp * 4;
+    if (my_row >= 0) {
+        const size_t base = (size_t)my_row * ldq + (size_t)my_head * HD + grp * 4;
         for (int d = wave; d < DT; d += NWV) {
             f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int w = 0; w < NWV; ++w) {
-                const f32x4 v = obuf[((w * QT + t) * DT + d) * 64 + lane];
+                const f32x4 v = obuf[(w * DT + d) * 64 + lane];
                 acc[0] += v[0]; acc[1] += v[1]; acc[2] += v[2]; acc[3] += v[3];
             }
             if (n_parts > 1) {
                 // partial: O (at the workgroup's max) for the combine kernel
-                float* po = a.part_o + (((size_t)my_row[t] * a.nh_l + my_head) * a.max_parts + blockIdx.z) * HD + d * 16 + grp * 4;
+                float* po = a.part_o + (((size_t)my_row * a.nh_l + my_head) * a.max_parts + blockIdx.z) * HD + d * 16 + grp * 4;
                 *reinterpret_cast<float4*>(po) = make_float4(acc[0], acc[1], acc[2], acc[3]);
                 continue;
             }
-            const float inv = 1.0f / ltot[t];
+            const float inv = 1.0f / ltot;
             const float y0 = acc[0] * inv, y1 = acc[1] * inv, y2 = acc[2] * inv, y3 = acc[3] * inv;
             if (a.out_f32) *reinterpret_cast<float4*>(a.out_f32 + base + d * 16) = make_float4(y0, y1, y2, y3);
             if (a.out_hi) {
                 uint16_t h0, h1, h2, h3, l0, l1, l2, l3;
                 split_bf16(y0, h0, l0); split_bf16(y1, h1, l1); split_bf16(y2, h2, l2); split_bf16(y3, h3, l3);
-                const size_t xo = a.out_packed ? xpack_off(my_row[t], my_head * HD + d * 16 + grp * 4, ldq >> 5) : base + d * 16;
+                const size_t xo = a.out_packed ? xpack_off(my_row, my_head * HD + d * 16 + grp * 4, ldq >> 5) : base + d * 16;
                 *reinterpret_cast<uint2*>(a.out_hi + xo) = make_uint2(h0 | ((uint32_t)h1 << 16), h2 | ((uint32_t)h3 << 16));
                 *reinterpret_cast<uint2*>(a.out_lo + xo) = make_uint2(l0 | ((uint32_t)l1 << 16), l2 | ((uint32_t)l3 << 16));
             }
         }
         if (n_parts > 1 && wave == 0 && grp == 0) {
-            float ms = -1e30f;
-#pragma unroll
-            for (int w = 0; w < NWV; ++w) ms = fmaxf(ms, ml[((w * QT + t) * 2 + 0) * 16 + l15]);
-            float* pm = a.part_ml + (((size_t)my_row[t] * a.nh_l + my_head) * a.max_parts + blockIdx.z) * 2;
+            float* pm = a.part_ml + (((size_t)my_row * a.nh_l + my_head) * a.max_parts + blockIdx.z) * 2;
             pm[0] = ms;
-            pm[1] = ltot[t];
+            pm[1] = ltot;
         }
     }
     NVLLM_STAMP(a, 4);
@@ -2686,25 +2653,25 @@ __global__ void __launch_bounds__(256) attn_combine_kernel(AttnArgs a, int rows)
     }
 }
 
-template <int HD, int QT, int NWV, bool FUSED, int VLO>
+template <int HD, int NWV, bool FUSED, int VLO>
 static hipError_t attn_launch_v(const AttnArgs& a, int n_tiles, int grid_z, hipStream_t s) {
     constexpr int DT = HD / 16;
-    const size_t lds = (size_t)NWV * QT * 2 * 16 * 4 + (size_t)NWV * QT * DT * 64 * 16;
+    const size_t lds = (size_t)NWV * 2 * 16 * 4 + (size_t)NWV * DT * 64 * 16;
     static std::atomic<uint64_t> lds_set{0};
-    ensure_dyn_lds(reinterpret_cast<const void*>(attn_paged_kernel<HD, QT, NWV, FUSED, VLO>), lds, lds_set);
+    ensure_dyn_lds(reinterpret_cast<const void*>(attn_paged_kernel<HD, NWV, FUSED, VLO>), lds, lds_set);
     dim3 grid = FUSED ? dim3(a.kv.kv_l, n_tiles, grid_z) : dim3(n_tiles * a.kv.kv_l, 1, grid_z);
-    attn_paged_kernel<HD, QT, NWV, FUSED, VLO><<<grid, NWV * 64, lds, s>>>(a);
+    attn_paged_kernel<HD, NWV, FUSED, VLO><<<grid, NWV * 64, lds, s>>>(a);
     return hipGetLastError();
 }
-template <int HD, int QT, int NWV, bool FUSED>
+template <int HD, int NWV, bool FUSED>
 static hipError_t attn_launch_t(const AttnArgs& a, int n_tiles, int grid_z, hipStream_t s) {
     // 24-bit V (KvLayout::vlo) is served for head_dim 128 only (every Qwen3 size); the pool refuses it otherwise
     if (a.kv.klo && !a.kv.vlo) return hipErrorInvalidValue;  // 24-bit K comes with 24-bit V only
     if constexpr (HD == 128) {
-        if (a.kv.klo) return attn_launch_v<HD, QT, NWV, FUSED, 2>(a, n_tiles, grid_z, s);
-        if (a.kv.vlo) return attn_launch_v<HD, QT, NWV, FUSED, 1>(a, n_tiles, grid_z, s);
+        if (a.kv.klo) return attn_launch_v<HD, NWV, FUSED, 2>(a, n_tiles, grid_z, s);
+        if (a.kv.vlo) return attn_launch_v<HD, NWV, FUSED, 1>(a, n_tiles, grid_z, s);
     } else if (a.kv.vlo) return hipErrorNotSupported;
-    return attn_launch_v<HD, QT, NWV, FUSED, 0>(a, n_tiles, grid_z, s);
+    return attn_launch_v<HD, NWV, FUSED, 0>(a, n_tiles, grid_z, s);
 }
 
 template <int HD, int NH, int VLO>
@@ -2759,8 +2726,8 @@ hipError_t launch_attn_paged(const AttnArgs& a, int n_tiles, int rows, int n_par
     hipError_t e = hipErrorInvalidValue;
     const bool fused = a.qkv != nullptr;  // decode rows straight from the QKV GEMM's slabs
     if (fused && (n_tiles != rows || rows > kAttnFusedMaxRows)) return hipErrorInvalidValue;  // fused decode: tile i is row i
-    if (a.kv.hd == 128) e = fused ? attn_launch_t<128, 1, 4, true>(b, n_tiles, gz, s) : attn_launch_t<128, 1, 4, false>(b, n_tiles, gz, s);
-    else if (a.kv.hd == 64) e = fused ? attn_launch_t<64, 1, 4, true>(b, n_tiles, gz, s) : attn_launch_t<64, 1, 4, false>(b, n_tiles, gz, s);
+    if (a.kv.hd == 128) e = fused ? attn_launch_t<128, 4, true>(b, n_tiles, gz, s) : attn_launch_t<128, 4, false>(b, n_tiles, gz, s);
+    else if (a.kv.hd == 64) e = fused ? attn_launch_t<64, 4, true>(b, n_tiles, gz, s) : attn_launch_t<64, 4, false>(b, n_tiles, gz, s);
     if (e != hipSuccess || !split) return e;
     const int items = rows * a.nh_l;
     if (a.kv.hd == 128) attn_combine_kernel<128><<<(items + 3) / 4, 256, 0, s>>>(b, rows);
