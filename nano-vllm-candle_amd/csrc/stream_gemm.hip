@@ -59,7 +59,8 @@ __global__ void __launch_bounds__(NW * 64) gemm_stream_kernel(StreamArgs a, cons
 #pragma unroll
     for (int i = 0; i < PER_WAVE; ++i) {
         const int f = min(wave + i * NW, FRAGS - 1), kst = f % KC, pb = f / KC, b = pb % MT;
-        xoff[i] = a.x_packed ? (unsigned)((b * (a.ldx >> 5) + kt_begin + kst) * 512 + lane * 8)
+        // past the last row block, the last one again (its products are not stored): the planes may end there
+        xoff[i] = a.x_packed ? (unsigned)((min(b, (M - 1) >> 4) * (a.ldx >> 5) + kt_begin + kst) * 512 + lane * 8)
                              : (unsigned)min(b * 16 + l15, M - 1) * (unsigned)a.ldx + (unsigned)((kt_begin + kst) * 32 + grp * 8);
     }
     f32x4 acc[NT][MT];

@@ -29,3 +29,21 @@ def test_rows_of_a_batch_equal_the_rows_alone(hidden, inter, heads, kv, combine)
                 assert np.abs(got[i] - want).max() < 2.0 ** -11 * np.abs(want).max(), (rows, i)
         assert np.isfinite(got).all()
     m.close()
+
+
+@pytest.mark.parametrize("rows", [17, 33, 40, 48])
+def test_planes_that_end_with_the_batch(rows):
+    """a pool of as many rows as the batch has: row blocks past the planes are not read, and nothing else is"""
+    import nano_vllm_candle_amd as pkg
+
+    cfg = pkg.Qwen3Config.tiny(hidden_size=4096, intermediate_size=12288, num_attention_heads=32, num_key_value_heads=8, head_dim=128, num_hidden_layers=1)
+    m = pkg.Qwen3ForCausalLM.from_synthetic(cfg, 3)
+    seqs = [np.random.default_rng(i).integers(0, cfg.vocab_size, 1 + i % 3) for i in range(rows)]
+    out = []
+    for most in (rows, 256):
+        m.kv_alloc(rows, rows, most)
+        for i, s in enumerate(seqs):  # one by one: the same cache in both pools
+            m.step([i], [s], True)
+        out.append(m.step(list(range(rows)), [np.append(s, 5) for s in seqs], False, want_logits=True)[1])
+    m.close()
+    assert np.array_equal(out[0], out[1])
