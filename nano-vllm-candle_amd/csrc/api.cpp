@@ -1196,6 +1196,7 @@ static int forward_chunk_fused(nvllm_model* m, const FusedPlan& fp, int R, int n
         if (qt == 1 && R <= m->max_seqs) {
             aa.part_tiles = m->attn_part_tiles; aa.max_parts = kAttnMaxParts; aa.part_o = m->attn_po; aa.part_ml = m->attn_pml;
             parts_max = m->attn_parts_max;
+            if (fuse_qk) aa.waves = m->attn_waves;
         }
         PROF(m, PROF_EMPTY, hipSuccess);  // calibration: an event pair around nothing, at the attention launch's place
         STAMPS(aa, m);
@@ -1354,6 +1355,7 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
         if (qt == 1 && R <= m->max_seqs) {  // decode rows: split the context over workgroups
             aa.part_tiles = m->attn_part_tiles; aa.max_parts = kAttnMaxParts; aa.part_o = m->attn_po; aa.part_ml = m->attn_pml;
             parts_max = m->attn_parts_max;
+            if (fuse_qk) aa.waves = m->attn_waves;
         }
         STAMPS(aa, m);
         if (qt == 2) PROF(m, PROF_ATTN, launch_attn_prefill(aa, n_tiles, s));
@@ -1450,14 +1452,20 @@ static int ensure_blocks(nvllm_model* m, SeqState& s, int len) {
 
 // Split a sequence's context over several workgroups only when (sequences x kv heads) alone cannot fill
 // the chip (small batches, long contexts); a full batch already has >= 2 workgroups per CU.
+// Launches of up to 256 workgroups leave a CU one of them: eight waves instead of four halve its chain of tiles, the registers allow no more.
+// Attention and its combine pass, us a layer, four waves / eight.  0.6B (8 kv heads): 8 rows of 64 to 1500 tokens 18.1 / 16.8, 16 of 100 to 800
+// 18.0 / 16.4, 24 of 64 to 512 17.3 / 14.7, 32 of 64 to 512 19.3 / 15.5, 32 of 131 to 1500 31.5 / 27.7, one of 2000 15.3 / 13.9, of 900 12.0 /
+// 12.3, of 400 11.5 / 11.6, of 137 8.4 / 8.8; 24 with a 24-bit cache 20.1 / 17.3; 8B: 16 of 64 to 600 16.2 / 14.2, 24 of 256 to 2048 32.2 / 33.1.
 static void set_attn_split(nvllm_model* m, int n_seqs, int max_len) {
     const int tiles = (max_len + 31) / 32;
     const int base_wgs = std::max(1, n_seqs * m->kv_l);
-    int want = std::min(kAttnMaxParts, std::max(1, 512 / base_wgs));
-    // <= 256 tokens: four waves hold the whole context in one round; <= 512: two more rounds of the loop (~2.6 us) still cost
-    // less than the combine launch and its boundary (4.7 + 1.4 us, batch-1 profile)
-    if (tiles <= 16) want = 1;
-    int part = std::max(4, (tiles + want - 1) / want);  // >= 128 tokens per workgroup
+    const bool eight = m->hd == 128 && base_wgs <= 256 && tiles > (base_wgs < 64 ? 8 : 4);
+    m->attn_waves = eight ? 8 : 4;
+    int want = std::min(kAttnMaxParts, std::max(1, (eight ? 256 : 512) / base_wgs));
+    // a few more rounds of the loop cost less than the combine launch and its boundary (4.7 + 1.4 us): up to 512 tokens, and up to 1024 where
+    // there would be two parts at most (16 rows of 100 to 800, in parts 17.5 us, whole 16.4; one row of 900 12.3 and 16.9)
+    if (tiles <= (eight && base_wgs >= 128 ? 32 : 16)) want = 1;
+    int part = std::max(eight ? 8 : 4, (tiles + want - 1) / want);  // a tile of every wave at least
     m->attn_part_tiles = part;
     m->attn_parts_max = (tiles + part - 1) / part;
 }

@@ -1753,7 +1753,7 @@ hipError_t launch_kv_write_plain(const float* k, const float* v, int rows, const
 // f32 softmax, p.v.  A KV cache is mathematically equivalent to the reference's full recompute (causal).
 //
 // One workgroup = one row (its gqa q-heads in the 16 MFMA rows) x one kv head.
-// Its 4 waves take alternate 32-token KV tiles; K and V fragments go straight from HBM to VGPRs:
+// Its 4 or 8 waves (8: launches of one workgroup per CU at most) take alternate 32-token KV tiles; K and V fragments go straight from HBM to VGPRs:
 //   S^T[token][qrow]  = K[token][:] . q[qrow][:]      A = K frag (16 rows x 64 B per wave-load), B = q (f16 hi+lo)
 //   O^T[dim][qrow]   += V^T[dim][token] . P[token][qrow]   A = V packed frag (1 KiB wave-load), B = P straight
 //                                                          from the S accumulators (no lane movement)
@@ -1802,8 +1802,16 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
     constexpr bool ONE_SET = VLO != 0;  // decode with a 24-bit cache: one tile set in flight per wave (see the loop)
     constexpr int RL = DL + (KLO ? DC : 0);  // residual registers per tile: V's DL, then K's [token half][DC / 2]
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
-    float* ml = reinterpret_cast<float*>(smem_raw);                          // [NWV][2][16]
-    f32x4* obuf = reinterpret_cast<f32x4*>(smem_raw + NWV * 2 * 16 * 4);  // [NWV][DT][64]
+    // [NWV][2][16] m and l of the waves; [NWV][columns][HD] their O; fused: q as f16 hi and lo [2][gqa][HD], the new token's K and V and the
+    // residual bytes of both
+    float* ml = reinterpret_cast<float*>(smem_raw);
+    const int cols = FUSED ? a.gqa : 16;  // MFMA columns that are rows of q
+    f32x4* obuf = reinterpret_cast<f32x4*>(smem_raw + NWV * 2 * 16 * 4);
+    [[maybe_unused]] const int q_at = NWV * (2 * 16 * 4 + cols * HD * 4), new_at = q_at + cols * HD * 4;  // bytes
+    // (offsets, not pointers to choose between: the compiler must see that every access is to LDS, a generic one would wait for the tiles)
+    [[maybe_unused]] auto lds16 = [&](int byte) { return reinterpret_cast<_Float16*>(smem_raw + byte); };
+    [[maybe_unused]] auto lds8 = [&](int byte) { return reinterpret_cast<uint8_t*>(smem_raw + byte); };
+    [[maybe_unused]] const int new_v_at = new_at + HD * 2, new_kl_at = new_at + HD * 4, new_vl_at = new_at + HD * 5;
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l15 = lane & 15, grp = lane >> 4;
@@ -1827,19 +1835,28 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
     // fused decode: every q-tile is one row and tile i is row i (no tile_row0/tile_nrows round trip)
     const int row0 = FUSED ? tile : a.tile_row0[tile], nrows = FUSED ? 1 : a.tile_nrows[tile];
     const int gqa = a.gqa, tpq = 16 / gqa;
-    // fused decode: what needs the row alone is asked for before the slot, the position and the block table are waited for (a 0.6B step of
-    // one row 0.907 -> 0.890 ms, of 16 rows 1.227 -> 1.208, of 64 with a 24-bit cache 1.890 -> 1.846; 64 and more rows the same)
-    [[maybe_unused]] float x[DC][8], qw[DC][8], ssq_g = 0.f;
+    // fused decode: the workgroup's gqa q heads, its k head and its v head are its items, LPH lanes each, HPW to a wave, dealt out to the waves
+    // and shared through LDS; what needs the row alone is asked for before the slot, the position and the block table are waited for.  Every
+    // wave making all of q for itself, with the 14 empty columns of 16, was 24 16-byte loads and 400 instructions a lane: 64 rows of 64 to 512
+    // tokens 21.7 -> 19.8 us a layer, one row of 137 9.7 -> 8.7, 24 8B rows of 256 to 2048 39.1 -> 32.2; with a 24-bit cache, where it spilled,
+    // 24 rows of 48 to 400 23.6 -> 20.1 (all before the eight waves).  Both tile sets are on their way before it starts now.
+    constexpr int half = HD / 2, LPH = HD / 4, HPW = 64 / LPH, NI = 2;  // NI: rounds of items loaded up front, all of them up to gqa = NI * NWV * HPW - 2
+    [[maybe_unused]] const int kv_heads = a.kv.kv_l, items = gqa + 2, hl = lane / LPH, hd2 = lane % LPH * 2;  // this lane's dims: hd2, hd2 + 1 and the two half a head further
     [[maybe_unused]] const float* qkv_row = FUSED ? a.qkv + (size_t)row0 * a.ldqkv : nullptr;
-    [[maybe_unused]] const int qrow_ok = l15 < gqa;
-    [[maybe_unused]] const float* pq = qkv_row + (size_t)(qrow_ok ? kh * gqa + l15 : 0) * HD + grp * 8;
+    [[maybe_unused]] auto item_of = [&](int it) { return (it * NWV + wave) * HPW + hl; };
+    [[maybe_unused]] auto item_src = [&](int item) {
+        return qkv_row + (size_t)(item < gqa ? kh * gqa + item : item == gqa ? a.nh_l + kh : a.nh_l + kv_heads + kh) * HD + hd2;
+    };
+    [[maybe_unused]] auto load2 = [](const float* p) { return *reinterpret_cast<const float2*>(p); };
+    [[maybe_unused]] float2 xa[NI], xb[NI], wa[NI], wb[NI];
+    [[maybe_unused]] float ssq_g = 0.f;
     if constexpr (FUSED) {
 #pragma unroll
-        for (int c = 0; c < DC; ++c) {
-            *reinterpret_cast<float4*>(&x[c][0]) = *reinterpret_cast<const float4*>(pq + c * 32);
-            *reinterpret_cast<float4*>(&x[c][4]) = *reinterpret_cast<const float4*>(pq + c * 32 + 4);
-            *reinterpret_cast<float4*>(&qw[c][0]) = *reinterpret_cast<const float4*>(a.qn + c * 32 + grp * 8);
-            *reinterpret_cast<float4*>(&qw[c][4]) = *reinterpret_cast<const float4*>(a.qn + c * 32 + grp * 8 + 4);
+        for (int it = 0; it < NI; ++it) {
+            const int item = min(item_of(it), items - 1);
+            const float *p = item_src(item), *w = (item < gqa ? a.qn : a.kn) + hd2;
+            xa[it] = load2(p); xb[it] = load2(p + half);
+            wa[it] = load2(w); wb[it] = load2(w + half);
         }
         // deferred input norm of this row: lane g loads group g (groups <= 64), summed below
         if (a.rn.ssq && lane < a.rn.groups) ssq_g = a.rn.ssq[(size_t)lane * a.rn.stride + row0];
@@ -1869,23 +1886,15 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
     // one 32-token KV tile: 2*DC K fragments (the two 16-token tiles are contiguous) + DT V fragments, 16 KiB in 1 KiB wave-loads.  A tile
     // past the end (kt >= t_end: a wave leaves its loop with up to two such prefetches) is the same instructions over buffers of no bytes:
     // they return zeros and cost no access.  A branch around the loads instead makes hipcc wait for vmcnt(0) per load.
-    auto load_tile = [&](int kt, uint4 (&ka)[DC], uint4 (&kb2)[DC], uint4 (&vf)[DT], uint4 (&vl)[RL]) {
+    auto load_k = [&](int kt, uint4 (&ka)[DC], uint4 (&kb2)[DC], [[maybe_unused]] uint4 (&vl)[RL]) {
         const int T0 = min(kt, t_end - 1) << 5;
         const int slab = bt[T0 >> 8] * kv_l + kh, tb = T0 & 255, bytes = kt < t_end ? kBlockTokens * HD * 2 : 0;
         const auto rk = buffer_of(reinterpret_cast<const char*>(a.kv.k) + (size_t)slab * (kBlockTokens * HD * 2), bytes);
-        const auto rv = buffer_of(reinterpret_cast<const char*>(a.kv.v) + (size_t)slab * (kBlockTokens * HD * 2), bytes);
-        const int ko = (tb >> 4) * (DC * 1024), vo = (tb >> 5) * (DT * 1024);
+        const int ko = (tb >> 4) * (DC * 1024);
 #pragma unroll
         for (int c = 0; c < DC; ++c) {
             ka[c] = buffer_stream16(rk, lane * 16 + c * 1024, ko);
             kb2[c] = buffer_stream16(rk, lane * 16 + c * 1024, ko + DC * 1024);
-        }
-#pragma unroll
-        for (int d = 0; d < DT; ++d) vf[d] = buffer_stream16(rv, lane * 16 + (d % 4) * 1024, vo + d / 4 * 4096);
-        if constexpr (VLO) {
-            const auto rl = buffer_of(a.kv.vlo + (size_t)slab * (kBlockTokens * HD), bytes / 2);
-#pragma unroll
-            for (int d = 0; d < DL; ++d) vl[d] = buffer_stream16(rl, lane * 16 + d * 1024, (tb >> 5) * (DL * 1024));
         }
         if constexpr (KLO) {
             const auto rl = buffer_of(a.kv.klo + (size_t)slab * (kBlockTokens * HD), bytes / 2);
@@ -1893,136 +1902,125 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
             for (int i = 0; i < DC; ++i) vl[DL + i] = buffer_stream16(rl, lane * 16 + i * 1024, (tb >> 4) * ((DC / 2) * 1024));
         }
     };
+    auto load_v = [&](int kt, uint4 (&vf)[DT], [[maybe_unused]] uint4 (&vl)[RL]) {
+        const int T0 = min(kt, t_end - 1) << 5;
+        const int slab = bt[T0 >> 8] * kv_l + kh, tb = T0 & 255, bytes = kt < t_end ? kBlockTokens * HD * 2 : 0;
+        const auto rv = buffer_of(reinterpret_cast<const char*>(a.kv.v) + (size_t)slab * (kBlockTokens * HD * 2), bytes);
+        const int vo = (tb >> 5) * (DT * 1024);
+#pragma unroll
+        for (int d = 0; d < DT; ++d) vf[d] = buffer_stream16(rv, lane * 16 + (d % 4) * 1024, vo + d / 4 * 4096);
+        if constexpr (VLO) {
+            const auto rl = buffer_of(a.kv.vlo + (size_t)slab * (kBlockTokens * HD), bytes / 2);
+#pragma unroll
+            for (int d = 0; d < DL; ++d) vl[d] = buffer_stream16(rl, lane * 16 + d * 1024, (tb >> 5) * (DL * 1024));
+        }
+    };
+    auto load_tile = [&](int kt, uint4 (&ka)[DC], uint4 (&kb2)[DC], uint4 (&vf)[DT], uint4 (&vl)[RL]) {
+        load_k(kt, ka, kb2, vl);
+        load_v(kt, vf, vl);
+    };
     // register sets: two 32-token tiles (32 KiB) of this wave are in flight at any time
     uint4 kaA[DC], kbA[DC], vfA[DT], kaB[DC], kbB[DC], vfB[DT];
     uint4 vlA[RL], vlB[RL];
     f16x8 qh[DC], ql[DC];
-    // fused decode: the new token's K and V, and the residual bytes of both, from the wave whose tile it falls into to that wave's lanes
-    // (over obuf, which nobody writes before every wave is through its tiles)
-    _Float16* new_k = reinterpret_cast<_Float16*>(obuf);
-    _Float16* new_v = new_k + HD;
-    uint8_t *new_kl = reinterpret_cast<uint8_t*>(new_v + HD), *new_vl = new_kl + HD;
-    int new_tile = -1;  // ... the tile, in that wave
+    int new_tile = -1;  // fused decode: the tile of the new token, in the wave that has it
     if constexpr (FUSED) {
         // Decode, fused prologue (replaces a separate launch): this workgroup is the only consumer of q heads
         // kh*gqa.. of its row and the only producer of that row's K/V for kv head kh.  The QKV GEMM's split-K
         // slabs are summed here; q/k get RMSNorm over head_dim then RoPE (qwen3.rs:224-234) exactly as
         // qk_norm_rope_kvwrite_kernel does for prefill.
-        constexpr int half = HD / 2;
-        const int row = row0;
-        const int pos = a.pos[row];
-        // the wave whose tile holds the new token makes its K and V, patches them into the tile it has loaded and stores them for later steps:
-        // no wave waits for another one, for a store or with its first tile (split-KV: one workgroup has such a wave).  With wave 0 as the
-        // maker, its stores waited for and a barrier behind them, and with prefetches past the end that read a shared dummy tile: a 0.6B step
-        // of one row of 137 tokens 0.974 ms, now 0.908; 32 rows of 131 to 638 1.435 -> 1.388; 64 of 64 to 512 1.479 -> 1.429; 130 of 64 to
-        // 1024 3.456 -> 3.302; with a 24-bit cache 64 rows 1.995 -> 1.907.
-        const int last = pos >> 5;
-        const bool maker = last >= t_begin && last < t_end && ((last - t_begin) % NWV) == wave;
-        // ---- every load of the prologue first, unconditionally (clamped lanes), so they overlap: a branch
-        // ---- around a load costs a full vmcnt(0) round trip each on this compiler
-        const int ln = min(lane, half - 1);
-        const float* pk = qkv_row + (size_t)(a.nh_l + kh) * HD;
-        const float* pv = qkv_row + (size_t)(a.nh_l + kv_l + kh) * HD;
-        float kx1 = 0.f, kx2 = 0.f, vx1 = 0.f, vx2 = 0.f, knw1 = 0.f, knw2 = 0.f, kc = 0.f, ks = 0.f;
-        if (maker) {
-            kx1 = pk[ln]; kx2 = pk[ln + half]; vx1 = pv[ln]; vx2 = pv[ln + half];
-            knw1 = a.kn[ln]; knw2 = a.kn[ln + half];
-            kc = a.cos[(size_t)pos * half + ln]; ks = a.sin[(size_t)pos * half + ln];
-        }
-        float cs[DC / 2][8], sn[DC / 2][8];
+        const int pos = pmax, last = pos >> 5;
+        const bool has_new = last >= t_begin && last < t_end;  // split-KV: one workgroup of the row makes the new token's K and V
+        const float2 cs = load2(a.cos + (size_t)pos * half + hd2), sn = load2(a.sin + (size_t)pos * half + hd2);
+        auto add_slabs = [&](const float* p, float2& u, float2& w) __attribute__((always_inline)) {  // split-K slabs of the generic path's QKV GEMM, four per trip
+            for (int s0 = 1; s0 < a.n_slabs; s0 += 4) {
+                float2 pu[4], pw[4];
 #pragma unroll
-        for (int c = 0; c < DC / 2; ++c) {
-            const size_t o = (size_t)pos * half + c * 32 + grp * 8;
-            *reinterpret_cast<float4*>(&cs[c][0]) = *reinterpret_cast<const float4*>(a.cos + o);
-            *reinterpret_cast<float4*>(&cs[c][4]) = *reinterpret_cast<const float4*>(a.cos + o + 4);
-            *reinterpret_cast<float4*>(&sn[c][0]) = *reinterpret_cast<const float4*>(a.sin + o);
-            *reinterpret_cast<float4*>(&sn[c][4]) = *reinterpret_cast<const float4*>(a.sin + o + 4);
-        }
-        // This wave's first KV tile goes in flight BEHIND the prologue's own loads (vmcnt retires in order, so the prologue never waits for
-        // it) and lands while it computes; a second set would push the kernel to one wave per SIMD.  The new token's place in its tile still
-        // holds old bytes, or the new ones if the stores below pass first: the tile is patched before it is used.
-        load_tile(t_begin + wave, kaA, kbA, vfA, vlA);
-        const float ri = a.rn.ssq ? 1.0f / sqrtf(wave_sum(ssq_g) * a.rn.inv_h + a.rn.eps) : 1.0f;
-        for (int sl0 = 1; sl0 < a.n_slabs; sl0 += 2) {  // split-K slabs of the generic path's QKV GEMM, two per trip
-            const size_t so0 = (size_t)sl0 * a.slab_stride, so1 = (size_t)min(sl0 + 1, a.n_slabs - 1) * a.slab_stride;
-            const float m1 = sl0 + 1 < a.n_slabs ? 1.f : 0.f;
-            if (maker) {
-                const float a0 = pk[so0 + ln], a1 = pk[so0 + ln + half], a2 = pv[so0 + ln], a3 = pv[so0 + ln + half];
-                const float b0 = pk[so1 + ln], b1 = pk[so1 + ln + half], b2 = pv[so1 + ln], b3 = pv[so1 + ln + half];
-                kx1 += a0; kx2 += a1; vx1 += a2; vx2 += a3;
-                kx1 += m1 * b0; kx2 += m1 * b1; vx1 += m1 * b2; vx2 += m1 * b3;
-            }
-            float4 q0[DC][2], q1[DC][2];
+                for (int i = 0; i < 4; ++i) {
+                    const float* ps = p + (size_t)min(s0 + i, a.n_slabs - 1) * a.slab_stride;
+                    pu[i] = load2(ps); pw[i] = load2(ps + half);
+                }
 #pragma unroll
-            for (int c = 0; c < DC; ++c) {
-                q0[c][0] = *reinterpret_cast<const float4*>(pq + so0 + c * 32); q0[c][1] = *reinterpret_cast<const float4*>(pq + so0 + c * 32 + 4);
-                q1[c][0] = *reinterpret_cast<const float4*>(pq + so1 + c * 32); q1[c][1] = *reinterpret_cast<const float4*>(pq + so1 + c * 32 + 4);
-            }
-#pragma unroll
-            for (int c = 0; c < DC; ++c) {
-                x[c][0] += q0[c][0].x; x[c][1] += q0[c][0].y; x[c][2] += q0[c][0].z; x[c][3] += q0[c][0].w;
-                x[c][4] += q0[c][1].x; x[c][5] += q0[c][1].y; x[c][6] += q0[c][1].z; x[c][7] += q0[c][1].w;
-                x[c][0] += m1 * q1[c][0].x; x[c][1] += m1 * q1[c][0].y; x[c][2] += m1 * q1[c][0].z; x[c][3] += m1 * q1[c][0].w;
-                x[c][4] += m1 * q1[c][1].x; x[c][5] += m1 * q1[c][1].y; x[c][6] += m1 * q1[c][1].z; x[c][7] += m1 * q1[c][1].w;
-            }
-        }
-        // ---- q: deferred input norm, RMSNorm over head_dim, RoPE (chunk c pairs with c + DC/2 in the same lane)
-        float ss = 0.f;
-#pragma unroll
-        for (int c = 0; c < DC; ++c)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                x[c][j] = qrow_ok ? x[c][j] * ri : 0.f;
-                ss += x[c][j] * x[c][j];
-            }
-        ss += __shfl_xor(ss, 16);
-        ss += __shfl_xor(ss, 32);
-        const float rinv = 1.0f / sqrtf(ss / (float)HD + a.eps);
-#pragma unroll
-        for (int c = 0; c < DC / 2; ++c) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float n1 = (x[c][j] * rinv) * qw[c][j], n2 = (x[c + DC / 2][j] * rinv) * qw[c + DC / 2][j];
-                const float y1 = (n1 * cs[c][j] - n2 * sn[c][j]) * a.q_scale;
-                const float y2 = (n2 * cs[c][j] + n1 * sn[c][j]) * a.q_scale;
-                const _Float16 h1 = (_Float16)y1, h2 = (_Float16)y2;
-                qh[c][j] = h1;
-                ql[c][j] = (_Float16)(y1 - (float)h1);
-                qh[c + DC / 2][j] = h2;
-                ql[c + DC / 2][j] = (_Float16)(y2 - (float)h2);
-            }
-        }
-        // ---- K / V of the new token
-        if (maker) {
-            new_tile = last;
-            const bool act = lane < half;
-            kx1 = act ? kx1 * ri : 0.f; kx2 = act ? kx2 * ri : 0.f;
-            const float kss = wave_sum(kx1 * kx1 + kx2 * kx2);
-            const float krinv = 1.0f / sqrtf(kss / (float)HD + a.eps);
-            if (act) {
-                const int blk = bt[pos >> 8];
-                const float n1 = (kx1 * krinv) * knw1, n2 = (kx2 * krinv) * knw2;
-                const float y[4] = {n1 * kc - n2 * ks, n2 * kc + n1 * ks, vx1 * ri, vx2 * ri};
-                const size_t vo = (size_t)(blk * kv_l + kh) * kBlockTokens * HD;
-                _Float16* k = reinterpret_cast<_Float16*>(a.kv.k) + vo;
-                uint8_t* klo = KLO ? a.kv.klo + vo : nullptr;
-                _Float16* v = reinterpret_cast<_Float16*>(a.kv.v) + vo;
-                uint8_t* vlo = VLO ? a.kv.vlo + vo : nullptr;
-#pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    const int dim = lane + e * half;
-                    store_k24(k, klo, pos & 255, dim, HD, y[e]);
-                    store_v24(v, vlo, pos & 255, dim, HD, y[2 + e]);
-                    new_k[dim] = f16_sat(y[e]);
-                    new_v[dim] = f16_sat(y[2 + e]);
-                    if constexpr (KLO) new_kl[dim] = residual24(y[e], f16_sat(y[e]));
-                    if constexpr (VLO != 0) new_vl[dim] = residual24(y[2 + e], f16_sat(y[2 + e]));
+                for (int i = 0; i < 4; ++i) {
+                    const float f = s0 + i < a.n_slabs ? 1.f : 0.f;
+                    u.x += f * pu[i].x; u.y += f * pu[i].y; w.x += f * pw[i].x; w.y += f * pw[i].y;
                 }
             }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        };
+        if (a.n_slabs > 1)
+#pragma unroll
+            for (int it = 0; it < NI; ++it) add_slabs(item_src(min(item_of(it), items - 1)), xa[it], xb[it]);
+        // This wave's first KV tiles go in flight BEHIND the prologue's own loads (vmcnt retires in order, so the prologue never waits for
+        // them) and land while it computes.  The new token's place in its tile still holds old bytes, or the new ones if the stores below
+        // pass first: the tile is patched before it is used.
+        load_tile(t_begin + wave, kaA, kbA, vfA, vlA);
+        if constexpr (!ONE_SET) load_tile(t_begin + wave + NWV, kaB, kbB, vfB, vlB);
+        auto make = [&](int item, float2 u, float2 w, float2 nu, float2 nw) __attribute__((always_inline)) {
+            const float ri = a.rn.ssq ? 1.0f / sqrtf(wave_sum(ssq_g) * a.rn.inv_h + a.rn.eps) : 1.0f;
+            u.x *= ri; u.y *= ri; w.x *= ri; w.y *= ri;
+            float ss = u.x * u.x + u.y * u.y + w.x * w.x + w.y * w.y;
+#pragma unroll
+            for (int d = 1; d < LPH; d *= 2) ss += __shfl_xor(ss, d);
+            const float rinv = 1.0f / sqrtf(ss / (float)HD + a.eps);
+            const float y[4] = {u.x, u.y, w.x, w.y}, g[4] = {nu.x, nu.y, nw.x, nw.y}, c[2] = {cs.x, cs.y}, s_[2] = {sn.x, sn.y};
+            float z[4];  // dims hd2, hd2 + 1, half + hd2, half + hd2 + 1
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const float n1 = (y[e] * rinv) * g[e], n2 = (y[2 + e] * rinv) * g[2 + e];
+                z[e] = n1 * c[e] - n2 * s_[e];
+                z[2 + e] = n2 * c[e] + n1 * s_[e];
+            }
+            if (item < gqa) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float v = z[e] * a.q_scale;
+                    const _Float16 h = (_Float16)v;
+                    const int to = q_at + (item * HD + (e >> 1) * half + hd2 + (e & 1)) * 2;
+                    *lds16(to) = h;
+                    *lds16(to + cols * HD * 2) = (_Float16)(v - (float)h);
+                }
+            } else if (has_new && item < items) {
+                const size_t vo = (size_t)(bt[pos >> 8] * kv_l + kh) * kBlockTokens * HD;
+                const bool isv = item > gqa;
+                _Float16* const to = reinterpret_cast<_Float16*>(isv ? a.kv.v : a.kv.k) + vo;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int dim = (e >> 1) * half + hd2 + (e & 1);
+                    const float v = isv ? y[e] : z[e];
+                    const _Float16 h = f16_sat(v);
+                    to[isv ? v_packed_offset(pos & 255, dim, HD) : k_packed_offset(pos & 255, dim, HD)] = h;
+                    *lds16(new_at + (isv ? HD * 2 : 0) + dim * 2) = h;
+                    if constexpr (VLO != 0) {
+                        const uint8_t lo = residual24(v, h);
+                        *lds8(new_kl_at + (isv ? HD : 0) + dim) = lo;
+                        if (isv) (a.kv.vlo + vo)[vlo_packed_offset(pos & 255, dim, HD)] = lo;
+                        else if constexpr (KLO) (a.kv.klo + vo)[klo_packed_offset(pos & 255, dim, HD)] = lo;
+                    }
+                }
+            }
+        };
+#pragma unroll
+        for (int it = 0; it < NI; ++it)
+            if ((it * NWV + wave) * HPW < items) make(item_of(it), xa[it], xb[it], wa[it], wb[it]);
+        for (int it = NI; (it * NWV + wave) * HPW < items; ++it) {
+            const int item = min(item_of(it), items - 1);
+            const float *p = item_src(item), *w = (item < gqa ? a.qn : a.kn) + hd2;
+            float2 u = load2(p), v = load2(p + half);
+            const float2 nu = load2(w), nw = load2(w + half);
+            add_slabs(p, u, v);
+            make(item_of(it), u, v, nu, nw);
         }
         NVLLM_STAMP(a, 1);
-        NVLLM_STAMP(a, 2);  // no barrier in between any more: the loop's segment starts here
+        // q and the new token are published; the tiles stay in flight
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (has_new && (last - t_begin) % NWV == wave) new_tile = last;
+        const int at = q_at + ((l15 % gqa) * HD + grp * 8) * 2;  // columns of no row repeat one: nothing of theirs is stored
+#pragma unroll
+        for (int c = 0; c < DC; ++c) {
+            qh[c] = *reinterpret_cast<const f16x8*>(smem_raw + at + c * 64);
+            ql[c] = *reinterpret_cast<const f16x8*>(smem_raw + at + cols * HD * 2 + c * 64);
+        }
+        NVLLM_STAMP(a, 2);
     } else {
 #pragma unroll
         for (int c = 0; c < DC; ++c) {
@@ -2053,7 +2051,8 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
 #pragma unroll
     for (int d = 0; d < DT; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    auto compute_tile = [&](int kt, const uint4 (&ka)[DC], const uint4 (&kb2)[DC], const uint4 (&vf)[DT], const uint4 (&vl)[RL]) {
+    // after_scores: what may overwrite ka, kb2 and K's residuals
+    auto compute_tile = [&](int kt, uint4 (&ka)[DC], uint4 (&kb2)[DC], uint4 (&vf)[DT], uint4 (&vl)[RL], auto after_scores) {
         const int T0 = kt << 5;
         const int tokA = T0 + grp * 4, tokB = T0 + 16 + grp * 4;
         f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
@@ -2077,6 +2076,7 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
                 mfma_result_settled(sb);
             }
         }
+        after_scores();
         float mt = -1e30f;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
@@ -2131,8 +2131,10 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
             // decode: two named register sets, both in flight; a set is refilled (two tiles ahead) right after it is
             // consumed.  Prefetches are unconditional (tile index clamped): no branch around loads.
             int kt = t_begin + wave;
-            if constexpr (!FUSED) load_tile(kt, kaA, kbA, vfA, vlA);  // (the fused prologue has sent for it)
-            if constexpr (!ONE_SET) load_tile(kt + NWV, kaB, kbB, vfB, vlB);
+            if constexpr (!FUSED) {  // (the fused prologue has sent for them)
+                load_tile(kt, kaA, kbA, vfA, vlA);
+                if constexpr (!ONE_SET) load_tile(kt + NWV, kaB, kbB, vfB, vlB);
+            }
             // the new token into its place of a tile: K's lanes l15 == token % 16 of the token half, V's lane group and halfword
             auto patch = [&](uint4 (&ka)[DC], uint4 (&kb2)[DC], uint4 (&vf)[DT], uint4 (&vl)[RL]) {
                 const int tt = pmax & 31, e = (tt >> 4) * 4 + (tt & 3);
@@ -2140,14 +2142,14 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
                 const bool ka_lane = kl && tt < 16, kb_lane = kl && tt >= 16, v_lane = grp == ((tt & 15) >> 2);
 #pragma unroll
                 for (int c = 0; c < DC; ++c) {
-                    const uint4 n = *reinterpret_cast<const uint4*>(new_k + c * 32 + grp * 8);
+                    const uint4 n = *reinterpret_cast<const uint4*>(lds16(new_at) + c * 32 + grp * 8);
                     ka[c].x = ka_lane ? n.x : ka[c].x; ka[c].y = ka_lane ? n.y : ka[c].y; ka[c].z = ka_lane ? n.z : ka[c].z; ka[c].w = ka_lane ? n.w : ka[c].w;
                     kb2[c].x = kb_lane ? n.x : kb2[c].x; kb2[c].y = kb_lane ? n.y : kb2[c].y; kb2[c].z = kb_lane ? n.z : kb2[c].z; kb2[c].w = kb_lane ? n.w : kb2[c].w;
                 }
                 uint32_t mask[4];
 #pragma unroll
                 for (int i = 0; i < 4; ++i) mask[i] = v_lane && (e >> 1) == i ? ((e & 1) ? 0xffff0000u : 0x0000ffffu) : 0u;
-                const uint16_t* nv = reinterpret_cast<const uint16_t*>(new_v);
+                const uint16_t* nv = reinterpret_cast<const uint16_t*>(smem_raw + new_v_at);
 #pragma unroll
                 for (int d = 0; d < DT; ++d) {
                     const uint32_t n = nv[d * 16 + l15] * 0x10001u;
@@ -2160,7 +2162,7 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
                     for (int i = 0; i < 2; ++i) m8[i] = v_lane && (e >> 2) == i ? 0xffu << ((e & 3) * 8) : 0u;
 #pragma unroll
                     for (int d = 0; d < DT; ++d) {
-                        const uint32_t n = new_vl[d * 16 + l15] * 0x1010101u;
+                        const uint32_t n = lds8(new_vl_at)[d * 16 + l15] * 0x1010101u;
                         uint32_t &w0 = (d & 1) ? vl[d >> 1].z : vl[d >> 1].x, &w1 = (d & 1) ? vl[d >> 1].w : vl[d >> 1].y;
                         w0 = (w0 & ~m8[0]) | (n & m8[0]);
                         w1 = (w1 & ~m8[1]) | (n & m8[1]);
@@ -2169,7 +2171,7 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
                 if constexpr (KLO) {
 #pragma unroll
                     for (int c = 0; c < DC; ++c) {
-                        const uint2 n = *reinterpret_cast<const uint2*>(new_kl + c * 32 + grp * 8);
+                        const uint2 n = *reinterpret_cast<const uint2*>(lds8(new_kl_at) + c * 32 + grp * 8);
                         uint4 &pa = vl[DL + (c >> 1)], &pb = vl[DL + DC / 2 + (c >> 1)];
                         uint32_t &a0 = (c & 1) ? pa.z : pa.x, &a1 = (c & 1) ? pa.w : pa.y, &b0 = (c & 1) ? pb.z : pb.x, &b1 = (c & 1) ? pb.w : pb.y;
                         a0 = ka_lane ? n.x : a0; a1 = ka_lane ? n.y : a1;
@@ -2179,22 +2181,23 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
             };
             if constexpr (ONE_SET) {
                 // 24-bit cache: one 24 KiB set per wave and two waves per SIMD (a second set needs > 256 registers: half the
-                // workgroups resident, two rounds) -- the other seven waves of the CU cover this wave's round trip
+                // workgroups resident, two rounds) -- the other seven waves of the CU cover this wave's round trip; the next tile's K is sent
+                // for as soon as the scores are made (24 rows of 48 to 400 tokens 17.3 -> 16.5 us, 64 of 64 to 512 28.5)
                 while (kt < t_end) {
                     if (FUSED && kt == new_tile) patch(kaA, kbA, vfA, vlA);
-                    compute_tile(kt, kaA, kbA, vfA, vlA);
-                    load_tile(kt + NWV, kaA, kbA, vfA, vlA);
+                    compute_tile(kt, kaA, kbA, vfA, vlA, [&] { load_k(kt + NWV, kaA, kbA, vlA); });
+                    load_v(kt + NWV, vfA, vlA);
                     kt += NWV;
                 }
             } else {
                 while (kt < t_end) {
                     if (FUSED && kt == new_tile) patch(kaA, kbA, vfA, vlA);
-                    compute_tile(kt, kaA, kbA, vfA, vlA);
+                    compute_tile(kt, kaA, kbA, vfA, vlA, [] {});
                     load_tile(kt + 2 * NWV, kaA, kbA, vfA, vlA);
                     kt += NWV;
                     if (kt >= t_end) break;
                     if (FUSED && kt == new_tile) patch(kaB, kbB, vfB, vlB);
-                    compute_tile(kt, kaB, kbB, vfB, vlB);
+                    compute_tile(kt, kaB, kbB, vfB, vlB, [] {});
                     load_tile(kt + 2 * NWV, kaB, kbB, vfB, vlB);
                     kt += NWV;
                 }
@@ -2202,62 +2205,56 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
         }
     }
 
-    // combine the NWV waves' partial (m, l, O)
+    // merge the NWV waves' partial (m, l, O): columns that are rows of q only, one barrier; a thread then owns four dims of a column
     NVLLM_STAMP(a, 3);
     lsum += __shfl_xor(lsum, 16);
     lsum += __shfl_xor(lsum, 32);
-    if (grp == 0) {
-        ml[(wave * 2 + 0) * 16 + l15] = m;
-        ml[(wave * 2 + 1) * 16 + l15] = lsum;
+    if (l15 < cols) {
+        if (grp == 0) {
+            ml[(wave * 2 + 0) * 16 + l15] = m;
+            ml[(wave * 2 + 1) * 16 + l15] = lsum;
+        }
+#pragma unroll
+        for (int d = 0; d < DT; ++d) obuf[(wave * cols + l15) * (HD / 4) + d * 4 + grp] = o[d];
     }
-    __syncthreads();
-    float ms = -1e30f;
-#pragma unroll
-    for (int w = 0; w < NWV; ++w) ms = fmaxf(ms, ml[(w * 2 + 0) * 16 + l15]);
-    float ltot = 0.f;
-#pragma unroll
-    for (int w = 0; w < NWV; ++w)
-        ltot += ml[(w * 2 + 1) * 16 + l15] * exp2f(ml[(w * 2 + 0) * 16 + l15] - ms);
-    const float f = exp2f(m - ms);
-#pragma unroll
-    for (int d = 0; d < DT; ++d) {
-        o[d][0] *= f; o[d][1] *= f; o[d][2] *= f; o[d][3] *= f;
-    }
-    // every wave publishes its rescaled O; then wave w sums dim-tiles w, w+NWV, ... over all waves
-#pragma unroll
-    for (int d = 0; d < DT; ++d) obuf[(wave * DT + d) * 64 + lane] = o[d];
     __syncthreads();
     const int n_parts = a.part_tiles ? (n_kv_tiles + a.part_tiles - 1) / a.part_tiles : 1;
-    if (my_row >= 0) {
-        const size_t base = (size_t)my_row * ldq + (size_t)my_head * HD + grp * 4;
-        for (int d = wave; d < DT; d += NWV) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int i = threadIdx.x; i < cols * (HD / 4); i += NWV * 64) {
+        const int col = i / (HD / 4), d4 = i % (HD / 4), tok = FUSED ? 0 : col / gqa;
+        if (tok >= nrows || (!FUSED && col >= tpq * gqa)) continue;
+        const int row = row0 + tok, head = kh * gqa + (FUSED ? col : col % gqa);
+        float ms = -1e30f;
 #pragma unroll
-            for (int w = 0; w < NWV; ++w) {
-                const f32x4 v = obuf[(w * DT + d) * 64 + lane];
-                acc[0] += v[0]; acc[1] += v[1]; acc[2] += v[2]; acc[3] += v[3];
-            }
-            if (n_parts > 1) {
-                // partial: O (at the workgroup's max) for the combine kernel
-                float* po = a.part_o + (((size_t)my_row * a.nh_l + my_head) * a.max_parts + blockIdx.z) * HD + d * 16 + grp * 4;
-                *reinterpret_cast<float4*>(po) = make_float4(acc[0], acc[1], acc[2], acc[3]);
-                continue;
-            }
-            const float inv = 1.0f / ltot;
-            const float y0 = acc[0] * inv, y1 = acc[1] * inv, y2 = acc[2] * inv, y3 = acc[3] * inv;
-            if (a.out_f32) *reinterpret_cast<float4*>(a.out_f32 + base + d * 16) = make_float4(y0, y1, y2, y3);
-            if (a.out_hi) {
-                uint16_t h0, h1, h2, h3, l0, l1, l2, l3;
-                split_bf16(y0, h0, l0); split_bf16(y1, h1, l1); split_bf16(y2, h2, l2); split_bf16(y3, h3, l3);
-                const size_t xo = a.out_packed ? xpack_off(my_row, my_head * HD + d * 16 + grp * 4, ldq >> 5) : base + d * 16;
-                *reinterpret_cast<uint2*>(a.out_hi + xo) = make_uint2(h0 | ((uint32_t)h1 << 16), h2 | ((uint32_t)h3 << 16));
-                *reinterpret_cast<uint2*>(a.out_lo + xo) = make_uint2(l0 | ((uint32_t)l1 << 16), l2 | ((uint32_t)l3 << 16));
-            }
+        for (int w = 0; w < NWV; ++w) ms = fmaxf(ms, ml[(w * 2 + 0) * 16 + col]);
+        float ltot = 0.f;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < NWV; ++w) {
+            const float f = exp2f(ml[(w * 2 + 0) * 16 + col] - ms);
+            const f32x4 v = obuf[(w * cols + col) * (HD / 4) + d4];
+            ltot += ml[(w * 2 + 1) * 16 + col] * f;
+            acc[0] += v[0] * f; acc[1] += v[1] * f; acc[2] += v[2] * f; acc[3] += v[3] * f;
         }
-        if (n_parts > 1 && wave == 0 && grp == 0) {
-            float* pm = a.part_ml + (((size_t)my_row * a.nh_l + my_head) * a.max_parts + blockIdx.z) * 2;
-            pm[0] = ms;
-            pm[1] = ltot;
+        if (n_parts > 1) {
+            // partial: O (at the workgroup's max) for the combine kernel
+            const size_t part = ((size_t)row * a.nh_l + head) * a.max_parts + blockIdx.z;
+            *reinterpret_cast<float4*>(a.part_o + part * HD + d4 * 4) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+            if (d4 == 0) {
+                a.part_ml[part * 2] = ms;
+                a.part_ml[part * 2 + 1] = ltot;
+            }
+            continue;
+        }
+        const float inv = 1.0f / ltot;
+        const float y0 = acc[0] * inv, y1 = acc[1] * inv, y2 = acc[2] * inv, y3 = acc[3] * inv;
+        const size_t base = (size_t)row * ldq + (size_t)head * HD + d4 * 4;
+        if (a.out_f32) *reinterpret_cast<float4*>(a.out_f32 + base) = make_float4(y0, y1, y2, y3);
+        if (a.out_hi) {
+            uint16_t h0, h1, h2, h3, l0, l1, l2, l3;
+            split_bf16(y0, h0, l0); split_bf16(y1, h1, l1); split_bf16(y2, h2, l2); split_bf16(y3, h3, l3);
+            const size_t xo = a.out_packed ? xpack_off(row, head * HD + d4 * 4, ldq >> 5) : base;
+            *reinterpret_cast<uint2*>(a.out_hi + xo) = make_uint2(h0 | ((uint32_t)h1 << 16), h2 | ((uint32_t)h3 << 16));
+            *reinterpret_cast<uint2*>(a.out_lo + xo) = make_uint2(l0 | ((uint32_t)l1 << 16), l2 | ((uint32_t)l3 << 16));
         }
     }
     NVLLM_STAMP(a, 4);
@@ -2655,10 +2652,10 @@ __global__ void __launch_bounds__(256) attn_combine_kernel(AttnArgs a, int rows)
 
 template <int HD, int NWV, bool FUSED, int VLO>
 static hipError_t attn_launch_v(const AttnArgs& a, int n_tiles, int grid_z, hipStream_t s) {
-    constexpr int DT = HD / 16;
-    const size_t lds = (size_t)NWV * 2 * 16 * 4 + (size_t)NWV * DT * 64 * 16;
+    auto lds_of = [](int gqa) { return NWV * 2 * 16 * 4 + (size_t)NWV * gqa * HD * 4 + (FUSED ? (size_t)gqa * HD * 4 + HD * 6 : 0); };
+    const size_t lds = lds_of(FUSED ? a.gqa : 16);
     static std::atomic<uint64_t> lds_set{0};
-    ensure_dyn_lds(reinterpret_cast<const void*>(attn_paged_kernel<HD, NWV, FUSED, VLO>), lds, lds_set);
+    ensure_dyn_lds(reinterpret_cast<const void*>(attn_paged_kernel<HD, NWV, FUSED, VLO>), lds_of(16), lds_set);
     dim3 grid = FUSED ? dim3(a.kv.kv_l, n_tiles, grid_z) : dim3(n_tiles * a.kv.kv_l, 1, grid_z);
     attn_paged_kernel<HD, NWV, FUSED, VLO><<<grid, NWV * 64, lds, s>>>(a);
     return hipGetLastError();
@@ -2726,7 +2723,9 @@ hipError_t launch_attn_paged(const AttnArgs& a, int n_tiles, int rows, int n_par
     hipError_t e = hipErrorInvalidValue;
     const bool fused = a.qkv != nullptr;  // decode rows straight from the QKV GEMM's slabs
     if (fused && (n_tiles != rows || rows > kAttnFusedMaxRows)) return hipErrorInvalidValue;  // fused decode: tile i is row i
-    if (a.kv.hd == 128) e = fused ? attn_launch_t<128, 4, true>(b, n_tiles, gz, s) : attn_launch_t<128, 4, false>(b, n_tiles, gz, s);
+    if (a.waves != 4 && (a.waves != 8 || !fused || a.kv.hd != 128)) return hipErrorInvalidValue;
+    if (a.waves == 8) e = attn_launch_t<128, 8, true>(b, n_tiles, gz, s);
+    else if (a.kv.hd == 128) e = fused ? attn_launch_t<128, 4, true>(b, n_tiles, gz, s) : attn_launch_t<128, 4, false>(b, n_tiles, gz, s);
     else if (a.kv.hd == 64) e = fused ? attn_launch_t<64, 4, true>(b, n_tiles, gz, s) : attn_launch_t<64, 4, false>(b, n_tiles, gz, s);
     if (e != hipSuccess || !split) return e;
     const int items = rows * a.nh_l;

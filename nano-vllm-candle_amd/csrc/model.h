@@ -179,7 +179,7 @@ struct nvllm_model {
     float* qkv_out = nullptr;                // complete QKV sums of the streaming GEMM (its combine reads the slabs in m->slabs)
     uint32_t* d_next = nullptr;
     float *attn_po = nullptr, *attn_pml = nullptr;  // split-KV partials [max_seqs][nh_l][kAttnMaxParts][hd] / [..][2]
-    int attn_part_tiles = 4, attn_parts_max = 1;   // this step's split geometry (decode only)
+    int attn_part_tiles = 4, attn_parts_max = 1, attn_waves = 4;   // this step's split geometry and waves of a workgroup (decode only)
     float* part_val = nullptr;  // fused LM-head arg-max partials [V_l/16][max_seqs]
     int* part_idx = nullptr;
     unsigned long long* argmax_scratch = nullptr;  // ticket + per-row keys of argmax_parts_kernel

@@ -1,0 +1,36 @@
+"""GPU test of the decode attention's two workgroup sizes (eight waves where a launch is one workgroup per CU at most, four above) and of its
+shared prologue: heads of a group that fit the rounds loaded up front and that do not, contexts on both sides of a wave's, a part's and the
+unsplit form's ends."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+LENGTHS = [1, 31, 33, 126, 127, 128, 159, 255, 256, 257, 510, 511, 512, 1021, 1022, 1023, 1024]
+
+
+# workgroups: 256 and 264 of 8 kv heads; 128 and 124 of 4 (whole and in parts from 513 tokens on); 2 and 257 of one, whose 18 heads take
+# more rounds of four waves than are loaded up front; 8 heads of 64
+@pytest.mark.parametrize("hd,kv,heads,rows,bits", [(128, 8, 16, 32, 16), (128, 8, 16, 33, 16), (128, 4, 8, 32, 16), (128, 4, 8, 31, 24), (128, 1, 16, 2, 16),
+                                                   (128, 1, 16, 257, 16), (128, 1, 8, 17, 24), (64, 1, 8, 17, 16), (64, 1, 16, 3, 16)])
+def test_a_step_equals_the_prompt(hd, kv, heads, rows, bits):
+    import nano_vllm_candle_amd as pkg
+
+    cfg = pkg.Qwen3Config.tiny(hidden_size=256, head_dim=hd, num_attention_heads=heads, num_key_value_heads=kv)
+    m = pkg.Qwen3ForCausalLM.from_synthetic(cfg, 3)
+    if bits == 24:
+        m.set_option("kv_v_bits", 24)
+        m.set_option("kv_k_bits", 24)
+    lens = [LENGTHS[(i * 7) % len(LENGTHS)] for i in range(rows)]
+    m.kv_alloc(sum(n // 256 + 1 for n in lens) + 8, rows + 1, 2048)
+    rng = np.random.default_rng(rows + heads)
+    seqs = [rng.integers(0, cfg.vocab_size, n + 1) for n in lens]
+    m.step(list(range(rows)), [s[:-1] for s in seqs], True, want_logits=False)
+    _, got = m.step(list(range(rows)), seqs, False, want_logits=True)
+    # the prompt's kernels sum in another order, from keys whose f16 may round the other way: 2^-11 of the largest logit, 2^-14 with the residuals
+    bound = 2.0 ** (-11 if bits == 16 else -14)
+    for i in range(min(rows, 34)):
+        _, want = m.step([rows], [seqs[i]], True, want_logits=True)
+        m.seq_free(rows)
+        assert np.abs(got[i] - want[0]).max() < bound * np.abs(want).max(), (i, lens[i])
+    m.close()
