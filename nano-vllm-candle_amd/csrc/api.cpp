@@ -450,11 +450,11 @@ static void free_kv(nvllm_model* m) {
     for (auto p : m->klocache) (void)hipFree(p);
     m->kcache.clear(); m->vcache.clear(); m->vlocache.clear(); m->klocache.clear();
     void* ptrs[] = {m->d_block_tables, m->d_ids, m->d_pos, m->d_slot, m->d_tile_row0, m->d_tile_nrows, m->d_tile_slot,
-                    m->d_last_rows, m->d_tile_order, m->d_tile_last, m->d_group_order, m->resid, m->slabs, m->qbuf, m->logits, m->d_maxval, m->red, m->xh, m->xl, m->xh2, m->xl2, m->ctxh, m->ctxl, m->ssqA, m->ssqB, m->d_next,
+                    m->d_last_rows, m->d_tile_order, m->d_tile_last, m->d_group_order, m->resid, m->last_resid, m->slabs, m->qbuf, m->logits, m->d_maxval, m->red, m->xh, m->xl, m->xh2, m->xl2, m->ctxh, m->ctxl, m->ssqA, m->ssqB, m->d_next,
                     m->part_val, m->part_idx, m->argmax_scratch, m->attn_po, m->attn_pml, m->tap_h, m->tap_res, m->cosv, m->sinv, m->tickets, m->qkv_out, m->d_keys, m->d_temps};
     for (void* p : ptrs) if (p) (void)hipFree(p);
     m->d_block_tables = nullptr; m->d_ids = nullptr; m->d_pos = m->d_slot = m->d_tile_row0 = m->d_tile_nrows = m->d_tile_slot = m->d_last_rows = m->d_tile_order = m->d_tile_last = m->d_group_order = nullptr;
-    m->resid = m->slabs = m->qbuf = m->logits = m->d_maxval = m->red = nullptr; m->xh = m->xl = m->xh2 = m->xl2 = m->ctxh = m->ctxl = nullptr; m->ssqA = m->ssqB = nullptr; m->d_next = nullptr; m->part_val = nullptr; m->part_idx = nullptr; m->argmax_scratch = nullptr; m->attn_po = m->attn_pml = nullptr;
+    m->resid = m->last_resid = m->slabs = m->qbuf = m->logits = m->d_maxval = m->red = nullptr; m->xh = m->xl = m->xh2 = m->xl2 = m->ctxh = m->ctxl = nullptr; m->ssqA = m->ssqB = nullptr; m->d_next = nullptr; m->part_val = nullptr; m->part_idx = nullptr; m->argmax_scratch = nullptr; m->attn_po = m->attn_pml = nullptr;
     m->tap_h = m->tap_res = nullptr; m->cosv = m->sinv = nullptr; m->tickets = nullptr; m->qkv_out = nullptr; m->d_keys = nullptr; m->d_temps = nullptr;
     stage_release(m);
     m->num_blocks = 0;
@@ -786,6 +786,7 @@ static int qwen3_kv_alloc(nvllm_model* m) {
     const size_t nmax = std::max<size_t>({(size_t)(m->nh_l + 2 * m->kv_l) * m->hd, (size_t)m->H, (size_t)2 * m->I_l});
     m->slab_floats = std::max<size_t>(R * nmax, (size_t)32 * std::min<size_t>(R, 128) * nmax);
     if (!rc) rc = dmalloc(ctx, &m->resid, R * m->H);
+    if (!rc) rc = dmalloc(ctx, &m->last_resid, last_rows_cap(m) * m->H);
     if (!rc) rc = dmalloc(ctx, &m->slabs, m->slab_floats);
     if (!rc) rc = dmalloc(ctx, &m->qbuf, R * m->nh_l * m->hd);
     if (!rc) rc = dmalloc(ctx, &m->red, R * m->H);
@@ -879,7 +880,7 @@ extern "C" int nvllm_kv_alloc(nvllm_model* m, int num_blocks, int block_size, in
     if (!rc) rc = dmalloc(ctx, &m->d_last_rows, (size_t)max_seqs);
     if (!rc) rc = dmalloc(ctx, &m->d_tile_order, 4 * R);
     if (!rc) rc = dmalloc(ctx, &m->d_tile_last, 4 * R);
-    if (!rc) rc = dmalloc(ctx, &m->d_group_order, R + 4);
+    if (!rc) rc = dmalloc(ctx, &m->d_group_order, 2 * (R + 4));
     if (!rc) rc = dmalloc(ctx, &m->logits, (size_t)max_seqs * m->cfg.vocab_size);  // full vocab: TP gathers here
     if (!rc) rc = dmalloc(ctx, &m->d_maxval, (size_t)max_seqs * std::max(1, ctx->tp_size) * 2);
     if (!rc) rc = dmalloc(ctx, &m->d_keys, (size_t)max_seqs);
@@ -892,10 +893,10 @@ extern "C" int nvllm_kv_alloc(nvllm_model* m, int num_blocks, int block_size, in
     if (!rc) HIPCHK(ctx, hipMemsetAsync(m->argmax_scratch, 0, ((size_t)max_seqs + 1) * 8, ctx->stream));
     if (rc) return rc;
     rc = m->dec ? m->dec->kv_alloc(m) : qwen3_kv_alloc(m);
-    // a chunk's metadata at most: three ints a row, five and a quarter a tile (every tile has a row, but for up to three that fill a
+    // a chunk's metadata at most: three ints a row, five and a half a tile (every tile has a row, but for up to three that fill a
     // sequence's last group of four), the head's rows, a pair for every block a step can take; each run padded to four
     const size_t tiles = std::min(4 * R, R + 3 * (size_t)max_seqs);
-    if (!rc) rc = stage_alloc(m, 3 * R + 5 * tiles + tiles / 4 + (size_t)max_seqs + 2 * (size_t)num_blocks + (m->dec ? m->dec->plan_ints(m) : 0) + 4 * kStageRuns);
+    if (!rc) rc = stage_alloc(m, 3 * R + 5 * tiles + tiles / 2 + (size_t)max_seqs + 2 * (size_t)num_blocks + (m->dec ? m->dec->plan_ints(m) : 0) + 4 * kStageRuns);
     if (rc) { m->num_blocks = 0; return rc; }
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
     return NVLLM_OK;
@@ -972,7 +973,8 @@ extern "C" int nvllm_debug_layer_tap(nvllm_model* m, int layer, int what, float*
 // norm should read (with n_slabs = 1).  Row-parallel outputs only (o_proj, down_proj): the
 // all-reduce the reference's RowParallelLinear lacks (src/layers/linear.rs:184-198).
 // *stride: floats between the slabs the consumer has to sum
-static int tp_reduce(nvllm_model* m, int rows, int ns, const float** in, int* n_slabs, int64_t* stride) {
+// (chunk: rows of the whole chunk, which decide the way: its last layer's few rows go the way of the others)
+static int tp_reduce(nvllm_model* m, int rows, int chunk, int ns, const float** in, int* n_slabs, int64_t* stride) {
     nvllm_ctx* ctx = m->ctx;
     *stride = (int64_t)rows * m->H;
     if (ctx->tp_size == 1) { *in = m->slabs; *n_slabs = ns; return NVLLM_OK; }
@@ -981,7 +983,7 @@ static int tp_reduce(nvllm_model* m, int rows, int ns, const float** in, int* n_
         HIPCHK(ctx, launch_slab_sum(m->slabs, ns, (int64_t)rows * m->H, nullptr, rows, m->H, m->red, ctx->stream));
         buf = m->red;
     }
-    if (ctx->oneshot && (size_t)rows * m->H <= ctx->os_slot && ((size_t)rows * m->H) % 4 == 0) {
+    if (ctx->oneshot && (size_t)chunk * m->H <= ctx->os_slot && ((size_t)rows * m->H) % 4 == 0) {
         // one-shot all-reduce (oneshot.hip): the consumer sums the tp slots like split-K slabs
         const int gen = (int)(ctx->os_calls & 1);
         const uint32_t seq = (uint32_t)(++ctx->os_calls);
@@ -1301,16 +1303,31 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
     // K splits (f32 slabs summed by the consumer): up to 4 on prompt chunks; a few hundred decode rows are MFMA-bound
     // too (hi + lo planes: 4 flops per weight byte and row) and need up to 8 to fill the chip
     const int max_ks = R <= 512 ? 8 : 4;
-    const int o_ks = tile_on ? gemm_tile_splits(R, H, KO, tmin, max_ks) : 0, d_ks = tile_on ? gemm_tile_splits(R, H, m->I_l, tmin, max_ks) : 0;
     const int q_ks = tile_on ? gemm_tile_splits(R, NQ, H, tmin, max_ks) : 0;
     const bool t_qkv = q_ks > 0 && (size_t)q_ks * R * NQ <= m->slab_floats;
     const bool t_qkv_fused = t_qkv && m->opt_tile_fuse_qk && gemm_tile_qkv_ok(R, NQ, H, hd, tmin);
-    const bool t_o = o_ks > 0 && (size_t)o_ks * R * H <= m->slab_floats;
-    const bool t_gu = tile_on && gemm_tile_ok(R, 2 * m->I_l, H, 2, tmin);
-    const bool t_down = t_gu && m->I_l % 32 == 0 && d_ks > 0 && (size_t)d_ks * R * H <= m->slab_floats;
-    m->tile_launches += (int64_t)m->L * ((int)t_qkv + (int)t_o + (int)t_gu + (int)t_down);
+    // ... and the products of `rows` rows from the output projection on
+    struct Rest { int packed; bool t_o, t_gu, t_down; };
+    auto rest_of = [&](int rows) {
+        const bool on = tmin > 0 && rows > kRowMaxRows;
+        Rest t;
+        t.packed = rows == R ? packed : 0;
+        const int ks = rows <= 512 ? 8 : 4;
+        const int o_ks = on && !t.packed ? gemm_tile_splits(rows, H, KO, tmin, ks) : 0, d_ks = on && !t.packed ? gemm_tile_splits(rows, H, m->I_l, tmin, ks) : 0;
+        t.t_o = o_ks > 0 && (size_t)o_ks * rows * H <= m->slab_floats;
+        t.t_gu = on && !t.packed && gemm_tile_ok(rows, 2 * m->I_l, H, 2, tmin);
+        t.t_down = t.t_gu && m->I_l % 32 == 0 && d_ks > 0 && (size_t)d_ks * rows * H <= m->slab_floats;
+        return t;
+    };
+    const bool alone = qt == 2 && last_rows_alone(m, R, n_last);
+    const Rest all = rest_of(R);
+    const float* resid = m->resid;
     for (int l = 0; l < m->L; ++l) {
         const LayerW& w = m->layers[l];
+        const bool trim = alone && l + 1 == m->L;
+        const Rest t = trim ? rest_of(n_last) : all;
+        const int rows = trim ? n_last : R;
+        m->tile_launches += (int)t_qkv + (int)(t.t_o && rows) + (int)(t.t_gu && rows) + (int)(t.t_down && rows);
         NormArgs na;
         na.weight = w.ln1; na.eps = eps; na.H = H; na.xh = m->xh; na.xl = m->xl; na.residual_out = m->resid; na.out_packed = packed || t_qkv;
         if (l == 0) {  // residual None: normed = norm(x), residual = x  (qwen3.rs:382-386)
@@ -1340,12 +1357,14 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
             if (rcg) return rcg;
             if (!fuse_qk) PROF(m, PROF_QK, launch_qk_norm_rope_kvwrite(qa, R, s));
         }
+        if (trim && n_last == 0) return NVLLM_OK;  // keys and values are written, nothing else of this layer is read
         AttnArgs aa;
         aa.q = m->qbuf; aa.kv = qa.kv; aa.block_tables = m->d_block_tables; aa.max_blocks = m->max_blocks;
         aa.tile_row0 = m->d_tile_row0; aa.tile_nrows = m->d_tile_nrows; aa.tile_slot = m->d_tile_slot; aa.pos = m->d_pos;
         aa.tile_last = m->d_tile_last;
         if (qt == 2) { aa.group_order = m->d_group_order; aa.longest = m->cur_max_len; }
-        aa.nh_l = m->nh_l; aa.gqa = m->gqa; aa.out_hi = m->xh; aa.out_lo = m->xl; aa.out_packed = packed || t_o;
+        const int o_packed = t.packed || t.t_o;
+        aa.nh_l = m->nh_l; aa.gqa = m->gqa; aa.out_hi = m->xh; aa.out_lo = m->xl; aa.out_packed = o_packed;
         if (qt == 1) aa.tile_order = m->d_tile_order;
         if (fuse_qk) {
             aa.qkv = qa.qkv; aa.n_slabs = qa.n_slabs; aa.slab_stride = qa.slab_stride; aa.ldqkv = NQ; aa.qn = w.qn; aa.kn = w.kn;
@@ -1358,47 +1377,62 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
             if (fuse_qk) aa.waves = m->attn_waves;
         }
         STAMPS(aa, m);
-        if (qt == 2) PROF(m, PROF_ATTN, launch_attn_prefill(aa, n_tiles, s));
+        int attn_tiles = n_tiles;
+        if (trim && qt == 2) {  // the q-tiles of wanted rows
+            aa.group_order = m->d_group_order + n_tiles / kPrefillTileGroup;
+            attn_tiles = m->last_groups * kPrefillTileGroup;
+        }
+        if (qt == 2) PROF(m, PROF_ATTN, launch_attn_prefill(aa, attn_tiles, s));
         else PROF(m, PROF_ATTN, launch_attn_paged(aa, n_tiles, R, parts_max, s));
+        const bf16_bits *ch = m->xh, *cl = m->xl;
+        float* resid_out = m->resid;
+        if (trim) {
+            GatherArgs ga;
+            ga.idx = m->d_last_rows; ga.sets = 1; ga.resid = m->resid; ga.resid_out = resid_out = m->last_resid; ga.ldr = H;
+            ga.set[0].h = m->xh; ga.set[0].l = m->xl; ga.set[0].oh = m->ctxh; ga.set[0].ol = m->ctxl;
+            ga.set[0].ld = KO; ga.set[0].in_packed = ga.set[0].out_packed = o_packed;
+            PROF(m, PROF_NORM, launch_gather_rows(ga, n_last, s));
+            ch = m->ctxh; cl = m->ctxl; resid = m->last_resid;
+        }
         // output projection (qwen3.rs:278) + TP all-reduce
         int o_slabs = 1;
-        if (t_o) PROF(m, PROF_GEMM, launch_gemm_tile(m->xh, m->xl, w.o, R, 0, m->slabs, nullptr, nullptr, 0, tmin, max_ks, &o_slabs, s));
-        else rcg = gemm_slabs(m, m->xh, m->xl, KO, w.o, m->slabs, R, 8, &o_slabs, packed);
+        if (t.t_o) PROF(m, PROF_GEMM, launch_gemm_tile(ch, cl, w.o, rows, 0, m->slabs, nullptr, nullptr, 0, tmin, max_ks, &o_slabs, s));
+        else rcg = gemm_slabs(m, ch, cl, KO, w.o, m->slabs, rows, 8, &o_slabs, t.packed);
         if (rcg) return rcg;
         const float* oin; int ons;
         int64_t ostride = 0;
-        int rc = tp_reduce(m, R, o_slabs, &oin, &ons, &ostride);
+        int rc = tp_reduce(m, rows, R, o_slabs, &oin, &ons, &ostride);
         if (rc) return rc;
         NormArgs nb;  // post-attention add + norm (qwen3.rs:393)
-        nb.in = oin; nb.n_slabs = ons; nb.slab_stride = ostride; nb.residual_in = m->resid; nb.residual_out = m->resid;
-        nb.weight = w.ln2; nb.eps = eps; nb.H = H; nb.xh = m->xh; nb.xl = m->xl; nb.out_packed = packed || t_gu;
-        PROF(m, PROF_NORM, launch_add_rmsnorm(nb, R, s));
+        nb.in = oin; nb.n_slabs = ons; nb.slab_stride = ostride; nb.residual_in = resid; nb.residual_out = resid_out;
+        nb.weight = w.ln2; nb.eps = eps; nb.H = H; nb.xh = m->xh; nb.xl = m->xl; nb.out_packed = t.packed || t.t_gu;
+        PROF(m, PROF_NORM, launch_add_rmsnorm(nb, rows, s));
         // MLP (qwen3.rs:323-327)
-        if (t_gu) {
-            PROF(m, PROF_GEMM, launch_gemm_tile(m->xh, m->xl, w.gu, R, 2, nullptr, m->xh2, m->xl2, t_down ? 1 : 0, tmin, 1, nullptr, s));
-        } else if (!packed && R <= kRowMaxRows && gemm_rowpar_ok(2 * m->I_l, H, 1, R)) {
+        if (t.t_gu) {
+            PROF(m, PROF_GEMM, launch_gemm_tile(m->xh, m->xl, w.gu, rows, 2, nullptr, m->xh2, m->xl2, t.t_down ? 1 : 0, tmin, 1, nullptr, s));
+        } else if (!t.packed && rows <= kRowMaxRows && gemm_rowpar_ok(2 * m->I_l, H, 1, rows)) {
             // small gate/up: whole-K row-parallel kernel with the SiLU*mul epilogue
             RowParArgs rg;
-            rg.xh = m->xh; rg.xl = m->xl; rg.ldx = H; rg.oh = m->xh2; rg.ol = m->xl2; rg.M = R;
+            rg.xh = m->xh; rg.xl = m->xl; rg.ldx = H; rg.oh = m->xh2; rg.ol = m->xl2; rg.M = rows;
             PROF(m, PROF_GEMM, launch_gemm_rowpar(rg, w.gu, 1, s));
-        } else if (packed || (R <= kRowMaxRows && gemm_rowpar_ok(2 * m->I_l, H, 2, R) &&
-                              (size_t)gemm_rowpar_splits(2 * m->I_l, H, 2, R) * R * 2 * m->I_l <= m->slab_floats && !m->opt_no_rowpar)) {
+        } else if (t.packed || (rows <= kRowMaxRows && gemm_rowpar_ok(2 * m->I_l, H, 2, rows) &&
+                              (size_t)gemm_rowpar_splits(2 * m->I_l, H, 2, rows) * rows * 2 * m->I_l <= m->slab_floats && !m->opt_no_rowpar)) {
             // big gate/up at few rows: stream it with K slices (f32 slabs of the INTERLEAVED gate/up rows),
             // then SiLU*mul on the summed slabs
             int gs = 1;
-            rcg = gemm_slabs(m, m->xh, m->xl, H, w.gu, m->slabs, R, 8, &gs, packed);
+            rcg = gemm_slabs(m, m->xh, m->xl, H, w.gu, m->slabs, rows, 8, &gs, t.packed);
             if (rcg) return rcg;
-            PROF(m, PROF_SILU, launch_silu_mul_interleaved(m->slabs, gs, (int64_t)R * 2 * m->I_l, R, m->I_l, m->xh2, m->xl2, packed, s));
+            PROF(m, PROF_SILU, launch_silu_mul_interleaved(m->slabs, gs, (int64_t)rows * 2 * m->I_l, rows, m->I_l, m->xh2, m->xl2, t.packed, s));
         } else {
             // gate/up GEMM with the SiLU*mul epilogue: act hi/lo written directly, no slabs, no extra launch
-            GemmPlan pg = plan_gemm_swiglu(R, 2 * m->I_l, H);
-            PROF(m, PROF_GEMM, launch_gemm_swiglu(pg, m->xh, m->xl, H, w.gu, R, m->xh2, m->xl2, nullptr, s));
+            GemmPlan pg = plan_gemm_swiglu(rows, 2 * m->I_l, H);
+            PROF(m, PROF_GEMM, launch_gemm_swiglu(pg, m->xh, m->xl, H, w.gu, rows, m->xh2, m->xl2, nullptr, s));
         }
         int d_slabs = 1;
-        if (t_down) PROF(m, PROF_GEMM, launch_gemm_tile(m->xh2, m->xl2, w.down, R, 0, m->slabs, nullptr, nullptr, 0, tmin, max_ks, &d_slabs, s));
-        else rcg = gemm_slabs(m, m->xh2, m->xl2, m->I_l, w.down, m->slabs, R, 8, &d_slabs, packed);
+        if (t.t_down) PROF(m, PROF_GEMM, launch_gemm_tile(m->xh2, m->xl2, w.down, rows, 0, m->slabs, nullptr, nullptr, 0, tmin, max_ks, &d_slabs, s));
+        else rcg = gemm_slabs(m, m->xh2, m->xl2, m->I_l, w.down, m->slabs, rows, 8, &d_slabs, t.packed);
         if (rcg) return rcg;
-        rc = tp_reduce(m, R, d_slabs, &prev, &prev_ns, &prev_stride);
+        rc = tp_reduce(m, rows, R, d_slabs, &prev, &prev_ns, &prev_stride);
         if (rc) return rc;
         if (m->taps) {
             HIPCHK(ctx, launch_slab_sum(prev, prev_ns, prev_stride, nullptr, R, H, m->tap_h + (size_t)l * m->max_rows * H, s));
@@ -1409,7 +1443,8 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
         // final add + norm on the rows that are a sequence's last token only (qwen3.rs:497), then LM head
         // on those rows (qwen3.rs:542-550 computes all rows; only row len-1 is used, llm_engine.rs:181-183)
         NormArgs nf;
-        nf.in = prev; nf.n_slabs = prev_ns; nf.slab_stride = prev_stride; nf.residual_in = m->resid; nf.row_idx = m->d_last_rows;
+        nf.in = prev; nf.n_slabs = prev_ns; nf.slab_stride = prev_stride; nf.residual_in = resid;
+        if (!alone) nf.row_idx = m->d_last_rows;
         nf.weight = m->norm; nf.eps = eps; nf.H = H; nf.xh = m->xh; nf.xl = m->xl;
         HIPCHK(ctx, launch_add_rmsnorm(nf, n_last, s));
         GemmPlan pl = plan_lmhead(n_last, m->V_l, H);
@@ -1646,6 +1681,21 @@ static int upload_chunk(nvllm_model* m, const RowPlan& p, int r0, int R, int t0,
             h_go[g] = g;
         }
         std::stable_sort(h_go, h_go + G, [&](int x, int y) { return glast[x] > glast[y]; });
+        m->last_groups = 0;
+    }
+    if (G && !m->dec && 2 * (int)last_local.size() <= R) {  // the groups with a row the head wants, in the same order
+        std::vector<char> wanted(G, 0);
+        int tile = 0;
+        for (int r : last_local) {
+            while (tile + 1 < T && (h_tn[tile] == 0 || h_t0[tile] + h_tn[tile] <= r)) ++tile;
+            wanted[tile / kPrefillTileGroup] = 1;
+        }
+        m->last_groups = (int)std::count(wanted.begin(), wanted.end(), 1);
+        if (m->last_groups) {
+            int* h_lg = put(nullptr, m->d_group_order + G, m->last_groups);
+            if (!h_lg) return fail(m->ctx, NVLLM_ESTATE, "internal: metadata block of %zu ints too small", m->stage.ints);
+            for (int g = 0, n = 0; g < G; ++g) if (wanted[h_go[g]]) h_lg[n++] = h_go[g];
+        }
     }
     return NVLLM_OK;
 }

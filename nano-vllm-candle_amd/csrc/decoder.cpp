@@ -109,6 +109,33 @@ int exact_product(nvllm_model* m, const float* x, const PackedW& w, float* out, 
     return NVLLM_OK;
 }
 
+int LastRows::alloc(nvllm_model* m, bool f32, size_t width0, size_t width1, int ldr) {
+    nvllm_ctx* ctx = m->ctx;
+    const size_t n = last_rows_cap(m), n16 = (n + 15) / 16 * 16, width[2] = {width0, width1};
+    int rc = dmalloc(ctx, &m->last_resid, n * ldr);
+    for (int i = 0; i < 2 && !rc; ++i) {
+        if (!width[i]) continue;
+        if (f32) { rc = dmalloc(ctx, &f[i], n * width[i]); continue; }
+        for (bf16_bits** p : {&h[i], &l[i]}) {  // read in whole 16-row blocks
+            if (!rc) rc = dmalloc(ctx, p, n16 * width[i]);
+            if (!rc) HIPCHK(ctx, hipMemsetAsync(*p, 0, n16 * width[i] * 2, ctx->stream));
+        }
+    }
+    return rc;
+}
+void LastRows::free() {
+    for (int i = 0; i < 2; ++i) {
+        for (void* p : {(void*)h[i], (void*)l[i], (void*)f[i]}) if (p) (void)hipFree(p);
+        h[i] = l[i] = nullptr;
+        f[i] = nullptr;
+    }
+}
+GatherSet LastRows::set(int i, const bf16_bits* xh, const bf16_bits* xl, const float* x, int ld, int in_packed, int out_packed) const {
+    GatherSet g;
+    g.h = xh; g.l = xl; g.f = x; g.oh = h[i]; g.ol = l[i]; g.of = f[i]; g.ld = ld; g.in_packed = in_packed; g.out_packed = out_packed;
+    return g;
+}
+
 int output_head(nvllm_model* m, const PackedW& head, int Kw, int Vp, const float* y, float cap, int n_last, int logits_row0) {
     nvllm_ctx* ctx = m->ctx;
     hipStream_t s = ctx->stream;

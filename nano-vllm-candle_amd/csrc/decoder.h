@@ -104,5 +104,15 @@ int run_act(nvllm_model* m, const ProductPlan& p, nvllm::Act act, const bf16_bit
 // 32-bit product of row-major f32 rows
 int exact_product(nvllm_model* m, const float* x, const PackedW& w, float* out, int R);
 
+// The last layer past its mixer (last_rows_alone): planes or f32 rows of up to two sets, and the stream in m->last_resid
+struct LastRows {
+    bf16_bits *h[2] = {nullptr, nullptr}, *l[2] = {nullptr, nullptr};
+    float* f[2] = {nullptr, nullptr};
+    int alloc(nvllm_model* m, bool f32, size_t width0, size_t width1, int ldr);  // width1 0: one set
+    void free();
+    // set i of a gather into these buffers
+    GatherSet set(int i, const bf16_bits* xh, const bf16_bits* xl, const float* x, int ld, int in_packed, int out_packed) const;
+};
+
 // logits (soft-capped when cap > 0) and arg-max of n_last normed rows: f32 rows y, or the planes m->xh / m->xl (row-major) when y is null
 int output_head(nvllm_model* m, const PackedW& head, int Kw, int Vp, const float* y, float cap, int n_last, int logits_row0);

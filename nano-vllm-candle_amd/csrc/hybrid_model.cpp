@@ -77,6 +77,7 @@ struct HybridModel : DecoderImpl {
     float *y = nullptr, *ctx_f[2] = {nullptr, nullptr}, *act_f = nullptr;  // 32-bit mode
     bf16_bits *ctx2h = nullptr, *ctx2l = nullptr;                          // the second mixer's context
     ExpertsScratch experts;
+    LastRows last_rows;
     int *d_seg = nullptr, n_seg = 0;                         // first row, rows, slot, first piece of every segment of the chunk
     int *d_piece = nullptr, n_piece = 0, piece_cap = 0;      // first row, rows of every 16-token piece
     float *pc_pair = nullptr, *pc_q = nullptr, *pc_w = nullptr, *pc_k = nullptr, *pc_decay = nullptr;
@@ -330,6 +331,7 @@ int HybridModel::create_mixer(nvllm_ctx* ctx, HybridMixer& w, const nvllm_hybrid
 }
 
 void HybridModel::free_kv() {
+    last_rows.free();
     for (HybridRun& r : runs)
         for (MixerState& s : r.st) {
             for (void* p : {s.kc, s.vc, (void*)s.state, (void*)s.history}) if (p) (void)hipFree(p);
@@ -704,6 +706,7 @@ int HybridModel::kv_alloc(nvllm_model* m) {
         if (two) for (bf16_bits** p : {&ctx2h, &ctx2l}) if (!rc) rc = zalloc((void**)p, R16 * kc * 2);
         if (ffp) for (bf16_bits** p : {&m->xh2, &m->xl2}) if (!rc) rc = zalloc((void**)p, R16 * ffp * 2);
     }
+    if (!rc) rc = last_rows.alloc(m, f32, kc, two ? kc : 0, ldr);
     piece_cap = (int)(R / kPiece) + m->max_seqs;
     struct { float** p; size_t n; } pieces[] = {{&pc_pair, ph * kPiece * kPiece}, {&pc_k, pd * kPiece}, {&pc_q, pdd * kPiece}, {&pc_w, pdd * kPiece}, {&pc_decay, pdd}};
     for (auto& b : pieces) if (!rc && b.n) rc = dmalloc(ctx, b.p, (size_t)piece_cap * b.n);
@@ -880,7 +883,11 @@ int HybridModel::forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n
     AddNormArgs base;
     base.W = cfg.width; base.ldr = ldr; base.ldx = Kw; base.eps = (float)cfg.norm_eps;
     base.ids = m->d_ids; base.embed = embed; base.embed_scale = (float)cfg.embed_scale;
-    auto plan = [&](const PackedW& w) { return f32 ? ProductPlan() : plan_product(m, R, w); };
+    // rows that go on past the last layer's mixer, and their stream
+    const bool alone = qt == 2 && last_rows_alone(m, R, n_last);
+    int rows = R;
+    float* resid = m->resid;
+    auto plan = [&](const PackedW& w) { return f32 ? ProductPlan() : plan_product(m, rows, w); };
     // the next sublayer's input: the stream or its norm `pre`, as planes in the order its product wants
     auto outputs = [&](AddNormArgs& a, const float* pre, int packed) {
         a.w[0] = pre;
@@ -905,33 +912,33 @@ int HybridModel::forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n
         a.in = sum.in; a.n_slabs = sum.n_slabs; a.slab_stride = sum.slab_stride;
         a.gather = sum.gather; a.gather_row = sum.gather_row; a.n_gather = sum.n_gather;
         a.residual_out = m->red;
-        HIPCHK(ctx, launch_add_norm(a, R, s));
+        HIPCHK(ctx, launch_add_norm(a, rows, s));
         if (sum.in2) {
-            a.in = sum.in2; a.n_slabs = sum.n_slabs2; a.slab_stride = sum.slab_stride2; a.residual_out = m->red + (size_t)R * ldr;
-            HIPCHK(ctx, launch_add_norm(a, R, s));
+            a.in = sum.in2; a.n_slabs = sum.n_slabs2; a.slab_stride = sum.slab_stride2; a.residual_out = m->red + (size_t)rows * ldr;
+            HIPCHK(ctx, launch_add_norm(a, rows, s));
         }
-        int rc = comm_allreduce_sum(ctx, m->red, (size_t)R * ldr * (sum.in2 ? 2 : 1));
+        int rc = comm_allreduce_sum(ctx, m->red, (size_t)rows * ldr * (sum.in2 ? 2 : 1));
         if (rc) return rc;
         sum.in = m->red; sum.n_slabs = 1; sum.n_gather = 0;
-        if (sum.in2) { sum.in2 = m->red + (size_t)R * ldr; sum.n_slabs2 = 1; }
+        if (sum.in2) { sum.in2 = m->red + (size_t)rows * ldr; sum.n_slabs2 = 1; }
         return NVLLM_OK;
     };
     auto add = [&](const float* weight, const float* pre, int packed, bool again) -> int {
         int rc = reduce();
         if (rc) return rc;
         AddNormArgs a = sum;
-        a.post_w = weight; a.post_mult = (float)cfg.residual_mult; a.residual_in = m->resid;
-        a.residual_out = m->resid; a.again = again;
+        a.post_w = weight; a.post_mult = (float)cfg.residual_mult; a.residual_in = resid;
+        a.residual_out = resid; a.again = again;
         outputs(a, pre, packed);
-        PROF(m, PROF_NORM, launch_add_norm(a, R, s));
+        PROF(m, PROF_NORM, launch_add_norm(a, rows, s));
         return NVLLM_OK;
     };
     auto add_tap = [&](const float* weight) -> int {  // the stream after this sublayer, left beside the stream itself
         int rc = reduce();
         if (rc) return rc;
         AddNormArgs t = sum;
-        t.post_w = weight; t.post_mult = (float)cfg.residual_mult; t.residual_in = m->resid; t.residual_out = tap;
-        HIPCHK(ctx, launch_add_norm(t, R, s));
+        t.post_w = weight; t.post_mult = (float)cfg.residual_mult; t.residual_in = resid; t.residual_out = tap;
+        HIPCHK(ctx, launch_add_norm(t, rows, s));
         return NVLLM_OK;
     };
     for (size_t run = 0; run < runs.size(); ++run) {
@@ -940,43 +947,56 @@ int HybridModel::forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n
         const HybridLayer* next = last ? nullptr : &layers[runs[run + 1].layer];
         const bool again = !last && runs[run + 1].again;
         const ProductPlan pnext = last ? ProductPlan() : plan(next->in);
+        if (last && alone) rows = n_last;
         ProductPlan po[2], pu, pd;
-        for (int b = 0; b < w.branches; ++b) po[b] = plan(w.mix[b].o);
-        if (w.ff) { pu = plan(w.up); pd = plan(w.down); }
+        for (int b = 0; b < w.branches && rows; ++b) po[b] = plan(w.mix[b].o);
+        if (w.ff && rows) { pu = plan(w.up); pd = plan(w.down); }
         int ns = 1, rc = product(m, pin, y, m->xh, m->xl, w.in, m->slabs, R, &ns);
         for (int b = 0; b < w.branches && !rc; ++b)
             rc = w.mix[b].attention() ? attention(m, w.mix[b], runs[run].st[b], b, ns, w.N, R, n_tiles, qt, po[b].packed)
                                       : recurrence(m, w.mix[b], runs[run].st[b], b, ns, w.N, R, qt, po[b].packed);
+        if (rc || !rows) return rc;  // no row of this chunk is wanted: caches and states are written
+        const bf16_bits *ch[2] = {m->ctxh, ctx2h}, *cl[2] = {m->ctxl, ctx2l};
+        const float* cf[2] = {ctx_f[0], ctx_f[1]};
+        if (last && alone) {
+            GatherArgs ga;
+            ga.idx = m->d_last_rows; ga.sets = w.branches; ga.resid = m->resid; ga.resid_out = resid = m->last_resid; ga.ldr = ldr;
+            for (int b = 0; b < w.branches; ++b) {
+                ga.set[b] = last_rows.set(b, ch[b], cl[b], cf[b], w.mix[b].Kc, po[b].packed, po[b].packed);
+                ch[b] = last_rows.h[b]; cl[b] = last_rows.l[b]; cf[b] = last_rows.f[b];
+            }
+            PROF(m, PROF_NORM, launch_gather_rows(ga, rows, s));
+        }
         sum = base;
         reduced = false;
-        sum.in = m->slabs; sum.slab_stride = (int64_t)R * ldr; sum.in_bias = w.mix[0].ob;
-        if (!rc) rc = product(m, po[0], ctx_f[0], m->ctxh, m->ctxl, w.mix[0].o, m->slabs, R, &sum.n_slabs);
+        sum.in = m->slabs; sum.slab_stride = (int64_t)rows * ldr; sum.in_bias = w.mix[0].ob;
+        rc = product(m, po[0], cf[0], ch[0], cl[0], w.mix[0].o, m->slabs, rows, &sum.n_slabs);
         if (!rc && w.branches == 2) {
-            sum.in2 = slabs2; sum.slab_stride2 = (int64_t)R * ldr;
+            sum.in2 = slabs2; sum.slab_stride2 = (int64_t)rows * ldr;
             sum.branch_w[0] = w.mix[0].out_norm; sum.branch_w[1] = w.mix[1].out_norm;
-            rc = product(m, po[1], ctx_f[1], ctx2h, ctx2l, w.mix[1].o, slabs2, R, &sum.n_slabs2);
+            rc = product(m, po[1], cf[1], ch[1], cl[1], w.mix[1].o, slabs2, rows, &sum.n_slabs2);
         }
         if (rc) return rc;
         const float* weight = w.norm1;
         if (mlp) {
-            const int packed = w.ff ? pu.packed : f32 || experts_gather(m, w.experts, R) ? 0 : 1;
+            const int packed = w.ff ? pu.packed : f32 || experts_gather(m, w.experts, rows) ? 0 : 1;
             rc = add(w.norm1, w.pre2, packed, false);
             if (rc) return rc;
             sum = base;
             reduced = false;
             if (w.ff && f32) {
-                rc = exact_product(m, y, w.up, m->slabs, R);
+                rc = exact_product(m, y, w.up, m->slabs, rows);
                 if (rc) return rc;
-                PROF(m, PROF_SILU, launch_act(w.act(), m->slabs, 1, 0, R, w.ff_p, nullptr, nullptr, 0, act_f, s));
+                PROF(m, PROF_SILU, launch_act(w.act(), m->slabs, 1, 0, rows, w.ff_p, nullptr, nullptr, 0, act_f, s));
             } else if (w.ff) {
-                rc = run_act(m, pu, w.act(), m->xh, m->xl, w.up, R, m->xh2, m->xl2, pd.packed);
+                rc = run_act(m, pu, w.act(), m->xh, m->xl, w.up, rows, m->xh2, m->xl2, pd.packed);
             }
             if (!rc && w.ff) {
-                sum.in = m->slabs; sum.slab_stride = (int64_t)R * ldr;
-                rc = product(m, pd, act_f, m->xh2, m->xl2, w.down, m->slabs, R, &sum.n_slabs);
+                sum.in = m->slabs; sum.slab_stride = (int64_t)rows * ldr;
+                rc = product(m, pd, act_f, m->xh2, m->xl2, w.down, m->slabs, rows, &sum.n_slabs);
             } else if (!rc) {
                 BranchSum ff;
-                rc = run_experts(m, w.experts, experts, m->xh, m->xl, packed, m->xh, m->xl, f32 ? y : nullptr, R, nullptr, &ff);
+                rc = run_experts(m, w.experts, experts, m->xh, m->xl, packed, m->xh, m->xl, f32 ? y : nullptr, rows, nullptr, &ff);
                 sum.gather = ff.gather; sum.gather_row = ff.gather_row; sum.n_gather = ff.n_gather;
             }
             if (rc) return rc;
@@ -993,8 +1013,8 @@ int HybridModel::forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n
             rc = reduce();
             if (rc) return rc;
             AddNormArgs a = sum;
-            a.post_w = weight; a.post_mult = (float)cfg.residual_mult; a.residual_in = m->resid;
-            a.row_idx = m->d_last_rows;
+            a.post_w = weight; a.post_mult = (float)cfg.residual_mult; a.residual_in = resid;
+            if (!alone) a.row_idx = m->d_last_rows;
             outputs(a, final_norm, 0);
             PROF(m, PROF_NORM, launch_add_norm(a, n_last, s));
         }

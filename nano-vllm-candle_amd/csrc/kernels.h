@@ -162,6 +162,24 @@ struct NormArgs {
 };
 hipError_t launch_add_rmsnorm(const NormArgs& a, int rows, hipStream_t s);
 
+// Rows idx[0..n) of activations and of the residual stream, compact
+struct GatherSet {
+    const bf16_bits *h = nullptr, *l = nullptr;  // planes [rows][ld], row-major or in fragment order ...
+    const float* f = nullptr;                    // ... or f32 rows
+    bf16_bits *oh = nullptr, *ol = nullptr;
+    float* of = nullptr;
+    int ld = 0, in_packed = 0, out_packed = 0;   // ld: a multiple of 32
+};
+struct GatherArgs {
+    const int* idx = nullptr;
+    GatherSet set[2];
+    int sets = 0;
+    const float* resid = nullptr;                // [rows][ldr], ldr a multiple of 4
+    float* resid_out = nullptr;
+    int ldr = 0;
+};
+hipError_t launch_gather_rows(const GatherArgs& a, int n, hipStream_t s);
+
 // ---- q/k norm + RoPE + KV cache write -------------------------------------------------------------
 struct KvLayout {
     f16_bits* k = nullptr;  // [num_blocks][kv_l][16 tiles][hd/32][64 lanes][8] f16 (QK^T A-fragment packed)

@@ -1747,6 +1747,38 @@ hipError_t launch_kv_write_plain(const float* k, const float* v, int rows, const
 }
 
 // ---------------------------------------------------------------------------------------------------
+// Rows the head wants, compact (what the last layer of a prompt works on after its mixer): one workgroup a row and a set.  A few hundred KB:
+// a launch's own 4 us
+// ---------------------------------------------------------------------------------------------------
+__global__ void __launch_bounds__(256) gather_rows_kernel(GatherArgs a) {
+    const int r = blockIdx.x, src = a.idx[r];
+    if ((int)blockIdx.y == a.sets) {
+        for (int i = threadIdx.x * 4; i < a.ldr; i += 1024)
+            *reinterpret_cast<float4*>(a.resid_out + (size_t)r * a.ldr + i) = *reinterpret_cast<const float4*>(a.resid + (size_t)src * a.ldr + i);
+        return;
+    }
+    const GatherSet& t = a.set[blockIdx.y];
+    if (t.f) {
+        for (int i = threadIdx.x * 4; i < t.ld; i += 1024)
+            *reinterpret_cast<float4*>(t.of + (size_t)r * t.ld + i) = *reinterpret_cast<const float4*>(t.f + (size_t)src * t.ld + i);
+        return;
+    }
+    for (int i = threadIdx.x * 8; i < t.ld; i += 2048) {
+        const size_t in = t.in_packed ? xpack_off(src, i, t.ld >> 5) : (size_t)src * t.ld + i;
+        const size_t out = t.out_packed ? xpack_off(r, i, t.ld >> 5) : (size_t)r * t.ld + i;
+        *reinterpret_cast<uint4*>(t.oh + out) = *reinterpret_cast<const uint4*>(t.h + in);
+        *reinterpret_cast<uint4*>(t.ol + out) = *reinterpret_cast<const uint4*>(t.l + in);
+    }
+}
+hipError_t launch_gather_rows(const GatherArgs& a, int n, hipStream_t s) {
+    if (n <= 0) return hipSuccess;
+    if (a.ldr % 4) return hipErrorInvalidValue;
+    for (int i = 0; i < a.sets; ++i) if (a.set[i].ld % 32) return hipErrorInvalidValue;
+    gather_rows_kernel<<<dim3(n, a.sets + 1), 256, 0, s>>>(a);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------------------------------
 // Paged causal GQA attention of decode rows.
 // Replaces qwen3.rs:236-277: GQA interleaved expand (q head h -> kv head h/(nh/kv)), scores*scale,
 // additive -1e9 mask for j>i (masked terms are exactly 0 after the f32 softmax, so they are skipped),

@@ -53,6 +53,7 @@ struct LatentModel : DecoderImpl {
     // pool and step buffers
     std::vector<void*> cache;          // per run
     float *slabs2 = nullptr, *q = nullptr, *qlat = nullptr, *olat = nullptr, *part_o = nullptr, *part_ml = nullptr, *tap = nullptr;
+    LastRows last_rows;
     bf16_bits *x2h = nullptr, *x2l = nullptr;                                                 // second norm's planes
     // expanded prompt attention: scratch keys / values, the chunk's cache tiles (device) and segments
     f16_bits *kx = nullptr, *vx = nullptr;
@@ -205,6 +206,7 @@ void LatentModel::free_kv() {
     for (size_t i = 0; i < L.cache.size(); ++i)
         if (L.cache[i] && L.layers[L.order[i]].own_kv()) (void)hipFree(L.cache[i]);
     L.cache.clear();
+    L.last_rows.free();
     L.experts.release();
     L.scan.release();
     for (LatentLayer& w : L.layers) w.scan.free_kv();
@@ -494,6 +496,7 @@ int LatentModel::kv_alloc(nvllm_model* m) {
         for (bf16_bits** p : {&m->ctxh, &m->ctxl}) if (!rc) rc = zalloc((void**)p, R16 * kc * 2);
         if (ffp) for (bf16_bits** p : {&m->xh2, &m->xl2}) if (!rc) rc = zalloc((void**)p, R16 * ffp * 2);
     }
+    if (!rc) rc = L.last_rows.alloc(m, f32, kc, L.Kw, L.ldr);
     size_t kx_row = 0, vx_row = 0;  // scratch elements per token
     for (const LatentLayer& w : L.layers)
         if (w.expands) {
@@ -692,18 +695,23 @@ int LatentModel::forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n
     base.center = L.cfg.norm == NVLLM_NORM_LAYER;
     base.W = L.cfg.width; base.ldr = L.ldr; base.ldx = L.Kw; base.eps = (float)L.cfg.norm_eps;
     base.ids = m->d_ids; base.embed = L.embed; base.embed_scale = (float)L.cfg.embed_scale;
+    // rows that go on past the last layer's mixer
+    const bool alone = qt == 2 && last_rows_alone(m, R, n_last) && !L.layers[L.order.back()].experts.on();
+    int rows = R;
     for (size_t run = 0; run < L.order.size(); ++run) {
         LatentLayer& w = L.layers[L.order[run]];
+        const bool trim = alone && run + 1 == L.order.size();
+        if (trim) rows = n_last;
         const bool gelu = w.c.glu == NVLLM_GLU_GELU;
         const GluSpec spec{gelu ? 0.f : (float)w.c.glu_limit, (float)w.c.glu_alpha, (float)w.c.glu_shift, gelu};
         ProductPlan pq, po, pd;
         GluPlan pg;
         if (!f32) {
             pq = plan_product(m, R, w.first());
-            po = plan_product(m, R, w.o);
-            if (w.ff) {
-                pd = plan_product(m, R, w.down);
-                pg = plan_glu(m, R, w.gu, pd.kind == P_TILE);
+            if (rows) po = plan_product(m, rows, w.o);
+            if (w.ff && rows) {
+                pd = plan_product(m, rows, w.down);
+                pg = plan_glu(m, rows, w.gu, pd.kind == P_TILE);
                 if (pd.packed && !pg.out_packed_ok) {
                     if (pd.kind == P_TILE) pd = ProductPlan{P_GENERIC, 0, pd.max_split};
                     else pd.packed = 0;
@@ -728,39 +736,51 @@ int LatentModel::forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n
         int ns = 1, rc = f32 ? exact_product(m, L.y1, w.first(), m->slabs, R) : run_product(m, pq, m->xh, m->xl, w.first(), m->slabs, R, &ns);
         if (!rc && w.scan.on()) rc = run_scan(m, w.scan, L.scan, m->slabs, ns, L.slabs2, R, qt, f32 ? L.ctx_f : nullptr, po.packed);
         else if (!rc) rc = latent_attention(m, w, L.cache[run], m->slabs, ns, R, n_tiles, qt, po.packed);
-        if (rc) return rc;
+        if (rc || !rows) return rc;  // no row of this chunk is wanted: caches and states are written
+        const bf16_bits *ch = m->ctxh, *cl = m->ctxl;
+        const float *cf = L.ctx_f, *resid = m->resid;
+        if (trim) {
+            GatherArgs ga;
+            ga.idx = m->d_last_rows; ga.resid = m->resid; ga.resid_out = m->last_resid; ga.ldr = L.ldr;
+            ga.set[ga.sets++] = L.last_rows.set(0, ch, cl, f32 ? cf : nullptr, w.Kc, po.packed, po.packed);
+            if (mlp) ga.set[ga.sets++] = L.last_rows.set(1, ffh, ffl, f32 ? y_ff : nullptr, L.Kw, pg.packed, pg.packed);
+            PROF(m, PROF_NORM, launch_gather_rows(ga, rows, s));
+            ch = L.last_rows.h[0]; cl = L.last_rows.l[0]; cf = L.last_rows.f[0];
+            ffh = L.last_rows.h[1]; ffl = L.last_rows.l[1]; y_ff = L.last_rows.f[1];
+            resid = m->last_resid;
+        }
         int no = 1, nd = 1;
         BranchSum ff;
         if (w.experts.on()) {
             const bool two = gathers && L.cfg.one_norm && !same;  // the mixer's planes serve the shared expert and the router
-            rc = run_experts(m, w.experts, L.experts, two ? m->xh : ffh, two ? m->xl : ffl, two ? pq.packed : pg.packed, ffh, ffl, f32 ? y_ff : nullptr, R, L.slabs2, &ff);
+            rc = run_experts(m, w.experts, L.experts, two ? m->xh : ffh, two ? m->xl : ffl, two ? pq.packed : pg.packed, ffh, ffl, f32 ? y_ff : nullptr, rows, L.slabs2, &ff);
             if (rc) return rc;
         }
         if (w.ff) {
             if (f32) {
-                rc = exact_product(m, y_ff, w.gu, m->slabs, R);
+                rc = exact_product(m, y_ff, w.gu, m->slabs, rows);
                 if (rc) return rc;
-                PROF(m, PROF_SILU, launch_silu_mul_interleaved(m->slabs, 1, 0, R, w.ff_p, nullptr, nullptr, 0, s, spec, L.act_f));
-                rc = exact_product(m, L.act_f, w.down, L.slabs2, R);
+                PROF(m, PROF_SILU, launch_silu_mul_interleaved(m->slabs, 1, 0, rows, w.ff_p, nullptr, nullptr, 0, s, spec, L.act_f));
+                rc = exact_product(m, L.act_f, w.down, L.slabs2, rows);
             } else {
-                rc = run_glu(m, pg, ffh, ffl, w.gu, R, spec, m->xh2, m->xl2, pd.packed);
-                if (!rc) rc = run_product(m, pd, m->xh2, m->xl2, w.down, L.slabs2, R, &nd);
+                rc = run_glu(m, pg, ffh, ffl, w.gu, rows, spec, m->xh2, m->xl2, pd.packed);
+                if (!rc) rc = run_product(m, pd, m->xh2, m->xl2, w.down, L.slabs2, rows, &nd);
             }
             if (rc) return rc;
-            ff.in = L.slabs2; ff.n_slabs = nd; ff.slab_stride = (int64_t)R * L.ldr;
+            ff.in = L.slabs2; ff.n_slabs = nd; ff.slab_stride = (int64_t)rows * L.ldr;
         }
-        rc = f32 ? exact_product(m, L.ctx_f, w.o, m->slabs, R) : run_product(m, po, m->ctxh, m->ctxl, w.o, m->slabs, R, &no);
+        rc = f32 ? exact_product(m, cf, w.o, m->slabs, rows) : run_product(m, po, ch, cl, w.o, m->slabs, rows, &no);
         if (rc) return rc;
         base.ids = nullptr;
-        base.in = m->slabs; base.n_slabs = no; base.slab_stride = (int64_t)R * L.ldr;
+        base.in = m->slabs; base.n_slabs = no; base.slab_stride = (int64_t)rows * L.ldr;
         base.in2 = ff.in; base.n_slabs2 = ff.n_slabs; base.slab_stride2 = ff.slab_stride; base.in2_scale = ff.scale;
         base.gather = ff.gather; base.gather_row = ff.gather_row; base.n_gather = ff.n_gather;
-        base.residual_in = m->resid;
+        base.residual_in = resid;
         if (tp) {  // both branches of the layer in one all-reduce
             AddNormArgs sum = base;
             sum.residual_in = nullptr; sum.residual_out = m->red;
-            HIPCHK(ctx, launch_add_norm(sum, R, s));
-            rc = comm_allreduce_sum(ctx, m->red, (size_t)R * L.ldr);
+            HIPCHK(ctx, launch_add_norm(sum, rows, s));
+            rc = comm_allreduce_sum(ctx, m->red, (size_t)rows * L.ldr);
             if (rc) return rc;
             base.in = m->red; base.n_slabs = 1; base.in2 = nullptr; base.n_gather = 0;
         }
@@ -774,7 +794,7 @@ int LatentModel::forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n
     }
     if (n_last <= 0) return NVLLM_OK;
     AddNormArgs nf = base;
-    nf.row_idx = m->d_last_rows;
+    if (!alone) nf.row_idx = m->d_last_rows;
     nf.w[0] = L.final_norm;
     if (f32) nf.y[0] = L.y1; else { nf.xh[0] = m->xh; nf.xl[0] = m->xl; }
     PROF(m, PROF_NORM, launch_add_norm(nf, n_last, s));

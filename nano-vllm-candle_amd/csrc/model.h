@@ -150,6 +150,7 @@ struct nvllm_model {
     int *d_pos = nullptr, *d_slot = nullptr, *d_tile_row0 = nullptr, *d_tile_nrows = nullptr, *d_tile_slot = nullptr,
         *d_last_rows = nullptr, *d_tile_order = nullptr, *d_tile_last = nullptr, *d_group_order = nullptr;
     float *resid = nullptr, *slabs = nullptr, *qbuf = nullptr, *logits = nullptr, *d_maxval = nullptr, *red = nullptr;
+    float* last_resid = nullptr;  // the residual stream of the rows the head wants, in the last layer (last_rows_alone)
     bf16_bits *xh = nullptr, *xl = nullptr, *xh2 = nullptr, *xl2 = nullptr, *ctxh = nullptr, *ctxl = nullptr;
     float *ssqA = nullptr, *ssqB = nullptr;  // deferred-norm partial sums of squares [groups][kFusedMaxRows]
     uint64_t* d_keys = nullptr;              // device sampling: per-row RNG keys and temperatures
@@ -185,6 +186,7 @@ struct nvllm_model {
     unsigned long long* argmax_scratch = nullptr;  // ticket + per-row keys of argmax_parts_kernel
     bool want_logits = false;   // this step stores the last-row logits
     int cur_n = 0;              // sequences of the step in flight
+    int last_groups = 0;        // prompt attention: groups of the chunk's q-tiles with a row the head wants, listed behind group_order
     int cur_max_len = 0;        // longest of them (tokens, the new ones included)
     size_t slab_floats = 0;
     static constexpr size_t kOutSlot = 1 << 20;
@@ -254,6 +256,11 @@ enum { PROF_ATTN = 1, PROF_GEMM = 2, PROF_NORM = 3, PROF_QK = 4, PROF_SILU = 5, 
             HIPCHK((m_)->ctx, expr_);                                                     \
         }                                                                                 \
     } while (0)
+
+// Past the last layer's mixer only the rows the head wants go on: the stream of the others is read by nothing.  Taken for prompt chunks
+// (more rows than the products of few rows, whose time is their weights', handle) of which at most half is wanted; layer taps want all rows, and so does the prompt product forced on every projection (tile_min_wgs 1).
+inline bool last_rows_alone(const nvllm_model* m, int R, int n_last) { return R > kRowMaxRows && 2 * n_last <= R && !m->taps && m->opt_tile_min_wgs != 1; }
+inline size_t last_rows_cap(const nvllm_model* m) { return std::min((size_t)m->max_seqs, (size_t)m->max_rows / 2 + 1); }
 
 // y (f32 slabs) = x.W^T with the kernel that fits the row count (api.cpp)
 int gemm_slabs(nvllm_model* m, const bf16_bits* xh, const bf16_bits* xl, int ldx, const PackedW& w, float* out, int R,
