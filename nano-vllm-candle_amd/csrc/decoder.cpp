@@ -102,9 +102,14 @@ int run_act(nvllm_model* m, const ProductPlan& p, nvllm::Act act, const bf16_bit
 }
 
 // 32-bit product of row-major f32 rows
-int exact_product(nvllm_model* m, const float* x, const PackedW& w, float* out, int R) {
+int exact_product(nvllm_model* m, const float* x, const PackedW& w, float* out, int R, int* n_slabs) {
     HeadGemmArgs a;
     a.x = x; a.x_row = w.K; a.w = w.data; a.N = a.n_valid = w.N; a.K = w.K; a.M = R; a.exact = 1; a.y = out; a.y_row = w.N;
+    if (n_slabs) {
+        a.y_slab = (int64_t)R * w.N;
+        a.splits = (int)std::max<int64_t>(1, std::min<int64_t>(exact_splits(R, w.N, w.K), (int64_t)m->slab_floats / a.y_slab));
+        *n_slabs = a.splits;
+    }
     PROF(m, PROF_GEMM, launch_head_gemm(a, m->ctx->stream));
     return NVLLM_OK;
 }

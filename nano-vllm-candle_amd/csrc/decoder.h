@@ -101,8 +101,8 @@ int run_glu(nvllm_model* m, const GluPlan& g, const bf16_bits* xh, const bf16_bi
             bf16_bits* oh, bf16_bits* ol, int out_packed);
 // activation of x.W^T as hi/lo planes oh / ol on the plan of the product, through m->slabs where no epilogue fits
 int run_act(nvllm_model* m, const ProductPlan& p, nvllm::Act act, const bf16_bits* xh, const bf16_bits* xl, const PackedW& w, int R, bf16_bits* oh, bf16_bits* ol, int out_packed);
-// 32-bit product of row-major f32 rows
-int exact_product(nvllm_model* m, const float* x, const PackedW& w, float* out, int R);
+// 32-bit product of row-major f32 rows; n_slabs: the consumer sums slabs (out is m->slabs or as large)
+int exact_product(nvllm_model* m, const float* x, const PackedW& w, float* out, int R, int* n_slabs = nullptr);
 
 // The last layer past its mixer (last_rows_alone): planes or f32 rows of up to two sets, and the stream in m->last_resid
 struct LastRows {

@@ -105,7 +105,7 @@ struct HybridModel : DecoderImpl {
     }
     int product(nvllm_model* m, const ProductPlan& p, const float* f, const bf16_bits* xh, const bf16_bits* xl, const PackedW& w, float* out, int R, int* ns) {
         *ns = 1;
-        return cfg.f32 ? exact_product(m, f, w, out, R) : run_product(m, p, xh, xl, w, out, R, ns);
+        return cfg.f32 ? exact_product(m, f, w, out, R, ns) : run_product(m, p, xh, xl, w, out, R, ns);
     }
     Segments segments(const nvllm_model* m, int R, int qt) const {
         Segments s;

@@ -2979,10 +2979,18 @@ __global__ void __launch_bounds__(1024) argmax_kernel(const float* __restrict__ 
     const float* p = logits + (size_t)blockIdx.x * ld;
     float bv = -INFINITY;
     int bi = -1;
-    for (int i = threadIdx.x; i < V; i += blockDim.x) {
-        const float v = p[i];
-        if (v >= bv || bi < 0) { bv = v; bi = i; }  // i increases per thread: >= keeps the last
+    auto take = [&](int i, float v) { if (v >= bv || bi < 0) { bv = v; bi = i; } };  // i increases per thread: >= keeps the last
+    // eight loads at a time, independent of each other: one per trip was a round trip each, 16 rows of 32768 14.4 us, now 6.9
+    int i = threadIdx.x;
+    for (; i + 7 * (int)blockDim.x < V; i += 8 * blockDim.x) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = p[i + u * blockDim.x];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) take(i + u * blockDim.x, v[u]);
     }
+    for (; i < V; i += blockDim.x) take(i, p[i]);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
         const float ov = __shfl_xor(bv, o);

@@ -120,8 +120,12 @@ struct HeadGemmArgs {
     bf16_bits* yh = nullptr;
     bf16_bits* yl = nullptr;
     int ld = 0, packed = 0;
+    int splits = 1;                // of K, by exact_splits (one head, y): split i leaves the slab y + i * y_slab
+    int64_t y_slab = 0;
 };
 hipError_t launch_head_gemm(const HeadGemmArgs& a, hipStream_t s);
+// splits of K for a 32-bit product whose consumer sums slabs
+int exact_splits(int M, int N, int K);
 
 // ---- attention over the latent cache (absorbed form) ----------------------------------------------------------------------
 // score = qlat . c + qrot . k_rot (scale folded into q); weights over positions [pos - window + 1, pos]; output the weighted

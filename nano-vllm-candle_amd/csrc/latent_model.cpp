@@ -761,7 +761,7 @@ int LatentModel::forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n
                 rc = exact_product(m, y_ff, w.gu, m->slabs, rows);
                 if (rc) return rc;
                 PROF(m, PROF_SILU, launch_silu_mul_interleaved(m->slabs, 1, 0, rows, w.ff_p, nullptr, nullptr, 0, s, spec, L.act_f));
-                rc = exact_product(m, L.act_f, w.down, L.slabs2, rows);
+                rc = exact_product(m, L.act_f, w.down, L.slabs2, rows, &nd);
             } else {
                 rc = run_glu(m, pg, ffh, ffl, w.gu, rows, spec, m->xh2, m->xl2, pd.packed);
                 if (!rc) rc = run_product(m, pd, m->xh2, m->xl2, w.down, L.slabs2, rows, &nd);
@@ -769,7 +769,7 @@ int LatentModel::forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n
             if (rc) return rc;
             ff.in = L.slabs2; ff.n_slabs = nd; ff.slab_stride = (int64_t)rows * L.ldr;
         }
-        rc = f32 ? exact_product(m, cf, w.o, m->slabs, rows) : run_product(m, po, ch, cl, w.o, m->slabs, rows, &no);
+        rc = f32 ? exact_product(m, cf, w.o, m->slabs, rows, &no) : run_product(m, po, ch, cl, w.o, m->slabs, rows, &no);
         if (rc) return rc;
         base.ids = nullptr;
         base.in = m->slabs; base.n_slabs = no; base.slab_stride = (int64_t)rows * L.ldr;

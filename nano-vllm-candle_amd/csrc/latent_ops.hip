@@ -635,22 +635,25 @@ __global__ void __launch_bounds__(256) head_gemm_kernel(HeadGemmArgs a) {
 // A 32-bit product of up to 64 rows: 16 features x MT row tiles x the whole K per workgroup, K dealt out to its NW waves, partial sums
 // met in LDS.  Bound by latency: a wave asks for U k-tiles of weights and rows at once, so a K of 1024 is one or two round trips to
 // memory, where one wave walking all of K with one k-tile in flight made 32.  Measured, 16 rows: the thirteen products of a decode step of
-// three 1024-wide layers (K 1024 to 4608, N 1024 to 8192, the head of 32768 x 1024) 40 us each before, 10 now.
+// three 1024-wide layers (K 1024 to 4608, N 1024 to 8192, the head of 32768 x 1024) 40 us each before, 10 now (7 with the splits and the
+// head's form below).
 template <int MT, int NW>
 __global__ void __launch_bounds__(NW * 64) exact_rows_kernel(HeadGemmArgs a) {
     constexpr int U = MT == 1 ? 4 : MT == 2 ? 3 : 2;
     __shared__ f32x4 part[NW][MT][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int l15 = lane & 15, grp = lane >> 4;
-    const int KT = a.K >> 5, head = blockIdx.y, m0 = blockIdx.z * (MT * 16);
-    const uint4* wp = a.w + (size_t)head * a.w_head + (size_t)blockIdx.x * KT * 64 + lane;
+    // blockIdx.y: the head, or the split of K
+    const int KTA = a.K >> 5, head = a.splits > 1 ? 0 : blockIdx.y, split = a.splits > 1 ? blockIdx.y : 0, m0 = blockIdx.z * (MT * 16);
+    const int per = (KTA + a.splits - 1) / a.splits, KT = min(KTA, (split + 1) * per);
+    const uint4* wp = a.w + (size_t)head * a.w_head + (size_t)blockIdx.x * KTA * 64 + lane;
     const float* xp[MT];
 #pragma unroll
     for (int b = 0; b < MT; ++b) xp[b] = a.x + (size_t)min(m0 + b * 16 + l15, a.M - 1) * a.x_row + (size_t)head * a.x_head + grp * 8;
     f32x4 acc[MT];
 #pragma unroll
     for (int b = 0; b < MT; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = wave; k0 < KT; k0 += U * NW) {
+    for (int k0 = split * per + wave; k0 < KT; k0 += U * NW) {
         uint4 wf[U];
         float xv[U][MT][8];
 #pragma unroll
@@ -683,12 +686,79 @@ __global__ void __launch_bounds__(NW * 64) exact_rows_kernel(HeadGemmArgs a) {
     f32x4 v = part[0][wave][lane];
 #pragma unroll
     for (int w = 1; w < NW; ++w) v += part[w][wave][lane];
+    if (split) a.y += (size_t)split * a.y_slab;
     head_gemm_put(a, head, blockIdx.x * 16 + grp * 4, m0 + wave * 16 + l15, v);
+}
+// Many features over a K that a workgroup's waves hold in one round (the head): a workgroup walks features blockIdx.x, + gridDim.x, ... with
+// the rows in registers and the next weights on their way.  One tile to a workgroup read the rows again for each: 16 rows, 32768 x 1024
+// 21.5 us, now 17.9.
+template <int NW>
+__global__ void __launch_bounds__(NW * 64) exact_rows_loop_kernel(HeadGemmArgs a) {
+    constexpr int U = 4;
+    __shared__ f32x4 part[2][NW][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l15 = lane & 15, grp = lane >> 4;
+    const int KT = a.K >> 5, ntiles = a.N >> 4;
+    const float* xp = a.x + (size_t)min(l15, a.M - 1) * a.x_row + grp * 8;
+    float xv[U][8];
+    uint4 w0[U], w1[U];
+    auto load_w = [&](int nt, uint4 (&w)[U]) {  // past the end: the last tile again, not used
+        const uint4* wp = a.w + (size_t)min(nt, ntiles - 1) * KT * 64 + lane;
+#pragma unroll
+        for (int u = 0; u < U; ++u) w[u] = wp[(size_t)min(wave + u * NW, KT - 1) * 64];
+    };
+    load_w(blockIdx.x, w0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const float* p = xp + min(wave + u * NW, KT - 1) * 32;
+        *reinterpret_cast<float4*>(&xv[u][0]) = *reinterpret_cast<const float4*>(p);
+        *reinterpret_cast<float4*>(&xv[u][4]) = *reinterpret_cast<const float4*>(p + 4);
+    }
+    int buf = 0;
+    auto tile = [&](int nt, const uint4 (&w)[U], uint4 (&wn)[U]) {
+        load_w(nt + gridDim.x, wn);
+        __builtin_amdgcn_sched_barrier(0);
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (wave + u * NW >= KT) break;  // the same for every lane of the wave
+            const uint32_t wd[4] = {w[u].x, w[u].y, w[u].z, w[u].w};
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                const float wv = (j & 1) ? __builtin_bit_cast(float, wd[j >> 1] & 0xffff0000u) : __builtin_bit_cast(float, wd[j >> 1] << 16);
+                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(wv, xv[u][j], acc, 0, 0, 0);
+            }
+        }
+        part[buf][wave][lane] = acc;
+        // the other buffer's readers are through: they are a barrier ahead of its next writers.  The weights stay in flight
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (wave == (nt & (NW - 1))) {
+            f32x4 v = part[buf][0][lane];
+#pragma unroll
+            for (int i = 1; i < NW; ++i) v += part[buf][i][lane];
+            head_gemm_put(a, 0, nt * 16 + grp * 4, l15, v);
+        }
+        buf ^= 1;
+    };
+    for (int nt = blockIdx.x; nt < ntiles; nt += 2 * gridDim.x) {
+        tile(nt, w0, w1);
+        if (nt + (int)gridDim.x < ntiles) tile(nt + gridDim.x, w1, w0);
+    }
+}
+// K in four at most where its features alone leave CUs idle: 16 rows, 1024 features, K 2048 and 4608 11.0 us both before, in four 4.5 and 7.5
+int exact_splits(int M, int N, int K) {
+    if (M > 64 || K < 1024) return 1;
+    const int wgs = N / 16 * ((M + 63) / 64);
+    return std::max(1, std::min({4, 256 / std::max(1, wgs), K / 512}));
 }
 template <int MT>
 static hipError_t exact_rows_launch(const HeadGemmArgs& a, hipStream_t s) {
-    const dim3 grid(a.N / 16, a.heads, (a.M + MT * 16 - 1) / (MT * 16));
-    if (a.K >= 2048) exact_rows_kernel<MT, 16><<<grid, 1024, 0, s>>>(a);
+    const dim3 grid(a.N / 16, a.heads * a.splits, (a.M + MT * 16 - 1) / (MT * 16));
+    if (MT == 1 && a.heads == 1 && a.splits == 1 && a.K <= 1024 && a.N >= 16384) {
+        exact_rows_loop_kernel<8><<<512, 512, 0, s>>>(a);
+        return hipGetLastError();
+    }
+    if (a.K >= (a.splits > 1 ? 1056 * a.splits : 2048)) exact_rows_kernel<MT, 16><<<grid, 1024, 0, s>>>(a);
     else exact_rows_kernel<MT, 8><<<grid, 512, 0, s>>>(a);
     return hipGetLastError();
 }
@@ -819,6 +889,7 @@ static hipError_t head_gemm_launch(const HeadGemmArgs& a, hipStream_t s) {
 hipError_t launch_head_gemm(const HeadGemmArgs& a, hipStream_t s) {
     if (a.N % 16 || a.K % 32 || a.x_row % 4 || a.x_head % 4 || a.n_valid > a.N || (!a.y && !a.yh)) return hipErrorInvalidValue;
     if (a.M <= 0) return hipSuccess;
+    if (a.splits > 1 && (!a.exact || a.M > 64 || a.K < 256 || a.heads != 1 || !a.y || a.yh || a.decay_bias)) return hipErrorInvalidValue;
     // few rows in 32 bits: K over a workgroup's waves, unless it is too short for them
     if (a.exact && a.M <= 64 && a.K >= 256) return a.M <= 16 ? exact_rows_launch<1>(a, s) : a.M <= 32 ? exact_rows_launch<2>(a, s) : exact_rows_launch<4>(a, s);
     if (a.M <= 16) return head_gemm_launch<1, 1>(a, s);

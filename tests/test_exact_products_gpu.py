@@ -5,7 +5,7 @@ import pytest
 
 from oracle import gopunex_oracle as G
 from tests.berevik_util import row_err
-from tests.gopunex_util import CONFIGS, TOL, sharp_weights
+from tests.gopunex_util import CONFIGS, TOL, attn, config, light, sharp_weights
 
 pytestmark = pytest.mark.gpu
 
@@ -52,3 +52,23 @@ def test_infinite_weights(rows):
     assert np.isinf(got[:, [5, 300]]).all()
     keep = [i for i in range(cfg["vocab"]) if i not in (5, 300)]
     assert np.array_equal(got[:, keep], want[:, keep])
+
+
+# K in parts of unlike length (1056, 2080, 4608 in 2, 4, 4), a head walked by workgroups with the rows held (512 workgroups a few tiles each, K of
+# 3 and of 32 k-tiles), both with ragged rows
+@pytest.mark.parametrize("width,ffs,vocab", [(72, (1056, 2080), 16400), (1000, (4608, 1024), 16390)])
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 64])
+def test_deep_products_and_many_features(width, ffs, vocab, rows):
+    import nano_vllm_candle_amd as pkg
+
+    cfg = config([light(ff=ffs[0]), attn(ff=ffs[1])], width=width, vocab=vocab)
+    w = sharp_weights(cfg)
+    c = pkg.GopunexConfig.from_dict(cfg, {k: np.shape(v) for k, v in w.items()})
+    m = pkg.GopunexForCausalLM.from_state_dict(c, w, dtype="float32")
+    m.kv_alloc(4, 66, max_batched_tokens=256)
+    toks = np.random.default_rng(rows).integers(0, vocab, rows).tolist()
+    got, ref = m.step_score([0], [toks], True, [list(range(rows))]), np.asarray(G.forward(cfg, w, toks))  # every row through the head: 1 to 64
+    assert row_err(got, ref) < TOL["float32"]
+    ids, logits = m.step([0], [toks], True, want_logits=True)
+    assert ids[0] == np.flatnonzero(logits[0] == logits[0].max())[-1]
+    m.close()
