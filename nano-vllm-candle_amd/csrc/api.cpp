@@ -1307,12 +1307,12 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
     const bool t_qkv = q_ks > 0 && (size_t)q_ks * R * NQ <= m->slab_floats;
     const bool t_qkv_fused = t_qkv && m->opt_tile_fuse_qk && gemm_tile_qkv_ok(R, NQ, H, hd, tmin);
     // ... and the products of `rows` rows from the output projection on
-    struct Rest { int packed; bool t_o, t_gu, t_down; };
+    struct Rest { int packed, ks; bool t_o, t_gu, t_down; };
     auto rest_of = [&](int rows) {
         const bool on = tmin > 0 && rows > kRowMaxRows;
         Rest t;
         t.packed = rows == R ? packed : 0;
-        const int ks = rows <= 512 ? 8 : 4;
+        const int ks = t.ks = rows <= 512 ? 8 : 4;
         const int o_ks = on && !t.packed ? gemm_tile_splits(rows, H, KO, tmin, ks) : 0, d_ks = on && !t.packed ? gemm_tile_splits(rows, H, m->I_l, tmin, ks) : 0;
         t.t_o = o_ks > 0 && (size_t)o_ks * rows * H <= m->slab_floats;
         t.t_gu = on && !t.packed && gemm_tile_ok(rows, 2 * m->I_l, H, 2, tmin);
@@ -1396,7 +1396,7 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
         }
         // output projection (qwen3.rs:278) + TP all-reduce
         int o_slabs = 1;
-        if (t.t_o) PROF(m, PROF_GEMM, launch_gemm_tile(ch, cl, w.o, rows, 0, m->slabs, nullptr, nullptr, 0, tmin, max_ks, &o_slabs, s));
+        if (t.t_o) PROF(m, PROF_GEMM, launch_gemm_tile(ch, cl, w.o, rows, 0, m->slabs, nullptr, nullptr, 0, tmin, t.ks, &o_slabs, s));
         else rcg = gemm_slabs(m, ch, cl, KO, w.o, m->slabs, rows, 8, &o_slabs, t.packed);
         if (rcg) return rcg;
         const float* oin; int ons;
@@ -1429,7 +1429,7 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
             PROF(m, PROF_GEMM, launch_gemm_swiglu(pg, m->xh, m->xl, H, w.gu, rows, m->xh2, m->xl2, nullptr, s));
         }
         int d_slabs = 1;
-        if (t.t_down) PROF(m, PROF_GEMM, launch_gemm_tile(m->xh2, m->xl2, w.down, rows, 0, m->slabs, nullptr, nullptr, 0, tmin, max_ks, &d_slabs, s));
+        if (t.t_down) PROF(m, PROF_GEMM, launch_gemm_tile(m->xh2, m->xl2, w.down, rows, 0, m->slabs, nullptr, nullptr, 0, tmin, t.ks, &d_slabs, s));
         else rcg = gemm_slabs(m, m->xh2, m->xl2, m->I_l, w.down, m->slabs, rows, 8, &d_slabs, t.packed);
         if (rcg) return rcg;
         rc = tp_reduce(m, rows, R, d_slabs, &prev, &prev_ns, &prev_stride);

@@ -12,6 +12,15 @@ pytestmark = pytest.mark.gpu
 SHAPES = [([129], 2048), ([1, 128], 2048), ([3] * 100, 2048), ([2] * 66, 2048), ([300, 17, 45, 1, 133], 2048), ([700, 33], 256), ([257, 600], 512)]
 
 
+@pytest.mark.parametrize("rows", [130, 255, 300])
+def test_many_wanted_rows(rows):
+    """wanted rows enough for the prompt product, with a split of K of their own beside the chunk's"""
+    import nano_vllm_candle_amd as pkg
+
+    cfg = pkg.Qwen3Config.tiny(vocab_size=1024, hidden_size=512, head_dim=128, num_attention_heads=8, num_key_value_heads=8, intermediate_size=3072)
+    check(pkg.Qwen3ForCausalLM.from_synthetic(cfg, 3), [2 + i % 3 for i in range(rows)], 2048, 2.0 ** -11)
+
+
 def check(m, lens, chunk, bound):
     """wanted: the last position, the last and a middle one, or none, by sequence; against all positions"""
     n = len(lens)
