@@ -1285,6 +1285,166 @@ __global__ void __launch_bounds__(NWK * 64) gemm_rowdir_loop_kernel(RowParArgs a
     rowdir_body<NT, NWK, TK, EPI, true>(a, wp, N, KT);
 }
 
+// Register-direct products of 65 to 256 rows: RB row blocks at a time (blocks z, z + gz, ... of blockIdx.z = z), K split over NWK waves, the
+// weights kept.  Bound by what a CU takes in (x and W of its workgroup, 0.4 to 0.6 MB) and by the phases of a round: products, K slices to
+// LDS, their sums, the epilogue.  Eight waves instead of sixteen halve the slices and have registers for two blocks, so that a round's phases
+// serve 32 rows; gate and up of a feature meet in one wave; two n-tiles of o and down halve the rows a workgroup takes in.  0.6B, us a launch,
+// the 16-wave loop / this: 200 rows q/k/v 10.0 / 8.8, gate/up 15.0 / 12.4, o and down 12.5 / 9.6 each; 117 rows gate/up 11.6 / 9.8, o and down
+// 8.6 / 7.6; 250 rows 10.4 / 9.2, 15.5 / 12.7, 12.9 / 10.1.
+template <int NT, int NWK, int TK, int RB, int EPI>
+__global__ void __launch_bounds__(NWK * 64) gemm_rowpair_kernel(RowParArgs a, const uint4* __restrict__ wp, int N, int KT) {
+    constexpr int NR = 16, PER = EPI == 1 ? 2 : 1, UNITS = RB * NT / PER, UPW = (UNITS + NWK - 1) / NWK;  // a unit: a row block's n-tile, or its gate and up
+    extern __shared__ __attribute__((aligned(16))) char smem_raw[];
+    f32x4* red = reinterpret_cast<f32x4*>(smem_raw);                                     // [NWK][RB][NT][64]
+    float* sred = reinterpret_cast<float*>(smem_raw + (size_t)NWK * RB * NT * 1024);     // [row block][4][16] rinv partials (epilogue 1)
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l15 = lane & 15, grp = lane >> 4;
+    const int tile0 = (int)blockIdx.x * NT, k0 = wave * TK, M = a.M;
+    const int blocks = (M + NR - 1) / NR, gz = gridDim.z;
+    uint4 w[NT][TK];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int j = 0; j < TK; ++j) w[t][j] = wp[((size_t)(tile0 + t) * KT + k0 + j) * 64 + lane];
+    uint4 xh[RB][TK], xl[RB][TK];
+    auto load_x = [&](int blk) {  // a block past the end: the last one again, its products are not stored
+#pragma unroll
+        for (int b = 0; b < RB; ++b) {
+            const size_t xo = (((size_t)min(blk + b * gz, blocks - 1) * KT + k0) << 9) + (size_t)lane * 8;
+#pragma unroll
+            for (int j = 0; j < TK; ++j) {
+                xh[b][j] = *reinterpret_cast<const uint4*>(a.xh + xo + j * 512);
+                xl[b][j] = *reinterpret_cast<const uint4*>(a.xl + xo + j * 512);
+            }
+        }
+    };
+    int blk = blockIdx.z;
+    load_x(blk);
+    // a unit's residual rows (epilogue 0) come behind the streams
+    float4 r4[UPW], nw4[UPW];
+    auto load_resid = [&](int blk_) {
+#pragma unroll
+        for (int i = 0; i < UPW; ++i) {
+            const int u = min(wave + i * NWK, UNITS - 1), b = u / NT, t = u - b * NT;
+            const int row = min((blk_ + b * gz) * NR + l15, M - 1);
+            r4[i] = *reinterpret_cast<const float4*>(a.resid_in + (size_t)row * N + (size_t)(tile0 + t) * 16 + grp * 4);
+            nw4[i] = *reinterpret_cast<const float4*>(a.next_w + (size_t)(tile0 + t) * 16 + grp * 4);
+        }
+    };
+    if constexpr (EPI == 0) load_resid(blk);
+    if constexpr (EPI == 1) rownorm_partials_blocks<NR>(a.rn, blk * NR, gz * NR, M, sred);
+    __builtin_amdgcn_sched_barrier(0);
+    for (;;) {
+        const int next = blk + RB * gz;
+        f32x4 acc[RB][NT];
+#pragma unroll
+        for (int b = 0; b < RB; ++b)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[b][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int b = 0; b < RB; ++b)
+#pragma unroll
+            for (int j = 0; j < TK; ++j) {
+                const bf16x8 bh = __builtin_bit_cast(bf16x8, xh[b][j]), bl = __builtin_bit_cast(bf16x8, xl[b][j]);
+#pragma unroll
+                for (int t = 0; t < NT; ++t) {
+                    const bf16x8 wv = __builtin_bit_cast(bf16x8, w[t][j]);
+                    acc[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, bh, acc[b][t], 0, 0, 0);
+                    acc[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, bl, acc[b][t], 0, 0, 0);
+                }
+            }
+#pragma unroll
+        for (int b = 0; b < RB; ++b)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) red[(size_t)((wave * RB + b) * NT + t) * 64 + lane] = acc[b][t];
+        const bool more = next < blocks;  // the same for the whole workgroup
+        if (more) {
+            load_x(next);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (not a wait for the loads in flight)
+#pragma unroll
+        for (int i = 0; i < UPW; ++i) {
+            const int u = wave + i * NWK;
+            if (UNITS % NWK && u >= UNITS) break;
+            const int b = u / (NT / PER), t = (u - b * (NT / PER)) * PER, ntile = tile0 + t;
+            const int row = (blk + b * gz) * NR + l15;
+            f32x4 sum[PER];
+#pragma unroll
+            for (int q = 0; q < PER; ++q) {
+                sum[q] = red[(size_t)(b * NT + t + q) * 64 + lane];
+#pragma unroll
+                for (int k = 1; k < NWK; ++k) sum[q] += red[(size_t)((k * RB + b) * NT + t + q) * 64 + lane];
+            }
+            if constexpr (EPI == 0) {
+                float ssq_part = 0.f;
+                if (row < M) {
+                    const size_t o = (size_t)row * N + (size_t)ntile * 16 + grp * 4;
+                    const float s0 = sum[0][0] + r4[i].x, s1 = sum[0][1] + r4[i].y, s2 = sum[0][2] + r4[i].z, s3 = sum[0][3] + r4[i].w;
+                    *reinterpret_cast<float4*>(a.resid_out + o) = make_float4(s0, s1, s2, s3);
+                    uint16_t h[4], l[4];
+                    split_bf16(s0 * nw4[i].x, h[0], l[0]); split_bf16(s1 * nw4[i].y, h[1], l[1]); split_bf16(s2 * nw4[i].z, h[2], l[2]); split_bf16(s3 * nw4[i].w, h[3], l[3]);
+                    const size_t ob = a.o_packed ? xpack_off(row, ntile * 16 + grp * 4, N >> 5) : o;
+                    *reinterpret_cast<uint2*>(a.oh + ob) = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
+                    *reinterpret_cast<uint2*>(a.ol + ob) = make_uint2(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16));
+                    ssq_part = s0 * s0 + s1 * s1 + s2 * s2 + s3 * s3;
+                }
+                ssq_part += __shfl_xor(ssq_part, 16);
+                ssq_part += __shfl_xor(ssq_part, 32);
+                if (grp == 0 && row < M) a.ssq[(size_t)ntile * a.ssq_stride + row] = ssq_part;  // a group of the norm's sum to a tile
+            } else if constexpr (EPI == 1) {
+                if (row < M) {
+                    const int I = N >> 1, pair = ntile >> 1;
+                    const float ri = rownorm_rinv_lds<NR>(a.rn, sred + b * 4 * NR, l15);
+                    uint16_t h[4], l[4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) split_bf16(glu_mul(sum[0][r] * ri, sum[PER - 1][r] * ri, a.glu), h[r], l[r]);
+                    const size_t o = a.o_packed ? xpack_off(row, pair * 16 + grp * 4, I >> 5) : (size_t)row * I + (size_t)pair * 16 + grp * 4;
+                    *reinterpret_cast<uint2*>(a.oh + o) = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
+                    *reinterpret_cast<uint2*>(a.ol + o) = make_uint2(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16));
+                }
+            } else {
+                if (row < M)
+                    *reinterpret_cast<float4*>(a.out + (size_t)row * N + (size_t)ntile * 16 + grp * 4) = make_float4(sum[0][0], sum[0][1], sum[0][2], sum[0][3]);
+            }
+        }
+        if (!more) break;
+        if constexpr (EPI == 0) load_resid(next);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // red is read
+        blk = next;
+        if constexpr (EPI == 1) sred += RB * 4 * NR;
+    }
+}
+template <int NT, int NWK, int TK, int RB, int EPI>
+static hipError_t rowpair_launch(const RowParArgs& a, const PackedW& w, hipStream_t s) {
+    const int groups = w.N / 16 / NT, blocks = (a.M + 15) / 16;
+    const size_t lds = (size_t)NWK * RB * NT * 1024 + (EPI == 1 ? (size_t)16 * 64 * 4 : 0);
+    static std::atomic<uint64_t> lds_set{0};
+    ensure_dyn_lds(reinterpret_cast<const void*>(gemm_rowpair_kernel<NT, NWK, TK, RB, EPI>), lds, lds_set);
+    // one round of the CUs; epilogue 1 holds the norms of blockDim.x / 64 blocks
+    const int gz = std::min(blocks, std::max(256 / groups, (blocks + NWK - 1) / NWK));
+    gemm_rowpair_kernel<NT, NWK, TK, RB, EPI><<<dim3(groups, 1, gz), NWK * 64, lds, s>>>(a, w.data, w.N, w.K / 32);
+    return hipGetLastError();
+}
+// 65 to 256 rows of packed planes whose shape has an instance, else hipErrorNotReady.  Up to 64 rows every workgroup has one block: the
+// 16-wave forms below are as fast or faster there (64 rows, gate/up 8.1 us against 10.6, o 4.8 against 5.6)
+template <int EPI>
+static hipError_t rowpair_dispatch(const RowParArgs& a, const PackedW& w, hipStream_t s) {
+    if (a.M <= 64 || a.M > 256 || !a.x_packed) return hipErrorNotReady;
+    if constexpr (EPI == 0) {  // up to 64 tiles: each leaves its own group of the next norm's sum, as the 16-wave form's workgroups do
+        if (w.N % 32 || w.N > 1024) return hipErrorNotReady;
+        const bool one = (a.M + 15) / 16 <= 256 / (w.N / 32);  // a block to a workgroup
+        if (w.K == 1024) return one ? rowpair_launch<2, 8, 4, 1, 0>(a, w, s) : rowpair_launch<2, 8, 4, 2, 0>(a, w, s);
+        if (w.K == 2048) return one ? rowpair_launch<2, 8, 8, 1, 0>(a, w, s) : rowpair_launch<2, 8, 8, 2, 0>(a, w, s);
+        if (w.K == 3072) return rowpair_launch<2, 8, 12, 1, 0>(a, w, s);
+    } else if constexpr (EPI == 1) {
+        if (w.K == 1024 && w.N % 96 == 0) return rowpair_launch<6, 8, 4, 2, 1>(a, w, s);
+    } else if constexpr (EPI == 2) {
+        if (w.K == 1024 && w.N % 64 == 0) return rowpair_launch<4, 8, 4, 2, 2>(a, w, s);
+    }
+    return hipErrorNotReady;
+}
+
 // shape of the register-direct kernel for (N, K, epi, M): nt == 0 -> not applicable
 struct RowDirShape { int nt, nwk, tk; };
 static RowDirShape rowdir_shape(int N, int K, int epi, int M) {
@@ -1424,7 +1584,8 @@ hipError_t launch_gemm_rowdir_qkv(const RowParArgs& a, const PackedW& w, hipStre
     if (!gemm_rowdir_qkv_ok(w.N, w.K, a.q.kv.hd, a.M) || w.N != (a.q.nh_l + 2 * a.q.kv.kv_l) * 128) return hipErrorNotSupported;
     if (a.q.kv.klo && !a.q.kv.vlo) return hipErrorInvalidValue;  // 24-bit K comes with 24-bit V only
     if (a.M <= 0) return hipSuccess;
-    return rowdir_launch_t<8, 16, 2, 5>(a, w, s);
+    // eight waves halve the K slices that meet in LDS: 117 rows 10.0 -> 9.3 us; row-major fragments, which cost a wave more each, stay with sixteen
+    return a.x_packed ? rowdir_launch_t<8, 8, 4, 5>(a, w, s) : rowdir_launch_t<8, 16, 2, 5>(a, w, s);
 }
 
 template <int MT, int NWN, int NWK, int TPW, int PH, int EPI>
@@ -1460,6 +1621,10 @@ static hipError_t rowpar_dispatch(const RowParShape& sh, const RowParArgs& a, co
 hipError_t launch_gemm_rowpar(const RowParArgs& a, const PackedW& w, int epi, hipStream_t s) {
     if (const RowDirShape d = rowdir_shape(w.N, w.K, epi, a.M); d.nt) {
         if (a.M <= 0) return hipSuccess;
+        if (epi <= 2) {
+            const hipError_t e = epi == 0 ? rowpair_dispatch<0>(a, w, s) : epi == 1 ? rowpair_dispatch<1>(a, w, s) : rowpair_dispatch<2>(a, w, s);
+            if (e != hipErrorNotReady) return e;
+        }
         if (epi == 0) return rowdir_dispatch<0>(d, a, w, s);
         if (epi == 1) return rowdir_dispatch<1>(d, a, w, s);
         if (epi == 2) return rowdir_dispatch<2>(d, a, w, s);
