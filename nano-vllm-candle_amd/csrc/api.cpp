@@ -450,11 +450,11 @@ static void free_kv(nvllm_model* m) {
     for (auto p : m->klocache) (void)hipFree(p);
     m->kcache.clear(); m->vcache.clear(); m->vlocache.clear(); m->klocache.clear();
     void* ptrs[] = {m->d_block_tables, m->d_ids, m->d_pos, m->d_slot, m->d_tile_row0, m->d_tile_nrows, m->d_tile_slot,
-                    m->d_last_rows, m->d_tile_order, m->d_tile_last, m->d_group_order, m->resid, m->last_resid, m->slabs, m->qbuf, m->logits, m->d_maxval, m->red, m->xh, m->xl, m->xh2, m->xl2, m->ctxh, m->ctxl, m->ssqA, m->ssqB, m->d_next,
+                    m->d_last_rows, m->d_tile_order, m->d_tile_last, m->d_group_order, m->resid, m->last_resid, m->slabs, m->qbuf, m->logits, m->d_maxval, m->red, m->xh, m->xl, m->xh2, m->xl2, m->ctxh, m->ctxl, m->ssqA, m->ssqB, m->ssqT, m->d_next,
                     m->part_val, m->part_idx, m->argmax_scratch, m->attn_po, m->attn_pml, m->tap_h, m->tap_res, m->cosv, m->sinv, m->tickets, m->qkv_out, m->d_keys, m->d_temps};
     for (void* p : ptrs) if (p) (void)hipFree(p);
     m->d_block_tables = nullptr; m->d_ids = nullptr; m->d_pos = m->d_slot = m->d_tile_row0 = m->d_tile_nrows = m->d_tile_slot = m->d_last_rows = m->d_tile_order = m->d_tile_last = m->d_group_order = nullptr;
-    m->resid = m->last_resid = m->slabs = m->qbuf = m->logits = m->d_maxval = m->red = nullptr; m->xh = m->xl = m->xh2 = m->xl2 = m->ctxh = m->ctxl = nullptr; m->ssqA = m->ssqB = nullptr; m->d_next = nullptr; m->part_val = nullptr; m->part_idx = nullptr; m->argmax_scratch = nullptr; m->attn_po = m->attn_pml = nullptr;
+    m->resid = m->last_resid = m->slabs = m->qbuf = m->logits = m->d_maxval = m->red = nullptr; m->xh = m->xl = m->xh2 = m->xl2 = m->ctxh = m->ctxl = nullptr; m->ssqA = m->ssqB = m->ssqT = nullptr; m->d_next = nullptr; m->part_val = nullptr; m->part_idx = nullptr; m->argmax_scratch = nullptr; m->attn_po = m->attn_pml = nullptr;
     m->tap_h = m->tap_res = nullptr; m->cosv = m->sinv = nullptr; m->tickets = nullptr; m->qkv_out = nullptr; m->d_keys = nullptr; m->d_temps = nullptr;
     stage_release(m);
     m->num_blocks = 0;
@@ -796,6 +796,7 @@ static int qwen3_kv_alloc(nvllm_model* m) {
     if (!rc) { HIPCHK(ctx, hipMemsetAsync(m->xh, 0, R16 * wide * 2, ctx->stream)); HIPCHK(ctx, hipMemsetAsync(m->xl, 0, R16 * wide * 2, ctx->stream)); }
     if (!rc) rc = dmalloc(ctx, &m->ssqA, (size_t)64 * kFusedMaxRows);  // deferred-norm partials: <= 64 groups
     if (!rc) rc = dmalloc(ctx, &m->ssqB, (size_t)64 * kFusedMaxRows);
+    if (!rc && m->H % 128 == 0) rc = dmalloc(ctx, &m->ssqT, (size_t)(m->H / 128) * R);
     if (!rc) rc = dmalloc(ctx, &m->tickets, (size_t)1024);
     if (!rc) HIPCHK(ctx, hipMemsetAsync(m->tickets, 0, 1024 * sizeof(unsigned), ctx->stream));
     if (!rc) rc = dmalloc(ctx, &m->qkv_out, (size_t)std::min<size_t>(R, kFusedMaxRows) * (m->nh_l + 2 * m->kv_l) * m->hd);
@@ -1275,6 +1276,15 @@ int gemm_slabs(nvllm_model* m, const bf16_bits* xh, const bf16_bits* xl, int ldx
     return NVLLM_OK;
 }
 
+// A chunk's o_proj and down_proj with the residual and the norm's preparation in their epilogue (launch_tile_resid), or slabs and a norm launch.
+// The epilogue wants all of K in one workgroup: below 65 workgroups the K splits of the other way fill the chip better, and outputs wider than
+// 1024 have enough of the larger blocks.  0.6B prompts, ms without / with: 600 tokens 3.77 / 4.33, 1000 4.52 / 4.95, 1100 5.33 / 5.26, 1300
+// 5.73 / 5.56, 1500 5.88 / 5.86, 1900 6.39 / 6.35, 2100 7.14 / 6.58, 2391 7.51 / 6.83, two of 1900 8.92 / 8.14, 64 of 64 to 512 40.1 / 36.9;
+// with a 24-bit cache 1300 6.34 / 6.15.
+static bool tile_resid_wins(int R, int H, int KO, int I) {
+    return H <= 1024 && (R + 127) / 128 * (H / 128) > 64 && tile_resid_ok(R, H, KO) && tile_resid_ok(R, H, I);
+}
+
 // rows R (ids/pos/slot/tiles already on the device), n_last rows listed in d_last_rows -> logits rows
 static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last, int logits_row0) {
     if (m->dec) return m->dec->forward_chunk(m, R, n_tiles, qt, n_last, logits_row0);
@@ -1298,7 +1308,7 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
     // prompt chunks (MFMA-bound): projections whose grid fills the chip run the tile GEMM (tile_gemm.hip); it reads both
     // operands in fragment order, so the kernel that produces its input planes writes them that way
     const int KO = m->nh_l * hd;
-    const int tmin = m->opt_tile_min_wgs;
+    const int tmin = m->opt_tile_min_wgs, tp = ctx->tp_size;
     const bool tile_on = !packed && tmin > 0 && R > kRowMaxRows;
     // K splits (f32 slabs summed by the consumer): up to 4 on prompt chunks; a few hundred decode rows are MFMA-bound
     // too (hi + lo planes: 4 flops per weight byte and row) and need up to 8 to fill the chip
@@ -1321,6 +1331,14 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
     };
     const bool alone = qt == 2 && last_rows_alone(m, R, n_last);
     const Rest all = rest_of(R);
+    // residual add and the next norm's preparation in the epilogues of o_proj and down_proj: the norms between two products of this chunk
+    // are no launches of their own
+    const bool fused_norms = qt == 2 && tp == 1 && !m->taps && t_qkv && all.t_o && all.t_gu && all.t_down && tile_resid_wins(R, H, KO, m->I_l);
+    RowNorm rn;  // pending on xh / xl
+    auto resid_product = [&](const bf16_bits* xh, const bf16_bits* xl, const PackedW& w, const float* next_w) -> hipError_t {
+        rn.ssq = m->ssqT; rn.groups = H / 128; rn.stride = m->max_rows; rn.inv_h = 1.0f / (float)H; rn.eps = eps;
+        return launch_tile_resid(xh, xl, w, R, m->resid, next_w, m->xh, m->xl, m->ssqT, m->max_rows, s);
+    };
     const float* resid = m->resid;
     for (int l = 0; l < m->L; ++l) {
         const LayerW& w = m->layers[l];
@@ -1335,9 +1353,10 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
         } else {       // qwen3.rs:378
             na.in = prev; na.n_slabs = prev_ns; na.slab_stride = prev_stride; na.residual_in = m->resid;
         }
-        PROF(m, PROF_NORM, launch_add_rmsnorm(na, R, s));
+        if (!rn.ssq) PROF(m, PROF_NORM, launch_add_rmsnorm(na, R, s));
         // QKV projection (qwen3.rs:205)
         QkvArgs qa;
+        qa.rn = rn;
         qa.qkv = m->slabs; qa.slab_stride = (int64_t)R * NQ; qa.qn = w.qn; qa.kn = w.kn; qa.eps = eps;
         qa.cos = m->cosv; qa.sin = m->sinv; qa.pos = m->d_pos; qa.slot = m->d_slot; qa.block_tables = m->d_block_tables;
         qa.max_blocks = m->max_blocks; qa.nh_l = m->nh_l;
@@ -1364,7 +1383,7 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
         aa.tile_last = m->d_tile_last;
         if (qt == 2) { aa.group_order = m->d_group_order; aa.longest = m->cur_max_len; }
         const int o_packed = t.packed || t.t_o;
-        aa.nh_l = m->nh_l; aa.gqa = m->gqa; aa.out_hi = m->xh; aa.out_lo = m->xl; aa.out_packed = o_packed;
+        aa.nh_l = m->nh_l; aa.gqa = m->gqa; aa.out_hi = fused_norms && !trim ? m->ctxh : m->xh; aa.out_lo = fused_norms && !trim ? m->ctxl : m->xl; aa.out_packed = o_packed;
         if (qt == 1) aa.tile_order = m->d_tile_order;
         if (fuse_qk) {
             aa.qkv = qa.qkv; aa.n_slabs = qa.n_slabs; aa.slab_stride = qa.slab_stride; aa.ldqkv = NQ; aa.qn = w.qn; aa.kn = w.kn;
@@ -1395,21 +1414,27 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
             ch = m->ctxh; cl = m->ctxl; resid = m->last_resid;
         }
         // output projection (qwen3.rs:278) + TP all-reduce
-        int o_slabs = 1;
-        if (t.t_o) PROF(m, PROF_GEMM, launch_gemm_tile(ch, cl, w.o, rows, 0, m->slabs, nullptr, nullptr, 0, tmin, t.ks, &o_slabs, s));
-        else rcg = gemm_slabs(m, ch, cl, KO, w.o, m->slabs, rows, 8, &o_slabs, t.packed);
-        if (rcg) return rcg;
-        const float* oin; int ons;
-        int64_t ostride = 0;
-        int rc = tp_reduce(m, rows, R, o_slabs, &oin, &ons, &ostride);
-        if (rc) return rc;
-        NormArgs nb;  // post-attention add + norm (qwen3.rs:393)
-        nb.in = oin; nb.n_slabs = ons; nb.slab_stride = ostride; nb.residual_in = resid; nb.residual_out = resid_out;
-        nb.weight = w.ln2; nb.eps = eps; nb.H = H; nb.xh = m->xh; nb.xl = m->xl; nb.out_packed = t.packed || t.t_gu;
-        PROF(m, PROF_NORM, launch_add_rmsnorm(nb, rows, s));
+        int rc = NVLLM_OK;
+        rn = RowNorm();
+        if (fused_norms && !trim) {
+            PROF(m, PROF_GEMM, resid_product(m->ctxh, m->ctxl, w.o, w.ln2));
+        } else {
+            int o_slabs = 1;
+            if (t.t_o) PROF(m, PROF_GEMM, launch_gemm_tile(ch, cl, w.o, rows, 0, m->slabs, nullptr, nullptr, 0, tmin, t.ks, &o_slabs, s));
+            else rcg = gemm_slabs(m, ch, cl, KO, w.o, m->slabs, rows, 8, &o_slabs, t.packed);
+            if (rcg) return rcg;
+            const float* oin; int ons;
+            int64_t ostride = 0;
+            rc = tp_reduce(m, rows, R, o_slabs, &oin, &ons, &ostride);
+            if (rc) return rc;
+            NormArgs nb;  // post-attention add + norm (qwen3.rs:393)
+            nb.in = oin; nb.n_slabs = ons; nb.slab_stride = ostride; nb.residual_in = resid; nb.residual_out = resid_out;
+            nb.weight = w.ln2; nb.eps = eps; nb.H = H; nb.xh = m->xh; nb.xl = m->xl; nb.out_packed = t.packed || t.t_gu;
+            PROF(m, PROF_NORM, launch_add_rmsnorm(nb, rows, s));
+        }
         // MLP (qwen3.rs:323-327)
         if (t.t_gu) {
-            PROF(m, PROF_GEMM, launch_gemm_tile(m->xh, m->xl, w.gu, rows, 2, nullptr, m->xh2, m->xl2, t.t_down ? 1 : 0, tmin, 1, nullptr, s));
+            PROF(m, PROF_GEMM, launch_gemm_tile(m->xh, m->xl, w.gu, rows, 2, nullptr, m->xh2, m->xl2, t.t_down ? 1 : 0, tmin, 1, nullptr, s, GluSpec(), rn));
         } else if (!t.packed && rows <= kRowMaxRows && gemm_rowpar_ok(2 * m->I_l, H, 1, rows)) {
             // small gate/up: whole-K row-parallel kernel with the SiLU*mul epilogue
             RowParArgs rg;
@@ -1427,6 +1452,11 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
             // gate/up GEMM with the SiLU*mul epilogue: act hi/lo written directly, no slabs, no extra launch
             GemmPlan pg = plan_gemm_swiglu(rows, 2 * m->I_l, H);
             PROF(m, PROF_GEMM, launch_gemm_swiglu(pg, m->xh, m->xl, H, w.gu, rows, m->xh2, m->xl2, nullptr, s));
+        }
+        rn = RowNorm();
+        if (fused_norms && l + 1 < m->L) {
+            PROF(m, PROF_GEMM, resid_product(m->xh2, m->xl2, w.down, m->layers[l + 1].ln1));
+            continue;
         }
         int d_slabs = 1;
         if (t.t_down) PROF(m, PROF_GEMM, launch_gemm_tile(m->xh2, m->xl2, w.down, rows, 0, m->slabs, nullptr, nullptr, 0, tmin, t.ks, &d_slabs, s));
@@ -1452,7 +1482,6 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
         // GEMM epilogue's per-wave partial arg-max (LAST max wins), finished by one small kernel
         float* lg = m->want_logits ? m->logits + (size_t)logits_row0 * m->V_l : nullptr;
         PROF(m, PROF_LMHEAD, launch_gemm_argmax(pl, m->xh, m->xl, H, m->lm_head, lg, n_last, m->part_val, m->part_idx, nullptr, s));
-        const int tp = ctx->tp_size;
         uint32_t* ids_dst = tp == 1 ? m->d_next + logits_row0 : m->d_next + m->cur_n + (size_t)ctx->tp_rank * m->cur_n + logits_row0;
         float* val_dst = tp == 1 ? nullptr : m->d_maxval + (size_t)ctx->tp_rank * m->cur_n + logits_row0;
         if (pl.lm_nt > 0)

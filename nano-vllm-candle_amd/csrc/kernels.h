@@ -219,12 +219,17 @@ bool gemm_tile_act_ok(int M, int N, int K, int act, int min_wgs, int max_split);
 int gemm_tile_splits(int M, int N, int K, int min_wgs, int max_split);  // 0 = shape not covered
 hipError_t launch_gemm_tile(const bf16_bits* xh, const bf16_bits* xl, const PackedW& w, int M, int mode, float* out,
                             bf16_bits* act_hi, bf16_bits* act_lo, int act_packed, int min_wgs, int max_split, int* n_slabs,
-                            hipStream_t s, const GluSpec& glu = GluSpec());
+                            hipStream_t s, const GluSpec& glu = GluSpec(), const RowNorm& rn = RowNorm());  // rn: mode 2, deferred input norm
 // mode 3 = the QKV projection of a prompt chunk with q/k-norm + RoPE + KV-cache write + q output in the epilogue
 // (qwen3.rs:205-234): needs 256-wide blocks and head_dim 128 (one wave tile = one head); qa.qkv is ignored.
 bool gemm_tile_qkv_ok(int M, int N, int K, int hd, int min_wgs);
 hipError_t launch_gemm_tile_qkv(const bf16_bits* xh, const bf16_bits* xl, const PackedW& w, int M, const QkvArgs& qa, int min_wgs,
                                 hipStream_t s);
+// narrow outputs of a prompt chunk: resid += x.W^T, oh / ol = next_w (.) resid in xpack_off order, ssq[N / 128 groups][ssq_stride] the rows' sums of
+// squares (RowNorm: the consumer multiplies by 1 / rms).  x is not oh.
+bool tile_resid_ok(int M, int N, int K);
+hipError_t launch_tile_resid(const bf16_bits* xh, const bf16_bits* xl, const PackedW& w, int M, float* resid, const float* next_w, bf16_bits* oh, bf16_bits* ol, float* ssq, int ssq_stride,
+                             hipStream_t s);
 // rows in groups that start at multiples of `align` (128 or 256), every group with weights [N x K] of its own, group g's w_group uint4 behind
 // the first: post relu2(pre x.W_g^T), or gated the post silu(g) u of interleaved gate / up features, as planes in xpack_off order (x: row-major
 // planes [x_rows][K], position p is row src[p]), or plain f32 [positions][N] (x: planes of positions in xpack_off order).  w.N, w.K: sizes of

@@ -153,6 +153,7 @@ struct nvllm_model {
     float* last_resid = nullptr;  // the residual stream of the rows the head wants, in the last layer (last_rows_alone)
     bf16_bits *xh = nullptr, *xl = nullptr, *xh2 = nullptr, *xl2 = nullptr, *ctxh = nullptr, *ctxl = nullptr;
     float *ssqA = nullptr, *ssqB = nullptr;  // deferred-norm partial sums of squares [groups][kFusedMaxRows]
+    float* ssqT = nullptr;                   // the same of a prompt chunk [H / 128][max_rows]
     uint64_t* d_keys = nullptr;              // device sampling: per-row RNG keys and temperatures
     float* d_temps = nullptr;
     // The streaming GEMM's in-launch split-K combine (epilogues 1-3) is OFF by default: measured slower than slabs + a

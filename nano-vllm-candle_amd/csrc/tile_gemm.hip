@@ -47,6 +47,7 @@ struct TileArgs {
     uint16_t* act_lo = nullptr;
     int act_packed = 0;
     GluSpec glu;                // MODE 2
+    RowNorm rn;                 // MODE 2: deferred input norm (MODE 3, 9: q.rn)
     int M = 0, N = 0, KT = 0;
     int kts = 0;                // k-tiles per K split (blockIdx.y); split y writes slab out + y*M*N (MODE 0 only)
     int MB = 0, NB = 0;         // row blocks, feature blocks
@@ -110,6 +111,24 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
         wbase += (size_t)g * a.g.w_group;
     }
     NVLLM_STAMP(a, 0);
+    // deferred input norm: 1 / rms of the block's rows, behind the ring (the K loop's barriers publish it)
+    [[maybe_unused]] float* rinv = reinterpret_cast<float*>(smem_raw + 3 * FR * 1024);
+    [[maybe_unused]] const RowNorm& rn = QKV ? a.q.rn : a.rn;
+    if constexpr (QKV || MODE == 2) {
+        if (rn.ssq && (int)threadIdx.x < WM * 64) {
+            const int row = min(mb * (WM * 64) + (int)threadIdx.x, a.M - 1);
+            float t = 0.f;
+            for (int g = 0; g < rn.groups; g += 8) {
+                float v[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[i] = rn.ssq[(size_t)min(g + i, rn.groups - 1) * rn.stride + row];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) t += g + i < rn.groups ? v[i] : 0.f;
+            }
+            rinv[threadIdx.x] = 1.0f / sqrtf(t * rn.inv_h + rn.eps);
+        }
+    }
+    [[maybe_unused]] auto rinv_of = [&](int local) { return rn.ssq ? rinv[local] : 1.0f; };
     // MODE 3: position and cache block of this lane's four tokens, fetched NOW (two dependent loads each) so that they
     // land under the K loop; in the epilogue they were 8 us of latency chain per workgroup (stamps)
     [[maybe_unused]] int e_pos[4], e_blk[4], e_slot0 = 0;
@@ -279,8 +298,6 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
     } else if constexpr (QKV) {
         static_assert(!QKV || (NTW == 8 && WN == 2), "one wave tile = one 128-wide head");
         const QkvArgs& q = a.q;
-        // the rows of the deferred norm below: compared as unsigned, the prologue's signed indices are not taken for the same values and kept
-        // (spilled, in MODE 9) through the K loop
         const int hh = wn == 0 ? nb : a.NB + nb;  // this wave's head: [q heads | k heads | v heads]
         const int nh = q.nh_l, kvl = q.kv.kv_l;
         // V heads: in the cache's PV fragment order TOKENS are the fast index (8 per 16-byte slot), while a lane here
@@ -303,7 +320,7 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
                 const int sh = P0 & 3;
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
-                    const float ri = rownorm_rinv(q.rn, (int)min((unsigned)(row0 + b * 16 + l15), (unsigned)(a.M - 1)));
+                    const float ri = rinv_of(wm * 64 + b * 16 + l15);
 #pragma unroll
                     for (int j = 0; j < 8; ++j)
 #pragma unroll
@@ -368,7 +385,7 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
                 constexpr int b = decltype(bc)::value;
                 const int row = row0 + b * 16 + l15;
                 const int pos = e_pos[b];
-                const float ri = rownorm_rinv(q.rn, (int)min((unsigned)row, (unsigned)(a.M - 1)));  // deferred input norm (1 when the planes were normalised)
+                const float ri = rinv_of(wm * 64 + b * 16 + l15);  // deferred input norm (1 when the planes were normalised)
                 // whole-vector arithmetic on the f32x4 accumulators: hipcc pairs it into v_pk_mul / v_pk_fma (two lanes' worth
                 // of flops per instruction) -- this epilogue is VALU-bound (every wave of the chip is in it at once)
                 f32x4 ss4 = {0.f, 0.f, 0.f, 0.f};
@@ -435,7 +452,7 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
             for (int b = 0; b < 4; ++b) {
                 const int row = row0 + b * 16 + l15;
                 if (row < a.M) {
-                    const float ri = rownorm_rinv(q.rn, row);
+                    const float ri = rinv_of(wm * 64 + b * 16 + l15);
                     const int pos = e_pos[b];
                     _Float16* v = reinterpret_cast<_Float16*>(q.kv.v) + (size_t)(e_blk[b] * kvl + (hh - nh - kvl)) * kBlockTokens * 128;
 #pragma unroll
@@ -475,6 +492,7 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
             if (row < a.M) {
                 [[maybe_unused]] float post = 1.f;
                 if constexpr (MODE == 7) post = a.g.post[row];
+                [[maybe_unused]] const float ri = MODE == 2 ? rinv_of(wm * 64 + b * 16 + l15) : 1.f;
 #pragma unroll
                 for (int pr = 0; pr < NTW / 2; ++pr) {
                     const int f0 = ((nt0 >> 1) + pr) * 16 + grp * 4;
@@ -482,7 +500,7 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const float g = acc[2 * pr][b][r], u = acc[2 * pr + 1][b][r];
-                        split_bf16(MODE == 7 ? silu_mul(g, u) * post : glu_mul(g, u, a.glu), h[r], l[r]);
+                        split_bf16(MODE == 7 ? silu_mul(g, u) * post : glu_mul(g * ri, u * ri, a.glu), h[r], l[r]);
                     }
                     const size_t xo = a.act_packed ? xpack_off(row, f0, I >> 5) : (size_t)row * I + f0;
                     *reinterpret_cast<uint2*>(a.act_hi + xo) = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
@@ -492,6 +510,166 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
         }
     }
     NVLLM_STAMP(a, 3);
+}
+
+// ---- narrow output, residual add and the next norm's preparation in the epilogue --------------------------------------------
+struct TileResidArgs {
+    const uint4 *xh = nullptr, *xl = nullptr, *wp = nullptr;
+    const float *resid_in = nullptr, *next_w = nullptr;
+    float *resid_out = nullptr, *ssq = nullptr;
+    uint16_t *oh = nullptr, *ol = nullptr;
+    int ssq_stride = 0, M = 0, N = 0, KT = 0, MB = 0, NB = 0, band = 1;
+};
+// One workgroup = 128 rows x 128 features x the whole K, for outputs so narrow that wider blocks would have to split K over workgroups, whose
+// slabs then go to memory and back before the residual and the norm can be added.  Here the K split is inside the workgroup: waves 0 to 3 take
+// the even k-tiles, 4 to 7 the odd ones, 64 x 64 each (12 fragments read from LDS for 32 products; eight waves of 64 x 32 over the same block
+// need 10 for 16 and are bound by those reads).  A stage is two k-tiles; three stages in the ring, copies two stages ahead; all fragments of
+// the next stage are read under this stage's products, so a stage waits once, at its barrier.  At the end the halves of the split exchange two row
+// tiles each, add the residual and leave the stream, the next norm's planes (weight times stream) and the rows' sums of squares.
+// Bound by LDS (1152 cycles a stage against 1024 of products) and the epilogue's stores, 33 MB at 4096 rows from every CU at once.
+// 0.6B, 4096 rows, o and down: two splits of 128 x 256 and the norm 38.7 + 17.2 us each, this 42.9 each; 2391 rows 37.0 + 14.6, 39.8; prompts
+// of 64 sequences (18.4 k tokens) 40.1 -> 36.9 ms.
+__global__ void __launch_bounds__(512) tile_resid_kernel(TileResidArgs a) {
+    constexpr int FR1 = 24, FR = 2 * FR1;  // 1 KiB fragments of a k-tile (8 of W, 8 + 8 of x) and of a stage
+    extern __shared__ __attribute__((aligned(16))) char smem_raw[];
+    uint4* lds = reinterpret_cast<uint4*>(smem_raw);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l15 = lane & 15, grp = lane >> 4;
+    const int kg = wave >> 2, wm = (wave >> 1) & 1, wn = wave & 1;
+    int mb, nb;
+    {
+        const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, b = xcd * ((int)gridDim.x >> 3) + slot;
+        if (b >= a.MB * a.NB) return;  // whole workgroup, before any barrier
+        const int group = b / (a.band * a.NB), r = b - group * a.band * a.NB, high = min(a.band, a.MB - group * a.band);
+        nb = r / high;
+        mb = group * a.band + r - nb * high;
+    }
+    const int NS = a.KT >> 1, mtiles = (a.M + 15) >> 4;
+    // the residual of this wave's own two row tiles comes before the streams
+    const int row0 = mb * 128 + wm * 64 + kg * 32 + l15, f0 = nb * 128 + wn * 64 + grp * 4;
+    float4 r4[2][4];
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) r4[b][j] = *reinterpret_cast<const float4*>(a.resid_in + (size_t)min(row0 + b * 16, a.M - 1) * a.N + f0 + j * 16);
+    __builtin_amdgcn_sched_barrier(0);
+    const uint4* sw = a.wp + (size_t)(nb * 8 + wave) * a.KT * 64 + lane;
+    const size_t xo = (size_t)min(mb * 8 + wave, mtiles - 1) * a.KT * 64 + lane;  // past the end: the last row tile again, not stored
+    const uint4 *sh = a.xh + xo, *sl = a.xl + xo;
+    auto issue2 = [&](int s, int buf, int part) {  // copies 2 part and 2 part + 1 of the six of stage s (past the end: the last stage again)
+        const size_t koff = (size_t)min(s, NS - 1) * 128;
+#pragma unroll
+        for (int c = 2 * part; c < 2 * part + 2; ++c) {
+            const int h = c / 3, k = c % 3;
+            const uint4* src = (k == 0 ? sw : k == 1 ? sh : sl) + koff + h * 64;
+            __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)(lds + (size_t)(buf * FR + h * FR1 + k * 8 + wave) * 64), 16, 0, 0);
+        }
+    };
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(lptr_t)smem_raw;
+    uint32_t w_at[3], x_at[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        w_at[i] = lds0 + (uint32_t)((i * FR + kg * FR1 + wn * 4) * 64 + lane) * 16;
+        x_at[i] = lds0 + (uint32_t)((i * FR + kg * FR1 + 8 + wm * 4) * 64 + lane) * 16;
+    }
+    f32x4 acc[4][4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) acc[j][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 WA[4], HA[4], LA[4], WB[4], HB[4], LB[4];
+#define NVLLM_RD(DST_, ADDR_, OFF_) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(DST_) : "v"(ADDR_), "n"(OFF_))
+#define NVLLM_RD_SET(W_, H_, L_, WP_, XP_)                                                                                   \
+    do {                                                                                                                      \
+        NVLLM_RD(W_[0], WP_, 0); NVLLM_RD(W_[1], WP_, 1024); NVLLM_RD(W_[2], WP_, 2048); NVLLM_RD(W_[3], WP_, 3072);          \
+        NVLLM_RD(H_[0], XP_, 0); NVLLM_RD(L_[0], XP_, 8192); NVLLM_RD(H_[1], XP_, 1024); NVLLM_RD(L_[1], XP_, 9216);          \
+        NVLLM_RD(H_[2], XP_, 2048); NVLLM_RD(L_[2], XP_, 10240); NVLLM_RD(H_[3], XP_, 3072); NVLLM_RD(L_[3], XP_, 11264);     \
+    } while (0)
+// the set's reads have arrived (the operands tie it to their uses), this wave's copies of the stage after it too; then every wave's
+#define NVLLM_SET_READY(W_, H_, L_, VM_)                                                                                     \
+    asm volatile("s_waitcnt vmcnt(" VM_ ") lgkmcnt(0)\n\ts_barrier"                                                          \
+                 : "+v"(W_[0]), "+v"(W_[1]), "+v"(W_[2]), "+v"(W_[3]), "+v"(H_[0]), "+v"(H_[1]), "+v"(H_[2]), "+v"(H_[3]),    \
+                   "+v"(L_[0]), "+v"(L_[1]), "+v"(L_[2]), "+v"(L_[3])::"memory")
+#define NVLLM_MM(W_, H_, L_, B_)                                                                                             \
+    do {                                                                                                                      \
+        _Pragma("unroll") for (int j = 0; j < 4; ++j) acc[j][B_] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W_[j], H_[B_], acc[j][B_], 0, 0, 0); \
+        _Pragma("unroll") for (int j = 0; j < 4; ++j) acc[j][B_] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W_[j], L_[B_], acc[j][B_], 0, 0, 0); \
+        __builtin_amdgcn_sched_barrier(0);                                                                                    \
+    } while (0)
+#define NVLLM_STAGE(W_, H_, L_, WN_, HN_, LN_, S_)                                                                           \
+    do {                                                                                                                      \
+        NVLLM_SET_READY(W_, H_, L_, "6");                                                                                     \
+        NVLLM_RD_SET(WN_, HN_, LN_, w_at[1], x_at[1]);                                                                        \
+        __builtin_amdgcn_sched_barrier(0);                                                                                    \
+        NVLLM_MM(W_, H_, L_, 0);                                                                                              \
+        issue2((S_) + 3, cur, 0);                                                                                             \
+        __builtin_amdgcn_sched_barrier(0);                                                                                    \
+        NVLLM_MM(W_, H_, L_, 1);                                                                                              \
+        issue2((S_) + 3, cur, 1);                                                                                             \
+        __builtin_amdgcn_sched_barrier(0);                                                                                    \
+        NVLLM_MM(W_, H_, L_, 2);                                                                                              \
+        issue2((S_) + 3, cur, 2);                                                                                             \
+        __builtin_amdgcn_sched_barrier(0);                                                                                    \
+        NVLLM_MM(W_, H_, L_, 3);                                                                                              \
+        cur = cur == 2 ? 0 : cur + 1;                                                                                         \
+        { const uint32_t t_ = w_at[0]; w_at[0] = w_at[1]; w_at[1] = w_at[2]; w_at[2] = t_; }                                  \
+        { const uint32_t t_ = x_at[0]; x_at[0] = x_at[1]; x_at[1] = x_at[2]; x_at[2] = t_; }                                  \
+    } while (0)
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int p = 0; p < 3; ++p) issue2(i, i, p);
+    asm volatile("s_waitcnt vmcnt(12)\n\ts_barrier" ::: "memory");
+    NVLLM_RD_SET(WA, HA, LA, w_at[0], x_at[0]);
+    int cur = 0;
+    for (int s = 0; s < NS; s += 2) {  // NS is even (host)
+        NVLLM_STAGE(WA, HA, LA, WB, HB, LB, s);
+        NVLLM_STAGE(WB, HB, LB, WA, HA, LA, s + 1);
+    }
+    NVLLM_SET_READY(WA, HA, LA, "0");  // the reads and copies past the end; the ring is free
+#undef NVLLM_STAGE
+#undef NVLLM_MM
+#undef NVLLM_SET_READY
+#undef NVLLM_RD_SET
+#undef NVLLM_RD
+    // each half of the K split keeps two row tiles and hands the others to its partner
+    f32x4* xch = reinterpret_cast<f32x4*>(smem_raw);                        // [8 waves][2][4][64]
+    float* red = reinterpret_cast<float*>(smem_raw + 8 * 8 * 1024);         // [wm][4 row tiles][16]
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) xch[((wave * 2 + b) * 4 + j) * 64 + lane] = kg ? acc[j][b] : acc[j][2 + b];
+    __syncthreads();
+    float ss[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+        const int row = row0 + b * 16;
+        ss[b] = 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const f32x4 other = xch[(((wave ^ 4) * 2 + b) * 4 + j) * 64 + lane], own = kg ? acc[j][2 + b] : acc[j][b];
+            const f32x4 v = kg ? other + own : own + other;
+            const float s0 = v[0] + r4[b][j].x, s1 = v[1] + r4[b][j].y, s2 = v[2] + r4[b][j].z, s3 = v[3] + r4[b][j].w;
+            if (row < a.M) {
+                const float4 w4 = *reinterpret_cast<const float4*>(a.next_w + f0 + j * 16);
+                *reinterpret_cast<float4*>(a.resid_out + (size_t)row * a.N + f0 + j * 16) = make_float4(s0, s1, s2, s3);
+                uint16_t h[4], l[4];
+                split_bf16(s0 * w4.x, h[0], l[0]); split_bf16(s1 * w4.y, h[1], l[1]); split_bf16(s2 * w4.z, h[2], l[2]); split_bf16(s3 * w4.w, h[3], l[3]);
+                const size_t o = xpack_off(row, f0 + j * 16, a.N >> 5);
+                *reinterpret_cast<uint2*>(a.oh + o) = make_uint2(h[0] | ((uint32_t)h[1] << 16), h[2] | ((uint32_t)h[3] << 16));
+                *reinterpret_cast<uint2*>(a.ol + o) = make_uint2(l[0] | ((uint32_t)l[1] << 16), l[2] | ((uint32_t)l[3] << 16));
+            }
+            ss[b] += (s0 * s0 + s1 * s1) + (s2 * s2 + s3 * s3);
+        }
+        ss[b] += __shfl_xor(ss[b], 16);
+        ss[b] += __shfl_xor(ss[b], 32);
+        if (wn == 1 && grp == 0) red[(wm * 4 + kg * 2 + b) * 16 + l15] = ss[b];
+    }
+    __syncthreads();
+    if (wn == 0 && grp == 0)
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+            if (row0 + b * 16 < a.M) a.ssq[(size_t)nb * a.ssq_stride + row0 + b * 16] = ss[b] + red[(wm * 4 + kg * 2 + b) * 16 + l15];
 }
 
 // ---- host side -------------------------------------------------------------------------------------
@@ -526,6 +704,23 @@ static TileShape tile_shape(int M, int N, int K, int mode, int min_wgs, int max_
     return best;
 }
 
+bool tile_resid_ok(int M, int N, int K) { return M > 0 && N % 128 == 0 && N / 128 <= 64 && K % 128 == 0; }
+hipError_t launch_tile_resid(const bf16_bits* xh, const bf16_bits* xl, const PackedW& w, int M, float* resid, const float* next_w, bf16_bits* oh, bf16_bits* ol, float* ssq, int ssq_stride,
+                             hipStream_t s) {
+    if (!tile_resid_ok(M, w.N, w.K)) return hipErrorNotSupported;
+    TileResidArgs a;
+    a.xh = reinterpret_cast<const uint4*>(xh); a.xl = reinterpret_cast<const uint4*>(xl); a.wp = w.data;
+    a.resid_in = resid; a.resid_out = resid; a.next_w = next_w; a.oh = oh; a.ol = ol; a.ssq = ssq; a.ssq_stride = ssq_stride;
+    a.M = M; a.N = w.N; a.KT = w.K / 32; a.MB = (M + 127) / 128; a.NB = w.N / 128;
+    const int per = (a.MB * a.NB + 7) / 8;
+    a.band = std::min(a.MB, std::max(1, (int)std::lround(std::sqrt(per / 2.0))));
+    const size_t lds = (size_t)3 * 48 * 1024;
+    static std::atomic<uint64_t> lds_set{0};
+    ensure_dyn_lds(reinterpret_cast<const void*>(tile_resid_kernel), lds, lds_set);
+    tile_resid_kernel<<<8 * per, 512, lds, s>>>(a);
+    return hipGetLastError();
+}
+
 bool gemm_tile_ok(int M, int N, int K, int mode, int min_wgs) { return tile_shape(M, N, K, mode, min_wgs, 1).ntw != 0; }
 // An activation in the epilogue wants the whole K in one workgroup.  Where splitting K would fill the chip instead, the product of f32 slabs
 // and a launch that sums them and applies the activation, about 5 us, can be the faster pair; by the cost above.  129 rows, N 4608, K 1024:
@@ -554,7 +749,7 @@ static hipError_t tile_launch_t(TileArgs& a, int ks, hipStream_t s) {
     } else if (a.MB >= 8) { a.map = 1; grid = ((a.MB + 7) / 8) * 8 * a.NB; }
     else if (a.NB >= 8) { a.map = 2; grid = ((a.NB + 7) / 8) * 8 * a.MB; }
     else { a.map = 0; grid = a.MB * a.NB; }
-    const size_t lds = (size_t)3 * FR * 1024;
+    const size_t lds = (size_t)3 * FR * 1024 + (MODE == 2 || MODE == 3 || MODE == 9 ? (size_t)rows * 4 : 0);
     static std::atomic<uint64_t> lds_set{0};
     ensure_dyn_lds(reinterpret_cast<const void*>(gemm_tile_kernel<NTW, WN, MODE>), lds, lds_set);
 #ifdef NVLLM_STAMPS
@@ -568,14 +763,15 @@ static hipError_t tile_launch_t(TileArgs& a, int ks, hipStream_t s) {
 // n_slabs (nullable): K splits the launch wrote (out = [n_slabs][M][N]); nullptr -> never split
 hipError_t launch_gemm_tile(const bf16_bits* xh, const bf16_bits* xl, const PackedW& w, int M, int mode, float* out,
                             bf16_bits* act_hi, bf16_bits* act_lo, int act_packed, int min_wgs, int max_split, int* n_slabs,
-                            hipStream_t s, const GluSpec& glu) {
+                            hipStream_t s, const GluSpec& glu, const RowNorm& rn) {
     const TileShape t = tile_shape(M, w.N, w.K, mode, min_wgs, n_slabs ? max_split : 1);
     if (!t.ntw) return hipErrorNotSupported;
     if (mode == 2 && act_packed && (w.N / 2) % 32 != 0) return hipErrorNotSupported;
     if (mode >= 4 && act_packed && w.N % 32 != 0) return hipErrorNotSupported;
     TileArgs a;
     a.xh = reinterpret_cast<const uint4*>(xh); a.xl = reinterpret_cast<const uint4*>(xl); a.wp = w.data;
-    a.out = out; a.act_hi = act_hi; a.act_lo = act_lo; a.act_packed = act_packed; a.glu = glu;
+    if (rn.ssq && (mode != 2 || rn.row_idx)) return hipErrorNotSupported;
+    a.out = out; a.act_hi = act_hi; a.act_lo = act_lo; a.act_packed = act_packed; a.glu = glu; a.rn = rn;
     a.M = M; a.N = w.N; a.KT = w.K / 32;
     if (n_slabs) *n_slabs = t.ks;
     if (mode == 0) {
@@ -609,7 +805,6 @@ bool gemm_tile_qkv_ok(int M, int N, int K, int hd, int min_wgs) {
 hipError_t launch_gemm_tile_qkv(const bf16_bits* xh, const bf16_bits* xl, const PackedW& w, int M, const QkvArgs& qa, int min_wgs,
                                 hipStream_t s) {
     if (!gemm_tile_qkv_ok(M, w.N, w.K, qa.kv.hd, min_wgs) || w.N != (qa.nh_l + 2 * qa.kv.kv_l) * 128) return hipErrorNotSupported;
-    if (qa.rn.ssq && qa.rn.groups != 1) return hipErrorNotSupported;
     if (qa.kv.klo && !qa.kv.vlo) return hipErrorInvalidValue;  // 24-bit K comes with 24-bit V only
     TileArgs a;
     a.xh = reinterpret_cast<const uint4*>(xh); a.xl = reinterpret_cast<const uint4*>(xl); a.wp = w.data;
