@@ -175,10 +175,11 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
     }
     // k-tile s (clamped: the two issues past the end re-fetch the last k-tile into a stage nobody reads, so the
     // stage body has no branch) -> LDS stage `buf`
-    auto issue = [&](int s, int buf) {
+    auto issue_part = [&](int s, int buf, int i0, int i1) {  // copies i0 .. i1 - 1 of the stage
         const size_t koff = (size_t)min(s, KT - 1) * 64;
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
+            if (i < i0 || i >= i1) continue;
             const int f = wave + 8 * i;
             if constexpr (GATHER) {
                 if (FR % 8 == 0 || f < FR)
@@ -187,6 +188,7 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
                 __builtin_amdgcn_global_load_lds((gptr_t)(src[i] + koff + lane), (lptr_t)(lds + (size_t)(buf * FR + f) * 64), 16, 0, 0);
         }
     };
+    auto issue = [&](int s, int buf) { issue_part(s, buf, 0, NI); };
     // LDS byte addresses this lane reads in the three stages: W fragments of this wave's features, x fragments of its
     // rows.  The fragment reads are inline asm with hand-counted lgkmcnt waits: left to hipcc (ROCm 7.2) every wait in
     // this loop came out as lgkmcnt(0), i.e. each sub-step also waited for the reads it had just issued for the next one.
@@ -210,6 +212,63 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
     // barriers ago is free).  One asm statement: the compiler can neither split it nor move LDS reads across it.
     auto publish = [&]() { asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory"); };
 
+    if constexpr (NTW == 4) {
+        // 128 x 256 blocks are bound by LDS (1024 cycles a stage, as many as their products), and their sub-steps of eight products are too
+        // short to hide its reads: their accumulators leave registers for two whole sets of fragments, so the next stage's are read under
+        // this stage's products and a stage waits once, at its barrier; its slot is free from the start, and copies go two stages ahead
+        // (slot s % 3 takes stage s + 3).  6.9 k tokens of a 1024-wide decoder, o and down 39.8 -> 35.2 us, 800 of 0.6B, gate/up 30.9 -> 28.0.
+        // 256 x 192 blocks, bound by their products, lost (gate/up of 4096 rows 76.6 -> 80.4, 8B q/k/v 312 -> 322).
+        constexpr int VM = FR / 8;  // copies of a wave in a stage, at least: those of the stage after next stay in flight
+        bf16x8 WA[NTW], HA[4], LA[4], WB[NTW], HB[4], LB[4];
+#define NVLLM_RD_SET(W_, H_, L_, WP_, XP_)                                                                   \
+    do {                                                                                                     \
+        _Pragma("unroll") for (int j = 0; j < NTW; ++j) NVLLM_WF(W_[j], WP_, j);                             \
+        _Pragma("unroll") for (int b = 0; b < 4; ++b) { NVLLM_XF(H_[b], XP_, 0, b); NVLLM_XF(L_[b], XP_, 1, b); } \
+    } while (0)
+// the set's reads have arrived and the next stage's copies of every wave; the empty statements tie the registers to the wait
+#define NVLLM_SET_READY(W_, H_, L_, VM_)                                                                     \
+    do {                                                                                                     \
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(VM_) : "memory");                  \
+        _Pragma("unroll") for (int j = 0; j < NTW; ++j) asm volatile("" : "+v"(W_[j]));                      \
+        _Pragma("unroll") for (int b = 0; b < 4; ++b) { asm volatile("" : "+v"(H_[b])); asm volatile("" : "+v"(L_[b])); } \
+    } while (0)
+#define NVLLM_MM(W_, X_, B_)                                                                                 \
+    do {                                                                                                     \
+        _Pragma("unroll") for (int j = 0; j < NTW; ++j)                                                      \
+            acc[j][B_] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W_[j], X_, acc[j][B_], 0, 0, 0);            \
+    } while (0)
+#define NVLLM_TILE_STAGE(W_, H_, L_, WN_, HN_, LN_, S_)                                                      \
+    do {                                                                                                     \
+        NVLLM_SET_READY(W_, H_, L_, VM);                                                                     \
+        NVLLM_RD_SET(WN_, HN_, LN_, w_nxt, x_nxt);                                                           \
+        __builtin_amdgcn_sched_barrier(0);                                                                   \
+        _Pragma("unroll") for (int b = 0; b < 4; ++b) {                                                      \
+            NVLLM_MM(W_, H_[b], b);                                                                          \
+            NVLLM_MM(W_, L_[b], b);                                                                          \
+            __builtin_amdgcn_sched_barrier(0);                                                               \
+            issue_part((S_) + 3, cur_i, b * NI / 4, (b + 1) * NI / 4);                                       \
+            __builtin_amdgcn_sched_barrier(0);                                                               \
+        }                                                                                                    \
+        { const uint32_t t_ = w_cur; w_cur = w_nxt; w_nxt = w_fre; w_fre = t_; }                             \
+        { const uint32_t t_ = x_cur; x_cur = x_nxt; x_nxt = x_fre; x_fre = t_; }                             \
+        { const int t_ = cur_i; cur_i = nxt_i; nxt_i = fre; fre = t_; }                                      \
+    } while (0)
+        issue(0, 0);
+        issue(1, 1);
+        issue(2, 2);
+        asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * VM) : "memory");
+        NVLLM_STAMP(a, 1);
+        NVLLM_RD_SET(WA, HA, LA, w_cur, x_cur);
+        for (int s = 0; s < KT; s += 2) {  // KT is even (host)
+            NVLLM_TILE_STAGE(WA, HA, LA, WB, HB, LB, s);
+            NVLLM_TILE_STAGE(WB, HB, LB, WA, HA, LA, s + 1);
+        }
+        NVLLM_SET_READY(WA, HA, LA, 0);  // the reads and copies past the end
+#undef NVLLM_TILE_STAGE
+#undef NVLLM_MM
+#undef NVLLM_SET_READY
+#undef NVLLM_RD_SET
+    } else {
     issue(0, 0);
     issue(1, 1);
     publish();
@@ -272,6 +331,7 @@ __global__ void __launch_bounds__(512) gemm_tile_kernel(TileArgs a) {
 #undef NVLLM_TILE_STAGE
 #undef NVLLM_TILE_MFMA_HALF
 #undef NVLLM_SB
+    }
 #undef NVLLM_WF
 #undef NVLLM_XF
 #undef NVLLM_LDSR
