@@ -1277,12 +1277,12 @@ int gemm_slabs(nvllm_model* m, const bf16_bits* xh, const bf16_bits* xl, int ldx
 }
 
 // A chunk's o_proj and down_proj with the residual and the norm's preparation in their epilogue (launch_tile_resid), or slabs and a norm launch.
-// The epilogue wants all of K in one workgroup: below 65 workgroups the K splits of the other way fill the chip better, and outputs wider than
-// 1024 have enough of the larger blocks.  0.6B prompts, ms without / with: 600 tokens 3.77 / 4.33, 1000 4.52 / 4.95, 1100 5.33 / 5.26, 1300
-// 5.73 / 5.56, 1500 5.88 / 5.86, 1900 6.39 / 6.35, 2100 7.14 / 6.58, 2391 7.51 / 6.83, two of 1900 8.92 / 8.14, 64 of 64 to 512 40.1 / 36.9;
-// with a 24-bit cache 1300 6.34 / 6.15.
+// The epilogue wants all of K in one workgroup: below 128 workgroups of its smallest blocks the K splits of the other way fill the chip better,
+// and outputs wider than 1024 have enough of the larger blocks.  0.6B prompts, ms without / with: 300 tokens 3.05 / 3.14, 450 3.26 / 3.28, 600
+// 3.74 / 3.52, 800 4.18 / 3.92, 1000 4.41 / 4.11, 1280 5.19 / 4.77, 1500 5.64 / 5.14, 2020 6.63 / 6.07, 2391 7.51 / 6.79, 3000 8.56 / 8.05, 4000
+// 10.85 / 10.20; 64 of 64 to 512 40.1 / 36.9.
 static bool tile_resid_wins(int R, int H, int KO, int I) {
-    return H <= 1024 && (R + 127) / 128 * (H / 128) > 64 && tile_resid_ok(R, H, KO) && tile_resid_ok(R, H, I);
+    return H <= 1024 && (R + 31) / 32 * (H / 128) >= 128 && tile_resid_ok(R, H, KO) && tile_resid_ok(R, H, I);
 }
 
 // rows R (ids/pos/slot/tiles already on the device), n_last rows listed in d_last_rows -> logits rows

@@ -580,17 +580,20 @@ struct TileResidArgs {
     uint16_t *oh = nullptr, *ol = nullptr;
     int ssq_stride = 0, M = 0, N = 0, KT = 0, MB = 0, NB = 0, band = 1;
 };
-// One workgroup = 128 rows x 128 features x the whole K, for outputs so narrow that wider blocks would have to split K over workgroups, whose
+// One workgroup = 32 RT rows x 128 features x the whole K, for outputs so narrow that wider blocks would have to split K over workgroups, whose
 // slabs then go to memory and back before the residual and the norm can be added.  Here the K split is inside the workgroup: waves 0 to 3 take
-// the even k-tiles, 4 to 7 the odd ones, 64 x 64 each (12 fragments read from LDS for 32 products; eight waves of 64 x 32 over the same block
-// need 10 for 16 and are bound by those reads).  A stage is two k-tiles; three stages in the ring, copies two stages ahead; all fragments of
-// the next stage are read under this stage's products, so a stage waits once, at its barrier.  At the end the halves of the split exchange two row
-// tiles each, add the residual and leave the stream, the next norm's planes (weight times stream) and the rows' sums of squares.
-// Bound by LDS (1152 cycles a stage against 1024 of products) and the epilogue's stores, 33 MB at 4096 rows from every CU at once.
-// 0.6B, 4096 rows, o and down: two splits of 128 x 256 and the norm 38.7 + 17.2 us each, this 42.9 each; 2391 rows 37.0 + 14.6, 39.8; prompts
-// of 64 sequences (18.4 k tokens) 40.1 -> 36.9 ms.
+// the even k-tiles, 4 to 7 the odd ones, 16 RT x 64 each (at RT 4, 12 fragments read from LDS for 32 products; eight waves of 64 x 32 over the
+// same block need 10 for 16 and are bound by those reads).  A stage is two k-tiles; three stages in the ring, copies two stages ahead; all
+// fragments of the next stage are read under this stage's products, so a stage waits once, at its barrier.  At the end the halves of the split
+// exchange row tiles, add the residual and leave the stream, the next norm's planes (weight times stream) and the rows' sums of squares.
+// Bound by LDS (at RT 4 1152 cycles a stage against 1024 of products) and the epilogue's stores, 33 MB at 4096 rows from every CU at once.
+// RT: the smallest whose blocks are one round of the CUs, 4 above.  0.6B, o and down, us each at RT 1, 2, 3, 4: 1000 rows 22 / 26 / 30 / 36, 1280
+// 28 / 27 / 31 / 37, 2020 34 / 29 / 32 / 39, 2391 45 / 45 / 35 / 40, 3000 48 / 47 / 36 / 40, 4000 65 / 57 / 62 / 45; with K splits over
+// workgroups and a norm launch 22 + 9, 26 + 16, 26 + 17, 37 + 15 (2391) and 39 + 17 (4096).
+template <int RT>
 __global__ void __launch_bounds__(512) tile_resid_kernel(TileResidArgs a) {
-    constexpr int FR1 = 24, FR = 2 * FR1;  // 1 KiB fragments of a k-tile (8 of W, 8 + 8 of x) and of a stage
+    constexpr int XT = 2 * RT, FR1 = 8 + 2 * XT, FR = 2 * FR1;  // row tiles; 1 KiB fragments of a k-tile (8 of W, XT of each plane of x) and of a stage
+    constexpr int NI = FR / 8, OWN = (RT + 1) / 2;              // copies of a wave in a stage; row tiles of a half of the K split at the end
     extern __shared__ __attribute__((aligned(16))) char smem_raw[];
     uint4* lds = reinterpret_cast<uint4*>(smem_raw);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -606,50 +609,52 @@ __global__ void __launch_bounds__(512) tile_resid_kernel(TileResidArgs a) {
     }
     const int NS = a.KT >> 1, mtiles = (a.M + 15) >> 4;
     // the residual of this wave's own two row tiles comes before the streams
-    const int row0 = mb * 128 + wm * 64 + kg * 32 + l15, f0 = nb * 128 + wn * 64 + grp * 4;
-    float4 r4[2][4];
+    const int tile0 = kg * OWN, row0 = mb * (32 * RT) + wm * (16 * RT) + tile0 * 16 + l15, f0 = nb * 128 + wn * 64 + grp * 4;
+    float4 r4[OWN][4];
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < OWN; ++b)
 #pragma unroll
         for (int j = 0; j < 4; ++j) r4[b][j] = *reinterpret_cast<const float4*>(a.resid_in + (size_t)min(row0 + b * 16, a.M - 1) * a.N + f0 + j * 16);
     __builtin_amdgcn_sched_barrier(0);
-    const uint4* sw = a.wp + (size_t)(nb * 8 + wave) * a.KT * 64 + lane;
-    const size_t xo = (size_t)min(mb * 8 + wave, mtiles - 1) * a.KT * 64 + lane;  // past the end: the last row tile again, not stored
-    const uint4 *sh = a.xh + xo, *sl = a.xl + xo;
-    auto issue2 = [&](int s, int buf, int part) {  // copies 2 part and 2 part + 1 of the six of stage s (past the end: the last stage again)
+    const uint4* src[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int f = wave + 8 * i, h = f / FR1, g = f % FR1;  // k-tile of the stage; W's n-tiles, then [plane][row tile] of x
+        const int mt = min(mb * XT + (g - 8) % XT, mtiles - 1);  // past the end: the last row tile again, not stored
+        src[i] = (g < 8 ? a.wp + (size_t)(nb * 8 + g) * a.KT * 64 : (g - 8 >= XT ? a.xl : a.xh) + (size_t)mt * a.KT * 64) + h * 64 + lane;
+    }
+    auto issue = [&](int s, int buf, int i0, int i1) {  // copies i0 .. i1 - 1 of stage s (past the end: the last stage again)
         const size_t koff = (size_t)min(s, NS - 1) * 128;
 #pragma unroll
-        for (int c = 2 * part; c < 2 * part + 2; ++c) {
-            const int h = c / 3, k = c % 3;
-            const uint4* src = (k == 0 ? sw : k == 1 ? sh : sl) + koff + h * 64;
-            __builtin_amdgcn_global_load_lds((gptr_t)src, (lptr_t)(lds + (size_t)(buf * FR + h * FR1 + k * 8 + wave) * 64), 16, 0, 0);
-        }
+        for (int i = 0; i < NI; ++i)
+            if (i >= i0 && i < i1) __builtin_amdgcn_global_load_lds((gptr_t)(src[i] + koff), (lptr_t)(lds + (size_t)(buf * FR + wave + 8 * i) * 64), 16, 0, 0);
     };
     const uint32_t lds0 = (uint32_t)(uintptr_t)(lptr_t)smem_raw;
     uint32_t w_at[3], x_at[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
         w_at[i] = lds0 + (uint32_t)((i * FR + kg * FR1 + wn * 4) * 64 + lane) * 16;
-        x_at[i] = lds0 + (uint32_t)((i * FR + kg * FR1 + 8 + wm * 4) * 64 + lane) * 16;
+        x_at[i] = lds0 + (uint32_t)((i * FR + kg * FR1 + 8 + wm * RT) * 64 + lane) * 16;
     }
-    f32x4 acc[4][4];
+    f32x4 acc[4][RT];
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[j][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    bf16x8 WA[4], HA[4], LA[4], WB[4], HB[4], LB[4];
+        for (int b = 0; b < RT; ++b) acc[j][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 WA[4], HA[RT], LA[RT], WB[4], HB[RT], LB[RT];
 #define NVLLM_RD(DST_, ADDR_, OFF_) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(DST_) : "v"(ADDR_), "n"(OFF_))
 #define NVLLM_RD_SET(W_, H_, L_, WP_, XP_)                                                                                   \
     do {                                                                                                                      \
-        NVLLM_RD(W_[0], WP_, 0); NVLLM_RD(W_[1], WP_, 1024); NVLLM_RD(W_[2], WP_, 2048); NVLLM_RD(W_[3], WP_, 3072);          \
-        NVLLM_RD(H_[0], XP_, 0); NVLLM_RD(L_[0], XP_, 8192); NVLLM_RD(H_[1], XP_, 1024); NVLLM_RD(L_[1], XP_, 9216);          \
-        NVLLM_RD(H_[2], XP_, 2048); NVLLM_RD(L_[2], XP_, 10240); NVLLM_RD(H_[3], XP_, 3072); NVLLM_RD(L_[3], XP_, 11264);     \
+        _Pragma("unroll") for (int j = 0; j < 4; ++j) NVLLM_RD(W_[j], WP_, j * 1024);                                         \
+        _Pragma("unroll") for (int b = 0; b < RT; ++b) { NVLLM_RD(H_[b], XP_, b * 1024); NVLLM_RD(L_[b], XP_, (XT + b) * 1024); } \
     } while (0)
-// the set's reads have arrived (the operands tie it to their uses), this wave's copies of the stage after it too; then every wave's
+// the set's reads have arrived, this wave's copies of the stage after it too, then every wave's; the empty statements tie the registers to the wait
 #define NVLLM_SET_READY(W_, H_, L_, VM_)                                                                                     \
-    asm volatile("s_waitcnt vmcnt(" VM_ ") lgkmcnt(0)\n\ts_barrier"                                                          \
-                 : "+v"(W_[0]), "+v"(W_[1]), "+v"(W_[2]), "+v"(W_[3]), "+v"(H_[0]), "+v"(H_[1]), "+v"(H_[2]), "+v"(H_[3]),    \
-                   "+v"(L_[0]), "+v"(L_[1]), "+v"(L_[2]), "+v"(L_[3])::"memory")
+    do {                                                                                                                      \
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(VM_) : "memory");                                   \
+        _Pragma("unroll") for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(W_[j]));                                         \
+        _Pragma("unroll") for (int b = 0; b < RT; ++b) { asm volatile("" : "+v"(H_[b])); asm volatile("" : "+v"(L_[b])); }    \
+    } while (0)
 #define NVLLM_MM(W_, H_, L_, B_)                                                                                             \
     do {                                                                                                                      \
         _Pragma("unroll") for (int j = 0; j < 4; ++j) acc[j][B_] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(W_[j], H_[B_], acc[j][B_], 0, 0, 0); \
@@ -658,59 +663,53 @@ __global__ void __launch_bounds__(512) tile_resid_kernel(TileResidArgs a) {
     } while (0)
 #define NVLLM_STAGE(W_, H_, L_, WN_, HN_, LN_, S_)                                                                           \
     do {                                                                                                                      \
-        NVLLM_SET_READY(W_, H_, L_, "6");                                                                                     \
+        NVLLM_SET_READY(W_, H_, L_, NI);                                                                                      \
         NVLLM_RD_SET(WN_, HN_, LN_, w_at[1], x_at[1]);                                                                        \
         __builtin_amdgcn_sched_barrier(0);                                                                                    \
-        NVLLM_MM(W_, H_, L_, 0);                                                                                              \
-        issue2((S_) + 3, cur, 0);                                                                                             \
-        __builtin_amdgcn_sched_barrier(0);                                                                                    \
-        NVLLM_MM(W_, H_, L_, 1);                                                                                              \
-        issue2((S_) + 3, cur, 1);                                                                                             \
-        __builtin_amdgcn_sched_barrier(0);                                                                                    \
-        NVLLM_MM(W_, H_, L_, 2);                                                                                              \
-        issue2((S_) + 3, cur, 2);                                                                                             \
-        __builtin_amdgcn_sched_barrier(0);                                                                                    \
-        NVLLM_MM(W_, H_, L_, 3);                                                                                              \
+        _Pragma("unroll") for (int b = 0; b < RT; ++b) {                                                                      \
+            NVLLM_MM(W_, H_, L_, b);                                                                                          \
+            issue((S_) + 3, cur, b * NI / RT, (b + 1) * NI / RT);                                                             \
+            __builtin_amdgcn_sched_barrier(0);                                                                                \
+        }                                                                                                                     \
         cur = cur == 2 ? 0 : cur + 1;                                                                                         \
         { const uint32_t t_ = w_at[0]; w_at[0] = w_at[1]; w_at[1] = w_at[2]; w_at[2] = t_; }                                  \
         { const uint32_t t_ = x_at[0]; x_at[0] = x_at[1]; x_at[1] = x_at[2]; x_at[2] = t_; }                                  \
     } while (0)
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int p = 0; p < 3; ++p) issue2(i, i, p);
-    asm volatile("s_waitcnt vmcnt(12)\n\ts_barrier" ::: "memory");
+    for (int i = 0; i < 3; ++i) issue(i, i, 0, NI);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(2 * NI) : "memory");
     NVLLM_RD_SET(WA, HA, LA, w_at[0], x_at[0]);
     int cur = 0;
     for (int s = 0; s < NS; s += 2) {  // NS is even (host)
         NVLLM_STAGE(WA, HA, LA, WB, HB, LB, s);
         NVLLM_STAGE(WB, HB, LB, WA, HA, LA, s + 1);
     }
-    NVLLM_SET_READY(WA, HA, LA, "0");  // the reads and copies past the end; the ring is free
+    NVLLM_SET_READY(WA, HA, LA, 0);  // the reads and copies past the end; the ring is free
 #undef NVLLM_STAGE
 #undef NVLLM_MM
 #undef NVLLM_SET_READY
 #undef NVLLM_RD_SET
 #undef NVLLM_RD
-    // each half of the K split keeps two row tiles and hands the others to its partner
-    f32x4* xch = reinterpret_cast<f32x4*>(smem_raw);                        // [8 waves][2][4][64]
-    float* red = reinterpret_cast<float*>(smem_raw + 8 * 8 * 1024);         // [wm][4 row tiles][16]
+    // each half of the K split keeps its own row tiles and hands the others to its partner
+    f32x4* xch = reinterpret_cast<f32x4*>(smem_raw);                             // [8 waves][OWN][4][64]
+    float* red = reinterpret_cast<float*>(smem_raw + 8 * OWN * 4 * 1024);        // [wm][RT][16]
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
+    for (int b = 0; b < OWN; ++b)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) xch[((wave * 2 + b) * 4 + j) * 64 + lane] = kg ? acc[j][b] : acc[j][2 + b];
+        for (int j = 0; j < 4; ++j) xch[((wave * OWN + b) * 4 + j) * 64 + lane] = kg ? acc[j][b] : acc[j][min(OWN + b, RT - 1)];
     __syncthreads();
-    float ss[2];
+    float ss[OWN];
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
+    for (int b = 0; b < OWN; ++b) {
         const int row = row0 + b * 16;
+        const bool mine = tile0 + b < RT;  // an odd RT: the second half has one less
         ss[b] = 0.f;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const f32x4 other = xch[(((wave ^ 4) * 2 + b) * 4 + j) * 64 + lane], own = kg ? acc[j][2 + b] : acc[j][b];
+            const f32x4 other = xch[(((wave ^ 4) * OWN + b) * 4 + j) * 64 + lane], own = kg ? acc[j][min(OWN + b, RT - 1)] : acc[j][b];
             const f32x4 v = kg ? other + own : own + other;
             const float s0 = v[0] + r4[b][j].x, s1 = v[1] + r4[b][j].y, s2 = v[2] + r4[b][j].z, s3 = v[3] + r4[b][j].w;
-            if (row < a.M) {
+            if (mine && row < a.M) {
                 const float4 w4 = *reinterpret_cast<const float4*>(a.next_w + f0 + j * 16);
                 *reinterpret_cast<float4*>(a.resid_out + (size_t)row * a.N + f0 + j * 16) = make_float4(s0, s1, s2, s3);
                 uint16_t h[4], l[4];
@@ -723,13 +722,13 @@ __global__ void __launch_bounds__(512) tile_resid_kernel(TileResidArgs a) {
         }
         ss[b] += __shfl_xor(ss[b], 16);
         ss[b] += __shfl_xor(ss[b], 32);
-        if (wn == 1 && grp == 0) red[(wm * 4 + kg * 2 + b) * 16 + l15] = ss[b];
+        if (mine && wn == 1 && grp == 0) red[(wm * RT + tile0 + b) * 16 + l15] = ss[b];
     }
     __syncthreads();
     if (wn == 0 && grp == 0)
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
-            if (row0 + b * 16 < a.M) a.ssq[(size_t)nb * a.ssq_stride + row0 + b * 16] = ss[b] + red[(wm * 4 + kg * 2 + b) * 16 + l15];
+        for (int b = 0; b < OWN; ++b)
+            if (tile0 + b < RT && row0 + b * 16 < a.M) a.ssq[(size_t)nb * a.ssq_stride + row0 + b * 16] = ss[b] + red[(wm * RT + tile0 + b) * 16 + l15];
 }
 
 // ---- host side -------------------------------------------------------------------------------------
@@ -765,20 +764,30 @@ static TileShape tile_shape(int M, int N, int K, int mode, int min_wgs, int max_
 }
 
 bool tile_resid_ok(int M, int N, int K) { return M > 0 && N % 128 == 0 && N / 128 <= 64 && K % 128 == 0; }
+template <int RT>
+static hipError_t tile_resid_launch(TileResidArgs& a, hipStream_t s) {
+    a.MB = (a.M + 32 * RT - 1) / (32 * RT);
+    const int per = (a.MB * a.NB + 7) / 8;
+    a.band = std::min(a.MB, std::max(1, (int)std::lround(std::sqrt(per * 128.0 / (2.0 * 32 * RT)))));
+    const size_t lds = (size_t)3 * 2 * (8 + 4 * RT) * 1024;
+    static std::atomic<uint64_t> lds_set{0};
+    ensure_dyn_lds(reinterpret_cast<const void*>(tile_resid_kernel<RT>), lds, lds_set);
+    tile_resid_kernel<RT><<<8 * per, 512, lds, s>>>(a);
+    return hipGetLastError();
+}
 hipError_t launch_tile_resid(const bf16_bits* xh, const bf16_bits* xl, const PackedW& w, int M, float* resid, const float* next_w, bf16_bits* oh, bf16_bits* ol, float* ssq, int ssq_stride,
                              hipStream_t s) {
     if (!tile_resid_ok(M, w.N, w.K)) return hipErrorNotSupported;
     TileResidArgs a;
     a.xh = reinterpret_cast<const uint4*>(xh); a.xl = reinterpret_cast<const uint4*>(xl); a.wp = w.data;
     a.resid_in = resid; a.resid_out = resid; a.next_w = next_w; a.oh = oh; a.ol = ol; a.ssq = ssq; a.ssq_stride = ssq_stride;
-    a.M = M; a.N = w.N; a.KT = w.K / 32; a.MB = (M + 127) / 128; a.NB = w.N / 128;
-    const int per = (a.MB * a.NB + 7) / 8;
-    a.band = std::min(a.MB, std::max(1, (int)std::lround(std::sqrt(per / 2.0))));
-    const size_t lds = (size_t)3 * 48 * 1024;
-    static std::atomic<uint64_t> lds_set{0};
-    ensure_dyn_lds(reinterpret_cast<const void*>(tile_resid_kernel), lds, lds_set);
-    tile_resid_kernel<<<8 * per, 512, lds, s>>>(a);
-    return hipGetLastError();
+    a.M = M; a.N = w.N; a.KT = w.K / 32; a.NB = w.N / 128;
+    // the shortest blocks that are one round of the CUs
+    auto one_round = [&](int rt) { return (M + 32 * rt - 1) / (32 * rt) * a.NB <= 256; };
+    if (one_round(1)) return tile_resid_launch<1>(a, s);
+    if (one_round(2)) return tile_resid_launch<2>(a, s);
+    if (one_round(3)) return tile_resid_launch<3>(a, s);
+    return tile_resid_launch<4>(a, s);
 }
 
 bool gemm_tile_ok(int M, int N, int K, int mode, int min_wgs) { return tile_shape(M, N, K, mode, min_wgs, 1).ntw != 0; }

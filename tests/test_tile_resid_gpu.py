@@ -8,7 +8,7 @@ pytestmark = pytest.mark.gpu
 
 # (hidden, heads, intermediate): K of 1024 and 2048 beside 3072 and 1152 (an odd number of 128)
 @pytest.mark.parametrize("hidden,heads,inter", [(1024, 16, 3072), (1024, 8, 1152), (512, 8, 2048)])
-@pytest.mark.parametrize("lens,chunk,bits", [([1025], 4096, 16), ([1100, 3, 77], 4096, 24), ([2047], 4096, 16), ([2049], 4096, 16), ([1500, 1200, 1], 4096, 16),
+@pytest.mark.parametrize("lens,chunk,bits", [([497], 4096, 16), ([700, 45], 4096, 24), ([1024], 4096, 16), ([1025], 4096, 16), ([1100, 3, 77], 4096, 24), ([2047], 4096, 16), ([2049], 4096, 16), ([1500, 1200, 1], 4096, 16),
                                              ([2400], 1100, 24), ([4000, 350], 8192, 16)])
 def test_chunk(hidden, heads, inter, lens, chunk, bits):
     import nano_vllm_candle_amd as pkg
