@@ -1238,6 +1238,7 @@ static int forward_chunk_fused(nvllm_model* m, const FusedPlan& fp, int R, int n
         const int tps = ctx->tp_size;  // vocab-parallel: every rank leaves (id, max) of its shard for the gather in finish_logits
         uint32_t* ids_dst = tps == 1 ? m->d_next + logits_row0 : m->d_next + m->cur_n + (size_t)ctx->tp_rank * m->cur_n + logits_row0;
         float* val_dst = tps == 1 ? nullptr : m->d_maxval + (size_t)ctx->tp_rank * m->cur_n + logits_row0;
+        if (!m->want_ids) return NVLLM_OK;
         if (pl.lm_nt > 0)
             HIPCHK(ctx, launch_argmax_rows(m->part_val, m->part_idx, gemm_argmax_parts(pl, m->V_l), n_last, ids_dst, val_dst, s));
         else
@@ -1484,6 +1485,7 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
         PROF(m, PROF_LMHEAD, launch_gemm_argmax(pl, m->xh, m->xl, H, m->lm_head, lg, n_last, m->part_val, m->part_idx, nullptr, s));
         uint32_t* ids_dst = tp == 1 ? m->d_next + logits_row0 : m->d_next + m->cur_n + (size_t)ctx->tp_rank * m->cur_n + logits_row0;
         float* val_dst = tp == 1 ? nullptr : m->d_maxval + (size_t)ctx->tp_rank * m->cur_n + logits_row0;
+        if (!m->want_ids) return NVLLM_OK;
         if (pl.lm_nt > 0)
             HIPCHK(ctx, launch_argmax_rows(m->part_val, m->part_idx, gemm_argmax_parts(pl, m->V_l), n_last, ids_dst, val_dst, s));
         else
@@ -1829,6 +1831,7 @@ static int step_impl(nvllm_model* m, int n_seqs, const int64_t* seq_ids, const u
     // carried state moves on with the rows: if this step fails, the sequences start again
     if (recurrent) for (int i = 0; i < n_seqs; ++i) m->seqs[seq_ids[i]].cached = 0;
     m->want_logits = last_logits != nullptr || temperatures != nullptr || score != nullptr;  // sampling reads the last-row logits on the device
+    m->want_ids = !score && !temperatures;
     m->cur_n = n_seqs;
     m->cur_max_len = *std::max_element(lens, lens + n_seqs);
     set_attn_split(m, n_seqs, m->cur_max_len);
@@ -1991,6 +1994,7 @@ static int decode_core(nvllm_model* m) {
         m->decode_resident = true;
     }
     m->want_logits = false;
+    m->want_ids = true;
     m->cur_n = n;
     m->cur_max_len = *std::max_element(m->last_lens.begin(), m->last_lens.end()) + 1;
     set_attn_split(m, n, m->cur_max_len);

@@ -153,6 +153,7 @@ int output_head(nvllm_model* m, const PackedW& head, int Kw, int Vp, const float
         rn.softcap = cap;
         GemmPlan pl = plan_lmhead(n_last, m->V_l, Kw);
         PROF(m, PROF_LMHEAD, launch_gemm_argmax(pl, m->xh, m->xl, Kw, head, m->want_logits ? lg : nullptr, n_last, m->part_val, m->part_idx, &rn, s));
+        if (!m->want_ids) return NVLLM_OK;
         const int parts = gemm_argmax_parts(pl, m->V_l);
         if (pl.lm_nt > 0) HIPCHK(ctx, launch_argmax_rows(m->part_val, m->part_idx, parts, n_last, ids_dst, val_dst, s));
         else HIPCHK(ctx, launch_argmax_parts(m->part_val, m->part_idx, parts, n_last, m->argmax_scratch, ids_dst, val_dst, s));
@@ -166,6 +167,6 @@ int output_head(nvllm_model* m, const PackedW& head, int Kw, int Vp, const float
     }
     if (rc) return rc;
     HIPCHK(ctx, launch_logits_finish(m->slabs, ns, (int64_t)n_last * Vp, Vp, n_last, m->V_l, cap, lg, m->V_l, s));
-    HIPCHK(ctx, launch_argmax(lg, n_last, m->V_l, m->V_l, ids_dst, val_dst, s));
+    if (m->want_ids) HIPCHK(ctx, launch_argmax(lg, n_last, m->V_l, m->V_l, ids_dst, val_dst, s));
     return NVLLM_OK;
 }

@@ -186,6 +186,7 @@ struct nvllm_model {
     int* part_idx = nullptr;
     unsigned long long* argmax_scratch = nullptr;  // ticket + per-row keys of argmax_parts_kernel
     bool want_logits = false;   // this step stores the last-row logits
+    bool want_ids = true;       // ... and its greedy ids are read (not where positions are scored or the device samples)
     int cur_n = 0;              // sequences of the step in flight
     int last_groups = 0;        // prompt attention: groups of the chunk's q-tiles with a row the head wants, listed behind group_order
     int cur_max_len = 0;        // longest of them (tokens, the new ones included)
