@@ -96,6 +96,9 @@ struct GluPlan {
 // y = x.W^T left as f32 slabs
 ProductPlan plan_product(const nvllm_model* m, int R, const PackedW& w);
 int run_product(nvllm_model* m, const ProductPlan& p, const bf16_bits* xh, const bf16_bits* xl, const PackedW& w, float* out, int R, int* n_slabs);
+// two products whose inputs are there, in one launch where their shapes allow
+struct ProductJob { ProductPlan p; const bf16_bits *xh, *xl; const PackedW& w; float* out; int* n_slabs; };
+int run_two_products(nvllm_model* m, const ProductJob& a, const ProductJob& b, int R);
 GluPlan plan_glu(const nvllm_model* m, int R, const PackedW& w, bool want_packed_out);
 int run_glu(nvllm_model* m, const GluPlan& g, const bf16_bits* xh, const bf16_bits* xl, const PackedW& w, int R, const GluSpec& spec,
             bf16_bits* oh, bf16_bits* ol, int out_packed);

@@ -970,11 +970,15 @@ int HybridModel::forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n
         sum = base;
         reduced = false;
         sum.in = m->slabs; sum.slab_stride = (int64_t)rows * ldr; sum.in_bias = w.mix[0].ob;
-        rc = product(m, po[0], cf[0], ch[0], cl[0], w.mix[0].o, m->slabs, rows, &sum.n_slabs);
-        if (!rc && w.branches == 2) {
+        if (w.branches == 2) {
             sum.in2 = slabs2; sum.slab_stride2 = (int64_t)rows * ldr;
             sum.branch_w[0] = w.mix[0].out_norm; sum.branch_w[1] = w.mix[1].out_norm;
-            rc = product(m, po[1], cf[1], ch[1], cl[1], w.mix[1].o, slabs2, rows, &sum.n_slabs2);
+        }
+        if (w.branches == 2 && !f32) {
+            rc = run_two_products(m, {po[0], ch[0], cl[0], w.mix[0].o, m->slabs, &sum.n_slabs}, {po[1], ch[1], cl[1], w.mix[1].o, slabs2, &sum.n_slabs2}, rows);
+        } else {
+            rc = product(m, po[0], cf[0], ch[0], cl[0], w.mix[0].o, m->slabs, rows, &sum.n_slabs);
+            if (!rc && w.branches == 2) rc = product(m, po[1], cf[1], ch[1], cl[1], w.mix[1].o, slabs2, rows, &sum.n_slabs2);
         }
         if (rc) return rc;
         const float* weight = w.norm1;

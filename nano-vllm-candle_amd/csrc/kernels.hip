@@ -1044,7 +1044,7 @@ __global__ void __launch_bounds__(NWN * NWK * 64) gemm_rowpar_kernel(RowParArgs 
 // ---------------------------------------------------------------------------------------------------
 constexpr int kRowDirBlocks = 4;  // most row blocks of a workgroup
 template <int NT, int NWK, int TK, int EPI, bool LOOP>
-__device__ __forceinline__ void rowdir_body(const RowParArgs& a, const uint4* __restrict__ wp, int N, int KT) {
+__device__ __forceinline__ void rowdir_body(const RowParArgs& a, const uint4* __restrict__ wp, int N, int KT, int group) {
     constexpr int UNROLL = LOOP ? 4 : NWK;  // LDS reads at once where the K slices meet: beside the kept weights all of them would spill
     static_assert(NT <= NWK, "wave t finishes n-tile t");
     constexpr int NR = 16;
@@ -1056,7 +1056,7 @@ __device__ __forceinline__ void rowdir_body(const RowParArgs& a, const uint4* __
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int l15 = lane & 15, grp = lane >> 4;
     const int ntiles = N >> 4;
-    const int tile0 = (int)blockIdx.x * NT;
+    const int tile0 = group * NT;
     int m0 = blockIdx.z * NR;
     const int M = a.M, m_step = LOOP ? gridDim.z * NR : 1 << 30;
     const int k0 = wave * TK;
@@ -1141,8 +1141,8 @@ __device__ __forceinline__ void rowdir_body(const RowParArgs& a, const uint4* __
     // epilogue 5: what the rotation and the norm of this wave's 16 features and of those it is paired with need
     [[maybe_unused]] f32x4 cs, sn, w_own, w_other;
     if constexpr (EPI == 5) {
-        if (wave < NT && (int)blockIdx.x < a.q.nh_l + a.q.kv.kv_l) {
-            const float* w8 = (int)blockIdx.x < a.q.nh_l ? a.q.qn : a.q.kn;
+        if (wave < NT && group < a.q.nh_l + a.q.kv.kv_l) {
+            const float* w8 = group < a.q.nh_l ? a.q.qn : a.q.kn;
             const size_t at = (size_t)pos * 64 + (wave & 3) * 16 + grp * 4;
             cs = *reinterpret_cast<const f32x4*>(a.q.cos + at);
             sn = *reinterpret_cast<const f32x4*>(a.q.sin + at);
@@ -1177,7 +1177,7 @@ __device__ __forceinline__ void rowdir_body(const RowParArgs& a, const uint4* __
             ssq_part += __shfl_xor(ssq_part, 16);
             ssq_part += __shfl_xor(ssq_part, 32);
             if constexpr (NT == 1) {
-                if (grp == 0 && row < M) a.ssq[(size_t)blockIdx.x * a.ssq_stride + row] = ssq_part;
+                if (grp == 0 && row < M) a.ssq[(size_t)group * a.ssq_stride + row] = ssq_part;
             } else {
                 if (grp == 0) sred[wave * NR + l15] = ssq_part;
             }
@@ -1188,7 +1188,7 @@ __device__ __forceinline__ void rowdir_body(const RowParArgs& a, const uint4* __
                 float t = 0.f;
 #pragma unroll
                 for (int k = 0; k < NT; ++k) t += sred[k * NR + l15];
-                a.ssq[(size_t)blockIdx.x * a.ssq_stride + row] = t;
+                a.ssq[(size_t)group * a.ssq_stride + row] = t;
             }
         }
     } else if constexpr (EPI == 1) {
@@ -1217,7 +1217,7 @@ __device__ __forceinline__ void rowdir_body(const RowParArgs& a, const uint4* __
         // then q to the f32 buffer and k, v into the cache.  The f32 sums' way through memory and the row kernel's launch (4.5 us and the gap
         // before it) for a longer epilogue: rule and figures at gemm_rowdir_qkv_ok
         const QkvArgs& q = a.q;
-        const int head = blockIdx.x;
+        const int head = group;
         const float ri = rownorm_rinv_lds<NR>(a.rn, sred, l15);
         __syncthreads();  // every finishing wave is done reading red
         if (wave < NT) {
@@ -1278,11 +1278,20 @@ __device__ __forceinline__ void rowdir_body(const RowParArgs& a, const uint4* __
 }
 template <int NT, int NWK, int TK, int EPI>
 __global__ void __launch_bounds__(NWK * 64) gemm_rowdir_kernel(RowParArgs a, const uint4* __restrict__ wp, int N, int KT) {
-    rowdir_body<NT, NWK, TK, EPI, false>(a, wp, N, KT);
+    rowdir_body<NT, NWK, TK, EPI, false>(a, wp, N, KT, blockIdx.x);
 }
 template <int NT, int NWK, int TK, int EPI>
 __global__ void __launch_bounds__(NWK * 64) gemm_rowdir_loop_kernel(RowParArgs a, const uint4* __restrict__ wp, int N, int KT) {
-    rowdir_body<NT, NWK, TK, EPI, true>(a, wp, N, KT);
+    rowdir_body<NT, NWK, TK, EPI, true>(a, wp, N, KT, blockIdx.x);
+}
+
+// Two plain products of the same rows in one launch, where neither needs the other (the projections of a layer's two branches, whose outputs
+// the next norm adds up): workgroups below groups_a make the first.  Each alone is a launch's latency on a quarter of the chip: 24 rows, 1024
+// features of K 2048 and of K 3072, 5.2 and 6.5 us and the boundary between them, together 7.1.
+template <int NTA, int TKA, int NTB, int TKB>
+__global__ void __launch_bounds__(1024) gemm_rowdir_two_kernel(RowParArgs a, const uint4* __restrict__ wa, int NA, int groups_a, RowParArgs b, const uint4* __restrict__ wb, int NB) {
+    if ((int)blockIdx.x < groups_a) rowdir_body<NTA, 16, TKA, 2, false>(a, wa, NA, 16 * TKA, blockIdx.x);
+    else rowdir_body<NTB, 16, TKB, 2, false>(b, wb, NB, 16 * TKB, (int)blockIdx.x - groups_a);
 }
 
 // Register-direct products of 65 to 256 rows: RB row blocks at a time (blocks z, z + gz, ... of blockIdx.z = z), K split over NWK waves, the
@@ -1616,6 +1625,30 @@ static hipError_t rowpar_dispatch(const RowParShape& sh, const RowParArgs& a, co
 #undef NVLLM_RP_PH
 #undef NVLLM_RP
     return hipErrorNotSupported;
+}
+
+template <int NTA, int TKA, int NTB, int TKB>
+static hipError_t rowdir_two_launch(const RowParArgs& a, const PackedW& wa, const RowParArgs& b, const PackedW& wb, hipStream_t s) {
+    const int ga = (wa.N / 16 + NTA - 1) / NTA, gb = (wb.N / 16 + NTB - 1) / NTB;
+    const size_t lds = (size_t)16 * std::max(NTA, NTB) * 1024 + 4 * 16 * 4;
+    static std::atomic<uint64_t> lds_set{0};
+    ensure_dyn_lds(reinterpret_cast<const void*>(gemm_rowdir_two_kernel<NTA, TKA, NTB, TKB>), lds, lds_set);
+    gemm_rowdir_two_kernel<NTA, TKA, NTB, TKB><<<dim3(ga + gb, 1, (a.M + 15) / 16), 1024, lds, s>>>(a, wa.data, wa.N, ga, b, wb.data, wb.N);
+    return hipGetLastError();
+}
+// K of 1024, 2048 or 3072 each, one round of workgroups together (up to 64 rows); hipErrorNotReady: two launches
+hipError_t launch_gemm_rowdir_two(const RowParArgs& a, const PackedW& wa, const RowParArgs& b, const PackedW& wb, hipStream_t s) {
+    if (a.M != b.M || a.M > 64 || a.M < 1) return hipErrorNotReady;
+    const RowDirShape da = rowdir_shape(wa.N, wa.K, 2, a.M), db = rowdir_shape(wb.N, wb.K, 2, b.M);
+    if (!da.nt || !db.nt) return hipErrorNotReady;
+    const int blocks = (a.M + 15) / 16, wgs = ((wa.N / 16 + da.nt - 1) / da.nt + (wb.N / 16 + db.nt - 1) / db.nt) * blocks;
+    if (wgs > 256) return hipErrorNotReady;
+#define NVLLM_TWO(NTA_, TKA_, NTB_, TKB_) if (da.nt == NTA_ && da.tk == TKA_ && db.nt == NTB_ && db.tk == TKB_) return rowdir_two_launch<NTA_, TKA_, NTB_, TKB_>(a, wa, b, wb, s);
+#define NVLLM_TWO_N(TKA_, TKB_) NVLLM_TWO(1, TKA_, 1, TKB_) NVLLM_TWO(2, TKA_, 2, TKB_) NVLLM_TWO((TKA_ == 6 ? 2 : 4), TKA_, (TKB_ == 6 ? 2 : 4), TKB_)
+    NVLLM_TWO_N(2, 2) NVLLM_TWO_N(2, 4) NVLLM_TWO_N(2, 6) NVLLM_TWO_N(4, 2) NVLLM_TWO_N(4, 4) NVLLM_TWO_N(4, 6) NVLLM_TWO_N(6, 2) NVLLM_TWO_N(6, 4) NVLLM_TWO_N(6, 6)
+#undef NVLLM_TWO_N
+#undef NVLLM_TWO
+    return hipErrorNotReady;
 }
 
 hipError_t launch_gemm_rowpar(const RowParArgs& a, const PackedW& w, int epi, hipStream_t s) {

@@ -750,6 +750,7 @@ int LatentModel::forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n
             resid = m->last_resid;
         }
         int no = 1, nd = 1;
+        bool o_done = false;
         BranchSum ff;
         if (w.experts.on()) {
             const bool two = gathers && L.cfg.one_norm && !same;  // the mixer's planes serve the shared expert and the router
@@ -764,12 +765,13 @@ int LatentModel::forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n
                 rc = exact_product(m, L.act_f, w.down, L.slabs2, rows, &nd);
             } else {
                 rc = run_glu(m, pg, ffh, ffl, w.gu, rows, spec, m->xh2, m->xl2, pd.packed);
-                if (!rc) rc = run_product(m, pd, m->xh2, m->xl2, w.down, L.slabs2, rows, &nd);
+                if (!rc) rc = run_two_products(m, {pd, m->xh2, m->xl2, w.down, L.slabs2, &nd}, {po, ch, cl, w.o, m->slabs, &no}, rows);
+                o_done = true;
             }
             if (rc) return rc;
             ff.in = L.slabs2; ff.n_slabs = nd; ff.slab_stride = (int64_t)rows * L.ldr;
         }
-        rc = f32 ? exact_product(m, cf, w.o, m->slabs, rows, &no) : run_product(m, po, ch, cl, w.o, m->slabs, rows, &no);
+        if (!o_done) rc = f32 ? exact_product(m, cf, w.o, m->slabs, rows, &no) : run_product(m, po, ch, cl, w.o, m->slabs, rows, &no);
         if (rc) return rc;
         base.ids = nullptr;
         base.in = m->slabs; base.n_slabs = no; base.slab_stride = (int64_t)rows * L.ldr;
