@@ -35,7 +35,10 @@ constexpr int kMaxScanStates = 1024;
 struct ScanArgs {
     const float* x = nullptr;        // [rows][ldx]
     int ldx = 0;
-    const float* dt = nullptr;       // [rows][channels_p] step sizes
+    const float* dt = nullptr;       // [rows][channels_p] step sizes; decode: or, with gate_w, softplus(gate_w . bc's first rank_p columns + gate_b) made in the kernel
+    const uint4* gate_w = nullptr;   // [channels_p x rank_p] bf16 in fragment order
+    const float* gate_b = nullptr;   // [channels_p]
+    int rank_p = 0;
     const float* bc = nullptr;       // rows of stride ldbc: B at column b0, C at column c0 (states each)
     int ldbc = 0, b0 = 0, c0 = 0;
     const float* z = nullptr;        // gate, slabs of stride z_stride, rows of stride ldz

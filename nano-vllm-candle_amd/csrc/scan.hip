@@ -58,34 +58,48 @@ __global__ void __launch_bounds__(256) conv_rows_kernel(ConvRowsArgs a) {
     }
     conv_out(a, row, c, y);
 }
-// decode: the window moves on by one token (this half of the history to the other one)
+// decode: the window moves on by one token (this half of the history to the other one).  Bound by latency: the taps' loads are independent of
+// each other and of the sequence's age, four at a time; one by one behind a branch, 24 rows of 2048 channels took 6.3 us, now 5.4
 __global__ void __launch_bounds__(256) conv_decode_kernel(ConvRowsArgs a) {
     const int row = blockIdx.y, c = (blockIdx.x * 256 + threadIdx.x) * 4;
     if (c >= a.channels) return;
-    const int slot = a.slot[row], pos = a.pos[row], H = a.taps - 1;
-    const float* past = a.history + ((size_t)(pos & 1) * a.slots + slot) * H * a.channels;
-    float* next = a.history + ((size_t)((pos + 1) & 1) * a.slots + slot) * H * a.channels;
-    const float4 cur = conv_input4(a, row, c);
-    float4 y = row4(a.bias, c, a.channels);
-    for (int i = 0; i < H; ++i) {
-        float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (pos >= H - i) x = row4(past + (size_t)i * a.channels, c, a.channels);
-        fma4(y, x, row4(a.conv + (size_t)i * a.channels, c, a.channels));
-        if (i > 0) {
-            const float t[4] = {x.x, x.y, x.z, x.w};
+    auto run = [&](auto get, auto put) {
+        float4 y = get(a.bias);
+        const int slot = a.slot[row], pos = a.pos[row], H = a.taps - 1;
+        const float* past = a.history + ((size_t)(pos & 1) * a.slots + slot) * H * a.channels;
+        float* next = a.history + ((size_t)((pos + 1) & 1) * a.slots + slot) * H * a.channels;
+        const float4 cur = conv_input4(a, row, c), last = get(a.conv + (size_t)H * a.channels);
+        for (int i0 = 0; i0 < H; i0 += 4) {
+            float4 x[4], w[4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (c + e < a.channels) next[(size_t)(i - 1) * a.channels + c + e] = t[e];
+            for (int u = 0; u < 4; ++u) {
+                const size_t at = (size_t)min(i0 + u, H - 1) * a.channels;
+                x[u] = get(past + at);
+                w[u] = get(a.conv + at);
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int i = i0 + u;
+                if (i >= H) break;
+                if (pos < H - i) x[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+                fma4(y, x[u], w[u]);
+                if (i > 0) put(next + (size_t)(i - 1) * a.channels, x[u]);
+            }
         }
-    }
-    if (H > 0) {
-        const float t[4] = {cur.x, cur.y, cur.z, cur.w};
+        if (H > 0) put(next + (size_t)(H - 1) * a.channels, cur);
+        fma4(y, cur, last);
+        conv_out(a, row, c, y);
+    };
+    if ((a.channels & 3) == 0)
+        run([&](const float* p) { return *reinterpret_cast<const float4*>(p + c); }, [&](float* p, const float4& v) { *reinterpret_cast<float4*>(p + c) = v; });
+    else
+        run([&](const float* p) { return row4(p, c, a.channels); },
+            [&](float* p, const float4& v) {
+                const float t[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (c + e < a.channels) next[(size_t)(H - 1) * a.channels + c + e] = t[e];
-    }
-    fma4(y, cur, row4(a.conv + (size_t)H * a.channels, c, a.channels));
-    conv_out(a, row, c, y);
+                for (int e = 0; e < 4; ++e)
+                    if (c + e < a.channels) p[c + e] = t[e];
+            });
 }
 // prompt chunks: a wave owns 16 rows x 32 channels, lane (grp, l15) row l15's eight consecutive channels: its plane stores in fragment
 // order are one contiguous KiB
@@ -220,7 +234,26 @@ __global__ void __launch_bounds__(256) scan_decode_kernel(ScanArgs a) {
     load_states(B, bc + a.b0);
     load_states(C, bc + a.c0);
     const int cc = min(c, a.channels - 1);
-    const float x = a.x[(size_t)row * a.ldx + cc], dt = a.dt[(size_t)row * a.channels_p + c];
+    const float x = a.x[(size_t)row * a.ldx + cc];
+    // the step size: the channel's lanes share out its product with the row's rank_p numbers (a launch of its own was
+    // 4.1 us and a boundary, this is 1.5: 24 rows of 2048 channels, 64 numbers)
+    float dt;
+    if (a.gate_w) {
+        const int KT = a.rank_p >> 5;
+        float t = 0.f;
+        for (int i = q; i < KT * 4; i += NL) {
+            const uint4 w = a.gate_w[((size_t)(c >> 4) * KT + (i >> 2)) * 64 + (i & 3) * 16 + (c & 15)];
+            const float* r = a.bc + (size_t)row * a.ldbc + i * 8;
+            const float4 r0 = *reinterpret_cast<const float4*>(r), r1 = *reinterpret_cast<const float4*>(r + 4);
+            const uint32_t wd[4] = {w.x, w.y, w.z, w.w};
+            const float rv[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
+#pragma unroll
+            for (int j = 0; j < 8; ++j) t += __builtin_bit_cast(float, (j & 1) ? wd[j >> 1] & 0xffff0000u : wd[j >> 1] << 16) * rv[j];
+        }
+        dt = softplusf(lanes_sum<NL>(t) + a.gate_b[c]);
+    } else {
+        dt = a.dt[(size_t)row * a.channels_p + c];
+    }
     const float z = slab_elem(a.z + (size_t)row * a.ldz + cc, a.z_slabs, a.z_stride);
     const bool fresh = a.pos[row] == 0;
     const float dx = dt * x;

@@ -185,10 +185,12 @@ int run_scan(nvllm_model* m, ScanMixer& w, ScanScratch& x, const float* in, int 
         rc = comm_allreduce_sum(ctx, x.dbc, (size_t)R * w.Nx);
         if (rc) return rc;
     }
-    HeadGemmArgs ga;
-    ga.x = dbc; ga.x_row = w.Nx; ga.w = w.dt.data; ga.N = ga.n_valid = w.n_p; ga.K = w.rank_p; ga.M = R; ga.exact = f32;
-    ga.y = x.dt; ga.y_row = w.n_p; ga.decay_bias = w.dt_b;
-    PROF(m, PROF_GEMM, launch_delta_gates(ga, s));
+    if (qt != 1) {
+        HeadGemmArgs ga;
+        ga.x = dbc; ga.x_row = w.Nx; ga.w = w.dt.data; ga.N = ga.n_valid = w.n_p; ga.K = w.rank_p; ga.M = R; ga.exact = f32;
+        ga.y = x.dt; ga.y_row = w.n_p; ga.decay_bias = w.dt_b;
+        PROF(m, PROF_GEMM, launch_delta_gates(ga, s));
+    }
     ScanArgs sa;
     sa.x = x.x; sa.ldx = w.Kc; sa.dt = x.dt; sa.bc = dbc; sa.ldbc = w.Nx; sa.b0 = w.rank_p; sa.c0 = w.rank_p + w.S;
     sa.z = in + w.n; sa.z_slabs = n_slabs; sa.ldz = w.Nin; sa.z_stride = ca.slab_stride;
@@ -199,6 +201,7 @@ int run_scan(nvllm_model* m, ScanMixer& w, ScanScratch& x, const float* in, int 
     sa.ld = w.Kc; sa.packed = ctx_packed;
     if (f32) sa.of = ctx_f;
     else { sa.oh = m->ctxh; sa.ol = m->ctxl; }
+    if (qt == 1) { sa.gate_w = w.dt.data; sa.gate_b = w.dt_b; sa.rank_p = w.rank_p; }
     if (qt == 1) PROF(m, PROF_RECUR, launch_scan_decode(sa, R, s));
     else PROF(m, PROF_RECUR, launch_scan_prompt(sa, s));
     return NVLLM_OK;
