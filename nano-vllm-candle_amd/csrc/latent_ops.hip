@@ -745,11 +745,15 @@ __global__ void __launch_bounds__(NW * 64) exact_rows_loop_kernel(HeadGemmArgs a
         if (nt + (int)gridDim.x < ntiles) tile(nt + gridDim.x, w1, w0);
     }
 }
-// K in four at most where its features alone leave CUs idle: 16 rows, 1024 features, K 2048 and 4608 11.0 us both before, in four 4.5 and 7.5
+// K in four at most where the features (and, in the prompt form, the rows) alone leave places for workgroups idle.  16 rows, 1024 features, K 2048
+// and 4608: 11.0 us both before, in four 4.5 and 7.5.  1465 rows, 1024 features, K 4608: 184 workgroups, of which a CU holds two, 75 us, in two 51
 int exact_splits(int M, int N, int K) {
-    if (M > 64 || K < 1024) return 1;
-    const int wgs = N / 16 * ((M + 63) / 64);
-    return std::max(1, std::min({4, 256 / std::max(1, wgs), K / 512}));
+    if (K < 1024) return 1;
+    if (M > 64) {
+        const int wgs = (N + 127) / 128 * ((M + 63) / 64);
+        return std::max(1, std::min({4, 512 / wgs, K / 512}));
+    }
+    return std::max(1, std::min({4, 256 / std::max(1, N / 16), K / 512}));
 }
 template <int MT>
 static hipError_t exact_rows_launch(const HeadGemmArgs& a, hipStream_t s) {
@@ -763,13 +767,13 @@ static hipError_t exact_rows_launch(const HeadGemmArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// one element of a 32-bit product, term by term
-__device__ __forceinline__ float exact_dot(const HeadGemmArgs& a, int head, int tile, int feature, int row) {
+// one element of a 32-bit product over k-tiles kt0 .. end, term by term
+__device__ __forceinline__ float exact_dot(const HeadGemmArgs& a, int head, int tile, int feature, int row, int kt0, int end) {
     const int KT = a.K >> 5;
     const uint4* wp = a.w + (size_t)head * a.w_head + (size_t)tile * KT * 64 + feature;
     const float* xp = a.x + (size_t)row * a.x_row + (size_t)head * a.x_head;
     float sum = 0.f;
-    for (int k = 0; k < KT * 4; ++k) {  // eight at a time
+    for (int k = kt0 * 4; k < end * 4; ++k) {  // eight at a time
         const uint4 w = wp[k * 16];
         const uint32_t wd[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
@@ -809,7 +813,9 @@ __global__ void __launch_bounds__(256, 2) exact_tile_kernel(HeadGemmArgs a) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l15 = lane & 15, grp = lane >> 4;
     const int ntiles = a.N >> 4, KT = a.K >> 5;
-    const int nt0 = (blockIdx.x * 4 + wave) * NT, head = blockIdx.y, m0 = blockIdx.z * (MT * 16);
+    // blockIdx.y: the head, or the split of K
+    const int nt0 = (blockIdx.x * 4 + wave) * NT, head = a.splits > 1 ? 0 : blockIdx.y, split = a.splits > 1 ? blockIdx.y : 0, m0 = blockIdx.z * (MT * 16);
+    const int per = (KT + a.splits - 1) / a.splits, kt0 = split * per, end = min(KT, kt0 + per);
     const uint4* wp = a.w + (size_t)head * a.w_head + lane;
     const float* xp = a.x + (size_t)min(m0 + wave * 16 + l15, a.M - 1) * a.x_row + (size_t)head * a.x_head + grp * 8;
     f32x4 acc[NT][MT];
@@ -828,9 +834,9 @@ __global__ void __launch_bounds__(256, 2) exact_tile_kernel(HeadGemmArgs a) {
     };
     float x0[8], x1[8];
     uint4 w0[NT], w1[NT];
-    load_x(0, x0);
-    load_w(0, w0);
-    load_x(1, x1);
+    load_x(kt0, x0);
+    load_w(kt0, w0);
+    load_x(kt0 + 1, x1);
     auto step = [&](int kt, float (&x)[8], const uint4 (&w)[NT], uint4 (&wn)[NT]) {
         uint4 f[3];
         split_exact(x, f);
@@ -851,9 +857,9 @@ __global__ void __launch_bounds__(256, 2) exact_tile_kernel(HeadGemmArgs a) {
                 for (int n = 0; n < NT; ++n) acc[n][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, w[n]), v, acc[n][b], 0, 0, 0);
             }
     };
-    for (int kt = 0; kt < KT; kt += 2) {
+    for (int kt = kt0; kt < end; kt += 2) {
         step(kt, x0, w0, w1);
-        if (kt + 1 < KT) step(kt + 1, x1, w1, w0);
+        if (kt + 1 < end) step(kt + 1, x1, w1, w0);
     }
     // A second or third part that is zero times an infinite weight is NaN where the product is infinite: those elements again, undivided
     uint32_t nans = 0;
@@ -865,13 +871,14 @@ __global__ void __launch_bounds__(256, 2) exact_tile_kernel(HeadGemmArgs a) {
     while (nans) {
         const int at = __ffs(nans) - 1, n = at / (4 * MT), b = (at >> 2) % MT;
         nans &= nans - 1;
-        const float v = exact_dot(a, head, min(nt0 + n, ntiles - 1), grp * 4 + (at & 3), min(m0 + b * 16 + l15, a.M - 1));
+        const float v = exact_dot(a, head, min(nt0 + n, ntiles - 1), grp * 4 + (at & 3), min(m0 + b * 16 + l15, a.M - 1), kt0, end);
 #pragma unroll
         for (int i = 0; i < NT * MT * 4; ++i) {
             f32x4& to = acc[i / (4 * MT)][(i >> 2) % MT];
             to[i & 3] = i == at ? v : to[i & 3];
         }
     }
+    if (split) a.y += (size_t)split * a.y_slab;
 #pragma unroll
     for (int n = 0; n < NT; ++n)
         if (nt0 + n < ntiles)
@@ -889,13 +896,13 @@ static hipError_t head_gemm_launch(const HeadGemmArgs& a, hipStream_t s) {
 hipError_t launch_head_gemm(const HeadGemmArgs& a, hipStream_t s) {
     if (a.N % 16 || a.K % 32 || a.x_row % 4 || a.x_head % 4 || a.n_valid > a.N || (!a.y && !a.yh)) return hipErrorInvalidValue;
     if (a.M <= 0) return hipSuccess;
-    if (a.splits > 1 && (!a.exact || a.M > 64 || a.K < 256 || a.heads != 1 || !a.y || a.yh || a.decay_bias)) return hipErrorInvalidValue;
+    if (a.splits > 1 && (!a.exact || a.splits > a.K / 256 || a.heads != 1 || !a.y || a.yh || a.decay_bias)) return hipErrorInvalidValue;
     // few rows in 32 bits: K over a workgroup's waves, unless it is too short for them
     if (a.exact && a.M <= 64 && a.K >= 256) return a.M <= 16 ? exact_rows_launch<1>(a, s) : a.M <= 32 ? exact_rows_launch<2>(a, s) : exact_rows_launch<4>(a, s);
     if (a.M <= 16) return head_gemm_launch<1, 1>(a, s);
     if (a.M <= 64) return head_gemm_launch<2, 1>(a, s);
     if (a.exact) {
-        exact_tile_kernel<<<dim3((a.N / 16 + 7) / 8, a.heads, (a.M + 63) / 64), 256, 0, s>>>(a);
+        exact_tile_kernel<<<dim3((a.N / 16 + 7) / 8, a.heads * a.splits, (a.M + 63) / 64), 256, 0, s>>>(a);
         return hipGetLastError();
     }
     return head_gemm_launch<4, 2>(a, s);

@@ -72,3 +72,21 @@ def test_deep_products_and_many_features(width, ffs, vocab, rows):
     ids, logits = m.step([0], [toks], True, want_logits=True)
     assert ids[0] == np.flatnonzero(logits[0] == logits[0].max())[-1]
     m.close()
+
+
+# the same for prompts, whose products are cut over workgroups of 64 rows: K of 1056, 2080 and 4608 in two and four parts, one of them short
+@pytest.mark.parametrize("width,ffs", [(72, (1056, 2080)), (1000, (4608, 1024))])
+@pytest.mark.parametrize("rows", [65, 128, 193])
+def test_deep_products_of_prompts(width, ffs, rows):
+    import nano_vllm_candle_amd as pkg
+
+    cfg = config([light(ff=ffs[0]), attn(ff=ffs[1])], width=width)
+    w = sharp_weights(cfg)
+    c = pkg.GopunexConfig.from_dict(cfg, {k: np.shape(v) for k, v in w.items()})
+    m = pkg.GopunexForCausalLM.from_state_dict(c, w, dtype="float32")
+    m.kv_alloc(4, 2, max_batched_tokens=256)
+    toks = np.random.default_rng(rows).integers(0, cfg["vocab"], rows).tolist()
+    ask = [0, rows // 2, rows - 1]
+    got, ref = m.step_score([0], [toks], True, [ask]), np.asarray(G.forward(cfg, w, toks))[ask]
+    assert row_err(got, ref) < TOL["float32"]
+    m.close()
