@@ -24,8 +24,15 @@ int bias_attn_vdim(int vdim) {
 }
 
 // ---------------------------------------------------------------------------------------------------
-// plain form: one workgroup per (row, head); a wave takes 64 tokens at a time, one per lane for the scores, then one value
-// dimension per lane
+// plain form: one workgroup per (row, head), or, ROWS = 4, per four rows and a head; a wave takes 64 tokens at a time, one per lane for
+// the scores, then one value dimension per lane.  Bound by latency: a lane asks for 32 elements of its key at once, and for its values of
+// the 64 tokens.  Four waves to a row serve a decode step; a prompt's launch fills the chip without them, and a context below 256
+// tokens left some of them idle until the merge.
+// 16 heads of 128, f32 cache, us a launch: decode of 16 rows of 92 tokens on average 11.7 with eight elements asked for at a time, now 8.5; prompts,
+// which took 181 in 16 sequences of 92 tokens on average (four waves, eight elements):
+//                     1 x 260   2 x 260   8 x 65   16 x 92   1 x 1024   1 x 2000
+//   four waves a row     37        64       48       127        320       1138
+//   a wave a row         42        62       31        82        330       1091
 // ---------------------------------------------------------------------------------------------------
 template <typename T>
 __device__ __forceinline__ void load8(float (&x)[8], const T* p) {
@@ -38,17 +45,18 @@ __device__ __forceinline__ void load8(float (&x)[8], const T* p) {
         for (int j = 0; j < 8; ++j) x[j] = (float)v[j];
     }
 }
-template <typename T, int NE>
-__global__ void __launch_bounds__(256) bias_attn_plain_kernel(BiasAttnArgs a) {
+template <typename T, int NE, int ROWS>
+__global__ void __launch_bounds__(256) bias_attn_plain_kernel(BiasAttnArgs a, int rows) {
+    constexpr int WPR = 4 / ROWS;  // waves of a row
     extern __shared__ float sh[];
     __shared__ float pw[4][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int row = blockIdx.x, head = blockIdx.y;
+    const int r = wave / WPR, part = wave % WPR, row = min((int)blockIdx.x * ROWS + r, rows - 1), head = blockIdx.y;  // past the end: the last row again, not stored
     const PagedKV& c = a.kv;
     const int kvh = head / (a.heads / c.kv), pos = a.pos[row];
-    float* q = sh;                      // [dim_p]
-    float* acc = sh + c.dim_p;          // [4][vdim_p + 2]
-    for (int d = threadIdx.x; d < c.dim_p; d += 256) q[d] = a.q[((size_t)row * a.heads + head) * c.dim_p + d];
+    float* q = sh + (size_t)r * c.dim_p;      // [ROWS][dim_p]
+    float* acc = sh + (size_t)ROWS * c.dim_p;  // [4][vdim_p + 2]
+    for (int d = part * 64 + lane; d < c.dim_p; d += WPR * 64) q[d] = a.q[((size_t)row * a.heads + head) * c.dim_p + d];
     __syncthreads();
     const int* bt = a.block_tables + (size_t)a.slot[row] * a.max_blocks;
     const float* bias = a.bias + (size_t)head * a.n_bias;
@@ -56,7 +64,7 @@ __global__ void __launch_bounds__(256) bias_attn_plain_kernel(BiasAttnArgs a) {
 #pragma unroll
     for (int e = 0; e < NE; ++e) o[e] = 0.f;
     const int first = first_seen(pos, a.window);
-    for (int j0 = (first & ~63) + wave * 64; j0 <= pos; j0 += 256) {
+    for (int j0 = (first & ~63) + part * 64; j0 <= pos; j0 += WPR * 64) {
         const int j = j0 + lane;
         const size_t blk = (size_t)bt[j0 / kBlockTokens] * c.kv + kvh;
         const T* kp = reinterpret_cast<const T*>(c.k) + blk * kBlockTokens * c.dim_p + k_packed_offset(j & (kBlockTokens - 1), 0, c.dim_p);
@@ -64,11 +72,12 @@ __global__ void __launch_bounds__(256) bias_attn_plain_kernel(BiasAttnArgs a) {
         const bool seen = j >= first && j <= pos;
         if (seen) {
             s = 0.f;
-            for (int d = 0; d < c.dim_p; d += 8) {
-                float k[8];
-                load8(k, kp + (size_t)(d >> 5) * 512 + ((d & 31) >> 3) * 128);
+            for (int d = 0; d < c.dim_p; d += 32) {
+                float k[4][8];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) s += q[d + i] * k[i];
+                for (int u = 0; u < 4; ++u) load8(k[u], kp + (size_t)(d >> 5) * 512 + u * 128);
+#pragma unroll
+                for (int i = 0; i < 32; ++i) s += q[d + i] * k[i >> 3][i & 7];
             }
             if (a.n_bias) s += bias[min(pos - j, a.n_bias - 1)];
         }
@@ -86,13 +95,13 @@ __global__ void __launch_bounds__(256) bias_attn_plain_kernel(BiasAttnArgs a) {
             const int d = lane + e * 64;
             if (d >= c.vdim_p) continue;
             float t = o[e] * al;
-            for (int x = 0; x < 64; x += 32)
-                for (int g = 0; g < 4; ++g) {
-                    float v[8];
-                    load8(v, vp + v_packed_offset((j0 & (kBlockTokens - 1)) + x + g * 4, d, c.vdim_p));
+            float v[8][8];
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) t += pw[wave][x + (i >> 2) * 16 + g * 4 + (i & 3)] * v[i];
-                }
+            for (int g = 0; g < 8; ++g) load8(v[g], vp + v_packed_offset((j0 & (kBlockTokens - 1)) + (g >> 2) * 32 + (g & 3) * 4, d, c.vdim_p));
+#pragma unroll
+            for (int g = 0; g < 8; ++g)
+#pragma unroll
+                for (int i = 0; i < 8; ++i) t += pw[wave][(g >> 2) * 32 + (i >> 2) * 16 + (g & 3) * 4 + (i & 3)] * v[g][i];
             o[e] = t;
         }
         __builtin_amdgcn_wave_barrier();
@@ -103,18 +112,20 @@ __global__ void __launch_bounds__(256) bias_attn_plain_kernel(BiasAttnArgs a) {
     for (int e = 0; e < NE; ++e)
         if (lane + e * 64 < c.vdim_p) mine[2 + lane + e * 64] = o[e];
     __syncthreads();
+    if ((int)blockIdx.x * ROWS + r >= rows) return;
+    acc += (size_t)r * WPR * (c.vdim_p + 2);
     const float sink = a.sink ? a.sink[head] : 0.f;
-    float ms = a.sink ? sink : -1e30f, f[4];
-    for (int w = 0; w < 4; ++w) ms = fmaxf(ms, acc[(size_t)w * (c.vdim_p + 2)]);
+    float ms = a.sink ? sink : -1e30f, f[WPR];
+    for (int w = 0; w < WPR; ++w) ms = fmaxf(ms, acc[(size_t)w * (c.vdim_p + 2)]);
     float lt = a.sink ? exp2f(sink - ms) : 0.f;
-    for (int w = 0; w < 4; ++w) {
+    for (int w = 0; w < WPR; ++w) {
         f[w] = exp2f(acc[(size_t)w * (c.vdim_p + 2)] - ms);
         lt += f[w] * acc[(size_t)w * (c.vdim_p + 2) + 1];
     }
     const float inv = 1.0f / lt;
-    for (int d = threadIdx.x; d < c.vdim; d += 256) {
+    for (int d = part * 64 + lane; d < c.vdim; d += WPR * 64) {
         float v = 0.f;
-        for (int w = 0; w < 4; ++w) v += f[w] * acc[(size_t)w * (c.vdim_p + 2) + 2 + d];
+        for (int w = 0; w < WPR; ++w) v += f[w] * acc[(size_t)w * (c.vdim_p + 2) + 2 + d];
         v *= inv;
         const int col = head * c.vdim + d;
         if (a.of) a.of[(size_t)row * a.ld + col] = v;
@@ -124,22 +135,24 @@ __global__ void __launch_bounds__(256) bias_attn_plain_kernel(BiasAttnArgs a) {
         }
     }
 }
-template <typename T>
+template <typename T, int ROWS>
 static hipError_t plain_t(const BiasAttnArgs& a, int rows, hipStream_t s) {
-    const dim3 grid(rows, a.heads);
-    const size_t lds = ((size_t)a.kv.dim_p + 4 * (a.kv.vdim_p + 2)) * 4;
-    if (a.kv.vdim_p <= 64) bias_attn_plain_kernel<T, 1><<<grid, 256, lds, s>>>(a);
-    else if (a.kv.vdim_p <= 128) bias_attn_plain_kernel<T, 2><<<grid, 256, lds, s>>>(a);
-    else if (a.kv.vdim_p <= 256) bias_attn_plain_kernel<T, 4><<<grid, 256, lds, s>>>(a);
-    else if (a.kv.vdim_p <= 1024) bias_attn_plain_kernel<T, 16><<<grid, 256, lds, s>>>(a);
+    const dim3 grid((rows + ROWS - 1) / ROWS, a.heads);
+    const size_t lds = ((size_t)ROWS * a.kv.dim_p + 4 * (a.kv.vdim_p + 2)) * 4;
+    if (a.kv.vdim_p <= 64) bias_attn_plain_kernel<T, 1, ROWS><<<grid, 256, lds, s>>>(a, rows);
+    else if (a.kv.vdim_p <= 128) bias_attn_plain_kernel<T, 2, ROWS><<<grid, 256, lds, s>>>(a, rows);
+    else if (a.kv.vdim_p <= 256) bias_attn_plain_kernel<T, 4, ROWS><<<grid, 256, lds, s>>>(a, rows);
+    else if (a.kv.vdim_p <= 1024) bias_attn_plain_kernel<T, 16, ROWS><<<grid, 256, lds, s>>>(a, rows);
     else return hipErrorNotSupported;
     return hipGetLastError();
 }
+constexpr int kPlainRowsAlone = 8192;  // (row, head) pairs from which a wave to each is the faster: the table at the kernel
 hipError_t launch_bias_attn_plain(const BiasAttnArgs& a, int rows, hipStream_t s) {
     if (a.heads % a.kv.kv || a.kv.dim_p % 32 || a.kv.vdim_p % 16 || (!a.of && !a.oh)) return hipErrorInvalidValue;
     if (a.kv.dim_p > 4096) return hipErrorNotSupported;
     if (rows <= 0) return hipSuccess;
-    return a.kv.f32 ? plain_t<float>(a, rows, s) : plain_t<_Float16>(a, rows, s);
+    if ((int64_t)rows * a.heads >= kPlainRowsAlone && a.kv.dim_p <= 1024) return a.kv.f32 ? plain_t<float, 4>(a, rows, s) : plain_t<_Float16, 4>(a, rows, s);
+    return a.kv.f32 ? plain_t<float, 1>(a, rows, s) : plain_t<_Float16, 1>(a, rows, s);
 }
 
 // ---------------------------------------------------------------------------------------------------
