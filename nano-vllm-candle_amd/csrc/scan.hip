@@ -270,10 +270,13 @@ __global__ void __launch_bounds__(256) scan_decode_kernel(ScanArgs a) {
     if ((int)threadIdx.x * 4 < CH) put_row4(a, row, blockIdx.x * CH + threadIdx.x * 4, f32x4{ys[threadIdx.x * 4], ys[threadIdx.x * 4 + 1], ys[threadIdx.x * 4 + 2], ys[threadIdx.x * 4 + 3]});
 }
 
-// one workgroup: CH channels of one piece, TB tokens at a time staged through LDS, the next TB on their way in registers
+// one workgroup: CH channels of one piece, TB tokens at a time staged through LDS, the next TB on their way in registers.  Bound by the VALU
+// (an exponential and five other operations a state, token and channel: 4096 rows of 2048 channels x 16 states are 35 us of issue, measured 57 in equal
+// pieces) and, with unequal ones, by the longest: ScanScratch::plan.  A channel's lanes store one token's sum each, so that a group of
+// U tokens is one stretch of code without a branch, and the next group's operands leave LDS under it: one sequence of 2000 rows 70 -> 64.
 template <int NS, int NL, int TB, bool CARRY>
 __global__ void __launch_bounds__(256) scan_prompt_kernel(ScanArgs a) {
-    constexpr int CH = 256 / NL, ST = NS * NL, NX = (TB * CH + 255) / 256, NB = (TB * 2 * ST + 255) / 256;
+    constexpr int CH = 256 / NL, ST = NS * NL, NX = (TB * CH / 4 + 255) / 256, NB = (TB * 2 * ST / 4 + 255) / 256;
     extern __shared__ __attribute__((aligned(16))) float sm[];
     float *bcs = sm, *xs = bcs + TB * 2 * ST, *dts = xs + TB * CH, *zs = dts + TB * CH;  // zs becomes the output
     const int tid = threadIdx.x, q = tid % NL, lc = tid / NL, c0 = blockIdx.x * CH, c = c0 + lc;
@@ -311,71 +314,102 @@ __global__ void __launch_bounds__(256) scan_prompt_kernel(ScanArgs a) {
             }
         }
     }
-    float rx[NX], rd[NX], rz[NX], rb[NB];
+    f32x4 rx[NX], rd[NX], rz[NX], rb[NB];
+    // four channels at a time, one by one where the rows do not allow it
+    const bool vec = ((a.channels | a.ldx | a.ldz) & 3) == 0 && (((uintptr_t)a.x | (uintptr_t)a.z | (uintptr_t)a.z_stride * 4) & 15) == 0;
+    auto get4 = [&](const float* p, int ch) -> f32x4 {
+        if (vec) return *reinterpret_cast<const f32x4*>(p + min(ch, a.channels - 4));
+        const int last = a.channels - 1;
+        return f32x4{p[min(ch, last)], p[min(ch + 1, last)], p[min(ch + 2, last)], p[min(ch + 3, last)]};
+    };
     auto fetch = [&](int t0) {
 #pragma unroll
         for (int i = 0; i < NX; ++i) {
-            const int e = tid + i * 256, t = min(t0 + e / CH, n - 1), ch = min(c0 + e % CH, a.channels - 1);
+            const int e = (tid + i * 256) * 4, t = min(t0 + e / CH, n - 1), ch = c0 + e % CH;
             const size_t row = row0 + t;
-            rx[i] = a.x[row * a.ldx + ch];
-            rd[i] = a.dt[row * a.channels_p + ch];
-            if constexpr (!CARRY) rz[i] = slab_elem(a.z + row * a.ldz + ch, a.z_slabs, a.z_stride);
+            rx[i] = get4(a.x + row * a.ldx, ch);
+            rd[i] = *reinterpret_cast<const f32x4*>(a.dt + row * a.channels_p + ch);
+            if (t0 + e / CH >= n) rd[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (!CARRY) {
+                rz[i] = get4(a.z + row * a.ldz, ch);
+                for (int z = 1; z < a.z_slabs; ++z) rz[i] += get4(a.z + z * a.z_stride + row * a.ldz, ch);
+            }
         }
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
-            const int e = tid + i * 256, t = min(t0 + e / (2 * ST), n - 1), j = e % (2 * ST);
-            rb[i] = a.bc[(size_t)(row0 + t) * a.ldbc + (j < ST ? a.b0 + j : a.c0 + j - ST)];
+            const int e = (tid + i * 256) * 4, t = min(t0 + e / (2 * ST), n - 1), j = e % (2 * ST);
+            rb[i] = *reinterpret_cast<const f32x4*>(a.bc + (size_t)(row0 + t) * a.ldbc + (j < ST ? a.b0 + j : a.c0 + j - ST));
         }
     };
+    // U tokens at a time: everything but the state's own chain is independent.  Tokens past the end have dt = 0: the state stays.
+    constexpr int U = NS == 4 ? 4 : 1;
+    struct Group { float dt[U], x[U], B[U][NS], C[U][NS]; };
     fetch(0);
     for (int t0 = 0; t0 < n; t0 += TB) {
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < NX; ++i) {
-            const int e = tid + i * 256;
-            if (TB * CH % 256 && e >= TB * CH) continue;
-            xs[e] = rx[i];
-            dts[e] = rd[i];
-            if constexpr (!CARRY) zs[e] = rz[i];
+            const int e = (tid + i * 256) * 4;
+            if (TB * CH % 1024 && e >= TB * CH) continue;
+            *reinterpret_cast<f32x4*>(xs + e) = rx[i];
+            *reinterpret_cast<f32x4*>(dts + e) = rd[i];
+            if constexpr (!CARRY) *reinterpret_cast<f32x4*>(zs + e) = rz[i];
         }
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
-            const int e = tid + i * 256;
-            if (TB * 2 * ST % 256 == 0 || e < TB * 2 * ST) bcs[e] = rb[i];
+            const int e = (tid + i * 256) * 4;
+            if (TB * 2 * ST % 1024 == 0 || e < TB * 2 * ST) *reinterpret_cast<f32x4*>(bcs + e) = rb[i];
         }
         __syncthreads();
         if (t0 + TB < n) fetch(t0 + TB);
         const int m = min(TB, n - t0);
-        // U tokens at a time: everything but the state's own chain is independent.  Tokens past the end have dt = 0: the state stays.
-        constexpr int U = NS == 4 ? 4 : 1;
-        for (int t = 0; t < m; t += U) {
-            float dt[U], x[U], dx[U], B[U][NS], C[U][NS], y[U];
+        auto read = [&](int t, Group& g) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int tt = t + u;
-                dt[u] = tt < m ? dts[tt * CH + lc] : 0.f;
-                x[u] = xs[tt * CH + lc];
-                dx[u] = dt[u] * x[u];
-                load_states(B[u], bcs + tt * 2 * ST + q * NS);
-                if constexpr (!CARRY) load_states(C[u], bcs + tt * 2 * ST + ST + q * NS);
+                const int tt = min(t + u, TB - 1);
+                g.dt[u] = dts[tt * CH + lc];
+                g.x[u] = xs[tt * CH + lc];
+                load_states(g.B[u], bcs + tt * 2 * ST + q * NS);
+                if constexpr (!CARRY) load_states(g.C[u], bcs + tt * 2 * ST + ST + q * NS);
             }
+        };
+        auto step = [&](int t, const Group& g) {
+            float y[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
+                const float dx = g.dt[u] * g.x[u];
                 y[u] = 0.f;
 #pragma unroll
                 for (int i = 0; i < NS; ++i) {
-                    S[i] = S[i] * __builtin_amdgcn_exp2f(dt[u] * A[i]) + dx[u] * B[u][i];
-                    if constexpr (!CARRY) y[u] += S[i] * C[u][i];
+                    S[i] = S[i] * __builtin_amdgcn_exp2f(g.dt[u] * A[i]) + dx * g.B[u][i];
+                    if constexpr (!CARRY) y[u] += S[i] * g.C[u][i];
                 }
-                if constexpr (CARRY) total += dt[u];
+                if constexpr (CARRY) total += g.dt[u];
             }
             if constexpr (!CARRY) {
+                // this channel's x there has been read by its lanes' wave
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    y[u] = lanes_sum<NL>(y[u]);
-                    if (q == 0) xs[(t + u) * CH + lc] = y[u] + D * x[u];  // this channel's x there has been read by its lanes' wave
+                for (int u = 0; u < U; ++u) y[u] = lanes_sum<NL>(y[u]) + D * g.x[u];
+                if constexpr (NL >= U) {
+                    float v = y[0];
+#pragma unroll
+                    for (int u = 1; u < U; ++u) v = q == u ? y[u] : v;
+                    if (q < U) xs[(t + q) * CH + lc] = v;
+                } else if (q == 0) {
+#pragma unroll
+                    for (int u = 0; u < U; ++u) xs[(t + u) * CH + lc] = y[u];
                 }
             }
+        };
+        // the next group's operands leave LDS under this one's chain
+        Group g0, g1;
+        read(0, g0);
+        for (int t = 0; t < m; t += 2 * U) {
+            read(t + U, g1);
+            step(t, g0);
+            if (t + U >= m) break;
+            read(t + 2 * U, g0);
+            step(t + U, g1);
         }
         if constexpr (!CARRY) {
             __syncthreads();
