@@ -273,7 +273,8 @@ __global__ void __launch_bounds__(256) scan_decode_kernel(ScanArgs a) {
 // one workgroup: CH channels of one piece, TB tokens at a time staged through LDS, the next TB on their way in registers.  Bound by the VALU
 // (an exponential and five other operations a state, token and channel: 4096 rows of 2048 channels x 16 states are 35 us of issue, measured 57 in equal
 // pieces) and, with unequal ones, by the longest: ScanScratch::plan.  A channel's lanes store one token's sum each, so that a group of
-// U tokens is one stretch of code without a branch, and the next group's operands leave LDS under it: one sequence of 2000 rows 70 -> 64.
+// U tokens is one stretch of code without a branch: one sequence of 2000 rows 70 -> 60.  Reading the next group's operands ahead takes
+// registers from the four waves of a SIMD and gave nothing (64)
 template <int NS, int NL, int TB, bool CARRY>
 __global__ void __launch_bounds__(256) scan_prompt_kernel(ScanArgs a) {
     constexpr int CH = 256 / NL, ST = NS * NL, NX = (TB * CH / 4 + 255) / 256, NB = (TB * 2 * ST / 4 + 255) / 256;
@@ -366,7 +367,7 @@ __global__ void __launch_bounds__(256) scan_prompt_kernel(ScanArgs a) {
         auto read = [&](int t, Group& g) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int tt = min(t + u, TB - 1);
+                const int tt = t + u;
                 g.dt[u] = dts[tt * CH + lc];
                 g.x[u] = xs[tt * CH + lc];
                 load_states(g.B[u], bcs + tt * 2 * ST + q * NS);
@@ -401,15 +402,10 @@ __global__ void __launch_bounds__(256) scan_prompt_kernel(ScanArgs a) {
                 }
             }
         };
-        // the next group's operands leave LDS under this one's chain
-        Group g0, g1;
-        read(0, g0);
-        for (int t = 0; t < m; t += 2 * U) {
-            read(t + U, g1);
-            step(t, g0);
-            if (t + U >= m) break;
-            read(t + 2 * U, g0);
-            step(t + U, g1);
+        for (int t = 0; t < m; t += U) {
+            Group g;
+            read(t, g);
+            step(t, g);
         }
         if constexpr (!CARRY) {
             __syncthreads();

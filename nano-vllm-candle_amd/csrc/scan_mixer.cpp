@@ -133,8 +133,8 @@ int ScanScratch::plan(nvllm_model* m, const int* slot, const int* seq, int R) {
     if (!d_plan) return NVLLM_OK;
     // As many pieces as fill the chip beside the channels, of equal length -- but none where the longest sequence is at most half as long again: a
     // second pass over all pieces but the last costs more.  Longest first: the workgroups of the longest share their CUs with the
-    // shortest.  2048 channels, sequences of 64 to 512: 3456 rows 112 us a layer in chunk order and cut at 432, now 73; one of 2000 rows, cut in eight,
-    // 64, in four 124 and in two 235
+    // shortest.  2048 channels, sequences of 64 to 512: 3456 rows 112 us a layer in chunk order and cut at 432, now 72; one of 2000 rows, cut in eight,
+    // 60, in four 124 and in two 235
     const int want = std::max(1, kScanWaves / waves);
     int longest = std::max(kShortestPiece, up((R + want - 1) / want, 16)), pieces = 0;
     std::vector<std::pair<int, int>> segs;  // rows, first row
