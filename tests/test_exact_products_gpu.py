@@ -90,3 +90,27 @@ def test_deep_products_of_prompts(width, ffs, rows):
     got, ref = m.step_score([0], [toks], True, [ask]), np.asarray(G.forward(cfg, w, toks))[ask]
     assert row_err(got, ref) < TOL["float32"]
     m.close()
+
+
+# input projections in parts: every row kernel behind them reads two slabs of a prompt's rows
+@pytest.mark.parametrize("name", ["gopunex", "lefalix"])
+@pytest.mark.parametrize("rows", [65, 130])
+def test_split_input_projections_of_prompts(name, rows):
+    import nano_vllm_candle_amd as pkg
+    from oracle import lefalix_oracle as LO
+    from tests import gopunex_util as GU, lefalix_util as LU
+
+    if name == "gopunex":
+        cfg = config([light(ff=0), attn(ff=0), GU.delta(ff=0)], width=1024)
+        w, tol, make, conf = sharp_weights(cfg), TOL["float32"], pkg.GopunexForCausalLM, pkg.GopunexConfig
+    else:
+        cfg = LU.config([LU.par(mlp=LU.dense(1024)), LU.delta(LU.dense(1100))], width=1024)
+        w, tol, make, conf = LU.weights(cfg), LU.TOL["float32"], pkg.LefalixForCausalLM, pkg.LefalixConfig
+    m = make.from_state_dict(conf.from_dict(cfg, {k: np.shape(v) for k, v in w.items()}), {k: np.asarray(v, np.float32) for k, v in w.items()}, dtype="float32")
+    m.kv_alloc(4, 2, max_batched_tokens=256)
+    toks = np.random.default_rng(rows).integers(0, cfg["vocab"], rows).tolist()
+    ask = [0, 1, rows // 2, rows - 2, rows - 1]
+    ref = np.asarray(G.forward(cfg, w, toks) if name == "gopunex" else LO.run(cfg, w, toks)[0])
+    assert row_err(m.step_score([0], [toks], True, [ask]), ref[ask]) < tol
+    assert row_err(m.step([0], [toks + [3]], False, want_logits=True)[1], (G.forward(cfg, w, toks + [3]) if name == "gopunex" else LO.run(cfg, w, toks + [3])[0])[-1:]) < tol
+    m.close()
