@@ -1183,7 +1183,10 @@ static int forward_chunk_fused(nvllm_model* m, const FusedPlan& fp, int R, int n
             PROF(m, PROF_GEMM, launch_gemm(pq, m->xh, m->xl, H, w.qkv, m->slabs, R, s));
             qa.qkv = m->slabs; qa.n_slabs = pq.n_split;
         }
-        if (!fuse_qk && !qkv_whole) PROF(m, PROF_QK, launch_qk_norm_rope_kvwrite(qa, R, s));
+        if (!fuse_qk && !qkv_whole) {
+            PROF(m, PROF_QK, launch_qk_norm_rope_kvwrite(qa, R, s));
+            m->qk_rows16_launches += qk_rows16_wins(R, m->nh_l + 2 * m->kv_l, hd);
+        }
         AttnArgs aa;
         aa.q = m->qbuf; aa.kv = qa.kv; aa.block_tables = m->d_block_tables; aa.max_blocks = m->max_blocks;
         aa.tile_row0 = m->d_tile_row0; aa.tile_nrows = m->d_tile_nrows; aa.tile_slot = m->d_tile_slot; aa.pos = m->d_pos;
@@ -1375,7 +1378,10 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
             if (t_qkv) PROF(m, PROF_GEMM, launch_gemm_tile(m->xh, m->xl, w.qkv, R, 0, m->slabs, nullptr, nullptr, 0, tmin, max_ks, &qa.n_slabs, s));
             else rcg = gemm_slabs(m, m->xh, m->xl, H, w.qkv, m->slabs, R, 8, &qa.n_slabs, packed);
             if (rcg) return rcg;
-            if (!fuse_qk) PROF(m, PROF_QK, launch_qk_norm_rope_kvwrite(qa, R, s));
+            if (!fuse_qk) {
+                PROF(m, PROF_QK, launch_qk_norm_rope_kvwrite(qa, R, s));
+                m->qk_rows16_launches += qk_rows16_wins(R, m->nh_l + 2 * m->kv_l, hd);
+            }
         }
         if (trim && n_last == 0) return NVLLM_OK;  // keys and values are written, nothing else of this layer is read
         AttnArgs aa;
@@ -2103,13 +2109,15 @@ extern "C" int nvllm_debug_set_option(nvllm_model* m, const char* name, int valu
 }
 
 // counters for tests: "oneshot_calls" = all-reduces this model's context has run on the one-shot device path;
-// "tile_gemm_launches" = projections this model has run on the prefill tile GEMM; "table_copies" = whole block tables sent
+// "tile_gemm_launches" = projections this model has run on the prefill tile GEMM; "table_copies" = whole block tables sent;
+// "qk_rows16_launches" = q/k norm launches of 16 rows and a head per workgroup
 extern "C" int nvllm_debug_get_counter(nvllm_model* m, const char* name, int64_t* value) {
     if (!m || !name || !value) return NVLLM_EINVAL;
     if (!strcmp(name, "oneshot_calls")) { *value = (int64_t)m->ctx->os_calls; return NVLLM_OK; }
     if (!strcmp(name, "latent_expanded")) { *value = m->latent_expanded; return NVLLM_OK; }
     if (!strcmp(name, "table_copies")) { *value = m->table_copies; return NVLLM_OK; }
     if (!strcmp(name, "tile_gemm_launches")) { *value = m->tile_launches; return NVLLM_OK; }
+    if (!strcmp(name, "qk_rows16_launches")) { *value = m->qk_rows16_launches; return NVLLM_OK; }
     if (!strcmp(name, "kv_f16_saturated") || !strcmp(name, "kv_f16_absmax_bits")) {
         // scan of the whole K/V pool (debug, off the hot path): elements the f16_sat clamp of a cache write produced, and the
         // largest magnitude stored (f16 bits; 0x7BFF = 65504 is the clamp)

@@ -208,6 +208,7 @@ struct QkvArgs {
     RowNorm rn;                  // deferred input norm (qkv sums are multiplied by rinv[row] first)
 };
 hipError_t launch_qk_norm_rope_kvwrite(const QkvArgs& a, int rows, hipStream_t s);
+bool qk_rows16_wins(int rows, int heads, int hd);  // ... by 16 rows and a head per workgroup
 
 // ---- prefill GEMM (tile_gemm.hip): 256 x 256/192 output tile, both operands in fragment order -------------------
 // x planes in xpack_off order; mode 0: out f32 [M][N]; mode 2: w = interleaved gate/up, act hi/lo [M][N/2] (row-major or

@@ -1977,11 +1977,18 @@ __global__ void __launch_bounds__(256) qk_rows16_kernel(QkvArgs a, int rows) {
     }
 }
 
+// Enough workgroups of 16 rows and a head that every CU has one; below, a wave to each (row, head) spreads the same loads over more CUs.  us a
+// launch between two events, which are 5 of them, a wave per (row, head) / 16 rows: 32 heads (0.6B) 16 rows 6.8 / 7.6, 64 7.2 / 7.5, 129
+// 7.8 / 7.9, 160 8.1 / 8.1, 200 8.5 / 8.3, 300 10.7 / 9.6; with a 24-bit cache 16 rows 7.0 / 8.1, 64 7.2 / 8.1, 160 8.5 / 8.6, 256 9.5 / 9.2;
+// 48 heads (8B) 16 rows 6.6 / 6.9, 64 7.4 / 7.5, 100 8.3 / 8.1, 200 13.9 / 12.0.  0.6B prompts of 16 and 64 tokens 1.026 / 1.044 and 1.205 / 1.209 ms,
+// 24-bit 1.065 / 1.098 and 1.277 / 1.298.
+bool qk_rows16_wins(int rows, int heads, int hd) { return hd == 128 && (rows + 15) / 16 * heads >= 320; }
+
 hipError_t launch_qk_norm_rope_kvwrite(const QkvArgs& a, int rows, hipStream_t s) {
     if (a.kv.hd > 128 || a.kv.hd % 32 != 0) return hipErrorInvalidValue;
     if (rows <= 0) return hipSuccess;
     const int heads = a.nh_l + 2 * a.kv.kv_l;
-    if (a.kv.hd == 128) {
+    if (qk_rows16_wins(rows, heads, a.kv.hd)) {
         qk_rows16_kernel<<<dim3((rows + 15) / 16, heads), 256, 0, s>>>(a, rows);
         return hipGetLastError();
     }

@@ -219,6 +219,7 @@ struct nvllm_model {
     bool stamps_on = false;
     int stamp_launch = 0;
     int64_t tile_launches = 0;  // projections run by the tile GEMM so far (tests assert the path they force was taken)
+    int64_t qk_rows16_launches = 0;  // likewise: q/k norm, rotation and cache writes by 16 rows and a head
 
     // per-kernel-class HIP-event timing (bench roofline leg); 0 = off
     int prof_kind = 0;
