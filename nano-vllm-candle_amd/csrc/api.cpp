@@ -13,6 +13,7 @@
 #include <map>
 #include <memory>
 #include <mutex>
+#include <numeric>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -1203,6 +1204,7 @@ static int forward_chunk_fused(nvllm_model* m, const FusedPlan& fp, int R, int n
             aa.part_tiles = m->attn_part_tiles; aa.max_parts = kAttnMaxParts; aa.part_o = m->attn_po; aa.part_ml = m->attn_pml;
             parts_max = m->attn_parts_max;
             if (fuse_qk) aa.waves = m->attn_waves;
+            m->eight_wave_launches += aa.waves == 8;
         }
         PROF(m, PROF_EMPTY, hipSuccess);  // calibration: an event pair around nothing, at the attention launch's place
         STAMPS(aa, m);
@@ -1401,6 +1403,7 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
             aa.part_tiles = m->attn_part_tiles; aa.max_parts = kAttnMaxParts; aa.part_o = m->attn_po; aa.part_ml = m->attn_pml;
             parts_max = m->attn_parts_max;
             if (fuse_qk) aa.waves = m->attn_waves;
+            m->eight_wave_launches += aa.waves == 8;
         }
         STAMPS(aa, m);
         int attn_tiles = n_tiles;
@@ -1522,16 +1525,33 @@ static int ensure_blocks(nvllm_model* m, SeqState& s, int len) {
     return NVLLM_OK;
 }
 
+// Eight waves of a decode attention's workgroup instead of four halve its chain of tiles, but the merge and the two waves of a SIMD cost up to 1 us:
+// only where launches leave a CU one workgroup at most, and not
+//  - in a 16-bit cache on whole contexts (up to 16 tiles) of many workgroups or query heads, nor on 5 to 8 tiles;
+//  - while parts of four waves, a tile each, have a CU to themselves and are so few that the combine pass is no longer for them;
+//  - where parts that fit the CUs leave a quarter of them idle and the longest of ragged contexts is what the launch waits for.
+// Attention and its combine pass, us a layer between two events (5 of them the events'), four waves / eight; rows x tokens, 8 kv heads:
+//   gqa 2   whole 16 x 400 15.4 / 14.8, 20 x 500 17.4 / 16.8, 24 x 500 17.9 / 18.3, 32 x 400 18.3 / 19.3; 8 x 129 11.2 / 11.3
+//   gqa 4   whole 8 x 400 14.6 / 14.4, 16 x 400 15.4 / 15.7, 24 x 400 18.3 / 19.5, 32 x 280 17.4 / 18.6; 8 x 129 11.4 / 11.9
+//   gqa 1   whole 20 x 400 15.9 / 15.5, 24 x 511 18.1 / 18.8, 32 x 511 20.0 / 21.9
+//   gqa 2   parts 1 x 600 14.1 / 14.9, 1 x 1100 15.7 / 15.8, 1 x 1500 17.1 / 16.2, 4 x 600 14.8 / 15.4, 4 x 1100 19.4 / 16.9, 6 x 600 15.8 / 15.9, 6 x 700 18.1 / 16.1, 8 x 600 18.1 / 16.5
+//   gqa 4   parts 1 x 600 15.0 / 15.9, 1 x 1100 16.4 / 16.8, 1 x 2000 19.4 / 18.1, 4 x 700 16.1 / 16.4
+//   gqa 2   of 256 to 2048, 12 rows 25.1 / 25.2, 16 28.3 / 27.4, 20 31.9 / 33.6, 24 32.7 / 34.6, 28 36.8 / 36.1, 32 40.8 / 37.9; gqa 4, 24 rows 34.2 / 35.9
+//   gqa 2   of 64 to 512, 24 rows 18.7 / 16.8; 24 x 2000 43.9 / 39.5
+//   24 bits whole 8 x 400 20.7 / 17.1, 24 x 400 22.7 / 20.8, 32 x 400 24.3 / 23.6; 1 x 600 15.3 / 16.3; of 600 to 3000, 24 rows 59.5 / 65.1, 28 67.0 / 70.9, 32 75.3 / 74.3
+static bool eight_waves_win(const nvllm_model* m, int wgs, int tiles, bool ragged) {
+    if (m->hd != 128 || wgs > 256 || tiles <= (wgs < 64 ? 8 : 4)) return false;
+    const bool wide = !m->vlocache.empty();
+    if (tiles <= 16) return wide || wgs < 64 || (tiles > 8 && wgs <= 160 && wgs * m->gqa <= 320);
+    if (tiles <= std::min(wgs <= 16 ? 40 : 32, 1024 / wgs)) return false;
+    return !ragged || 256 / wgs * wgs > (wide ? 224 : 192) || tiles <= (wgs < 128 ? 48 : 32);
+}
 // Split a sequence's context over several workgroups only when (sequences x kv heads) alone cannot fill
 // the chip (small batches, long contexts); a full batch already has >= 2 workgroups per CU.
-// Launches of up to 256 workgroups leave a CU one of them: eight waves instead of four halve its chain of tiles, the registers allow no more.
-// Attention and its combine pass, us a layer, four waves / eight.  0.6B (8 kv heads): 8 rows of 64 to 1500 tokens 18.1 / 16.8, 16 of 100 to 800
-// 18.0 / 16.4, 24 of 64 to 512 17.3 / 14.7, 32 of 64 to 512 19.3 / 15.5, 32 of 131 to 1500 31.5 / 27.7, one of 2000 15.3 / 13.9, of 900 12.0 /
-// 12.3, of 400 11.5 / 11.6, of 137 8.4 / 8.8; 24 with a 24-bit cache 20.1 / 17.3; 8B: 16 of 64 to 600 16.2 / 14.2, 24 of 256 to 2048 32.2 / 33.1.
-static void set_attn_split(nvllm_model* m, int n_seqs, int max_len) {
+static void set_attn_split(nvllm_model* m, int n_seqs, int max_len, int64_t all_len) {
     const int tiles = (max_len + 31) / 32;
     const int base_wgs = std::max(1, n_seqs * m->kv_l);
-    const bool eight = m->hd == 128 && base_wgs <= 256 && tiles > (base_wgs < 64 ? 8 : 4);
+    const bool eight = eight_waves_win(m, base_wgs, tiles, 4 * all_len < 3 * (int64_t)n_seqs * max_len);
     m->attn_waves = eight ? 8 : 4;
     int want = std::min(kAttnMaxParts, std::max(1, (eight ? 256 : 512) / base_wgs));
     // a few more rounds of the loop cost less than the combine launch and its boundary (4.7 + 1.4 us): up to 512 tokens, and up to 1024 where
@@ -1840,7 +1860,7 @@ static int step_impl(nvllm_model* m, int n_seqs, const int64_t* seq_ids, const u
     m->want_ids = !score && !temperatures;
     m->cur_n = n_seqs;
     m->cur_max_len = *std::max_element(lens, lens + n_seqs);
-    set_attn_split(m, n_seqs, m->cur_max_len);
+    set_attn_split(m, n_seqs, m->cur_max_len, std::accumulate(lens, lens + n_seqs, (int64_t)0));
     // rows and q-tiles
     RowPlan p;
     bool all_single = true;
@@ -2003,7 +2023,7 @@ static int decode_core(nvllm_model* m) {
     m->want_ids = true;
     m->cur_n = n;
     m->cur_max_len = *std::max_element(m->last_lens.begin(), m->last_lens.end()) + 1;
-    set_attn_split(m, n, m->cur_max_len);
+    set_attn_split(m, n, m->cur_max_len, std::accumulate(m->last_lens.begin(), m->last_lens.end(), (int64_t)n));
     const bool recurrent = m->dec && m->dec->recurrent();
     if (recurrent) for (int64_t id : m->last_ids) m->seqs[id].cached = 0;  // until the step is on the stream
     int rc = forward_chunk(m, n, n, 1, n, 0);
@@ -2110,7 +2130,7 @@ extern "C" int nvllm_debug_set_option(nvllm_model* m, const char* name, int valu
 
 // counters for tests: "oneshot_calls" = all-reduces this model's context has run on the one-shot device path;
 // "tile_gemm_launches" = projections this model has run on the prefill tile GEMM; "table_copies" = whole block tables sent;
-// "qk_rows16_launches" = q/k norm launches of 16 rows and a head per workgroup
+// "qk_rows16_launches" = q/k norm launches of 16 rows and a head per workgroup; "eight_wave_launches" = decode attention on eight waves
 extern "C" int nvllm_debug_get_counter(nvllm_model* m, const char* name, int64_t* value) {
     if (!m || !name || !value) return NVLLM_EINVAL;
     if (!strcmp(name, "oneshot_calls")) { *value = (int64_t)m->ctx->os_calls; return NVLLM_OK; }
@@ -2118,6 +2138,7 @@ extern "C" int nvllm_debug_get_counter(nvllm_model* m, const char* name, int64_t
     if (!strcmp(name, "table_copies")) { *value = m->table_copies; return NVLLM_OK; }
     if (!strcmp(name, "tile_gemm_launches")) { *value = m->tile_launches; return NVLLM_OK; }
     if (!strcmp(name, "qk_rows16_launches")) { *value = m->qk_rows16_launches; return NVLLM_OK; }
+    if (!strcmp(name, "eight_wave_launches")) { *value = m->eight_wave_launches; return NVLLM_OK; }
     if (!strcmp(name, "kv_f16_saturated") || !strcmp(name, "kv_f16_absmax_bits")) {
         // scan of the whole K/V pool (debug, off the hot path): elements the f16_sat clamp of a cache write produced, and the
         // largest magnitude stored (f16 bits; 0x7BFF = 65504 is the clamp)

@@ -9,24 +9,21 @@ pytestmark = pytest.mark.gpu
 LENGTHS = [1, 31, 33, 126, 127, 128, 159, 255, 256, 257, 510, 511, 512, 1021, 1022, 1023, 1024]
 
 
-# workgroups: 256 and 264 of 8 kv heads; 128 and 124 of 4 (whole and in parts from 513 tokens on); 2 and 257 of one, whose 18 heads take
-# more rounds of four waves than are loaded up front; 8 heads of 64
-@pytest.mark.parametrize("hd,kv,heads,rows,bits", [(128, 8, 16, 32, 16), (128, 8, 16, 33, 16), (128, 4, 8, 32, 16), (128, 4, 8, 31, 24), (128, 1, 16, 2, 16),
-                                                   (128, 1, 16, 257, 16), (128, 1, 8, 17, 24), (64, 1, 8, 17, 16), (64, 1, 16, 3, 16)])
-def test_a_step_equals_the_prompt(hd, kv, heads, rows, bits):
+def check(hd, kv, heads, lens, bits, eight):
     import nano_vllm_candle_amd as pkg
 
+    rows = len(lens)
     cfg = pkg.Qwen3Config.tiny(hidden_size=256, head_dim=hd, num_attention_heads=heads, num_key_value_heads=kv)
     m = pkg.Qwen3ForCausalLM.from_synthetic(cfg, 3)
     if bits == 24:
         m.set_option("kv_v_bits", 24)
         m.set_option("kv_k_bits", 24)
-    lens = [LENGTHS[(i * 7) % len(LENGTHS)] for i in range(rows)]
     m.kv_alloc(sum(n // 256 + 1 for n in lens) + 8, rows + 1, 2048)
     rng = np.random.default_rng(rows + heads)
     seqs = [rng.integers(0, cfg.vocab_size, n + 1) for n in lens]
     m.step(list(range(rows)), [s[:-1] for s in seqs], True, want_logits=False)
     _, got = m.step(list(range(rows)), seqs, False, want_logits=True)
+    assert m.counter("eight_wave_launches") == eight * cfg.num_hidden_layers
     # the prompt's kernels sum in another order, from keys whose f16 may round the other way: 2^-11 of the largest logit, 2^-14 with the residuals
     bound = 2.0 ** (-11 if bits == 16 else -14)
     for i in range(min(rows, 34)):
@@ -34,3 +31,22 @@ def test_a_step_equals_the_prompt(hd, kv, heads, rows, bits):
         m.seq_free(rows)
         assert np.abs(got[i] - want[0]).max() < bound * np.abs(want).max(), (i, lens[i])
     m.close()
+
+
+# workgroups: 256 and 264 of 8 kv heads; 128 and 124 of 4 (whole and in parts from 513 tokens on); 2 and 257 of one, whose 18 heads take
+# more rounds of four waves than are loaded up front; 8 heads of 64
+@pytest.mark.parametrize("hd,kv,heads,rows,bits,eight", [(128, 8, 16, 32, 16, 1), (128, 8, 16, 33, 16, 0), (128, 4, 8, 32, 16, 1), (128, 4, 8, 31, 24, 1), (128, 1, 16, 2, 16, 0),
+                                                         (128, 1, 16, 257, 16, 0), (128, 1, 8, 17, 24, 1), (64, 1, 8, 17, 16, 0), (64, 1, 16, 3, 16, 0)])
+def test_a_step_equals_the_prompt(hd, kv, heads, rows, bits, eight):
+    check(hd, kv, heads, [LENGTHS[(i * 7) % len(LENGTHS)] for i in range(rows)], bits, eight)
+
+
+# both sides of each line of the rule: whole contexts by workgroups and query heads, parts of a tile a wave, ragged contexts whose parts leave CUs idle
+@pytest.mark.parametrize("kv,heads,lens,bits,eight", [
+    (8, 16, [255], 16, 0), (8, 16, [256], 16, 1), (8, 16, [255] * 8, 16, 0), (8, 16, [256] * 8, 16, 1), (8, 16, [130] * 8, 24, 1), (8, 16, [300] * 20, 16, 1), (8, 16, [300] * 21, 16, 0), (8, 16, [300] * 21, 24, 1),
+    (8, 32, [300] * 10, 16, 1), (8, 32, [300] * 11, 16, 0), (4, 4, [300] * 40, 16, 1), (4, 4, [300] * 41, 16, 0),
+    (8, 16, [511], 16, 1), (8, 16, [512], 16, 0), (8, 16, [1279], 16, 0), (8, 16, [1280], 16, 1), (8, 16, [1023] * 3, 16, 0), (8, 16, [1024] * 3, 16, 1), (8, 16, [671] * 6, 16, 0), (8, 16, [672] * 6, 16, 1), (8, 16, [512] * 8, 16, 1), (8, 16, [1279], 24, 0), (8, 16, [1280], 24, 1),
+    (8, 16, [256, 1023] * 12, 16, 1), (8, 16, [256, 1024] * 12, 16, 0), (8, 16, [1024] * 24, 16, 1), (8, 16, [256, 1024] * 16, 16, 1), (8, 16, [256, 1535] * 6, 16, 1), (8, 16, [256, 1536] * 6, 16, 0),
+    (8, 16, [256, 1024] * 14, 16, 1), (8, 16, [256, 1024] * 14, 24, 0), (8, 16, [256, 1024] * 16, 24, 1)])
+def test_the_rule(kv, heads, lens, bits, eight):
+    check(128, kv, heads, lens, bits, eight)
