@@ -236,7 +236,8 @@ __global__ void __launch_bounds__(256) scan_decode_kernel(ScanArgs a) {
     const int cc = min(c, a.channels - 1);
     const float x = a.x[(size_t)row * a.ldx + cc];
     // the step size: the channel's lanes share out its product with the row's rank_p numbers (a launch of its own was
-    // 4.1 us and a boundary, this is 1.5: 24 rows of 2048 channels, 64 numbers)
+    // 4.1 us and a boundary, this is 1.5: 24 rows of 2048 channels, 64 numbers), or it comes from such a launch (the rule and its
+    // figures: gates_in_scan)
     float dt;
     if (a.gate_w) {
         const int KT = a.rank_p >> 5;

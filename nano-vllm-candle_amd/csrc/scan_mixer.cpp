@@ -166,6 +166,16 @@ int ScanScratch::plan(nvllm_model* m, const int* slot, const int* seq, int R) {
     return NVLLM_OK;
 }
 
+// A decode step's step sizes in the scan itself or by a launch before it.  In the scan every row reads the channels' gate weights again; the launch
+// reads them once for 16 rows or more, but is one, and in 32 bits a slow one, of 64-row blocks from 65 rows on.  A layer's step with
+// the launch less one without, us, at rows x channels x rank of (64 x 4096 x 128 and 16 x 8192 x 256 are the same product: no line has both right)
+//   bf16    64 x 2048 x 64 +2.3, 100 -0.4, 128 +0.1, 200 -3.6; 16 x 4096 x 128 +1.1, 24 -0.1, 64 -3.9, 200 -20.8; 8 x 8192 x 256 +1.0, 16 -4.6, 64 -27.5, 200 -105
+//   32-bit  64 x 2048 x 64 +4.9, 256 +15.4; 48 x 4096 x 128 +2.3, 64 +0.8, 128 +5.6, 200 -2.3; 8 x 8192 x 256 +1.6, 16 -2.6, 64 -26.1, 200 -77
+static bool gates_in_scan(const ScanMixer& w, int R, bool f32) {
+    const int64_t limit = (int64_t)(!f32 ? 12 : R <= 64 ? 28 : 72) << 20;
+    return (int64_t)R * w.n_p * w.rank_p < limit;
+}
+
 int run_scan(nvllm_model* m, ScanMixer& w, ScanScratch& x, const float* in, int n_slabs, float* other_slabs, int R, int qt, float* ctx_f, int ctx_packed) {
     nvllm_ctx* ctx = m->ctx;
     hipStream_t s = ctx->stream;
@@ -192,11 +202,13 @@ int run_scan(nvllm_model* m, ScanMixer& w, ScanScratch& x, const float* in, int 
         rc = comm_allreduce_sum(ctx, x.dbc, (size_t)R * w.Nx);
         if (rc) return rc;
     }
-    if (qt != 1) {
+    const bool in_scan = qt == 1 && gates_in_scan(w, R, f32);
+    if (!in_scan) {
         HeadGemmArgs ga;
         ga.x = dbc; ga.x_row = w.Nx; ga.w = w.dt.data; ga.N = ga.n_valid = w.n_p; ga.K = w.rank_p; ga.M = R; ga.exact = f32;
         ga.y = x.dt; ga.y_row = w.n_p; ga.decay_bias = w.dt_b;
         PROF(m, PROF_GEMM, launch_delta_gates(ga, s));
+        m->scan_gate_launches += qt == 1;
     }
     ScanArgs sa;
     sa.x = x.x; sa.ldx = w.Kc; sa.dt = x.dt; sa.bc = dbc; sa.ldbc = w.Nx; sa.b0 = w.rank_p; sa.c0 = w.rank_p + w.S;
@@ -208,7 +220,7 @@ int run_scan(nvllm_model* m, ScanMixer& w, ScanScratch& x, const float* in, int 
     sa.ld = w.Kc; sa.packed = ctx_packed;
     if (f32) sa.of = ctx_f;
     else { sa.oh = m->ctxh; sa.ol = m->ctxl; }
-    if (qt == 1) { sa.gate_w = w.dt.data; sa.gate_b = w.dt_b; sa.rank_p = w.rank_p; }
+    if (in_scan) { sa.gate_w = w.dt.data; sa.gate_b = w.dt_b; sa.rank_p = w.rank_p; }
     if (qt == 1) PROF(m, PROF_RECUR, launch_scan_decode(sa, R, s));
     else PROF(m, PROF_RECUR, launch_scan_prompt(sa, s));
     return NVLLM_OK;
