@@ -38,6 +38,8 @@ int nvllm_profile_read(nvllm_model* m, double* total_ms, int64_t* launches);
  *   "stream_combine" (default 0): let the fused forward use the streaming GEMM's in-launch split-K combine epilogues (fewer
  *       launches; measured slower on MI355X than slabs + a consumer launch);
  *   "tile_min_wgs" (default 64; 0 never, 1 whenever the shape fits), "tile_fuse_qk" (default 1): the prefill tile GEMM;
+ *   "last_rows" (1, 0 never, default -1: 1 unless "tile_min_wgs" is 1): past the last layer's mixer a prompt chunk goes on with the rows
+ *       whose logits are wanted alone;
  *   "no_fused", "no_xpack", "no_rowpar", "no_attn_prologue" (default 0): force the generic decode path / row-major planes /
  *       no whole-K row-parallel GEMMs / q,k-norm + RoPE + KV write in their own row kernel. */
 int nvllm_debug_set_option(nvllm_model* m, const char* name, int value);

@@ -2123,6 +2123,7 @@ extern "C" int nvllm_debug_set_option(nvllm_model* m, const char* name, int valu
     if (!strcmp(name, "latent_wgs")) { m->opt_latent_wgs = std::max(0, value); return NVLLM_OK; }
     if (!strcmp(name, "latent_plain")) { m->opt_latent_plain = value; return NVLLM_OK; }
     if (!strcmp(name, "tile_fuse_qk")) { m->opt_tile_fuse_qk = value; return NVLLM_OK; }
+    if (!strcmp(name, "last_rows")) { m->opt_last_rows = value; return NVLLM_OK; }
     if (!strcmp(name, "tile_min_wgs")) { m->opt_tile_min_wgs = value; return NVLLM_OK; }  // <= 0: never use the tile GEMM
     if (m->dec && m->dec->option(name, value) == 0) return NVLLM_OK;
     return fail(m->ctx, NVLLM_EINVAL, "unknown option '%s'", name);

@@ -169,6 +169,7 @@ struct nvllm_model {
     int opt_no_fused = 0, opt_no_xpack = 0, opt_no_rowpar = 0;  // A/B switches (nvllm_debug_set_option): force the generic paths
     int opt_no_attn_prologue = 0;  // A/B: decode q/k-norm + RoPE + KV write in their own row kernel, not in the attention prologue
     int opt_tile_fuse_qk = 1;    // QKV tile GEMM with the q/k-norm + RoPE + KV-write epilogue (head_dim 128, 256-wide blocks)
+    int opt_last_rows = -1;      // last_rows_alone
     int opt_latent_absorb = 0;   // prompt chunks of latent attention: 1 always absorbed, -1 expanded whenever possible, 0 by cost
     int opt_latent_wgs = 0;      // decode: workgroups the split of the visible context aims at (0: by latent size)
     int64_t latent_expanded = 0; // layer runs served by the expanded form so far
@@ -263,8 +264,12 @@ enum { PROF_ATTN = 1, PROF_GEMM = 2, PROF_NORM = 3, PROF_QK = 4, PROF_SILU = 5, 
     } while (0)
 
 // Past the last layer's mixer only the rows the head wants go on: the stream of the others is read by nothing.  Taken for prompt chunks
-// (more rows than the products of few rows, whose time is their weights', handle) of which at most half is wanted; layer taps want all rows, and so does the prompt product forced on every projection (tile_min_wgs 1).
-inline bool last_rows_alone(const nvllm_model* m, int R, int n_last) { return R > kRowMaxRows && 2 * n_last <= R && !m->taps && m->opt_tile_min_wgs != 1; }
+// (more rows than the products of few rows, whose time is their weights', handle) of which at most half is wanted; layer taps want all rows.
+// Option "last_rows": 1 by this rule, 0 never, -1 (default) by this rule unless "tile_min_wgs" 1 forces the prompt product on every projection.
+inline bool last_rows_alone(const nvllm_model* m, int R, int n_last) {
+    const bool on = m->opt_last_rows < 0 ? m->opt_tile_min_wgs != 1 : m->opt_last_rows != 0;
+    return on && R > kRowMaxRows && 2 * n_last <= R && !m->taps;
+}
 inline size_t last_rows_cap(const nvllm_model* m) { return std::min((size_t)m->max_seqs, (size_t)m->max_rows / 2 + 1); }
 
 // y (f32 slabs) = x.W^T with the kernel that fits the row count (api.cpp)

@@ -85,3 +85,63 @@ def test_layered(name, dtype):
     for lens, chunk in (([129], 512), ([64, 65], 512), ([300, 17, 45, 1, 133], 256)):
         m = getattr(pkg, design + "ForCausalLM").from_state_dict(c, w, dtype=dtype)
         check(m, lens, chunk, {"bfloat16": 4e-3, "float32": 3e-5}[dtype])  # the tolerances of these decoders' parity tests
+
+
+def forced(make, lens, chunk, bound):
+    """the prompt product on every projection that fits it, of the last layer's gathered rows too"""
+    m = make()
+    m.set_option("tile_min_wgs", 1)
+    m.set_option("last_rows", 1)
+    check(m, lens, chunk, bound)
+    # launches of one prompt by the option: 0 keeps all rows, 1 the wanted ones, -1 all while the product is forced
+    counts = {}
+    for option in (0, 1, -1):
+        m = make()
+        m.set_option("tile_min_wgs", 1)
+        m.set_option("last_rows", option)
+        m.kv_alloc(sum(n // 256 + 1 for n in lens), len(lens), sum(lens))
+        rng = np.random.default_rng(1)
+        m.step(list(range(len(lens))), [rng.integers(0, m.vocab_size, n) for n in lens], True)
+        counts[option] = m.counter("tile_gemm_launches")
+        m.close()
+    return counts
+
+
+# wanted: one row, and 140 rows, which the prompt product takes as well
+@pytest.mark.parametrize("lens,rest", [([700, 33], 1), ([3] * 140, 4)])
+@pytest.mark.parametrize("fuse", [0, 1])
+def test_forced_products(lens, rest, fuse):
+    import nano_vllm_candle_amd as pkg
+
+    cfg = pkg.Qwen3Config.tiny(vocab_size=8192, hidden_size=1024, head_dim=128, num_hidden_layers=2, num_attention_heads=16, num_key_value_heads=8, intermediate_size=3072)
+
+    def make():
+        m = pkg.Qwen3ForCausalLM.from_synthetic(cfg, 3)
+        m.set_option("tile_fuse_qk", fuse)
+        return m
+
+    assert forced(make, lens, 4096, 2.0 ** -11) == {0: 8, 1: 4 + rest, -1: 8}
+
+
+_B, _G, _L = berevik_util, gopunex_util, lefalix_util
+WIDE = {
+    "berevik": ("Berevik", _B.config([_B.layer(heads=16, dim=64, rot=64, vdim=128, rank=256, ff=3072)] * 2, width=1024, vocab=1024), lambda c: _B.sharp_weights(c, 12, gain=1.5)),
+    "gopunex": ("Gopunex", _G.config([_G.light(heads=8, dim=128, vdim=128, ff=3072), _G.attn(heads=8, kv=4, dim=128, vdim=128, ff=3072, far=120)], width=1024, vocab=1024), lambda c: _G.sharp_weights(c, 12, gain=1.5)),
+    "gopunex delta rule": ("Gopunex", _G.config([_G.attn(heads=8, kv=4, dim=128, vdim=128, ff=3072, far=120), _G.delta(heads=8, kv=8, dim=128, vdim=128, ff=3072)], width=1024, vocab=1024), lambda c: _G.sharp_weights(c, 12, gain=1.5)),
+    "tafopel": ("Tafopel", _T.config([_T.attn(heads=8, dim=128, rot=64, vdim=128, rank=512, q_rank=768, mlp=_T.dense(3072)), _T.mamba(inner=2048, state=16, conv=4, rank=64, mlp=_T.dense(3072))], width=1024, vocab=1024), lambda c: _T.weights(c, 12, gain=1.5)),
+    "lefalix": ("Lefalix", _L.config([_L.delta(_L.dense(3072), heads=8, kv=8, dim=128, vdim=128), _L.par(_L.win(heads=8, kv=4, dim=128, vdim=128, window=100, rot=64, scale=0.2), _L.rule(heads=8, kv=4, dim=128, vdim=128), _L.dense(3072))], width=1024, vocab=1024), lambda c: _L.weights(c, 12)),
+}
+
+
+@pytest.mark.parametrize("lens", [[700, 33], [3] * 140])
+@pytest.mark.parametrize("name", sorted(WIDE))
+def test_forced_products_of_layered_decoders(name, lens):
+    import nano_vllm_candle_amd as pkg
+
+    design, cfg, weights = WIDE[name]
+    w = weights(cfg)
+    shapes = ({k: np.shape(v) for k, v in w.items()},) if design in ("Gopunex", "Lefalix") else ()
+    c = getattr(pkg, design + "Config").from_dict(cfg, *shapes)
+    counts = forced(lambda: getattr(pkg, design + "ForCausalLM").from_state_dict(c, w), lens, 4096, 4e-3)
+    assert counts[0] == counts[-1] >= counts[1] > 0
+    assert (counts[1] < counts[0]) == (len(lens) <= 128)  # more rows than that take the product as well
