@@ -48,9 +48,9 @@ int nvllm_debug_set_option(nvllm_model* m, const char* name, int value);
  * "table_copies" = whole block tables sent because a step's pinned block had no room for the new entries;
  * "tile_gemm_launches" = projections run by the prefill tile GEMM; "qk_rows16_launches" = q/k norm, rotation and cache writes by
  * 16 rows and a head per workgroup; "eight_wave_launches" = decode attention on eight waves a workgroup; "scan_gate_launches" = step
- * sizes of a decode step's selective scan by a launch of their own; "kv_f16_saturated" = elements of the K/V pool at the f16 clamp
- * (every cache write saturates at +-65504; a scan of the pool, off the hot path); "kv_f16_absmax_bits" = the largest magnitude the
- * pool holds, as f16 bits */
+ * sizes of a decode step's selective scan by a launch of their own; "two_product_launches" = pairs of products in one launch;
+ * "kv_f16_saturated" = elements of the K/V pool at the f16 clamp (every cache write saturates at +-65504; a scan of the pool, off the
+ * hot path); "kv_f16_absmax_bits" = the largest magnitude the pool holds, as f16 bits */
 int nvllm_debug_get_counter(nvllm_model* m, const char* name, int64_t* value);
 
 /* Diagnostic build only (make -C nano-vllm-candle_amd/csrc stamps -> libnvllm_amd_stamps.so, select it with NVLLM_LIB):

@@ -44,18 +44,16 @@ int run_product(nvllm_model* m, const ProductPlan& p, const bf16_bits* xh, const
 }
 
 int run_two_products(nvllm_model* m, const ProductJob& a, const ProductJob& b, int R) {
-    if (a.p.kind == P_ROW && b.p.kind == P_ROW) {
+    if (a.p.kind == P_ROW && b.p.kind == P_ROW && gemm_rowdir_two_ok(a.w, b.w, R)) {
         auto args = [&](const ProductJob& j) {
             RowParArgs r;
             r.xh = j.xh; r.xl = j.xl; r.ldx = j.w.K; r.out = j.out; r.M = R; r.x_packed = j.p.packed;
             return r;
         };
-        hipError_t e = hipSuccess;
-        PROF(m, PROF_GEMM, (e = launch_gemm_rowdir_two(args(a), a.w, args(b), b.w, m->ctx->stream)) == hipErrorNotReady ? hipSuccess : e);
-        if (e == hipSuccess) {
-            *a.n_slabs = *b.n_slabs = 1;
-            return NVLLM_OK;
-        }
+        PROF(m, PROF_GEMM, launch_gemm_rowdir_two(args(a), a.w, args(b), b.w, m->ctx->stream));
+        ++m->two_launches;
+        *a.n_slabs = *b.n_slabs = 1;
+        return NVLLM_OK;
     }
     int rc = run_product(m, a.p, a.xh, a.xl, a.w, a.out, R, a.n_slabs);
     if (!rc) rc = run_product(m, b.p, b.xh, b.xl, b.w, b.out, R, b.n_slabs);

@@ -352,7 +352,8 @@ struct RowParArgs {
 bool gemm_rowdir_qkv_ok(int N, int K, int hd, int M);
 hipError_t launch_gemm_rowdir_qkv(const RowParArgs& a, const PackedW& w, hipStream_t s);
 bool gemm_rowpar_supported(int N, int K);
-// two plain products (epi 2) of the same rows in one launch; hipErrorNotReady: not their shapes
+// two plain products (epi 2) of the same rows in one launch
+bool gemm_rowdir_two_ok(const PackedW& wa, const PackedW& wb, int M);
 hipError_t launch_gemm_rowdir_two(const RowParArgs& a, const PackedW& wa, const RowParArgs& b, const PackedW& wb, hipStream_t s);
 // true when launch_gemm_rowpar would run the register-direct kernel (the one that accepts packed planes)
 bool gemm_rowdir_ok(int N, int K, int epi, int M);

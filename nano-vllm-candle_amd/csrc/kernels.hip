@@ -1287,7 +1287,9 @@ __global__ void __launch_bounds__(NWK * 64) gemm_rowdir_loop_kernel(RowParArgs a
 
 // Two plain products of the same rows in one launch, where neither needs the other (the projections of a layer's two branches, whose outputs
 // the next norm adds up): workgroups below groups_a make the first.  Each alone is a launch's latency on a quarter of the chip: 24 rows, 1024
-// features of K 2048 and of K 3072, 5.2 and 6.5 us and the boundary between them, together 7.1.
+// features of K 2048 and of K 3072, 5.2 and 6.5 us and the boundary between them, together 7.1.  A step of six layers with each of the nine pairs of
+// K that gemm_rowdir_two_ok takes, 256 to 2048 features, 1 to 64 rows: 2.1 to 7.6 us a layer less, 1024 features 2.4 (K 1024 + 2048, 4
+// rows) to 7.5 (K 3072 + 2048, 64).
 template <int NTA, int TKA, int NTB, int TKB>
 __global__ void __launch_bounds__(1024) gemm_rowdir_two_kernel(RowParArgs a, const uint4* __restrict__ wa, int NA, int groups_a, RowParArgs b, const uint4* __restrict__ wb, int NB) {
     if ((int)blockIdx.x < groups_a) rowdir_body<NTA, 16, TKA, 2, false>(a, wa, NA, 16 * TKA, blockIdx.x);
@@ -1636,19 +1638,24 @@ static hipError_t rowdir_two_launch(const RowParArgs& a, const PackedW& wa, cons
     gemm_rowdir_two_kernel<NTA, TKA, NTB, TKB><<<dim3(ga + gb, 1, (a.M + 15) / 16), 1024, lds, s>>>(a, wa.data, wa.N, ga, b, wb.data, wb.N);
     return hipGetLastError();
 }
-// K of 1024, 2048 or 3072 each, one round of workgroups together (up to 64 rows); hipErrorNotReady: two launches
+// K of 1024, 2048 or 3072 each, one round of workgroups together (up to 64 rows)
+bool gemm_rowdir_two_ok(const PackedW& wa, const PackedW& wb, int M) {
+    if (M > 64 || M < 1) return false;
+    const RowDirShape da = rowdir_shape(wa.N, wa.K, 2, M), db = rowdir_shape(wb.N, wb.K, 2, M);
+    if (!da.nt || !db.nt || da.tk > 6 || db.tk > 6) return false;
+    auto most = [](const RowDirShape& d) { return d.nt == (d.tk == 6 ? 2 : 4); };  // n-tiles of a workgroup
+    if (!(da.nt == db.nt && da.nt <= 2) && !(most(da) && most(db))) return false;
+    return ((wa.N / 16 + da.nt - 1) / da.nt + (wb.N / 16 + db.nt - 1) / db.nt) * ((M + 15) / 16) <= 256;
+}
 hipError_t launch_gemm_rowdir_two(const RowParArgs& a, const PackedW& wa, const RowParArgs& b, const PackedW& wb, hipStream_t s) {
-    if (a.M != b.M || a.M > 64 || a.M < 1) return hipErrorNotReady;
+    if (a.M != b.M || !gemm_rowdir_two_ok(wa, wb, a.M)) return hipErrorNotSupported;
     const RowDirShape da = rowdir_shape(wa.N, wa.K, 2, a.M), db = rowdir_shape(wb.N, wb.K, 2, b.M);
-    if (!da.nt || !db.nt) return hipErrorNotReady;
-    const int blocks = (a.M + 15) / 16, wgs = ((wa.N / 16 + da.nt - 1) / da.nt + (wb.N / 16 + db.nt - 1) / db.nt) * blocks;
-    if (wgs > 256) return hipErrorNotReady;
 #define NVLLM_TWO(NTA_, TKA_, NTB_, TKB_) if (da.nt == NTA_ && da.tk == TKA_ && db.nt == NTB_ && db.tk == TKB_) return rowdir_two_launch<NTA_, TKA_, NTB_, TKB_>(a, wa, b, wb, s);
 #define NVLLM_TWO_N(TKA_, TKB_) NVLLM_TWO(1, TKA_, 1, TKB_) NVLLM_TWO(2, TKA_, 2, TKB_) NVLLM_TWO((TKA_ == 6 ? 2 : 4), TKA_, (TKB_ == 6 ? 2 : 4), TKB_)
     NVLLM_TWO_N(2, 2) NVLLM_TWO_N(2, 4) NVLLM_TWO_N(2, 6) NVLLM_TWO_N(4, 2) NVLLM_TWO_N(4, 4) NVLLM_TWO_N(4, 6) NVLLM_TWO_N(6, 2) NVLLM_TWO_N(6, 4) NVLLM_TWO_N(6, 6)
 #undef NVLLM_TWO_N
 #undef NVLLM_TWO
-    return hipErrorNotReady;
+    return hipErrorNotSupported;
 }
 
 hipError_t launch_gemm_rowpar(const RowParArgs& a, const PackedW& w, int epi, hipStream_t s) {

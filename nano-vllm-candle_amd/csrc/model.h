@@ -223,6 +223,7 @@ struct nvllm_model {
     int64_t qk_rows16_launches = 0;  // likewise: q/k norm, rotation and cache writes by 16 rows and a head
     int64_t eight_wave_launches = 0; // ... decode attention on eight waves
     int64_t scan_gate_launches = 0;  // ... step sizes of a decode step's scan by their own launch
+    int64_t two_launches = 0;        // ... two products in one launch
 
     // per-kernel-class HIP-event timing (bench roofline leg); 0 = off
     int prof_kind = 0;

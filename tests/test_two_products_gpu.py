@@ -22,8 +22,8 @@ def _lefalix():
     return "Lefalix", cfg, w, ({k: np.shape(v) for k, v in w.items()},)
 
 
-@pytest.mark.parametrize("make", [_tafopel, _lefalix])
-def test_steps_equal_the_prompt(make):
+@pytest.mark.parametrize("make,pairs,products", [(_tafopel, 4, 23), (_lefalix, 2, 9)])
+def test_steps_equal_the_prompt(make, pairs, products):
     import nano_vllm_candle_amd as pkg
 
     design, cfg, w, shapes = make()
@@ -36,6 +36,13 @@ def test_steps_equal_the_prompt(make):
         ids = list(range(rows))
         want = m.step_score(ids, seqs[:rows], True, [[len(s) - 1] for s in seqs[:rows]])
         m.step(ids, [s[:-1] for s in seqs[:rows]], True)
+        before = m.counter("two_product_launches")
+        m.profile_kernel("gemm")
         _, got = m.step(ids, seqs[:rows], False, want_logits=True)
+        launches = m.profile_read()[1]
+        m.profile_kernel(None)
+        shared = m.counter("two_product_launches") - before
+        assert shared == (pairs if rows <= 64 else 0), rows
+        assert launches == products - shared, rows  # an event pair to every launch made, none to one that was not
         assert np.abs(got - want).max() < 4e-3 * np.abs(want).max(), rows  # the tolerance of these decoders' parity tests
     m.close()
