@@ -2132,7 +2132,8 @@ extern "C" int nvllm_debug_set_option(nvllm_model* m, const char* name, int valu
 // counters for tests: "oneshot_calls" = all-reduces this model's context has run on the one-shot device path;
 // "tile_gemm_launches" = projections this model has run on the prefill tile GEMM; "table_copies" = whole block tables sent;
 // "qk_rows16_launches" = q/k norm launches of 16 rows and a head per workgroup; "eight_wave_launches" = decode attention on eight waves;
-// "scan_gate_launches" = step sizes of a decode step's selective scan by a launch of their own; "two_product_launches" = pairs of products in one launch
+// "scan_gate_launches" = step sizes of a decode step's selective scan by a launch of their own; "two_product_launches" = pairs of products in one launch;
+// "row_pair_launches" = products of two row blocks at a time, of all models of the process
 extern "C" int nvllm_debug_get_counter(nvllm_model* m, const char* name, int64_t* value) {
     if (!m || !name || !value) return NVLLM_EINVAL;
     if (!strcmp(name, "oneshot_calls")) { *value = (int64_t)m->ctx->os_calls; return NVLLM_OK; }
@@ -2142,6 +2143,7 @@ extern "C" int nvllm_debug_get_counter(nvllm_model* m, const char* name, int64_t
     if (!strcmp(name, "qk_rows16_launches")) { *value = m->qk_rows16_launches; return NVLLM_OK; }
     if (!strcmp(name, "scan_gate_launches")) { *value = m->scan_gate_launches; return NVLLM_OK; }
     if (!strcmp(name, "two_product_launches")) { *value = m->two_launches; return NVLLM_OK; }
+    if (!strcmp(name, "row_pair_launches")) { *value = rowpair_launches(); return NVLLM_OK; }
     if (!strcmp(name, "eight_wave_launches")) { *value = m->eight_wave_launches; return NVLLM_OK; }
     if (!strcmp(name, "kv_f16_saturated") || !strcmp(name, "kv_f16_absmax_bits")) {
         // scan of the whole K/V pool (debug, off the hot path): elements the f16_sat clamp of a cache write produced, and the

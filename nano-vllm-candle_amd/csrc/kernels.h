@@ -352,6 +352,7 @@ struct RowParArgs {
 bool gemm_rowdir_qkv_ok(int N, int K, int hd, int M);
 hipError_t launch_gemm_rowdir_qkv(const RowParArgs& a, const PackedW& w, hipStream_t s);
 bool gemm_rowpar_supported(int N, int K);
+int64_t rowpair_launches();  // of the form that takes two row blocks at a time, by this process so far (tests)
 // two plain products (epi 2) of the same rows in one launch
 bool gemm_rowdir_two_ok(const PackedW& wa, const PackedW& wb, int M);
 hipError_t launch_gemm_rowdir_two(const RowParArgs& a, const PackedW& wa, const RowParArgs& b, const PackedW& wb, hipStream_t s);

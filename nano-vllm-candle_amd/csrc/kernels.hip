@@ -1426,6 +1426,8 @@ __global__ void __launch_bounds__(NWK * 64) gemm_rowpair_kernel(RowParArgs a, co
         if constexpr (EPI == 1) sred += RB * 4 * NR;
     }
 }
+static std::atomic<int64_t> g_rowpair_launches{0};
+int64_t rowpair_launches() { return g_rowpair_launches.load(std::memory_order_relaxed); }
 template <int NT, int NWK, int TK, int RB, int EPI>
 static hipError_t rowpair_launch(const RowParArgs& a, const PackedW& w, hipStream_t s) {
     const int groups = w.N / 16 / NT, blocks = (a.M + 15) / 16;
@@ -1435,13 +1437,23 @@ static hipError_t rowpair_launch(const RowParArgs& a, const PackedW& w, hipStrea
     // one round of the CUs; epilogue 1 holds the norms of blockDim.x / 64 blocks
     const int gz = std::min(blocks, std::max(256 / groups, (blocks + NWK - 1) / NWK));
     gemm_rowpair_kernel<NT, NWK, TK, RB, EPI><<<dim3(groups, 1, gz), NWK * 64, lds, s>>>(a, w.data, w.N, w.K / 32);
+    g_rowpair_launches.fetch_add(1, std::memory_order_relaxed);
     return hipGetLastError();
 }
 // 65 to 256 rows of packed planes whose shape has an instance, else hipErrorNotReady.  Up to 64 rows every workgroup has one block: the
-// 16-wave forms below are as fast or faster there (64 rows, gate/up 8.1 us against 10.6, o 4.8 against 5.6)
+// 16-wave forms below are as fast or faster there (64 rows, gate/up 8.1 us against 10.6, o 4.8 against 5.6).  So they are, for q/k/v and gate/up,
+// while the grid gives every block its own workgroup, whose second block would be nothing, and for 5 blocks on two workgroups.  A product's time by
+// this less the 16-wave form's, us, at 5 to 16 blocks of 1024-wide rows:
+//   q/k/v    1536 features +0.5 to +0.9 up to 10 blocks, -0.3 to -0.7 above; 2048 +0.4 to +0.8 up to 8, -0.3 to -0.9; 2560 +0.9 +0.4 up to 6, -0.9 to
+//            +0.1; 3072 +0.5 at 5, -1.9 to +0.3; 4096 -1.3 to 0.0; 5120 -4.7 to +0.1; 6144 +0.9 at 5, -4.8 to +0.1
+//   gate/up  1536 +0.8 to +1.2, 3072 +0.8 to +1.5 (both up to 8); 4608 +1.4 at 5, -0.8 to -1.1; 6144 -2.5 to -0.4; 9216 +0.9 at 5, -0.6 to -3.9
 template <int EPI>
 static hipError_t rowpair_dispatch(const RowParArgs& a, const PackedW& w, hipStream_t s) {
     if (a.M <= 64 || a.M > 256 || !a.x_packed) return hipErrorNotReady;
+    [[maybe_unused]] auto pairs = [&](int nt) {  // row blocks for two at a time
+        const int blocks = (a.M + 15) / 16, room = 256 / (w.N / 16 / nt);
+        return blocks > room && !(room <= 2 && blocks <= 5);
+    };
     if constexpr (EPI == 0) {  // up to 64 tiles: each leaves its own group of the next norm's sum, as the 16-wave form's workgroups do
         if (w.N % 32 || w.N > 1024) return hipErrorNotReady;
         const bool one = (a.M + 15) / 16 <= 256 / (w.N / 32);  // a block to a workgroup
@@ -1449,9 +1461,9 @@ static hipError_t rowpair_dispatch(const RowParArgs& a, const PackedW& w, hipStr
         if (w.K == 2048) return one ? rowpair_launch<2, 8, 8, 1, 0>(a, w, s) : rowpair_launch<2, 8, 8, 2, 0>(a, w, s);
         if (w.K == 3072) return rowpair_launch<2, 8, 12, 1, 0>(a, w, s);
     } else if constexpr (EPI == 1) {
-        if (w.K == 1024 && w.N % 96 == 0) return rowpair_launch<6, 8, 4, 2, 1>(a, w, s);
+        if (w.K == 1024 && w.N % 96 == 0 && pairs(6)) return rowpair_launch<6, 8, 4, 2, 1>(a, w, s);
     } else if constexpr (EPI == 2) {
-        if (w.K == 1024 && w.N % 64 == 0) return rowpair_launch<4, 8, 4, 2, 2>(a, w, s);
+        if (w.K == 1024 && w.N % 64 == 0 && pairs(4)) return rowpair_launch<4, 8, 4, 2, 2>(a, w, s);
     }
     return hipErrorNotReady;
 }
