@@ -1928,7 +1928,7 @@ static int step_impl(nvllm_model* m, int n_seqs, const int64_t* seq_ids, const u
         r0 += R;
     }
     if (temperatures) {
-        // sample_token on the device (llm_engine.rs:97-133): overwrites the greedy ids the LM head's arg-max left.  Under
+        // sample_token on the device (llm_engine.rs:97-133), from the logits; no arg-max ran.  Under
         // TP every rank draws over its vocabulary shard with the SAME random stream (indexed by global id); the best
         // (score, id) pair wins in finish_logits exactly like the greedy (max, id) pair.
         std::vector<uint64_t> keys(n_seqs);

@@ -135,15 +135,8 @@ __device__ __forceinline__ float wave_sum_uniform(float v) {
            (__builtin_bit_cast(float, __builtin_amdgcn_readlane(x, 32)) + __builtin_bit_cast(float, __builtin_amdgcn_readlane(x, 48)));
 }
 
-// rinv[row] of a deferred RMSNorm (see RowNorm); 1 when the activations were normalised by the producer
-__device__ __forceinline__ float rownorm_rinv(const RowNorm& rn, int row) {
-    if (!rn.ssq) return 1.0f;
-    float t = 0.f;
-    for (int g = 0; g < rn.groups; ++g) t += rn.ssq[(size_t)g * rn.stride + row];
-    return 1.0f / sqrtf(t * rn.inv_h + rn.eps);
-}
-
-// Workgroup-cooperative form for kernels whose epilogue needs rinv of up to NR rows: every thread sums a
+// rinv[row] of a deferred RMSNorm (see RowNorm; 1 when the activations were normalised by the producer), workgroup-cooperative form for
+// kernels whose epilogue needs it of up to NR rows: every thread sums a
 // strided quarter of the groups of one row with independent (unrollable) loads and parks it in LDS;
 // after any later barrier rownorm_rinv_lds() finishes the sum.  groups <= 64.
 template <int NR>
