@@ -54,8 +54,8 @@ def test_infinite_weights(rows):
     assert np.array_equal(got[:, keep], want[:, keep])
 
 
-# K in parts of unlike length (1056, 2080, 4608 in 2, 4, 4), a head walked by workgroups with the rows held (512 workgroups a few tiles each, K of
-# 3 and of 32 k-tiles), both with ragged rows
+# K in parts of unlike length (1056, 2080, 4608 in 2, 4, 4), a head of K 128, by the kernel for short K, and of 1024, walked by workgroups with the rows
+# held (512 workgroups a few tiles each) up to 16 rows; all with ragged rows
 @pytest.mark.parametrize("width,ffs,vocab", [(72, (1056, 2080), 16400), (1000, (4608, 1024), 16390)])
 @pytest.mark.parametrize("rows", [1, 15, 16, 17, 64])
 def test_deep_products_and_many_features(width, ffs, vocab, rows):
@@ -71,6 +71,24 @@ def test_deep_products_and_many_features(width, ffs, vocab, rows):
     assert row_err(got, ref) < TOL["float32"]
     ids, logits = m.step([0], [toks], True, want_logits=True)
     assert ids[0] == np.flatnonzero(logits[0] == logits[0].max())[-1]
+    m.close()
+
+
+# a head walked by workgroups with the rows held (up to 16 rows): 8, 12, 28 and 32 k-tiles over eight waves that hold four each, so all but the last leave
+# places empty, 12 and 28 not in every wave alike; a last tile of 7 features
+@pytest.mark.parametrize("width", [250, 384, 890, 1024])
+@pytest.mark.parametrize("rows", [1, 15, 16, 17])
+def test_head_of_many_features(width, rows):
+    import nano_vllm_candle_amd as pkg
+
+    cfg = config([light(ff=64)], width=width, vocab=16391)
+    w = sharp_weights(cfg)
+    c = pkg.GopunexConfig.from_dict(cfg, {k: np.shape(v) for k, v in w.items()})
+    m = pkg.GopunexForCausalLM.from_state_dict(c, w, dtype="float32")
+    m.kv_alloc(4, 66, max_batched_tokens=256)
+    toks = np.random.default_rng(rows).integers(0, 16391, rows).tolist()
+    got, ref = m.step_score([0], [toks], True, [list(range(rows))]), np.asarray(G.forward(cfg, w, toks))
+    assert row_err(got, ref) < TOL["float32"]
     m.close()
 
 
