@@ -44,14 +44,15 @@ int nvllm_profile_read(nvllm_model* m, double* total_ms, int64_t* launches);
  *       no whole-K row-parallel GEMMs / q,k-norm + RoPE + KV write in their own row kernel. */
 int nvllm_debug_set_option(nvllm_model* m, const char* name, int value);
 
-/* counters for tests: "oneshot_calls" = all-reduces run on the one-shot device path by this model's context;
- * "table_copies" = whole block tables sent because a step's pinned block had no room for the new entries;
- * "tile_gemm_launches" = projections run by the prefill tile GEMM; "qk_rows16_launches" = q/k norm, rotation and cache writes by
- * 16 rows and a head per workgroup; "eight_wave_launches" = decode attention on eight waves a workgroup; "scan_gate_launches" = step
- * sizes of a decode step's selective scan by a launch of their own; "two_product_launches" = pairs of products in one launch;
- * "row_pair_launches" = products of two row blocks at a time, of all models of the process;
- * "kv_f16_saturated" = elements of the K/V pool at the f16 clamp (every cache write saturates at +-65504; a scan of the pool, off the
- * hot path); "kv_f16_absmax_bits" = the largest magnitude the pool holds, as f16 bits */
+/* counters for tests: "oneshot_calls" = all-reduces run on the one-shot device path by this model's context; "table_copies" =
+ * whole block tables sent because a step's pinned block had no room for the new entries; "tile_gemm_launches" = projections
+ * run by the prefill tile GEMM; "qk_rows16_launches" = q/k norm, rotation and cache writes by 16 rows and a head per
+ * workgroup; "eight_wave_launches" = decode attention on eight waves a workgroup; "scan_gate_launches" = step sizes of a
+ * decode step's selective scan by a launch of their own; "two_product_launches" = pairs of products in one launch;
+ * "row_pair_launches" = products of two row blocks at a time, of all models of the process; "tile_resid_launches" = products
+ * of a prompt chunk with residual and norm preparation in their epilogue; "kv_f16_saturated" = elements of the K/V pool at the
+ * f16 clamp (every cache write saturates at +-65504; a scan of the pool, off the hot path); "kv_f16_absmax_bits" = the largest
+ * magnitude the pool holds, as f16 bits */
 int nvllm_debug_get_counter(nvllm_model* m, const char* name, int64_t* value);
 
 /* Diagnostic build only (make -C nano-vllm-candle_amd/csrc stamps -> libnvllm_amd_stamps.so, select it with NVLLM_LIB):

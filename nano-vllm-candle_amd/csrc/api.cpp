@@ -1342,6 +1342,7 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
     const bool fused_norms = qt == 2 && tp == 1 && !m->taps && t_qkv && all.t_o && all.t_gu && all.t_down && tile_resid_wins(R, H, KO, m->I_l);
     RowNorm rn;  // pending on xh / xl
     auto resid_product = [&](const bf16_bits* xh, const bf16_bits* xl, const PackedW& w, const float* next_w) -> hipError_t {
+        ++m->tile_resid_launches;
         rn.ssq = m->ssqT; rn.groups = H / 128; rn.stride = m->max_rows; rn.inv_h = 1.0f / (float)H; rn.eps = eps;
         return launch_tile_resid(xh, xl, w, R, m->resid, next_w, m->xh, m->xl, m->ssqT, m->max_rows, s);
     };
@@ -2133,13 +2134,15 @@ extern "C" int nvllm_debug_set_option(nvllm_model* m, const char* name, int valu
 // "tile_gemm_launches" = projections this model has run on the prefill tile GEMM; "table_copies" = whole block tables sent;
 // "qk_rows16_launches" = q/k norm launches of 16 rows and a head per workgroup; "eight_wave_launches" = decode attention on eight waves;
 // "scan_gate_launches" = step sizes of a decode step's selective scan by a launch of their own; "two_product_launches" = pairs of products in one launch;
-// "row_pair_launches" = products of two row blocks at a time, of all models of the process
+// "row_pair_launches" = products of two row blocks at a time, of all models of the process; "tile_resid_launches" = products of a prompt chunk with
+// residual and norm preparation in their epilogue
 extern "C" int nvllm_debug_get_counter(nvllm_model* m, const char* name, int64_t* value) {
     if (!m || !name || !value) return NVLLM_EINVAL;
     if (!strcmp(name, "oneshot_calls")) { *value = (int64_t)m->ctx->os_calls; return NVLLM_OK; }
     if (!strcmp(name, "latent_expanded")) { *value = m->latent_expanded; return NVLLM_OK; }
     if (!strcmp(name, "table_copies")) { *value = m->table_copies; return NVLLM_OK; }
     if (!strcmp(name, "tile_gemm_launches")) { *value = m->tile_launches; return NVLLM_OK; }
+    if (!strcmp(name, "tile_resid_launches")) { *value = m->tile_resid_launches; return NVLLM_OK; }
     if (!strcmp(name, "qk_rows16_launches")) { *value = m->qk_rows16_launches; return NVLLM_OK; }
     if (!strcmp(name, "scan_gate_launches")) { *value = m->scan_gate_launches; return NVLLM_OK; }
     if (!strcmp(name, "two_product_launches")) { *value = m->two_launches; return NVLLM_OK; }

@@ -224,6 +224,7 @@ struct nvllm_model {
     int64_t eight_wave_launches = 0; // ... decode attention on eight waves
     int64_t scan_gate_launches = 0;  // ... step sizes of a decode step's scan by their own launch
     int64_t two_launches = 0;        // ... two products in one launch
+    int64_t tile_resid_launches = 0; // ... prompt products with residual and norm preparation in their epilogue
 
     // per-kernel-class HIP-event timing (bench roofline leg); 0 = off
     int prof_kind = 0;
