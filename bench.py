@@ -306,6 +306,7 @@ def live_traffic(a, dom_kernel):
     import subprocess
     import tempfile
 
+    names = {dom_kernel.replace("attn_paged_kernel<128, " + u, "attn_paged_kernel<128, " + v) for u, v in ("48", "84")}  # either number of waves
     if not shutil.which("rocprofv3"):
         return None, "rocprofv3 not on PATH"
     if any("rocprof" in os.environ.get(k, "").lower() for k in ("LD_PRELOAD", "ROCP_TOOL_LIBRARIES", "ROCPROFILER_LIBRARY_CTOR")):
@@ -326,7 +327,7 @@ def live_traffic(a, dom_kernel):
         n, tot = 0, 0.0
         with open(files[0]) as f:
             for row in csv.DictReader(f):
-                if row.get("Counter_Name") == "FETCH_SIZE" and dom_kernel in row["Kernel_Name"].replace("nvllm::", ""):
+                if row.get("Counter_Name") == "FETCH_SIZE" and any(k in row["Kernel_Name"].replace("nvllm::", "") for k in names):
                     n += 1
                     tot += float(row["Counter_Value"])
         if n == 0:
@@ -558,7 +559,8 @@ def main():
         dom_bytes = float(np.mean(attn_ctx)) * kv_layer
         _o = dict(o.partition("=")[::2] for o in a.option)  # the cache-width options select the kernel instantiation
         _vlo = 2 if _o.get("kv_k_bits") == "24" else (1 if _o.get("kv_v_bits") == "24" else 0)
-        dom_name = f"attn_paged_kernel<128, 1, 4, true, {_vlo}>"
+        # head size, waves of a workgroup (eight where the batch leaves CUs idle: by context, so both may have run), prologue, residual bytes of the cache
+        dom_name = f"attn_paged_kernel<128, {8 if model.counter('eight_wave_launches') else 4}, true, {_vlo}>"
     elif dom == "lm_head":
         dom_bytes = float(lm_bytes)
         dom_name = "lmhead_kernel"
