@@ -109,6 +109,10 @@ __device__ __forceinline__ uint4 ld_stream16(const void* p) {
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, int bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00027000);
 }
+// Numbers that no launch changes while it runs, read at uniform indices: scalar loads also behind the kernel's own stores and barriers, where hipcc
+// turns a plain read into a vector load and waits for everything in flight with it.
+typedef const __attribute__((address_space(4))) int* uniform_ints_t;
+__device__ __forceinline__ uniform_ints_t uniform_ints(const int* p) { return (uniform_ints_t)(uintptr_t)p; }
 // non-temporal, 16 bytes at lane offset + uniform offset
 __device__ __forceinline__ uint4 buffer_stream16(__amdgpu_buffer_rsrc_t r, int offset, int uniform_offset) {
     return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, offset, uniform_offset, 2));

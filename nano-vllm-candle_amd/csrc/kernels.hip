@@ -2206,7 +2206,8 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
     const int t_end = a.part_tiles ? min(n_kv_tiles, t_begin + a.part_tiles) : n_kv_tiles;
     if (t_begin >= n_kv_tiles) return;  // uniform for the whole workgroup
 
-    const int* bt = a.block_tables + (size_t)slot * a.max_blocks;
+    // (plain reads became vector loads behind the prologue's barrier, each with a wait that drained the tiles in flight)
+    const uniform_ints_t bt = uniform_ints(a.block_tables + (size_t)slot * a.max_blocks);
     // one 32-token KV tile: 2*DC K fragments (the two 16-token tiles are contiguous) + DT V fragments, 16 KiB in 1 KiB wave-loads.  A tile
     // past the end (kt >= t_end: a wave leaves its loop with up to two such prefetches) is the same instructions over buffers of no bytes:
     // they return zeros and cost no access.  A branch around the loads instead makes hipcc wait for vmcnt(0) per load.

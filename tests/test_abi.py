@@ -184,3 +184,30 @@ def test_later_kernels_keep_their_register_budget():
         assert len(hits) == count, (part, len(hits))
         for n, r in hits.items():
             assert r["ScratchSize [bytes/lane]"] == 0 and r["Occupancy [waves/SIMD]"] >= 2, (n, r)
+
+
+def test_decode_attention_reads_its_block_table_by_scalar_loads(tmp_path):
+    # A vector load of a block number in the tile loop waits for every tile that is in flight before it.  The code objects of this library, as
+    # hipcc made them here.
+    import shutil
+    import subprocess
+
+    from nano_vllm_candle_amd._lib import LIB_PATH
+
+    objdump = "/opt/rocm/llvm/bin/llvm-objdump"
+    if not os.path.exists(objdump):
+        pytest.skip("no llvm-objdump")
+    so = shutil.copy(LIB_PATH, tmp_path / "lib.so")
+    subprocess.run([objdump, "--offloading", str(so)], cwd=tmp_path, check=True, capture_output=True)
+    loops = 0
+    for obj in sorted(tmp_path.glob("lib.so.*gfx950")):
+        names = [l.split()[-1] for l in subprocess.run([objdump, "--syms", str(obj)], check=True, capture_output=True, text=True).stdout.splitlines() if "attn_paged_kernel" in l and " F " in l]
+        for name in names:
+            asm = subprocess.run([objdump, "-d", f"--disassemble-symbols={name}", str(obj)], check=True, capture_output=True, text=True).stdout.splitlines()
+            ops = [l.split()[0] for l in asm if l.startswith("\t")]
+            mfma = [i for i, o in enumerate(ops) if "mfma" in o]
+            loop = ops[mfma[0]:mfma[-1]]
+            assert any(o.startswith("buffer_load") for o in loop) and any(o.startswith("s_load") for o in loop), name
+            assert not [o for o in loop if o.startswith(("global_load", "flat_load"))], name
+            loops += 1
+    assert loops == 11  # head sizes, waves, prologue, forms of the cache
