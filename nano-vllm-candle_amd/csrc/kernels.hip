@@ -2130,8 +2130,10 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
     // residual bytes of both
     float* ml = reinterpret_cast<float*>(smem_raw);
     const int cols = FUSED ? a.gqa : 16;  // MFMA columns that are rows of q
+    // rows of O and of q are 16 bytes longer than their elements: a wave's lanes are columns of one dim, which would all be on the same banks
+    constexpr int OS = HD / 4 + 1, QS = HD + 8;
     f32x4* obuf = reinterpret_cast<f32x4*>(smem_raw + NWV * 2 * 16 * 4);
-    [[maybe_unused]] const int q_at = NWV * (2 * 16 * 4 + cols * HD * 4), new_at = q_at + cols * HD * 4;  // bytes
+    [[maybe_unused]] const int q_at = NWV * (2 * 16 * 4 + cols * OS * 16), new_at = q_at + cols * QS * 4;  // bytes
     // (offsets, not pointers to choose between: the compiler must see that every access is to LDS, a generic one would wait for the tiles)
     [[maybe_unused]] auto lds16 = [&](int byte) { return reinterpret_cast<_Float16*>(smem_raw + byte); };
     [[maybe_unused]] auto lds8 = [&](int byte) { return reinterpret_cast<uint8_t*>(smem_raw + byte); };
@@ -2300,9 +2302,9 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
                 for (int e = 0; e < 4; ++e) {
                     const float v = z[e] * a.q_scale;
                     const _Float16 h = (_Float16)v;
-                    const int to = q_at + (item * HD + (e >> 1) * half + hd2 + (e & 1)) * 2;
+                    const int to = q_at + (item * QS + (e >> 1) * half + hd2 + (e & 1)) * 2;
                     *lds16(to) = h;
-                    *lds16(to + cols * HD * 2) = (_Float16)(v - (float)h);
+                    *lds16(to + cols * QS * 2) = (_Float16)(v - (float)h);
                 }
             } else if (has_new && item < items) {
                 const size_t vo = (size_t)(bt[pos >> 8] * kv_l + kh) * kBlockTokens * HD;
@@ -2339,11 +2341,11 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
         // q and the new token are published; the tiles stay in flight
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         if (has_new && (last - t_begin) % NWV == wave) new_tile = last;
-        const int at = q_at + ((l15 % gqa) * HD + grp * 8) * 2;  // columns of no row repeat one: nothing of theirs is stored
+        const int at = q_at + ((l15 % gqa) * QS + grp * 8) * 2;  // columns of no row repeat one: nothing of theirs is stored
 #pragma unroll
         for (int c = 0; c < DC; ++c) {
             qh[c] = *reinterpret_cast<const f16x8*>(smem_raw + at + c * 64);
-            ql[c] = *reinterpret_cast<const f16x8*>(smem_raw + at + cols * HD * 2 + c * 64);
+            ql[c] = *reinterpret_cast<const f16x8*>(smem_raw + at + cols * QS * 2 + c * 64);
         }
         NVLLM_STAMP(a, 2);
     } else {
@@ -2540,7 +2542,7 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
             ml[(wave * 2 + 1) * 16 + l15] = lsum;
         }
 #pragma unroll
-        for (int d = 0; d < DT; ++d) obuf[(wave * cols + l15) * (HD / 4) + d * 4 + grp] = o[d];
+        for (int d = 0; d < DT; ++d) obuf[(wave * cols + l15) * OS + d * 4 + grp] = o[d];
     }
     __syncthreads();
     const int n_parts = a.part_tiles ? (n_kv_tiles + a.part_tiles - 1) / a.part_tiles : 1;
@@ -2556,7 +2558,7 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
 #pragma unroll
         for (int w = 0; w < NWV; ++w) {
             const float f = exp2f(ml[(w * 2 + 0) * 16 + col] - ms);
-            const f32x4 v = obuf[(w * cols + col) * (HD / 4) + d4];
+            const f32x4 v = obuf[(w * cols + col) * OS + d4];
             ltot += ml[(w * 2 + 1) * 16 + col] * f;
             acc[0] += v[0] * f; acc[1] += v[1] * f; acc[2] += v[2] * f; acc[3] += v[3] * f;
         }
@@ -2977,7 +2979,7 @@ __global__ void __launch_bounds__(256) attn_combine_kernel(AttnArgs a, int rows)
 
 template <int HD, int NWV, bool FUSED, int VLO>
 static hipError_t attn_launch_v(const AttnArgs& a, int n_tiles, int grid_z, hipStream_t s) {
-    auto lds_of = [](int gqa) { return NWV * 2 * 16 * 4 + (size_t)NWV * gqa * HD * 4 + (FUSED ? (size_t)gqa * HD * 4 + HD * 6 : 0); };
+    auto lds_of = [](int gqa) { return NWV * 2 * 16 * 4 + (size_t)NWV * gqa * (HD * 4 + 16) + (FUSED ? (size_t)gqa * (HD + 8) * 4 + HD * 6 : 0); };
     const size_t lds = lds_of(FUSED ? a.gqa : 16);
     static std::atomic<uint64_t> lds_set{0};
     ensure_dyn_lds(reinterpret_cast<const void*>(attn_paged_kernel<HD, NWV, FUSED, VLO>), lds_of(16), lds_set);

@@ -34,9 +34,10 @@ def check(hd, kv, heads, lens, bits, eight):
 
 
 # workgroups: 256 and 264 of 8 kv heads; 128 and 124 of 4 (whole and in parts from 513 tokens on); 2 and 257 of one, whose 18 heads take
-# more rounds of four waves than are loaded up front; 8 heads of 64
+# more rounds of four waves than are loaded up front; 8 heads of 64; 3 to 14 query heads a group, whose rows lie beside each other in LDS
 @pytest.mark.parametrize("hd,kv,heads,rows,bits,eight", [(128, 8, 16, 32, 16, 1), (128, 8, 16, 33, 16, 0), (128, 4, 8, 32, 16, 1), (128, 4, 8, 31, 24, 1), (128, 1, 16, 2, 16, 0),
-                                                         (128, 1, 16, 257, 16, 0), (128, 1, 8, 17, 24, 1), (64, 1, 8, 17, 16, 0), (64, 1, 16, 3, 16, 0)])
+                                                         (128, 1, 16, 257, 16, 0), (128, 1, 8, 17, 24, 1), (64, 1, 8, 17, 16, 0), (64, 1, 16, 3, 16, 0),
+                                                         (128, 2, 6, 3, 16, 0), (128, 8, 40, 33, 16, 0), (128, 1, 7, 5, 24, 0), (128, 2, 28, 129, 24, 0), (64, 2, 10, 9, 16, 0)])
 def test_a_step_equals_the_prompt(hd, kv, heads, rows, bits, eight):
     check(hd, kv, heads, [LENGTHS[(i * 7) % len(LENGTHS)] for i in range(rows)], bits, eight)
 
