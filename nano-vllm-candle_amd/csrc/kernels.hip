@@ -2282,12 +2282,12 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
         // pass first: the tile is patched before it is used.
         load_tile(t_begin + wave, kaA, kbA, vfA, vlA);
         if constexpr (!ONE_SET) load_tile(t_begin + wave + NWV, kaB, kbB, vfB, vlB);
+        const float ri = a.rn.ssq ? 1.0f / sqrtf(wave_sum_uniform(ssq_g) * a.rn.inv_h + a.rn.eps) : 1.0f;
         auto make = [&](int item, float2 u, float2 w, float2 nu, float2 nw) __attribute__((always_inline)) {
-            const float ri = a.rn.ssq ? 1.0f / sqrtf(wave_sum(ssq_g) * a.rn.inv_h + a.rn.eps) : 1.0f;
             u.x *= ri; u.y *= ri; w.x *= ri; w.y *= ri;
             float ss = u.x * u.x + u.y * u.y + w.x * w.x + w.y * w.y;
-#pragma unroll
-            for (int d = 1; d < LPH; d *= 2) ss += __shfl_xor(ss, d);
+            ss = row16_sum(ss);
+            if constexpr (LPH == 32) ss += __shfl_xor(ss, 16);
             const float rinv = 1.0f / sqrtf(ss / (float)HD + a.eps);
             const float y[4] = {u.x, u.y, w.x, w.y}, g[4] = {nu.x, nu.y, nw.x, nw.y}, c[2] = {cs.x, cs.y}, s_[2] = {sn.x, sn.y};
             float z[4];  // dims hd2, hd2 + 1, half + hd2, half + hd2 + 1
