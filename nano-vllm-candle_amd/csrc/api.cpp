@@ -1526,33 +1526,33 @@ static int ensure_blocks(nvllm_model* m, SeqState& s, int len) {
     return NVLLM_OK;
 }
 
-// Eight waves of a decode attention's workgroup instead of four halve its chain of tiles, but the merge and the two waves of a SIMD cost up to 1 us:
+// Eight waves of a decode attention's workgroup instead of four halve its chain of tiles, but the merge and the two waves of a SIMD cost up to 1.5 us:
 // only where launches leave a CU one workgroup at most, and not
-//  - in a 16-bit cache on whole contexts (up to 16 tiles) of many workgroups or query heads, nor on 5 to 8 tiles;
+//  - in a 16-bit cache on whole contexts (up to 16 tiles), where four waves have all of them in flight at once (with more than 14 query heads a
+//    group, four waves have a third round of prologue loads, behind the tiles');
 //  - while parts of four waves, a tile each, have a CU to themselves and are so few that the combine pass is no longer for them;
-//  - where parts that fit the CUs leave a quarter of them idle and the longest of ragged contexts is what the launch waits for.
+//  - in a 24-bit cache, where parts that fit the CUs leave a quarter of them idle and the longest of ragged contexts is what the launch waits for.
 // Attention and its combine pass, us a layer between two events (5 of them the events'), four waves / eight; rows x tokens, 8 kv heads:
-//   gqa 2   whole 16 x 400 15.4 / 14.8, 20 x 500 17.4 / 16.8, 24 x 500 17.9 / 18.3, 32 x 400 18.3 / 19.3; 8 x 129 11.2 / 11.3
-//   gqa 4   whole 8 x 400 14.6 / 14.4, 16 x 400 15.4 / 15.7, 24 x 400 18.3 / 19.5, 32 x 280 17.4 / 18.6; 8 x 129 11.4 / 11.9
-//   gqa 1   whole 20 x 400 15.9 / 15.5, 24 x 511 18.1 / 18.8, 32 x 511 20.0 / 21.9
-//   gqa 2   parts 1 x 600 14.1 / 14.9, 1 x 1100 15.7 / 15.8, 1 x 1500 17.1 / 16.2, 4 x 600 14.8 / 15.4, 4 x 1100 19.4 / 16.9, 6 x 600 15.8 / 15.9, 6 x 700 18.1 / 16.1, 8 x 600 18.1 / 16.5
-//   gqa 4   parts 1 x 600 15.0 / 15.9, 1 x 1100 16.4 / 16.8, 1 x 2000 19.4 / 18.1, 4 x 700 16.1 / 16.4
-//   gqa 2   of 256 to 2048, 12 rows 25.1 / 25.2, 16 28.3 / 27.4, 20 31.9 / 33.6, 24 32.7 / 34.6, 28 36.8 / 36.1, 32 40.8 / 37.9; gqa 4, 24 rows 34.2 / 35.9
-//   gqa 2   of 64 to 512, 24 rows 18.7 / 16.8; 24 x 2000 43.9 / 39.5
-//   24 bits whole 8 x 400 20.7 / 17.1, 24 x 400 22.7 / 20.8, 32 x 400 24.3 / 23.6; 1 x 600 15.3 / 16.3; of 600 to 3000, 24 rows 59.5 / 65.1, 28 67.0 / 70.9, 32 75.3 / 74.3
+//   gqa 2   whole 1 x 400 13.0 / 13.2, 8 x 400 13.5 / 14.0, 20 x 400 15.3 / 15.9, 32 x 400 17.5 / 19.3, 8 x 150..180 11.0 / 11.8
+//   gqa 4   whole 8 x 400 13.7 / 14.3, 32 x 400 17.5 / 19.4
+//   gqa 2   parts 1 x 900 14.5 / 14.9, 1 x 1500 15.8 / 15.5, 3 x 700 14.7 / 15.3, 4 x 900 16.5 / 16.5, 6 x 600 15.4 / 16.1, 6 x 700 17.8 / 16.1, 8 x 700 18.0 / 17.0, 32 x 1100 33.9 / 30.1
+//   gqa 2   of 6 x 64..512 14.4 / 15.6, 20 x 64..512 18.8 / 16.1, 12 x 256..2048 24.9 / 24.4, 20 x 256..2048 31.6 / 30.8, 24 x 256..2048 32.6 / 32.8, 32 x 256..2048 40.3 / 36.6
+//   24 bits whole 1 x 150..180 13.0 / 12.1, 1 x 400 16.7 / 16.1, 20 x 400 19.7 / 19.9, 32 x 150..180 16.0 / 16.0, 32 x 400 23.5 / 23.7, 8 x 100 11.5 / 12.5
+//   24 bits of 12 x 600..3000 38.4 / 39.4, 20 x 600..3000 55.0 / 58.3, 24 x 600..3000 60.6 / 63.7, 24 x 600..1500 40.4 / 39.2, 28 x 600..3000 70.4 / 69.0
+//   16 heads on one: whole 16 x 257 13.4 / 13.0, 32 x 400 14.7 / 14.3, 128 x 257 14.9 / 15.1, 192 x 257 16.4 / 16.8
 static bool eight_waves_win(const nvllm_model* m, int wgs, int tiles, bool ragged) {
-    if (m->hd != 128 || wgs > 256 || tiles <= (wgs < 64 ? 8 : 4)) return false;
+    if (m->hd != 128 || wgs > 256 || tiles <= 4) return false;
     const bool wide = !m->vlocache.empty();
-    if (tiles <= 16) return wide || wgs < 64 || (tiles > 8 && wgs <= 160 && wgs * m->gqa <= 320);
-    if (tiles <= std::min(wgs <= 16 ? 40 : 32, 1024 / wgs)) return false;
-    return !ragged || 256 / wgs * wgs > (wide ? 224 : 192) || tiles <= (wgs < 128 ? 48 : 32);
+    if (tiles <= 16) return wide ? tiles <= 8 || wgs <= 160 : m->gqa > 14 && wgs <= 128;
+    if (tiles <= std::min(wgs <= 16 ? 40 : 28, 1024 / wgs)) return false;
+    return !(wide && ragged) || 256 / wgs * wgs > 192 || tiles <= (wgs < 128 ? 48 : 32);
 }
 // Split a sequence's context over several workgroups only when (sequences x kv heads) alone cannot fill
 // the chip (small batches, long contexts); a full batch already has >= 2 workgroups per CU.
 static void set_attn_split(nvllm_model* m, int n_seqs, int max_len, int64_t all_len) {
     const int tiles = (max_len + 31) / 32;
     const int base_wgs = std::max(1, n_seqs * m->kv_l);
-    const bool eight = eight_waves_win(m, base_wgs, tiles, 4 * all_len < 3 * (int64_t)n_seqs * max_len);
+    const bool eight = eight_waves_win(m, base_wgs, tiles, 3 * all_len < 2 * (int64_t)n_seqs * max_len);
     m->attn_waves = eight ? 8 : 4;
     int want = std::min(kAttnMaxParts, std::max(1, (eight ? 256 : 512) / base_wgs));
     // a few more rounds of the loop cost less than the combine launch and its boundary (4.7 + 1.4 us): up to 512 tokens, and up to 1024 where

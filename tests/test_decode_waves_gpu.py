@@ -35,19 +35,21 @@ def check(hd, kv, heads, lens, bits, eight):
 
 # workgroups: 256 and 264 of 8 kv heads; 128 and 124 of 4 (whole and in parts from 513 tokens on); 2 and 257 of one, whose 18 heads take
 # more rounds of four waves than are loaded up front; 8 heads of 64; 3 to 14 query heads a group, whose rows lie beside each other in LDS
-@pytest.mark.parametrize("hd,kv,heads,rows,bits,eight", [(128, 8, 16, 32, 16, 1), (128, 8, 16, 33, 16, 0), (128, 4, 8, 32, 16, 1), (128, 4, 8, 31, 24, 1), (128, 1, 16, 2, 16, 0),
+@pytest.mark.parametrize("hd,kv,heads,rows,bits,eight", [(128, 8, 16, 32, 16, 1), (128, 8, 16, 33, 16, 0), (128, 4, 8, 32, 16, 1), (128, 4, 8, 31, 24, 1), (128, 1, 16, 2, 16, 1),
                                                          (128, 1, 16, 257, 16, 0), (128, 1, 8, 17, 24, 1), (64, 1, 8, 17, 16, 0), (64, 1, 16, 3, 16, 0),
                                                          (128, 2, 6, 3, 16, 0), (128, 8, 40, 33, 16, 0), (128, 1, 7, 5, 24, 0), (128, 2, 28, 129, 24, 0), (64, 2, 10, 9, 16, 0)])
 def test_a_step_equals_the_prompt(hd, kv, heads, rows, bits, eight):
     check(hd, kv, heads, [LENGTHS[(i * 7) % len(LENGTHS)] for i in range(rows)], bits, eight)
 
 
-# both sides of each line of the rule: whole contexts by workgroups and query heads, parts of a tile a wave, ragged contexts whose parts leave CUs idle
+# both sides of each line of the rule: whole contexts by workgroups, cache and query heads, parts of a tile a wave, ragged contexts whose parts leave CUs idle
 @pytest.mark.parametrize("kv,heads,lens,bits,eight", [
-    (8, 16, [255], 16, 0), (8, 16, [256], 16, 1), (8, 16, [255] * 8, 16, 0), (8, 16, [256] * 8, 16, 1), (8, 16, [130] * 8, 24, 1), (8, 16, [300] * 20, 16, 1), (8, 16, [300] * 21, 16, 0), (8, 16, [300] * 21, 24, 1),
-    (8, 32, [300] * 10, 16, 1), (8, 32, [300] * 11, 16, 0), (4, 4, [300] * 40, 16, 1), (4, 4, [300] * 41, 16, 0),
-    (8, 16, [511], 16, 1), (8, 16, [512], 16, 0), (8, 16, [1279], 16, 0), (8, 16, [1280], 16, 1), (8, 16, [1023] * 3, 16, 0), (8, 16, [1024] * 3, 16, 1), (8, 16, [671] * 6, 16, 0), (8, 16, [672] * 6, 16, 1), (8, 16, [512] * 8, 16, 1), (8, 16, [1279], 24, 0), (8, 16, [1280], 24, 1),
-    (8, 16, [256, 1023] * 12, 16, 1), (8, 16, [256, 1024] * 12, 16, 0), (8, 16, [1024] * 24, 16, 1), (8, 16, [256, 1024] * 16, 16, 1), (8, 16, [256, 1535] * 6, 16, 1), (8, 16, [256, 1536] * 6, 16, 0),
-    (8, 16, [256, 1024] * 14, 16, 1), (8, 16, [256, 1024] * 14, 24, 0), (8, 16, [256, 1024] * 16, 24, 1)])
+    (8, 16, [256], 16, 0), (8, 16, [300] * 20, 16, 0), (8, 16, [511], 16, 0), (8, 32, [300] * 10, 16, 0), (1, 14, [300], 16, 0),
+    (1, 15, [127], 16, 0), (1, 15, [128], 16, 1), (1, 16, [300] * 128, 16, 1), (1, 16, [300] * 129, 16, 0),
+    (8, 16, [127], 24, 0), (8, 16, [128], 24, 1), (8, 16, [255] * 32, 24, 1), (8, 16, [256] * 32, 24, 0), (8, 16, [300] * 20, 24, 1), (8, 16, [300] * 21, 24, 0),
+    (8, 16, [512], 16, 0), (8, 16, [1279], 16, 0), (8, 16, [1280], 16, 1), (8, 16, [1279], 24, 0), (8, 16, [1280], 24, 1),
+    (8, 16, [895] * 3, 16, 0), (8, 16, [896] * 3, 16, 1), (8, 16, [671] * 6, 16, 0), (8, 16, [672] * 6, 16, 1), (8, 16, [512] * 8, 16, 1),
+    (8, 16, [256, 1024] * 12, 16, 1), (8, 16, [256, 1023] * 12, 24, 1), (8, 16, [256, 1024] * 12, 24, 0), (8, 16, [512, 1024] * 12, 24, 1), (8, 16, [1024] * 24, 24, 1),
+    (8, 16, [256, 1024] * 14, 24, 1), (8, 16, [256, 1535] * 6, 24, 1), (8, 16, [256, 1536] * 6, 24, 0)])
 def test_the_rule(kv, heads, lens, bits, eight):
     check(128, kv, heads, lens, bits, eight)
