@@ -33,6 +33,8 @@ int bias_attn_vdim(int vdim) {
 //                     1 x 260   2 x 260   8 x 65   16 x 92   1 x 1024   1 x 2000
 //   four waves a row     37        64       48       127        320       1138
 //   a wave a row         42        62       31        82        330       1091
+// Values of up to 64 elements are asked for in two halves: 94 registers instead of 118 are a fifth workgroup on a CU, 64 heads of 64 a prompt of 64
+// 19.4 -> 18.7, 32 and 64 decode rows of 100 tokens on average 15.6 -> 15.1 and 24.5 -> 23.8 (with eight elements at a time 18.7, 15.3 and 23.8).
 // ---------------------------------------------------------------------------------------------------
 template <typename T>
 __device__ __forceinline__ void load8(float (&x)[8], const T* p) {
@@ -48,6 +50,7 @@ __device__ __forceinline__ void load8(float (&x)[8], const T* p) {
 template <typename T, int NE, int ROWS>
 __global__ void __launch_bounds__(256) bias_attn_plain_kernel(BiasAttnArgs a, int rows) {
     constexpr int WPR = 4 / ROWS;  // waves of a row
+    constexpr int VB = NE == 1 ? 4 : 8;  // 8-token value loads asked for at once
     extern __shared__ float sh[];
     __shared__ float pw[4][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -95,13 +98,16 @@ __global__ void __launch_bounds__(256) bias_attn_plain_kernel(BiasAttnArgs a, in
             const int d = lane + e * 64;
             if (d >= c.vdim_p) continue;
             float t = o[e] * al;
-            float v[8][8];
+#pragma unroll 1
+            for (int g0 = 0; g0 < 8; g0 += VB) {
+                float v[VB][8];
 #pragma unroll
-            for (int g = 0; g < 8; ++g) load8(v[g], vp + v_packed_offset((j0 & (kBlockTokens - 1)) + (g >> 2) * 32 + (g & 3) * 4, d, c.vdim_p));
+                for (int g = 0; g < VB; ++g) load8(v[g], vp + v_packed_offset((j0 & (kBlockTokens - 1)) + ((g0 + g) >> 2) * 32 + ((g0 + g) & 3) * 4, d, c.vdim_p));
 #pragma unroll
-            for (int g = 0; g < 8; ++g)
+                for (int g = 0; g < VB; ++g)
 #pragma unroll
-                for (int i = 0; i < 8; ++i) t += pw[wave][(g >> 2) * 32 + (i >> 2) * 16 + (g & 3) * 4 + (i & 3)] * v[g][i];
+                    for (int i = 0; i < 8; ++i) t += pw[wave][((g0 + g) >> 2) * 32 + (i >> 2) * 16 + ((g0 + g) & 3) * 4 + (i & 3)] * v[g][i];
+            }
             o[e] = t;
         }
         __builtin_amdgcn_wave_barrier();
