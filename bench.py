@@ -307,6 +307,7 @@ def live_traffic(a, dom_kernel):
     import tempfile
 
     names = {dom_kernel.replace("attn_paged_kernel<128, " + u, "attn_paged_kernel<128, " + v) for u, v in ("48", "84")}  # either number of waves
+    names |= {n.replace("attn_paged_kernel<128, 4, true, 0>", "attn_paged_ahead_kernel<128, 4>") for n in names}  # the form of many long contexts
     if not shutil.which("rocprofv3"):
         return None, "rocprofv3 not on PATH"
     if any("rocprof" in os.environ.get(k, "").lower() for k in ("LD_PRELOAD", "ROCP_TOOL_LIBRARIES", "ROCPROFILER_LIBRARY_CTOR")):

@@ -1203,8 +1203,9 @@ static int forward_chunk_fused(nvllm_model* m, const FusedPlan& fp, int R, int n
         if (qt == 1 && R <= m->max_seqs) {
             aa.part_tiles = m->attn_part_tiles; aa.max_parts = kAttnMaxParts; aa.part_o = m->attn_po; aa.part_ml = m->attn_pml;
             parts_max = m->attn_parts_max;
-            if (fuse_qk) aa.waves = m->attn_waves;
+            if (fuse_qk) { aa.waves = m->attn_waves; aa.ahead = m->attn_ahead; }
             m->eight_wave_launches += aa.waves == 8;
+            m->tiles_ahead_launches += aa.ahead;
         }
         PROF(m, PROF_EMPTY, hipSuccess);  // calibration: an event pair around nothing, at the attention launch's place
         STAMPS(aa, m);
@@ -1403,8 +1404,9 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
         if (qt == 1 && R <= m->max_seqs) {  // decode rows: split the context over workgroups
             aa.part_tiles = m->attn_part_tiles; aa.max_parts = kAttnMaxParts; aa.part_o = m->attn_po; aa.part_ml = m->attn_pml;
             parts_max = m->attn_parts_max;
-            if (fuse_qk) aa.waves = m->attn_waves;
+            if (fuse_qk) { aa.waves = m->attn_waves; aa.ahead = m->attn_ahead; }
             m->eight_wave_launches += aa.waves == 8;
+            m->tiles_ahead_launches += aa.ahead;
         }
         STAMPS(aa, m);
         int attn_tiles = n_tiles;
@@ -1533,19 +1535,30 @@ static int ensure_blocks(nvllm_model* m, SeqState& s, int len) {
 //  - while parts of four waves, a tile each, have a CU to themselves and are so few that the combine pass is no longer for them;
 //  - in a 24-bit cache, where parts that fit the CUs leave a quarter of them idle and the longest of ragged contexts is what the launch waits for.
 // Attention and its combine pass, us a layer between two events (5 of them the events'), four waves / eight; rows x tokens, 8 kv heads:
-//   gqa 2   whole 1 x 400 13.0 / 13.2, 8 x 400 13.5 / 14.0, 20 x 400 15.3 / 15.9, 32 x 400 17.5 / 19.3, 8 x 150..180 11.0 / 11.8
-//   gqa 4   whole 8 x 400 13.7 / 14.3, 32 x 400 17.5 / 19.4
-//   gqa 2   parts 1 x 900 14.5 / 14.9, 1 x 1500 15.8 / 15.5, 3 x 700 14.7 / 15.3, 4 x 900 16.5 / 16.5, 6 x 600 15.4 / 16.1, 6 x 700 17.8 / 16.1, 8 x 700 18.0 / 17.0, 32 x 1100 33.9 / 30.1
-//   gqa 2   of 6 x 64..512 14.4 / 15.6, 20 x 64..512 18.8 / 16.1, 12 x 256..2048 24.9 / 24.4, 20 x 256..2048 31.6 / 30.8, 24 x 256..2048 32.6 / 32.8, 32 x 256..2048 40.3 / 36.6
-//   24 bits whole 1 x 150..180 13.0 / 12.1, 1 x 400 16.7 / 16.1, 20 x 400 19.7 / 19.9, 32 x 150..180 16.0 / 16.0, 32 x 400 23.5 / 23.7, 8 x 100 11.5 / 12.5
-//   24 bits of 12 x 600..3000 38.4 / 39.4, 20 x 600..3000 55.0 / 58.3, 24 x 600..3000 60.6 / 63.7, 24 x 600..1500 40.4 / 39.2, 28 x 600..3000 70.4 / 69.0
-//   16 heads on one: whole 16 x 257 13.4 / 13.0, 32 x 400 14.7 / 14.3, 128 x 257 14.9 / 15.1, 192 x 257 16.4 / 16.8
+//   gqa 2   whole 1 x 400 12.3 / 13.0, 8 x 400 13.0 / 13.8, 20 x 400 14.9 / 16.1, 32 x 400 17.2 / 19.6, 8 x 150..180 10.5 / 11.3
+//   gqa 4   whole 8 x 400 12.9 / 13.9, 32 x 400 16.9 / 18.9
+//   gqa 2   parts 1 x 900 13.5 / 14.6, 1 x 1500 15.7 / 15.4, 3 x 700 14.1 / 14.8, 4 x 900 16.1 / 16.0, 6 x 600 14.8 / 15.6, 6 x 700 17.3 / 15.7, 8 x 700 17.7 / 16.6, 32 x 1100 33.6 / 30.1
+//   gqa 2   of 6 x 64..512 14.0 / 15.3, 20 x 64..512 18.2 / 16.0, 12 x 256..2048 24.3 / 24.2, 20 x 256..2048 31.5 / 30.6, 24 x 256..2048 32.5 / 32.6, 32 x 256..2048 40.1 / 36.3
+//   24 bits whole 1 x 150..180 13.1 / 12.3, 1 x 400 16.6 / 16.1, 20 x 400 19.8 / 19.6, 32 x 150..180 16.1 / 15.9, 32 x 400 23.3 / 23.7, 8 x 100 11.5 / 12.5
+//   24 bits of 12 x 600..3000 38.4 / 39.1, 20 x 600..3000 55.3 / 58.0, 24 x 600..3000 61.0 / 63.2, 24 x 600..1500 40.3 / 38.9, 28 x 600..3000 70.2 / 69.3
+//   16 heads on one: whole 16 x 257 12.6 / 12.2, 32 x 400 14.0 / 13.6, 128 x 257 14.3 / 14.2, 192 x 257 15.7 / 15.7
 static bool eight_waves_win(const nvllm_model* m, int wgs, int tiles, bool ragged) {
     if (m->hd != 128 || wgs > 256 || tiles <= 4) return false;
     const bool wide = !m->vlocache.empty();
     if (tiles <= 16) return wide ? tiles <= 8 || wgs <= 160 : m->gqa > 14 && wgs <= 128;
     if (tiles <= std::min(wgs <= 16 ? 40 : 28, 1024 / wgs)) return false;
     return !(wide && ragged) || 256 / wgs * wgs > 192 || tiles <= (wgs < 128 ? 48 : 32);
+}
+// A wave's second tile asked for together with its first, before the prologue, or behind the prologue: with both sets of four waves in flight the
+// prologue's own loads wait for up to 128 KB in the CU's queue.  16 query heads on one key head, 96 rows of 300 tokens: prologue 5.1 us a wave with
+// both, 4.5 behind, 3.3 with 20 tokens.  Together only where the chip holds all the workgroups it can (two a CU) and the contexts are long: the
+// launch is then bound by memory.  us a layer, 16 / 32 / 40 heads on 8, together / behind:
+//   8 x 20 9.6 / 9.1, 9.8 / 9.3, 9.8 / 9.4; 8 x 300 12.4 / 11.9, 12.6 / 12.0, 12.6 / 12.1; 1 x 900 15.8 / 14.9, 15.3 / 14.7, 15.6 / 14.8; 48 x 300 to 900 29.9 / 29.5, -, 29.6 / 29.5
+//   64 rows: 60 13.5 / 13.2, -, 13.2 / 12.9; 64 to 512 22.3 / 22.0, 22.5 / 22.4, 22.3 / 22.5; 300 to 900 34.0 / 35.0, 34.1 / 35.1, 34.2 / 34.4; 1000 49.8 / 52.4, -, 50.7 / 52.2
+//   200 rows: 130 39.0 / 38.0, -, 44.2 / 42.7; 64 to 512 55.2 / 55.0, -, 59.2 / 58.6; 64 to 1024 86.8 / 88.9, 89.2 / 90.2, 92.5 / 95.0; 1000 146 / 150, -, 152.5 / 153.6
+// (40 heads, rows of exactly 300: 64 rows 22.6 / 24.6, 200 64.2 / 68.8; 16 heads 24.0 / 24.6 and 62.6 / 61.4; 32 heads on 4, 128 and 400 rows 26.5 / 25.2 and 68.2 / 65.2.)
+static bool attn_tiles_ahead(const nvllm_model* m, int wgs, int n_seqs, int64_t all_len) {
+    return m->hd == 128 && m->vlocache.empty() && wgs >= 512 && all_len > (int64_t)512 * n_seqs;
 }
 // Split a sequence's context over several workgroups only when (sequences x kv heads) alone cannot fill
 // the chip (small batches, long contexts); a full batch already has >= 2 workgroups per CU.
@@ -1554,6 +1567,7 @@ static void set_attn_split(nvllm_model* m, int n_seqs, int max_len, int64_t all_
     const int base_wgs = std::max(1, n_seqs * m->kv_l);
     const bool eight = eight_waves_win(m, base_wgs, tiles, 3 * all_len < 2 * (int64_t)n_seqs * max_len);
     m->attn_waves = eight ? 8 : 4;
+    m->attn_ahead = !eight && attn_tiles_ahead(m, base_wgs, n_seqs, all_len);
     int want = std::min(kAttnMaxParts, std::max(1, (eight ? 256 : 512) / base_wgs));
     // a few more rounds of the loop cost less than the combine launch and its boundary (4.7 + 1.4 us): up to 512 tokens, and up to 1024 where
     // there would be two parts at most (16 rows of 100 to 800, in parts 17.5 us, whole 16.4; one row of 900 12.3 and 16.9)
@@ -2132,7 +2146,7 @@ extern "C" int nvllm_debug_set_option(nvllm_model* m, const char* name, int valu
 
 // counters for tests: "oneshot_calls" = all-reduces this model's context has run on the one-shot device path;
 // "tile_gemm_launches" = projections this model has run on the prefill tile GEMM; "table_copies" = whole block tables sent;
-// "qk_rows16_launches" = q/k norm launches of 16 rows and a head per workgroup; "eight_wave_launches" = decode attention on eight waves;
+// "qk_rows16_launches" = q/k norm launches of 16 rows and a head per workgroup; "eight_wave_launches" = decode attention on eight waves; "tiles_ahead_launches" = ... with a wave's second tile asked for before the prologue;
 // "scan_gate_launches" = step sizes of a decode step's selective scan by a launch of their own; "two_product_launches" = pairs of products in one launch;
 // "row_pair_launches" = products of two row blocks at a time, of all models of the process; "tile_resid_launches" = products of a prompt chunk with
 // residual and norm preparation in their epilogue
@@ -2148,6 +2162,7 @@ extern "C" int nvllm_debug_get_counter(nvllm_model* m, const char* name, int64_t
     if (!strcmp(name, "two_product_launches")) { *value = m->two_launches; return NVLLM_OK; }
     if (!strcmp(name, "row_pair_launches")) { *value = rowpair_launches(); return NVLLM_OK; }
     if (!strcmp(name, "eight_wave_launches")) { *value = m->eight_wave_launches; return NVLLM_OK; }
+    if (!strcmp(name, "tiles_ahead_launches")) { *value = m->tiles_ahead_launches; return NVLLM_OK; }
     if (!strcmp(name, "kv_f16_saturated") || !strcmp(name, "kv_f16_absmax_bits")) {
         // scan of the whole K/V pool (debug, off the hot path): elements the f16_sat clamp of a cache write produced, and the
         // largest magnitude stored (f16 bits; 0x7BFF = 65504 is the clamp)

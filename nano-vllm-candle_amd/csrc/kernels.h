@@ -305,6 +305,7 @@ struct AttnArgs {
     // split-KV (decode): each workgroup covers part_tiles 32-token tiles; partials merged by a combine pass
     int part_tiles = 0, max_parts = 0;
     int waves = 4;                     // of a workgroup; 8 with qkv and head_dim 128 only
+    bool ahead = false;                // a wave's second tile asked for before the prologue: with qkv, head_dim 128, four waves and a 16-bit cache only
     float* part_o = nullptr;           // [rows][nh_l][max_parts][hd]
     float* part_ml = nullptr;          // [rows][nh_l][max_parts][2]
 #ifdef NVLLM_STAMPS

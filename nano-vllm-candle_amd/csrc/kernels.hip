@@ -2119,8 +2119,9 @@ __device__ __forceinline__ long bf8_half(const uint4& w, int second) {
 
 // VLO: 0 = 16-bit cache, 1 = 24-bit V, 2 = 24-bit K and V (KvLayout::klo too: four more 1 KiB wave-loads per tile, one bf8 MFMA
 // per QK^T fragment against q in bf8)
-template <int HD, int NWV, bool FUSED, int VLO = 0>
-__global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
+// AHEAD: both tile sets are asked for before the prologue, see there
+template <int HD, int NWV, bool FUSED, int VLO, bool AHEAD>
+__device__ __forceinline__ void attn_paged_body(const AttnArgs& a) {
     constexpr int DC = HD / 32, DT = HD / 16, DL = VLO ? DT / 2 : 1;  // DL: 1 KiB residual fragments per tile (two PV fragments each)
     constexpr bool KLO = VLO == 2;
     constexpr bool ONE_SET = VLO != 0;  // decode with a 24-bit cache: one tile set in flight per wave (see the loop)
@@ -2165,7 +2166,7 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
     // and shared through LDS; what needs the row alone is asked for before the slot, the position and the block table are waited for.  Every
     // wave making all of q for itself, with the 14 empty columns of 16, was 24 16-byte loads and 400 instructions a lane: 64 rows of 64 to 512
     // tokens 21.7 -> 19.8 us a layer, one row of 137 9.7 -> 8.7, 24 8B rows of 256 to 2048 39.1 -> 32.2; with a 24-bit cache, where it spilled,
-    // 24 rows of 48 to 400 23.6 -> 20.1 (all before the eight waves).  Both tile sets are on their way before it starts now.
+    // 24 rows of 48 to 400 23.6 -> 20.1 (all before the eight waves).
     constexpr int half = HD / 2, LPH = HD / 4, HPW = 64 / LPH, NI = 2;  // NI: rounds of items loaded up front, all of them up to gqa = NI * NWV * HPW - 2
     [[maybe_unused]] const int kv_heads = a.kv.kv_l, items = gqa + 2, hl = lane / LPH, hd2 = lane % LPH * 2;  // this lane's dims: hd2, hd2 + 1 and the two half a head further
     [[maybe_unused]] const float* qkv_row = FUSED ? a.qkv + (size_t)row0 * a.ldqkv : nullptr;
@@ -2277,11 +2278,11 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
         if (a.n_slabs > 1)
 #pragma unroll
             for (int it = 0; it < NI; ++it) add_slabs(item_src(min(item_of(it), items - 1)), xa[it], xb[it]);
-        // This wave's first KV tiles go in flight BEHIND the prologue's own loads (vmcnt retires in order, so the prologue never waits for
-        // them) and land while it computes.  The new token's place in its tile still holds old bytes, or the new ones if the stores below
+        // This wave's first KV tile goes in flight BEHIND the prologue's own loads (vmcnt retires in order, so the prologue never waits for
+        // it) and lands while it computes; the second behind the prologue (AHEAD: with the first; rule and figures at attn_tiles_ahead).  The new token's place in its tile still holds old bytes, or the new ones if the stores below
         // pass first: the tile is patched before it is used.
         load_tile(t_begin + wave, kaA, kbA, vfA, vlA);
-        if constexpr (!ONE_SET) load_tile(t_begin + wave + NWV, kaB, kbB, vfB, vlB);
+        if constexpr (AHEAD && !ONE_SET) load_tile(t_begin + wave + NWV, kaB, kbB, vfB, vlB);
         const float ri = a.rn.ssq ? 1.0f / sqrtf(wave_sum_uniform(ssq_g) * a.rn.inv_h + a.rn.eps) : 1.0f;
         auto make = [&](int item, float2 u, float2 w, float2 nu, float2 nw) __attribute__((always_inline)) {
             u.x *= ri; u.y *= ri; w.x *= ri; w.y *= ri;
@@ -2336,6 +2337,11 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
             const float2 nu = load2(w), nw = load2(w + half);
             add_slabs(p, u, v);
             make(item_of(it), u, v, nu, nw);
+        }
+        if constexpr (!AHEAD && !ONE_SET) {
+            __builtin_amdgcn_sched_barrier(0);
+            load_tile(t_begin + wave + NWV, kaB, kbB, vfB, vlB);
+            __builtin_amdgcn_sched_barrier(0);
         }
         NVLLM_STAMP(a, 1);
         // q and the new token are published; the tiles stay in flight
@@ -2585,6 +2591,14 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
         }
     }
     NVLLM_STAMP(a, 4);
+}
+template <int HD, int NWV, bool FUSED, int VLO = 0>
+__global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
+    attn_paged_body<HD, NWV, FUSED, VLO, false>(a);
+}
+template <int HD, int NWV>
+__global__ void __launch_bounds__(NWV * 64, 2) attn_paged_ahead_kernel(AttnArgs a) {
+    attn_paged_body<HD, NWV, true, 0, true>(a);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -2977,14 +2991,16 @@ __global__ void __launch_bounds__(256) attn_combine_kernel(AttnArgs a, int rows)
     }
 }
 
-template <int HD, int NWV, bool FUSED, int VLO>
+template <int HD, int NWV, bool FUSED, int VLO, bool AHEAD = false>
 static hipError_t attn_launch_v(const AttnArgs& a, int n_tiles, int grid_z, hipStream_t s) {
     auto lds_of = [](int gqa) { return NWV * 2 * 16 * 4 + (size_t)NWV * gqa * (HD * 4 + 16) + (FUSED ? (size_t)gqa * (HD + 8) * 4 + HD * 6 : 0); };
     const size_t lds = lds_of(FUSED ? a.gqa : 16);
     static std::atomic<uint64_t> lds_set{0};
-    ensure_dyn_lds(reinterpret_cast<const void*>(attn_paged_kernel<HD, NWV, FUSED, VLO>), lds_of(16), lds_set);
+    void (*kernel)(AttnArgs) = attn_paged_kernel<HD, NWV, FUSED, VLO>;
+    if constexpr (AHEAD) kernel = attn_paged_ahead_kernel<HD, NWV>;
+    ensure_dyn_lds(reinterpret_cast<const void*>(kernel), lds_of(16), lds_set);
     dim3 grid = FUSED ? dim3(a.kv.kv_l, n_tiles, grid_z) : dim3(n_tiles * a.kv.kv_l, 1, grid_z);
-    attn_paged_kernel<HD, NWV, FUSED, VLO><<<grid, NWV * 64, lds, s>>>(a);
+    kernel<<<grid, NWV * 64, lds, s>>>(a);
     return hipGetLastError();
 }
 template <int HD, int NWV, bool FUSED>
@@ -3051,7 +3067,9 @@ hipError_t launch_attn_paged(const AttnArgs& a, int n_tiles, int rows, int n_par
     const bool fused = a.qkv != nullptr;  // decode rows straight from the QKV GEMM's slabs
     if (fused && (n_tiles != rows || rows > kAttnFusedMaxRows)) return hipErrorInvalidValue;  // fused decode: tile i is row i
     if (a.waves != 4 && (a.waves != 8 || !fused || a.kv.hd != 128)) return hipErrorInvalidValue;
+    if (a.ahead && (!fused || a.kv.hd != 128 || a.waves != 4 || a.kv.vlo)) return hipErrorInvalidValue;
     if (a.waves == 8) e = attn_launch_t<128, 8, true>(b, n_tiles, gz, s);
+    else if (a.ahead) e = attn_launch_v<128, 4, true, 0, true>(b, n_tiles, gz, s);
     else if (a.kv.hd == 128) e = fused ? attn_launch_t<128, 4, true>(b, n_tiles, gz, s) : attn_launch_t<128, 4, false>(b, n_tiles, gz, s);
     else if (a.kv.hd == 64) e = fused ? attn_launch_t<64, 4, true>(b, n_tiles, gz, s) : attn_launch_t<64, 4, false>(b, n_tiles, gz, s);
     if (e != hipSuccess || !split) return e;

@@ -183,6 +183,7 @@ struct nvllm_model {
     uint32_t* d_next = nullptr;
     float *attn_po = nullptr, *attn_pml = nullptr;  // split-KV partials [max_seqs][nh_l][kAttnMaxParts][hd] / [..][2]
     int attn_part_tiles = 4, attn_parts_max = 1, attn_waves = 4;   // this step's split geometry and waves of a workgroup (decode only)
+    bool attn_ahead = false;  // ... and AttnArgs::ahead
     float* part_val = nullptr;  // fused LM-head arg-max partials [V_l/16][max_seqs]
     int* part_idx = nullptr;
     unsigned long long* argmax_scratch = nullptr;  // ticket + per-row keys of argmax_parts_kernel
@@ -222,6 +223,7 @@ struct nvllm_model {
     int64_t tile_launches = 0;  // projections run by the tile GEMM so far (tests assert the path they force was taken)
     int64_t qk_rows16_launches = 0;  // likewise: q/k norm, rotation and cache writes by 16 rows and a head
     int64_t eight_wave_launches = 0; // ... decode attention on eight waves
+    int64_t tiles_ahead_launches = 0; // ... with both tile sets asked for before the prologue
     int64_t scan_gate_launches = 0;  // ... step sizes of a decode step's scan by their own launch
     int64_t two_launches = 0;        // ... two products in one launch
     int64_t tile_resid_launches = 0; // ... prompt products with residual and norm preparation in their epilogue

@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 LENGTHS = [1, 31, 33, 126, 127, 128, 159, 255, 256, 257, 510, 511, 512, 1021, 1022, 1023, 1024]
 
 
-def check(hd, kv, heads, lens, bits, eight):
+def check(hd, kv, heads, lens, bits, eight, ahead=0):
     import nano_vllm_candle_amd as pkg
 
     rows = len(lens)
@@ -24,6 +24,7 @@ def check(hd, kv, heads, lens, bits, eight):
     m.step(list(range(rows)), [s[:-1] for s in seqs], True, want_logits=False)
     _, got = m.step(list(range(rows)), seqs, False, want_logits=True)
     assert m.counter("eight_wave_launches") == eight * cfg.num_hidden_layers
+    assert m.counter("tiles_ahead_launches") == ahead * cfg.num_hidden_layers
     # the prompt's kernels sum in another order, from keys whose f16 may round the other way: 2^-11 of the largest logit, 2^-14 with the residuals
     bound = 2.0 ** (-11 if bits == 16 else -14)
     for i in range(min(rows, 34)):
@@ -53,3 +54,11 @@ def test_a_step_equals_the_prompt(hd, kv, heads, rows, bits, eight):
     (8, 16, [256, 1024] * 14, 24, 1), (8, 16, [256, 1535] * 6, 24, 1), (8, 16, [256, 1536] * 6, 24, 0)])
 def test_the_rule(kv, heads, lens, bits, eight):
     check(128, kv, heads, lens, bits, eight)
+
+
+# a wave's second tile asked for with its first: from 512 workgroups and more than 512 tokens a row on average, four waves, 16 bits, heads of 128
+@pytest.mark.parametrize("hd,kv,heads,lens,bits,ahead", [
+    (128, 8, 16, [512] * 64, 16, 1), (128, 8, 16, [511] * 64, 16, 0), (128, 8, 16, [512] * 63, 16, 0), (128, 8, 16, [1, 1100] * 32, 16, 1), (128, 8, 16, [1, 1020] * 32, 16, 0),
+    (128, 16, 80, [530] * 33, 16, 1), (128, 32, 64, [640, 700] * 8, 16, 1), (128, 8, 16, [520] * 64, 24, 0), (64, 8, 16, [520] * 64, 16, 0)])
+def test_two_tiles_ahead(hd, kv, heads, lens, bits, ahead):
+    check(hd, kv, heads, lens, bits, 0, ahead)
