@@ -1531,7 +1531,7 @@ static int ensure_blocks(nvllm_model* m, SeqState& s, int len) {
 // Eight waves of a decode attention's workgroup instead of four halve its chain of tiles, but the merge and the two waves of a SIMD cost up to 1.5 us:
 // only where launches leave a CU one workgroup at most, and not
 //  - in a 16-bit cache on whole contexts (up to 16 tiles), where four waves have all of them in flight at once (with more than 14 query heads a
-//    group, four waves have a third round of prologue loads, behind the tiles');
+//    group, four waves have a third round of prologue loads, behind the first tiles');
 //  - while parts of four waves, a tile each, have a CU to themselves and are so few that the combine pass is no longer for them;
 //  - in a 24-bit cache, where parts that fit the CUs leave a quarter of them idle and the longest of ragged contexts is what the launch waits for.
 // Attention and its combine pass, us a layer between two events (5 of them the events'), four waves / eight; rows x tokens, 8 kv heads:
