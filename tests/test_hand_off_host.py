@@ -1,0 +1,38 @@
+"""CPU: hand-offs between the waves of a launch and to the host, in the code objects as hipcc made them here.  Values rarely show a missing wait: what is late by a
+microsecond is there when the test looks."""
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+from nano_vllm_candle_amd._lib import LIB_PATH
+
+OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+
+
+@pytest.fixture(scope="module")
+def instructions(tmp_path_factory):
+    """instructions(part): the instructions of the kernel whose name holds `part`"""
+    if not os.path.exists(OBJDUMP):
+        pytest.skip("no llvm-objdump")
+    d = tmp_path_factory.mktemp("objects")
+    run = lambda *a: subprocess.run([OBJDUMP, *map(str, a)], cwd=d, check=True, capture_output=True, text=True).stdout.splitlines()
+    shutil.copy(LIB_PATH, d / "lib.so")
+    run("--offloading", d / "lib.so")
+    found = [(obj, line.split()[-1]) for obj in sorted(d.glob("lib.so.*gfx950")) for line in run("--syms", obj) if " F " in line]
+
+    def of(part):
+        (obj, name), = [f for f in found if part in f[1]]
+        return [re.sub(r"\s*//.*", "", line).strip() for line in run("-d", f"--disassemble-symbols={name}", obj) if line.startswith("\t")]
+
+    return of
+
+
+def test_a_copy_to_the_host_waits_for_the_stores_of_every_wave(instructions):
+    # One thread counts for its workgroup.  On gfx950 neither a barrier nor another wave's fence waits for a wave's stores.
+    ops = instructions("copy_out_kernel")
+    barrier = ops.index("s_barrier")
+    stores = [i for i, o in enumerate(ops[:barrier]) if o.startswith("global_store")]
+    assert stores and any(re.match(r"s_waitcnt .*vmcnt\(0\)", o) for o in ops[stores[-1]:barrier]), ops[stores[-1]:barrier + 1]
