@@ -3727,9 +3727,9 @@ hipError_t launch_bhtd_to_rows(const float* x, int B, int heads, int T, int hd, 
 __global__ void advance_decode_kernel(uint32_t* ids, const uint32_t* next, int* pos, int n, DecodeRow* rows, const int* block_tables, int max_blocks) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) { ids[i] = next[i]; pos[i] += 1; }
-    const int r = i / kDecodeRowInts, e = i % kDecodeRowInts;  // a record's ints are lanes of one wave: all have read before one writes
+    const int r = i / kDecodeRowInts, e = i % kDecodeRowInts;  // a record's ints are neighbouring lanes of one wave
     if (rows && r < n) {
-        const int p = rows[r].pos + 1;
+        const int p = __shfl(e == 2 ? rows[r].pos + 1 : 0, 2, kDecodeRowInts);  // read by the lane that writes it
         const int* table = block_tables + (size_t)rows[r].slot * max_blocks;
         int* const d = reinterpret_cast<int*>(rows + r);
         if (e == 2) d[e] = p;

@@ -36,3 +36,14 @@ def test_a_copy_to_the_host_waits_for_the_stores_of_every_wave(instructions):
     barrier = ops.index("s_barrier")
     stores = [i for i, o in enumerate(ops[:barrier]) if o.startswith("global_store")]
     assert stores and any(re.match(r"s_waitcnt .*vmcnt\(0\)", o) for o in ops[stores[-1]:barrier]), ops[stores[-1]:barrier + 1]
+
+
+def test_a_decode_records_position_is_read_by_the_lane_that_writes_it(instructions):
+    # Sixteen lanes move a record on and all of them need the position that one of them overwrites: they have it from that lane, and no store comes before.
+    ops = instructions("advance_decode_kernel")
+    across = [i for i, o in enumerate(ops) if re.match(r"ds_bpermute|ds_swizzle|v_readlane|v_mov_b32_dpp", o)]
+    assert across, ops
+    stores = [i for i, o in enumerate(ops) if o.startswith("global_store")]
+    record = [i for i in stores if i > across[0]]
+    reads = [i for i, o in enumerate(ops) if o.startswith("global_load") and i > across[0]]
+    assert record and reads and not any("offset:8" in ops[i] for i in reads), ops
