@@ -152,7 +152,7 @@ __device__ __forceinline__ float workgroup_sum(float v, float (&red)[NW]) {
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
     if constexpr (NW == 16) return row16_sum(red[threadIdx.x & 15]);
-    else if constexpr (NW == 8) return 0.5f * row16_sum(red[threadIdx.x & 7]);  // every one twice
+    else if constexpr (NW == 8) return row16_sum(threadIdx.x & 8 ? 0.f : red[threadIdx.x & 7]);  // (each twice and halved, a sum above half the range would be infinite)
     else {
         const float4 t = *reinterpret_cast<const float4*>(&red[0]);
         return (t.x + t.y) + (t.z + t.w);
