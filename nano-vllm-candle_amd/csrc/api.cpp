@@ -1109,7 +1109,10 @@ static int forward_chunk_fused(nvllm_model* m, const FusedPlan& fp, int R, int n
     };
     // row-parallel projection (o_proj, down_proj) of input planes (xh_, xl_) [R, K]: tp = 1 epilogue or partial + all-reduce + prep
     // one to a few rows: o_proj and down_proj leave slabs (behind the QKV product's output) that the next product adds to the stream; the stream changes buffers
-    const bool sums = !tp && fp.qkv == G_ROW && fp.o == G_ROW && fp.gu == G_ROW && fp.down == G_ROW && gemm_rowsum_ok(H, KO, m->I_l, R);
+    // (not where the QKV product has an epilogue of its own: that one reads planes, which no product writes between two layers then)
+    const bool fuse_qk = qt == 1 && n_tiles == R && !m->opt_no_attn_prologue;
+    const bool qkv_whole = !fuse_qk && fp.qkv == G_ROW && m->opt_tile_fuse_qk && gemm_rowdir_qkv_ok(NQ, H, hd, R);
+    const bool sums = !tp && !qkv_whole && fp.qkv == G_ROW && fp.o == G_ROW && fp.gu == G_ROW && fp.down == G_ROW && gemm_rowsum_ok(H, KO, m->I_l, R);
     float* const sum_slabs = m->slabs + ((size_t)R * NQ + 3) / 4 * 4;
     float *stream = m->resid, *stream_next = m->red;
     auto row_slabs = [&](const PackedW& w, const bf16_bits* xh_, const bf16_bits* xl_, int K) -> int {
@@ -1191,8 +1194,6 @@ static int forward_chunk_fused(nvllm_model* m, const FusedPlan& fp, int R, int n
         qa.kv.k = m->kcache[l]; qa.kv.v = m->vcache[l]; qa.kv.kv_l = m->kv_l; qa.kv.hd = hd;
         qa.kv.vlo = m->vlocache.empty() ? nullptr : m->vlocache[l];
         qa.kv.klo = m->klocache.empty() ? nullptr : m->klocache[l];
-        const bool fuse_qk = qt == 1 && n_tiles == R && !m->opt_no_attn_prologue;
-        const bool qkv_whole = !fuse_qk && fp.qkv == G_ROW && m->opt_tile_fuse_qk && gemm_rowdir_qkv_ok(NQ, H, hd, R);
         if (qkv_whole) {
             RowParArgs rq;
             rq.xh = m->xh; rq.xl = m->xl; rq.ldx = H; rq.M = R; rq.x_packed = packed; rq.rn = rn; rq.q = qa;
