@@ -1247,9 +1247,10 @@ static int forward_chunk_fused(nvllm_model* m, const FusedPlan& fp, int R, int n
         PROF(m, PROF_EMPTY, hipSuccess);  // calibration: an event pair around nothing, at the attention launch's place
         STAMPS(aa, m);
         if (qt == 2) {
-            aa.deal = m->opt_prefill_deal;
-            m->prefill_dealt_launches += attn_prefill_deals(aa, n_tiles);
-            PROF(m, PROF_ATTN, launch_attn_prefill(aa, n_tiles, s));
+            aa.deal = m->prefill_all.deal;
+            m->prefill_dealt_launches += aa.deal;
+            m->prefill_dealt_tiles += aa.deal ? m->prefill_all.tiles : 0;
+            PROF(m, PROF_ATTN, launch_attn_prefill(aa, m->prefill_all.tiles, s));
         }
         else PROF(m, PROF_ATTN, launch_attn_paged(aa, n_tiles, R, parts_max, s));
         // o_proj (+ residual + post-attention norm prep; qwen3.rs:278, :393)
@@ -1456,15 +1457,13 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
             m->tiles_ahead_launches += aa.ahead;
         }
         STAMPS(aa, m);
-        int attn_tiles = n_tiles;
-        if (trim && qt == 2) {  // the q-tiles of wanted rows
-            aa.tiles = m->d_prefill_tiles + n_tiles;
-            attn_tiles = m->last_groups * kPrefillTileGroup;
-        }
         if (qt == 2) {
-            aa.deal = m->opt_prefill_deal;
-            m->prefill_dealt_launches += attn_prefill_deals(aa, attn_tiles);
-            PROF(m, PROF_ATTN, launch_attn_prefill(aa, attn_tiles, s));
+            const nvllm_model::PrefillList& list = trim ? m->prefill_last : m->prefill_all;  // trim: the q-tiles of wanted rows
+            if (trim) aa.tiles = m->d_prefill_tiles + n_tiles;
+            aa.deal = list.deal;
+            m->prefill_dealt_launches += list.deal;
+            m->prefill_dealt_tiles += list.deal ? list.tiles : 0;
+            PROF(m, PROF_ATTN, launch_attn_prefill(aa, list.tiles, s));
         }
         else PROF(m, PROF_ATTN, launch_attn_paged(aa, n_tiles, R, parts_max, s));
         const bf16_bits *ch = m->xh, *cl = m->xl;
@@ -1840,7 +1839,7 @@ static int upload_chunk(nvllm_model* m, const RowPlan& p, int qt, int r0, int R,
             for (int b = 0; b < kDecodeRowBlocks; ++b) d.block[b] = b < m->max_blocks ? table[b] : 0;
         }
     }
-    m->last_groups = 0;
+    m->prefill_all = m->prefill_last = nvllm_model::PrefillList();
     if (G) {  // prefill attention: groups of four q-tiles, longest context first
         constexpr int n = kPrefillTileGroup;
         std::vector<int> glast(G), order(G);
@@ -1849,11 +1848,18 @@ static int upload_chunk(nvllm_model* m, const RowPlan& p, int qt, int r0, int R,
             order[g] = g;
         }
         std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return glast[x] > glast[y]; });
-        auto put_group = [&](PrefillTile* to, int g) {
-            for (int k = 0, i = g * n; k < n; ++k, ++i)
-                to[k] = PrefillTile{h_t0[i], h_tn[i], h_ts[i], tl[i] - h_tn[i] + 1, glast[g], m->h_block_tables[(size_t)h_ts[i] * m->max_blocks], {0, 0}};
+        auto put_groups = [&](PrefillTile* to, const std::vector<int>& groups) {
+            nvllm_model::PrefillList list;
+            list.deal = m->opt_prefill_deal >= 0 ? m->opt_prefill_deal != 0 : attn_prefill_deals(m->hd, m->kv_l, !m->vlocache.empty(), (int)groups.size(), m->cur_max_len);
+            for (int g : groups)
+                for (int k = 0; k < n; ++k) {
+                    const int i = g * n + (list.deal ? n - 1 - k : k);  // dealt: the longest context of a group first, and no empty tiles
+                    if (h_tn[i] || !list.deal)
+                        to[list.tiles++] = PrefillTile{h_t0[i], h_tn[i], h_ts[i], tl[i] - h_tn[i] + 1, glast[g], m->h_block_tables[(size_t)h_ts[i] * m->max_blocks], {0, 0}};
+                }
+            return list;
         };
-        for (int g = 0; g < G; ++g) put_group(h_pt + g * n, order[g]);
+        m->prefill_all = put_groups(h_pt, order);
         if (2 * (int)last_local.size() <= R) {  // again those with a row the head wants, in the same order
             std::vector<char> wanted(G, 0);
             int tile = 0;
@@ -1861,12 +1867,11 @@ static int upload_chunk(nvllm_model* m, const RowPlan& p, int qt, int r0, int R,
                 while (tile + 1 < T && (h_tn[tile] == 0 || h_t0[tile] + h_tn[tile] <= r)) ++tile;
                 wanted[tile / n] = 1;
             }
-            m->last_groups = (int)std::count(wanted.begin(), wanted.end(), 1);
-            if (m->last_groups) {
-                PrefillTile* to = (PrefillTile*)put(nullptr, (int*)(m->d_prefill_tiles + T), (size_t)m->last_groups * n * kPrefillTileInts);
+            order.erase(std::remove_if(order.begin(), order.end(), [&](int g) { return !wanted[g]; }), order.end());
+            if (!order.empty()) {
+                PrefillTile* to = (PrefillTile*)put(nullptr, (int*)(m->d_prefill_tiles + T), order.size() * n * kPrefillTileInts);
                 if (!to) return fail(m->ctx, NVLLM_ESTATE, "internal: metadata block of %zu ints too small", m->stage.ints);
-                for (int g : order)
-                    if (wanted[g]) { put_group(to, g); to += n; }
+                m->prefill_last = put_groups(to, order);
             }
         }
     }
@@ -2241,7 +2246,7 @@ extern "C" int nvllm_debug_set_option(nvllm_model* m, const char* name, int valu
 // counters for tests: "oneshot_calls" = all-reduces this model's context has run on the one-shot device path;
 // "tile_gemm_launches" = projections this model has run on the prefill tile GEMM; "table_copies" = whole block tables sent;
 // "qk_rows16_launches" = q/k norm launches of 16 rows and a head per workgroup; "eight_wave_launches" = decode attention on eight waves; "tiles_ahead_launches" = ... with a wave's second tile asked for before the prologue;
-// "prefill_dealt_launches" = prompt attention with a q-tile to a workgroup; "row_sum_launches" = products of a few rows that add up the slabs of the one before;
+// "prefill_dealt_launches" = prompt attention with a q-tile to a workgroup, "prefill_dealt_tiles" = q-tiles of those; "row_sum_launches" = products of a few rows that add up the slabs of the one before;
 // "scan_gate_launches" = step sizes of a decode step's selective scan by a launch of their own; "two_product_launches" = pairs of products in one launch;
 // "row_pair_launches" = products of two row blocks at a time, of all models of the process; "tile_resid_launches" = products of a prompt chunk with
 // residual and norm preparation in their epilogue
@@ -2254,6 +2259,7 @@ extern "C" int nvllm_debug_get_counter(nvllm_model* m, const char* name, int64_t
     if (!strcmp(name, "tile_resid_launches")) { *value = m->tile_resid_launches; return NVLLM_OK; }
     if (!strcmp(name, "qk_rows16_launches")) { *value = m->qk_rows16_launches; return NVLLM_OK; }
     if (!strcmp(name, "prefill_dealt_launches")) { *value = m->prefill_dealt_launches; return NVLLM_OK; }
+    if (!strcmp(name, "prefill_dealt_tiles")) { *value = m->prefill_dealt_tiles; return NVLLM_OK; }
     if (!strcmp(name, "row_sum_launches")) { *value = m->row_sum_launches; return NVLLM_OK; }
     if (!strcmp(name, "scan_gate_launches")) { *value = m->scan_gate_launches; return NVLLM_OK; }
     if (!strcmp(name, "two_product_launches")) { *value = m->two_launches; return NVLLM_OK; }
@@ -2505,6 +2511,7 @@ extern "C" int nvllm_op_attention(nvllm_ctx* ctx, const float* q, const float* k
     HIPCHK(ctx, launch_kv_write_plain(kr, vr, rows, dpos, dslot, dbt, bps, kvl, s));
     AttnArgs a;
     a.q = qr; a.kv = kvl; a.block_tables = dbt; a.max_blocks = bps; a.tiles = dtiles; a.nh_l = nh; a.gqa = gqa; a.out_f32 = out; a.longest = T;
+    a.deal = attn_prefill_deals(hd, kv, false, nt / kPrefillTileGroup, T);
     HIPCHK(ctx, launch_attn_prefill(a, nt, s));
     HIPCHK(ctx, hipStreamSynchronize(s));
     return NVLLM_OK;

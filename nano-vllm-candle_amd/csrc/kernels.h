@@ -274,7 +274,7 @@ struct alignas(16) PrefillTile {
     int row0, nrows;   // nrows 0: fills up its group
     int slot;          // of the sequence
     int first;         // position of row0
-    int group_last;    // last position in the four tiles of the group
+    int group_last;    // last position in the four tiles of the group (shared form)
     int block0;        // the sequence's first cache block
     int pad[2];
 };
@@ -294,13 +294,13 @@ struct AttnArgs {
     const int* tile_row0 = nullptr;    // per q-tile: first row, #rows, sequence slot
     const int* tile_nrows = nullptr;
     const int* tile_slot = nullptr;
-    const PrefillTile* tiles = nullptr;  // prefill: the q-tiles in groups of kPrefillTileGroup, longest context first; the workgroups beyond the
-                                         // resident set then are the short ones, not whatever came last
+    const PrefillTile* tiles = nullptr;  // prefill: the q-tiles, longest context first: the workgroups beyond the resident set then are the short ones, not
+                                         // whatever came last.  In groups of kPrefillTileGroup, or (deal) those with rows alone
     const DecodeRow* rows = nullptr;   // with qkv: a workgroup row's record each
     bool in_order = false;             // record i is row i
     const int* pos = nullptr;          // [rows]
     int longest = 0;                   // prefill: tokens of the longest context among the rows, or an upper bound
-    int deal = -1;                     // prefill: a q-tile's K/V tiles dealt to the waves of a workgroup of its own: 1 yes, 0 no, -1 by attn_prefill_deals' rule
+    bool deal = false;                 // prefill: a q-tile's K/V tiles dealt to the waves of a workgroup of its own (attn_prefill_deals)
     // load balance (decode without qkv): tile_order[rank] = tile index, longest context first; walked forwards in even and backwards in odd
     // runs of 256 workgroups, so that co-resident workgroups (ids i and i+256 share a CU when two fit) pair a long sequence with a short one.
     // nullptr = launch order.
@@ -336,9 +336,9 @@ constexpr int kAttnFusedMaxRows = 65535;  // with AttnArgs::qkv the rows are the
 hipError_t launch_attn_paged(const AttnArgs& a, int n_tiles, int rows, int n_parts_max, hipStream_t s);
 // qt = q sub-tiles (of 16 MFMA rows) per q-tile: 1 (decode) or 2 (prefill)
 inline int attn_tokens_per_tile(int gqa, int qt) { return (16 / gqa) * qt; }
-// prefill (qt = 2): n_tiles of AttnArgs::tiles, a multiple of 4; tiles 4b..4b+3 belong to one sequence, its last group is padded with empty tiles
+// prefill (qt = 2): n_tiles of AttnArgs::tiles.  Not dealt a multiple of 4; tiles 4b..4b+3 belong to one sequence, its last group is padded with empty tiles
 constexpr int kPrefillTileGroup = 4;
-bool attn_prefill_deals(const AttnArgs& a, int n_tiles);
+bool attn_prefill_deals(int hd, int kv_l, bool wide_cache, int groups, int longest);
 hipError_t launch_attn_prefill(const AttnArgs& a, int n_tiles, hipStream_t s);
 
 // ---- row-parallel projection with residual + next-norm epilogue (decode, tp == 1) ---------------------

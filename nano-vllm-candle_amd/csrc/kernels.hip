@@ -3054,7 +3054,8 @@ __global__ void __launch_bounds__(NH * 256, 2) attn_prefill_kernel(AttnArgs a) {
 // to four waves, which take theirs straight to registers (K of the next tile behind the scores, V behind the products) and meet in LDS at the
 // end.  A wave's chain is a quarter of the context where four q-tiles and two sets of waves to a workgroup leave it half, a prompt of 117 tokens is 64 workgroups
 // instead of 16; for it K and V come through L2 once per q-tile instead of once per four, so a launch that fills the chip with short contexts keeps the form
-// above.  By events, 16 heads on 8: 117 tokens 14.2 -> 10.8 us (in the kernel 6.7: 2.3 to the first scores, 2.1 for the one tile of each wave, 1.8 to merge and store),
+// above.  Its q-tiles are those with rows: an empty one that fills up a group ends at once, but workgroups go out in turn, and where every fourth has work (24 prompts of
+// 5 to 9 tokens that continue 1000) the work met on a part of the CUs: 42.4 us a launch with the empty ones, 27.2 without.  By events, 16 heads on 8: 117 tokens 14.2 -> 10.8 us (in the kernel 6.7: 2.3 to the first scores, 2.1 for the one tile of each wave, 1.8 to merge and store),
 // 500 24.1 -> 13.3, 1000 34.7 -> 19.6, 2391 67.7 -> 51.6.  There it is bound by what a CU takes in, 2.8 MB, and by the matrix cores and VALU of eight waves a CU
 // (36 us of 51.6 at the rate of the form above when full).
 // ---------------------------------------------------------------------------------------------------
@@ -3070,7 +3071,7 @@ __global__ void __launch_bounds__(256, 2) attn_prefill_dealt_kernel(AttnArgs a) 
     const int l15 = lane & 15, grp = lane >> 4;
     const int kv_l = a.kv.kv_l, ti = (int)blockIdx.x / kv_l, kh = (int)blockIdx.x - ti * kv_l;
     NVLLM_STAMP(a, 0);
-    const PrefillTile q = prefill_tile(a, ti ^ (kPrefillTileGroup - 1));  // a group's longest context first
+    const PrefillTile q = prefill_tile(a, ti);
     if (q.nrows <= 0) return;
     W w;
     w.rows(q, a.gqa, l15);
@@ -3290,12 +3291,11 @@ static hipError_t attn_prefill_launch(const AttnArgs& a, int groups, hipStream_t
 //   24 bits  1 x 16 11.6 / 10.5, 117 17.8 / 11.3, 1000 49.2 / 24.1, 2391 100 / 69; 16 x 60 15.6 / 14.6, 24 x 100 20.1 / 29.3, 8 x 250 25.0 / 24.3,
 //            8 x 380 34.7 / 35.4, 4 x 1000 69.2 / 64.0, 8 x 16 to 900 60.8 / 52.0, 12 x 64 to 512 40.8 / 42.5
 //   heads of 64  1 x 117 11.1 / 8.7, 1000 22.9 / 12.2, 5 x 700 24.5 / 23.4, 4 x 1000 31.1 / 29.4, 24 x 100 12.8 / 17.3
-bool attn_prefill_deals(const AttnArgs& a, int n_tiles) {
-    if (a.deal >= 0) return a.deal != 0;
-    const int64_t wgs = (int64_t)n_tiles / kPrefillTileGroup * a.kv.kv_l;
-    if (a.kv.vlo) return wgs <= std::min(512, 80 + a.longest * 3 / 4);
-    if (a.longest <= 16) return false;  // one tile: nothing to deal
-    return wgs <= (a.kv.hd == 64 ? std::min(512, 80 + a.longest * 3 / 4) : std::min(600, 40 + a.longest * 9 / 20));
+bool attn_prefill_deals(int hd, int kv_l, bool wide_cache, int groups, int longest) {
+    const int64_t wgs = (int64_t)groups * kv_l;
+    if (wide_cache) return wgs <= std::min(512, 80 + longest * 3 / 4);
+    if (longest <= 16) return false;  // one tile: nothing to deal
+    return wgs <= (hd == 64 ? std::min(512, 80 + longest * 3 / 4) : std::min(600, 40 + longest * 9 / 20));
 }
 // Two sets of waves halve the chain of the longest context and pay a merge, and 512 threads with twice the LDS leave a CU one workgroup
 // where it took two: they need fewer than 512 workgroups (measurements at the kernel), and contexts long enough for it, longer ones where
@@ -3312,9 +3312,9 @@ static bool attn_prefill_two(int wgs, int longest, bool lo) {
 hipError_t launch_attn_prefill(const AttnArgs& a, int n_tiles, hipStream_t s) {
     if (n_tiles <= 0) return hipSuccess;
     if (a.kv.klo && !a.kv.vlo) return hipErrorInvalidValue;  // 24-bit K comes with 24-bit V only
-    if (!a.tiles || n_tiles % kPrefillTileGroup || a.gqa < 1 || a.gqa > 16 || (a.kv.hd != 128 && a.kv.hd != 64)) return hipErrorInvalidValue;
+    if (!a.tiles || (!a.deal && n_tiles % kPrefillTileGroup) || a.gqa < 1 || a.gqa > 16 || (a.kv.hd != 128 && a.kv.hd != 64)) return hipErrorInvalidValue;
     const int groups = n_tiles / 4;
-    if (attn_prefill_deals(a, n_tiles)) return a.kv.hd == 128 ? attn_prefill_dealt<128>(a, n_tiles, s) : attn_prefill_dealt<64>(a, n_tiles, s);
+    if (a.deal) return a.kv.hd == 128 ? attn_prefill_dealt<128>(a, n_tiles, s) : attn_prefill_dealt<64>(a, n_tiles, s);
     const bool two = attn_prefill_two(groups * a.kv.kv_l, a.longest, a.kv.vlo);
     if (a.kv.hd == 128) return two ? attn_prefill_launch<128, 2>(a, groups, s) : attn_prefill_launch<128, 1>(a, groups, s);
     return two ? attn_prefill_launch<64, 2>(a, groups, s) : attn_prefill_launch<64, 1>(a, groups, s);

@@ -194,7 +194,8 @@ struct nvllm_model {
     bool want_logits = false;   // this step stores the last-row logits
     bool want_ids = true;       // ... and its greedy ids are read (not where positions are scored or the device samples)
     int cur_n = 0;              // sequences of the step in flight
-    int last_groups = 0;        // prompt attention: groups of the chunk's q-tiles with a row the head wants, listed behind all of them in d_prefill_tiles
+    struct PrefillList { int tiles = 0; bool deal = false; };
+    PrefillList prefill_all, prefill_last;  // the chunk's q-tiles in d_prefill_tiles, and behind room for all of them those of the groups with a row the head wants
     int cur_max_len = 0;        // longest of them (tokens, the new ones included)
     size_t slab_floats = 0;
     static constexpr size_t kOutSlot = 1 << 20;
@@ -231,6 +232,7 @@ struct nvllm_model {
     int64_t tile_launches = 0;  // projections run by the tile GEMM so far (tests assert the path they force was taken)
     int64_t qk_rows16_launches = 0;  // likewise: q/k norm, rotation and cache writes by 16 rows and a head
     int64_t prefill_dealt_launches = 0; // ... prompt attention with a q-tile to a workgroup
+    int64_t prefill_dealt_tiles = 0;    // ... q-tiles of those
     int64_t row_sum_launches = 0;       // ... products that add up the slabs of the one before (launch_gemm_rowsum)
     int64_t eight_wave_launches = 0; // ... decode attention on eight waves
     int64_t tiles_ahead_launches = 0; // ... with both tile sets asked for before the prologue
