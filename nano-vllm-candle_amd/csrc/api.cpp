@@ -1850,7 +1850,18 @@ static int upload_chunk(nvllm_model* m, const RowPlan& p, int qt, int r0, int R,
         std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return glast[x] > glast[y]; });
         auto put_groups = [&](PrefillTile* to, const std::vector<int>& groups) {
             nvllm_model::PrefillList list;
-            list.deal = m->opt_prefill_deal >= 0 ? m->opt_prefill_deal != 0 : attn_prefill_deals(m->hd, m->kv_l, !m->vlocache.empty(), (int)groups.size(), m->cur_max_len);
+            PrefillWork w{m->hd, m->kv_l, !m->vlocache.empty(), (int)groups.size(), m->cur_max_len, 0, 0};
+            std::vector<char> seen(m->max_seqs, 0);
+            int64_t contexts = 0, longest = 0;
+            for (int g : groups) {  // a sequence's longest comes first
+                for (int i = g * n; i < (g + 1) * n; ++i)
+                    if (h_tn[i]) w.kv_tiles += tl[i] / 32 + 1;
+                char& s = seen[h_ts[g * n]];
+                if (!s) { contexts += glast[g] + 1; longest = std::max<int64_t>(longest, glast[g] + 1); }
+                s = 1;
+            }
+            w.others = contexts - longest;
+            list.deal = m->opt_prefill_deal >= 0 ? m->opt_prefill_deal != 0 : attn_prefill_deals(w);
             for (int g : groups)
                 for (int k = 0; k < n; ++k) {
                     const int i = g * n + (list.deal ? n - 1 - k : k);  // dealt: the longest context of a group first, and no empty tiles
@@ -2511,7 +2522,9 @@ extern "C" int nvllm_op_attention(nvllm_ctx* ctx, const float* q, const float* k
     HIPCHK(ctx, launch_kv_write_plain(kr, vr, rows, dpos, dslot, dbt, bps, kvl, s));
     AttnArgs a;
     a.q = qr; a.kv = kvl; a.block_tables = dbt; a.max_blocks = bps; a.tiles = dtiles; a.nh_l = nh; a.gqa = gqa; a.out_f32 = out; a.longest = T;
-    a.deal = attn_prefill_deals(hd, kv, false, nt / kPrefillTileGroup, T);
+    PrefillWork work{hd, kv, false, nt / kPrefillTileGroup, T, 0, (int64_t)(B - 1) * T};
+    for (const PrefillTile& q : tiles) work.kv_tiles += q.nrows ? (q.first + q.nrows - 1) / 32 + 1 : 0;
+    a.deal = attn_prefill_deals(work);
     HIPCHK(ctx, launch_attn_prefill(a, nt, s));
     HIPCHK(ctx, hipStreamSynchronize(s));
     return NVLLM_OK;

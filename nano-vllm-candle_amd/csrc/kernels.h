@@ -338,7 +338,14 @@ hipError_t launch_attn_paged(const AttnArgs& a, int n_tiles, int rows, int n_par
 inline int attn_tokens_per_tile(int gqa, int qt) { return (16 / gqa) * qt; }
 // prefill (qt = 2): n_tiles of AttnArgs::tiles.  Not dealt a multiple of 4; tiles 4b..4b+3 belong to one sequence, its last group is padded with empty tiles
 constexpr int kPrefillTileGroup = 4;
-bool attn_prefill_deals(int hd, int kv_l, bool wide_cache, int groups, int longest);
+struct PrefillWork {
+    int hd, kv_l;
+    bool wide_cache;      // 24 bits
+    int groups, longest;  // groups of q-tiles; tokens of the longest context
+    int64_t kv_tiles;     // 32-token K/V tiles of every q-tile, one key head
+    int64_t others;       // tokens of all contexts but the longest
+};
+bool attn_prefill_deals(const PrefillWork& w);
 hipError_t launch_attn_prefill(const AttnArgs& a, int n_tiles, hipStream_t s);
 
 // ---- row-parallel projection with residual + next-norm epilogue (decode, tp == 1) ---------------------

@@ -32,3 +32,22 @@ def test_tiles_with_rows_alone(heads, kv, tile, cached, new):
     m.step(ids, seqs, not cached)
     assert m.counter("prefill_dealt_tiles") - before == cfg.num_hidden_layers * sum(-(-n // tile) for n in new)
     m.close()
+
+
+# many contexts behind cached prefixes, on both sides of the rule: contexts but the longest in an XCD's L2 or not (key heads / 8 x tokens x 512 bytes against 5.5 MB, 20 MB with more than
+# 256 workgroups of the shared form), K/V tiles of all q-tiles against 512 x 1.3 and x 2 those of the longest; heads of 64, whose line is 96 + half of the longest
+@pytest.mark.parametrize("heads,kv,hd,bits,cached,new,seqs,dealt", [
+    (16, 2, 128, 16, 500, 20, 64, 0), (16, 2, 128, 16, 500, 20, 16, 1), (8, 8, 128, 16, 1000, 60, 64, 0), (8, 8, 128, 16, 1000, 60, 8, 1), (32, 8, 128, 16, 2000, 100, 8, 0),
+    (16, 8, 128, 16, 2000, 100, 8, 1), (32, 2, 128, 24, 500, 20, 64, 0), (16, 8, 128, 24, 1000, 16, 40, 1), (14, 2, 64, 16, 0, 264, 8, 0), (14, 2, 64, 16, 0, 264, 6, 1)])
+def test_the_rule_behind_prefixes(heads, kv, hd, bits, cached, new, seqs, dealt):
+    cfg, m = model(heads, kv, seqs * (-(-(cached + new) // 256)), seqs, 8192, hd=hd, bits=bits)
+    m.set_option("last_rows", 0)
+    rng = np.random.default_rng(1)
+    toks = [rng.integers(0, cfg.vocab_size, cached + new) for _ in range(seqs)]
+    ids = list(range(seqs))
+    for i in range(0, seqs if cached else 0, 4):
+        m.step(ids[i:i + 4], [t[:cached] for t in toks[i:i + 4]], True)
+    before = m.counter("prefill_dealt_launches")
+    m.step(ids, toks, False)
+    assert m.counter("prefill_dealt_launches") - before == dealt * cfg.num_hidden_layers
+    m.close()
