@@ -295,7 +295,7 @@ struct AttnArgs {
     const int* tile_nrows = nullptr;
     const int* tile_slot = nullptr;
     const PrefillTile* tiles = nullptr;  // prefill: the q-tiles, longest context first: the workgroups beyond the resident set then are the short ones, not
-                                         // whatever came last.  In groups of kPrefillTileGroup, or (deal) those with rows alone
+                                         // whatever came last.  In groups of kPrefillTileGroup, or (deal) in any number
     const DecodeRow* rows = nullptr;   // with qkv: a workgroup row's record each
     bool in_order = false;             // record i is row i
     const int* pos = nullptr;          // [rows]

@@ -3294,7 +3294,7 @@ static hipError_t attn_prefill_launch(const AttnArgs& a, int groups, hipStream_t
 // (heads of 64, 14 on 2: 8 x 250 15.2 / 17.2, 12 x 64 to 512 20.3 / 22.4, 16 x 100 behind a cached 100 13.6 / 15.6)
 // That line is a prompt's, whose contexts are half of the longest on the average.  Behind cached prefixes all are as long as the longest, and where many such contexts do not
 // fit an XCD's L2 (4 MB; with fewer than eight key heads several XCDs read each) what the q-tiles read again comes from further away: then the K/V tiles of all q-tiles, over 512
-// workgroups, may be 1.3 times the longest context's, twice where the shared form has more than 256 workgroups and so one set of waves.  16 bits unless noted, cached + new:
+// workgroups, may be 1.2 times the longest context's, twice where the shared form has more than 256 workgroups and so one set of waves.  16 bits unless noted, cached + new:
 //   8 on 8  64 x 1000 + 60 71.7 / 83.7;  16 on 2  64 x 500 + 20 29.7 / 39.3, 100 x 600 + 10 29.9 / 40.9;  40 on 8  16 x 1500 + 40 53.5 / 65.3;  32 on 8  8 x 2000 + 100 65.1 / 72.7
 //   32 on 2, 24 bits  40 x 1000 + 16 54.4 / 80.8, 64 x 500 + 20 71.6 / 94.9, 24 x 500 + 30 38.3 / 48.0;  but 16 on 8  3 x 2000 + 500 69.5 / 60.5, 8 x 2000 + 100 61.3 / 43.8,
 //   40 x 1000 + 16 56.9 / 49.3;  32 on 8  1 x 4000 + 500 111 / 69, 3 x 2000 + 500 129 / 111;  40 on 8  8 x 2000 + 100 117 / 88
@@ -3306,7 +3306,7 @@ bool attn_prefill_deals(const PrefillWork& w) {
                        wgs > (w.hd == 64 ? std::min(512, 96 + w.longest / 2) : std::min(600, 40 + w.longest * 9 / 20))) return false;
     const double mb = (double)w.others * w.hd * (w.wide_cache ? 6 : 4) * std::max(1, w.kv_l / 8) / (1 << 20);
     const double work = (double)w.kv_tiles * w.kv_l / 512 * (w.kv_l < 8 ? 1.25 : 1), chain = w.longest / 32.0;
-    return wgs <= 256 ? mb <= 5.5 || work <= 1.3 * chain : mb <= 20 || work <= 2 * chain;
+    return wgs <= 256 ? mb <= 5.5 || work <= 1.2 * chain : mb <= 20 || work <= 2 * chain;
 }
 // Two sets of waves halve the chain of the longest context and pay a merge, and 512 threads with twice the LDS leave a CU one workgroup
 // where it took two: they need fewer than 512 workgroups (measurements at the kernel), and contexts long enough for it, longer ones where

@@ -34,8 +34,21 @@ def test_tiles_with_rows_alone(heads, kv, tile, cached, new):
     m.close()
 
 
+@pytest.mark.parametrize("new,every", [([70] * 8, 1), ([80] * 7 + [16] * 2, 1), ([70] * 6, 0), ([70] * 9, 0)])
+def test_groups_stay_whole_where_all_fit_at_once(new, every):
+    # 8 key heads: more than 32 q-tiles with rows (a CU's two workgroups), at most 64 with those that fill up the groups
+    cfg, m = model(16, 8, 16, len(new))
+    m.set_option("prefill_deal", 1)
+    m.set_option("last_rows", 0)
+    rng = np.random.default_rng(2)
+    m.step(list(range(len(new))), [rng.integers(0, cfg.vocab_size, n) for n in new], True)
+    tiles = [-(-n // 16) for n in new]
+    assert m.counter("prefill_dealt_tiles") == cfg.num_hidden_layers * sum(-(-t // 4) * 4 if every else t for t in tiles)
+    m.close()
+
+
 # many contexts behind cached prefixes, on both sides of the rule: contexts but the longest in an XCD's L2 or not (key heads / 8 x tokens x 512 bytes against 5.5 MB, 20 MB with more than
-# 256 workgroups of the shared form), K/V tiles of all q-tiles against 512 x 1.3 and x 2 those of the longest; heads of 64, whose line is 96 + half of the longest
+# 256 workgroups of the shared form), K/V tiles of all q-tiles against 512 x 1.2 and x 2 those of the longest; heads of 64, whose line is 96 + half of the longest
 @pytest.mark.parametrize("heads,kv,hd,bits,cached,new,seqs,dealt", [
     (16, 2, 128, 16, 500, 20, 64, 0), (16, 2, 128, 16, 500, 20, 16, 1), (8, 8, 128, 16, 1000, 60, 64, 0), (8, 8, 128, 16, 1000, 60, 8, 1), (32, 8, 128, 16, 2000, 100, 8, 0),
     (16, 8, 128, 16, 2000, 100, 8, 1), (32, 2, 128, 24, 500, 20, 64, 0), (16, 8, 128, 24, 1000, 16, 40, 1), (14, 2, 64, 16, 0, 264, 8, 0), (14, 2, 64, 16, 0, 264, 6, 1)])
