@@ -5,6 +5,8 @@
 #include <system_error>
 #include <thread>
 #include <chrono>
+#include <condition_variable>
+#include <mutex>
 #include <sys/mman.h>
 #include <hip/hip_runtime.h>
 #include <rccl/rccl.h>
@@ -1659,12 +1661,17 @@ static hipError_t out_copy(nvllm_model* m, int i, const void* src, size_t at, si
     return launch_copy_out(src, m->dev_out + at, bytes, m->out_done + i, &m->dev_out_flag[i].seq, ++m->out_seq[i], m->ctx->stream);
 }
 static bool out_there(nvllm_model* m, int i) { return __atomic_load_n(&m->out_flag[i].seq, __ATOMIC_ACQUIRE) == m->out_seq[i]; }
-static hipError_t out_wait(nvllm_model* m, int i) {  // the flag; or the stream has ended without it
-    auto asked = std::chrono::steady_clock::now();
+// The flag; or the stream has ended without it.  The wait is a core's for 10 ms, which is a decode step or a prompt of a few thousand tokens: nothing tells the thread sooner.
+// Then it sleeps, 75 us at a time with the kernel's slack: 64 prompts in 36.6 ms take 0.55 of a core (3.8 with all of download()'s threads awake) and
+// no longer; a decode step, 1.2 to 1.5 with the copies' threads.
+static hipError_t out_wait(nvllm_model* m, int i) {
+    const auto start = std::chrono::steady_clock::now();
+    auto asked = start;
     for (unsigned n = 1; !out_there(m, i); ++n) {
         if (n % 64) { __builtin_ia32_pause(); continue; }
-        std::this_thread::yield();
         const auto now = std::chrono::steady_clock::now();
+        if (now - start < std::chrono::milliseconds(10)) std::this_thread::yield();
+        else std::this_thread::sleep_for(std::chrono::microseconds(20));
         if (now - asked < std::chrono::milliseconds(20)) continue;
         asked = now;
         const hipError_t e = hipStreamQuery(m->ctx->stream);
@@ -1681,46 +1688,65 @@ static hipError_t out_wait(nvllm_model* m, int i) {  // the flag; or the stream 
 // runtime's copies and events / these / these and the caller's pages made while the step runs: 0.6 MB 0.09 / 0.08 / 0.08 ms, 14.6 MB 0.53 / 0.44 / 0.39, 39 MB 1.51 / 1.31 / 1.01,
 // 121 MB 4.14 / 3.65 / 3.08; in slots of 2 MB 121 MB 2.95, 39 MB the same.  Two threads start to pay at 1.8 MB.
 static constexpr int kPopulateWrite = 23;  // MADV_POPULATE_WRITE, which older headers lack
-static int download_slots(nvllm_model* m, int first, int step, int per, const char* src, char* dst, size_t bytes) {
-    constexpr size_t C = nvllm_model::kOutSlot;
-    const int chunks = (int)((bytes + C - 1) / C);
-    auto slot = [&](int c) { return first * per + c / step % per; };  // this thread's chunks: first, first + step, ...
-    auto size = [&](int c) { return std::min(C, bytes - (size_t)c * C); };
-    auto issue = [&](int c) { return out_copy(m, slot(c), src + (size_t)c * C, (size_t)slot(c) * C, size(c)); };
-    auto there = [&](int c) { return out_there(m, slot(c)); };
-    hipError_t e = hipSetDevice(m->ctx->device);
-    for (int c = first, k = 0; c < chunks && k < per && e == hipSuccess; c += step, ++k) e = issue(c);
-    // the caller's fresh pages, while the device is busy with what comes before the copies (an older kernel refuses: then they come with the copy)
-    for (int c = first; c < chunks && e == hipSuccess && !there(first); c += step) {
-        constexpr uintptr_t page = 4096;
-        const uintptr_t at = (uintptr_t)dst + (size_t)c * C, from = (at + page - 1) / page * page, to = (at + size(c)) / page * page;
-        if (to > from && madvise((void*)from, to - from, kPopulateWrite)) break;
+// The first thread's first copy comes before the others' on the stream; they sleep until it is there.
+struct OutGate {
+    std::mutex mu;
+    std::condition_variable cv;
+    bool open = false;
+    void wait() { std::unique_lock<std::mutex> l(mu); cv.wait(l, [&] { return open; }); }
+    void pass() { { std::lock_guard<std::mutex> l(mu); open = true; } cv.notify_all(); }
+};
+struct OutPart {  // chunks first, first + step, ... by way of slots first * per and on
+    nvllm_model* m; int first, step, per; const char* src; char* dst; size_t bytes;
+    static constexpr size_t C = nvllm_model::kOutSlot;
+    int chunks() const { return (int)((bytes + C - 1) / C); }
+    int slot(int c) const { return first * per + c / step % per; }
+    size_t size(int c) const { return std::min(C, bytes - (size_t)c * C); }
+    hipError_t issue(int c) const { return out_copy(m, slot(c), src + (size_t)c * C, (size_t)slot(c) * C, size(c)); }
+    hipError_t begin() const {
+        hipError_t e = hipSetDevice(m->ctx->device);
+        for (int c = first, k = 0; c < chunks() && k < per && e == hipSuccess; c += step, ++k) e = issue(c);
+        return e;
     }
-    for (int c = first; c < chunks && e == hipSuccess; c += step) {
-        e = out_wait(m, slot(c));
-        if (e != hipSuccess) break;
-        memcpy(dst + (size_t)c * C, m->pin_out + (size_t)slot(c) * C, size(c));
-        if (c + step * per < chunks) e = issue(c + step * per);
+    hipError_t finish(OutGate& gate) const {
+        // the caller's fresh pages, while the device is busy with what comes before the copies (an older kernel refuses: then they come with the copy)
+        for (int c = first; c < chunks() && !out_there(m, slot(first)); c += step) {
+            constexpr uintptr_t page = 4096;
+            const uintptr_t at = (uintptr_t)dst + (size_t)c * C, from = (at + page - 1) / page * page, to = (at + size(c)) / page * page;
+            if (to > from && madvise((void*)from, to - from, kPopulateWrite)) break;
+        }
+        if (first) gate.wait();
+        hipError_t e = hipSuccess;
+        for (int c = first; c < chunks() && e == hipSuccess; c += step) {
+            e = out_wait(m, slot(c));
+            if (c == 0) gate.pass();
+            if (e != hipSuccess) break;
+            memcpy(dst + (size_t)c * C, m->pin_out + (size_t)slot(c) * C, size(c));
+            if (c + step * per < chunks()) e = issue(c + step * per);
+        }
+        return e;
     }
-    return (int)e;
-}
+};
 static int download(nvllm_model* m, const void* src, void* dst, size_t bytes) {
     nvllm_ctx* ctx = m->ctx;
     const int slots = m->out_slots, want = bytes < (size_t)1500000 ? 1 : bytes < (size_t)2500000 ? 2 : 4, T = std::max(1, std::min(want, slots));
-    int err[4] = {0, 0, 0, 0};
+    hipError_t err[4] = {hipSuccess, hipSuccess, hipSuccess, hipSuccess};
     std::thread th[4];
+    OutGate gate;
     int run = 1;  // threads that exist; the others' chunks are this one's
-    auto part = [&](int t) { err[t] = download_slots(m, t, T, slots / T, (const char*)src, (char*)dst, bytes); };
+    auto part = [&](int t) { return OutPart{m, t, T, slots / T, (const char*)src, (char*)dst, bytes}; };
+    err[0] = part(0).begin();
     try {
-        for (; run < T; ++run) th[run] = std::thread(part, run);
+        for (; run < T && !err[0]; ++run) th[run] = std::thread([&, t = run] { if (!(err[t] = part(t).begin())) err[t] = part(t).finish(gate); });
     } catch (const std::system_error&) {}
-    part(0);
-    for (int t = run; t < T; ++t) part(t);
+    if (!err[0]) err[0] = part(0).finish(gate);
+    gate.pass();
+    for (int t = run; t < T && !err[0]; ++t) if (!(err[t] = part(t).begin())) err[t] = part(t).finish(gate);
     for (int t = 1; t < run; ++t) th[t].join();
-    for (int e : err)
+    for (hipError_t e : err)
         if (e) {
             (void)hipStreamSynchronize(ctx->stream);  // nothing is on its way into the slots any more
-            HIPCHK(ctx, (hipError_t)e);
+            HIPCHK(ctx, e);
         }
     return NVLLM_OK;
 }
