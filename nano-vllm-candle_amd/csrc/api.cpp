@@ -1582,18 +1582,19 @@ static int ensure_blocks(nvllm_model* m, SeqState& s, int len) {
 
 // Eight waves of a decode attention's workgroup instead of four halve its chain of tiles, but the merge and the two waves of a SIMD cost up to 1.5 us:
 // only where launches leave a CU one workgroup at most, and not
-//  - in a 16-bit cache on whole contexts (up to 16 tiles), where four waves have all of them in flight at once (with more than 14 query heads a
-//    group, four waves have a third round of prologue loads, behind the first tiles');
+//  - in a 16-bit cache on whole contexts (up to 16 tiles), where four waves have all of them in flight at once;
 //  - while parts of four waves, a tile each, have a CU to themselves and are so few that the combine pass is no longer for them;
 //  - in a 24-bit cache, where parts that fit the CUs leave a quarter of them idle and the longest of ragged contexts is what the launch waits for.
+// Whole contexts of a 24-bit cache and of more than 14 query heads a group keep eight waves where tests/test_decode_waves_gpu.py has them; with a tile's arithmetic and the
+// prologue as they are four are the better there too, by 0 to 9 % (1.6 % over all 24-bit launches, 1.0 % over those of 16 heads on one).
 // Attention and its combine pass, us a layer between two events (5 of them the events'), four waves / eight; rows x tokens, 8 kv heads:
-//   gqa 2   whole 1 x 400 12.3 / 13.0, 8 x 400 13.0 / 13.8, 20 x 400 14.9 / 16.1, 32 x 400 17.2 / 19.6, 8 x 150..180 10.5 / 11.3
-//   gqa 4   whole 8 x 400 12.9 / 13.9, 32 x 400 16.9 / 18.9
-//   gqa 2   parts 1 x 900 13.5 / 14.6, 1 x 1500 15.7 / 15.4, 3 x 700 14.1 / 14.8, 4 x 900 16.1 / 16.0, 6 x 600 14.8 / 15.6, 6 x 700 17.3 / 15.7, 8 x 700 17.7 / 16.6, 32 x 1100 33.6 / 30.1
-//   gqa 2   of 6 x 64..512 14.0 / 15.3, 20 x 64..512 18.2 / 16.0, 12 x 256..2048 24.3 / 24.2, 20 x 256..2048 31.5 / 30.6, 24 x 256..2048 32.5 / 32.6, 32 x 256..2048 40.1 / 36.3
-//   24 bits whole 1 x 150..180 13.1 / 12.3, 1 x 400 16.6 / 16.1, 20 x 400 19.8 / 19.6, 32 x 150..180 16.1 / 15.9, 32 x 400 23.3 / 23.7, 8 x 100 11.5 / 12.5
-//   24 bits of 12 x 600..3000 38.4 / 39.1, 20 x 600..3000 55.3 / 58.0, 24 x 600..3000 61.0 / 63.2, 24 x 600..1500 40.3 / 38.9, 28 x 600..3000 70.2 / 69.3
-//   16 heads on one: whole 16 x 257 12.6 / 12.2, 32 x 400 14.0 / 13.6, 128 x 257 14.3 / 14.2, 192 x 257 15.7 / 15.7
+//   gqa 2   whole 1 x 400 11.3 / 12.2, 8 x 400 11.8 / 13.0, 20 x 400 13.5 / 14.8, 32 x 400 16.4 / 18.5, 8 x 150..180 9.5 / 10.9
+//   gqa 4   whole 8 x 400 12.1 / 13.0, 32 x 400 15.9 / 18.2
+//   gqa 2   parts 1 x 900 13.6 / 14.4, 1 x 1500 15.2 / 15.4, 3 x 700 13.4 / 14.6, 4 x 900 15.2 / 15.4, 6 x 520..600 14.1 / 15.1, 6 x 700 16.6 / 15.4, 8 x 700 16.6 / 15.5, 32 x 1100 32.6 / 29.2
+//   gqa 2   of 6 x 64..512 13.2 / 14.7, 20 x 64..512 17.3 / 14.7, 12 x 256..2048 23.2 / 23.4, 20 x 256..2048 29.4 / 29.9, 24 x 256..2048 31.3 / 30.6, 32 x 256..2048 38.0 / 34.6
+//   24 bits whole 1 x 150..180 11.2 / 11.6, 1 x 400 14.1 / 14.8, 20 x 400 16.5 / 17.6, 32 x 150..180 14.0 / 15.2, 32 x 400 20.8 / 21.7, 8 x 100 10.2 / 11.4, 24 x 48..408 16.3 / 17.0
+//   24 bits parts 8 x 700 19.7 / 17.6, 32 x 1100 45.8 / 42.0; of 12 x 600..3000 37.1 / 38.6, 20 x 600..3000 53.4 / 55.8, 24 x 600..3000 59.5 / 60.5, 24 x 600..1500 38.2 / 35.9, 28 x 600..3000 66.4 / 64.4
+//   16 heads on one: whole 16 x 257 11.7 / 11.8, 32 x 400 12.9 / 12.7, 128 x 257 13.4 / 14.0, 128 x 500 15.7 / 16.8, 192 x 257 16.6 / 16.4
 static bool eight_waves_win(const nvllm_model* m, int wgs, int tiles, bool ragged) {
     if (m->hd != 128 || wgs > 256 || tiles <= 4) return false;
     const bool wide = !m->vlocache.empty();
@@ -1602,13 +1603,14 @@ static bool eight_waves_win(const nvllm_model* m, int wgs, int tiles, bool ragge
     return !(wide && ragged) || 256 / wgs * wgs > 192 || tiles <= (wgs < 128 ? 48 : 32);
 }
 // A wave's second tile asked for together with its first, before the prologue, or behind the prologue: with both sets of four waves in flight the
-// prologue's own loads wait for up to 128 KB in the CU's queue.  16 query heads on one key head, 96 rows of 300 tokens: prologue 5.1 us a wave with
+// prologue's own loads wait for up to 128 KB in the CU's queue.  16 query heads on one key head, 96 rows of 300 tokens, before a row's record: prologue 5.1 us a wave with
 // both, 4.5 behind, 3.3 with 20 tokens.  Together only where the chip holds all the workgroups it can (two a CU) and the contexts are long: the
-// launch is then bound by memory.  us a layer, 16 / 32 / 40 heads on 8, together / behind:
-//   8 x 20 9.6 / 9.1, 9.8 / 9.3, 9.8 / 9.4; 8 x 300 12.4 / 11.9, 12.6 / 12.0, 12.6 / 12.1; 1 x 900 15.8 / 14.9, 15.3 / 14.7, 15.6 / 14.8; 48 x 300 to 900 29.9 / 29.5, -, 29.6 / 29.5
-//   64 rows: 60 13.5 / 13.2, -, 13.2 / 12.9; 64 to 512 22.3 / 22.0, 22.5 / 22.4, 22.3 / 22.5; 300 to 900 34.0 / 35.0, 34.1 / 35.1, 34.2 / 34.4; 1000 49.8 / 52.4, -, 50.7 / 52.2
-//   200 rows: 130 39.0 / 38.0, -, 44.2 / 42.7; 64 to 512 55.2 / 55.0, -, 59.2 / 58.6; 64 to 1024 86.8 / 88.9, 89.2 / 90.2, 92.5 / 95.0; 1000 146 / 150, -, 152.5 / 153.6
-// (40 heads, rows of exactly 300: 64 rows 22.6 / 24.6, 200 64.2 / 68.8; 16 heads 24.0 / 24.6 and 62.6 / 61.4; 32 heads on 4, 128 and 400 rows 26.5 / 25.2 and 68.2 / 65.2.)
+// launch is then bound by memory, and it matters little: over 1195 launches of five groupings within 0.1 % of the better one, never together 0.15 %.  us a layer, 8 / 16 / 32 / 40
+// heads on 8, together / behind:
+//   8 x 20 9.1 / 8.4, 8.7 / 8.5, 8.8 / 9.0, 8.9 / 8.4; 8 x 300 11.6 / 11.0, 11.5 / 11.0, 11.4 / 11.0, 11.4 / 11.4; 1 x 900 14.3 / 13.8, 14.1 / 13.6, 12.9 / 12.2, 13.9 / 13.6
+//   64 rows: 100 15.3 / 14.3, 15.2 / 14.3, 15.3 / 14.5, 15.2 / 14.8; 64 to 512 21.7 / 21.7, 21.5 / 21.5, 22.3 / 22.1, 22.3 / 22.5; 700 36.0 / 35.7, 35.5 / 35.5, 36.0 / 35.8, 35.8 / 35.8;
+//   900 45.2 / 46.6, 44.7 / 45.7, 45.2 / 46.1, 44.9 / 47.8;  200 rows: 20 27.9 / 27.1, 28.0 / 27.2, 28.0 / 27.3, 28.4 / 27.7; 64 to 512 55.5 / 54.8, 55.6 / 55.1, 56.9 / 56.3, 58.5 / 57.2
+// (64 rows of 300 22.9 / 23.6, 22.6 / 22.6, 23.0 / 23.3, 23.0 / 24.0; 200 of 400 72.7 / 71.5, 72.8 / 71.7, 74.6 / 75.6, 71.9 / 73.2.)
 static bool attn_tiles_ahead(const nvllm_model* m, int wgs, int n_seqs, int64_t all_len) {
     return m->hd == 128 && m->vlocache.empty() && wgs >= 512 && all_len > (int64_t)512 * n_seqs;
 }

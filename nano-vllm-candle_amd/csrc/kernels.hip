@@ -2878,8 +2878,8 @@ __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_ahead_kernel(AttnArgs 
 // matrix cores are busy 45 % of the time, the VALU another 45 %.  NH = 2 halves the chain of the longest context, which sets the end of
 // a launch that does not fill the chip twice over.  Measured per launch (16 / 8 heads of 128) with a maximum across lanes, a rescale and
 // a drained ring in every tile, NH = 1: one prompt of 2391 tokens 109 us, now 65; 18.7 k tokens in prompts of 64 to 512, chunks of 4096
-// rows, 34.5 -> 30.7; 32 / 8 heads, 4050 tokens in prompts of 700 to 2000, 152 -> 118.  Both prompts with the other NH: 80, 42 (before
-// the other changes); when to take which: attn_prefill_two.  VLO: a 24-bit cache (see attn_paged_kernel), whose residual fragments ride in the same ring: 5.4 k tokens in prompts
+// rows, 34.5 -> 30.7; 32 / 8 heads, 4050 tokens in prompts of 700 to 2000, 152 -> 118.  When to take which: attn_prefill_two (most launches that two sets
+// once were for are the dealt form's below).  VLO: a 24-bit cache (see attn_paged_kernel), whose residual fragments ride in the same ring: 5.4 k tokens in prompts
 // of 48 to 400, 88 us with K and V straight to registers for every q-tile of its own, now 39 and, with NH = 2, 30.
 // ---------------------------------------------------------------------------------------------------
 template <int HD, int QT, int NH, int VLO>
@@ -3308,18 +3308,14 @@ bool attn_prefill_deals(const PrefillWork& w) {
     const double work = (double)w.kv_tiles * w.kv_l / 512 * (w.kv_l < 8 ? 1.25 : 1), chain = w.longest / 32.0;
     return wgs <= 256 ? mb <= 5.5 || work <= 1.2 * chain : mb <= 20 || work <= 2 * chain;
 }
-// Two sets of waves halve the chain of the longest context and pay a merge, and 512 threads with twice the LDS leave a CU one workgroup
-// where it took two: they need fewer than 512 workgroups (measurements at the kernel), and contexts long enough for it, longer ones where
-// the launch is more than one round of the 256 CUs.  A 24-bit cache, with half as much work again in a tile, gains earlier.  0.6B, prompts x
-// tokens, ms with one set and with two.  16 bits, one round: 1 x 100 1.368 / 1.417, 1 x 250 2.100 / 2.113, 1 x 380 3.177 / 3.156, 1 x 500
-// 3.341 / 3.283, 1 x 1000 4.649 / 4.493; more: 48 x 20 4.06 / 4.28, 60 x 60 7.64 / 7.94, 8 x 380 7.32 / 7.49, 5 x 700 7.80 / 7.89, 3 x 1000
-// 7.71 / 7.68, 2 x 1300 7.59 / 7.34, 1 x 2391 7.99 / 7.53.  24 bits, one round: 1 x 100 1.492 / 1.508, 1 x 150 1.890 / 1.877, 1 x 250 2.351 /
-// 2.256; more: 24 x 100 6.51 / 6.79, 8 x 380 7.80 / 7.83, 5 x 500 7.06 / 6.87, 1 x 2391 10.10 / 8.65.
-static bool attn_prefill_two(int wgs, int longest, bool lo) {
-    const int from = lo ? 160 : 384;
-    return wgs < 512 && longest >= (wgs > 256 ? from * 8 / 3 : from);
-}
-// prefill: n_tiles (a multiple of 4: every sequence's tile list padded with empty tiles) q-tiles of 2 sub-tiles each
+// Two sets of waves halve the chain of the longest context and pay a merge, and 512 threads with twice the LDS leave a CU one workgroup where it took two: up to one round of
+// the 256 CUs, and contexts long enough for it.  What the dealt form leaves of that: several contexts, most of them behind cached prefixes.  A 24-bit cache, with half as much work again
+// in a tile, gains earlier.  us a launch with one set and with two, heads, sequences x cached + new:
+//   16 bits  8 on 8  24 x 200 + 60 19.5 / 20.3, 8 x 380 23.0 / 23.3;  16 on 2  64 x 500 + 20 30.0 / 29.7, 100 x 600 + 10 32.1 / 29.9;  32 on 4  24 x 500 + 30 31.3 / 29.6, 16 x 1500 + 40 62.8 / 50.1;
+//            32 on 8  8 x 2000 + 100 79.7 / 65.1;  past 256 workgroups  16 on 8  24 x 100 18.5 / 27.7, 64 x 500 + 20 41.3 / 49.4, 4 x 900 41.3 / 44.6;  8 on 8  64 x 1000 + 60 71.7 / 78.7
+//   24 bits  8 on 8  24 x 100 19.4 / 20.1;  32 on 2  100 x 150 + 4 21.8 / 23.1, 64 x 200 + 8 27.5 / 26.7, 40 x 300 + 16 32.8 / 29.4, 24 x 500 + 30 46.0 / 38.3, 8 x 2000 + 100 137 / 94;
+//            past 256 workgroups  32 on 2  64 x 500 + 20 56.6 / 71.6;  16 on 8  8 x 380 34.9 / 40.0, 12 x 64 to 512 41.8 / 41.4
+static bool attn_prefill_two(int wgs, int longest, bool lo) { return wgs <= 256 && longest >= (lo ? 180 : 480); }
 hipError_t launch_attn_prefill(const AttnArgs& a, int n_tiles, hipStream_t s) {
     if (n_tiles <= 0) return hipSuccess;
     if (a.kv.klo && !a.kv.vlo) return hipErrorInvalidValue;  // 24-bit K comes with 24-bit V only
