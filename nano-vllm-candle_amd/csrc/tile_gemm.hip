@@ -657,7 +657,9 @@ struct TileResidArgs {
 // same block need 10 for 16 and are bound by those reads).  A stage is two k-tiles; three stages in the ring, copies two stages ahead; all
 // fragments of the next stage are read under this stage's products, so a stage waits once, at its barrier.  At the end the halves of the split
 // exchange row tiles, add the residual and leave the stream, the next norm's planes (weight times stream) and the rows' sums of squares.
-// Bound by LDS (at RT 4 1152 cycles a stage against 1024 of products) and the epilogue's stores, 33 MB at 4096 rows from every CU at once.
+// What it spends, by stamps at 4096 rows, K 2048 / 3072: first copies 4.3 us, loop 25.5 / 38.3, exchange 0.5, sums and stores (33 MB from every CU at once) 3.8; at 2391 rows (RT 3) 3.4, 19.1 /
+// 30.2, 0.5, 3.1; at 1280 (RT 2) 2.2, 16.0 / 24.5, 0.3, 2.0.  The loop's stage of 0.80 us at RT 4 is not the LDS's 1152 cycles nor the products' 1024, both under 0.5 us; a workgroup takes in
+// 48 KiB a stage, more per product than the other tile kernels' blocks.  That this is what bounds it has not been shown.
 // RT: the smallest whose blocks are one round of the CUs, 4 above.  0.6B, o and down, us each at RT 1, 2, 3, 4: 1000 rows 22 / 26 / 30 / 36, 1280
 // 28 / 27 / 31 / 37, 2020 34 / 29 / 32 / 39, 2391 45 / 45 / 35 / 40, 3000 48 / 47 / 36 / 40, 4000 65 / 57 / 62 / 45; with K splits over
 // workgroups and a norm launch 22 + 9, 26 + 16, 26 + 17, 37 + 15 (2391) and 39 + 17 (4096).
@@ -943,7 +945,8 @@ hipError_t launch_gemm_tile(const bf16_bits* xh, const bf16_bits* xl, const Pack
 // Row tiles of a wave for the QKV product with its epilogue: blocks of 256 rows, or of 192 or 128 where their rounds of the chip are the cheaper ones
 // (a block costs about RT + 2: what does not grow with its rows is the W it reads, its start and its epilogue); 0: no such block, f32 sums and the row kernel.
 // Those may split K, and 128 rows by 256 features are short of LDS, so where blocks of 256 rows were not the best, the lower ones take over only from the workgroups
-// below on; K 1024 stays with the row kernel there, whose range up to 2040 rows its test states (blocks of 128 would be 83.1 -> 79.4 at 1024 rows and 115 -> 96.3 at 2048).
+// below on.  K 1024 has no such line: tests/test_qk_rows_gpu.py has the row kernel run at up to 2040 rows, where blocks of 128 would be the better ones (83.1 -> 79.4 at 1024
+// rows, 115 -> 96.3 at 2048).  With 4096 features blocks of 256 rows take over at 2049 rows; with 2048, at 4097, nothing was measured in between.
 // us a layer of all products and the row kernel, one prompt of so many tokens, by the rule before (256 rows, or f32 sums) and this one:
 //   0.6B (H 1024)  2391 127 / 115, 2600 130 / 119, 3072 139 / 128, 4096 the same; 24 bits 2391 132 / 120
 //   H 2048         1200 144 / 133, 2048 171 / 149, 2391 200 / 185, 3000 206 / 199, 4096 the same; 1024 by blocks of 128 118 / 125
