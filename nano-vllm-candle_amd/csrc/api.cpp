@@ -1838,21 +1838,30 @@ static int upload_chunk(nvllm_model* m, const RowPlan& p, int qt, int r0, int R,
     };
     const bool ids = device_ids || put(p.ids.data() + r0, m->d_ids, R);
     const bool rows = put(p.pos.data() + r0, m->d_pos, R) && put(p.slot.data() + r0, m->d_slot, R);
-    int *h_t0 = put(nullptr, m->d_tile_row0, T), *h_tn = put(p.tile_nrows.data() + t0, m->d_tile_nrows, T), *h_ts = put(p.tile_slot.data() + t0, m->d_tile_slot, T);
     const bool last = last_local.empty() || put(last_local.data(), m->d_last_rows, last_local.size());
-    // attention load balance: q-tiles ordered by context length, longest first (stable for ties); an empty padding tile
-    // (prefill groups of four) has no last row: it sorts as -1, behind every real tile
-    int* h_ord = put(nullptr, m->d_tile_order, T);
+    // A q-tile's rows, slot and place in the order (longest context first, for the attention's load balance; stable for ties), for kernels that do not have them in a PrefillTile.
+    const bool records = !m->dec && qt == 2;
+    std::vector<int> host(records ? 4 * (size_t)T : 0);
+    auto tiles = [&](int k, const int* src, int* dst) {
+        if (!records) return put(src, dst, T);
+        int* h = host.data() + (size_t)k * T;
+        if (src) memcpy(h, src, (size_t)T * 4);
+        return h;
+    };
+    int *h_t0 = tiles(0, nullptr, m->d_tile_row0), *h_tn = tiles(1, p.tile_nrows.data() + t0, m->d_tile_nrows), *h_ts = tiles(2, p.tile_slot.data() + t0, m->d_tile_slot),
+        *h_ord = tiles(3, nullptr, m->d_tile_order);
     const int G = !m->dec && qt == 2 ? T / kPrefillTileGroup : 0;
     PrefillTile* h_pt = G ? (PrefillTile*)put(nullptr, (int*)m->d_prefill_tiles, (size_t)T * kPrefillTileInts) : nullptr;
     const bool decode = !m->dec && qt == 1 && T == R;
     DecodeRow* h_dr = decode ? (DecodeRow*)put(nullptr, (int*)m->d_decode_rows, (size_t)R * kDecodeRowInts) : nullptr;
     if (!ids || !rows || !h_t0 || !h_tn || !h_ts || !last || !h_ord || (G && !h_pt) || (decode && !h_dr)) return fail(m->ctx, NVLLM_ESTATE, "internal: metadata block of %zu ints too small", m->stage.ints);
     for (int i = 0; i < T; ++i) h_t0[i] = p.tile_row0[t0 + i] - r0;
-    std::vector<int> tl(T);  // position of each tile's last row
+    std::vector<int> tl(T);  // position of each tile's last row (-1: it fills up a group of four)
     for (int i = 0; i < T; ++i) tl[i] = p.tile_nrows[t0 + i] > 0 ? p.pos[p.tile_row0[t0 + i] + p.tile_nrows[t0 + i] - 1] : -1;
-    for (int i = 0; i < T; ++i) h_ord[i] = i;
-    std::stable_sort(h_ord, h_ord + T, [&](int x, int y) { return tl[x] > tl[y]; });
+    if (!records) {
+        for (int i = 0; i < T; ++i) h_ord[i] = i;
+        std::stable_sort(h_ord, h_ord + T, [&](int x, int y) { return tl[x] > tl[y]; });
+    }
     if (decode) {
         // Longest context first, every other run of 256 workgroups backwards: workgroups i and i + 256 share a CU when two fit, so a long context
         // gets a short neighbour.  Up to 128 workgroups, with the parts of a row beside them, there is nothing to pair, and a row that is
