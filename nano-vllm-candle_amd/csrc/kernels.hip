@@ -2277,12 +2277,12 @@ struct AttnWave {
             my_pos[t] = valid ? q.first + tok : -1;
         }
     }
-    // q as it is stored, for begin(): every lane loads, those of no row read row 0
-    __device__ __forceinline__ void load_q(const AttnArgs& a, int my_head, int grp, float4 (&x)[QT][DC][2]) const {
+    // q as it is stored, for begin(): every lane loads, those of no row the tile's first
+    __device__ __forceinline__ void load_q(const AttnArgs& a, const PrefillTile& q, int my_head, int grp, float4 (&x)[QT][DC][2]) const {
         const int ldq = a.nh_l * HD;
 #pragma unroll
         for (int t = 0; t < QT; ++t) {
-            const float4* p = reinterpret_cast<const float4*>(a.q + (size_t)max(my_row[t], 0) * ldq + (size_t)my_head * HD + grp * 8);
+            const float4* p = reinterpret_cast<const float4*>(a.q + (size_t)(my_row[t] < 0 ? q.row0 : my_row[t]) * ldq + (size_t)my_head * HD + grp * 8);
 #pragma unroll
             for (int c = 0; c < DC; ++c) { x[t][c][0] = p[c * 8]; x[t][c][1] = p[c * 8 + 1]; }
         }
@@ -2946,8 +2946,10 @@ __global__ void __launch_bounds__(NH * 256, 2) attn_prefill_kernel(AttnArgs a) {
     stage(0, 0, q.block0);
     if (last_set >= 1) stage(1, 1, q.block0);
     int blk_pf = blk_load(2);
-    float4 q_raw[QT][DC][2];
-    w.load_q(a, my_head, grp, q_raw);
+    // A wave whose tile fills up the group reads no q: prompts of 2 or 3 tokens, of whose waves three in four are that, 47 of them, 16 heads on 8, 11.4 us a launch with it, now 10.6.  The
+    // others ask for all of it at once (by sub-tile, where it has rows: 64 x 200, 40 heads on 8, 187 -> 194).
+    float4 q_raw[QT][DC][2] = {};
+    if (q.nrows > 0) w.load_q(a, q, my_head, grp, q_raw);
     w.begin(q_raw);
     NVLLM_STAMP(a, 1);
 #ifdef NVLLM_STAMPS
@@ -3078,7 +3080,7 @@ __global__ void __launch_bounds__(256, 2) attn_prefill_dealt_kernel(AttnArgs a) 
     const int end = ((q.first + q.nrows - 1) >> 5) + 1;  // K/V tiles of this q-tile
     const int my_head = kh * a.gqa + (l15 % a.gqa), ldq = a.nh_l * HD;
     float4 q_raw[QT][DC][2];
-    w.load_q(a, my_head, grp, q_raw);
+    w.load_q(a, q, my_head, grp, q_raw);
     const uniform_ints_t bt = uniform_ints(a.block_tables + (size_t)q.slot * a.max_blocks);
     uint4 fr[2 * DC], frl[KLO ? DC : 1], fv[DT], fvl[VLO ? DL : 1];
     // tiles past the end are loads from buffers of no bytes (see attn_paged_kernel)
