@@ -1,5 +1,5 @@
 """CPU: hand-offs between the waves of a launch and to the host, in the code objects as hipcc made them here.  Values rarely show a missing wait: what is late by a
-microsecond is there when the test looks."""
+microsecond is there when the test looks.  And what a loop hands to its next turn."""
 import os
 import re
 import shutil
@@ -47,3 +47,12 @@ def test_a_decode_records_position_is_read_by_the_lane_that_writes_it(instructio
     record = [i for i in stores if i > across[0]]
     reads = [i for i, o in enumerate(ops) if o.startswith("global_load") and i > across[0]]
     assert record and reads and not any("offset:8" in ops[i] for i in reads), ops
+
+
+@pytest.mark.parametrize("hd,sets,lo", [(128, 1, 0), (128, 1, 1), (128, 1, 2), (128, 2, 0), (128, 2, 1), (128, 2, 2), (64, 1, 0), (64, 2, 0)])
+def test_the_sum_over_v_stays_in_its_registers_from_tile_to_tile(instructions, hd, sets, lo):
+    # A K/V tile's last products write where the next tile's read: no pair of registers moves between the first product and the last.
+    ops = instructions(f"attn_prefill_kernelILi{hd}ELi2ELi{sets}ELi{lo}E")
+    products = [i for i, o in enumerate(ops) if "mfma" in o]
+    moves = [o for o in ops[products[0]:products[-1]] if o.startswith("v_mov_b64")]
+    assert products and not moves, moves
