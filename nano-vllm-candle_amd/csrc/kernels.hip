@@ -3306,7 +3306,9 @@ static hipError_t attn_prefill_launch(const AttnArgs& a, int groups, hipStream_t
 //   8 on 8  64 x 1000 + 60 71.7 / 83.7;  16 on 2  64 x 500 + 20 29.7 / 39.3, 100 x 600 + 10 29.9 / 40.9;  40 on 8  16 x 1500 + 40 53.5 / 65.3;  32 on 8  8 x 2000 + 100 65.1 / 72.7
 //   32 on 2, 24 bits  40 x 1000 + 16 54.4 / 80.8, 64 x 500 + 20 71.6 / 94.9, 24 x 500 + 30 38.3 / 48.0;  but 16 on 8  3 x 2000 + 500 69.5 / 60.5, 8 x 2000 + 100 61.3 / 43.8,
 //   40 x 1000 + 16 56.9 / 49.3;  32 on 8  1 x 4000 + 500 111 / 69, 3 x 2000 + 500 129 / 111;  40 on 8  8 x 2000 + 100 117 / 88
-// Over 858 launches of 13 groupings of heads, a half of them behind cached prefixes, within 1.2 % of the faster form (2.2 % behind prefixes without it).
+// Over 858 launches of 13 groupings of heads, a half of them behind cached prefixes, within 1.0 % of the faster form (2.2 % behind prefixes without it); over 778 of 19 groupings at random, 1 to 80
+// sequences, 1.2 %.  It misses most where few key heads' contexts are a little over the line (16 on 2, 17 x 1817 + 92, 98.7 shared and dealt 120) and where prompts of very different length
+// fill groups up with empty q-tiles (8 on 8, 900 and 60 x 20, 36.9 and 21.9).
 bool attn_prefill_deals(const PrefillWork& w) {
     const int64_t wgs = (int64_t)w.groups * w.kv_l;
     if (w.wide_cache ? wgs > std::min(512, 80 + w.longest * 3 / 4)
