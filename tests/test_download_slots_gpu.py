@@ -30,3 +30,27 @@ def test_every_row_arrives(vocab, rows):
         # another kernel for one row: two 16-bit planes a product, 2^-15, one layer and the head
         assert np.abs(one - got[i]).max() < 2.0 ** -13 * np.abs(one).max()
     m.close()
+
+
+@pytest.mark.parametrize("at", [1, 2, 3, 1021])  # floats behind the start of a page; what lies around stays
+def test_arrays_at_odd_places(at):
+    import ctypes as C
+
+    import nano_vllm_candle_amd as pkg
+    from nano_vllm_candle_amd import _lib
+
+    cfg = pkg.Qwen3Config.tiny(vocab_size=32784, hidden_size=256, intermediate_size=256, num_hidden_layers=1, max_position_embeddings=256)
+    rows, n = 17, 17 * 32784
+    m = pkg.Qwen3ForCausalLM.from_synthetic(cfg, 3)
+    m.kv_alloc(rows, rows, 1024)
+    ids, seqs = list(range(rows)), [[5 + i, 9] for i in range(rows)]
+    m.step(ids, [s[:1] for s in seqs], True)
+    want_ids, want = m.step(ids, seqs, False, want_logits=True)
+    memory = np.full(n + 4096, 7.0, np.float32)
+    start = -memory.ctypes.data % 4096 // 4 + at
+    next_ids = np.full(rows + 2, 77, np.uint32)
+    u32p, seq_ids, ptrs, lens, _keep = m._step_args(ids, seqs)
+    _lib.check(_lib.lib().nvllm_step(m.h, rows, seq_ids, ptrs, lens, 0, next_ids[1:].ctypes.data_as(u32p), memory[start:].ctypes.data_as(C.POINTER(C.c_float))), m.ctx.h)
+    m.close()
+    assert np.array_equal(memory[start:start + n].reshape(rows, -1), want) and np.array_equal(next_ids[1:-1], want_ids)
+    assert (memory[:start] == 7).all() and (memory[start + n:] == 7).all() and next_ids[0] == next_ids[-1] == 77
