@@ -41,6 +41,7 @@ int nvllm_profile_read(nvllm_model* m, double* total_ms, int64_t* launches);
  *   "last_rows" (1, 0 never, default -1: 1 unless "tile_min_wgs" is 1): past the last layer's mixer a prompt chunk goes on with the rows
  *       whose logits are wanted alone;
  *   "prefill_deal" (1, 0 never, default -1: by size): prompt attention with a q-tile to a workgroup, its K/V tiles dealt to the waves;
+ *   "resident" (default 1): decode steps of one to eight rows in one launch where sizes and cache fit it; "resident_spins": turns of a wait in it (test hook);
  *   "no_fused", "no_xpack", "no_rowpar", "no_attn_prologue" (default 0): force the generic decode path / row-major planes /
  *       no whole-K row-parallel GEMMs / q,k-norm + RoPE + KV write in their own row kernel. */
 int nvllm_debug_set_option(nvllm_model* m, const char* name, int value);
@@ -49,7 +50,7 @@ int nvllm_debug_set_option(nvllm_model* m, const char* name, int value);
  * whole block tables sent because a step's pinned block had no room for the new entries; "tile_gemm_launches" = projections
  * run by the prefill tile GEMM; "qk_rows16_launches" = q/k norm, rotation and cache writes by 16 rows and a head per
  * workgroup; "eight_wave_launches" = decode attention on eight waves a workgroup; "prefill_dealt_launches" = prompt attention
- * with a q-tile to a workgroup, "prefill_dealt_tiles" = q-tiles of those; "row_sum_launches" = products of one to a few rows that add up the slabs of the one before; "scan_gate_launches" = step sizes of a
+ * with a q-tile to a workgroup, "prefill_dealt_tiles" = q-tiles of those; "resident_launches" = decode steps in one launch; "row_sum_launches" = products of one to a few rows that add up the slabs of the one before; "scan_gate_launches" = step sizes of a
  * decode step's selective scan by a launch of their own; "two_product_launches" = pairs of products in one launch;
  * "row_pair_launches" = products of two row blocks at a time, of all models of the process; "tile_resid_launches" = products
  * of a prompt chunk with residual and norm preparation in their epilogue; "kv_f16_saturated" = elements of the K/V pool at the

@@ -30,6 +30,7 @@
 #include "../../include/nvllm_amd_debug.h"
 #include "kernels.h"
 #include "decoder.h"
+#include "resident.h"
 #include "synth_device.h"
 
 // ---------------------------------------------------------------------------------------------------
@@ -243,6 +244,32 @@ static int oneshot_setup(nvllm_ctx* ctx, size_t slot_floats) {
     return NVLLM_OK;
 }
 
+// Resident steps (resident.hip) of one device one after the other: each wants every CU, and two that had a part of them each would wait for one another until they
+// give up.  The stream of the last one; a step on another stream waits for what that one holds so far.
+static std::mutex g_resident_mu;
+static std::map<int, nvllm_ctx*> g_resident_last;
+static hipError_t resident_turn(nvllm_ctx* ctx, const ResidentArgs& a) {
+    std::lock_guard<std::mutex> lk(g_resident_mu);
+    nvllm_ctx*& last = g_resident_last[ctx->device];
+    if (last && last != ctx) {
+        hipError_t e = hipSuccess;
+        if (!ctx->resident_ev) e = hipEventCreateWithFlags(&ctx->resident_ev, hipEventDisableTiming);
+        if (e == hipSuccess) e = hipEventRecord(ctx->resident_ev, last->stream);
+        if (e == hipSuccess) e = hipStreamWaitEvent(ctx->stream, ctx->resident_ev, 0);
+        if (e != hipSuccess) return e;
+    }
+    last = ctx;
+    return launch_resident(a, ctx->stream);
+}
+static void resident_leave(nvllm_ctx* ctx) {  // its stream is idle
+    {
+        std::lock_guard<std::mutex> lk(g_resident_mu);
+        const auto it = g_resident_last.find(ctx->device);
+        if (it != g_resident_last.end() && it->second == ctx) g_resident_last.erase(it);
+    }
+    if (ctx->resident_ev) (void)hipEventDestroy(ctx->resident_ev);
+}
+
 extern "C" const char* nvllm_last_error(const nvllm_ctx* ctx) { return ctx ? ctx->err.c_str() : g_create_err.c_str(); }
 
 extern "C" int nvllm_rccl_unique_id(void* out_id) {
@@ -326,6 +353,7 @@ extern "C" int nvllm_ctx_destroy(nvllm_ctx* c) {
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
     oneshot_free(c);
+    resident_leave(c);
     if (c->comm) ncclCommDestroy(c->comm);
     (void)hipEventDestroy(c->ev0);
     (void)hipEventDestroy(c->ev1);
@@ -456,11 +484,12 @@ static void free_kv(nvllm_model* m) {
     m->kcache.clear(); m->vcache.clear(); m->vlocache.clear(); m->klocache.clear();
     void* ptrs[] = {m->d_block_tables, m->d_ids, m->d_pos, m->d_slot, m->d_tile_row0, m->d_tile_nrows, m->d_tile_slot,
                     m->d_last_rows, m->d_tile_order, m->d_prefill_tiles, m->d_decode_rows, m->resid, m->last_resid, m->slabs, m->qbuf, m->logits, m->d_maxval, m->red, m->xh, m->xl, m->xh2, m->xl2, m->ctxh, m->ctxl, m->ssqA, m->ssqB, m->ssqT, m->d_next,
-                    m->part_val, m->part_idx, m->argmax_scratch, m->attn_po, m->attn_pml, m->tap_h, m->tap_res, m->cosv, m->sinv, m->tickets, m->qkv_out, m->d_keys, m->d_temps};
+                    m->part_val, m->part_idx, m->argmax_scratch, m->attn_po, m->attn_pml, m->tap_h, m->tap_res, m->cosv, m->sinv, m->tickets, m->qkv_out, m->d_keys, m->d_temps, m->d_resident_layers, m->resident_buffer, m->resident_gave_up};
     for (void* p : ptrs) if (p) (void)hipFree(p);
     m->d_block_tables = nullptr; m->d_ids = nullptr; m->d_pos = m->d_slot = m->d_tile_row0 = m->d_tile_nrows = m->d_tile_slot = m->d_last_rows = m->d_tile_order = nullptr; m->d_prefill_tiles = nullptr; m->d_decode_rows = nullptr;
     m->resid = m->last_resid = m->slabs = m->qbuf = m->logits = m->d_maxval = m->red = nullptr; m->xh = m->xl = m->xh2 = m->xl2 = m->ctxh = m->ctxl = nullptr; m->ssqA = m->ssqB = m->ssqT = nullptr; m->d_next = nullptr; m->part_val = nullptr; m->part_idx = nullptr; m->argmax_scratch = nullptr; m->attn_po = m->attn_pml = nullptr;
     m->tap_h = m->tap_res = nullptr; m->cosv = m->sinv = nullptr; m->tickets = nullptr; m->qkv_out = nullptr; m->d_keys = nullptr; m->d_temps = nullptr;
+    m->d_resident_layers = nullptr; m->resident_buffer = nullptr; m->resident_gave_up = nullptr; m->h_resident = m->dev_resident = nullptr;
     stage_release(m);
     m->num_blocks = 0;
 }
@@ -472,7 +501,7 @@ int stage_alloc(nvllm_model* m, size_t ints) {
     const size_t in = g.ints * Staging::kSlots * sizeof(int), most = (size_t)m->max_seqs * m->cfg.vocab_size * 4, C = nvllm_model::kOutSlot;
     m->out_slots = (int)std::min<size_t>(nvllm_model::kOutSlots, (most + C - 1) / C);
     m->out_ids = ((size_t)m->max_seqs * 4 + 63) / 64 * 64;
-    const size_t flags_at = in + m->out_slots * C + (1 + kMaxPending) * m->out_ids, flags = nvllm_model::kOutFlags * sizeof(nvllm_model::OutFlag);
+    const size_t flags_at = in + m->out_slots * C + (1 + kMaxPending) * m->out_ids, flags = (nvllm_model::kOutFlags + 1) * sizeof(nvllm_model::OutFlag);
     HIPCHK(m->ctx, hipHostMalloc((void**)&g.host, flags_at + flags, hipHostMallocMapped | hipHostMallocCoherent));
     HIPCHK(m->ctx, hipHostGetDevicePointer((void**)&g.dev, g.host, 0));
     m->pin_out = (char*)g.host + in;
@@ -480,6 +509,8 @@ int stage_alloc(nvllm_model* m, size_t ints) {
     m->out_flag = (nvllm_model::OutFlag*)((char*)g.host + flags_at);
     m->dev_out_flag = (nvllm_model::OutFlag*)((char*)g.dev + flags_at);
     memset(m->out_flag, 0, flags);
+    m->h_resident = (int*)&m->out_flag[nvllm_model::kOutFlags].seq;
+    m->dev_resident = (int*)&m->dev_out_flag[nvllm_model::kOutFlags].seq;
     memset(m->out_seq, 0, sizeof(m->out_seq));
     HIPCHK(m->ctx, hipMalloc((void**)&m->out_done, nvllm_model::kOutFlags * sizeof(unsigned)));
     HIPCHK(m->ctx, hipMemsetAsync(m->out_done, 0, nvllm_model::kOutFlags * sizeof(unsigned), m->ctx->stream));
@@ -769,6 +800,38 @@ extern "C" int64_t nvllm_model_weight_bytes(const nvllm_model* m) {
 // KV pool
 // ---------------------------------------------------------------------------------------------------
 // K/V caches, step buffers and rotation table of a Qwen3 model (pool sizes are set)
+static ResidentSizes resident_sizes(const nvllm_model* m) {
+    ResidentSizes z;
+    z.NQ = (m->nh_l + 2 * m->kv_l) * m->hd; z.KO = m->nh_l * m->hd; z.I = m->I_l; z.nh = m->nh_l; z.kv = m->kv_l; z.hd = m->hd;
+    return z;
+}
+static int resident_empty(nvllm_model* m) {
+    HIPCHK(m->ctx, hipMemsetAsync(m->resident_buffer, 0xFF, resident_buffer_words(resident_sizes(m)) * 4, m->ctx->stream));
+    HIPCHK(m->ctx, hipMemsetAsync(m->resident_gave_up, 0, 4, m->ctx->stream));
+    return NVLLM_OK;
+}
+static int resident_alloc(nvllm_model* m) {
+    nvllm_ctx* ctx = m->ctx;
+    const ResidentSizes z = resident_sizes(m);
+    m->resident_closed = false;
+    if (ctx->tp_size > 1 || !m->vlocache.empty() || !resident_sizes_ok(m->H, z) || m->L < kResidentLayers) return NVLLM_OK;
+    int cus = 0;
+    HIPCHK(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+    if (cus < kResidentGroups) return NVLLM_OK;
+    std::vector<ResidentLayer> layers(m->L);
+    for (int l = 0; l < m->L; ++l) {
+        const LayerW& w = m->layers[l];
+        layers[l] = ResidentLayer{w.qkv.data, w.o.data, w.gu.data, w.down.data, w.ln1, w.ln2, w.qn, w.kn, m->kcache[l], m->vcache[l]};
+    }
+    int rc = dmalloc(ctx, &m->d_resident_layers, layers.size());
+    if (!rc) rc = dmalloc(ctx, &m->resident_buffer, resident_buffer_words(z));
+    if (!rc) rc = dmalloc(ctx, &m->resident_gave_up, (size_t)1);
+    if (rc) return rc;
+    HIPCHK(ctx, hipMemcpyAsync(m->d_resident_layers, layers.data(), layers.size() * sizeof(ResidentLayer), hipMemcpyHostToDevice, ctx->stream));
+    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    return resident_empty(m);
+}
+
 static int qwen3_kv_alloc(nvllm_model* m) {
     nvllm_ctx* ctx = m->ctx;
     const int num_blocks = m->num_blocks, max_seqs = m->max_seqs;
@@ -826,6 +889,7 @@ static int qwen3_kv_alloc(nvllm_model* m) {
     }
     if (!rc) rc = dmalloc(ctx, &m->attn_po, (size_t)max_seqs * m->nh_l * kAttnMaxParts * m->hd);
     if (!rc) rc = dmalloc(ctx, &m->attn_pml, (size_t)max_seqs * m->nh_l * kAttnMaxParts * 2);
+    if (!rc) rc = resident_alloc(m);
     if (rc) return rc;
     // RoPE table: rotary_embedding.rs:56-80 (f32: inv_freq = 1/base^(2j/hd); angle = pos * inv_freq)
     m->rope_len = std::min(m->cfg.max_position_embeddings, m->max_blocks * kBlockTokens);
@@ -1080,6 +1144,67 @@ static bool fused_plan(const nvllm_model* m, int R, FusedPlan& p) {
     return true;
 }
 
+// LM head on the last-token rows only (gathered by row_idx), logits scaled by the final norm's rinv
+static int head_of_planes(nvllm_model* m, RowNorm rn, int n_last, int logits_row0) {
+    nvllm_ctx* ctx = m->ctx;
+    hipStream_t s = ctx->stream;
+    const int H = m->H;
+    if (n_last > 0) {
+        GemmPlan pl = plan_lmhead(n_last, m->V_l, H);
+        float* lg = m->want_logits ? m->logits + (size_t)logits_row0 * m->V_l : nullptr;
+        rn.row_idx = m->d_last_rows;
+        PROF(m, PROF_LMHEAD, launch_gemm_argmax(pl, m->xh, m->xl, H, m->lm_head, lg, n_last, m->part_val, m->part_idx, &rn, s));
+        const int tps = ctx->tp_size;  // vocab-parallel: every rank leaves (id, max) of its shard for the gather in finish_logits
+        uint32_t* ids_dst = tps == 1 ? m->d_next + logits_row0 : m->d_next + m->cur_n + (size_t)ctx->tp_rank * m->cur_n + logits_row0;
+        float* val_dst = tps == 1 ? nullptr : m->d_maxval + (size_t)ctx->tp_rank * m->cur_n + logits_row0;
+        if (!m->want_ids) return NVLLM_OK;
+        if (pl.lm_nt > 0)
+            HIPCHK(ctx, launch_argmax_rows(m->part_val, m->part_idx, gemm_argmax_parts(pl, m->V_l), n_last, ids_dst, val_dst, s));
+        else
+            HIPCHK(ctx, launch_argmax_parts(m->part_val, m->part_idx, gemm_argmax_parts(pl, m->V_l), n_last, m->argmax_scratch,
+                                            ids_dst, val_dst, s));
+    }
+    return NVLLM_OK;
+}
+
+// A decode step of one to kResidentRows rows in one launch and the head's, wherever sizes, cache and device are its own (resident_alloc).  Not where the next step is enqueued
+// before this one's results are waited for: a launch that gives up is made good by running the step again.  Nor where a part of a context would be longer than 64 tiles, 8 rows of
+// 8000 tokens, where launches are as fast.  0.6B, one step with its logits, us, as launches / resident:
+//   1 row of 137 774 / 555, of 2000 982 / 598, of 16000 1378 / 874;  2 rows of 137 850 / 635, 3 890 / 715, 4 910 / 745, 6 1011 / 920, 8 1040 / 990
+//   4 x 2000 1183 / 849, 8 x 1000 1277 / 1079, 8 x 4000 1621 / 1500, 8 x 8000 2221 / 2126
+// A context is one workgroup's up to 8 tiles (1 x 250, us: whole 548, in parts of 4 tiles 551; 8 x 250 844, 839); above, in the smallest parts that give every wave a tile and that there are
+// workgroups for (1 x 500 in parts of 4 tiles 557, of 8 590, whole 616; 8 x 500 846, 890, 930).
+static bool resident_plan(const nvllm_model* m, int R, int n_tiles, int qt, int& part_tiles, int& parts) {
+    if (!m->resident_buffer || m->resident_closed || !m->opt_resident || !m->resident_waited || qt != 1 || n_tiles != R || m->cur_n != R || R > kResidentRows || !m->decode_in_order) return false;
+    if (m->taps || m->opt_no_fused || m->opt_no_xpack || m->opt_no_attn_prologue || m->prof_kind || m->stamps_on) return false;
+    const int tiles = (m->cur_max_len + 31) / 32, most = std::min(kResidentParts, kResidentGroups / (R * m->kv_l));
+    part_tiles = tiles <= 8 ? tiles : std::max(4, (tiles + most - 1) / most);
+    parts = (tiles + part_tiles - 1) / part_tiles;
+    return part_tiles <= 64;
+}
+static int forward_resident(nvllm_model* m, int R, int part_tiles, int parts, int n_last, int logits_row0) {
+    ResidentArgs a;
+    a.layers = m->d_resident_layers; a.L = m->L; a.R = R; a.z = resident_sizes(m);
+    a.ids = m->d_ids; a.embed = m->embed; a.norm = m->norm; a.rows = m->d_decode_rows; a.block_tables = m->d_block_tables; a.max_blocks = m->max_blocks;
+    a.cos = m->cosv; a.sin = m->sinv; a.eps = (float)m->cfg.rms_norm_eps; a.q_scale = powf((float)m->hd, -0.5f) * 1.4426950408889634f;
+    a.part_tiles = part_tiles; a.parts = parts; a.buffer = m->resident_buffer; a.set = m->resident_set;
+    a.xh = m->xh; a.xl = m->xl; a.ssq = m->ssqB; a.gave_up = m->resident_gave_up; a.host_gave_up = m->dev_resident; a.spins = m->opt_resident_spins;
+    HIPCHK(m->ctx, resident_turn(m->ctx, a));
+    m->resident_set ^= 1;
+    ++m->resident_launches;
+    RowNorm rn;
+    rn.ssq = m->ssqB; rn.groups = 1; rn.stride = kFusedMaxRows; rn.inv_h = 1.0f / (float)m->H; rn.eps = a.eps;
+    return head_of_planes(m, rn, n_last, logits_row0);
+}
+// After a step's results are there: did its launch give up?  Then they are none, and the model's steps are launches from here on.
+static bool resident_gave_up(nvllm_model* m) { return m->h_resident && __atomic_load_n(m->h_resident, __ATOMIC_ACQUIRE) != 0; }
+static int resident_close(nvllm_model* m) {
+    HIPCHK(m->ctx, hipStreamSynchronize(m->ctx->stream));
+    m->resident_closed = true;
+    *m->h_resident = 0;
+    return resident_empty(m);
+}
+
 static int forward_chunk_fused(nvllm_model* m, const FusedPlan& fp, int R, int n_tiles, int qt, int n_last, int logits_row0) {
     nvllm_ctx* ctx = m->ctx;
     hipStream_t s = ctx->stream;
@@ -1285,23 +1410,7 @@ static int forward_chunk_fused(nvllm_model* m, const FusedPlan& fp, int R, int n
                                         packed && !last);  // the LM head (chunked kernel) reads row-major planes
         if (rc) return rc;
     }
-    if (n_last > 0) {
-        // LM head on the last-token rows only (gathered by row_idx), logits scaled by the final norm's rinv
-        GemmPlan pl = plan_lmhead(n_last, m->V_l, H);
-        float* lg = m->want_logits ? m->logits + (size_t)logits_row0 * m->V_l : nullptr;
-        rn.row_idx = m->d_last_rows;
-        PROF(m, PROF_LMHEAD, launch_gemm_argmax(pl, m->xh, m->xl, H, m->lm_head, lg, n_last, m->part_val, m->part_idx, &rn, s));
-        const int tps = ctx->tp_size;  // vocab-parallel: every rank leaves (id, max) of its shard for the gather in finish_logits
-        uint32_t* ids_dst = tps == 1 ? m->d_next + logits_row0 : m->d_next + m->cur_n + (size_t)ctx->tp_rank * m->cur_n + logits_row0;
-        float* val_dst = tps == 1 ? nullptr : m->d_maxval + (size_t)ctx->tp_rank * m->cur_n + logits_row0;
-        if (!m->want_ids) return NVLLM_OK;
-        if (pl.lm_nt > 0)
-            HIPCHK(ctx, launch_argmax_rows(m->part_val, m->part_idx, gemm_argmax_parts(pl, m->V_l), n_last, ids_dst, val_dst, s));
-        else
-            HIPCHK(ctx, launch_argmax_parts(m->part_val, m->part_idx, gemm_argmax_parts(pl, m->V_l), n_last, m->argmax_scratch,
-                                            ids_dst, val_dst, s));
-    }
-    return NVLLM_OK;
+    return head_of_planes(m, rn, n_last, logits_row0);
 }
 
 // y (f32 slabs) = x.W^T on the generic path: for few rows the row-parallel streaming kernel (every load of a
@@ -1345,6 +1454,8 @@ static bool tile_resid_wins(int R, int H, int KO, int I) {
 // rows R (ids/pos/slot/tiles already on the device), n_last rows listed in d_last_rows -> logits rows
 static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last, int logits_row0) {
     if (m->dec) return m->dec->forward_chunk(m, R, n_tiles, qt, n_last, logits_row0);
+    int part_tiles = 0, parts = 0;
+    if (resident_plan(m, R, n_tiles, qt, part_tiles, parts)) return forward_resident(m, R, part_tiles, parts, n_last, logits_row0);
     FusedPlan fp;
     if (fused_plan(m, R, fp)) return forward_chunk_fused(m, fp, R, n_tiles, qt, n_last, logits_row0);
     nvllm_ctx* ctx = m->ctx;
@@ -2033,6 +2144,7 @@ static int step_impl(nvllm_model* m, int n_seqs, const int64_t* seq_ids, const u
     m->want_logits = last_logits != nullptr || temperatures != nullptr || score != nullptr;  // sampling reads the last-row logits on the device
     m->want_ids = !score && !temperatures;
     m->cur_n = n_seqs;
+    m->resident_waited = true;
     m->cur_max_len = *std::max_element(lens, lens + n_seqs);
     set_attn_split(m, n_seqs, m->cur_max_len, std::accumulate(lens, lens + n_seqs, (int64_t)0));
     // rows and q-tiles
@@ -2101,26 +2213,41 @@ static int step_impl(nvllm_model* m, int n_seqs, const int64_t* seq_ids, const u
         logits_row += (int)last_local.size();
         r0 += R;
     }
-    if (temperatures) {
-        // sample_token on the device (llm_engine.rs:97-133), from the logits; no arg-max ran.  Under
-        // TP every rank draws over its vocabulary shard with the SAME random stream (indexed by global id); the best
-        // (score, id) pair wins in finish_logits exactly like the greedy (max, id) pair.
-        std::vector<uint64_t> keys(n_seqs);
-        for (int i = 0; i < n_seqs; ++i) keys[i] = sample_key(seed, seq_ids[i], lens[i]);
-        HIPCHK(ctx, hipMemcpyAsync(m->d_keys, keys.data(), (size_t)n_seqs * 8, hipMemcpyHostToDevice, ctx->stream));
-        HIPCHK(ctx, hipMemcpyAsync(m->d_temps, temperatures, (size_t)n_seqs * 4, hipMemcpyHostToDevice, ctx->stream));
-        const int tps = ctx->tp_size;
-        uint32_t* ids_dst = tps == 1 ? m->d_next : m->d_next + n_seqs + (size_t)ctx->tp_rank * n_seqs;
-        float* val_dst = tps == 1 ? nullptr : m->d_maxval + (size_t)ctx->tp_rank * n_seqs;
-        HIPCHK(ctx, launch_sample_rows(m->logits, n_seqs, m->V_l, m->V_l, m->d_temps, m->d_keys, ctx->tp_rank * m->V_l, ids_dst, val_dst, ctx->stream));
-        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));  // keys / temperatures are read from pageable host memory above
+    auto sample = [&]() -> int {
+        if (temperatures) {
+            // sample_token on the device (llm_engine.rs:97-133), from the logits; no arg-max ran.  Under
+            // TP every rank draws over its vocabulary shard with the SAME random stream (indexed by global id); the best
+            // (score, id) pair wins in finish_logits exactly like the greedy (max, id) pair.
+            std::vector<uint64_t> keys(n_seqs);
+            for (int i = 0; i < n_seqs; ++i) keys[i] = sample_key(seed, seq_ids[i], lens[i]);
+            HIPCHK(ctx, hipMemcpyAsync(m->d_keys, keys.data(), (size_t)n_seqs * 8, hipMemcpyHostToDevice, ctx->stream));
+            HIPCHK(ctx, hipMemcpyAsync(m->d_temps, temperatures, (size_t)n_seqs * 4, hipMemcpyHostToDevice, ctx->stream));
+            const int tps = ctx->tp_size;
+            uint32_t* ids_dst = tps == 1 ? m->d_next : m->d_next + n_seqs + (size_t)ctx->tp_rank * n_seqs;
+            float* val_dst = tps == 1 ? nullptr : m->d_maxval + (size_t)ctx->tp_rank * n_seqs;
+            HIPCHK(ctx, launch_sample_rows(m->logits, n_seqs, m->V_l, m->V_l, m->d_temps, m->d_keys, ctx->tp_rank * m->V_l, ids_dst, val_dst, ctx->stream));
+            HIPCHK(ctx, hipStreamSynchronize(ctx->stream));  // keys / temperatures are read from pageable host memory above
+        }
+        return NVLLM_OK;
+    };
+    // the step's results to the host
+    auto leave = [&]() -> int {
+        int rc = sample();
+        if (rc) return rc;
+        if (!score) return finish_logits(m, n_seqs, next_ids, last_logits);
+        if (!score_at_once && !head_rows.empty()) return download_logits(m, (int)head_rows.size(), score->logits);
+        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));  // (the logits are the last of the step on the stream)
+        return NVLLM_OK;
+    };
+    int rc = leave();
+    if (!rc && resident_gave_up(m)) {  // the one chunk of a decode step: its metadata is where it was
+        rc = resident_close(m);
+        if (!rc) rc = forward_chunk(m, total_rows, (int)p.tile_row0.size(), qt, (int)head_rows.size(), 0);
+        if (!rc) rc = leave();
     }
+    if (rc) return rc;
+    stage_idle(m);
     if (score) {
-        if (!score_at_once && !head_rows.empty()) {
-            const int rc = download_logits(m, (int)head_rows.size(), score->logits);
-            if (rc) return rc;
-        } else HIPCHK(ctx, hipStreamSynchronize(ctx->stream));  // (the logits are the last of the step on the stream)
-        stage_idle(m);
         const int rc_os = oneshot_check(ctx);
         if (rc_os) return rc_os;
         for (int i = 0; i < n_seqs; ++i) {
@@ -2132,9 +2259,6 @@ static int step_impl(nvllm_model* m, int n_seqs, const int64_t* seq_ids, const u
         m->decode_resident = false;
         return NVLLM_OK;
     }
-    int rc = finish_logits(m, n_seqs, next_ids, last_logits);
-    if (rc) return rc;
-    stage_idle(m);
     m->last_ids.assign(seq_ids, seq_ids + n_seqs);
     m->last_lens.assign(lens, lens + n_seqs);
     m->decode_resident = all_single && total_rows <= m->max_rows;
@@ -2151,7 +2275,7 @@ static int step_impl(nvllm_model* m, int n_seqs, const int64_t* seq_ids, const u
 }
 
 // enqueue one more decode step for the resident batch (no host sync): everything up to the device arg-max
-static int decode_core(nvllm_model* m) {
+static int decode_core(nvllm_model* m, bool waited) {
     nvllm_ctx* ctx = m->ctx;
     const int n = (int)m->last_ids.size();
     if (n == 0) return fail(ctx, NVLLM_ESTATE, "no previous step to continue");
@@ -2195,6 +2319,7 @@ static int decode_core(nvllm_model* m) {
     m->want_logits = false;
     m->want_ids = true;
     m->cur_n = n;
+    m->resident_waited = waited;
     m->cur_max_len = *std::max_element(m->last_lens.begin(), m->last_lens.end()) + 1;
     set_attn_split(m, n, m->cur_max_len, std::accumulate(m->last_lens.begin(), m->last_lens.end(), (int64_t)n));
     const bool recurrent = m->dec && m->dec->recurrent();
@@ -2220,9 +2345,16 @@ static int decode_core(nvllm_model* m) {
 extern "C" int nvllm_decode_next(nvllm_model* m, uint32_t* next_ids) {
     if (!m) return NVLLM_EINVAL;
     if (!m->pending.empty()) return fail(m->ctx, NVLLM_ESTATE, "collect the enqueued decode steps first");
-    int rc = decode_core(m);
+    int rc = decode_core(m, true);
     if (rc) return rc;
-    return finish_logits(m, (int)m->last_ids.size(), next_ids, nullptr);
+    const int n = (int)m->last_ids.size();
+    rc = finish_logits(m, n, next_ids, nullptr);
+    if (!rc && resident_gave_up(m)) {
+        rc = resident_close(m);
+        if (!rc) rc = forward_chunk(m, n, n, 1, n, 0);
+        if (!rc) rc = finish_logits(m, n, next_ids, nullptr);
+    }
+    return rc;
 }
 
 // Pipelined form: enqueue returns as soon as the step is on the stream (its ids travel to a pinned slot behind
@@ -2234,7 +2366,7 @@ extern "C" int nvllm_decode_enqueue(nvllm_model* m) {
     nvllm_ctx* ctx = m->ctx;
     const int n = (int)m->last_ids.size();
     if ((int)m->pending.size() >= kMaxPending) return fail(ctx, NVLLM_ESTATE, "too many decode steps in flight (max %d)", kMaxPending);
-    int rc = decode_core(m);
+    int rc = decode_core(m, false);
     if (rc) return rc;
     const int slot = m->pend_next, flag = nvllm_model::kOutSlots + 1 + slot;
     m->pend_next = (m->pend_next + 1) % kMaxPending;
@@ -2281,6 +2413,8 @@ extern "C" int nvllm_debug_set_option(nvllm_model* m, const char* name, int valu
     }
     if (!strcmp(name, "oneshot_skip_push")) { m->opt_oneshot_skip_push = std::max(0, value); return NVLLM_OK; }  // test hook
     if (!strcmp(name, "stage_fail")) { m->opt_stage_fail = std::max(0, value); return NVLLM_OK; }  // test hook
+    if (!strcmp(name, "resident")) { m->opt_resident = value; return NVLLM_OK; }
+    if (!strcmp(name, "resident_spins")) { m->opt_resident_spins = std::max(0, value); return NVLLM_OK; }  // test hook
     if (!strcmp(name, "no_fused")) { m->opt_no_fused = value; return NVLLM_OK; }    // decode through the generic path
     if (!strcmp(name, "no_xpack")) { m->opt_no_xpack = value; return NVLLM_OK; }    // row-major activation planes
     if (!strcmp(name, "no_rowpar")) { m->opt_no_rowpar = value; return NVLLM_OK; }  // generic path: no whole-K row-parallel GEMMs
@@ -2300,6 +2434,7 @@ extern "C" int nvllm_debug_set_option(nvllm_model* m, const char* name, int valu
 // "tile_gemm_launches" = projections this model has run on the prefill tile GEMM; "table_copies" = whole block tables sent;
 // "qk_rows16_launches" = q/k norm launches of 16 rows and a head per workgroup; "eight_wave_launches" = decode attention on eight waves; "tiles_ahead_launches" = ... with a wave's second tile asked for before the prologue;
 // "prefill_dealt_launches" = prompt attention with a q-tile to a workgroup, "prefill_dealt_tiles" = q-tiles of those; "row_sum_launches" = products of a few rows that add up the slabs of the one before;
+// "resident_launches" = decode steps in one launch;
 // "scan_gate_launches" = step sizes of a decode step's selective scan by a launch of their own; "two_product_launches" = pairs of products in one launch;
 // "row_pair_launches" = products of two row blocks at a time, of all models of the process; "tile_resid_launches" = products of a prompt chunk with
 // residual and norm preparation in their epilogue
@@ -2313,6 +2448,7 @@ extern "C" int nvllm_debug_get_counter(nvllm_model* m, const char* name, int64_t
     if (!strcmp(name, "qk_rows16_launches")) { *value = m->qk_rows16_launches; return NVLLM_OK; }
     if (!strcmp(name, "prefill_dealt_launches")) { *value = m->prefill_dealt_launches; return NVLLM_OK; }
     if (!strcmp(name, "prefill_dealt_tiles")) { *value = m->prefill_dealt_tiles; return NVLLM_OK; }
+    if (!strcmp(name, "resident_launches")) { *value = m->resident_launches; return NVLLM_OK; }
     if (!strcmp(name, "row_sum_launches")) { *value = m->row_sum_launches; return NVLLM_OK; }
     if (!strcmp(name, "scan_gate_launches")) { *value = m->scan_gate_launches; return NVLLM_OK; }
     if (!strcmp(name, "two_product_launches")) { *value = m->two_launches; return NVLLM_OK; }

@@ -14,6 +14,7 @@
 #include "../../include/nvllm_amd_debug.h"
 #include "kernels.h"
 #include "latent.h"
+#include "resident.h"
 
 using namespace nvllm;
 
@@ -50,6 +51,7 @@ struct nvllm_ctx {
     size_t os_slot = 0, os_data_bytes = 0, os_flag_bytes = 0;
     uint64_t os_calls = 0;
     OneShotPeers os_peers;
+    hipEvent_t resident_ev = nullptr;  // see resident_turn
     std::vector<void*> os_ipc;    // peer mappings opened with hipIpcOpenMemHandle
 };
 
@@ -182,6 +184,17 @@ struct nvllm_model {
     // one sequence on Qwen3-0.6B, smallest grid 192 / 128 / 64: 300 rows 3.97 / 3.93 / 3.43 ms, 512 rows 4.42 / 4.32 / 3.76, 1300 rows
     // 6.89 / 5.79 / 5.78, 2391 rows 8.65 / 7.65 / 7.65 (800 rows 4.73 / 4.35 / 4.44); four 8B layers, 257 rows 1.74 / 1.65 / 1.65
     int opt_tile_min_wgs = 64;
+    // the resident decode step (resident.hip); empty where sizes, device or cache are not its own
+    nvllm::ResidentLayer* d_resident_layers = nullptr;
+    uint32_t* resident_buffer = nullptr;
+    int* resident_gave_up = nullptr;       // device: a wait of the last launch ran out ...
+    int *h_resident = nullptr, *dev_resident = nullptr;  // ... and the same in pinned memory
+    int resident_set = 0;
+    bool resident_closed = false;          // a launch gave up: launches from then on
+    bool resident_waited = false;          // the step's results are waited for before the next one is enqueued
+    int opt_resident = 1;                  // 0: never
+    int opt_resident_spins = 1000000;      // turns of a wait, about a second
+    int64_t resident_launches = 0;
     unsigned* tickets = nullptr;             // arrival counters of the streaming GEMM's in-launch combine (zero between launches)
     float* qkv_out = nullptr;                // complete QKV sums of the streaming GEMM (its combine reads the slabs in m->slabs)
     uint32_t* d_next = nullptr;
