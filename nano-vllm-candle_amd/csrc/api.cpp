@@ -1169,9 +1169,9 @@ static int head_of_planes(nvllm_model* m, RowNorm rn, int n_last, int logits_row
 
 // A decode step of one to kResidentRows rows in one launch and the head's, wherever sizes, cache and device are its own (resident_alloc).  Not where the next step is enqueued
 // before this one's results are waited for: a launch that gives up is made good by running the step again.  Nor where a part of a context would be longer than 64 tiles, 8 rows of
-// 8000 tokens, where launches are as fast.  0.6B, one step with its logits, us, as launches / resident:
-//   1 row of 137 774 / 555, of 2000 982 / 598, of 16000 1378 / 874;  2 rows of 137 850 / 635, 3 890 / 715, 4 910 / 745, 6 1011 / 920, 8 1040 / 990
-//   4 x 2000 1183 / 849, 8 x 1000 1277 / 1079, 8 x 4000 1621 / 1500, 8 x 8000 2221 / 2126
+// 8000 tokens, where launches are nearly as fast.  0.6B, one step with its logits, us, as launches / resident:
+//   1 row of 137 774 / 542, of 2000 982 / 590, of 16000 1378 / 868;  2 rows of 137 860 / 602, 4 910 / 685, 6 1006 / 810, 8 1040 / 855
+//   4 x 2000 1183 / 793, 8 x 1000 1280 / 966, 8 x 4000 1625 / 1400, 8 x 8000 2225 / 2020
 // A context is one workgroup's up to 8 tiles (1 x 250, us: whole 548, in parts of 4 tiles 551; 8 x 250 844, 839); above, in the smallest parts that give every wave a tile and that there are
 // workgroups for (1 x 500 in parts of 4 tiles 557, of 8 590, whole 616; 8 x 500 846, 890, 930).
 static bool resident_plan(const nvllm_model* m, int R, int n_tiles, int qt, int& part_tiles, int& parts) {

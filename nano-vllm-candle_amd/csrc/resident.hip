@@ -3,13 +3,15 @@
 // As launches a layer of so few rows is five of 3.6 to 7 us for 1 us of work each: start, kernel arguments, the first loads' round trip, the end and 1.4 us to the next.
 // Here 256 workgroups, one to a CU, walk through the layers together.  What a phase leaves for the next goes through memory at device scope without flags: a place of a
 // hand-off buffer is empty (kResidentEmpty) until its value is there, and whoever needs the values reads them until none is empty.  A layer of Qwen3-0.6B with one row of 137 tokens
-// takes 16.5 us, 27 as launches: five hand-offs of 1.8 to 2.4, four products of 0.4, their sums 0.4, the attention 3.5; the weights (31.5 MB) are 6.2 of memory behind them.
+// takes 16.3 us, 27 as launches: five hand-offs of 1.8 to 2.4, four products of 0.4, their sums 0.4, the attention 3.5; the weights (31.5 MB) are 6.2 of memory behind them.
 //
 // What a hand-off costs with 256 workgroups that all read what all wrote, measured alone: 1.44 us; with a flag a workgroup, waited for before the values are read, 3.4.  And:
 //  - a wave's loads return behind its own earlier stores, which take 2 us to be there: one wave hands on and empties, others read (22 -> 20.5 us a layer);
 //  - with 8 or 32 workgroups' words to a line 2.8 to 4 us: each has lines of its own (45 -> 34 us a layer of 8 rows with its places side by side, 32 in lines of their own);
 //  - 8 MB of weights asked for at once meanwhile: 2.9 us.  They come a few at a time, and not before the hand-on is on its way (20.5 -> 16.7);
-//  - many values a reader: one of them until it is there, then all (8 rows 31.5 -> 27.5 us a layer, 4 rows 24 -> 21).
+//  - many values a reader: one of them until it is there, then all (8 rows 31.5 -> 27.5 us a layer, 4 rows 24 -> 21);
+//  - what a reader does with a value: a place within a block for each reader, of every B-th block, so that the steps from one to the next are constants of the loads and LDS
+//    writes (a step of 8 rows 983 -> 880 us, of 4 737 -> 696, of 2 635 -> 608; with the steps in registers 8 rows took 998).
 //
 // A workgroup is four row waves and four weight waves.  Weight waves hold what the workgroup needs of the weights in registers (30 KB a wave), asked for one or two phases ahead,
 // because a wave's loads return in order: a value asked for behind weights would wait for them.  Row waves wait for values, lay them into LDS as bf16 planes, run the attention, add up
@@ -33,9 +35,9 @@ namespace {
 
 constexpr int H = 1024;                       // the stream: a quad to a workgroup
 constexpr int kMaxQ = 4, kMaxO = 2, kMaxI = 3;  // NQ, KO, I in 1024ths: 8 + 4 + 12 + 6 fragments of 4 registers a lane are a layer's weights
-// Turns of 64 cycles between two weight fragments, and before the first behind a hand-on.  One row, us a step: 5 and 12 556, 2 and 12 549, 8 and 12 562, 5 and 4 573, 5 and 20 581, none
-// 640; four rows 804, 814, 798, 811, 811, 868
-constexpr int kPace = 5, kBehind = 12;
+// Turns of 64 cycles between two weight fragments, and before the first behind a hand-on.  One and eight rows of 137 tokens, us a step: 8 and 8 542, 855; 5 and 12 554, 876; 8 and 12
+// 556, 860; 8 and 5 550, 859; 8 and 2 551, 843; 5 and 5 561, 847; 11 and 5 565, 863; without a pause 640 (one row)
+constexpr int kPace = 8, kBehind = 8;
 constexpr int kSlot = 20;                     // float4 from one (quad, row)'s partial sums to the next's: 16 and 4 to be on other banks
 
 // What a workgroup hands on is a block of lines of its own: with 8 or 32 workgroups to a line a hand-on took 2 us longer.
@@ -108,7 +110,7 @@ struct Waiting {
             if (__builtin_amdgcn_ballot_w64(!read()) == 0) return !over;
             asm volatile("" ::: "memory");
             if (over) return false;
-            if (n < spins && ((n & 63) != 63 || __hip_atomic_load(gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)) continue;
+            if (n < spins && ((n & 63) != 63 || __builtin_amdgcn_readfirstlane(__hip_atomic_load(gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == 0)) continue;
             over = true;
             if ((threadIdx.x & 63) == 0) {
                 __hip_atomic_store(gave_up, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -348,81 +350,102 @@ __global__ void __launch_bounds__(512, 2) resident_step_kernel(ResidentArgs a) {
         int t = t0, lane = t0 & 63;
         asm volatile("" : "+v"(t), "+v"(lane));
         const int reader = t - 64;          // of 192
-        // four words of planes into LDS, at element `col` of a row
-        auto lay = [&](const uint4& v, int row, int col, int S) __attribute__((always_inline)) {
-            char* p = smem + row * S + col * 2;
+        // four words of planes into LDS
+        auto lay = [&](const uint4& v, char* p) __attribute__((always_inline)) {
             *reinterpret_cast<uint2*>(p) = make_uint2(__builtin_amdgcn_perm(v.y, v.x, 0x07060302), __builtin_amdgcn_perm(v.w, v.z, 0x07060302));
             *reinterpret_cast<uint2*>(p + lds.lo) = make_uint2(__builtin_amdgcn_perm(v.y, v.x, 0x05040100), __builtin_amdgcn_perm(v.w, v.z, 0x05040100));
         };
-        // NU units of 16 bytes a reader, at place(i) of `r`; past its end they are zeros
-        auto read = [&](auto& v, __amdgpu_buffer_rsrc_t r, auto place) __attribute__((always_inline)) {
+        // units of 16 bytes, v[i] at `at` + i * step of `r`, but the last one at `at_last`; past its end they are zeros.  Many: one of them until it is there, then all
+        auto read = [&](auto& v, __amdgpu_buffer_rsrc_t r, int at, int step, int at_last) __attribute__((always_inline)) {
             constexpr int NU = sizeof(v) / 16;
-            if constexpr (NU > 4) {  // one unit until it is there, then all
-                uint32_t m;
-                waiting.until([&]() __attribute__((always_inline)) {
-                    m = most(load_shared16(r, place(NU / 2)));
-                    return m != kResidentEmpty;
-                });
-            }
+            if constexpr (NU > 4)
+                waiting.until([&]() __attribute__((always_inline)) { return most(load_shared16(r, at, NU / 2 * step)) != kResidentEmpty; });
             waiting.until([&]() __attribute__((always_inline)) {
 #pragma unroll
-                for (int i = 0; i < NU; ++i) v[i] = load_shared16(r, place(i));
+                for (int i = 0; i < NU - 1; ++i) v[i] = load_shared16(r, at, i * step);
+                v[NU - 1] = load_shared16(r, at_last);
                 uint32_t m = 0;
 #pragma unroll
                 for (int i = 0; i < NU; ++i) m = max(m, most(v[i]));
                 return m != kResidentEmpty;
             });
         };
-        // the stream and its rows' sums of squares: blocks of RP + SQ units
+        constexpr int kNowhere = 0x7ffffff0;
+        // A reader has one unit of a block, of every B-th block: what is left of the readers has none.  The stream and its rows' sums of squares: blocks of RP + SQ units
         auto read_stream = [&](const uint32_t* from) __attribute__((always_inline)) {
-            constexpr int U = RP + SQ, NU = (kResidentGroups * U + 191) / 192;
+            constexpr int U = RP + SQ, B = 192 / U, NU = (kResidentGroups + B - 1) / B;
+            const int g0 = reader / U, in = reader % U, at = (g0 * kStream + in * 4) * 4, S = L::x_bytes(H);
+            const bool any = g0 < B, last = any && g0 + (NU - 1) * B < kResidentGroups;
             uint4 v[NU];
-            read(v, buffer_of(from, kStream * kResidentGroups * 4), [&](int i) { const int u = reader + 192 * i; return (u / U * kStream + u % U * 4) * 4; });
-            float4 sq[SQ];
+            read(v, buffer_of(from, kStream * kResidentGroups * 4), any ? at : 0, B * kStream * 4, last ? at + (NU - 1) * B * kStream * 4 : kNowhere);
+            float4 sq = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (in < RP && any) {
+                char* const p = smem + in * S + g0 * 8;
 #pragma unroll
-            for (int s = 0; s < SQ; ++s) sq[s] = make_float4(0.f, 0.f, 0.f, 0.f);
+                for (int i = 0; i < NU - 1; ++i) lay(v[i], p + i * B * 8);
+                if (last) lay(v[NU - 1], p + (NU - 1) * B * 8);
+            } else if (any) {
 #pragma unroll
-            for (int i = 0; i < NU; ++i) {
-                const int u = reader + 192 * i, g = u / U, in = u % U;
-                if (in < RP && g < kResidentGroups) lay(v[i], in, g * 4, L::x_bytes(H));
-#pragma unroll
-                for (int s = 0; s < SQ; ++s) {
+                for (int i = 0; i < NU; ++i) {  // (a last one that is not there is zeros)
                     const float4 f = __builtin_bit_cast(float4, v[i]);
-                    const bool is = in == RP + s;
-                    sq[s].x += is ? f.x : 0.f; sq[s].y += is ? f.y : 0.f; sq[s].z += is ? f.z : 0.f; sq[s].w += is ? f.w : 0.f;
+                    sq.x += f.x; sq.y += f.y; sq.z += f.z; sq.w += f.w;
                 }
             }
 #pragma unroll
             for (int r = 0; r < RP; ++r) {
-                const float4 f = sq[r >> 2];
-                const float sum = wave_sum_uniform((r & 3) == 0 ? f.x : (r & 3) == 1 ? f.y : (r & 3) == 2 ? f.z : f.w);
+                const float own = (r & 3) == 0 ? sq.x : (r & 3) == 1 ? sq.y : (r & 3) == 2 ? sq.z : sq.w;
+                const float sum = wave_sum_uniform(SQ == 1 || in == RP + r / 4 ? own : 0.f);
                 if (lane == 0) ssq[r * 4 + wave] = sum;
             }
         };
-        // the activations: blocks of RP x ni units; / ni by a multiplication, exact up to 32768
+        // the activations: blocks of RP x ni units
         auto read_act = [&]() __attribute__((always_inline)) {
-            constexpr int NU = kMaxI * RP * kResidentGroups / 192;
-            const int block = lines(act_words), by_ni = ni == 1 ? 65536 : ni == 2 ? 32768 : 21846;
+            constexpr int NU = 4 * RP;  // of blocks of 3 RP; those of 2 RP and RP are fewer
+            const int block = lines(act_words), B = ni == 3 ? 64 / RP : ni == 2 ? 96 / RP : 192 / RP, by_ni = ni == 1 ? 65536 : ni == 2 ? 32768 : 21846;
+            const int v_at = reader * by_ni >> 16, g0 = v_at / RP, in = reader - g0 * RP * ni, row = in * by_ni >> 16, S = L::x_bytes(ni << 10);  // (/ ni by a multiplication)
+            const int at = (g0 * block + in * 4) * 4, step = B * block * 4;
+            char* const p = smem + row * S + (g0 * ni + in - row * ni) * 8;
             uint4 v[NU];
-            read(v, buffer_of(b_act, block * kResidentGroups * 4), [&](int i) {
-                const int u = reader + 192 * i, g = (u * by_ni >> 16) / RP;
-                return RP * 4 % 32 == 0 ? u * 16 : (g * block + (u - g * RP * ni) * 4) * 4;  // (blocks that are whole lines lie in a row)
-            });
+            if (ni == 3) {  // (steps that are known here)
+                constexpr int step3 = 64 / RP * lines(RP * 12) * 4;
+                read(v, buffer_of(b_act, lines(RP * 12) * kResidentGroups * 4), at, step3, at + (NU - 1) * step3);
 #pragma unroll
-            for (int i = 0; i < NU; ++i) {
-                const int u = reader + 192 * i, g = (u * by_ni >> 16) / RP, in = u - g * RP * ni, row = in * by_ni >> 16;
-                if (g < kResidentGroups) lay(v[i], row, (g * ni + in - row * ni) * 4, L::x_bytes(ni << 10));
+                for (int i = 0; i < NU; ++i) lay(v[i], p + i * (64 / RP) * 24);
+            } else {
+                const auto r = buffer_of(b_act, block * kResidentGroups * 4);
+                waiting.until([&]() __attribute__((always_inline)) {
+                    uint32_t m = 0;
+#pragma unroll
+                    for (int i = 0; i < NU; ++i) {
+                        v[i] = load_shared16(r, g0 + i * B < kResidentGroups ? at + i * step : kNowhere);
+                        m = max(m, most(v[i]));
+                    }
+                    return m != kResidentEmpty;
+                });
+#pragma unroll
+                for (int i = 0; i < NU; ++i)
+                    if (g0 + i * B < kResidentGroups) lay(v[i], p + i * B * ni * 8);
             }
         };
-        // the attention's output: R rows of ko * 256 units
+        // the attention's output: R rows of ko * 256 units, 16 bytes of LDS between two rows
         auto read_ctx = [&]() __attribute__((always_inline)) {
             constexpr int NU = (kMaxO * RP * kResidentGroups + 191) / 192;
+            const auto r = buffer_of(b_ctx, R * ko * 4096);
             uint4 v[NU];
-            read(v, buffer_of(b_ctx, R * ko * 4096), [&](int i) { return (reader + 192 * i) * 16; });
+            auto all = [&]() __attribute__((always_inline)) {
+                uint32_t m = 0;
+#pragma unroll
+                for (int i = 0; i < NU; ++i) v[i] = load_shared16(r, (reader + 192 * i) * 16);  // (past the last row: zeros)
+#pragma unroll
+                for (int i = 0; i < NU; ++i) m = max(m, most(v[i]));
+                return m != kResidentEmpty;
+            };
+            if constexpr (NU > 4) waiting.until([&]() __attribute__((always_inline)) { return most(load_shared16(r, (reader + 192 * (NU / 2)) * 16)) != kResidentEmpty; });
+            waiting.until(all);
 #pragma unroll
             for (int i = 0; i < NU; ++i) {
                 const int u = reader + 192 * i, row = u >> (7 + ko);
-                if (row < R) lay(v[i], row, (u - (row << (7 + ko))) * 4, L::x_bytes(ko << 10));
+                if (u < R * ko * 256) lay(v[i], smem + u * 8 + row * 16);
             }
         };
         // wave 0: this lane's feature of (quad q, row), a lane of the four that add up the weight waves' partial sums and then own a feature each
@@ -465,7 +488,7 @@ __global__ void __launch_bounds__(512, 2) resident_step_kernel(ResidentArgs a) {
                 uint4 v;
                 v.x = planes_word(x[0] * n.x); v.y = planes_word(x[1] * n.y); v.z = planes_word(x[2] * n.z); v.w = planes_word(x[3] * n.w);
                 const float s = wave_sum_uniform((x[0] * x[0] + x[1] * x[1]) + (x[2] * x[2] + x[3] * x[3]));
-                lay(v, r, t * 4, L::x_bytes(H));
+                lay(v, smem + r * L::x_bytes(H) + t * 8);
                 if (lane == 0) ssq[r * 4 + wave] = s;
             }
         } else if (wave) read_stream(b_out);
