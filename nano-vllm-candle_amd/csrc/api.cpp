@@ -484,10 +484,10 @@ static void free_kv(nvllm_model* m) {
     m->kcache.clear(); m->vcache.clear(); m->vlocache.clear(); m->klocache.clear();
     void* ptrs[] = {m->d_block_tables, m->d_ids, m->d_pos, m->d_slot, m->d_tile_row0, m->d_tile_nrows, m->d_tile_slot,
                     m->d_last_rows, m->d_tile_order, m->d_prefill_tiles, m->d_decode_rows, m->resid, m->last_resid, m->slabs, m->qbuf, m->logits, m->d_maxval, m->red, m->xh, m->xl, m->xh2, m->xl2, m->ctxh, m->ctxl, m->ssqA, m->ssqB, m->ssqT, m->d_next,
-                    m->part_val, m->part_idx, m->argmax_scratch, m->attn_po, m->attn_pml, m->tap_h, m->tap_res, m->cosv, m->sinv, m->tickets, m->qkv_out, m->d_keys, m->d_temps, m->d_resident_layers, m->resident_buffer, m->resident_gave_up};
+                    m->part_val, m->part_idx, m->argmax_scratch, m->attn_po, m->attn_pml, m->attn_done, m->tap_h, m->tap_res, m->cosv, m->sinv, m->tickets, m->qkv_out, m->d_keys, m->d_temps, m->d_resident_layers, m->resident_buffer, m->resident_gave_up};
     for (void* p : ptrs) if (p) (void)hipFree(p);
     m->d_block_tables = nullptr; m->d_ids = nullptr; m->d_pos = m->d_slot = m->d_tile_row0 = m->d_tile_nrows = m->d_tile_slot = m->d_last_rows = m->d_tile_order = nullptr; m->d_prefill_tiles = nullptr; m->d_decode_rows = nullptr;
-    m->resid = m->last_resid = m->slabs = m->qbuf = m->logits = m->d_maxval = m->red = nullptr; m->xh = m->xl = m->xh2 = m->xl2 = m->ctxh = m->ctxl = nullptr; m->ssqA = m->ssqB = m->ssqT = nullptr; m->d_next = nullptr; m->part_val = nullptr; m->part_idx = nullptr; m->argmax_scratch = nullptr; m->attn_po = m->attn_pml = nullptr;
+    m->resid = m->last_resid = m->slabs = m->qbuf = m->logits = m->d_maxval = m->red = nullptr; m->xh = m->xl = m->xh2 = m->xl2 = m->ctxh = m->ctxl = nullptr; m->ssqA = m->ssqB = m->ssqT = nullptr; m->d_next = nullptr; m->part_val = nullptr; m->part_idx = nullptr; m->argmax_scratch = nullptr; m->attn_po = m->attn_pml = nullptr; m->attn_done = nullptr;
     m->tap_h = m->tap_res = nullptr; m->cosv = m->sinv = nullptr; m->tickets = nullptr; m->qkv_out = nullptr; m->d_keys = nullptr; m->d_temps = nullptr;
     m->d_resident_layers = nullptr; m->resident_buffer = nullptr; m->resident_gave_up = nullptr; m->h_resident = m->dev_resident = nullptr;
     stage_release(m);
@@ -889,6 +889,8 @@ static int qwen3_kv_alloc(nvllm_model* m) {
     }
     if (!rc) rc = dmalloc(ctx, &m->attn_po, (size_t)max_seqs * m->nh_l * kAttnMaxParts * m->hd);
     if (!rc) rc = dmalloc(ctx, &m->attn_pml, (size_t)max_seqs * m->nh_l * kAttnMaxParts * 2);
+    if (!rc) rc = dmalloc(ctx, &m->attn_done, (size_t)max_seqs * m->kv_l);
+    if (!rc) HIPCHK(ctx, hipMemsetAsync(m->attn_done, 0, (size_t)max_seqs * m->kv_l * sizeof(int), ctx->stream));
     if (!rc) rc = resident_alloc(m);
     if (rc) return rc;
     // RoPE table: rotary_embedding.rs:56-80 (f32: inv_freq = 1/base^(2j/hd); angle = pos * inv_freq)
@@ -1365,7 +1367,7 @@ static int forward_chunk_fused(nvllm_model* m, const FusedPlan& fp, int R, int n
         }
         int parts_max = 1;
         if (qt == 1 && R <= m->max_seqs) {
-            aa.part_tiles = m->attn_part_tiles; aa.max_parts = kAttnMaxParts; aa.part_o = m->attn_po; aa.part_ml = m->attn_pml;
+            aa.part_tiles = m->attn_part_tiles; aa.max_parts = kAttnMaxParts; aa.part_o = m->attn_po; aa.part_ml = m->attn_pml; aa.part_done = m->attn_done;
             parts_max = m->attn_parts_max;
             if (fuse_qk) { aa.waves = m->attn_waves; aa.ahead = m->attn_ahead; }
             m->eight_wave_launches += aa.waves == 8;
@@ -1563,7 +1565,7 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
         }
         int parts_max = 1;
         if (qt == 1 && R <= m->max_seqs) {  // decode rows: split the context over workgroups
-            aa.part_tiles = m->attn_part_tiles; aa.max_parts = kAttnMaxParts; aa.part_o = m->attn_po; aa.part_ml = m->attn_pml;
+            aa.part_tiles = m->attn_part_tiles; aa.max_parts = kAttnMaxParts; aa.part_o = m->attn_po; aa.part_ml = m->attn_pml; aa.part_done = m->attn_done;
             parts_max = m->attn_parts_max;
             if (fuse_qk) { aa.waves = m->attn_waves; aa.ahead = m->attn_ahead; }
             m->eight_wave_launches += aa.waves == 8;
@@ -1694,11 +1696,11 @@ static int ensure_blocks(nvllm_model* m, SeqState& s, int len) {
 // Eight waves of a decode attention's workgroup instead of four halve its chain of tiles, but the merge and the two waves of a SIMD cost up to 1.5 us:
 // only where launches leave a CU one workgroup at most, and not
 //  - in a 16-bit cache on whole contexts (up to 16 tiles), where four waves have all of them in flight at once;
-//  - while parts of four waves, a tile each, have a CU to themselves and are so few that the combine pass is no longer for them;
+//  - while parts of four waves, a tile each, have a CU to themselves and are so few that merging them takes no longer;
 //  - in a 24-bit cache, where parts that fit the CUs leave a quarter of them idle and the longest of ragged contexts is what the launch waits for.
 // Whole contexts of a 24-bit cache and of more than 14 query heads a group keep eight waves where tests/test_decode_waves_gpu.py has them; with a tile's arithmetic and the
 // prologue as they are four are the better there too, by 0 to 9 % (1.6 % over all 24-bit launches, 1.0 % over those of 16 heads on one).
-// Attention and its combine pass, us a layer between two events (5 of them the events'), four waves / eight; rows x tokens, 8 kv heads:
+// Attention and a combine pass of its own behind parts, us a layer between two events (5 of them the events'), four waves / eight; rows x tokens, 8 kv heads:
 //   gqa 2   whole 1 x 400 11.3 / 12.2, 8 x 400 11.8 / 13.0, 20 x 400 13.5 / 14.8, 32 x 400 16.4 / 18.5, 8 x 150..180 9.5 / 10.9
 //   gqa 4   whole 8 x 400 12.1 / 13.0, 32 x 400 15.9 / 18.2
 //   gqa 2   parts 1 x 900 13.6 / 14.4, 1 x 1500 15.2 / 15.4, 3 x 700 13.4 / 14.6, 4 x 900 15.2 / 15.4, 6 x 520..600 14.1 / 15.1, 6 x 700 16.6 / 15.4, 8 x 700 16.6 / 15.5, 32 x 1100 32.6 / 29.2
@@ -1734,8 +1736,9 @@ static void set_attn_split(nvllm_model* m, int n_seqs, int max_len, int64_t all_
     m->attn_waves = eight ? 8 : 4;
     m->attn_ahead = !eight && attn_tiles_ahead(m, base_wgs, n_seqs, all_len);
     int want = std::min(kAttnMaxParts, std::max(1, (eight ? 256 : 512) / base_wgs));
-    // a few more rounds of the loop cost less than the combine launch and its boundary (4.7 + 1.4 us): up to 512 tokens, and up to 1024 where
-    // there would be two parts at most (16 rows of 100 to 800, in parts 17.5 us, whole 16.4; one row of 900 12.3 and 16.9)
+    // A few more rounds of the loop cost less than a prologue a part and the merge: up to 512 tokens, and up to 1024 where there would be two parts at most.  Steps of 0.6B, us, whole contexts up to
+    // 512 (of eight waves from 128 workgroups on 1024) tokens / up to 256: 9 x 300 932 / 966, 9 x 400 to 500 964 / 1023, 16 x 500 996 / 1072, 24 x 48 to 400 1017 / 1106, 32 x 500 1146 / 1250, but
+    // 16 x 100 to 1000 1148 / 1120; two parts for 96 to 255 workgroups of eight waves: 16 x 100 to 1000 1254, 24 x 256 to 2048 1508 / 1492, 24 x 700 1180 / 1415
     if (tiles <= (eight && base_wgs >= 128 ? 32 : 16)) want = 1;
     int part = std::max(eight ? 8 : 4, (tiles + want - 1) / want);  // a tile of every wave at least
     m->attn_part_tiles = part;

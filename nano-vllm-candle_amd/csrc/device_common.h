@@ -124,6 +124,22 @@ __device__ __forceinline__ uint4 buffer_stream16(__amdgpu_buffer_rsrc_t r, int o
     return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, offset, uniform_offset, 2));
 }
 
+// between workgroups of one launch: past the L2s, which are an XCD's own
+__device__ __forceinline__ void hand_on(uint32_t* p, uint32_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ void hand_on8(uint32_t* p, uint32_t v, uint32_t w) {
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(p), (uint64_t)w << 32 | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void hand_on16(uint32_t* p, uint32_t v0, uint32_t v1, uint32_t v2, uint32_t v3) {
+    hand_on8(p, v0, v1);
+    hand_on8(p + 2, v2, v3);
+}
+__device__ __forceinline__ uint4 load_shared16(__amdgpu_buffer_rsrc_t r, int offset, int uniform_offset = 0) {
+    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(r, offset, uniform_offset, 16));  // sc1: at device scope
+}
+__device__ __forceinline__ uint2 load_shared8(__amdgpu_buffer_rsrc_t r, int offset) {
+    return __builtin_bit_cast(uint2, __builtin_amdgcn_raw_buffer_load_b64(r, offset, 0, 16));
+}
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);

@@ -321,12 +321,13 @@ struct AttnArgs {
     const float* sin = nullptr;
     float eps = 1e-6f, q_scale = 1.f;
     RowNorm rn;                        // deferred input norm for the fused prologue
-    // split-KV (decode): each workgroup covers part_tiles 32-token tiles; partials merged by a combine pass
+    // split-KV (decode): each workgroup covers part_tiles 32-token tiles; partials merged by the part that ends last (with qkv) or a combine pass
     int part_tiles = 0, max_parts = 0;
     int waves = 4;                     // of a workgroup; 8 with qkv and head_dim 128 only
     bool ahead = false;                // a wave's second tile asked for before the prologue: with qkv, head_dim 128, four waves and a 16-bit cache only
     float* part_o = nullptr;           // [rows][nh_l][max_parts][hd]
     float* part_ml = nullptr;          // [rows][nh_l][max_parts][2]
+    int* part_done = nullptr;          // with qkv: [rows][kv_l] parts that have ended, 0 between launches
 #ifdef NVLLM_STAMPS
     unsigned long long* stamps = nullptr;  // diagnostic build only: [workgroup][16 waves][8] s_memrealtime stamps
 #endif

@@ -2604,6 +2604,19 @@ __device__ __forceinline__ void attn_paged_body(const AttnArgs& a) {
         for (int d = 0; d < DT; ++d) obuf[(wave * cols + l15) * OS + d * 4 + grp] = w.o[0][d];
     }
     __syncthreads();
+    auto finish = [&](int row, int head, int d4, const f32x4& acc, float ltot) __attribute__((always_inline)) {
+        const float inv = 1.0f / ltot;
+        const float y0 = acc[0] * inv, y1 = acc[1] * inv, y2 = acc[2] * inv, y3 = acc[3] * inv;
+        const size_t base = (size_t)row * ldq + (size_t)head * HD + d4 * 4;
+        if (a.out_f32) *reinterpret_cast<float4*>(a.out_f32 + base) = make_float4(y0, y1, y2, y3);
+        if (a.out_hi) {
+            uint16_t h0, h1, h2, h3, l0, l1, l2, l3;
+            split_bf16(y0, h0, l0); split_bf16(y1, h1, l1); split_bf16(y2, h2, l2); split_bf16(y3, h3, l3);
+            const size_t xo = a.out_packed ? xpack_off(row, head * HD + d4 * 4, ldq >> 5) : base;
+            *reinterpret_cast<uint2*>(a.out_hi + xo) = make_uint2(h0 | ((uint32_t)h1 << 16), h2 | ((uint32_t)h3 << 16));
+            *reinterpret_cast<uint2*>(a.out_lo + xo) = make_uint2(l0 | ((uint32_t)l1 << 16), l2 | ((uint32_t)l3 << 16));
+        }
+    };
     const int n_parts = a.part_tiles ? (n_kv_tiles + a.part_tiles - 1) / a.part_tiles : 1;
     for (int i = threadIdx.x; i < cols * (HD / 4); i += NWV * 64) {
         const int col = i / (HD / 4), d4 = i % (HD / 4), tok = FUSED ? 0 : col / gqa;
@@ -2622,25 +2635,64 @@ __device__ __forceinline__ void attn_paged_body(const AttnArgs& a) {
             acc[0] += v[0] * f; acc[1] += v[1] * f; acc[2] += v[2] * f; acc[3] += v[3] * f;
         }
         if (n_parts > 1) {
-            // partial: O (at the workgroup's max) for the combine kernel
+            // partial: O (at the workgroup's max) for whoever merges the parts
             const size_t part = ((size_t)row * a.nh_l + head) * a.max_parts + blockIdx.z;
-            *reinterpret_cast<float4*>(a.part_o + part * HD + d4 * 4) = make_float4(acc[0], acc[1], acc[2], acc[3]);
-            if (d4 == 0) {
-                a.part_ml[part * 2] = ms;
-                a.part_ml[part * 2 + 1] = ltot;
+            float *const to = a.part_o + part * HD + d4 * 4, *const to_ml = a.part_ml + part * 2;
+            if constexpr (FUSED) {
+                auto word = [](float v) { return __builtin_bit_cast(uint32_t, v); };
+                hand_on16(reinterpret_cast<uint32_t*>(to), word(acc[0]), word(acc[1]), word(acc[2]), word(acc[3]));
+                if (d4 == 0) hand_on8(reinterpret_cast<uint32_t*>(to_ml), word(ms), word(ltot));
+            } else {
+                *reinterpret_cast<float4*>(to) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+                if (d4 == 0) { to_ml[0] = ms; to_ml[1] = ltot; }
             }
             continue;
         }
-        const float inv = 1.0f / ltot;
-        const float y0 = acc[0] * inv, y1 = acc[1] * inv, y2 = acc[2] * inv, y3 = acc[3] * inv;
-        const size_t base = (size_t)row * ldq + (size_t)head * HD + d4 * 4;
-        if (a.out_f32) *reinterpret_cast<float4*>(a.out_f32 + base) = make_float4(y0, y1, y2, y3);
-        if (a.out_hi) {
-            uint16_t h0, h1, h2, h3, l0, l1, l2, l3;
-            split_bf16(y0, h0, l0); split_bf16(y1, h1, l1); split_bf16(y2, h2, l2); split_bf16(y3, h3, l3);
-            const size_t xo = a.out_packed ? xpack_off(row, head * HD + d4 * 4, ldq >> 5) : base;
-            *reinterpret_cast<uint2*>(a.out_hi + xo) = make_uint2(h0 | ((uint32_t)h1 << 16), h2 | ((uint32_t)h3 << 16));
-            *reinterpret_cast<uint2*>(a.out_lo + xo) = make_uint2(l0 | ((uint32_t)l1 << 16), l2 | ((uint32_t)l3 << 16));
+        finish(row, head, d4, acc, ltot);
+    }
+    if constexpr (FUSED) {
+        if (n_parts > 1) {
+            // The part that ends last merges them, in their order: which one it is changes nothing.  Parts are handed on past the L2s, each wave waits for its own stores and the barrier for
+            // the waves, so that who counts n_parts - 1 others can read them.  As a launch of its own behind this one, steps of 0.6B: 9 rows of 600 tokens 1065 us, now 1031, 10 of 100 to 1000
+            // 1086 and 1053, 16 of 1500 1340 and 1306; four layers of 8B, 1 x 3000 698 and 689, 8 x 100 to 1500 754 and 748.
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            int* const seen = reinterpret_cast<int*>(smem_raw);  // (ml and obuf are read)
+            if (threadIdx.x == 0) *seen = __hip_atomic_fetch_add(a.part_done + (size_t)row0 * a.kv.kv_l + kh, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __syncthreads();
+            if (*seen != n_parts - 1) return;
+            if (threadIdx.x == 0) __hip_atomic_store(a.part_done + (size_t)row0 * a.kv.kv_l + kh, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            for (int i = threadIdx.x; i < cols * (HD / 4); i += NWV * 64) {
+                const int col = i / (HD / 4), d4 = i % (HD / 4), head = kh * gqa + col;
+                const size_t part = ((size_t)row0 * a.nh_l + head) * a.max_parts;
+                const auto ro = buffer_of(a.part_o + part * HD, n_parts * HD * 4), rm = buffer_of(a.part_ml + part * 2, n_parts * 8);
+                float ms = -1e30f, ltot = 0.f;
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+                constexpr int B = 8;  // parts at a time
+                for (int s0 = 0; s0 < n_parts; s0 += B) {
+                    float2 pm[B];
+                    float4 po[B];
+#pragma unroll
+                    for (int s = 0; s < B; ++s) {  // (past the last one: zeros, which count nothing)
+                        pm[s] = __builtin_bit_cast(float2, load_shared8(rm, (s0 + s) * 8));
+                        po[s] = __builtin_bit_cast(float4, load_shared16(ro, ((s0 + s) * HD + d4 * 4) * 4));
+                    }
+                    float to = ms;
+#pragma unroll
+                    for (int s = 0; s < B; ++s) to = s0 + s < n_parts ? fmaxf(to, pm[s].x) : to;
+                    const float f0 = exp2f(ms - to);
+                    ms = to;
+                    ltot *= f0;
+                    acc[0] *= f0; acc[1] *= f0; acc[2] *= f0; acc[3] *= f0;
+#pragma unroll
+                    for (int s = 0; s < B; ++s) {
+                        const float f = s0 + s < n_parts ? exp2f(pm[s].x - ms) : 0.f;
+                        ltot += pm[s].y * f;
+                        acc[0] += po[s].x * f; acc[1] += po[s].y * f; acc[2] += po[s].z * f; acc[3] += po[s].w * f;
+                    }
+                }
+                finish(row0, head, d4, acc, ltot);
+            }
         }
     }
     NVLLM_STAMP(a, 4);
@@ -3124,17 +3176,17 @@ hipError_t launch_attn_prefill(const AttnArgs& a, int n_tiles, hipStream_t s) {
     return two ? attn_prefill_launch<64, 2>(a, groups, s) : attn_prefill_launch<64, 1>(a, groups, s);
 }
 
-// rows: number of q rows (needed by the combine pass); n_parts_max: ceil(max context tiles / part_tiles)
+// rows: number of q rows (needed by the combine pass, which the fused form has no need of); n_parts_max: ceil(max context tiles / part_tiles)
 hipError_t launch_attn_paged(const AttnArgs& a, int n_tiles, int rows, int n_parts_max, hipStream_t s) {
     if (n_tiles <= 0) return hipSuccess;
     if (a.gqa < 1 || a.gqa > 16) return hipErrorInvalidValue;
     const bool split = a.part_tiles > 0 && n_parts_max > 1;
-    if (split && (!a.part_o || !a.part_ml || n_parts_max > a.max_parts)) return hipErrorInvalidValue;
+    const bool fused = a.qkv != nullptr;  // decode rows straight from the QKV GEMM's slabs
+    if (split && (!a.part_o || !a.part_ml || n_parts_max > a.max_parts || (fused && !a.part_done))) return hipErrorInvalidValue;
     AttnArgs b = a;
     if (!split) b.part_tiles = 0;
     const int gz = split ? n_parts_max : 1;
     hipError_t e = hipErrorInvalidValue;
-    const bool fused = a.qkv != nullptr;  // decode rows straight from the QKV GEMM's slabs
     if (fused && (!a.rows || n_tiles != rows || rows > kAttnFusedMaxRows)) return hipErrorInvalidValue;  // fused decode: tile i is row i
     if (a.waves != 4 && (a.waves != 8 || !fused || a.kv.hd != 128)) return hipErrorInvalidValue;
     if (a.ahead && (!fused || a.kv.hd != 128 || a.waves != 4 || a.kv.vlo)) return hipErrorInvalidValue;
@@ -3142,7 +3194,7 @@ hipError_t launch_attn_paged(const AttnArgs& a, int n_tiles, int rows, int n_par
     else if (a.ahead) e = attn_launch_v<128, 4, true, 0, true>(b, n_tiles, gz, s);
     else if (a.kv.hd == 128) e = fused ? attn_launch_t<128, 4, true>(b, n_tiles, gz, s) : attn_launch_t<128, 4, false>(b, n_tiles, gz, s);
     else if (a.kv.hd == 64) e = fused ? attn_launch_t<64, 4, true>(b, n_tiles, gz, s) : attn_launch_t<64, 4, false>(b, n_tiles, gz, s);
-    if (e != hipSuccess || !split) return e;
+    if (e != hipSuccess || !split || fused) return e;
     const int items = rows * a.nh_l;
     if (a.kv.hd == 128) attn_combine_kernel<128><<<(items + 3) / 4, 256, 0, s>>>(b, rows);
     else attn_combine_kernel<64><<<(items + 3) / 4, 256, 0, s>>>(b, rows);

@@ -199,6 +199,7 @@ struct nvllm_model {
     float* qkv_out = nullptr;                // complete QKV sums of the streaming GEMM (its combine reads the slabs in m->slabs)
     uint32_t* d_next = nullptr;
     float *attn_po = nullptr, *attn_pml = nullptr;  // split-KV partials [max_seqs][nh_l][kAttnMaxParts][hd] / [..][2]
+    int* attn_done = nullptr;                       // [max_seqs][kv_l]: their parts that have ended, 0 between launches
     int attn_part_tiles = 4, attn_parts_max = 1, attn_waves = 4;   // this step's split geometry and waves of a workgroup (decode only)
     bool attn_ahead = false;  // ... and AttnArgs::ahead
     float* part_val = nullptr;  // fused LM-head arg-max partials [V_l/16][max_seqs]
