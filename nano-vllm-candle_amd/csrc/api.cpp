@@ -1098,6 +1098,17 @@ static int tp_reduce(nvllm_model* m, int rows, int chunk, int ns, const float** 
 // the matching in-launch-combine epilogue (stream_gemm.hip: 17..64 rows), else -- where slabs are acceptable -- the
 // generic kernel.  fused_plan() says whether every GEMM of the layer has such a form at this row count.
 // ---------------------------------------------------------------------------------------------------
+// Does this product of R rows stream?  (Up to 16 of them on one GPU; the shards' products are measured from 17 on.)  Three layers, 32768 tokens, a step, us, by rows and generic products / streamed at 1, 8
+// and 16 rows: 8B 403 435 499 / 352 356 367, width 5120 with 17408 525 530 576 / 520 515 528, with 25600 731 733 787 / 654 669 669.
+bool gemm_streams(const nvllm_model* m, const PackedW& w, int R) {
+    const int ss = gemm_stream_splits(R, w.N, w.K);
+    return ss > 0 && (size_t)ss * R * w.N <= m->slab_floats && (R > 16 || m->ctx->tp_size == 1);
+}
+static bool all_stream(const nvllm_model* m, int R) {
+    if (m->layers.empty() || m->I_l % 32) return false;
+    const LayerW& w = m->layers[0];
+    return gemm_streams(m, w.qkv, R) && gemm_streams(m, w.o, R) && gemm_streams(m, w.gu, R) && gemm_streams(m, w.down, R);
+}
 enum { G_NONE = 0, G_ROW, G_STREAM, G_GENERIC };
 struct FusedPlan {
     int qkv = G_NONE, o = G_NONE, gu = G_NONE, down = G_NONE;
@@ -1137,7 +1148,7 @@ static bool fused_plan(const nvllm_model* m, int R, FusedPlan& p) {
     if (tp && (p.o == G_GENERIC || p.down == G_GENERIC)) return false;
     if (gemm_rowpar_ok(I2, H, 1, R)) p.gu = G_ROW;
     else if (fits(I2, H, 2)) p.gu = G_STREAM;
-    else if (gemm_stream_splits(R, I2, H) > 0) return false;  // big gate/up: streaming slabs + SiLU launch beat the unsplit generic kernel
+    else if (R > 16 && gemm_streams(m, m->layers[0].gu, R)) return false;  // big gate/up: streaming slabs + SiLU launch beat the unsplit generic kernel
     else p.gu = G_GENERIC;  // generic kernel with the SwiGLU epilogue (no K split)
     const bool no_xpack = m->opt_no_xpack != 0;
     auto takes_packed = [&](int kind, int N, int K, int epi) { return kind == G_STREAM || (kind == G_ROW && gemm_rowdir_ok(N, K, epi, R)); };
@@ -1417,10 +1428,6 @@ static int forward_chunk_fused(nvllm_model* m, const FusedPlan& fp, int R, int n
 
 // y (f32 slabs) = x.W^T on the generic path: for few rows the row-parallel streaming kernel (every load of a
 // workgroup issued up front) beats the chunked kernel on big matrices; otherwise the chunked kernel.
-static bool gemm_streams(const nvllm_model* m, const PackedW& w, int R) {
-    const int ss = gemm_stream_splits(R, w.N, w.K);
-    return ss > 0 && (size_t)ss * R * w.N <= m->slab_floats;
-}
 int gemm_slabs(nvllm_model* m, const bf16_bits* xh, const bf16_bits* xl, int ldx, const PackedW& w, float* out, int R,
                       int max_split, int* n_slabs, int x_packed) {
     nvllm_ctx* ctx = m->ctx;
@@ -1473,8 +1480,7 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
     // big-model decode: when all four projections of a layer run the streaming GEMM, the activation planes between
     // the row kernels and the GEMMs stay in MFMA fragment order (xpack_off): x staging costs 3x per byte otherwise
     const bool no_xpack = m->opt_no_xpack != 0;
-    const int packed = !no_xpack && !m->layers.empty() && gemm_streams(m, m->layers[0].qkv, R) && gemm_streams(m, m->layers[0].o, R) &&
-                       gemm_streams(m, m->layers[0].gu, R) && gemm_streams(m, m->layers[0].down, R) && m->I_l % 32 == 0;
+    const int packed = !no_xpack && all_stream(m, R);
     // prompt chunks (MFMA-bound): projections whose grid fills the chip run the tile GEMM (tile_gemm.hip); it reads both
     // operands in fragment order, so the kernel that produces its input planes writes them that way
     const int KO = m->nh_l * hd;

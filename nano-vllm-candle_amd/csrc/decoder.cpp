@@ -4,6 +4,10 @@
 
 #include <algorithm>
 
+// Up to 16 rows a short K is the row kernels', whose activation needs no launch of its own.  A product of 1 / 16 rows, us, streamed and by rows: 9216 x 2048 9.9 / 10.4 and 11.0 / 13.2, 16384 x 1024
+// 9.4 / 9.7 and 8.6 / 9.7; 9216 x 3072 13.3 / 14.2 and 17.3 / 25.0, 6144 x 4096 11.5 / 12.7 and 15.3 / 25.1, 24576 x 4096 34 / 37 and 50 / 62.  A step of layers 4096 wide, us, 1, 8 and 16 rows, before
+// and with it: three of gopunex 494 538 570 and 409 424 445, two of berevik 317 347 369 and 290 291 300, two scans of tafopel 378 417 448 and 329 345 356.
+static bool row_wins(const PackedW& w, int epi, int R) { return R <= 16 && w.K <= 2048 && gemm_rowpar_ok(w.N, w.K, epi, R); }
 // y = x.W^T left as f32 slabs
 ProductPlan plan_product(const nvllm_model* m, int R, const PackedW& w) {
     ProductPlan p;
@@ -14,8 +18,7 @@ ProductPlan plan_product(const nvllm_model* m, int R, const PackedW& w) {
         const int ks = gemm_tile_splits(R, w.N, w.K, tmin, std::min(p.max_split, R <= 512 ? 8 : 4));
         if (ks > 0) { p.kind = P_TILE; p.packed = 1; p.max_split = std::min(p.max_split, R <= 512 ? 8 : 4); return p; }
     }
-    const int ss = gemm_stream_splits(R, w.N, w.K);
-    if (ss > 0 && (size_t)ss * one <= m->slab_floats) { p.kind = P_STREAM; p.packed = 1; return p; }
+    if (gemm_streams(m, w, R) && !row_wins(w, 2, R)) { p.kind = P_STREAM; p.packed = 1; return p; }
     if (R <= kRowMaxRows && gemm_rowpar_ok(w.N, w.K, 2, R) && (size_t)gemm_rowpar_splits(w.N, w.K, 2, R) * one <= m->slab_floats) {
         p.kind = P_ROW;
         p.packed = R >= kPackedMinRows && gemm_rowdir_ok(w.N, w.K, 2, R);
@@ -64,7 +67,7 @@ GluPlan plan_glu(const nvllm_model* m, int R, const PackedW& w, bool want_packed
     GluPlan g;
     const int tmin = m->opt_tile_min_wgs;
     if (tmin > 0 && R > kRowMaxRows && gemm_tile_ok(R, w.N, w.K, 2, tmin)) { g.kind = P_TILE; g.packed = 1; g.out_packed_ok = 1; return g; }
-    if (R <= kRowMaxRows && gemm_rowpar_ok(w.N, w.K, 1, R)) {
+    if (R <= kRowMaxRows && gemm_rowpar_ok(w.N, w.K, 1, R) && !(R <= 16 && gemm_streams(m, w, R) && !row_wins(w, 1, R))) {
         g.kind = P_ROW;
         const bool dir = gemm_rowdir_ok(w.N, w.K, 1, R);
         g.packed = R >= kPackedMinRows && dir;

@@ -87,7 +87,7 @@ struct GemmPlan {
     int lm_nt = 0;       // > 0: launch_gemm_argmax runs the streaming LM-head kernel with lm_nt n-tiles per wave
 };
 GemmPlan plan_gemm(int M, int N, int K, int max_split);  // K % 128 == 0 required
-// streaming GEMM for big decode matrices (>= 24 MB, 17..64 rows): f32 slabs out[gemm_stream_splits][M][N];
+// streaming GEMM for big decode matrices (>= 24 MB, up to 64 rows): f32 slabs out[gemm_stream_splits][M][N];
 // gemm_stream_splits == 0 -> shape not covered (use launch_gemm / launch_gemm_rowpar)
 int gemm_stream_splits(int M, int N, int K);
 // x_packed: the planes are in xpack_off order (ldx = K either way)

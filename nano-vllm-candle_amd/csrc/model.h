@@ -303,6 +303,7 @@ inline bool last_rows_alone(const nvllm_model* m, int R, int n_last) {
 inline size_t last_rows_cap(const nvllm_model* m) { return std::min((size_t)m->max_seqs, (size_t)m->max_rows / 2 + 1); }
 
 // y (f32 slabs) = x.W^T with the kernel that fits the row count (api.cpp)
+bool gemm_streams(const nvllm_model* m, const PackedW& w, int R);
 int gemm_slabs(nvllm_model* m, const bf16_bits* xh, const bf16_bits* xl, int ldx, const PackedW& w, float* out, int R,
                int max_split, int* n_slabs, int x_packed = 0);
 uint16_t host_f32_to_bf16(float f);

@@ -1,5 +1,5 @@
 // Streaming GEMM of the decode path for matrices too big (or too oddly shaped) for the whole-K register-direct kernel:
-// Qwen3-8B / 32B layers, tensor-parallel shards.  y[M][N] = x[M][K] . W[N][K]^T for 17..64 rows
+// Qwen3-8B / 32B layers, tensor-parallel shards.  y[M][N] = x[M][K] . W[N][K]^T for up to 64 rows
 // (replaces candle_nn::Linear::forward, src/layers/linear.rs:35-36,72-77,184-198; src/models/qwen3.rs:205,278,324,326).
 //
 // One workgroup of 8 waves per (n-group, K slice): a wave owns NT n-tiles over its slice and keeps two SC-k-tile weight
@@ -322,8 +322,11 @@ __global__ void __launch_bounds__(NW * 64) gemm_stream_kernel(StreamArgs a, cons
 struct StreamShape { int nt, ks, kc, nw; };
 static StreamShape stream_shape(int M, int N, int K, int epi, bool any_size) {
     StreamShape none{0, 0, 0, 8};
-    if (M <= 16 || M > 64 || N % 16 || K % 32) return none;
-    if (!any_size && (size_t)N * K * 2 < ((size_t)24 << 20)) return none;  // small matrices: whole-K kernels when they apply
+    if (M < (epi == 0 ? 1 : 17) || M > 64 || N % 16 || K % 32) return none;
+    // small matrices: whole-K kernels when they apply.  Up to 16 rows these, and the generic kernel, lose less: 1 and 16 rows, us, streamed / not, 6144 x 2560 8.8 9.4 / 8.5 10.0, 1024 x 16384 12.5 13.6 /
+    // 10.3 11.8, 3072 x 8192 11.6 12.4 / 11.4 12.8, 2048 x 9216 10.6 11.5 / 11.4 12.9 and as much more in the sum of its 12 slabs; 4096 x 4096 9.3 9.6 / 9.7 14.6, 4096 x 12288 20.3 21.9 / 26.5 30.2
+    if (!any_size && (size_t)N * K * 2 < ((size_t)(M <= 16 ? 32 : 24) << 20)) return none;
+    if (!any_size && M <= 16 && N < 4096) return none;
     if (epi == 2 && (N / 16) % 2) return none;
     const int KT = K / 32, ntiles = N / 16;
     StreamShape best = none;
