@@ -1378,12 +1378,14 @@ __global__ void __launch_bounds__(1024) gemm_rowdir_two_kernel(RowParArgs a, con
     else rowdir_body<NTB, 16, TKB, 2, false>(b, wb, NB, 16 * TKB, (int)blockIdx.x - groups_a);
 }
 
-// Register-direct products of 65 to 256 rows: RB row blocks at a time (blocks z, z + gz, ... of blockIdx.z = z), K split over NWK waves, the
+// Register-direct products of 65 to 480 rows: RB row blocks at a time (blocks z, z + gz, ... of blockIdx.z = z), K split over NWK waves, the
 // weights kept.  Bound by what a CU takes in (x and W of its workgroup, 0.4 to 0.6 MB) and by the phases of a round: products, K slices to
 // LDS, their sums, the epilogue.  Eight waves instead of sixteen halve the slices and have registers for two blocks, so that a round's phases
 // serve 32 rows; gate and up of a feature meet in one wave; two n-tiles of o and down halve the rows a workgroup takes in.  0.6B, us a launch,
 // the 16-wave loop / this: 200 rows q/k/v 10.0 / 8.8, gate/up 15.0 / 12.4, o and down 12.5 / 9.6 each; 117 rows gate/up 11.6 / 9.8, o and down
 // 8.6 / 7.6; 250 rows 10.4 / 9.2, 15.5 / 12.7, 12.9 / 10.1.
+// Past 256 rows a round more to every 128 rows, against tile products with K slices, whose slabs are launches more, and which fill and drain a CU for a few stages: up to where o and down are one
+// launch each as tiles too (tile_resid_kernel).  A prompt of 0.6B, ms, tile products / these: 257 tokens 2.63 / 1.94, 300 2.67 / 1.98, 384 2.84 / 2.04, 480 2.88 / 2.34; a step of 257 rows 3.30 / 2.49.
 template <int NT, int NWK, int TK, int RB, int EPI>
 __global__ void __launch_bounds__(NWK * 64) gemm_rowpair_kernel(RowParArgs a, const uint4* __restrict__ wp, int N, int KT) {
     constexpr int NR = 16, PER = EPI == 1 ? 2 : 1, UNITS = RB * NT / PER, UPW = (UNITS + NWK - 1) / NWK;  // a unit: a row block's n-tile, or its gate and up
@@ -1522,39 +1524,44 @@ static hipError_t rowpair_launch(const RowParArgs& a, const PackedW& w, hipStrea
     g_rowpair_launches.fetch_add(1, std::memory_order_relaxed);
     return hipGetLastError();
 }
-// 65 to 256 rows of packed planes whose shape has an instance, else hipErrorNotReady.  Up to 64 rows every workgroup has one block: the
+// Products of 65 to kRowPairRows rows of packed planes whose shape has an instance (else hipErrorNotReady).  Up to 64 rows every workgroup has one block: the
 // 16-wave forms below are as fast or faster there (64 rows, gate/up 8.1 us against 10.6, o 4.8 against 5.6).  So they are, for q/k/v and gate/up,
 // while the grid gives every block its own workgroup, whose second block would be nothing, and for 5 blocks on two workgroups.  A product's time by
 // this less the 16-wave form's, us, at 5 to 16 blocks of 1024-wide rows:
 //   q/k/v    1536 features +0.5 to +0.9 up to 10 blocks, -0.3 to -0.7 above; 2048 +0.4 to +0.8 up to 8, -0.3 to -0.9; 2560 +0.9 +0.4 up to 6, -0.9 to
 //            +0.1; 3072 +0.5 at 5, -1.9 to +0.3; 4096 -1.3 to 0.0; 5120 -4.7 to +0.1; 6144 +0.9 at 5, -4.8 to +0.1
 //   gate/up  1536 +0.8 to +1.2, 3072 +0.8 to +1.5 (both up to 8); 4608 +1.4 at 5, -0.8 to -1.1; 6144 -2.5 to -0.4; 9216 +0.9 at 5, -0.6 to -3.9
-template <int EPI>
-static hipError_t rowpair_dispatch(const RowParArgs& a, const PackedW& w, hipStream_t s) {
-    if (a.M <= 64 || a.M > 256 || !a.x_packed) return hipErrorNotReady;
-    [[maybe_unused]] auto pairs = [&](int nt) {  // row blocks for two at a time
-        const int blocks = (a.M + 15) / 16, room = 256 / (w.N / 16 / nt);
+static bool rowpair_ok(int N, int K, int epi, int M) {
+    if (M <= 64 || M > kRowPairRows) return false;
+    auto pairs = [&](int nt) {  // row blocks for two at a time
+        const int blocks = (M + 15) / 16, room = 256 / (N / 16 / nt);
         return blocks > room && !(room <= 2 && blocks <= 5);
     };
-    if constexpr (EPI == 0) {  // up to 64 tiles: each leaves its own group of the next norm's sum, as the 16-wave form's workgroups do
-        if (w.N % 32 || w.N > 1024) return hipErrorNotReady;
+    // epilogue 0, up to 64 tiles: each leaves its own group of the next norm's sum, as the 16-wave form's workgroups do
+    if (epi == 0) return N % 32 == 0 && N <= 1024 && (K == 1024 || K == 2048 || K == 3072);
+    if (epi == 1) return K == 1024 && N % 96 == 0 && pairs(6);
+    return epi == 2 && K == 1024 && N % 64 == 0 && pairs(4);
+}
+template <int EPI>
+static hipError_t rowpair_dispatch(const RowParArgs& a, const PackedW& w, hipStream_t s) {
+    if (!a.x_packed || !rowpair_ok(w.N, w.K, EPI, a.M)) return hipErrorNotReady;
+    if constexpr (EPI == 0) {
         const bool one = (a.M + 15) / 16 <= 256 / (w.N / 32);  // a block to a workgroup
         if (w.K == 1024) return one ? rowpair_launch<2, 8, 4, 1, 0>(a, w, s) : rowpair_launch<2, 8, 4, 2, 0>(a, w, s);
         if (w.K == 2048) return one ? rowpair_launch<2, 8, 8, 1, 0>(a, w, s) : rowpair_launch<2, 8, 8, 2, 0>(a, w, s);
-        if (w.K == 3072) return rowpair_launch<2, 8, 12, 1, 0>(a, w, s);
+        return rowpair_launch<2, 8, 12, 1, 0>(a, w, s);
     } else if constexpr (EPI == 1) {
-        if (w.K == 1024 && w.N % 96 == 0 && pairs(6)) return rowpair_launch<6, 8, 4, 2, 1>(a, w, s);
-    } else if constexpr (EPI == 2) {
-        if (w.K == 1024 && w.N % 64 == 0 && pairs(4)) return rowpair_launch<4, 8, 4, 2, 2>(a, w, s);
+        return rowpair_launch<6, 8, 4, 2, 1>(a, w, s);
+    } else {
+        return rowpair_launch<4, 8, 4, 2, 2>(a, w, s);
     }
-    return hipErrorNotReady;
 }
 
 // shape of the register-direct kernel for (N, K, epi, M): nt == 0 -> not applicable
 struct RowDirShape { int nt, nwk, tk; };
 static RowDirShape rowdir_shape(int N, int K, int epi, int M) {
     RowDirShape none{0, 0, 0};
-    if (N % 16 || K % 32 || M > 256) return none;
+    if (N % 16 || K % 32 || (M > 256 && !rowpair_ok(N, K, epi, M))) return none;
     const int KT = K / 32, ntiles = N / 16;
     if (KT % 16 || KT / 16 < 2 || KT / 16 > 8 || (KT / 16) % 2) return none;  // K in {1024, 2048, 3072, 4096}
     const int tk = KT / 16;
