@@ -1511,7 +1511,14 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
     // residual add and the next norm's preparation in the epilogues of o_proj and down_proj: the norms between two products of this chunk
     // are no launches of their own
     const bool fused_norms = qt == 2 && tp == 1 && !m->taps && t_qkv && all.t_o && all.t_gu && all.t_down && tile_resid_wins(R, H, KO, m->I_l);
+    // ... and of few enough rows the QKV and gate/up products take two row blocks at a time (figures at gemm_rowpair_kernel)
+    const bool pairs = fused_norms && R <= kRowPairRows && tmin > 1 && gemm_rowpair_ok(NQ, H, 2, R) && gemm_rowpair_ok(2 * m->I_l, H, 1, R);
     RowNorm rn;  // pending on xh / xl
+    auto pair_args = [&]() {
+        RowParArgs ra;
+        ra.xh = m->xh; ra.xl = m->xl; ra.ldx = H; ra.M = R; ra.x_packed = ra.o_packed = 1;
+        return ra;
+    };
     auto resid_product = [&](const bf16_bits* xh, const bf16_bits* xl, const PackedW& w, const float* next_w) -> hipError_t {
         ++m->tile_resid_launches;
         rn.ssq = m->ssqT; rn.groups = H / 128; rn.stride = m->max_rows; rn.inv_h = 1.0f / (float)H; rn.eps = eps;
@@ -1523,7 +1530,8 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
         const bool trim = alone && l + 1 == m->L;
         const Rest t = trim ? rest_of(n_last) : all;
         const int rows = trim ? n_last : R;
-        m->tile_launches += (int)t_qkv + (int)(t.t_o && rows) + (int)(t.t_gu && rows) + (int)(t.t_down && rows);
+        const bool gu_pairs = pairs && !trim;
+        m->tile_launches += (int)(t_qkv && !pairs) + (int)(t.t_o && rows) + (int)(t.t_gu && rows && !gu_pairs) + (int)(t.t_down && rows);
         NormArgs na;
         na.weight = w.ln1; na.eps = eps; na.H = H; na.xh = m->xh; na.xl = m->xl; na.residual_out = m->resid; na.out_packed = packed || t_qkv;
         if (l == 0) {  // residual None: normed = norm(x), residual = x  (qwen3.rs:382-386)
@@ -1545,11 +1553,15 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
         qa.kv.klo = m->klocache.empty() ? nullptr : m->klocache[l];
         const bool fuse_qk = qt == 1 && n_tiles == R && R <= kAttnFusedMaxRows;  // decode: every q-tile is one row
         int rcg = NVLLM_OK;
-        if (t_qkv_fused && !fuse_qk) {
+        if (t_qkv_fused && !pairs && !fuse_qk) {
             // prompt chunk: q/k-norm + RoPE + KV write + q output in the QKV GEMM's epilogue (one wave tile = one head)
             PROF(m, PROF_GEMM, launch_gemm_tile_qkv(m->xh, m->xl, w.qkv, R, qa, tmin, s));
         } else {
-            if (t_qkv) PROF(m, PROF_GEMM, launch_gemm_tile(m->xh, m->xl, w.qkv, R, 0, m->slabs, nullptr, nullptr, 0, tmin, max_ks, &qa.n_slabs, s));
+            if (pairs) {
+                RowParArgs ra = pair_args();
+                ra.out = m->slabs;
+                PROF(m, PROF_GEMM, launch_gemm_rowpar(ra, w.qkv, 2, s));
+            } else if (t_qkv) PROF(m, PROF_GEMM, launch_gemm_tile(m->xh, m->xl, w.qkv, R, 0, m->slabs, nullptr, nullptr, 0, tmin, max_ks, &qa.n_slabs, s));
             else rcg = gemm_slabs(m, m->xh, m->xl, H, w.qkv, m->slabs, R, 8, &qa.n_slabs, packed);
             if (rcg) return rcg;
             if (!fuse_qk) {
@@ -1618,7 +1630,11 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
             PROF(m, PROF_NORM, launch_add_rmsnorm(nb, rows, s));
         }
         // MLP (qwen3.rs:323-327)
-        if (t.t_gu) {
+        if (gu_pairs) {
+            RowParArgs ra = pair_args();
+            ra.oh = m->xh2; ra.ol = m->xl2; ra.rn = rn;
+            PROF(m, PROF_GEMM, launch_gemm_rowpar(ra, w.gu, 1, s));
+        } else if (t.t_gu) {
             PROF(m, PROF_GEMM, launch_gemm_tile(m->xh, m->xl, w.gu, rows, 2, nullptr, m->xh2, m->xl2, t.t_down ? 1 : 0, tmin, 1, nullptr, s, GluSpec(), rn));
         } else if (!t.packed && rows <= kRowMaxRows && gemm_rowpar_ok(2 * m->I_l, H, 1, rows)) {
             // small gate/up: whole-K row-parallel kernel with the SiLU*mul epilogue

@@ -1378,7 +1378,7 @@ __global__ void __launch_bounds__(1024) gemm_rowdir_two_kernel(RowParArgs a, con
     else rowdir_body<NTB, 16, TKB, 2, false>(b, wb, NB, 16 * TKB, (int)blockIdx.x - groups_a);
 }
 
-// Register-direct products of 65 to 480 rows: RB row blocks at a time (blocks z, z + gz, ... of blockIdx.z = z), K split over NWK waves, the
+// Register-direct products of 65 to 896 rows: RB row blocks at a time (blocks z, z + gz, ... of blockIdx.z = z), K split over NWK waves, the
 // weights kept.  Bound by what a CU takes in (x and W of its workgroup, 0.4 to 0.6 MB) and by the phases of a round: products, K slices to
 // LDS, their sums, the epilogue.  Eight waves instead of sixteen halve the slices and have registers for two blocks, so that a round's phases
 // serve 32 rows; gate and up of a feature meet in one wave; two n-tiles of o and down halve the rows a workgroup takes in.  0.6B, us a launch,
@@ -1386,6 +1386,7 @@ __global__ void __launch_bounds__(1024) gemm_rowdir_two_kernel(RowParArgs a, con
 // 8.6 / 7.6; 250 rows 10.4 / 9.2, 15.5 / 12.7, 12.9 / 10.1.
 // Past 256 rows a round more to every 128 rows, against tile products with K slices, whose slabs are launches more, and which fill and drain a CU for a few stages: up to where o and down are one
 // launch each as tiles too (tile_resid_kernel).  A prompt of 0.6B, ms, tile products / these: 257 tokens 2.63 / 1.94, 300 2.67 / 1.98, 384 2.84 / 2.04, 480 2.88 / 2.34; a step of 257 rows 3.30 / 2.49.
+// Past 480 q/k/v and gate/up alone: 481 tokens 2.91 / 2.60, 512 2.93 / 2.62, 640 3.25 / 2.88, 768 3.36 / 3.10, 896 3.45 / 3.30, 897 3.45 / 3.43, 1024 3.53 / 3.52.
 template <int NT, int NWK, int TK, int RB, int EPI>
 __global__ void __launch_bounds__(NWK * 64) gemm_rowpair_kernel(RowParArgs a, const uint4* __restrict__ wp, int N, int KT) {
     constexpr int NR = 16, PER = EPI == 1 ? 2 : 1, UNITS = RB * NT / PER, UPW = (UNITS + NWK - 1) / NWK;  // a unit: a row block's n-tile, or its gate and up
@@ -1427,7 +1428,10 @@ __global__ void __launch_bounds__(NWK * 64) gemm_rowpair_kernel(RowParArgs a, co
         }
     };
     if constexpr (EPI == 0) load_resid(blk);
-    if constexpr (EPI == 1) rownorm_partials_blocks<NR>(a.rn, blk * NR, gz * NR, M, sred);
+    if constexpr (EPI == 1) {
+        rownorm_partials_blocks<NR>(a.rn, blk * NR, gz * NR, M, sred);
+        if (blk + NWK * gz < blocks) rownorm_partials_blocks<NR>(a.rn, (blk + NWK * gz) * NR, gz * NR, M, sred + NWK * 4 * NR);
+    }
     __builtin_amdgcn_sched_barrier(0);
     for (;;) {
         const int next = blk + RB * gz;
@@ -1518,8 +1522,8 @@ static hipError_t rowpair_launch(const RowParArgs& a, const PackedW& w, hipStrea
     const size_t lds = (size_t)NWK * RB * NT * 1024 + (EPI == 1 ? (size_t)16 * 64 * 4 : 0);
     static std::atomic<uint64_t> lds_set{0};
     ensure_dyn_lds(reinterpret_cast<const void*>(gemm_rowpair_kernel<NT, NWK, TK, RB, EPI>), lds, lds_set);
-    // one round of the CUs; epilogue 1 holds the norms of blockDim.x / 64 blocks
-    const int gz = std::min(blocks, std::max(256 / groups, (blocks + NWK - 1) / NWK));
+    // one round of the CUs; epilogue 1 holds the norms of two blocks a wave
+    const int gz = std::min(blocks, std::max(256 / groups, (blocks + 2 * NWK - 1) / (2 * NWK)));
     gemm_rowpair_kernel<NT, NWK, TK, RB, EPI><<<dim3(groups, 1, gz), NWK * 64, lds, s>>>(a, w.data, w.N, w.K / 32);
     g_rowpair_launches.fetch_add(1, std::memory_order_relaxed);
     return hipGetLastError();
@@ -1531,7 +1535,7 @@ static hipError_t rowpair_launch(const RowParArgs& a, const PackedW& w, hipStrea
 //   q/k/v    1536 features +0.5 to +0.9 up to 10 blocks, -0.3 to -0.7 above; 2048 +0.4 to +0.8 up to 8, -0.3 to -0.9; 2560 +0.9 +0.4 up to 6, -0.9 to
 //            +0.1; 3072 +0.5 at 5, -1.9 to +0.3; 4096 -1.3 to 0.0; 5120 -4.7 to +0.1; 6144 +0.9 at 5, -4.8 to +0.1
 //   gate/up  1536 +0.8 to +1.2, 3072 +0.8 to +1.5 (both up to 8); 4608 +1.4 at 5, -0.8 to -1.1; 6144 -2.5 to -0.4; 9216 +0.9 at 5, -0.6 to -3.9
-static bool rowpair_ok(int N, int K, int epi, int M) {
+bool gemm_rowpair_ok(int N, int K, int epi, int M) {
     if (M <= 64 || M > kRowPairRows) return false;
     auto pairs = [&](int nt) {  // row blocks for two at a time
         const int blocks = (M + 15) / 16, room = 256 / (N / 16 / nt);
@@ -1544,7 +1548,7 @@ static bool rowpair_ok(int N, int K, int epi, int M) {
 }
 template <int EPI>
 static hipError_t rowpair_dispatch(const RowParArgs& a, const PackedW& w, hipStream_t s) {
-    if (!a.x_packed || !rowpair_ok(w.N, w.K, EPI, a.M)) return hipErrorNotReady;
+    if (!a.x_packed || !gemm_rowpair_ok(w.N, w.K, EPI, a.M)) return hipErrorNotReady;
     if constexpr (EPI == 0) {
         const bool one = (a.M + 15) / 16 <= 256 / (w.N / 32);  // a block to a workgroup
         if (w.K == 1024) return one ? rowpair_launch<2, 8, 4, 1, 0>(a, w, s) : rowpair_launch<2, 8, 4, 2, 0>(a, w, s);
@@ -1561,7 +1565,7 @@ static hipError_t rowpair_dispatch(const RowParArgs& a, const PackedW& w, hipStr
 struct RowDirShape { int nt, nwk, tk; };
 static RowDirShape rowdir_shape(int N, int K, int epi, int M) {
     RowDirShape none{0, 0, 0};
-    if (N % 16 || K % 32 || (M > 256 && !rowpair_ok(N, K, epi, M))) return none;
+    if (N % 16 || K % 32 || (M > 256 && !gemm_rowpair_ok(N, K, epi, M))) return none;
     const int KT = K / 32, ntiles = N / 16;
     if (KT % 16 || KT / 16 < 2 || KT / 16 > 8 || (KT / 16) % 2) return none;  // K in {1024, 2048, 3072, 4096}
     const int tk = KT / 16;

@@ -82,7 +82,7 @@ static int dmalloc(nvllm_ctx* c, T** p, size_t count) {
 // Steps of 0.6B, row-major and packed, ms: 1 row 0.885 / 0.930, 2 0.936 / 0.965, 3 0.957 / 0.967, 4 0.974 / 0.969, 8 1.044 / 0.980,
 // 15 1.166 / 0.992; a 1024-wide decoder of another design 4 rows 0.239 / 0.233, 15 0.265 / 0.232; a prompt of 15 tokens 1.323 / 1.196.
 constexpr int kPackedMinRows = 4;
-constexpr int kFusedMaxRows = kRowPairRows;  // the fused decode path (deferred norms, row-parallel epilogues) handles up to this many rows ...
+constexpr int kFusedMaxRows = 480;  // the fused decode path (deferred norms, row-parallel epilogues) handles up to this many rows ...
 constexpr int kRowMaxRows = 128;    // ... and so many where a projection of the layer has no register-direct form; row-parallel products elsewhere
 // one-shot all-reduce: messages of up to this many rows; its slots are sized for them (uncached memory on every peer).  Longer ones go
 // through the communicator, in decode steps of more rows too: what the one-shot form does for those was never measured
