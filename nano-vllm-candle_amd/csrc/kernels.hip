@@ -2234,7 +2234,8 @@ __device__ __forceinline__ PrefillTile prefill_tile(const AttnArgs& a, int i) {
 // VLO: 0 = 16-bit cache, 1 = 24-bit V, 2 = 24-bit K and V (KvLayout::klo too: four more 1 KiB wave-loads per tile, one bf8 MFMA
 // per QK^T fragment against q in bf8)
 // AHEAD: both tile sets are asked for before the prologue, see there
-template <int HD, int NWV, bool FUSED, int VLO, bool AHEAD>
+// PARTS: contexts may be in parts
+template <int HD, int NWV, bool FUSED, int VLO, bool AHEAD, bool PARTS>
 __device__ __forceinline__ void attn_paged_body(const AttnArgs& a) {
     constexpr int DC = HD / 32, DT = HD / 16, DL = VLO ? DT / 2 : 1;  // DL: 1 KiB residual fragments per tile (two PV fragments each)
     constexpr bool KLO = VLO == 2;
@@ -2281,7 +2282,7 @@ __device__ __forceinline__ void attn_paged_body(const AttnArgs& a) {
     // split-KV (flash-decoding): workgroup blockIdx.z owns 32-token tiles [t_begin, t_end) and leaves an
     // un-normalised partial (m, l, O); every workgroup then has the same short dependent-load chain
     // whatever the context length.  part_tiles == 0: one workgroup does the whole context.
-    const int t_begin = a.part_tiles ? (int)blockIdx.z * a.part_tiles : 0;
+    const int t_begin = PARTS && a.part_tiles ? (int)blockIdx.z * a.part_tiles : 0;
     [[maybe_unused]] int first_slab[2] = {0, 0};  // cache blocks of this wave's first two tiles
     if constexpr (FUSED) {
 #pragma unroll
@@ -2333,7 +2334,7 @@ __device__ __forceinline__ void attn_paged_body(const AttnArgs& a) {
     const int pmax = FUSED ? rec[2] : a.pos[row0 + nrows - 1];
     if constexpr (FUSED) my_pos = pmax;  // uniform; what the lanes of no row (q = 0) sum up is never stored
     const int n_kv_tiles = (pmax >> 5) + 1;
-    const int t_end = a.part_tiles ? min(n_kv_tiles, t_begin + a.part_tiles) : n_kv_tiles;
+    const int t_end = PARTS && a.part_tiles ? min(n_kv_tiles, t_begin + a.part_tiles) : n_kv_tiles;
     if (t_begin >= n_kv_tiles) return;  // uniform for the whole workgroup
 
     // (plain reads became vector loads behind the prologue's barrier, each with a wait that drained the tiles in flight)
@@ -2628,7 +2629,7 @@ __device__ __forceinline__ void attn_paged_body(const AttnArgs& a) {
             *reinterpret_cast<uint2*>(a.out_lo + xo) = make_uint2(l0 | ((uint32_t)l1 << 16), l2 | ((uint32_t)l3 << 16));
         }
     };
-    const int n_parts = a.part_tiles ? (n_kv_tiles + a.part_tiles - 1) / a.part_tiles : 1;
+    const int n_parts = PARTS && a.part_tiles ? (n_kv_tiles + a.part_tiles - 1) / a.part_tiles : 1;
     for (int i = threadIdx.x; i < cols * (HD / 4); i += NWV * 64) {
         const int col = i / (HD / 4), d4 = i % (HD / 4), tok = FUSED ? 0 : col / gqa;
         if (tok >= nrows || (!FUSED && col >= tpq * gqa)) continue;
@@ -2661,7 +2662,7 @@ __device__ __forceinline__ void attn_paged_body(const AttnArgs& a) {
         }
         finish(row, head, d4, acc, ltot);
     }
-    if constexpr (FUSED) {
+    if constexpr (FUSED && PARTS) {
         if (n_parts > 1) {
             // The part that ends last merges them, in their order: which one it is changes nothing.  Parts are handed on past the L2s, each wave waits for its own stores and the barrier for
             // the waves, so that who counts n_parts - 1 others can read them.  As a launch of its own behind this one, steps of 0.6B: 9 rows of 600 tokens 1065 us, now 1031, 10 of 100 to 1000
@@ -2710,11 +2711,16 @@ __device__ __forceinline__ void attn_paged_body(const AttnArgs& a) {
 }
 template <int HD, int NWV, bool FUSED, int VLO = 0>
 __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_kernel(AttnArgs a) {
-    attn_paged_body<HD, NWV, FUSED, VLO, false>(a);
+    attn_paged_body<HD, NWV, FUSED, VLO, false, !FUSED>(a);
+}
+// The fused form where contexts are in parts.  With the merge behind the whole contexts too, 16 steps of 64 rows of 64 to 512 tokens took 23.2 ms, not 22.96.
+template <int HD, int NWV, int VLO>
+__global__ void __launch_bounds__(NWV * 64, 2) attn_parts_kernel(AttnArgs a) {
+    attn_paged_body<HD, NWV, true, VLO, false, true>(a);
 }
 template <int HD, int NWV>
 __global__ void __launch_bounds__(NWV * 64, 2) attn_paged_ahead_kernel(AttnArgs a) {
-    attn_paged_body<HD, NWV, true, 0, true>(a);
+    attn_paged_body<HD, NWV, true, 0, true, false>(a);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -3088,7 +3094,10 @@ static hipError_t attn_launch_v(const AttnArgs& a, int n_tiles, int grid_z, hipS
     static std::atomic<uint64_t> lds_set{0};
     void (*kernel)(AttnArgs) = attn_paged_kernel<HD, NWV, FUSED, VLO>;
     if constexpr (AHEAD) kernel = attn_paged_ahead_kernel<HD, NWV>;
-    ensure_dyn_lds(reinterpret_cast<const void*>(kernel), lds_of(16), lds_set);
+    static std::atomic<uint64_t> lds_set_parts{0};
+    const bool parts = FUSED && a.part_tiles;
+    if constexpr (FUSED) if (parts) kernel = attn_parts_kernel<HD, NWV, VLO>;
+    ensure_dyn_lds(reinterpret_cast<const void*>(kernel), lds_of(16), parts ? lds_set_parts : lds_set);
     dim3 grid = FUSED ? dim3(a.kv.kv_l, n_tiles, grid_z) : dim3(n_tiles * a.kv.kv_l, 1, grid_z);
     kernel<<<grid, NWV * 64, lds, s>>>(a);
     return hipGetLastError();
