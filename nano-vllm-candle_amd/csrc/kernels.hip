@@ -1528,14 +1528,14 @@ static hipError_t rowpair_launch(const RowParArgs& a, const PackedW& w, hipStrea
     g_rowpair_launches.fetch_add(1, std::memory_order_relaxed);
     return hipGetLastError();
 }
-// Products of 65 to kRowPairRows rows of packed planes whose shape has an instance (else hipErrorNotReady).  Up to 64 rows every workgroup has one block: the
+// Products of 65 to kRowPairRows rows of packed planes whose shape has an instance (else hipErrorNotReady); whether such a product is register-direct at all says rowdir_shape.  Up to 64 rows every workgroup has one block: the
 // 16-wave forms below are as fast or faster there (64 rows, gate/up 8.1 us against 10.6, o 4.8 against 5.6).  So they are, for q/k/v and gate/up,
 // while the grid gives every block its own workgroup, whose second block would be nothing, and for 5 blocks on two workgroups.  A product's time by
 // this less the 16-wave form's, us, at 5 to 16 blocks of 1024-wide rows:
 //   q/k/v    1536 features +0.5 to +0.9 up to 10 blocks, -0.3 to -0.7 above; 2048 +0.4 to +0.8 up to 8, -0.3 to -0.9; 2560 +0.9 +0.4 up to 6, -0.9 to
 //            +0.1; 3072 +0.5 at 5, -1.9 to +0.3; 4096 -1.3 to 0.0; 5120 -4.7 to +0.1; 6144 +0.9 at 5, -4.8 to +0.1
 //   gate/up  1536 +0.8 to +1.2, 3072 +0.8 to +1.5 (both up to 8); 4608 +1.4 at 5, -0.8 to -1.1; 6144 -2.5 to -0.4; 9216 +0.9 at 5, -0.6 to -3.9
-bool gemm_rowpair_ok(int N, int K, int epi, int M) {
+static bool rowpair_ok(int N, int K, int epi, int M) {
     if (M <= 64 || M > kRowPairRows) return false;
     auto pairs = [&](int nt) {  // row blocks for two at a time
         const int blocks = (M + 15) / 16, room = 256 / (N / 16 / nt);
@@ -1548,7 +1548,7 @@ bool gemm_rowpair_ok(int N, int K, int epi, int M) {
 }
 template <int EPI>
 static hipError_t rowpair_dispatch(const RowParArgs& a, const PackedW& w, hipStream_t s) {
-    if (!a.x_packed || !gemm_rowpair_ok(w.N, w.K, EPI, a.M)) return hipErrorNotReady;
+    if (!a.x_packed || !rowpair_ok(w.N, w.K, EPI, a.M)) return hipErrorNotReady;
     if constexpr (EPI == 0) {
         const bool one = (a.M + 15) / 16 <= 256 / (w.N / 32);  // a block to a workgroup
         if (w.K == 1024) return one ? rowpair_launch<2, 8, 4, 1, 0>(a, w, s) : rowpair_launch<2, 8, 4, 2, 0>(a, w, s);
@@ -1565,7 +1565,7 @@ static hipError_t rowpair_dispatch(const RowParArgs& a, const PackedW& w, hipStr
 struct RowDirShape { int nt, nwk, tk; };
 static RowDirShape rowdir_shape(int N, int K, int epi, int M) {
     RowDirShape none{0, 0, 0};
-    if (N % 16 || K % 32 || (M > 256 && !gemm_rowpair_ok(N, K, epi, M))) return none;
+    if (N % 16 || K % 32 || (M > 256 && !rowpair_ok(N, K, epi, M))) return none;
     const int KT = K / 32, ntiles = N / 16;
     if (KT % 16 || KT / 16 < 2 || KT / 16 > 8 || (KT / 16) % 2) return none;  // K in {1024, 2048, 3072, 4096}
     const int tk = KT / 16;
