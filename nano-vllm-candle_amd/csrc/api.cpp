@@ -1511,9 +1511,8 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
     // residual add and the next norm's preparation in the epilogues of o_proj and down_proj: the norms between two products of this chunk
     // are no launches of their own
     const bool fused_norms = qt == 2 && tp == 1 && !m->taps && t_qkv && all.t_o && all.t_gu && all.t_down && tile_resid_wins(R, H, KO, m->I_l);
-    // ... and of few enough rows the QKV and gate/up products take two row blocks at a time (figures at gemm_rowpair_kernel).  The launch's own rule, which leaves matrices of 24 MB and more to
-    // the tile products
-    const bool pairs = fused_norms && R > 256 && tmin > 1 && gemm_rowdir_ok(NQ, H, 2, R) && gemm_rowdir_ok(2 * m->I_l, H, 1, R);
+    // ... and of few enough rows the QKV and gate/up products take two row blocks at a time (figures at gemm_rowpair_kernel)
+    const bool pairs = fused_norms && R > 256 && tmin > 1 && gemm_rowpair_at_once(NQ, H, 2, R) && gemm_rowpair_at_once(2 * m->I_l, H, 1, R);
     RowNorm rn;  // pending on xh / xl
     auto pair_args = [&]() {
         RowParArgs ra;

@@ -1387,6 +1387,9 @@ __global__ void __launch_bounds__(1024) gemm_rowdir_two_kernel(RowParArgs a, con
 // Past 256 rows a round more to every 128 rows, against tile products with K slices, whose slabs are launches more, and which fill and drain a CU for a few stages: up to where o and down are one
 // launch each as tiles too (tile_resid_kernel).  A prompt of 0.6B, ms, tile products / these: 257 tokens 2.63 / 1.94, 300 2.67 / 1.98, 384 2.84 / 2.04, 480 2.88 / 2.34; a step of 257 rows 3.30 / 2.49.
 // Past 480 q/k/v and gate/up alone: 481 tokens 2.91 / 2.60, 512 2.93 / 2.62, 640 3.25 / 2.88, 768 3.36 / 3.10, 896 3.45 / 3.30, 897 3.45 / 3.43, 1024 3.53 / 3.52.
+// But only while the CUs hold all of their workgroups at once: 16 blocks each at most makes it more than that of wide layers.  A prompt of 12 layers, ms, tile products / these, the last row count in one round and
+// the first in two: gate/up of 9216 features 512 rows 1.36 / 1.35 and 528 1.40 / 1.54, of 6912 768 1.45 / 1.40 and 832 1.47 / 1.65; q/k/v of 5120 768 1.58 / 1.51 and 832 1.64 / 1.72, of 6144 512 1.45 / 1.32 and
+// 528 1.46 / 1.44 (640 1.49 / 1.53, 896 1.68 / 1.77), of 9216, never in one, 512 1.52 / 1.56 and 896 1.80 / 2.02.
 template <int NT, int NWK, int TK, int RB, int EPI>
 __global__ void __launch_bounds__(NWK * 64) gemm_rowpair_kernel(RowParArgs a, const uint4* __restrict__ wp, int N, int KT) {
     constexpr int NR = 16, PER = EPI == 1 ? 2 : 1, UNITS = RB * NT / PER, UPW = (UNITS + NWK - 1) / NWK;  // a unit: a row block's n-tile, or its gate and up
@@ -1516,14 +1519,15 @@ __global__ void __launch_bounds__(NWK * 64) gemm_rowpair_kernel(RowParArgs a, co
 }
 static std::atomic<int64_t> g_rowpair_launches{0};
 int64_t rowpair_launches() { return g_rowpair_launches.load(std::memory_order_relaxed); }
+// workgroups that share a product's row blocks: one round of the CUs, 16 blocks each at most, for epilogue 1 holds the norms of two blocks a wave
+static int rowpair_groups(int groups, int blocks) { return std::min(blocks, std::max(256 / groups, (blocks + 15) / 16)); }
 template <int NT, int NWK, int TK, int RB, int EPI>
 static hipError_t rowpair_launch(const RowParArgs& a, const PackedW& w, hipStream_t s) {
     const int groups = w.N / 16 / NT, blocks = (a.M + 15) / 16;
     const size_t lds = (size_t)NWK * RB * NT * 1024 + (EPI == 1 ? (size_t)16 * 64 * 4 : 0);
     static std::atomic<uint64_t> lds_set{0};
     ensure_dyn_lds(reinterpret_cast<const void*>(gemm_rowpair_kernel<NT, NWK, TK, RB, EPI>), lds, lds_set);
-    // one round of the CUs; epilogue 1 holds the norms of two blocks a wave
-    const int gz = std::min(blocks, std::max(256 / groups, (blocks + 2 * NWK - 1) / (2 * NWK)));
+    const int gz = rowpair_groups(groups, blocks);
     gemm_rowpair_kernel<NT, NWK, TK, RB, EPI><<<dim3(groups, 1, gz), NWK * 64, lds, s>>>(a, w.data, w.N, w.K / 32);
     g_rowpair_launches.fetch_add(1, std::memory_order_relaxed);
     return hipGetLastError();
@@ -1651,6 +1655,11 @@ int gemm_rowpar_groups(int N, int K) {
     return (N / 16 + sh.nwn - 1) / sh.nwn;
 }
 bool gemm_rowdir_ok(int N, int K, int epi, int M) { return rowdir_shape(N, K, epi, M).nt != 0; }
+bool gemm_rowpair_at_once(int N, int K, int epi, int M) {
+    if (!rowpair_ok(N, K, epi, M) || !rowdir_shape(N, K, epi, M).nt) return false;
+    const int groups = N / 16 / (epi == 0 ? 2 : epi == 1 ? 6 : 4);
+    return groups * rowpair_groups(groups, (M + 15) / 16) <= 256;
+}
 int gemm_rowpar_splits(int N, int K, int epi, int M) {
     if (rowdir_shape(N, K, epi, M).nt) return 1;
     RowParShape sh;
