@@ -1383,6 +1383,7 @@ static int forward_chunk_fused(nvllm_model* m, const FusedPlan& fp, int R, int n
             parts_max = m->attn_parts_max;
             if (fuse_qk) { aa.waves = m->attn_waves; aa.ahead = m->attn_ahead; }
             m->eight_wave_launches += aa.waves == 8;
+            m->merged_parts_launches += parts_max > 1 && fuse_qk;
             m->tiles_ahead_launches += aa.ahead;
         }
         PROF(m, PROF_EMPTY, hipSuccess);  // calibration: an event pair around nothing, at the attention launch's place
@@ -1588,6 +1589,7 @@ static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last,
             parts_max = m->attn_parts_max;
             if (fuse_qk) { aa.waves = m->attn_waves; aa.ahead = m->attn_ahead; }
             m->eight_wave_launches += aa.waves == 8;
+            m->merged_parts_launches += parts_max > 1 && fuse_qk;
             m->tiles_ahead_launches += aa.ahead;
         }
         STAMPS(aa, m);
@@ -2458,7 +2460,7 @@ extern "C" int nvllm_debug_set_option(nvllm_model* m, const char* name, int valu
 
 // counters for tests: "oneshot_calls" = all-reduces this model's context has run on the one-shot device path;
 // "tile_gemm_launches" = projections this model has run on the prefill tile GEMM; "table_copies" = whole block tables sent;
-// "qk_rows16_launches" = q/k norm launches of 16 rows and a head per workgroup; "eight_wave_launches" = decode attention on eight waves; "tiles_ahead_launches" = ... with a wave's second tile asked for before the prologue;
+// "qk_rows16_launches" = q/k norm launches of 16 rows and a head per workgroup; "eight_wave_launches" = decode attention on eight waves; "merged_parts_launches" = ... in parts that are merged in the launch; "tiles_ahead_launches" = ... with a wave's second tile asked for before the prologue;
 // "prefill_dealt_launches" = prompt attention with a q-tile to a workgroup, "prefill_dealt_tiles" = q-tiles of those; "row_sum_launches" = products of a few rows that add up the slabs of the one before;
 // "resident_launches" = decode steps in one launch;
 // "scan_gate_launches" = step sizes of a decode step's selective scan by a launch of their own; "two_product_launches" = pairs of products in one launch;
@@ -2480,6 +2482,7 @@ extern "C" int nvllm_debug_get_counter(nvllm_model* m, const char* name, int64_t
     if (!strcmp(name, "two_product_launches")) { *value = m->two_launches; return NVLLM_OK; }
     if (!strcmp(name, "row_pair_launches")) { *value = rowpair_launches(); return NVLLM_OK; }
     if (!strcmp(name, "eight_wave_launches")) { *value = m->eight_wave_launches; return NVLLM_OK; }
+    if (!strcmp(name, "merged_parts_launches")) { *value = m->merged_parts_launches; return NVLLM_OK; }
     if (!strcmp(name, "tiles_ahead_launches")) { *value = m->tiles_ahead_launches; return NVLLM_OK; }
     if (!strcmp(name, "kv_f16_saturated") || !strcmp(name, "kv_f16_absmax_bits")) {
         // scan of the whole K/V pool (debug, off the hot path): elements the f16_sat clamp of a cache write produced, and the

@@ -2674,8 +2674,8 @@ __device__ __forceinline__ void attn_paged_body(const AttnArgs& a) {
     if constexpr (FUSED && PARTS) {
         if (n_parts > 1) {
             // The part that ends last merges them, in their order: which one it is changes nothing.  Parts are handed on past the L2s, each wave waits for its own stores and the barrier for
-            // the waves, so that who counts n_parts - 1 others can read them.  As a launch of its own behind this one, steps of 0.6B: 9 rows of 600 tokens 1065 us, now 1031, 10 of 100 to 1000
-            // 1086 and 1053, 16 of 1500 1340 and 1306; four layers of 8B, 1 x 3000 698 and 689, 8 x 100 to 1500 754 and 748.
+            // the waves, so that who counts n_parts - 1 others can read them.  As a launch of its own behind this one, steps of 0.6B: 9 rows of 600 tokens 1063 us, now 1006, 10 of 100 to 1000 1089 and 1032,
+            // 16 of 1500 1337 and 1290, 1 of 16000 1344 and 1106.
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
             int* const seen = reinterpret_cast<int*>(smem_raw);  // (ml and obuf are read)
@@ -2683,20 +2683,23 @@ __device__ __forceinline__ void attn_paged_body(const AttnArgs& a) {
             __syncthreads();
             if (*seen != n_parts - 1) return;
             if (threadIdx.x == 0) __hip_atomic_store(a.part_done + (size_t)row0 * a.kv.kv_l + kh, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            // One buffer for all of the row's heads: with a head's own, which differs between the lanes of a wave, each load was a loop over the wave's heads, two of 128 or four of 64.  Six layers with 16
+            // heads of 64 on four, 2 x 9000 tokens, us: the merge as a launch 271, with such loops 336, now 220; 14 heads of 128 on two, 1 x 16000: 462, 412, 368.
+            const size_t row_parts = (size_t)row0 * a.nh_l * a.max_parts;
+            const auto ro = buffer_of(a.part_o + row_parts * HD, a.nh_l * a.max_parts * HD * 4), rm = buffer_of(a.part_ml + row_parts * 2, a.nh_l * a.max_parts * 8);
             for (int i = threadIdx.x; i < cols * (HD / 4); i += NWV * 64) {
-                const int col = i / (HD / 4), d4 = i % (HD / 4), head = kh * gqa + col;
-                const size_t part = ((size_t)row0 * a.nh_l + head) * a.max_parts;
-                const auto ro = buffer_of(a.part_o + part * HD, n_parts * HD * 4), rm = buffer_of(a.part_ml + part * 2, n_parts * 8);
+                const int col = i / (HD / 4), d4 = i % (HD / 4), head = kh * gqa + col, part = head * a.max_parts;
                 float ms = -1e30f, ltot = 0.f;
                 f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-                constexpr int B = 8;  // parts at a time
+                constexpr int B = 8, kNoPart = 0x7ffffff0;  // parts at a time; a place past any buffer's end
                 for (int s0 = 0; s0 < n_parts; s0 += B) {
                     float2 pm[B];
                     float4 po[B];
 #pragma unroll
                     for (int s = 0; s < B; ++s) {  // (past the last one: zeros, which count nothing)
-                        pm[s] = __builtin_bit_cast(float2, load_shared8(rm, (s0 + s) * 8));
-                        po[s] = __builtin_bit_cast(float4, load_shared16(ro, ((s0 + s) * HD + d4 * 4) * 4));
+                        const bool there = s0 + s < n_parts;
+                        pm[s] = __builtin_bit_cast(float2, load_shared8(rm, there ? (part + s0 + s) * 8 : kNoPart));
+                        po[s] = __builtin_bit_cast(float4, load_shared16(ro, there ? ((part + s0 + s) * HD + d4 * 4) * 4 : kNoPart));
                     }
                     float to = ms;
 #pragma unroll

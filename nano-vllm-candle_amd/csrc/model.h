@@ -249,6 +249,7 @@ struct nvllm_model {
     int64_t prefill_dealt_tiles = 0;    // ... q-tiles of those
     int64_t row_sum_launches = 0;       // ... products that add up the slabs of the one before (launch_gemm_rowsum)
     int64_t eight_wave_launches = 0; // ... decode attention on eight waves
+    int64_t merged_parts_launches = 0; // ... decode attention in parts that are merged in the launch
     int64_t tiles_ahead_launches = 0; // ... with both tile sets asked for before the prologue
     int64_t scan_gate_launches = 0;  // ... step sizes of a decode step's scan by their own launch
     int64_t two_launches = 0;        // ... two products in one launch

@@ -23,7 +23,9 @@ def test_parts(hd, kv, heads, lens, bits):
     seqs = [rng.integers(0, cfg.vocab_size, n + 1) for n in lens]
     for i in range(rows):
         m.step([i], [seqs[i][:-1]], True, want_logits=False)
+    before = m.counter("merged_parts_launches")
     steps = [m.step(list(range(rows)), seqs, False, want_logits=True)[1] for _ in range(4)]
+    assert m.counter("merged_parts_launches") - before == 4 * cfg.num_hidden_layers
     # whichever part merges, it takes them in their order
     assert all(np.array_equal(s.view(np.uint32), steps[0].view(np.uint32)) for s in steps)
     # the prompt's kernels sum in another order, from keys whose f16 may round the other way: 2^-11 of the largest logit, 2^-14 with the residuals
