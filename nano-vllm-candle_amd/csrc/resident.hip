@@ -11,7 +11,8 @@
 //  - 8 MB of weights asked for at once meanwhile: 2.9 us.  They come a few at a time, and not before the hand-on is on its way (20.5 -> 16.7);
 //  - many values a reader: one of them until it is there, then all (8 rows 31.5 -> 27.5 us a layer, 4 rows 24 -> 21);
 //  - what a reader does with a value: a place within a block for each reader, of every B-th block, so that the steps from one to the next are constants of the loads and LDS
-//    writes (a step of 8 rows 983 -> 880 us, of 4 737 -> 696, of 2 635 -> 608; with the steps in registers 8 rows took 998).
+//    writes (a step of 8 rows 983 -> 880 us, of 4 737 -> 696, of 2 635 -> 608; with the steps in registers 8 rows took 998).  That goes for every width of the feed-forward: with steps in registers where
+//    it is not 3072, four layers of 1024 features took 8 rows 121 us, 110 as launches, and now 109; 28 layers of 8 heads on 8 681, 661 and 605.
 //
 // A workgroup is four row waves and four weight waves.  Weight waves hold what the workgroup needs of the weights in registers (30 KB a wave), asked for one or two phases ahead,
 // because a wave's loads return in order: a value asked for behind weights would wait for them.  Row waves wait for values, lay them into LDS as bf16 planes, run the attention, add up
@@ -384,34 +385,17 @@ __global__ void __launch_bounds__(512, 2) resident_step_kernel(ResidentArgs a) {
                 if (lane == 0) ssq[r * 4 + wave] = sum;
             }
         };
-        // the activations: blocks of RP x ni units
-        auto read_act = [&]() __attribute__((always_inline)) {
-            constexpr int NU = 4 * RP;  // of blocks of 3 RP; those of 2 RP and RP are fewer
-            const int block = lines(act_words), B = ni == 3 ? 64 / RP : ni == 2 ? 96 / RP : 192 / RP, by_ni = ni == 1 ? 65536 : ni == 2 ? 32768 : 21846;
-            const int v_at = reader * by_ni >> 16, g0 = v_at / RP, in = reader - g0 * RP * ni, row = in * by_ni >> 16, S = L::x_bytes(ni << 10);  // (/ ni by a multiplication)
-            const int at = (g0 * block + in * 4) * 4, step = B * block * 4;
-            char* const p = smem + row * S + (g0 * ni + in - row * ni) * 8;
+        // the activations: blocks of RP x NI units
+        auto read_act = [&](auto wide) __attribute__((always_inline)) {
+            constexpr int NI = decltype(wide)::value, U = RP * NI, B = 192 / U, NU = (kResidentGroups + B - 1) / B, block = lines(U * 4), step = B * block * 4;
+            const int g0 = reader / U, in = reader % U, row = in / NI, at = (g0 * block + in * 4) * 4, S = L::x_bytes(NI << 10);
+            const bool last = kResidentGroups % B == 0 || g0 + (NU - 1) * B < kResidentGroups;
             uint4 v[NU];
-            if (ni == 3) {  // (steps that are known here)
-                constexpr int step3 = 64 / RP * lines(RP * 12) * 4;
-                read(v, buffer_of(b_act, lines(RP * 12) * kResidentGroups * 4), at, step3, at + (NU - 1) * step3);
+            read(v, buffer_of(b_act, block * kResidentGroups * 4), at, step, last ? at + (NU - 1) * step : kNowhere);
+            char* const p = smem + row * S + (g0 * NI + in - row * NI) * 8;
 #pragma unroll
-                for (int i = 0; i < NU; ++i) lay(v[i], p + i * (64 / RP) * 24);
-            } else {
-                const auto r = buffer_of(b_act, block * kResidentGroups * 4);
-                waiting.until([&]() __attribute__((always_inline)) {
-                    uint32_t m = 0;
-#pragma unroll
-                    for (int i = 0; i < NU; ++i) {
-                        v[i] = load_shared16(r, g0 + i * B < kResidentGroups ? at + i * step : kNowhere);
-                        m = max(m, most(v[i]));
-                    }
-                    return m != kResidentEmpty;
-                });
-#pragma unroll
-                for (int i = 0; i < NU; ++i)
-                    if (g0 + i * B < kResidentGroups) lay(v[i], p + i * B * ni * 8);
-            }
+            for (int i = 0; i < NU - 1; ++i) lay(v[i], p + i * B * NI * 8);
+            if (last) lay(v[NU - 1], p + (NU - 1) * B * NI * 8);
         };
         // the attention's output: R rows of ko * 256 units, 16 bytes of LDS between two rows
         auto read_ctx = [&]() __attribute__((always_inline)) {
@@ -719,7 +703,11 @@ __global__ void __launch_bounds__(512, 2) resident_step_kernel(ResidentArgs a) {
         }
 
         // ---- down
-        if (wave) read_act();
+        if (wave) {
+            if (ni == 3) read_act(integral_constant<int, 3>());
+            else if (ni == 2) read_act(integral_constant<int, 2>());
+            else read_act(integral_constant<int, 1>());
+        }
         else stores_there();
         meet();
         meet();
