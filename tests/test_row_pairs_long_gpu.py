@@ -1,4 +1,6 @@
-"""GPU test of the register-direct products of more than 256 rows."""
+"""GPU test of the register-direct products of more than 256 rows, against the tile products: both ends of the ranges and of a round of row blocks,
+the norms of more blocks than a workgroup has waves, rows that end within a block, prompts of one and of several sequences, a decode step, 16- and 24-bit caches, and widths whose grids leave other numbers of
+blocks to a workgroup.  Which form ran is counted: q/k/v, o, gate/up and down of two layers, past 480 rows q/k/v and the first layer's gate/up."""
 import numpy as np
 import pytest
 
@@ -52,4 +54,57 @@ def test_one_round_of_workgroups(inter, heads, kv, last):
     # two layers, the last one's gate/up on the rows that are asked for alone
     assert last == 480 or prompt(m, cfg, last) == 3
     assert prompt(m, cfg, last + 1) == 0
+    m.close()
+
+
+def compare(m, call, pairs, bits=16):
+    def counted():
+        n, t = m.counter("row_pair_launches"), m.counter("tile_gemm_launches")
+        return call(), m.counter("row_pair_launches") - n, m.counter("tile_gemm_launches") - t
+
+    got, taken, tiles = counted()
+    m.set_option("no_fused", 1)
+    m.set_option("tile_min_wgs", 1)  # tile products wherever they fit
+    want, none, all_tiles = counted()
+    m.set_option("no_fused", 0)
+    m.set_option("tile_min_wgs", 64)
+    assert taken == pairs and none == 0 and all_tiles > 0 and (tiles == 0) == (pairs == 8)
+    # products summed in another order; a cached f16 key or value may round the other way: 2^-11 of the largest logit, 2^-14 with the residuals
+    assert np.isfinite(got).all() and np.abs(got - want).max() < 2.0 ** (-11 if bits == 16 else -14) * np.abs(want).max()
+
+
+@pytest.mark.parametrize("rows,bits", [(256, 16), (257, 16), (272, 24), (273, 16), (384, 16), (385, 24), (479, 16), (480, 16), (481, 16), (512, 24), (513, 16), (640, 16), (641, 16), (768, 16), (895, 24), (896, 16), (897, 16)])
+def test_a_prompt(rows, bits):
+    import nano_vllm_candle_amd as pkg
+
+    cfg, m = model(pkg, 4, bits)
+    t = np.random.default_rng(rows).integers(0, cfg.vocab_size, rows)
+    want = [0, 15, 16, rows // 2, rows - 2]  # (the head's buffers hold five rows)
+    compare(m, lambda: m.step_score([0], [t], True, [want]), 8 if rows <= 480 else 3 if rows <= 896 else 0, bits)
+    m.close()
+
+
+# gate/up of 2048 and 4096 features are no multiple of 96: tile products
+@pytest.mark.parametrize("inter,heads,kv,lens,pairs", [(3072, 16, 8, [100, 1, 230], 8), (1024, 8, 2, [300], 0), (2048, 8, 8, [17] * 28, 0), (3072, 24, 4, [90, 380], 8), (3072, 16, 8, [400, 1, 260], 3),
+                                                       (3072, 24, 4, [520], 3), (3072, 24, 24, [300], 8), (1536, 16, 8, [500], 3)])
+def test_prompts_of_other_widths(inter, heads, kv, lens, pairs):
+    import nano_vllm_candle_amd as pkg
+
+    cfg, m = model(pkg, len(lens), 16, inter, heads, kv)
+    rng = np.random.default_rng(inter)
+    seqs = [rng.integers(0, cfg.vocab_size, n) for n in lens]
+    compare(m, lambda: m.step_score(list(range(len(lens))), seqs, True, [[n - 1] for n in lens]), pairs)
+    m.close()
+
+
+@pytest.mark.parametrize("rows", [257, 300, 480])
+def test_a_decode_step(rows):
+    import nano_vllm_candle_amd as pkg
+
+    cfg, m = model(pkg, rows)
+    rng = np.random.default_rng(rows)
+    seqs = [rng.integers(0, cfg.vocab_size, 2 + i % 3) for i in range(rows)]
+    ids = list(range(rows))
+    m.step(ids, [s[:-1] for s in seqs], True)
+    compare(m, lambda: m.step_score(ids, seqs, False, [[len(s) - 1] for s in seqs]), 8)
     m.close()
