@@ -34,7 +34,7 @@ int nvllm_profile_read(nvllm_model* m, double* total_ms, int64_t* launches);
  *   "kv_k_bits" (16 | 24; at the next nvllm_kv_alloc, which refuses it without "kv_v_bits" = 24): the same for K;
  *   "oneshot_allreduce" (0 | 1; at the next nvllm_kv_alloc, every rank alike): one-shot all-reduce for decode messages;
  *       "oneshot_spins": bound of its wait kernel's poll; "oneshot_skip_push": test hook (this rank skips N pushes);
- *   "stage_fail": test hook (the next N launches of a step's metadata fail);
+ *   "stage_fail": test hook (the next N launches of a step's metadata fail); "leave_fail": test hook (the next N steps fail when their results are to leave);
  *   "stream_combine" (default 0): let the fused forward use the streaming GEMM's in-launch split-K combine epilogues (fewer
  *       launches; measured slower on MI355X than slabs + a consumer launch);
  *   "tile_min_wgs" (default 64; 0 never, 1 whenever the shape fits), "tile_fuse_qk" (default 1): the prefill tile GEMM;

@@ -1205,13 +1205,14 @@ static int forward_resident(nvllm_model* m, int R, int part_tiles, int parts, in
     a.xh = m->xh; a.xl = m->xl; a.ssq = m->ssqB; a.gave_up = m->resident_gave_up; a.host_gave_up = m->dev_resident; a.spins = m->opt_resident_spins;
     HIPCHK(m->ctx, resident_turn(m->ctx, a));
     m->resident_set ^= 1;
+    m->resident_ran = true;
     ++m->resident_launches;
     RowNorm rn;
     rn.ssq = m->ssqB; rn.groups = 1; rn.stride = kFusedMaxRows; rn.inv_h = 1.0f / (float)m->H; rn.eps = a.eps;
     return head_of_planes(m, rn, n_last, logits_row0);
 }
 // After a step's results are there: did its launch give up?  Then they are none, and the model's steps are launches from here on.
-static bool resident_gave_up(nvllm_model* m) { return m->h_resident && __atomic_load_n(m->h_resident, __ATOMIC_ACQUIRE) != 0; }
+static bool resident_gave_up(nvllm_model* m) { return m->resident_ran && __atomic_load_n(m->h_resident, __ATOMIC_ACQUIRE) != 0; }
 static int resident_close(nvllm_model* m) {
     HIPCHK(m->ctx, hipStreamSynchronize(m->ctx->stream));
     m->resident_closed = true;
@@ -1466,7 +1467,11 @@ static bool tile_resid_wins(int R, int H, int KO, int I) {
 static int forward_chunk(nvllm_model* m, int R, int n_tiles, int qt, int n_last, int logits_row0) {
     if (m->dec) return m->dec->forward_chunk(m, R, n_tiles, qt, n_last, logits_row0);
     int part_tiles = 0, parts = 0;
-    if (resident_plan(m, R, n_tiles, qt, part_tiles, parts)) return forward_resident(m, R, part_tiles, parts, n_last, logits_row0);
+    if (resident_plan(m, R, n_tiles, qt, part_tiles, parts)) {
+        if (__atomic_load_n(m->h_resident, __ATOMIC_ACQUIRE) == 0) return forward_resident(m, R, part_tiles, parts, n_last, logits_row0);
+        const int rc = resident_close(m);  // the launch of a step that failed before anybody looked
+        if (rc) return rc;
+    }
     FusedPlan fp;
     if (fused_plan(m, R, fp)) return forward_chunk_fused(m, fp, R, n_tiles, qt, n_last, logits_row0);
     nvllm_ctx* ctx = m->ctx;
@@ -1921,6 +1926,7 @@ static int finish_logits(nvllm_model* m, int n, uint32_t* next_ids, float* last_
     if (tp == 1) {
         uint32_t* ids = reinterpret_cast<uint32_t*>(m->pin_out + (size_t)m->out_slots * nvllm_model::kOutSlot);
         constexpr int slot = nvllm_model::kOutSlots;
+        if (m->opt_leave_fail > 0 && m->opt_leave_fail--) return fail(ctx, NVLLM_EHIP, "leave_fail");
         if (next_ids) HIPCHK(ctx, out_copy(m, slot, m->d_next, (size_t)m->out_slots * nvllm_model::kOutSlot, (size_t)n * 4));
         if (last_logits) {
             const int rc = download_logits(m, n, last_logits);
@@ -2173,6 +2179,7 @@ static int step_impl(nvllm_model* m, int n_seqs, const int64_t* seq_ids, const u
     m->want_ids = !score && !temperatures;
     m->cur_n = n_seqs;
     m->resident_waited = true;
+    m->resident_ran = false;
     m->cur_max_len = *std::max_element(lens, lens + n_seqs);
     set_attn_split(m, n_seqs, m->cur_max_len, std::accumulate(lens, lens + n_seqs, (int64_t)0));
     // rows and q-tiles
@@ -2348,6 +2355,7 @@ static int decode_core(nvllm_model* m, bool waited) {
     m->want_ids = true;
     m->cur_n = n;
     m->resident_waited = waited;
+    m->resident_ran = false;
     m->cur_max_len = *std::max_element(m->last_lens.begin(), m->last_lens.end()) + 1;
     set_attn_split(m, n, m->cur_max_len, std::accumulate(m->last_lens.begin(), m->last_lens.end(), (int64_t)n));
     const bool recurrent = m->dec && m->dec->recurrent();
@@ -2441,6 +2449,7 @@ extern "C" int nvllm_debug_set_option(nvllm_model* m, const char* name, int valu
     }
     if (!strcmp(name, "oneshot_skip_push")) { m->opt_oneshot_skip_push = std::max(0, value); return NVLLM_OK; }  // test hook
     if (!strcmp(name, "stage_fail")) { m->opt_stage_fail = std::max(0, value); return NVLLM_OK; }  // test hook
+    if (!strcmp(name, "leave_fail")) { m->opt_leave_fail = std::max(0, value); return NVLLM_OK; }  // test hook
     if (!strcmp(name, "resident")) { m->opt_resident = value; return NVLLM_OK; }
     if (!strcmp(name, "resident_spins")) { m->opt_resident_spins = std::max(0, value); return NVLLM_OK; }  // test hook
     if (!strcmp(name, "no_fused")) { m->opt_no_fused = value; return NVLLM_OK; }    // decode through the generic path

@@ -169,6 +169,7 @@ struct nvllm_model {
     int opt_kv_v_bits = 16;            // 24: V as f16 + e5m2 residual (13..14 significant bits, V bytes x1.5); read at kv_alloc
     int opt_kv_k_bits = 16;            // 24: K likewise (needs kv_v_bits = 24: K/V bytes x1.5 together); read at kv_alloc
     int opt_stage_fail = 0;            // test hook: the next N metadata launches fail before they are made
+    int opt_leave_fail = 0;            // test hook: the next N steps fail when their results are to leave
     int opt_oneshot_skip_push = 0;     // test hook: this rank "forgets" its next N pushes (the give-up path of its peers' waits)
     int opt_oneshot_spins = 20000000;  // bound of the one-shot wait kernel's poll (~ seconds): a missing peer is an error code
     int opt_no_fused = 0, opt_no_xpack = 0, opt_no_rowpar = 0;  // A/B switches (nvllm_debug_set_option): force the generic paths
@@ -192,6 +193,7 @@ struct nvllm_model {
     int resident_set = 0;
     bool resident_closed = false;          // a launch gave up: launches from then on
     bool resident_waited = false;          // the step's results are waited for before the next one is enqueued
+    bool resident_ran = false;             // this step is such a launch
     int opt_resident = 1;                  // 0: never
     int opt_resident_spins = 1000000;      // turns of a wait, about a second
     int64_t resident_launches = 0;

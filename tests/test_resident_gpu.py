@@ -112,6 +112,35 @@ def test_a_launch_that_gives_up(lens):
     assert taken == 1 and all(np.array_equal(a, b) for a, b in zip(got, want))
 
 
+def test_a_step_that_gives_up_and_then_fails():
+    # the next step is a prompt of several chunks: it is not that step's to run again, nor is the first decode step a launch that may read what is left
+    import nano_vllm_candle_amd as pkg
+
+    cfg, _ = config()
+    rng = np.random.default_rng(2)
+    first, prompt = rng.integers(0, 512, 30), rng.integers(0, 512, 200)
+    out = []
+    for fails in (1, 0):
+        m = pkg.Qwen3ForCausalLM.from_synthetic(cfg, seed=4)
+        m.kv_alloc(8, 2, 64)
+        m.step([0], [first], True)
+        if fails:
+            m.set_option("resident_spins", 0)
+            m.set_option("leave_fail", 1)
+            with pytest.raises(pkg._lib.NvllmError, match="leave_fail"):
+                m.step([0], [np.append(first, 7)], False)
+            m.set_option("resident_spins", 1000000)
+            assert m.counter("resident_launches") == 1
+        else:
+            m.set_option("resident", 0)
+        steps = [m.step([1], [prompt], True, want_logits=True)[1].copy()]
+        for k in (1, 2):
+            steps += [m.step([1], [np.append(prompt, [3] * k)], False, want_logits=True)[1].copy(), m.step([0], [np.append(first, [7] * k)], False, want_logits=True)[1].copy()]
+        out.append(steps)
+        m.close()
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
+
+
 def test_two_models_at_once():
     # each on its own thread and stream: their launches take turns
     import nano_vllm_candle_amd as pkg
