@@ -813,7 +813,8 @@ static int resident_empty(nvllm_model* m) {
 static int resident_alloc(nvllm_model* m) {
     nvllm_ctx* ctx = m->ctx;
     const ResidentSizes z = resident_sizes(m);
-    m->resident_closed = false;
+    m->resident_rest = 0;
+    m->resident_give_ups = 0;
     if (ctx->tp_size > 1 || !m->vlocache.empty() || !resident_sizes_ok(m->H, z) || m->L < kResidentLayers) return NVLLM_OK;
     int cus = 0;
     HIPCHK(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
@@ -1188,13 +1189,15 @@ static int head_of_planes(nvllm_model* m, RowNorm rn, int n_last, int logits_row
 //   4 x 2000 1183 / 793, 8 x 1000 1280 / 966, 8 x 4000 1625 / 1400, 8 x 8000 2225 / 2020
 // A context is one workgroup's up to 8 tiles (1 x 250, us: whole 548, in parts of 4 tiles 551; 8 x 250 844, 839); above, in the smallest parts that give every wave a tile and that there are
 // workgroups for (1 x 500 in parts of 4 tiles 557, of 8 590, whole 616; 8 x 500 846, 890, 930).
-static bool resident_plan(const nvllm_model* m, int R, int n_tiles, int qt, int& part_tiles, int& parts) {
-    if (!m->resident_buffer || m->resident_closed || !m->opt_resident || !m->resident_waited || qt != 1 || n_tiles != R || m->cur_n != R || R > kResidentRows || !m->decode_in_order) return false;
+static bool resident_plan(nvllm_model* m, int R, int n_tiles, int qt, int& part_tiles, int& parts) {
+    if (!m->resident_buffer || !m->opt_resident || !m->resident_waited || qt != 1 || n_tiles != R || m->cur_n != R || R > kResidentRows || !m->decode_in_order) return false;
     if (m->taps || m->opt_no_fused || m->opt_no_xpack || m->opt_no_attn_prologue || m->prof_kind || m->stamps_on) return false;
     const int tiles = (m->cur_max_len + 31) / 32, most = std::min(kResidentParts, kResidentGroups / (R * m->kv_l));
     part_tiles = tiles <= 8 ? tiles : std::max(4, (tiles + most - 1) / most);
     parts = (tiles + part_tiles - 1) / part_tiles;
-    return part_tiles <= 64;
+    if (part_tiles > 64) return false;
+    if (m->resident_rest > 0) { --m->resident_rest; return false; }
+    return true;
 }
 static int forward_resident(nvllm_model* m, int R, int part_tiles, int parts, int n_last, int logits_row0) {
     ResidentArgs a;
@@ -1211,11 +1214,13 @@ static int forward_resident(nvllm_model* m, int R, int part_tiles, int parts, in
     rn.ssq = m->ssqB; rn.groups = 1; rn.stride = kFusedMaxRows; rn.inv_h = 1.0f / (float)m->H; rn.eps = a.eps;
     return head_of_planes(m, rn, n_last, logits_row0);
 }
-// After a step's results are there: did its launch give up?  Then they are none, and the model's steps are launches from here on.
+// After a step's results are there: did its launch give up?  Then they are none, and the model's next steps are launches: kResidentRest, twice as many each time, for a wait that runs out
+// takes a second (so many steps of 0.6B as launches do, too), and what kept the launch off the chip may stay or end.
 static bool resident_gave_up(nvllm_model* m) { return m->resident_ran && __atomic_load_n(m->h_resident, __ATOMIC_ACQUIRE) != 0; }
 static int resident_close(nvllm_model* m) {
     HIPCHK(m->ctx, hipStreamSynchronize(m->ctx->stream));
-    m->resident_closed = true;
+    m->resident_rest = kResidentRest << std::min<int64_t>(m->resident_give_ups, 10);
+    ++m->resident_give_ups;
     *m->h_resident = 0;
     return resident_empty(m);
 }
@@ -2471,7 +2476,7 @@ extern "C" int nvllm_debug_set_option(nvllm_model* m, const char* name, int valu
 // "tile_gemm_launches" = projections this model has run on the prefill tile GEMM; "table_copies" = whole block tables sent;
 // "qk_rows16_launches" = q/k norm launches of 16 rows and a head per workgroup; "eight_wave_launches" = decode attention on eight waves; "merged_parts_launches" = ... in parts that are merged in the launch; "tiles_ahead_launches" = ... with a wave's second tile asked for before the prologue;
 // "prefill_dealt_launches" = prompt attention with a q-tile to a workgroup, "prefill_dealt_tiles" = q-tiles of those; "row_sum_launches" = products of a few rows that add up the slabs of the one before;
-// "resident_launches" = decode steps in one launch;
+// "resident_launches" = decode steps in one launch, "resident_give_ups" = those that gave up since kv_alloc;
 // "scan_gate_launches" = step sizes of a decode step's selective scan by a launch of their own; "two_product_launches" = pairs of products in one launch;
 // "row_pair_launches" = products of two row blocks at a time, of all models of the process; "tile_resid_launches" = products of a prompt chunk with
 // residual and norm preparation in their epilogue
@@ -2486,6 +2491,7 @@ extern "C" int nvllm_debug_get_counter(nvllm_model* m, const char* name, int64_t
     if (!strcmp(name, "prefill_dealt_launches")) { *value = m->prefill_dealt_launches; return NVLLM_OK; }
     if (!strcmp(name, "prefill_dealt_tiles")) { *value = m->prefill_dealt_tiles; return NVLLM_OK; }
     if (!strcmp(name, "resident_launches")) { *value = m->resident_launches; return NVLLM_OK; }
+    if (!strcmp(name, "resident_give_ups")) { *value = m->resident_give_ups; return NVLLM_OK; }
     if (!strcmp(name, "row_sum_launches")) { *value = m->row_sum_launches; return NVLLM_OK; }
     if (!strcmp(name, "scan_gate_launches")) { *value = m->scan_gate_launches; return NVLLM_OK; }
     if (!strcmp(name, "two_product_launches")) { *value = m->two_launches; return NVLLM_OK; }

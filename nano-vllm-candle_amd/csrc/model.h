@@ -191,7 +191,8 @@ struct nvllm_model {
     int* resident_gave_up = nullptr;       // device: a wait of the last launch ran out ...
     int *h_resident = nullptr, *dev_resident = nullptr;  // ... and the same in pinned memory
     int resident_set = 0;
-    bool resident_closed = false;          // a launch gave up: launches from then on
+    int resident_rest = 0;                 // after a launch that gave up: steps that stay launches
+    int64_t resident_give_ups = 0;         // since kv_alloc
     bool resident_waited = false;          // the step's results are waited for before the next one is enqueued
     bool resident_ran = false;             // this step is such a launch
     int opt_resident = 1;                  // 0: never

@@ -7,6 +7,7 @@ namespace nvllm {
 constexpr int kResidentGroups = 256;   // workgroups, all of them on the chip at once, one to a CU
 constexpr int kResidentRows = 8;       // rows of a step at most
 constexpr int kResidentLayers = 4;     // layers of a model at least
+constexpr int kResidentRest = 1024;    // steps as launches behind one that gave up, the first time
 constexpr int kResidentParts = 16;     // parts of a context at most
 constexpr int kResidentPart = 132;     // a part's result: 128 sums, the softmax's reference and its sum
 constexpr uint32_t kResidentEmpty = 0xFFFFFFFFu;  // a place of the hand-off buffers that holds no value

@@ -112,6 +112,30 @@ def test_a_launch_that_gives_up(lens):
     assert taken == 1 and all(np.array_equal(a, b) for a, b in zip(got, want))
 
 
+def test_giving_up_is_not_for_good():
+    # counted, and after some steps as launches (the one that is run again is the first), twice as many each time, the model tries again
+    import nano_vllm_candle_amd as pkg
+
+    m = pkg.Qwen3ForCausalLM.from_synthetic(config()[0], seed=4)
+    m.kv_alloc(2, 1, 256)
+    m.step([0], [[1, 2, 3]], True)
+
+    def launches_until_the_next():
+        at, n = m.counter("resident_launches"), 0
+        while m.counter("resident_launches") == at:
+            m.step([0], [[1, 2, 3, 4]], False)
+            n += 1
+        return n - 1
+
+    m.set_option("resident_spins", 0)
+    assert launches_until_the_next() == 0 and m.counter("resident_give_ups") == 1
+    assert launches_until_the_next() == 1023 and m.counter("resident_give_ups") == 2
+    m.set_option("resident_spins", 1000000)
+    assert launches_until_the_next() == 2047 and m.counter("resident_give_ups") == 2
+    assert launches_until_the_next() == 0
+    m.close()
+
+
 def test_a_step_that_gives_up_and_then_fails():
     # the next step is a prompt of several chunks: it is not that step's to run again, nor is the first decode step a launch that may read what is left
     import nano_vllm_candle_amd as pkg
