@@ -18,6 +18,7 @@
 #include <memory>
 #include <mutex>
 #include <numeric>
+#include <set>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -245,27 +246,43 @@ static int oneshot_setup(nvllm_ctx* ctx, size_t slot_floats) {
 }
 
 // Resident steps (resident.hip) of one device one after the other: each wants every CU, and two that had a part of them each would wait for one another until they
-// give up.  The stream of the last one; a step on another stream waits for what that one holds so far.
+// give up.  A step waits for the last such launch of another stream and for nothing behind it.  While a device has one context with such steps there is no event to record.
+struct ResidentTurns {
+    nvllm_ctx* last = nullptr;      // whose launch was the last one
+    std::set<nvllm_ctx*> contexts;  // that have made one
+};
 static std::mutex g_resident_mu;
-static std::map<int, nvllm_ctx*> g_resident_last;
+static std::map<int, ResidentTurns> g_resident_turns;
 static hipError_t resident_turn(nvllm_ctx* ctx, const ResidentArgs& a) {
     std::lock_guard<std::mutex> lk(g_resident_mu);
-    nvllm_ctx*& last = g_resident_last[ctx->device];
-    if (last && last != ctx) {
+    ResidentTurns& t = g_resident_turns[ctx->device];
+    t.contexts.insert(ctx);
+    auto record = [](nvllm_ctx* c) {
         hipError_t e = hipSuccess;
-        if (!ctx->resident_ev) e = hipEventCreateWithFlags(&ctx->resident_ev, hipEventDisableTiming);
-        if (e == hipSuccess) e = hipEventRecord(ctx->resident_ev, last->stream);
-        if (e == hipSuccess) e = hipStreamWaitEvent(ctx->stream, ctx->resident_ev, 0);
-        if (e != hipSuccess) return e;
+        if (!c->resident_ev) e = hipEventCreateWithFlags(&c->resident_ev, hipEventDisableTiming);
+        if (e == hipSuccess) e = hipEventRecord(c->resident_ev, c->stream);
+        c->resident_recorded = e == hipSuccess;
+        return e;
+    };
+    hipError_t e = hipSuccess;
+    if (t.last && t.last != ctx) {
+        if (!t.last->resident_recorded) e = record(t.last);  // (its launches were the only ones so far: behind all that its stream holds)
+        if (e == hipSuccess) e = hipStreamWaitEvent(ctx->stream, t.last->resident_ev, 0);
     }
-    last = ctx;
-    return launch_resident(a, ctx->stream);
+    if (e == hipSuccess) e = launch_resident(a, ctx->stream);
+    if (e != hipSuccess) return e;
+    t.last = ctx;
+    ctx->resident_recorded = false;
+    return t.contexts.size() > 1 ? record(ctx) : hipSuccess;
 }
 static void resident_leave(nvllm_ctx* ctx) {  // its stream is idle
     {
         std::lock_guard<std::mutex> lk(g_resident_mu);
-        const auto it = g_resident_last.find(ctx->device);
-        if (it != g_resident_last.end() && it->second == ctx) g_resident_last.erase(it);
+        const auto it = g_resident_turns.find(ctx->device);
+        if (it != g_resident_turns.end()) {
+            it->second.contexts.erase(ctx);
+            if (it->second.last == ctx) it->second.last = nullptr;
+        }
     }
     if (ctx->resident_ev) (void)hipEventDestroy(ctx->resident_ev);
 }

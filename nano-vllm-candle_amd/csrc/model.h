@@ -51,7 +51,8 @@ struct nvllm_ctx {
     size_t os_slot = 0, os_data_bytes = 0, os_flag_bytes = 0;
     uint64_t os_calls = 0;
     OneShotPeers os_peers;
-    hipEvent_t resident_ev = nullptr;  // see resident_turn
+    hipEvent_t resident_ev = nullptr;  // see resident_turn: behind this context's last resident step, if recorded
+    bool resident_recorded = false;
     std::vector<void*> os_ipc;    // peer mappings opened with hipIpcOpenMemHandle
 };
 

@@ -192,3 +192,40 @@ def test_two_models_at_once():
     [t.join() for t in threads]
     for k in lens:
         assert got[k][1] == 40 and all(np.array_equal(a, b) for a, b in zip(got[k][0], want[k][0]))
+
+
+def test_a_turn_does_not_wait_for_other_work():
+    # behind the other context's last one-launch step comes its queue of many rows: only the former is waited for
+    import time
+
+    import nano_vllm_candle_amd as pkg
+
+    rows = 200
+    one = pkg.Qwen3ForCausalLM.from_synthetic(config()[0], seed=4)
+    one.kv_alloc(2, 1, 256)
+    many = pkg.Qwen3ForCausalLM.from_synthetic(config(layers=28)[0], seed=4)
+    many.kv_alloc(rows + 1, rows + 1, 1024)
+    alone, ids = many.max_seqs - 1, list(range(rows))
+    one.step([0], [[1, 2, 3]], True)
+    many.step([alone], [[1, 2, 3]], True)
+    for k in range(2):  # both have made such steps, each behind the other's
+        one.decode_next()
+        many.step([alone], [[1, 2, 3, 4]], False)
+    assert one.counter("resident_launches") == 2 and many.counter("resident_launches") == 2
+    many.step(ids, [[1 + i, 2, 3] for i in ids], True)
+    shares = []
+    for _ in range(5):
+        many.step([alone], [[1, 2, 3, 4]], False)
+        many.step(ids, [[1 + i, 2, 3, 4] for i in ids], False)
+        t0 = time.perf_counter()
+        for _ in range(4):
+            many.decode_enqueue()
+        one.decode_next()
+        t1 = time.perf_counter()
+        for _ in range(4):
+            many.decode_collect()
+        shares.append((t1 - t0) / (time.perf_counter() - t0))
+    assert one.counter("resident_launches") == 7 and many.counter("resident_launches") == 7 and one.counter("resident_give_ups") == 0
+    assert sorted(shares)[2] < 0.7, shares  # all of it, where the queue is waited for
+    one.close()
+    many.close()
