@@ -74,7 +74,7 @@ GluPlan plan_glu(const nvllm_model* m, int R, const PackedW& w, bool want_packed
         g.out_packed_ok = dir;
         return g;
     }
-    if (gemm_stream_splits(R, w.N, w.K) > 0 || want_packed_out) {
+    if ((R > 16 ? gemm_stream_splits(R, w.N, w.K) > 0 : gemm_streams(m, w, R)) || want_packed_out) {
         g.kind = P_STREAM;
         g.slabs = plan_product(m, R, w);
         g.packed = g.slabs.packed;

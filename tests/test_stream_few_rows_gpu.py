@@ -43,3 +43,24 @@ def test_a_gated_feed_forward(oracle):
         # the same products of the same planes, summed in another order; a cached key or value may round the other way (2^-11 of itself)
         assert np.abs(got - want[:rows]).max() < 2.0 ** -11 * np.abs(want).max(), rows
     m.close()
+
+
+@pytest.mark.parametrize("tp,launches", [(1, 1), (2, 0)])
+def test_a_shard_keeps_its_own_rule(tp, launches):
+    # gate/up of 80 MB with no row form: slabs and an activation launch on one GPU, of a shard of two (communication left out) one product with the activation in its epilogue, up to 16 rows
+    import nano_vllm_candle_amd as pkg
+    from bench_berevik import SIZES, berevik_config
+
+    z = dict(SIZES["4k"], width=5120, ff=4096 * tp, layers=1)
+    ctx = pkg.Context(0, tp_rank=0, tp_size=tp, null_comm=True)
+    m = pkg.BerevikForCausalLM.from_random(berevik_config(pkg, z, 1024, 1 << 20), ctx=ctx)
+    m.kv_alloc(20, 17, 256)
+    seqs = [[1 + i, 2, 3] for i in range(17)]
+    m.step(list(range(17)), [s[:2] for s in seqs], True)
+    for rows in (1, 8, 16, 17):
+        m.profile_kernel("silu")
+        m.step(list(range(rows)), seqs[:rows], False)
+        assert m.profile_read()[1] == (launches if rows <= 16 else 1), rows
+        m.profile_kernel(None)
+    m.close()
+    ctx.close()
