@@ -1136,7 +1136,8 @@ static bool fused_plan(const nvllm_model* m, int R, FusedPlan& p) {
     const int H = m->H, hd = m->hd, NQ = (m->nh_l + 2 * m->kv_l) * hd, KO = m->nh_l * hd, I2 = 2 * m->I_l;
     const bool tp = m->ctx->tp_size > 1;
     if (R > (tp ? 256 : kFusedMaxRows) || m->taps || m->opt_no_fused) return false;
-    if (R > 256 && m->opt_tile_min_wgs == 1) return false;  // (the option asks for tile products wherever they fit)
+    // past 256 rows row pairs alone, which take packed planes; and one option asks for tile products wherever they fit
+    if (R > 256 && (m->opt_no_xpack || m->opt_tile_min_wgs == 1)) return false;
     // more than kRowMaxRows: only where every projection is the register-direct kernel's (below, slabs and staged forms fall behind the
     // prompt path's tile products)
     if (R > kRowMaxRows && !(gemm_rowdir_ok(NQ, H, 2, R) && gemm_rowdir_ok(H, KO, tp ? 2 : 0, R) && gemm_rowdir_ok(I2, H, 1, R) && gemm_rowdir_ok(H, m->I_l, tp ? 2 : 0, R)))

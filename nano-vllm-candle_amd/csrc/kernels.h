@@ -393,9 +393,9 @@ int64_t rowpair_launches();  // of the form that takes two row blocks at a time,
 // two plain products (epi 2) of the same rows in one launch
 bool gemm_rowdir_two_ok(const PackedW& wa, const PackedW& wb, int M);
 hipError_t launch_gemm_rowdir_two(const RowParArgs& a, const PackedW& wa, const RowParArgs& b, const PackedW& wb, hipStream_t s);
-// true when launch_gemm_rowpar would run the register-direct kernel (the one that accepts packed planes)
-constexpr int kRowPairRows = 896;  // of the products of two row blocks at a time; a shape that has no such form is none of this kernel's past 256
+constexpr int kRowPairRows = 896;  // of the products of two row blocks at a time, of packed planes; a shape that has no such form is not register-direct past 256
 bool gemm_rowpair_at_once(int N, int K, int epi, int M);  // is the product such a one, and are there CUs for all of its workgroups?
+// true when launch_gemm_rowpar would run the register-direct kernel (the one that accepts packed planes)
 bool gemm_rowdir_ok(int N, int K, int epi, int M);
 bool gemm_rowpar_ok(int N, int K, int epi, int M);
 int gemm_rowpar_splits(int N, int K, int epi, int M);  // f32 slabs the plain epilogue leaves (1 = complete sums)

@@ -108,3 +108,21 @@ def test_a_decode_step(rows):
     m.step(ids, [s[:-1] for s in seqs], True)
     compare(m, lambda: m.step_score(ids, seqs, False, [[len(s) - 1] for s in seqs]), 8)
     m.close()
+
+
+@pytest.mark.parametrize("rows", [257, 480])
+def test_row_major_planes(rows):
+    # row pairs read packed planes: without them tile products, as past 480 rows
+    import nano_vllm_candle_amd as pkg
+
+    cfg, m = model(pkg, 4)
+    t = np.random.default_rng(rows).integers(0, cfg.vocab_size, rows)
+    m.set_option("no_xpack", 1)
+    n, tiles = m.counter("row_pair_launches"), m.counter("tile_gemm_launches")
+    got = m.step_score([0], [t], True, [[rows - 1]])
+    assert m.counter("row_pair_launches") == n and m.counter("tile_gemm_launches") > tiles
+    m.set_option("no_xpack", 0)
+    want = m.step_score([0], [t], True, [[rows - 1]])
+    # as in compare()
+    assert m.counter("row_pair_launches") == n + 8 and np.abs(got - want).max() < 2.0 ** -11 * np.abs(want).max()
+    m.close()
