@@ -14,8 +14,8 @@
 #include "../../include/nvllm_amd_debug.h"
 #include "kernels.h"
 #include "latent.h"
-#include "resident.h"
 
+namespace nvllm { struct ResidentLayer; }
 using namespace nvllm;
 
 // In-process loopback communicator (tests only): contexts created with the same group name by different
