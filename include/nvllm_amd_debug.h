@@ -52,7 +52,7 @@ int nvllm_debug_set_option(nvllm_model* m, const char* name, int value);
  * workgroup; "eight_wave_launches" = decode attention on eight waves a workgroup, "merged_parts_launches" = ... in parts that are merged in the launch; "prefill_dealt_launches" = prompt attention
  * with a q-tile to a workgroup, "prefill_dealt_tiles" = q-tiles of those; "resident_launches" = decode steps in one launch, "resident_give_ups" = those that gave up since kv_alloc (what else holds the device's CUs kept them off the chip; the next 1024 steps are launches, twice as many each time); "row_sum_launches" = products of one to a few rows that add up the slabs of the one before; "scan_gate_launches" = step sizes of a
  * decode step's selective scan by a launch of their own; "two_product_launches" = pairs of products in one launch;
- * "row_pair_launches" = products of two row blocks at a time, of all models of the process; "tile_resid_launches" = products
+ * "row_pair_launches" = products of two row blocks at a time, "stream_launches" = streaming products, of all models of the process; "tile_resid_launches" = products
  * of a prompt chunk with residual and norm preparation in their epilogue; "kv_f16_saturated" = elements of the K/V pool at the
  * f16 clamp (every cache write saturates at +-65504; a scan of the pool, off the hot path); "kv_f16_absmax_bits" = the largest
  * magnitude the pool holds, as f16 bits */

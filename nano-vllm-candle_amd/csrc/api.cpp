@@ -2496,7 +2496,7 @@ extern "C" int nvllm_debug_set_option(nvllm_model* m, const char* name, int valu
 // "prefill_dealt_launches" = prompt attention with a q-tile to a workgroup, "prefill_dealt_tiles" = q-tiles of those; "row_sum_launches" = products of a few rows that add up the slabs of the one before;
 // "resident_launches" = decode steps in one launch, "resident_give_ups" = those that gave up since kv_alloc;
 // "scan_gate_launches" = step sizes of a decode step's selective scan by a launch of their own; "two_product_launches" = pairs of products in one launch;
-// "row_pair_launches" = products of two row blocks at a time, of all models of the process; "tile_resid_launches" = products of a prompt chunk with
+// "row_pair_launches" = products of two row blocks at a time, "stream_launches" = streaming products, of all models of the process; "tile_resid_launches" = products of a prompt chunk with
 // residual and norm preparation in their epilogue
 extern "C" int nvllm_debug_get_counter(nvllm_model* m, const char* name, int64_t* value) {
     if (!m || !name || !value) return NVLLM_EINVAL;
@@ -2514,6 +2514,7 @@ extern "C" int nvllm_debug_get_counter(nvllm_model* m, const char* name, int64_t
     if (!strcmp(name, "scan_gate_launches")) { *value = m->scan_gate_launches; return NVLLM_OK; }
     if (!strcmp(name, "two_product_launches")) { *value = m->two_launches; return NVLLM_OK; }
     if (!strcmp(name, "row_pair_launches")) { *value = rowpair_launches(); return NVLLM_OK; }
+    if (!strcmp(name, "stream_launches")) { *value = stream_launches(); return NVLLM_OK; }
     if (!strcmp(name, "eight_wave_launches")) { *value = m->eight_wave_launches; return NVLLM_OK; }
     if (!strcmp(name, "merged_parts_launches")) { *value = m->merged_parts_launches; return NVLLM_OK; }
     if (!strcmp(name, "tiles_ahead_launches")) { *value = m->tiles_ahead_launches; return NVLLM_OK; }

@@ -93,6 +93,7 @@ int gemm_stream_splits(int M, int N, int K);
 // x_packed: the planes are in xpack_off order (ldx = K either way)
 hipError_t launch_gemm_stream(const bf16_bits* xh, const bf16_bits* xl, int ldx, const PackedW& w, float* out, int M, int x_packed,
                               hipStream_t s);
+int64_t stream_launches();  // of launch_gemm_stream, by this process so far (tests)
 // The same kernel with an epilogue on COMPLETE sums (stream_gemm.hip): epi 1 plain f32 [M][N], 2 SwiGLU (w = interleaved
 // gate/up, act hi/lo [M][N/2], input norm rn deferred), 3 residual + next-norm prep (as gemm_rowpar epilogue 0).  K slices
 // combine inside the launch through `slabs` ([gemm_stream_slab_floats] f32 scratch) and `tickets` ([n-groups] unsigned,

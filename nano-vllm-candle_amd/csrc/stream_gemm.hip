@@ -430,11 +430,14 @@ hipError_t launch_gemm_stream_epi(const StreamArgs& a, const PackedW& w, int epi
     if (epi == 3) return stream_dispatch<3>(sh, a, w, s);
     return hipErrorInvalidValue;
 }
+static std::atomic<int64_t> g_stream_launches{0};
+int64_t stream_launches() { return g_stream_launches.load(std::memory_order_relaxed); }
 hipError_t launch_gemm_stream(const bf16_bits* xh, const bf16_bits* xl, int ldx, const PackedW& w, float* out, int M, int x_packed,
                               hipStream_t s) {
     if (!stream_shape(M, w.N, w.K, 0, false).nt) return hipErrorNotSupported;
     StreamArgs a;
     a.xh = xh; a.xl = xl; a.ldx = ldx; a.x_packed = x_packed; a.M = M; a.slabs = out;
+    g_stream_launches.fetch_add(1, std::memory_order_relaxed);
     return launch_gemm_stream_epi(a, w, 0, s);
 }
 

@@ -1,4 +1,4 @@
-"""GPU test of the streaming products of one to 16 rows: Qwen3 layers whose four products stream, with planes of one row and of a whole row block, against the oracle, and a layer of another design,
+"""GPU test of the streaming products of one to 16 rows: Qwen3 layers whose four products stream, and where two do beside others, with planes of one row and of a whole row block, against the oracle, and a layer of another design,
 whose gated feed-forward streams, against the same rows in a batch of 17."""
 import numpy as np
 import pytest
@@ -8,8 +8,8 @@ from tests.util import LOGITS_TOL, oracle_config, row_rel_err
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("hidden,inter,heads,kv", [(4096, 12288, 32, 8), (5120, 6528, 40, 8)])
-def test_qwen_layers_against_the_oracle(oracle, hidden, inter, heads, kv):
+@pytest.mark.parametrize("hidden,inter,heads,kv,streams", [(4096, 12288, 32, 8, 4), (5120, 6528, 40, 8, 2)])
+def test_qwen_layers_against_the_oracle(oracle, hidden, inter, heads, kv, streams):
     import nano_vllm_candle_amd as pkg
 
     cfg = pkg.Qwen3Config.tiny(vocab_size=1024, hidden_size=hidden, intermediate_size=inter, num_attention_heads=heads, num_key_value_heads=kv, head_dim=128, num_hidden_layers=1)
@@ -22,7 +22,9 @@ def test_qwen_layers_against_the_oracle(oracle, hidden, inter, heads, kv):
         m.step([i], [s[:-1]], True)
     _, want = om.run_greedy(seqs)
     for rows in (1, 3, 4, 15, 16):
+        n = m.counter("stream_launches")
         _, got = m.step(list(range(rows)), seqs[:rows], False, want_logits=True)
+        assert m.counter("stream_launches") - n == streams
         assert row_rel_err(got, want[:rows]) < LOGITS_TOL, rows
     m.close()
 
@@ -39,7 +41,9 @@ def test_a_gated_feed_forward(oracle):
     m.step(list(range(17)), [s[:2] for s in seqs], True)
     want = m.step_score(list(range(17)), seqs, False, [[2]] * 17)
     for rows in (1, 3, 4, 16):
+        n = m.counter("stream_launches")
         got = m.step_score(list(range(rows)), seqs[:rows], False, [[2]] * rows)
+        assert m.counter("stream_launches") - n == 4
         # the same products of the same planes, summed in another order; a cached key or value may round the other way (2^-11 of itself)
         assert np.abs(got - want[:rows]).max() < 2.0 ** -11 * np.abs(want).max(), rows
     m.close()
