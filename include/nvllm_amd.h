@@ -256,7 +256,8 @@ int nvllm_decode_next(nvllm_model* m, uint32_t* next_ids);
 
 /* Pipelined form of nvllm_decode_next: enqueue puts one more decode step on the stream and returns at once (up to 4
  * in flight); collect waits for the OLDEST enqueued step and returns its ids.  Enqueueing step t+1 before collecting
- * step t hides the host round trip between steps. */
+ * step t hides the host round trip between steps.  The results agree with nvllm_decode_next within rounding and not bit
+ * for bit: a step of few rows whose results are waited for may run in one launch, which adds up in another order. */
 int nvllm_decode_enqueue(nvllm_model* m);
 int nvllm_decode_collect(nvllm_model* m, uint32_t* next_ids);
 

@@ -25,7 +25,8 @@ int nvllm_ctx_create_null_comm(int device_ordinal, int tp_rank, int tp_size, nvl
  * 7 calibration (an event pair around NO launch, recorded where the decode attention launch sits: the elapsed
  * time of an empty bracket between busy kernels, to be subtracted from the bracketed durations).
  * While a kind is set every launch of that class is bracketed by two events; read returns the summed
- * elapsed ms and the number of launches since the last read. */
+ * elapsed ms and the number of launches since the last read.  Decode steps that run in one launch otherwise ("resident"
+ * below) run as launches then, and with layer taps on: what is read describes those. */
 int nvllm_profile_kernel(nvllm_model* m, int kind);
 int nvllm_profile_read(nvllm_model* m, double* total_ms, int64_t* launches);
 /* Per-model options (A/B runs, tests, and two deployment knobs).  The library reads no environment variable.

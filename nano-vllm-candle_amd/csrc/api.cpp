@@ -1203,8 +1203,8 @@ static int head_of_planes(nvllm_model* m, RowNorm rn, int n_last, int logits_row
 // A decode step of one to kResidentRows rows in one launch and the head's, wherever sizes, cache and device are its own (resident_alloc).  Not where the next step is enqueued
 // before this one's results are waited for: a launch that gives up is made good by running the step again.  Nor where a part of a context would be longer than 64 tiles, 8 rows of
 // 8000 tokens, where launches are nearly as fast.  0.6B, one step with its logits, us, as launches / resident:
-//   1 row of 137 774 / 542, of 2000 982 / 590, of 16000 1378 / 868;  2 rows of 137 860 / 602, 4 910 / 685, 6 1006 / 810, 8 1040 / 855
-//   4 x 2000 1183 / 793, 8 x 1000 1280 / 966, 8 x 4000 1625 / 1400, 8 x 8000 2225 / 2020
+//   1 row of 137 780 / 548, of 2000 864 / 598, of 16000 1145 / 870;  2 rows of 137 836 / 606, 4 914 / 693, 6 1000 / 805, 8 1024 / 842
+//   4 x 2000 1091 / 805, 8 x 1000 1204 / 956, 8 x 4000 1562 / 1427, 8 x 8000 2186 / 2032
 // A context is one workgroup's up to 8 tiles (1 x 250, us: whole 548, in parts of 4 tiles 551; 8 x 250 844, 839); above, in the smallest parts that give every wave a tile and that there are
 // workgroups for (1 x 500 in parts of 4 tiles 557, of 8 590, whole 616; 8 x 500 846, 890, 930).
 static bool resident_plan(nvllm_model* m, int R, int n_tiles, int qt, int& part_tiles, int& parts) {
